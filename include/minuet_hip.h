@@ -587,6 +587,60 @@ int mnt_sparse_convolution_forward_implicit(const void *sources, const void *wei
 int mnt_kernel_map_invert(const int32_t *kernel_map, int64_t num_offsets, int64_t num_targets,
                           int64_t num_sources, int32_t *inverse_out, void *stream);
 
+/* ---- Map: the coordinates and kernel maps of a whole pass in one build ------ */
+
+/* A network asks for the same coordinate levels and kernel maps for every
+ * cloud.  With the list of them (kept from an earlier pass) all levels are
+ * marked, counted and written together and all maps are looked up together:
+ * about ten launches and one wait on the host instead of 60 launches and one
+ * wait per level.  Results are those of mnt_target_coordinates,
+ * mnt_kernel_map_dense, mnt_kernel_map_invert, mnt_kernel_map_offset_groups and
+ * mnt_kernel_map_build called one after another.  The reference builds each of
+ * them at the first layer that asks (minuet/nn/convolutions.py:58-173).
+ *
+ * Two calls, with no other library call on that stream in between:
+ *   mnt_pass_levels  marks the levels (level l + 1 = levels[l], its stride a
+ *                    multiple of the cloud's; level 0 is the cloud itself),
+ *                    waits for their row counts and works out where in one
+ *                    block of total_bytes_out bytes every result goes (the
+ *                    `at` fields, byte offsets at multiples of 256);
+ *   mnt_pass_build   writes everything into the block at `base` (256-byte
+ *                    aligned); waits once more if tables were asked for.
+ * supported_out is 0, and nothing is left pending, where this form does not
+ * apply (keys of the levels over 28 bits together, frames over 63 bits, more
+ * offsets than fit its tables ...): the caller then builds one by one. */
+#define MNT_PASS_INVERSE 1   /* the inverse map [O, S] of the dense one */
+#define MNT_PASS_GROUPS 2    /* offset groups (27 offsets, group_offsets_host given) */
+#define MNT_PASS_TABLES 4    /* sizes, order, rank tables and pair lists */
+
+typedef struct mnt_pass_level {
+  int64_t stride[4];         /* coordinates are floor(c / stride) * stride */
+  int64_t count;             /* out: rows */
+  int64_t coords_at;         /* out: [count, ndim] of the coordinate type */
+  int64_t batch_dims_at;     /* out: [num_batches + 1] of the index type (-1: no batches) */
+} mnt_pass_level;
+
+typedef struct mnt_pass_map {
+  int32_t source_level, target_level;
+  int32_t want;              /* MNT_PASS_*; the dense map is always made */
+  int32_t reorder;           /* tables: rows by ascending size */
+  const int64_t *offsets_host;          /* [num_offsets, ndim] */
+  int64_t num_offsets;
+  const int32_t *group_offsets_host;    /* [3, 9, 3] */
+  int64_t *sizes_host, *order_host;     /* tables: [num_offsets] each, written by mnt_pass_build */
+  int64_t num_sources, num_targets;     /* out */
+  /* out, -1 where not wanted: dense, inverse, rank, src, head, source_masks,
+   * target_masks, in_idx, out_idx, sizes, order */
+  int64_t at[11];
+} mnt_pass_map;
+
+int mnt_pass_levels(const void *coords, int64_t n, int ndim, int coord_dtype, const void *batch_dims,
+                    int64_t num_batches, int index_dtype, const int64_t *bounds_host,
+                    mnt_pass_level *levels, int num_levels, mnt_pass_map *maps, int num_maps,
+                    int64_t *bounds_host_out, int64_t *total_bytes_out, int *supported_out, void *stream);
+int mnt_pass_build(const void *coords, const void *batch_dims, mnt_pass_level *levels, mnt_pass_map *maps,
+                   void *base, void *stream);
+
 /* ---- Map: building a pass's coordinates and kernel maps ahead ------------- */
 
 /* A network that has seen one cloud asks for the same coordinate levels and

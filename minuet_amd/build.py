@@ -11,7 +11,8 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(_HERE, "csrc")
 LIB_DIR = os.path.join(_HERE, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libminuet_hip.so")
-SOURCES = ["runtime.hip", "sort.hip", "unique.hip", "query.hip", "conv.hip", "implicit.hip", "lookahead.hip"]
+HOST_PATH = os.path.join(LIB_DIR, "minuet_host.so")
+SOURCES = ["runtime.hip", "sort.hip", "unique.hip", "query.hip", "pass.hip", "conv.hip", "implicit.hip", "lookahead.hip"]
 ARCH = "gfx950"
 FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC",
@@ -37,11 +38,34 @@ def _compile(src: str) -> str:
     return obj
 
 
-def build_library(verbose: bool = True) -> str:
-    """Compile every HIP source and link the shared library.  Always rebuilds."""
+def build_host() -> str:
+    """Compile the Python extension module with the host side of layer calls
+    (csrc/host.cpp, plain C++ against torch's headers)."""
+    import sysconfig
+    import torch
+    from torch.utils.cpp_extension import include_paths
     os.makedirs(LIB_DIR, exist_ok=True)
-    with ThreadPoolExecutor(max_workers=min(8, len(SOURCES))) as pool:
+    libraries = os.path.join(os.path.dirname(torch.__file__), "lib")
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__",
+           "-DUSE_ROCM", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *[f"-I{path}" for path in include_paths()], f"-I{sysconfig.get_paths()['include']}",
+           f"-I{os.path.join(os.environ.get('ROCM_PATH', '/opt/rocm'), 'include')}",
+           os.path.join(CSRC, "host.cpp"), "-o", HOST_PATH, f"-L{libraries}", "-ltorch_python", "-ltorch_cpu",
+           "-ltorch_hip", "-lc10", "-lc10_hip"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"{cmd[0]} failed on host.cpp:\n{proc.stdout}\n{proc.stderr}")
+    return HOST_PATH
+
+
+def build_library(verbose: bool = True) -> str:
+    """Compile every HIP source, link the shared library and build the host
+    extension.  Always rebuilds."""
+    os.makedirs(LIB_DIR, exist_ok=True)
+    with ThreadPoolExecutor(max_workers=min(8, len(SOURCES) + 1)) as pool:
+        host = pool.submit(build_host)
         objects = list(pool.map(_compile, SOURCES))
+        host.result()
     cmd = [_hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *objects, "-o", LIB_PATH]
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:

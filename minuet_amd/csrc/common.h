@@ -8,6 +8,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -129,9 +130,11 @@ class Arena {
   unsigned long long next_sequence() { return ++sequence_; }
   unsigned long long *flag_device(int slot);
   void wait_flag(int slot, unsigned long long sequence);
+  // The same for any word of the pinned block.
+  void wait_word(volatile unsigned long long *word, unsigned long long sequence);
   // Long-lived device blocks that survive scopes (state of the two-phase entry
-  // points; slot 0: target coordinates, slot 1: kernel-map build).  Grows to
-  // at least `bytes`; 0 returns the current block.
+  // points; slot 0: target coordinates, slot 1: kernel-map build, slot 2: pass
+  // builder).  Grows to at least `bytes`; 0 returns the current block.
   void *persistent(int slot, size_t bytes);
 
   hipStream_t stream() const { return stream_; }
@@ -153,6 +156,9 @@ class Arena {
 
   // State handed from mnt_kernel_map_query to mnt_kernel_map_emit.
   bool map_state_valid = false;
+  // What mnt_pass_levels leaves for mnt_pass_build.
+  bool pass_pending = false;
+  std::shared_ptr<void> pass_state;
   alignas(8) unsigned char map_state[64] = {0};
 
  private:
@@ -173,8 +179,9 @@ class Arena {
   void *pinned_ = nullptr;
   void *pinned_device_ = nullptr;
   unsigned long long sequence_ = 0;
-  void *persistent_[2] = {nullptr, nullptr};
-  size_t persistent_size_[2] = {0, 0};
+  static constexpr int kPersistentSlots = 3;
+  void *persistent_[kPersistentSlots] = {nullptr, nullptr, nullptr};
+  size_t persistent_size_[kPersistentSlots] = {0, 0, 0};
   // guarded by the registry's mutex
   bool held_ = false, pinned_by_thread_ = false;
   unsigned long long holder_ = 0;            // token of the thread inside a call / that pinned it

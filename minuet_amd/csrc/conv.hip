@@ -15,6 +15,7 @@
 
 #include "conv_device.h"
 #include "device_utils.h"
+#include "pass.h"
 #include "sort.h"
 
 namespace mnt {
@@ -1066,6 +1067,20 @@ struct GroupOffsets {
 };
 constexpr int kGroupTile = 256;
 
+// The maps of one launch of each of the three steps (blockIdx.z, or blockIdx.x
+// of the scan, is the map): a network's wide levels are built together.
+constexpr int kGroupMaps = 4;
+struct GroupJob {
+  const int *dense;
+  int *tile_counts, *head, *rank;
+  int4 *src;
+  int num_targets, tiles;
+  GroupOffsets tab;
+};
+struct GroupJobs {
+  GroupJob job[kGroupMaps];
+};
+
 __device__ __forceinline__ bool group_reaches(const int *__restrict__ dense, long long num_targets,
                                               const GroupOffsets &tab, int slot, long long t, int (&row)[3]) {
   bool any = false;
@@ -1077,10 +1092,15 @@ __device__ __forceinline__ bool group_reaches(const int *__restrict__ dense, lon
   return any;
 }
 
-__global__ __launch_bounds__(kGroupTile) void group_count_kernel(const int *__restrict__ dense,
-                                                                  long long num_targets, GroupOffsets tab,
-                                                                  int tiles, int *__restrict__ tile_counts) {
+__global__ __launch_bounds__(kGroupTile) void group_count_kernel(GroupJobs jobs) {
   __shared__ int s_count[kGroupTile / kWave];
+  const GroupJob &job = jobs.job[blockIdx.z];
+  const int *__restrict__ dense = job.dense;
+  int *__restrict__ tile_counts = job.tile_counts;
+  const GroupOffsets &tab = job.tab;
+  const long long num_targets = job.num_targets;
+  const int tiles = job.tiles;
+  if (static_cast<int>(blockIdx.x) >= tiles) return;
   const int slot = blockIdx.y;                                   // axis * 9 + group
   const long long t = static_cast<long long>(blockIdx.x) * kGroupTile + threadIdx.x;
   int row[3];
@@ -1096,8 +1116,10 @@ __global__ __launch_bounds__(kGroupTile) void group_count_kernel(const int *__re
   }
 }
 
-__global__ __launch_bounds__(1024) void group_scan_kernel(int *__restrict__ tile_counts, int tiles,
-                                                           int *__restrict__ head) {
+__global__ __launch_bounds__(1024) void group_scan_kernel(GroupJobs jobs) {
+  int *__restrict__ tile_counts = jobs.job[blockIdx.x].tile_counts;
+  int *__restrict__ head = jobs.job[blockIdx.x].head;
+  const int tiles = jobs.job[blockIdx.x].tiles;
   constexpr int kWaves = 1024 / kWave;
   constexpr int kBatch = 8;                          // loads a lane keeps in flight
   __shared__ int s_part[3][kWaves];
@@ -1157,13 +1179,18 @@ __global__ __launch_bounds__(1024) void group_scan_kernel(int *__restrict__ tile
   if (lane == 0) head[1 + wave] = carry;
 }
 
-__global__ __launch_bounds__(kGroupTile) void group_emit_kernel(const int *__restrict__ dense,
-                                                                 long long num_targets, GroupOffsets tab,
-                                                                 int tiles, const int *__restrict__ tile_counts,
-                                                                 const int *__restrict__ head,
-                                                                 int *__restrict__ rank_out,
-                                                                 int4 *__restrict__ src_out) {
+__global__ __launch_bounds__(kGroupTile) void group_emit_kernel(GroupJobs jobs) {
   __shared__ int s_count[kGroupTile / kWave];
+  const GroupJob &job = jobs.job[blockIdx.z];
+  const int *__restrict__ dense = job.dense;
+  const int *__restrict__ tile_counts = job.tile_counts;
+  const int *__restrict__ head = job.head;
+  int *__restrict__ rank_out = job.rank;
+  int4 *__restrict__ src_out = job.src;
+  const GroupOffsets &tab = job.tab;
+  const long long num_targets = job.num_targets;
+  const int tiles = job.tiles;
+  if (static_cast<int>(blockIdx.x) >= tiles) return;
   const int axis = head[0];
   const int group = blockIdx.y;
   const int slot = axis * kGroupCount + group;
@@ -1181,6 +1208,34 @@ __global__ __launch_bounds__(kGroupTile) void group_emit_kernel(const int *__res
   if (t < num_targets) {
     rank_out[static_cast<long long>(group) * num_targets + t] = any ? rank : -1;
     if (any) src_out[static_cast<long long>(group) * num_targets + rank] = make_int4(row[0], row[1], row[2], 0);
+  }
+}
+
+void enqueue_offset_groups(const std::vector<GroupWork> &work, Scope &scope, hipStream_t stream) {
+  for (size_t from = 0; from < work.size(); from += kGroupMaps) {
+    GroupJobs jobs;
+    std::memset(&jobs, 0, sizeof(jobs));
+    const unsigned count = static_cast<unsigned>(std::min<size_t>(kGroupMaps, work.size() - from));
+    int most_tiles = 1;
+    for (unsigned i = 0; i < count; ++i) {
+      const GroupWork &w = work[from + i];
+      GroupJob &job = jobs.job[i];
+      job.dense = w.kernel_map;
+      job.num_targets = w.num_targets;
+      job.tiles = static_cast<int>(std::max<int64_t>(1, div_ceil(w.num_targets, kGroupTile)));
+      job.tile_counts = scope.alloc<int>(static_cast<size_t>(3) * kGroupCount * job.tiles);
+      job.head = w.head;
+      job.rank = w.rank;
+      job.src = reinterpret_cast<int4 *>(w.src);
+      for (int k = 0; k < 3 * kGroupCount * kGroupMembers; ++k) job.tab.o[k] = w.offsets_host[k];
+      most_tiles = std::max(most_tiles, job.tiles);
+    }
+    group_count_kernel<<<dim3(most_tiles, 3 * kGroupCount, count), kGroupTile, 0, stream>>>(jobs);
+    check_launch("group_count_kernel");
+    group_scan_kernel<<<count, 1024, 0, stream>>>(jobs);
+    check_launch("group_scan_kernel");
+    group_emit_kernel<<<dim3(most_tiles, kGroupCount, count), kGroupTile, 0, stream>>>(jobs);
+    check_launch("group_emit_kernel");
   }
 }
 
@@ -2003,19 +2058,9 @@ extern "C" int mnt_kernel_map_offset_groups(const int32_t *kernel_map, int64_t T
     MNT_CHECK(head_out != nullptr, "head_out is null");
     MNT_CHECK(reinterpret_cast<uintptr_t>(src_out) % 16 == 0, "src_out is not 16-byte aligned");
     Scope scope(stream);
-    GroupOffsets tab;
-    for (int i = 0; i < 3 * kGroupCount * kGroupMembers; ++i) tab.o[i] = group_offsets_host[i];
-    const int tiles = static_cast<int>(std::max<int64_t>(1, div_ceil(T, kGroupTile)));
-    int *tile_counts = scope.alloc<int>(static_cast<size_t>(3) * kGroupCount * tiles);
     if (T > 0) MNT_CHECK(kernel_map != nullptr && rank_out != nullptr && src_out != nullptr, "null argument");
-    group_count_kernel<<<dim3(tiles, 3 * kGroupCount), kGroupTile, 0, stream>>>(kernel_map, T, tab, tiles,
-                                                                                 tile_counts);
-    check_launch("group_count_kernel");
-    group_scan_kernel<<<1, 1024, 0, stream>>>(tile_counts, tiles, head_out);
-    check_launch("group_scan_kernel");
-    group_emit_kernel<<<dim3(tiles, kGroupCount), kGroupTile, 0, stream>>>(
-        kernel_map, T, tab, tiles, tile_counts, head_out, rank_out, reinterpret_cast<int4 *>(src_out));
-    check_launch("group_emit_kernel");
+    enqueue_offset_groups({{kernel_map, static_cast<int>(T), group_offsets_host, rank_out, src_out, head_out}}, scope,
+                          stream);
     profile_mark("offset_groups", stream);
   });
 }

@@ -1,0 +1,709 @@
+// The host side of a layer call, as a Python extension module.
+//
+// A layer of a network is one or two kernel launches of 5 to 30 us, and a
+// launch costs the host about 3 us.  Written in Python, everything around
+// them (checks, cache lookups, the output tensor, a ctypes call of 17 to 29
+// arguments) took 15 to 25 us more per layer, which left the GPU waiting in
+// every network but the largest.  This module does the same work in about
+// 2 us: a Layer holds what depends on the module alone (weights, their packed
+// copy, widths, tunables), a MapEntry what depends on the kernel map, and
+// Layer.run checks that both still describe the call at hand.  Whatever is
+// not exactly as it was when the two were made sends the caller (None is
+// returned) through the Python code that makes them.
+#include <Python.h>
+
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <ATen/ATen.h>
+#include <ATen/hip/EmptyTensor.h>
+#include <c10/core/GradMode.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+
+#include <cstdint>
+
+namespace {
+
+// ------------------------------------------------------- the library's calls ----
+
+using ImplicitFn = int (*)(const void *, const void *, const int32_t *, int64_t, int64_t, int64_t, int64_t, int64_t,
+                           int, const float *, const float *, const void *, int, float, const void *, void *, void *);
+using GroupsFn = int (*)(const void *, const void *, const int32_t *, const int32_t *, const int32_t *,
+                         const int32_t *, int64_t, int64_t, int64_t, int64_t, int, const float *, const float *,
+                         const void *, int, float, void *, void *);
+using TablesFn = int (*)(int64_t, int64_t, int, int64_t, int, double, const void *, const void *, const void *,
+                         const void *, const void *, const void *, const int64_t *, int64_t, int64_t, int64_t,
+                         int64_t, int64_t, int, int, const int32_t *, const float *, const float *, const void *,
+                         int, float, const void *, const int64_t *, void *, void *);
+using ErrorFn = const char *(*)();
+
+ImplicitFn g_implicit = nullptr;
+GroupsFn g_groups = nullptr;
+TablesFn g_tables = nullptr;
+ErrorFn g_error = nullptr;
+
+// ------------------------------------------------------------ Python objects ----
+
+// What the Python side hands over once (bind): classes and modules' dicts.
+PyTypeObject *g_sparse_tensor = nullptr;          // minuet_amd.SparseTensor
+PyObject *g_conv_types = nullptr;                 // tuple of the exact convolution classes
+PyObject *g_norm_types = nullptr;                 // tuple of the exact BatchNorm classes
+PyObject *g_activations = nullptr;                // dict: exact activation class -> activation code
+PyObject *g_global_hooks = nullptr;               // tuple of torch's global module hook dicts
+PyObject *g_conv_namespace = nullptr;             // dict of minuet_amd.nn.convolutions.SparseConv at bind time
+PyObject *g_forward = nullptr;                    // SparseConv.forward at bind time
+PyObject *g_no_arguments = nullptr;               // an empty tuple
+
+#define MNT_NAMES(X)                                                                                        \
+  X(_features) X(_coordinates) X(_stride) X(_batch_dims) X(_parameters) X(_buffers) X(kernel) X(bias)        \
+  X(_kernel_map_cache) X(_tunable_config) X(_tuning_data) X(stride) X(dilation) X(kernel_size) X(_fast)      \
+  X(_fast_maps) X(dataflow) X(threshold) X(gather_tile_size) X(scatter_tile_size) X(scale) X(shift)          \
+  X(residual) X(activation) X(negative_slope) X(_forward_hooks) X(_forward_pre_hooks) X(_backward_hooks)     \
+  X(_backward_pre_hooks) X(_compiled_call_impl) X(forward) X(training) X(weight) X(running_mean)             \
+  X(running_var) X(eps) X(_minuet_affine) X(_identity_map) X(relu) X(leaky_relu) X(relu6)
+#define MNT_DECLARE(name) PyObject *s_##name = nullptr;
+MNT_NAMES(MNT_DECLARE)
+#undef MNT_DECLARE
+
+// The instance dictionary of an object (borrowed), or null.
+inline PyObject *dict_of(PyObject *object) {
+  PyObject **at = _PyObject_GetDictPtr(object);
+  return at == nullptr ? nullptr : *at;
+}
+
+// Borrowed lookup; null when the key is missing (no exception set).
+inline PyObject *look(PyObject *dict, PyObject *key) { return PyDict_GetItem(dict, key); }
+
+inline bool is_none(PyObject *o) { return o == nullptr || o == Py_None; }
+
+inline const at::Tensor *tensor_of(PyObject *o) {
+  return o != nullptr && THPVariable_Check(o) ? &THPVariable_Unpack(o) : nullptr;
+}
+
+inline int64_t version_of(const at::Tensor &t) {
+  return t.is_inference() ? -1 : static_cast<int64_t>(t.unsafeGetTensorImpl()->version_counter().current_version());
+}
+
+// A tensor that derived data was made from: unchanged while the object under
+// its name is the same one, with the same storage and version counter.
+struct Watched {
+  PyObject *object = nullptr;      // owned
+  const void *data = nullptr;
+  int64_t version = 0;
+
+  void set(PyObject *o) {
+    Py_XINCREF(o);
+    Py_XDECREF(object);
+    object = o;
+    if (const at::Tensor *t = tensor_of(o)) {
+      data = t->const_data_ptr();
+      version = version_of(*t);
+    }
+  }
+  bool same(PyObject *o) const {
+    if (o != object) return false;
+    const at::Tensor *t = tensor_of(o);
+    return t == nullptr || (t->const_data_ptr() == data && version_of(*t) == version);
+  }
+  void clear() { Py_CLEAR(object); }
+};
+
+// --------------------------------------------------------------- MapEntry ----
+
+enum Kind { kImplicit = 0, kGroups = 1, kTables = 2, kPointwise = 3 };
+
+// One kernel map as one kind of layer reads it: the coordinates its output
+// carries and the device addresses of its tables (`keep` holds their owners).
+struct MapEntry {
+  PyObject_HEAD
+  PyObject *coordinates, *stride, *batch_dims, *keep;
+  int kind;
+  int device;
+  int index_code;
+  int64_t num_sources, num_targets;
+  const void *at[8];       // kind's own pointers, in the order of the entry point's arguments
+  // Of a map built ahead of the layer that asks for it: the source coordinates
+  // it was built from (null: the cache serves it to whoever asks), and whether
+  // any layer has used it.
+  const void *built_from;
+  char used;
+};
+
+void map_entry_dealloc(PyObject *self) {
+  MapEntry *e = reinterpret_cast<MapEntry *>(self);
+  Py_XDECREF(e->coordinates);
+  Py_XDECREF(e->stride);
+  Py_XDECREF(e->batch_dims);
+  Py_XDECREF(e->keep);
+  Py_TYPE(self)->tp_free(self);
+}
+
+PyObject *map_entry_new(PyTypeObject *type, PyObject *args, PyObject *) {
+  PyObject *coordinates, *stride, *batch_dims, *keep, *pointers;
+  int kind, device, index_code;
+  long long num_sources, num_targets;
+  unsigned long long built_from = 0;
+  if (!PyArg_ParseTuple(args, "iOOOOiiLLO!|K", &kind, &coordinates, &stride, &batch_dims, &keep, &device, &index_code,
+                        &num_sources, &num_targets, &PyTuple_Type, &pointers, &built_from)) {
+    return nullptr;
+  }
+  MapEntry *e = reinterpret_cast<MapEntry *>(type->tp_alloc(type, 0));
+  if (e == nullptr) return nullptr;
+  auto hold = [](PyObject *o) {
+    Py_INCREF(o);
+    return o;
+  };
+  e->coordinates = hold(coordinates);
+  e->stride = hold(stride);
+  e->batch_dims = hold(batch_dims);
+  e->keep = hold(keep);
+  e->kind = kind;
+  e->device = device;
+  e->index_code = index_code;
+  e->num_sources = num_sources;
+  e->num_targets = num_targets;
+  e->built_from = reinterpret_cast<const void *>(static_cast<uintptr_t>(built_from));
+  e->used = 0;
+  for (Py_ssize_t i = 0; i < 8; ++i) {
+    e->at[i] = nullptr;
+    if (i < PyTuple_GET_SIZE(pointers) && !is_none(PyTuple_GET_ITEM(pointers, i))) {
+      e->at[i] = PyLong_AsVoidPtr(PyTuple_GET_ITEM(pointers, i));
+    }
+  }
+  if (PyErr_Occurred()) {
+    Py_DECREF(e);
+    return nullptr;
+  }
+  return reinterpret_cast<PyObject *>(e);
+}
+
+PyObject *map_entry_used(PyObject *self, void *) {
+  return PyBool_FromLong(reinterpret_cast<MapEntry *>(self)->used);
+}
+
+PyGetSetDef map_entry_getset[] = {{"used", map_entry_used, nullptr, "Whether a layer has run with this map.", nullptr},
+                                  {nullptr, nullptr, nullptr, nullptr, nullptr}};
+
+PyTypeObject MapEntryType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+// ------------------------------------------------------------------ Layer ----
+
+// A convolution module as it was when its last call went through the Python code.
+struct Layer {
+  PyObject_HEAD
+  Watched kernel, bias;
+  PyObject *weights, *packed;                 // what is multiplied by (padded where rows are), its packed copy
+  PyObject *stride, *dilation, *kernel_size;  // the module's settings, by identity
+  PyObject *shape_id;                         // key of this layer's map inside the cache's _fast_maps
+  PyObject *dataflow, *threshold, *gather_tile, *scatter_tile;
+  PyObject *bias_shift;                       // fp32 copy of the bias, or None
+  int kind, float_code, device;
+  int shortcut, has_threshold;
+  double threshold_value;
+  int64_t gather_tile_value, scatter_tile_value;
+  int64_t num_offsets, in_channels, out_channels;
+  int64_t item_size;
+};
+
+void layer_dealloc(PyObject *self) {
+  Layer *l = reinterpret_cast<Layer *>(self);
+  l->kernel.clear();
+  l->bias.clear();
+  for (PyObject **o : {&l->weights, &l->packed, &l->stride, &l->dilation, &l->kernel_size, &l->shape_id,
+                       &l->dataflow, &l->threshold, &l->gather_tile, &l->scatter_tile, &l->bias_shift}) {
+    Py_CLEAR(*o);
+  }
+  Py_TYPE(self)->tp_free(self);
+}
+
+// Layer(module, kind, weights, packed, shape_id, shortcut, bias_shift)
+PyObject *layer_new(PyTypeObject *type, PyObject *args, PyObject *) {
+  PyObject *module, *weights, *packed, *shape_id, *bias_shift;
+  int kind, shortcut;
+  if (!PyArg_ParseTuple(args, "OiOOOiO", &module, &kind, &weights, &packed, &shape_id, &shortcut, &bias_shift)) {
+    return nullptr;
+  }
+  PyObject *d = dict_of(module);
+  const at::Tensor *w = tensor_of(weights);
+  PyObject *parameters = d == nullptr ? nullptr : look(d, s__parameters);
+  PyObject *config = d == nullptr ? nullptr : look(d, s__tunable_config);
+  if (parameters == nullptr || config == nullptr || w == nullptr || w->dim() != 3 || tensor_of(packed) == nullptr ||
+      !w->is_contiguous()) {
+    PyErr_SetString(PyExc_ValueError, "Layer needs a convolution module, its weights and their packed copy");
+    return nullptr;
+  }
+  Layer *l = reinterpret_cast<Layer *>(type->tp_alloc(type, 0));
+  if (l == nullptr) return nullptr;
+  new (&l->kernel) Watched();
+  new (&l->bias) Watched();
+  l->kernel.set(look(parameters, s_kernel));
+  l->bias.set(look(parameters, s_bias));
+  auto hold = [](PyObject *o) {
+    o = o == nullptr ? Py_None : o;
+    Py_INCREF(o);
+    return o;
+  };
+  l->weights = hold(weights);
+  l->packed = hold(packed);
+  l->stride = hold(look(d, s_stride));
+  l->dilation = hold(look(d, s_dilation));
+  l->kernel_size = hold(look(d, s_kernel_size));
+  l->shape_id = hold(shape_id);
+  l->dataflow = hold(look(config, s_dataflow));
+  l->threshold = hold(look(config, s_threshold));
+  l->gather_tile = hold(look(config, s_gather_tile_size));
+  l->scatter_tile = hold(look(config, s_scatter_tile_size));
+  l->bias_shift = hold(bias_shift);
+  l->kind = kind;
+  l->shortcut = shortcut;
+  l->device = w->device().index();
+  l->float_code = w->scalar_type() == at::kFloat ? 0 : w->scalar_type() == at::kHalf ? 1 : 2;
+  l->item_size = static_cast<int64_t>(w->element_size());
+  l->num_offsets = w->size(0);
+  l->in_channels = w->size(1);
+  l->out_channels = w->size(2);
+  l->has_threshold = l->threshold == Py_None ? 0 : 1;
+  l->threshold_value = l->has_threshold ? PyFloat_AsDouble(l->threshold) : 0.0;
+  l->gather_tile_value = l->gather_tile == Py_None ? 0 : PyLong_AsLongLong(l->gather_tile);
+  l->scatter_tile_value = l->scatter_tile == Py_None ? 0 : PyLong_AsLongLong(l->scatter_tile);
+  if (PyErr_Occurred()) {
+    Py_DECREF(l);
+    return nullptr;
+  }
+  return reinterpret_cast<PyObject *>(l);
+}
+
+PyTypeObject LayerType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+// ------------------------------------------------------------------- runs ----
+
+struct EpilogueArgs {
+  PyObject *scale = nullptr, *shift = nullptr, *residual = nullptr;
+  int activation = 0;
+  float slope = 0.0f;
+};
+
+// fp32 [channels] on `device`, contiguous: the form the kernels read.
+inline bool vector_fits(const at::Tensor *t, int64_t channels, int device) {
+  return t->scalar_type() == at::kFloat && t->dim() == 1 && t->size(0) == channels && t->is_contiguous() &&
+         t->is_cuda() && t->device().index() == device;
+}
+
+PyObject *none() { Py_RETURN_NONE; }
+
+// The layer on `inputs`; None when anything is not as the Layer describes it.
+PyObject *run_layer(Layer *l, PyObject *module_dict, PyObject *inputs, const EpilogueArgs &ep) {
+  // the module: same parameters, same settings, not being tuned
+  PyObject *parameters = look(module_dict, s__parameters);
+  PyObject *config = look(module_dict, s__tunable_config);
+  if (parameters == nullptr || config == nullptr || !l->kernel.same(look(parameters, s_kernel)) ||
+      !l->bias.same(look(parameters, s_bias)) || look(module_dict, s_stride) != l->stride ||
+      look(module_dict, s_dilation) != l->dilation || look(module_dict, s_kernel_size) != l->kernel_size ||
+      look(config, s_dataflow) != l->dataflow || look(config, s_threshold) != l->threshold ||
+      look(config, s_gather_tile_size) != l->gather_tile || look(config, s_scatter_tile_size) != l->scatter_tile ||
+      !is_none(look(module_dict, s__tuning_data))) {
+    return none();
+  }
+  const at::Tensor &kernel = THPVariable_Unpack(l->kernel.object);
+  if (c10::GradMode::is_enabled()) {
+    const at::Tensor *b = tensor_of(l->bias.object);
+    if (kernel.requires_grad() || (b != nullptr && b->requires_grad())) return none();
+  }
+  // the input
+  if (Py_TYPE(inputs) != g_sparse_tensor) return none();
+  PyObject *in = dict_of(inputs);
+  if (in == nullptr) return none();
+  const at::Tensor *x = tensor_of(look(in, s__features));
+  PyObject *coordinates = look(in, s__coordinates), *stride = look(in, s__stride);
+  PyObject *batch_dims = look(in, s__batch_dims);
+  if (x == nullptr || coordinates == nullptr || stride == nullptr || batch_dims == nullptr) return none();
+  if (x->dim() != 2 || x->size(1) != l->in_channels || x->scalar_type() != kernel.scalar_type() || !x->is_cuda() ||
+      x->device().index() != l->device || !x->is_contiguous() || (c10::GradMode::is_enabled() && x->requires_grad())) {
+    return none();
+  }
+  const void *source = x->const_data_ptr();
+  if (reinterpret_cast<uintptr_t>(source) % 16 != 0 || c10::hip::current_device() != l->device) return none();
+  // its kernel map
+  PyObject *out_coordinates = coordinates, *out_stride = stride, *out_batch_dims = batch_dims;
+  const int64_t S = x->size(0);
+  int64_t T = S;
+  MapEntry *map = nullptr;
+  const at::Tensor *identity = nullptr;
+  if (l->kind == kPointwise) {
+    // 1 x 1 x 1: every row is its own source
+    identity = tensor_of(look(module_dict, s__identity_map));
+    if (identity == nullptr || identity->dim() != 2 || identity->size(1) < S || identity->device() != x->device()) {
+      return none();
+    }
+    if (batch_dims != Py_None) {
+      const at::Tensor *dims = tensor_of(batch_dims);
+      if (dims == nullptr || dims->dim() != 1 || dims->size(0) <= 2) return none();
+    }
+  } else {
+    PyObject *cache = look(module_dict, s__kernel_map_cache);
+    PyObject *cache_dict = is_none(cache) ? nullptr : dict_of(cache);
+    PyObject *maps = cache_dict == nullptr ? nullptr : look(cache_dict, s__fast_maps);
+    PyObject *by_stride = maps == nullptr ? nullptr : look(maps, l->shape_id);
+    PyObject *found = by_stride == nullptr ? nullptr : look(by_stride, stride);
+    if (found == nullptr || Py_TYPE(found) != &MapEntryType) return none();
+    map = reinterpret_cast<MapEntry *>(found);
+    if (map->kind != l->kind || map->num_sources != S || map->device != l->device) return none();
+    if (map->built_from != nullptr) {
+      const at::Tensor *rows = tensor_of(coordinates);
+      if (rows == nullptr || rows->const_data_ptr() != map->built_from) return none();
+    }
+    map->used = 1;
+    T = map->num_targets;
+    out_coordinates = map->coordinates;
+    out_stride = map->stride;
+    out_batch_dims = map->batch_dims;
+  }
+  // the epilogue; a bias is one more per-channel shift where there is none yet
+  const at::Tensor *scale = nullptr, *shift = nullptr, *residual = nullptr;
+  if (!is_none(ep.scale)) {
+    scale = tensor_of(ep.scale);
+    if (scale == nullptr || !vector_fits(scale, l->out_channels, l->device)) return none();
+  }
+  PyObject *shift_object = ep.shift;
+  if (!is_none(l->bias.object)) {
+    if (!is_none(ep.scale) || !is_none(ep.shift)) return none();
+    shift_object = l->bias_shift;
+    if (is_none(shift_object)) return none();
+  }
+  if (!is_none(shift_object)) {
+    shift = tensor_of(shift_object);
+    if (shift == nullptr || !vector_fits(shift, l->out_channels, l->device)) return none();
+  }
+  if (!is_none(ep.residual)) {
+    residual = tensor_of(ep.residual);
+    if (residual == nullptr || residual->scalar_type() != kernel.scalar_type() || residual->dim() != 2 ||
+        residual->size(0) != T || residual->size(1) != l->out_channels || !residual->is_contiguous() ||
+        !residual->is_cuda() || residual->device().index() != l->device ||
+        reinterpret_cast<uintptr_t>(residual->const_data_ptr()) % 16 != 0) {
+      return none();
+    }
+  }
+  at::Tensor out = at::detail::empty_cuda({T, l->out_channels}, kernel.scalar_type(), kernel.device(), std::nullopt);
+  void *stream = c10::hip::getCurrentHIPStream(l->device).stream();
+  auto data = [](const at::Tensor *t) -> const void * { return t == nullptr ? nullptr : t->const_data_ptr(); };
+  const float *scale_at = static_cast<const float *>(data(scale));
+  const float *shift_at = static_cast<const float *>(data(shift));
+  const void *weights_at = THPVariable_Unpack(l->weights).const_data_ptr();
+  const void *packed_at = THPVariable_Unpack(l->packed).const_data_ptr();
+  int status = 0;
+  switch (l->kind) {
+    case kImplicit:
+      status = g_implicit(source, weights_at, static_cast<const int32_t *>(map->at[0]), S, T, l->num_offsets,
+                          l->in_channels, l->out_channels, l->float_code, scale_at, shift_at, data(residual),
+                          ep.activation, ep.slope, packed_at, out.mutable_data_ptr(), stream);
+      break;
+    case kGroups:
+      status = g_groups(source, packed_at, static_cast<const int32_t *>(map->at[0]),
+                        static_cast<const int32_t *>(map->at[1]), static_cast<const int32_t *>(map->at[2]),
+                        static_cast<const int32_t *>(map->at[3]), S, T, l->in_channels, l->out_channels,
+                        l->float_code, scale_at, shift_at, data(residual), ep.activation, ep.slope,
+                        out.mutable_data_ptr(), stream);
+      break;
+    case kTables:
+      // source_masks, target_masks, order, sizes, sizes on the host, order on the host, pair list
+      status = g_tables(l->gather_tile_value, l->scatter_tile_value, l->shortcut, 4, l->has_threshold,
+                        l->threshold_value, source, weights_at, map->at[0], map->at[1], map->at[2], map->at[3],
+                        static_cast<const int64_t *>(map->at[4]), S, T, l->num_offsets, l->in_channels,
+                        l->out_channels, map->index_code, l->float_code, static_cast<const int32_t *>(map->at[6]),
+                        scale_at, shift_at, data(residual), ep.activation, ep.slope, packed_at,
+                        static_cast<const int64_t *>(map->at[5]), out.mutable_data_ptr(), stream);
+      break;
+    default:
+      status = g_implicit(source, weights_at, static_cast<const int32_t *>(identity->const_data_ptr()), S, T, 1,
+                          l->in_channels, l->out_channels, l->float_code, scale_at, shift_at, data(residual),
+                          ep.activation, ep.slope, packed_at, out.mutable_data_ptr(), stream);
+      break;
+  }
+  if (status != 0) {
+    PyErr_SetString(PyExc_RuntimeError, g_error());
+    return nullptr;
+  }
+  // the result: a SparseTensor like the ones SparseTensor.like makes
+  PyObject *result = g_sparse_tensor->tp_new(g_sparse_tensor, g_no_arguments, nullptr);
+  if (result == nullptr) return nullptr;
+  PyObject *features = THPVariable_Wrap(std::move(out));
+  const bool ok = features != nullptr && PyObject_SetAttr(result, s__features, features) == 0 &&
+                  PyObject_SetAttr(result, s__coordinates, out_coordinates) == 0 &&
+                  PyObject_SetAttr(result, s__stride, out_stride) == 0 &&
+                  PyObject_SetAttr(result, s__batch_dims, out_batch_dims) == 0;
+  Py_XDECREF(features);
+  if (!ok) {
+    Py_DECREF(result);
+    return nullptr;
+  }
+  return result;
+}
+
+// The Layer a module keeps, or null.
+Layer *layer_of(PyObject *module_dict) {
+  PyObject *fast = look(module_dict, s__fast);
+  return fast != nullptr && Py_TYPE(fast) == &LayerType ? reinterpret_cast<Layer *>(fast) : nullptr;
+}
+
+int activation_code(PyObject *name) {
+  if (is_none(name)) return 0;
+  if (name == s_relu) return 1;
+  if (name == s_leaky_relu) return 2;
+  if (name == s_relu6) return 3;
+  if (!PyUnicode_Check(name)) return -1;
+  if (PyUnicode_Compare(name, s_relu) == 0) return 1;
+  if (PyUnicode_Compare(name, s_leaky_relu) == 0) return 2;
+  if (PyUnicode_Compare(name, s_relu6) == 0) return 3;
+  return -1;
+}
+
+// run(module, inputs, epilogue): the module's forward, or None.
+PyObject *py_run(PyObject *, PyObject *const *args, Py_ssize_t count) {
+  if (count != 3) {
+    PyErr_SetString(PyExc_TypeError, "run(module, inputs, epilogue)");
+    return nullptr;
+  }
+  PyObject *d = dict_of(args[0]);
+  Layer *l = d == nullptr ? nullptr : layer_of(d);
+  if (l == nullptr) return none();
+  EpilogueArgs ep;
+  PyObject *held[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
+  if (args[2] != Py_None) {
+    PyObject *names[5] = {s_scale, s_shift, s_residual, s_activation, s_negative_slope};
+    for (int i = 0; i < 5; ++i) {
+      held[i] = PyObject_GetAttr(args[2], names[i]);
+      if (held[i] == nullptr) {
+        for (PyObject *h : held) Py_XDECREF(h);
+        return nullptr;
+      }
+    }
+    ep.scale = held[0];
+    ep.shift = held[1];
+    ep.residual = held[2];
+    ep.activation = activation_code(held[3]);
+    ep.slope = static_cast<float>(PyFloat_AsDouble(held[4]));
+  }
+  PyObject *result = nullptr;
+  if (!PyErr_Occurred()) {
+    Py_INCREF(l);
+    result = ep.activation < 0 ? none() : run_layer(l, d, args[1], ep);
+    Py_DECREF(l);
+  }
+  for (PyObject *h : held) Py_XDECREF(h);
+  return result;
+}
+
+// ----------------------------------------------------------------- Affine ----
+
+// scale and shift of a BatchNorm in evaluation mode, and the tensors they were made from.
+struct Affine {
+  PyObject_HEAD
+  Watched mean, var, weight, bias;
+  PyObject *eps;
+  PyObject *scale, *shift;
+};
+
+void affine_dealloc(PyObject *self) {
+  Affine *a = reinterpret_cast<Affine *>(self);
+  for (Watched *w : {&a->mean, &a->var, &a->weight, &a->bias}) w->clear();
+  Py_CLEAR(a->eps);
+  Py_CLEAR(a->scale);
+  Py_CLEAR(a->shift);
+  Py_TYPE(self)->tp_free(self);
+}
+
+// Affine(norm, scale, shift)
+PyObject *affine_new(PyTypeObject *type, PyObject *args, PyObject *) {
+  PyObject *norm, *scale, *shift;
+  if (!PyArg_ParseTuple(args, "OOO", &norm, &scale, &shift)) return nullptr;
+  PyObject *d = dict_of(norm);
+  PyObject *buffers = d == nullptr ? nullptr : look(d, s__buffers);
+  PyObject *parameters = d == nullptr ? nullptr : look(d, s__parameters);
+  if (buffers == nullptr || parameters == nullptr) {
+    PyErr_SetString(PyExc_ValueError, "Affine needs a module with buffers and parameters");
+    return nullptr;
+  }
+  Affine *a = reinterpret_cast<Affine *>(type->tp_alloc(type, 0));
+  if (a == nullptr) return nullptr;
+  for (Watched *w : {&a->mean, &a->var, &a->weight, &a->bias}) new (w) Watched();
+  a->mean.set(look(buffers, s_running_mean));
+  a->var.set(look(buffers, s_running_var));
+  a->weight.set(look(parameters, s_weight));
+  a->bias.set(look(parameters, s_bias));
+  PyObject *eps = look(d, s_eps);
+  a->eps = eps == nullptr ? Py_None : eps;
+  a->scale = scale;
+  a->shift = shift;
+  Py_INCREF(a->eps);
+  Py_INCREF(scale);
+  Py_INCREF(shift);
+  return reinterpret_cast<PyObject *>(a);
+}
+
+PyTypeObject AffineType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+// The valid Affine of a BatchNorm module in evaluation mode, or null.
+Affine *affine_of(PyObject *norm) {
+  PyObject *d = dict_of(norm);
+  if (d == nullptr || look(d, s_training) != Py_False) return nullptr;
+  PyObject *kept = look(d, s__minuet_affine);
+  PyObject *buffers = look(d, s__buffers), *parameters = look(d, s__parameters);
+  if (kept == nullptr || !PyTuple_Check(kept) || buffers == nullptr || parameters == nullptr) return nullptr;
+  PyObject *last = PyTuple_GET_ITEM(kept, PyTuple_GET_SIZE(kept) - 1);
+  if (Py_TYPE(last) != &AffineType) return nullptr;
+  Affine *a = reinterpret_cast<Affine *>(last);
+  return a->mean.same(look(buffers, s_running_mean)) && a->var.same(look(buffers, s_running_var)) &&
+                 a->weight.same(look(parameters, s_weight)) && a->bias.same(look(parameters, s_bias)) &&
+                 look(d, s_eps) == a->eps
+             ? a
+             : nullptr;
+}
+
+inline bool exact_type_in(PyObject *object, PyObject *types) {
+  PyObject *type = reinterpret_cast<PyObject *>(Py_TYPE(object));
+  for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(types); ++i) {
+    if (PyTuple_GET_ITEM(types, i) == type) return true;
+  }
+  return false;
+}
+
+inline bool empty_dict(PyObject *d) { return d == nullptr || (PyDict_Check(d) && PyDict_GET_SIZE(d) == 0); }
+
+// conv_norm_act(conv, norm, act, x, residual): conv -> norm -> (+ residual) ->
+// act as one call of the library, or None.  The module is called around
+// torch's Module.__call__, so it must be one whose call is its forward alone:
+// no hooks on it, none global, nothing overridden.
+PyObject *py_conv_norm_act(PyObject *, PyObject *const *args, Py_ssize_t count) {
+  if (count != 5) {
+    PyErr_SetString(PyExc_TypeError, "conv_norm_act(conv, norm, act, x, residual)");
+    return nullptr;
+  }
+  PyObject *conv = args[0], *norm = args[1], *act = args[2];
+  if (!exact_type_in(conv, g_conv_types)) return none();
+  PyObject *d = dict_of(conv);
+  Layer *l = d == nullptr ? nullptr : layer_of(d);
+  if (l == nullptr) return none();
+  if (!empty_dict(look(d, s__forward_hooks)) || !empty_dict(look(d, s__forward_pre_hooks)) ||
+      !empty_dict(look(d, s__backward_hooks)) || !empty_dict(look(d, s__backward_pre_hooks)) ||
+      !is_none(look(d, s__compiled_call_impl)) || look(d, s_forward) != nullptr ||
+      look(g_conv_namespace, s_forward) != g_forward) {
+    return none();
+  }
+  for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(g_global_hooks); ++i) {
+    if (!empty_dict(PyTuple_GET_ITEM(g_global_hooks, i))) return none();
+  }
+  EpilogueArgs ep;
+  if (norm != Py_None) {
+    if (!exact_type_in(norm, g_norm_types)) return none();
+    Affine *a = affine_of(norm);
+    if (a == nullptr) return none();
+    ep.scale = a->scale;
+    ep.shift = a->shift;
+  }
+  if (act != Py_None) {
+    PyObject *code = look(g_activations, reinterpret_cast<PyObject *>(Py_TYPE(act)));
+    if (code == nullptr) return none();
+    ep.activation = static_cast<int>(PyLong_AsLong(code));
+    if (ep.activation == 2) {
+      PyObject *ad = dict_of(act);
+      PyObject *slope = ad == nullptr ? nullptr : look(ad, s_negative_slope);
+      if (slope == nullptr || !PyFloat_Check(slope)) return none();
+      ep.slope = static_cast<float>(PyFloat_AS_DOUBLE(slope));
+    }
+  }
+  ep.residual = args[4];
+  Py_INCREF(l);
+  PyObject *result = run_layer(l, d, args[3], ep);
+  Py_DECREF(l);
+  return result;
+}
+
+// bind(addresses: dict name -> int, sparse_tensor, conv_types, norm_types, activations, global_hooks)
+PyObject *py_bind(PyObject *, PyObject *args) {
+  PyObject *addresses, *sparse_tensor, *conv_types, *norm_types, *activations, *hooks;
+  if (!PyArg_ParseTuple(args, "O!O!O!O!O!O!", &PyDict_Type, &addresses, &PyType_Type, &sparse_tensor, &PyTuple_Type,
+                        &conv_types, &PyTuple_Type, &norm_types, &PyDict_Type, &activations, &PyTuple_Type, &hooks)) {
+    return nullptr;
+  }
+  auto address = [&](const char *name) -> void * {
+    PyObject *value = PyDict_GetItemString(addresses, name);
+    if (value == nullptr) {
+      PyErr_Format(PyExc_KeyError, "no address for %s", name);
+      return nullptr;
+    }
+    return PyLong_AsVoidPtr(value);
+  };
+  g_implicit = reinterpret_cast<ImplicitFn>(address("mnt_sparse_convolution_forward_implicit"));
+  g_groups = reinterpret_cast<GroupsFn>(address("mnt_sparse_convolution_forward_groups"));
+  g_tables = reinterpret_cast<TablesFn>(address("mnt_sparse_convolution_forward_fused"));
+  g_error = reinterpret_cast<ErrorFn>(address("mnt_last_error"));
+  if (PyErr_Occurred()) return nullptr;
+  g_sparse_tensor = reinterpret_cast<PyTypeObject *>(sparse_tensor);
+  g_conv_types = conv_types;
+  g_norm_types = norm_types;
+  g_activations = activations;
+  g_global_hooks = hooks;
+  for (PyObject *o : {sparse_tensor, conv_types, norm_types, activations, hooks}) Py_INCREF(o);
+  PyTypeObject *base = reinterpret_cast<PyTypeObject *>(PyTuple_GET_ITEM(conv_types, 0));
+  g_conv_namespace = base->tp_dict;
+  g_forward = look(g_conv_namespace, s_forward);
+  Py_XINCREF(g_forward);
+  Py_RETURN_NONE;
+}
+
+// A copied or unpickled module keeps None in the place of these objects and
+// makes its own at its first call.
+PyObject *py_reduce(PyObject *, PyObject *) {
+  return Py_BuildValue("(O())", reinterpret_cast<PyObject *>(Py_TYPE(Py_None)));
+}
+
+PyMethodDef object_methods[] = {{"__reduce__", py_reduce, METH_NOARGS, "Copies as None."},
+                                {nullptr, nullptr, 0, nullptr}};
+
+PyMethodDef methods[] = {
+    {"bind", py_bind, METH_VARARGS, "Takes the library's addresses and the package's classes."},
+    {"run", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_run)), METH_FASTCALL,
+     "run(module, inputs, epilogue) -> SparseTensor, or None where the Python code has to look."},
+    {"conv_norm_act", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_conv_norm_act)), METH_FASTCALL,
+     "conv_norm_act(conv, norm, act, x, residual) -> SparseTensor, or None where the Python code has to look."},
+    {nullptr, nullptr, 0, nullptr}};
+
+PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "minuet_host", "Host side of layer calls.", -1, methods};
+
+bool ready(PyTypeObject &type, const char *name, size_t size, destructor dealloc, newfunc make) {
+  type.tp_name = name;
+  type.tp_basicsize = static_cast<Py_ssize_t>(size);
+  type.tp_flags = Py_TPFLAGS_DEFAULT;
+  type.tp_dealloc = dealloc;
+  type.tp_new = make;
+  type.tp_methods = object_methods;
+  return PyType_Ready(&type) == 0;
+}
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit_minuet_host() {
+#define MNT_INTERN(name) s_##name = PyUnicode_InternFromString(#name);
+  MNT_NAMES(MNT_INTERN)
+#undef MNT_INTERN
+  MapEntryType.tp_getset = map_entry_getset;
+  if (!ready(MapEntryType, "minuet_host.MapEntry", sizeof(MapEntry), map_entry_dealloc, map_entry_new) ||
+      !ready(LayerType, "minuet_host.Layer", sizeof(Layer), layer_dealloc, layer_new) ||
+      !ready(AffineType, "minuet_host.Affine", sizeof(Affine), affine_dealloc, affine_new)) {
+    return nullptr;
+  }
+  g_no_arguments = PyTuple_New(0);
+  PyObject *module = PyModule_Create(&module_def);
+  if (module == nullptr) return nullptr;
+  Py_INCREF(&MapEntryType);
+  Py_INCREF(&LayerType);
+  Py_INCREF(&AffineType);
+  PyModule_AddObject(module, "MapEntry", reinterpret_cast<PyObject *>(&MapEntryType));
+  PyModule_AddObject(module, "Layer", reinterpret_cast<PyObject *>(&LayerType));
+  PyModule_AddObject(module, "Affine", reinterpret_cast<PyObject *>(&AffineType));
+  PyModule_AddIntConstant(module, "IMPLICIT", kImplicit);
+  PyModule_AddIntConstant(module, "GROUPS", kGroups);
+  PyModule_AddIntConstant(module, "TABLES", kTables);
+  PyModule_AddIntConstant(module, "POINTWISE", kPointwise);
+  return module;
+}

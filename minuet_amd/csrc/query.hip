@@ -22,6 +22,7 @@
 #include <mutex>
 
 #include "device_utils.h"
+#include "pass.h"
 #include "query_plan.h"
 #include "sort.h"
 
@@ -398,13 +399,68 @@ struct CarriedTables {
   int v[kCarriedInts];
 };
 
-template <typename CT, typename BT, typename OT, bool kLists>
+// Several maps in one launch (the maps of a network's levels, most of them too
+// small to fill the chip alone): workgroups [first_block, first_block +
+// num_tiles * splits) belong to a job, `splits` of them to each of its tiles.
+// Frame, deltas and tables of a job start at tables[tables_at].
+constexpr int kJobHead = 24;              // ints of a job's frame and deltas before its tables
+struct QueryJob {
+  const void *sources, *targets, *source_batch_dims, *target_batch_dims;
+  int *kernel_map;
+  int num_sources, num_targets, first_block, num_tiles, splits, tables_at, num_groups, num_offsets, dir_rows;
+};
+struct QueryJobs {
+  static constexpr bool kMany = true;
+  int count;
+  QueryJob job[kPassMaps];
+};
+struct OneQuery {
+  static constexpr bool kMany = false;
+};
+
+template <typename CT, typename BT, typename OT, bool kLists, typename Jobs>
 __global__ __launch_bounds__(kQueryThreads) void query_kernel(
     KeyReader<CT, BT> src, KeyReader<CT, BT> tgt, Frame frame, const int *__restrict__ tables,
     CarriedTables carried, int num_groups, int num_offsets, long long delta_min, long long delta_max,
     OT *__restrict__ kernel_map, unsigned *__restrict__ tile_counts, int num_tiles, int dir_rows,
-    HitSink sink, const DevicePlan *__restrict__ device_plan) {
+    HitSink sink, const DevicePlan *__restrict__ device_plan, Jobs jobs) {
   extern __shared__ __align__(16) unsigned s_dynamic[];
+  int block_x = static_cast<int>(blockIdx.x), block_y = static_cast<int>(blockIdx.y), splits = static_cast<int>(gridDim.y);
+  if constexpr (Jobs::kMany) {
+    int j = 0;
+    while (j + 1 < jobs.count && jobs.job[j + 1].first_block <= block_x) ++j;
+    const QueryJob &job = jobs.job[j];
+    src = KeyReader<CT, BT>{static_cast<const CT *>(job.sources), static_cast<const BT *>(job.source_batch_dims),
+                            src.num_batches, job.num_sources};
+    tgt = KeyReader<CT, BT>{static_cast<const CT *>(job.targets), static_cast<const BT *>(job.target_batch_dims),
+                            src.num_batches, job.num_targets};
+    const int *head = tables + job.tables_at;
+    auto wide = [&](int i) {
+      return static_cast<long long>(static_cast<unsigned long long>(static_cast<unsigned>(head[i])) |
+                                    (static_cast<unsigned long long>(static_cast<unsigned>(head[i + 1])) << 32));
+    };
+#pragma unroll
+    for (int k = 0; k < MNT_MAX_NDIM; ++k) {
+      frame.lo[k] = uniform64(wide(2 * k));
+      frame.shift[k] = __builtin_amdgcn_readfirstlane(head[8 + k]);
+      frame.width[k] = __builtin_amdgcn_readfirstlane(head[12 + k]);
+    }
+    frame.batch_shift = __builtin_amdgcn_readfirstlane(head[16]);
+    frame.batch_width = __builtin_amdgcn_readfirstlane(head[17]);
+    frame.total_bits = __builtin_amdgcn_readfirstlane(head[18]);
+    delta_min = uniform64(wide(20));
+    delta_max = uniform64(wide(22));
+    tables = head + kJobHead;
+    num_groups = job.num_groups;
+    num_offsets = job.num_offsets;
+    kernel_map = reinterpret_cast<OT *>(job.kernel_map);
+    num_tiles = job.num_tiles;
+    dir_rows = job.dir_rows;
+    splits = job.splits;
+    block_x -= job.first_block;
+    block_y = block_x / num_tiles;
+    block_x -= block_y * num_tiles;
+  }
   // Only half of the offsets are looked up (a cloud mapped onto itself under
   // offsets that come in pairs d / -d; see DevicePlan): the totals of the other
   // half are kept here as well, and equal rows, which break the symmetry, are
@@ -438,13 +494,13 @@ __global__ __launch_bounds__(kQueryThreads) void query_kernel(
   __shared__ unsigned long long s_wave_first[kQueryThreads / kWave + 1];
   // dynamic LDS: [group table: 4 words each][member table: 2 words each][hit counts]
   // [row directory: dir_rows 16-bit entries]
-  // With gridDim.y > 1 the offset groups are dealt over the y index: every
+  // With several splits the offset groups are dealt over the y index: every
   // workgroup of a tile finds and stages the same window and resolves its
   // share of the groups (a cloud of a few tiles fills the chip that way).
   int my_first_group = 0, my_groups = num_groups;
-  if (gridDim.y > 1) {
-    const int share = (num_groups + static_cast<int>(gridDim.y) - 1) / static_cast<int>(gridDim.y);
-    my_first_group = static_cast<int>(blockIdx.y) * share;
+  if (splits > 1) {
+    const int share = (num_groups + splits - 1) / splits;
+    my_first_group = block_y * share;
     my_groups = min(num_groups, my_first_group + share) - my_first_group;
     if (my_groups <= 0) return;
   }
@@ -461,7 +517,7 @@ __global__ __launch_bounds__(kQueryThreads) void query_kernel(
   const int w = tid >> 6;
   const long long num_sources = src.count;
   const long long num_targets = tgt.count;
-  const long long t0 = static_cast<long long>(blockIdx.x) * kTargetsPerTile;
+  const long long t0 = static_cast<long long>(block_x) * kTargetsPerTile;
   const long long t_end = t0 + kTargetsPerTile < num_targets ? t0 + kTargetsPerTile : num_targets;
 
   if (tables != nullptr) {
@@ -630,20 +686,20 @@ __global__ __launch_bounds__(kQueryThreads) void query_kernel(
     for (int m = s_groups[0].z + tid; m < last_group.z + last_group.w; m += kQueryThreads) {
       const int o = s_members[m].y;
       const unsigned hits = s_counts[o];
-      tile_counts[static_cast<long long>(o) * num_tiles + blockIdx.x] = hits;
+      tile_counts[static_cast<long long>(o) * num_tiles + block_x] = hits;
       if (kLists && hits != 0) {
-        unsigned *totals = sink.row_totals + static_cast<int>(blockIdx.x % sink.total_copies) * sink.total_stride;
+        unsigned *totals = sink.row_totals + (block_x % sink.total_copies) * sink.total_stride;
         atomicAdd(&totals[o], hits);
         if (halves) atomicAdd(&totals[s_mirror[o]], hits);               // the mirror image has the same hits
       }
     }
     // the zero offset: every target of the tile is its own hit
     if (kLists && halves && tid == 0 && s_zero_offset >= 0) {
-      unsigned *totals = sink.row_totals + static_cast<int>(blockIdx.x % sink.total_copies) * sink.total_stride;
+      unsigned *totals = sink.row_totals + (block_x % sink.total_copies) * sink.total_stride;
       atomicAdd(&totals[s_zero_offset], static_cast<unsigned>(t_end - t0));
     }
   }
-  if (kLists && tid == 0) sink.tile_mode[blockIdx.x] = num_chunks == 1 ? 0u : 1u;
+  if (kLists && tid == 0) sink.tile_mode[block_x] = num_chunks == 1 ? 0u : 1u;
 }
 
 // The query for frames too wide for a packed key (more than 63 bits of
@@ -717,7 +773,7 @@ __global__ __launch_bounds__(kQueryBlock) void query_tuples_kernel(
 
 // Hit counts of every (row, tile of 512 targets) of an existing dense map.
 template <typename IT>
-__global__ __launch_bounds__(kQueryBlock) void count_tiles_kernel(
+__device__ __forceinline__ void count_tiles_body(
     const IT *__restrict__ kernel_map, long long num_targets, unsigned *__restrict__ tile_counts,
     int num_tiles) {
   __shared__ unsigned s_sum;
@@ -737,11 +793,17 @@ __global__ __launch_bounds__(kQueryBlock) void count_tiles_kernel(
   if (threadIdx.x == 0) tile_counts[static_cast<long long>(o) * num_tiles + blockIdx.x] = s_sum;
 }
 
+template <typename IT>
+__global__ __launch_bounds__(kQueryBlock) void count_tiles_kernel(
+    const IT *__restrict__ kernel_map, long long num_targets, unsigned *__restrict__ tile_counts,
+    int num_tiles) {
+  count_tiles_body<IT>(kernel_map, num_targets, tile_counts, num_tiles);
+}
+
 // One workgroup per row: exclusive scan of its tile counts in place and the
 // row total.
-__global__ __launch_bounds__(256) void tile_scan_kernel(unsigned *__restrict__ tile_counts,
-                                                        int num_tiles,
-                                                        unsigned *__restrict__ row_sizes) {
+__device__ __forceinline__ void tile_scan_body(unsigned *__restrict__ tile_counts, int num_tiles,
+                                               unsigned *__restrict__ row_sizes) {
   __shared__ unsigned wave_sums[256 / kWave];
   unsigned *row = tile_counts + static_cast<long long>(blockIdx.x) * num_tiles;
   const int t = threadIdx.x;
@@ -772,6 +834,12 @@ __global__ __launch_bounds__(256) void tile_scan_kernel(unsigned *__restrict__ t
     run += v;
   }
   if (t == 0) row_sizes[blockIdx.x] = total;
+}
+
+__global__ __launch_bounds__(256) void tile_scan_kernel(unsigned *__restrict__ tile_counts,
+                                                        int num_tiles,
+                                                        unsigned *__restrict__ row_sizes) {
+  tile_scan_body(tile_counts, num_tiles, row_sizes);
 }
 
 // The row order from the row totals, stable ascending by size (reorder) or
@@ -853,7 +921,7 @@ __global__ __launch_bounds__(256) void fill_kernel(T *__restrict__ data, long lo
 // lists.  `position_of` maps an offset to its output row (null = identity) and
 // `row_base` gives the list position of the first hit of an output row.
 template <typename IT>
-__global__ __launch_bounds__(kQueryBlock) void emit_kernel(
+__device__ __forceinline__ void emit_body(
     const IT *__restrict__ kernel_map, long long num_sources, long long num_targets,
     int num_offsets, const unsigned *__restrict__ tile_bases, int num_tiles,
     const unsigned *__restrict__ position_of, const unsigned *__restrict__ row_base,
@@ -893,6 +961,59 @@ __global__ __launch_bounds__(kQueryBlock) void emit_kernel(
     }
     running += __popcll(votes);
   }
+}
+
+
+template <typename IT>
+__global__ __launch_bounds__(kQueryBlock) void emit_kernel(
+    const IT *__restrict__ kernel_map, long long num_sources, long long num_targets,
+    int num_offsets, const unsigned *__restrict__ tile_bases, int num_tiles,
+    const unsigned *__restrict__ position_of, const unsigned *__restrict__ row_base,
+    IT *__restrict__ source_masks, IT *__restrict__ target_masks, int *__restrict__ in_idx,
+    int *__restrict__ out_idx, const unsigned *__restrict__ plan, int *__restrict__ sizes_out,
+    int *__restrict__ order_out) {
+  emit_body<IT>(kernel_map, num_sources, num_targets, num_offsets, tile_bases, num_tiles, position_of, row_base,
+                source_masks, target_masks, in_idx, out_idx, plan, sizes_out, order_out);
+}
+
+// The four steps from dense maps to rank tables for several maps at once
+// (blockIdx.z, or .y / .x where a step needs fewer dimensions, is the map): a
+// network in the reference's dataflow has one such map per level, and step by
+// step for each of them they were 40 launches of 2 to 6 us.
+struct TableJob {
+  const int *kernel_map;
+  unsigned *tile_counts, *row_sizes, *plan, *plan_host;
+  unsigned long long *flag;
+  int *source_masks, *target_masks, *in_idx, *out_idx, *sizes, *order;
+  int num_sources, num_targets, num_offsets, num_tiles, reorder;
+};
+struct TableJobs {
+  TableJob job[kPassMaps];
+};
+
+__global__ __launch_bounds__(kQueryBlock) void count_tiles_many_kernel(TableJobs jobs) {
+  const TableJob &job = jobs.job[blockIdx.z];
+  if (static_cast<int>(blockIdx.x) >= job.num_tiles || static_cast<int>(blockIdx.y) >= job.num_offsets) return;
+  count_tiles_body<int>(job.kernel_map, job.num_targets, job.tile_counts, job.num_tiles);
+}
+
+__global__ __launch_bounds__(256) void tile_scan_many_kernel(TableJobs jobs) {
+  const TableJob &job = jobs.job[blockIdx.y];
+  if (static_cast<int>(blockIdx.x) >= job.num_offsets) return;
+  tile_scan_body(job.tile_counts, job.num_tiles, job.row_sizes);
+}
+
+__global__ __launch_bounds__(256) void map_plan_many_kernel(TableJobs jobs, unsigned long long sequence) {
+  const TableJob &job = jobs.job[blockIdx.x];
+  plan_from_sizes(job.row_sizes, job.num_offsets, job.reorder, job.plan, job.plan_host, job.flag, sequence);
+}
+
+__global__ __launch_bounds__(kQueryBlock) void emit_many_kernel(TableJobs jobs) {
+  const TableJob &job = jobs.job[blockIdx.z];
+  if (static_cast<int>(blockIdx.x) >= job.num_tiles) return;
+  emit_body<int>(job.kernel_map, job.num_sources, job.num_targets, job.num_offsets, job.tile_counts, job.num_tiles,
+                 job.plan + job.num_offsets, job.plan + 3 * job.num_offsets, job.source_masks, job.target_masks,
+                 job.in_idx, job.out_idx, job.plan, job.sizes, job.order);
 }
 
 
@@ -1409,9 +1530,9 @@ static void launch_query(const QueryArgs &a, const QueryPlan &plan, const int *d
     split = static_cast<int>(div_ceil(plan.num_groups, share));
   }
   const dim3 grid(static_cast<unsigned>(num_tiles), static_cast<unsigned>(split));
-  query_kernel<CT, BT, OT, kLists><<<grid, kQueryThreads, dyn, stream>>>(
+  query_kernel<CT, BT, OT, kLists, OneQuery><<<grid, kQueryThreads, dyn, stream>>>(
       src, tgt, plan.frame, d_tables, carried, plan.num_groups, num_offsets, plan.delta_min,
-      plan.delta_max, kernel_map, tile_counts, num_tiles, dir_rows, sink, nullptr);
+      plan.delta_max, kernel_map, tile_counts, num_tiles, dir_rows, sink, nullptr, OneQuery{});
   check_launch("query_kernel");
 }
 
@@ -1585,6 +1706,155 @@ static void enqueue_emit(const IT *kernel_map, int64_t num_sources, int64_t num_
                                                    source_masks, target_masks, in_idx, out_idx,
                                                    plan, sizes_out, order_out);
   check_launch("emit_kernel");
+}
+
+QueryTables make_query_tables(const long long *source_bounds, const long long *target_bounds,
+                              const int64_t *offsets, int64_t num_offsets, int ndim, int64_t num_batches) {
+  QueryTables t;
+  const QueryPlan plan = make_plan(source_bounds, target_bounds, offsets, num_offsets, ndim, num_batches);
+  t.num_groups = plan.num_groups;
+  t.num_offsets = static_cast<int>(num_offsets);
+  t.groups_in_rows = plan.groups_in_rows;
+  t.last_width = plan.frame.width[ndim - 1];
+  if (!plan.fits) return t;
+  t.ints.assign(kJobHead, 0);
+  auto put = [&](int i, long long v) {
+    t.ints[i] = static_cast<int>(static_cast<unsigned>(static_cast<unsigned long long>(v) & 0xffffffffull));
+    t.ints[i + 1] = static_cast<int>(static_cast<unsigned>(static_cast<unsigned long long>(v) >> 32));
+  };
+  for (int k = 0; k < MNT_MAX_NDIM; ++k) {
+    put(2 * k, plan.frame.lo[k]);
+    t.ints[8 + k] = plan.frame.shift[k];
+    t.ints[12 + k] = plan.frame.width[k];
+  }
+  t.ints[16] = plan.frame.batch_shift;
+  t.ints[17] = plan.frame.batch_width;
+  t.ints[18] = plan.frame.total_bits;
+  put(20, plan.delta_min);
+  put(22, plan.delta_max);
+  t.ints.insert(t.ints.end(), plan.tables.begin(), plan.tables.end());
+  return t;
+}
+
+void enqueue_queries(const std::vector<QueryWork> &work, const std::vector<QueryTables> &plans,
+                     const std::vector<int> &tables_at, const int *tables, int ndim, int coord_dtype,
+                     int batch_dtype, int64_t num_batches, hipStream_t stream) {
+  for (size_t from = 0; from < work.size(); from += kPassMaps) {
+    QueryJobs jobs;
+    memset(&jobs, 0, sizeof(jobs));
+    jobs.count = static_cast<int>(std::min<size_t>(kPassMaps, work.size() - from));
+    // Maps of fewer tiles than compute units share the chip: the tiles of a map
+    // are split over its offset groups as far as the whole launch leaves room.
+    int64_t tiles = 0;
+    for (int i = 0; i < jobs.count; ++i) tiles += div_ceil(work[from + i].num_targets, kTargetsPerTile);
+    int blocks = 0;
+    size_t dyn = 0;
+    for (int i = 0; i < jobs.count; ++i) {
+      const QueryWork &w = work[from + i];
+      const QueryTables &t = plans[w.plan];
+      QueryJob &job = jobs.job[i];
+      job.sources = w.sources;
+      job.targets = w.targets;
+      job.source_batch_dims = w.source_batch_dims;
+      job.target_batch_dims = w.target_batch_dims;
+      job.kernel_map = w.kernel_map;
+      job.num_sources = static_cast<int>(w.num_sources);
+      job.num_targets = static_cast<int>(w.num_targets);
+      job.num_tiles = static_cast<int>(div_ceil(w.num_targets, kTargetsPerTile));
+      job.tables_at = tables_at[w.plan];
+      job.num_groups = t.num_groups;
+      job.num_offsets = t.num_offsets;
+      const size_t table_ints = t.ints.size() - kJobHead;
+      job.dir_rows = t.groups_in_rows && table_ints * sizeof(int) <= 2048 && t.last_width >= 3 ? kDirectoryRows : 0;
+      const int wanted = std::min<int64_t>(t.num_groups, std::max<int64_t>(1, 2 * compute_units() / std::max<int64_t>(1, tiles)));
+      const int share = static_cast<int>(div_ceil(t.num_groups, std::max(1, wanted)));
+      job.splits = static_cast<int>(div_ceil(t.num_groups, std::max(1, share)));
+      job.first_block = blocks;
+      blocks += job.num_tiles * job.splits;
+      dyn = std::max(dyn, sizeof(unsigned) * (table_ints + static_cast<size_t>(t.num_offsets) + 4) +
+                              sizeof(unsigned short) * static_cast<size_t>(job.dir_rows));
+    }
+    if (blocks == 0) continue;
+    Frame frame;
+    memset(&frame, 0, sizeof(frame));
+    frame.ndim = ndim;
+    CarriedTables carried;
+    memset(&carried, 0, sizeof(carried));
+    const HitSink none{nullptr, nullptr, nullptr, nullptr, 0, 0, nullptr, 1, 0};
+#define MNT_QM(CT, BT)                                                                                        \
+  query_kernel<CT, BT, int32_t, false, QueryJobs><<<blocks, kQueryThreads, dyn, stream>>>(                      \
+      KeyReader<CT, BT>{nullptr, nullptr, static_cast<int>(num_batches), 0},                                  \
+      KeyReader<CT, BT>{nullptr, nullptr, static_cast<int>(num_batches), 0}, frame, tables, carried, 0, 0, 0, 0, \
+      nullptr, nullptr, 0, 0, none, nullptr, jobs)
+    const bool c32 = coord_dtype == MNT_INT32;
+    const bool b32 = num_batches <= 1 || batch_dtype == MNT_INT32;
+    if (c32 && b32) MNT_QM(int32_t, int32_t);
+    else if (c32) MNT_QM(int32_t, int64_t);
+    else if (b32) MNT_QM(int64_t, int32_t);
+    else MNT_QM(int64_t, int64_t);
+#undef MNT_QM
+    check_launch("query_kernel");
+  }
+}
+
+void enqueue_tables(std::vector<TableWork> &work, Scope &scope, unsigned long long sequence, hipStream_t stream) {
+  Arena &arena = scope.arena();
+  size_t host_at = Arena::kPlanOffset;
+  for (size_t from = 0; from < work.size(); from += kPassMaps) {
+    TableJobs jobs;
+    memset(&jobs, 0, sizeof(jobs));
+    const unsigned count = static_cast<unsigned>(std::min<size_t>(kPassMaps, work.size() - from));
+    int most_tiles = 1, most_offsets = 1;
+    for (unsigned i = 0; i < count; ++i) {
+      TableWork &w = work[from + i];
+      TableJob &job = jobs.job[i];
+      job.kernel_map = w.kernel_map;
+      job.num_sources = w.num_sources;
+      job.num_targets = w.num_targets;
+      job.num_offsets = w.num_offsets;
+      job.num_tiles = static_cast<int>(div_ceil(w.num_targets, kTargetsPerTile));
+      job.reorder = w.reorder;
+      job.tile_counts = scope.alloc<unsigned>(static_cast<size_t>(w.num_offsets) * job.num_tiles);
+      job.row_sizes = scope.alloc<unsigned>(w.num_offsets);
+      job.plan = scope.alloc<unsigned>(4 * static_cast<size_t>(w.num_offsets) + 1);
+      job.source_masks = w.source_masks;
+      job.target_masks = w.target_masks;
+      job.in_idx = w.in_idx;
+      job.out_idx = w.out_idx;
+      job.sizes = w.sizes;
+      job.order = w.order;
+      // pinned: the map's own flag, then order, positions and sizes
+      const size_t bytes = 8 + sizeof(unsigned) * 3 * static_cast<size_t>(w.num_offsets);
+      MNT_CHECK(host_at + bytes <= Arena::kPinnedBytes, "too many kernel offsets for one batch of tables");
+      w.host_at = static_cast<int>(host_at);
+      char *host = static_cast<char *>(arena.pinned_device()) + host_at;
+      job.flag = reinterpret_cast<unsigned long long *>(host);
+      job.plan_host = reinterpret_cast<unsigned *>(host + 8);
+      host_at = (host_at + bytes + 63) / 64 * 64;
+      most_tiles = std::max(most_tiles, job.num_tiles);
+      most_offsets = std::max(most_offsets, job.num_offsets);
+    }
+    count_tiles_many_kernel<<<dim3(most_tiles, most_offsets, count), kQueryBlock, 0, stream>>>(jobs);
+    check_launch("count_tiles_many_kernel");
+    tile_scan_many_kernel<<<dim3(most_offsets, count), 256, 0, stream>>>(jobs);
+    check_launch("tile_scan_many_kernel");
+    map_plan_many_kernel<<<count, 256, 0, stream>>>(jobs, sequence);
+    check_launch("map_plan_many_kernel");
+    emit_many_kernel<<<dim3(most_tiles, static_cast<unsigned>(div_ceil(most_offsets, kQueryBlock / kWave)), count),
+                       kQueryBlock, 0, stream>>>(jobs);
+    check_launch("emit_many_kernel");
+  }
+}
+
+void collect_tables(const TableWork &work, Arena &arena, unsigned long long sequence, int64_t *sizes_host,
+                    int64_t *order_host) {
+  char *host = static_cast<char *>(arena.pinned()) + work.host_at;
+  arena.wait_word(reinterpret_cast<volatile unsigned long long *>(host), sequence);
+  const unsigned *plan = reinterpret_cast<const unsigned *>(host + 8);
+  for (int j = 0; j < work.num_offsets; ++j) {
+    order_host[j] = plan[j];
+    sizes_host[j] = plan[2 * work.num_offsets + j];
+  }
 }
 
 // persistent-state header of the two-phase kernel-map build
@@ -1979,9 +2249,9 @@ static void launch_query_chain(const CT *sorted, int64_t n, int ndim, int num_of
   // LDS for the largest tables these offsets can make and for the row directory
   const size_t dyn = sizeof(unsigned) * (6 * static_cast<size_t>(num_offsets) + num_offsets + 4) +
                      sizeof(unsigned short) * static_cast<size_t>(kDirectoryRows);
-  query_kernel<CT, int32_t, int32_t, true><<<num_tiles, kQueryThreads, dyn, stream>>>(
+  query_kernel<CT, int32_t, int32_t, true, OneQuery><<<num_tiles, kQueryThreads, dyn, stream>>>(
       rows, rows, frame, nullptr, carried, 0, num_offsets, 0, 0, nullptr, tile_counts, num_tiles,
-      kDirectoryRows, sink, plan);
+      kDirectoryRows, sink, plan, OneQuery{});
   check_launch("query_kernel");
 }
 

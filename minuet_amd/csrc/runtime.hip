@@ -135,7 +135,7 @@ void Arena::free_all(bool synchronise) {
   for (auto &p : pages_) MNT_HIP(hipFree(p.base));
   pages_.clear();
   cursor_ = 0;
-  for (int slot = 0; slot < 2; ++slot) {
+  for (int slot = 0; slot < kPersistentSlots; ++slot) {
     if (persistent_[slot]) {
       MNT_HIP(hipFree(persistent_[slot]));
       persistent_[slot] = nullptr;
@@ -144,6 +144,7 @@ void Arena::free_all(bool synchronise) {
   }
   pending.valid = false;
   map_state_valid = false;
+  pass_pending = false;
   zero_bitmap_words = 0;
 }
 
@@ -211,8 +212,12 @@ unsigned long long *Arena::flag_device(int slot) {
 static std::atomic<long long> g_host_waits{0}, g_host_wait_ns{0};
 
 void Arena::wait_flag(int slot, unsigned long long sequence) {
-  volatile unsigned long long *flag = reinterpret_cast<volatile unsigned long long *>(
-      static_cast<char *>(pinned()) + kFlagOffset + static_cast<size_t>(slot) * 64);
+  wait_word(reinterpret_cast<volatile unsigned long long *>(static_cast<char *>(pinned()) + kFlagOffset +
+                                                            static_cast<size_t>(slot) * 64),
+            sequence);
+}
+
+void Arena::wait_word(volatile unsigned long long *flag, unsigned long long sequence) {
   const auto start = std::chrono::steady_clock::now();
   struct Tally {
     std::chrono::steady_clock::time_point since;

@@ -9,12 +9,9 @@
 
 #include "device_utils.h"
 #include "sort.h"
+#include "target_keys.h"
 
 namespace mnt {
-
-constexpr int kScanBlock = 256;
-constexpr int kScanItems = 8;
-constexpr int kScanTile = kScanBlock * kScanItems;
 
 // Row i closes a run: it is the last row, differs from row i+1, or a batch
 // ends right after it.
@@ -28,28 +25,6 @@ __device__ __forceinline__ bool row_ends_run(const CT *__restrict__ coords, long
   if (!same) return true;
   if (batch_dims != nullptr) return is_batch_end<IT>(i + 1, batch_dims, num_batches);
   return false;
-}
-
-// Exclusive scan of `flag` over the workgroup; returns this thread's exclusive
-// prefix and the workgroup total through *total.
-__device__ __forceinline__ unsigned block_exclusive_scan(unsigned value, unsigned *total) {
-  __shared__ unsigned wave_sums[kScanBlock / kWave];
-  unsigned inclusive = value;
-  for (int off = 1; off < kWave; off <<= 1) {
-    unsigned v = __shfl_up(inclusive, off);
-    if (static_cast<int>(lane_id()) >= off) inclusive += v;
-  }
-  const int w = threadIdx.x >> 6;
-  if (lane_id() == kWave - 1) wave_sums[w] = inclusive;
-  __syncthreads();
-  unsigned base = 0, sum = 0;
-  for (int ww = 0; ww < kScanBlock / kWave; ++ww) {
-    if (ww < w) base += wave_sums[ww];
-    sum += wave_sums[ww];
-  }
-  __syncthreads();
-  *total = sum;
-  return base + inclusive - value;
 }
 
 template <typename CT, typename IT>
@@ -129,21 +104,6 @@ static void unique_typed(const CT *coords, int64_t n, int ndim, const IT *batch_
 
 // ------------------------------------------------- fused target coordinates ----
 
-struct TargetSpec {
-  long long base[MNT_MAX_NDIM];     // floor(min / stride) per dimension
-  long long stride[MNT_MAX_NDIM];
-  int shift[MNT_MAX_NDIM];
-  unsigned long long mask[MNT_MAX_NDIM];
-  int batch_shift;
-  int ndim;
-  int num_batches;                  // 0 when there is no batch field
-};
-
-__device__ __forceinline__ long long floor_div(long long a, long long b) {
-  long long q = a / b;
-  return (a % b != 0 && ((a < 0) != (b < 0))) ? q - 1 : q;
-}
-
 template <typename CT, typename IT>
 __global__ __launch_bounds__(256) void pack_target_keys_kernel(
     const CT *__restrict__ coords, long long n, TargetSpec spec,
@@ -156,7 +116,7 @@ __global__ __launch_bounds__(256) void pack_target_keys_kernel(
 #pragma unroll
     for (int k = 0; k < MNT_MAX_NDIM; ++k) {
       if (k < spec.ndim) {
-        long long cell = floor_div(static_cast<long long>(coords[i * spec.ndim + k]), spec.stride[k]);
+        long long cell = cell_of(static_cast<long long>(coords[i * spec.ndim + k]), spec, k);
         key |= (static_cast<unsigned long long>(cell - spec.base[k]) & spec.mask[k]) << spec.shift[k];
       }
     }
@@ -245,66 +205,12 @@ __global__ __launch_bounds__(256) void emit_targets_kernel(
   }
 }
 
-static int bit_width64(unsigned long long range) {
-  return range == 0 ? 0 : 64 - __builtin_clzll(range);
-}
-
-// ---- bitmap form: when the packed keys span at most 2^28 values, the set of
-// distinct keys is a bitmap.  Marking it and walking it in key order yields
-// the sorted, duplicate-free targets without any sort.
-
-constexpr int kBitmapMaxBits = 28;                   // 32 MiB of bits
-constexpr int kBitmapWords = 8;                      // 32-bit words per thread
-constexpr int kBitmapTile = kScanBlock * kBitmapWords;
-// persistent block 0 in the bitmap form: the tile bases of the largest bitmap
-// first, so that the bitmap itself always starts at the same place
-constexpr size_t kBitmapBasesBytes =
-    ((((size_t{1} << (kBitmapMaxBits - 5)) / kBitmapTile + 1) * 4 + 255) / 256) * 256;
-
-template <typename CT, typename IT>
-__device__ __forceinline__ unsigned long long target_key(const CT *__restrict__ coords, long long i,
-                                                         const TargetSpec &spec,
-                                                         const IT *__restrict__ batch_dims) {
-  unsigned long long key = 0;
-#pragma unroll
-  for (int k = 0; k < MNT_MAX_NDIM; ++k) {
-    if (k < spec.ndim) {
-      long long cell = floor_div(static_cast<long long>(coords[i * spec.ndim + k]), spec.stride[k]);
-      key |= (static_cast<unsigned long long>(cell - spec.base[k]) & spec.mask[k]) << spec.shift[k];
-    }
-  }
-  if (spec.num_batches > 0) {
-    key |= static_cast<unsigned long long>(batch_of<IT>(i, batch_dims, spec.num_batches))
-           << spec.batch_shift;
-  }
-  return key;
-}
-
 template <typename CT, typename IT>
 __global__ __launch_bounds__(256) void mark_targets_kernel(const CT *__restrict__ coords, long long n,
                                                            TargetSpec spec,
                                                            const IT *__restrict__ batch_dims,
                                                            unsigned *__restrict__ bitmap) {
-  // Rows that follow each other in a sorted cloud fall into the same word of
-  // the bitmap more often than not (their cells differ in the last coordinate
-  // only): a run of neighbouring lanes with one word ORs its bits into the
-  // run's first lane, which issues the run's only atomic.
-  const long long stride = static_cast<long long>(gridDim.x) * blockDim.x;
-  const int lane = static_cast<int>(lane_id());
-  for (long long first = static_cast<long long>(blockIdx.x) * blockDim.x; first < n; first += stride) {
-    const long long i = first + threadIdx.x;
-    const bool valid = i < n;
-    const unsigned long long key = valid ? target_key<CT, IT>(coords, i, spec, batch_dims) : 0ull;
-    const unsigned word = valid ? static_cast<unsigned>(key >> 5) : 0xffffffffu;   // no word has this index
-    unsigned bits = valid ? 1u << (key & 31u) : 0u;
-    for (int off = 1; off < kWave; off <<= 1) {
-      const unsigned next_word = __shfl_down(word, off);
-      const unsigned next_bits = __shfl_down(bits, off);
-      if (lane + off < kWave && next_word == word) bits |= next_bits;
-    }
-    const unsigned word_before = __shfl_up(word, 1);
-    if (valid && (lane == 0 || word_before != word)) atomicOr(&bitmap[word], bits);
-  }
+  mark_rows<CT, IT>(coords, n, spec, batch_dims, bitmap);
 }
 
 __global__ __launch_bounds__(kScanBlock) void bitmap_tile_sums_kernel(const unsigned *__restrict__ bitmap,
@@ -327,38 +233,8 @@ __global__ __launch_bounds__(1024) void bitmap_scan_kernel(unsigned *__restrict_
                                                            unsigned *host_count,
                                                            unsigned long long *flag,
                                                            unsigned long long sequence) {
-  __shared__ unsigned wave_sums[1024 / kWave];
-  const int t = threadIdx.x;
-  const int chunk = (tiles + 1023) / 1024;
-  const int lo = t * chunk;
-  const int hi = min(tiles, lo + chunk);
-  unsigned sum = 0;
-  for (int i = lo; i < hi; ++i) sum += tile_sums[i];
-  // scan of the 1 024 per-thread sums: inside each wavefront by shuffles, then
-  // every thread adds the wavefronts before its own
-  unsigned inclusive = sum;
-  for (int off = 1; off < kWave; off <<= 1) {
-    const unsigned v = __shfl_up(inclusive, off);
-    if (static_cast<int>(lane_id()) >= off) inclusive += v;
-  }
-  const int w = t >> 6;
-  if (lane_id() == kWave - 1) wave_sums[w] = inclusive;
-  __syncthreads();
-  unsigned before = 0, all = 0;
-  for (int ww = 0; ww < 1024 / kWave; ++ww) {
-    const unsigned v = wave_sums[ww];
-    before += ww < w ? v : 0u;
-    all += v;
-  }
-  unsigned run = before + inclusive - sum;
-  for (int i = lo; i < hi; ++i) {
-    const unsigned v = tile_sums[i];
-    tile_sums[i] = run;
-    run += v;
-  }
-  if (t == 1023) {
-    const unsigned total = all;
-    tile_sums[tiles] = total;
+  const unsigned total = scan_in_place(tile_sums, tiles);
+  if (threadIdx.x == 1023) {
     *host_count = total;
     __threadfence_system();
     __hip_atomic_store(flag, sequence, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -369,80 +245,8 @@ template <typename CT, typename IT>
 __global__ __launch_bounds__(kScanBlock) void bitmap_emit_kernel(
     unsigned *__restrict__ bitmap, long long words, const unsigned *__restrict__ tile_bases,
     int tiles, TargetSpec spec, CT *__restrict__ out, IT *__restrict__ batch_dims_out) {
-  const long long base = static_cast<long long>(blockIdx.x) * kBitmapTile + threadIdx.x * kBitmapWords;
-  // a tile without a set bit has nothing to write, unless a batch boundary
-  // falls into it (then it is read like any other)
-  if (batch_dims_out == nullptr && tile_bases[blockIdx.x] == tile_bases[blockIdx.x + 1]) return;
-  unsigned word[kBitmapWords];
-  unsigned count = 0;
-#pragma unroll
-  for (int r = 0; r < kBitmapWords; ++r) {
-    word[r] = base + r < words ? bitmap[base + r] : 0u;
-    count += __popc(word[r]);
-  }
-  // Set bits cluster (cells that differ in the last coordinate share a word):
-  // a thread that walked its own 8 words would hold up its wavefront for up to
-  // 256 rows while others have none.  The tile's non-empty words, with the rank
-  // of their first row, are therefore listed in LDS and dealt round-robin.
-  __shared__ unsigned s_word[kBitmapTile], s_rank[kBitmapTile];
-  __shared__ unsigned short s_at[kBitmapTile];
-  unsigned total;
-  unsigned run = block_exclusive_scan(count, &total) + tile_bases[blockIdx.x];
-  unsigned filled = 0;
-#pragma unroll
-  for (int r = 0; r < kBitmapWords; ++r) filled += word[r] != 0u ? 1u : 0u;
-  unsigned listed;
-  unsigned slot = block_exclusive_scan(filled, &listed);
-#pragma unroll
-  for (int r = 0; r < kBitmapWords; ++r) {
-    const unsigned long long first_key = static_cast<unsigned long long>(base + r) << 5;
-    if (batch_dims_out != nullptr && base + r < words) {
-      // batch boundaries g << batch_shift that fall into this word
-      const unsigned long long step = 1ull << spec.batch_shift;
-      for (unsigned long long g = (first_key + step - 1) >> spec.batch_shift;
-           g < static_cast<unsigned long long>(spec.num_batches) && (g << spec.batch_shift) < first_key + 32;
-           ++g) {
-        const unsigned bit = static_cast<unsigned>((g << spec.batch_shift) - first_key);
-        batch_dims_out[g] = static_cast<IT>(run + __popc(word[r] & ((1u << bit) - 1u)));
-      }
-    }
-    if (word[r] != 0u) {
-      bitmap[base + r] = 0u;                     // the bitmap goes back all zero: the next build clears nothing
-      s_word[slot] = word[r];
-      s_rank[slot] = run;
-      s_at[slot] = static_cast<unsigned short>(threadIdx.x * kBitmapWords + r);
-      ++slot;
-      run += __popc(word[r]);
-    }
-  }
-  __syncthreads();
-  // Keys of the bitmap form have at most 28 bits, and (field + base) * stride
-  // worked out in CT wraps exactly as the wide product cut to CT does: the
-  // loop stays in 32-bit arithmetic for 32-bit coordinates.
-  const unsigned tile_key = static_cast<unsigned>(static_cast<unsigned long long>(blockIdx.x) * kBitmapTile << 5);
-  for (unsigned i = threadIdx.x; i < listed; i += kScanBlock) {
-    unsigned bits = s_word[i];
-    unsigned at = s_rank[i];
-    const unsigned first_key = tile_key + (static_cast<unsigned>(s_at[i]) << 5);
-    while (bits != 0u) {
-      const unsigned bit = __ffs(bits) - 1;
-      bits &= bits - 1u;
-      const unsigned key = first_key | bit;
-      CT *row = out + static_cast<long long>(at) * spec.ndim;
-#pragma unroll
-      for (int k = 0; k < MNT_MAX_NDIM; ++k) {
-        if (k < spec.ndim) {
-          const CT cell = static_cast<CT>((key >> spec.shift[k]) & static_cast<unsigned>(spec.mask[k])) +
-                          static_cast<CT>(spec.base[k]);
-          row[k] = cell * static_cast<CT>(spec.stride[k]);
-        }
-      }
-      ++at;
-    }
-  }
-  if (batch_dims_out != nullptr && blockIdx.x == 0 && threadIdx.x == 0) {
-    batch_dims_out[spec.num_batches] = static_cast<IT>(tile_bases[tiles]);
-  }
+  emit_bitmap_tile<CT, IT>(bitmap, words, static_cast<int>(blockIdx.x), tile_bases[blockIdx.x],
+                           tile_bases[blockIdx.x + 1], tile_bases[tiles], spec, out, batch_dims_out, nullptr);
 }
 
 // What phase 2 needs to know about phase 1 (kept in the arena's pending blob).
@@ -464,8 +268,8 @@ static void target_count_typed(const CT *coords, int64_t n, int ndim, const int6
   Arena &arena = Arena::of(stream);
   arena.pending.valid = false;
   const bool batched = batch_dims != nullptr && num_batches > 1;
+  arena.pass_pending = false;
   TargetSpec spec;
-  memset(&spec, 0, sizeof(spec));
   {
     Scope scope(stream);
     long long h_bounds[16];
@@ -474,28 +278,11 @@ static void target_count_typed(const CT *coords, int64_t n, int ndim, const int6
     } else {
       read_bounds(coords, n, nullptr, 0, ndim, sizeof(CT) == 4 ? MNT_INT32 : MNT_INT64, h_bounds, scope, stream);
     }
-    int bits = 0;
-    spec.ndim = ndim;
-    for (int k = ndim - 1; k >= 0; --k) {
+    for (int k = 0; k < ndim; ++k) {
       MNT_CHECK(target_stride[k] > 0, "target stride must be positive but found %lld",
                 static_cast<long long>(target_stride[k]));
-      auto fdiv = [](long long a, long long b) {
-        long long q = a / b;
-        return (a % b != 0 && ((a < 0) != (b < 0))) ? q - 1 : q;
-      };
-      long long lo = fdiv(h_bounds[k], target_stride[k]);
-      long long hi = fdiv(h_bounds[MNT_MAX_NDIM + k], target_stride[k]);
-      int width = bit_width64(static_cast<unsigned long long>(hi) - static_cast<unsigned long long>(lo));
-      spec.base[k] = lo;
-      spec.stride[k] = target_stride[k];
-      spec.shift[k] = bits < 64 ? bits : 63;
-      spec.mask[k] = width >= 64 ? ~0ull : ((1ull << width) - 1ull);
-      bits += width;
     }
-    int batch_width = batched ? bit_width64(static_cast<unsigned long long>(num_batches - 1)) : 0;
-    spec.batch_shift = bits < 64 ? bits : 63;
-    spec.num_batches = batched ? static_cast<int>(num_batches) : 0;
-    bits += batch_width;
+    const int bits = make_target_spec(h_bounds, target_stride, ndim, batched ? num_batches : 0, spec);
     MNT_CHECK(bits <= 64,
               "coordinate range needs %d key bits; strided target generation supports at most 64",
               bits);
@@ -640,19 +427,6 @@ static void target_fill_typed(CT *out, IT *batch_dims_out, hipStream_t stream) {
 }  // namespace mnt
 
 using namespace mnt;
-
-#define MNT_DISPATCH_CI(coord_dtype, index_dtype, CALL) \
-  do {                                                  \
-    if (coord_dtype == MNT_INT32 && index_dtype == MNT_INT32) { \
-      CALL(int32_t, int32_t);                           \
-    } else if (coord_dtype == MNT_INT32) {              \
-      CALL(int32_t, int64_t);                           \
-    } else if (index_dtype == MNT_INT32) {              \
-      CALL(int64_t, int32_t);                           \
-    } else {                                            \
-      CALL(int64_t, int64_t);                           \
-    }                                                   \
-  } while (0)
 
 extern "C" int mnt_unique_coordinates(const void *sorted_coords, int64_t n, int ndim,
                                       int coord_dtype, const void *batch_dims,

@@ -8,6 +8,7 @@ forward pass never reads them back from the device, and orders offsets by
 size with a STABLE sort (the reference's device sort is unstable, so its tie
 order is not reproducible)."""
 import contextlib
+import ctypes
 import functools
 import os
 import operator
@@ -51,7 +52,11 @@ class KernelMapCache(object):
     are the same; the price is one worst-case allocation per pass (no level has
     more rows than the input cloud) and one such session per process at a time
     (a second cache builds the ordinary way meanwhile).  ``num_ahead_hits``
-    counts the requests served that way."""
+    counts the requests served that way.
+
+    Without it the cache keeps the list of what the last pass asked for and
+    builds all of it at once at the first request after a ``reset()``
+    (:mod:`minuet_amd.nn.passplan`)."""
 
     def __init__(self, ndim: int, dtype: torch.dtype, device: Union[str, torch.device],
                  layout: str = "minuet", disable_reordering: bool = False, lookahead: bool = False):
@@ -68,6 +73,10 @@ class KernelMapCache(object):
         self._offset_groups_cache = dict()      # key -> offset-group tables of the dense map (False: none)
         self._coordinates_cache = dict()
         self._bounds_cache = dict()
+        self._requests = dict()                 # what this pass has asked for, in order (values unused)
+        self._pass_plan = None                  # PassPlan of the last pass (False: it cannot be built at once)
+        self._built = None                      # what it built for the present cloud
+        self._fast_maps = dict()                # layer shape -> source stride -> the extension's view of a map
         self.num_map_builds = 0
         self.num_coordinate_builds = 0
         # look-ahead: the requests of the last pass that built something, and the
@@ -106,6 +115,7 @@ class KernelMapCache(object):
                 self._recipe_rest = recipe[1:] if alone and len(recipe) > 1 else None
             self._recording = []
         self._ahead_tried = False
+        self._plan_next_pass()
         self._coordinates_cache.clear()
         self._kernel_maps_cache.clear()
         self._swapped_maps_cache.clear()
@@ -113,6 +123,70 @@ class KernelMapCache(object):
         self._inverse_maps_cache.clear()
         self._offset_groups_cache.clear()
         self._bounds_cache.clear()
+        self._fast_maps.clear()
+
+    def _plan_next_pass(self):
+        """Turns the requests of the pass that ends here into the plan of the next one."""
+        if self._built is not None:
+            for entry, request in self._built.entries:
+                if entry.used:                   # a layer that never came through Python
+                    self._note_fast(request)
+            self._built = None
+        requests, self._requests = self._requests, dict()
+        if self._lookahead or not requests or not self._coordinates_cache:
+            return
+        plan = self._pass_plan
+        stride, (coordinates, _, batch_dims) = next(iter(self._coordinates_cache.items()))
+        index_dtype = coordinates.dtype if batch_dims is None else batch_dims.dtype
+        if (plan is not None and plan.stride == stride and plan.index_dtype == index_dtype
+                and len(plan.requests) == len(requests) and all(entry in requests for entry in plan.requests)):
+            return
+        from minuet_amd.nn.passplan import PassPlan
+        try:
+            self._pass_plan = PassPlan(requests, self._kernel_offsets, stride, index_dtype)
+        except ValueError:
+            self._pass_plan = None
+
+    def _note_fast(self, request):
+        """A layer ran with the map of ``request`` (see ``PassPlan``): so it has
+        asked for that map, and for the level it leads to."""
+        _, _, _, kind, key, transposed = request
+        if key[0] != key[1]:
+            self._requests.setdefault(("coords", key[0], key[1]))
+        if kind == "IMPLICIT":
+            self._requests.setdefault(("dense", key))
+            if transposed:
+                self._requests.setdefault(("invert", key))
+        elif kind == "GROUPS":
+            self._requests.setdefault(("dense", key))
+            self._requests.setdefault(("groups", key))
+        else:
+            self._requests.setdefault(("dense", key))
+            self._requests.setdefault(("tables", key, not self._disable_reordering))
+        self._requests.setdefault(request)
+
+    def _open_pass(self, coordinates, stride, batch_dims):
+        """First request of a pass: with a plan of the last one, builds everything on it."""
+        plan = self._pass_plan
+        if (plan is None or self._lookahead or plan.stride != stride or not coordinates.is_cuda
+                or coordinates.shape[0] == 0 or not coordinates.is_contiguous()
+                or (batch_dims is not None and not batch_dims.is_contiguous())
+                or plan.index_dtype != (coordinates.dtype if batch_dims is None else batch_dims.dtype)
+                or torch.cuda.is_current_stream_capturing()):
+            return
+        known = self._known_bounds(coordinates)
+        if known is None:
+            known = _C.remembered_bounds(coordinates)
+        built = plan.build(coordinates, batch_dims, known)
+        if built is None:
+            self._pass_plan = None
+            return
+        self._built = built
+        self._coordinates_cache.update(built.coordinates)
+        self.num_coordinate_builds += plan.num_levels
+        self.num_map_builds += len(plan.map_of)
+        self._remember_bounds(coordinates, built.bounds)
+        built.fill_fast(self._fast_maps)
 
     def _from_ahead(self, tag, record, coordinates, stride, batch_dims):
         """Notes the request ``record`` for the next pass's recipe and, with the
@@ -169,11 +243,16 @@ class KernelMapCache(object):
         ndim = source_coordinates.shape[1]
         source_stride = as_tuple(source_stride, size=ndim, name="source_stride")
         kernel_stride = as_tuple(kernel_stride, size=ndim, name="kernel_stride")
-        self._coordinates_cache.setdefault(
-            source_stride, (source_coordinates, source_stride, source_batch_dims))
+        if source_stride not in self._coordinates_cache:
+            first = not self._coordinates_cache
+            self._coordinates_cache[source_stride] = (source_coordinates, source_stride, source_batch_dims)
+            if first:
+                self._open_pass(source_coordinates, source_stride, source_batch_dims)
         combine = operator.floordiv if transposed else operator.mul
         target_stride = tuple(combine(a, b) for a, b in zip(source_stride, kernel_stride))
         hit = self._coordinates_cache.get(target_stride)
+        if not transposed and target_stride != source_stride:
+            self._requests.setdefault(("coords", source_stride, target_stride))
         if hit is not None:
             return hit
         if transposed:
@@ -205,8 +284,11 @@ class KernelMapCache(object):
         open if it is new."""
         entry = self._coordinates_cache.get(stride)
         if entry is None:
+            first = not self._coordinates_cache
             entry = (coordinates, stride, batch_dims)
             self._coordinates_cache[stride] = entry
+            if first:
+                self._open_pass(coordinates, stride, batch_dims)
         return entry
 
     def _map_key(self, ndim, source_stride, target_stride, kernel_size, kernel_dilation, transposed):
@@ -246,6 +328,12 @@ class KernelMapCache(object):
             source_coordinates.shape[1], source_stride, target_stride, kernel_size, kernel_dilation,
             transposed)
         entry = self._dense_maps_cache.get(key)
+        self._requests.setdefault(("dense", key))
+        if entry is None and transposed and self._built is not None and key in self._built.shape:
+            self._take_dense(key, self._built.coordinates[key[0]][0])
+            entry = self._dense_maps_cache.get(key)
+        elif entry is None and not transposed:
+            entry = self._take_dense(key, source_coordinates)
         if entry is None:
             if transposed:
                 raise RuntimeError(_TRANSPOSED_FIRST)
@@ -269,6 +357,16 @@ class KernelMapCache(object):
             return entry[0]
         return self._inverse_of(key)
 
+    def _take_dense(self, key, source_coordinates):
+        """The dense map ``key`` as the pass build left it, filed like one built on request."""
+        if self._built is None:
+            return None
+        dense = self._built.dense(key, source_coordinates)
+        if dense is None:
+            return None
+        entry = self._dense_maps_cache[key] = (dense, source_coordinates.shape[0])
+        return entry
+
     def get_offset_groups(self, source_coordinates: torch.Tensor, source_stride,
                           source_batch_dims: Optional[torch.Tensor],
                           target_coordinates: torch.Tensor, target_stride,
@@ -287,12 +385,20 @@ class KernelMapCache(object):
         entry = self._offset_groups_cache.get(key)
         if entry is None:
             offsets = self._kernel_offsets(stride_key, size_key, dilation_key)
+            entry = self._built.groups(key, source_coordinates) if self._built is not None else None
+            if entry is not None:
+                self._requests.setdefault(("dense", key))
+                self._requests.setdefault(("groups", key))
+                self._offset_groups_cache[key] = entry
+                return entry
             entry = False
             if offsets.shape == (27, 3) and _C.offset_group_table(offsets) is not None:
                 dense = self.get_dense_kernel_map(source_coordinates, source_stride, source_batch_dims,
                                                   target_coordinates, target_stride, target_batch_dims,
                                                   kernel_size, kernel_dilation)
                 entry = _C.kernel_map_offset_groups(dense, offsets) or False
+                if entry:
+                    self._requests.setdefault(("groups", key))
             self._offset_groups_cache[key] = entry
         return entry or None
 
@@ -301,6 +407,12 @@ class KernelMapCache(object):
         inverse = self._inverse_maps_cache.get(key)
         if inverse is None:
             dense, num_sources = self._dense_maps_cache[key]
+            self._requests.setdefault(("invert", key))
+            if self._built is not None:
+                inverse = self._built.inverse(key)
+                if inverse is not None:
+                    self._inverse_maps_cache[key] = inverse
+                    return inverse
             inverse = self._from_ahead(("invert", key), [("invert", key)], None, None, None)
             if inverse is None:
                 inverse = _C.kernel_map_invert(dense, num_sources)
@@ -324,11 +436,12 @@ class KernelMapCache(object):
             return hit
         forward = self._kernel_maps_cache.get(key)
         if forward is None:
-            if transposed and key not in self._dense_maps_cache:
+            if transposed and key not in self._dense_maps_cache and (
+                    self._built is None or key not in self._built.shape):
                 raise RuntimeError(_TRANSPOSED_FIRST)
             forward = self._build_tables(key, source_coordinates, source_batch_dims, target_coordinates,
                                          target_batch_dims, source_stride, kernel_size, kernel_dilation,
-                                         disable_reordering)
+                                         disable_reordering, transposed)
         if not transposed:
             return forward
         swapped = forward.swapped(dense=self._inverse_of(key))
@@ -337,12 +450,22 @@ class KernelMapCache(object):
 
     def _build_tables(self, key, source_coordinates, source_batch_dims, target_coordinates,
                       target_batch_dims, source_stride, kernel_size, kernel_dilation,
-                      disable_reordering):
+                      disable_reordering, transposed=False):
         """Rank tables, order and sizes of the forward layer of ``key``: from the
         dense map when a layer already asked for that, else everything at once.
         (For a transposed caller the coordinate arguments are the other way
         round, but then the dense map exists and they are not used.)"""
         reorder = not self._disable_reordering and not disable_reordering
+        self._requests.setdefault(("dense", key))
+        self._requests.setdefault(("tables", key, reorder))
+        if self._built is not None and key in self._built.shape:
+            # (a transposed caller's source coordinates are the map's targets)
+            kernel_map = self._built.tables(key, source_coordinates if not transposed
+                                            else self._built.coordinates[key[0]][0], reorder)
+            if kernel_map is not None:
+                self._dense_maps_cache[key] = (kernel_map.dense, kernel_map.num_sources)
+                self._kernel_maps_cache[key] = kernel_map
+                return kernel_map
         entry = self._dense_maps_cache.get(key)
         if entry is None and self._lookahead:
             # the worker builds the two halves as two items: take the dense map first
@@ -431,6 +554,7 @@ class SparseConv(Module):
         factory = {"device": device, "dtype": dtype}
         volume = int(np.prod(self.kernel_size))
         self._packed = None
+        self._fast = None
         self.kernel = torch.nn.Parameter(torch.empty(volume, in_channels, out_channels, **factory))
         if bias:
             self.bias = torch.nn.Parameter(torch.empty(out_channels, **factory))
@@ -506,6 +630,7 @@ class SparseConv(Module):
         nothing, so call this after them (``reset_parameters``, ``load_state_dict``
         and ``.to()`` / ``.half()`` / ``.cuda()`` do it themselves)."""
         self._packed = None
+        self._fast = None
 
     def _load_from_state_dict(self, *args, **kwargs):
         super()._load_from_state_dict(*args, **kwargs)
@@ -699,7 +824,7 @@ class SparseConv(Module):
             return False
         return dataflow == "offset_groups" or self.in_channels * features.element_size() >= 256
 
-    def _pointwise(self, features: torch.Tensor, epilogue: Optional[F.Epilogue]) -> torch.Tensor:
+    def _pointwise(self, features: torch.Tensor, epilogue: Optional[F.Epilogue]):
         """1x1x1 kernel, stride 1: a plain ``features @ W`` (reference:
         convolutions.py:452-455).  Where the single-kernel forward takes the
         shape it runs there, as one offset whose kernel map is the identity,
@@ -718,11 +843,12 @@ class SparseConv(Module):
             if identity is None or identity.shape[1] < rows or identity.device != features.device:
                 identity = torch.arange(rows, dtype=torch.int32, device=features.device).view(1, rows)
                 self._identity_map = identity
-            return _C.sparse_convolution_forward_implicit(features, weights, identity[:, :rows],
-                                                          epilogue=epilogue,
-                                                          packed_weights=self._packed_kernel()[1])
+            packed = self._packed_kernel()[1]
+            out = _C.sparse_convolution_forward_implicit(features, weights, identity[:, :rows],
+                                                         epilogue=epilogue, packed_weights=packed)
+            return out, ("POINTWISE", weights.detach(), packed, None, None, 0)
         out = torch.mm(features, weights[0])
-        return out if epilogue is None else epilogue.apply(out)
+        return out if epilogue is None else epilogue.apply(out), None
 
     def forward(self, inputs: SparseTensor,
                 epilogue: Optional[F.Epilogue] = None) -> SparseTensor:
@@ -730,15 +856,29 @@ class SparseConv(Module):
         convolutions.py:446-499) is applied to the output rows in the same pass
         that writes them: ``act(conv(x) * scale + shift + residual)``, with the
         bias, if any, added before the scale."""
-        if epilogue is not None and self.bias is not None:
-            bias = self.bias.float()
-            shift = bias if epilogue.scale is None else bias * epilogue.scale.float()
-            if epilogue.shift is not None:
-                shift = shift + epilogue.shift.float()
-            epilogue = F.Epilogue(epilogue.scale, shift, epilogue.residual, epilogue.activation,
-                                  epilogue.negative_slope)
+        if self._fast is not None:                  # as the last call left it: no Python in between
+            result = _C._host.run(self, inputs, epilogue)
+            if result is not None:
+                return result
+        original = epilogue
+        bias = self.bias
+        if bias is not None and (epilogue is not None or (inputs.F.is_cuda and not (
+                torch.is_grad_enabled() and (bias.requires_grad or inputs.F.requires_grad)))):
+            # one more per-channel shift of the output pass
+            shift = bias.float()
+            if epilogue is None:
+                epilogue = F.Epilogue(shift=shift)
+            else:
+                if epilogue.scale is not None:
+                    shift = shift * epilogue.scale.float()
+                if epilogue.shift is not None:
+                    shift = shift + epilogue.shift.float()
+                epilogue = F.Epilogue(epilogue.scale, shift, epilogue.residual, epilogue.activation,
+                                      epilogue.negative_slope)
+            bias = None
+        made = None                                 # (kind, weights, packed, map pointers, owners, index code)
         if self.is_trivial:
-            features = self._pointwise(inputs.F, epilogue)
+            features, made = self._pointwise(inputs.F, epilogue)
             coordinates, stride, batch_dims = inputs.C, inputs.stride, inputs.batch_dims
         else:
             cache = self._kernel_map_cache
@@ -752,6 +892,10 @@ class SparseConv(Module):
                     transposed=self.transposed, source_coordinates=inputs.C,
                     source_batch_dims=inputs.batch_dims, source_stride=inputs.stride,
                     kernel_stride=self.stride)
+            if self._fast is not None and cache._built is not None:
+                result = _C._host.run(self, inputs, original)     # the pass has just been built
+                if result is not None:
+                    return result
             map_args = dict(transposed=self.transposed, source_coordinates=inputs.C,
                             source_stride=inputs.stride, source_batch_dims=inputs.batch_dims,
                             target_coordinates=coordinates, target_stride=stride,
@@ -774,6 +918,7 @@ class SparseConv(Module):
                 weights, packed = self._packed_kernel()
                 features = _C.sparse_convolution_forward_groups(sources, weights, groups, epilogue=epilogue,
                                                                 packed_weights=packed)
+                made = ("GROUPS", weights, packed, groups.pointers(), groups, 0)
             elif implicit and self._tuning_data is None:
                 # single-kernel dataflow: the dense map is all it needs
                 dense = cache.get_dense_kernel_map(**map_args)
@@ -783,13 +928,38 @@ class SparseConv(Module):
                 features = _C.sparse_convolution_forward_implicit(sources, weights, dense,
                                                                   epilogue=epilogue,
                                                                   packed_weights=packed)
+                if not pad and dense.is_contiguous():
+                    made = ("IMPLICIT", weights, packed, (dense.data_ptr(),), dense, 0)
             else:
-                features = self._forward_tables(cache, map_args, sources, epilogue)
-        if self.bias is not None and epilogue is None:
-            features += self.bias
+                features, made = self._forward_tables(cache, map_args, sources, epilogue)
+        if bias is not None:
+            features += bias
         if batch_dims is not None and len(batch_dims) <= 2:
             batch_dims = None
+        if made is not None and made[2] is not None and self._tuning_data is None:
+            self._keep_fast(made, inputs, features, coordinates, stride, batch_dims)
         return SparseTensor.like(inputs, features, coordinates, stride, batch_dims)
+
+    def _keep_fast(self, made, inputs, features, coordinates, stride, batch_dims):
+        """Leaves what this call worked out for the extension module: the module's
+        side of it in ``_fast``, the map's side in the cache's ``_fast_maps``."""
+        name, weights, packed, pointers, owners, index_code = made
+        host = _C.load_host()
+        kind = getattr(host, name)
+        shape_id = None
+        if pointers is not None:
+            shape_id = (kind, self.kernel_size, self.stride, self.dilation, self.transposed)
+            entry = host.MapEntry(kind, coordinates, stride, batch_dims, owners, features.device.index, index_code,
+                                  inputs.F.shape[0], features.shape[0], pointers)
+            cache = self._kernel_map_cache
+            cache._fast_maps.setdefault(shape_id, {})[inputs.stride] = entry
+            key = cache._map_key(self.ndim, inputs.stride, stride, self.kernel_size, self.dilation, self.transposed)[0]
+            cache._note_fast(("fast", shape_id, inputs.stride, name, key, self.transposed))
+        if not weights.is_contiguous():
+            return
+        self._fast = host.Layer(self, kind, weights, packed, shape_id, 1 if name == "TABLES" and
+                                self._allow_shortcut_matmul else 0,
+                                None if self.bias is None else self.bias.detach().float())
 
     def _forward_tables(self, cache, map_args, sources, epilogue):
         """Gather -> GEMM -> Scatter through the rank tables (the reference's
@@ -802,13 +972,20 @@ class SparseConv(Module):
                 and sources.is_cuda and kernel_map.ensure_row_lists()):
             dataflow = "list_driven"
         weights, packed = self._packed_kernel() if sources.is_cuda else (self.kernel, None)
-        return F.sparse_convolution_forward(
+        features = F.sparse_convolution_forward(
             sources=sources, weights=weights, kernel_map=kernel_map,
             gather_tile_size=self._tunable_config["gather_tile_size"],
             scatter_tile_size=self._tunable_config["scatter_tile_size"],
             allow_shortcut_matmul=self._allow_shortcut_matmul,
             threshold=self._tunable_config["threshold"], epilogue=epilogue,
             dataflow=dataflow, packed_weights=packed)
+        if dataflow != "gather_gemm_scatter" or kernel_map.prepared is None or kernel_map.order_host is None:
+            return features, None
+        (_, _, _, index_code, _, source_masks, target_masks, order, sizes, sizes_host, order_host, in_idx,
+         _) = kernel_map.prepared
+        address = lambda pointer: None if pointer is None else ctypes.cast(pointer, ctypes.c_void_p).value
+        return features, ("TABLES", weights, packed, (source_masks, target_masks, order, sizes, address(sizes_host),
+                                                      address(order_host), in_idx), kernel_map, index_code)
 
 
 class SparseConv3d(SparseConv):

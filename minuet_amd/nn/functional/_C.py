@@ -46,6 +46,9 @@ SIGNATURES = {
     "mnt_stream_acquire": (_int, [_vp]),
     "mnt_stream_release": (_int, [_vp]),
     "mnt_host_wait_stats": (_int, [_pi64, _pi64, _int]),
+    "mnt_pass_levels": (_int, [_vp, _i64, _int, _int, _vp, _i64, _int, _vp, _vp, _int, _vp, _int, _vp, _pi64,
+                               _c.POINTER(_int), _vp]),
+    "mnt_pass_build": (_int, [_vp, _vp, _vp, _vp, _vp, _vp]),
     "mnt_lookahead_start": (_int, [_vp, _i64, _int, _int, _vp, _i64, _int, _pi64, _vp, _int, _int, _pi64,
                                    _vp, _vp]),
     "mnt_lookahead_wait": (_int, [_int, _vp, _pi64]),
@@ -137,6 +140,42 @@ def load_library():
     import atexit
     atexit.register(lambda: lib.mnt_lookahead_finish(None))
     return lib
+
+
+_host = None
+
+
+def load_host():
+    """The extension module with the host side of layer calls (csrc/host.cpp),
+    bound to the library's entry points; loaded once, built first only when no
+    build exists."""
+    global _host
+    if _host is not None:
+        return _host
+    import importlib.util
+    import torch.nn.modules.module as torch_module
+    from minuet_amd.build import HOST_PATH, build_host
+    from minuet_amd.nn import activations, convolutions, normalizations
+    from minuet_amd.tensors import SparseTensor
+    lib = load_library()
+    if not os.path.exists(HOST_PATH):
+        build_host()
+    spec = importlib.util.spec_from_file_location("minuet_host", HOST_PATH)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    names = ("mnt_sparse_convolution_forward_implicit", "mnt_sparse_convolution_forward_groups",
+             "mnt_sparse_convolution_forward_fused", "mnt_last_error")
+    hooks = tuple(getattr(torch_module, name) for name in (
+        "_global_forward_hooks", "_global_forward_pre_hooks", "_global_backward_hooks",
+        "_global_backward_pre_hooks"))
+    codes = {activations.ReLU: "relu", torch.nn.ReLU: "relu", activations.LeakyReLU: "leaky_relu",
+             torch.nn.LeakyReLU: "leaky_relu", activations.ReLU6: "relu6", torch.nn.ReLU6: "relu6"}
+    module.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in names}, SparseTensor,
+                (convolutions.SparseConv, convolutions.SparseConv3d),
+                (normalizations.BatchNorm, torch.nn.BatchNorm1d),
+                {cls: ACTIVATION_CODES[name] for cls, name in codes.items()}, hooks)
+    _host = module
+    return module
 
 
 def _check(status: int):
@@ -289,9 +328,22 @@ def sort_coordinates(coordinates: torch.Tensor, batch_dims: Optional[torch.Tenso
             _ptr(coordinates), n, ndim, ccode, _ptr(batch_dims),
             batch_dims.numel() - 1 if batch_dims is not None else 1, _INT[itype], _ptr(indices),
             _ptr(out), bounds.ctypes.data_as(_pi64), _stream(device)))
+    remember_bounds(out, bounds)
     if return_bounds:
         return indices, out, bounds
     return indices, out
+
+
+def remember_bounds(coordinates: torch.Tensor, bounds: np.ndarray):
+    """Notes the extremes of a coordinate tensor on the tensor itself, for as long
+    as its version counter stands still."""
+    if coordinates.shape[0] > 0 and not coordinates.is_inference():
+        coordinates._minuet_bounds = (coordinates._version, bounds)
+
+
+def remembered_bounds(coordinates: torch.Tensor):
+    noted = getattr(coordinates, "_minuet_bounds", None)
+    return noted[1] if noted is not None and noted[0] == coordinates._version else None
 
 
 # ------------------------------------------------------------------ unique ----
@@ -1237,6 +1289,10 @@ class OffsetGroups:
         self.rank, self.src, self.head, self.offsets, self.num_targets = rank, src, head, offsets, num_targets
         self._offsets_address = offsets.ctypes.data
 
+    def pointers(self):
+        """Addresses of rank, src, head (device) and offsets (host)."""
+        return _ptr(self.rank), _ptr(self.src), _ptr(self.head), self._offsets_address
+
 
 def kernel_map_offset_groups(kernel_map: torch.Tensor, offsets_host: np.ndarray) -> Optional[OffsetGroups]:
     """Offset groups of a dense int32 kernel map ``[27, T]`` whose offsets form a
@@ -1533,6 +1589,52 @@ def host_wait_stats(reset: bool = False):
     waits, ns = ctypes.c_int64(0), ctypes.c_int64(0)
     _check(load_library().mnt_host_wait_stats(ctypes.byref(waits), ctypes.byref(ns), 1 if reset else 0))
     return waits.value, ns.value * 1e-9
+
+
+class PassLevel(ctypes.Structure):
+    """``mnt_pass_level`` of include/minuet_hip.h."""
+    _fields_ = [("stride", ctypes.c_int64 * 4), ("count", ctypes.c_int64), ("coords_at", ctypes.c_int64),
+                ("batch_dims_at", ctypes.c_int64)]
+
+
+class PassMap(ctypes.Structure):
+    """``mnt_pass_map`` of include/minuet_hip.h."""
+    _fields_ = [("source_level", ctypes.c_int32), ("target_level", ctypes.c_int32), ("want", ctypes.c_int32),
+                ("reorder", ctypes.c_int32), ("offsets_host", ctypes.c_void_p), ("num_offsets", ctypes.c_int64),
+                ("group_offsets_host", ctypes.c_void_p), ("sizes_host", ctypes.c_void_p),
+                ("order_host", ctypes.c_void_p), ("num_sources", ctypes.c_int64), ("num_targets", ctypes.c_int64),
+                ("at", ctypes.c_int64 * 11)]
+
+
+def pass_levels(coordinates: torch.Tensor, batch_dims: Optional[torch.Tensor], bounds, levels, num_levels: int,
+                maps, accept=None):
+    """First half of a pass build (mnt_pass_levels): ``(bytes of the block, bounds of
+    the cloud)``, or None where the library does not take the list.  ``levels`` /
+    ``maps``: ctypes arrays of :class:`PassLevel` / :class:`PassMap`, filled in;
+    ``accept(rows)`` may turn a cloud down beforehand."""
+    device = coordinates.device
+    n, ndim = coordinates.shape
+    if accept is not None and not accept(n):
+        return None
+    known = None if bounds is None else np.ascontiguousarray(bounds, dtype=np.int64)
+    found = np.empty(8, dtype=np.int64)
+    total, supported = ctypes.c_int64(0), ctypes.c_int(0)
+    with _on(device):
+        _check(load_library().mnt_pass_levels(
+            coordinates.data_ptr(), n, ndim, _INT[coordinates.dtype], _ptr(batch_dims),
+            batch_dims.numel() - 1 if batch_dims is not None else 1,
+            _INT[batch_dims.dtype] if batch_dims is not None else 0, None if known is None else known.ctypes.data,
+            ctypes.addressof(levels), num_levels, ctypes.addressof(maps), len(maps), found.ctypes.data,
+            ctypes.byref(total), ctypes.byref(supported), _stream(device)))
+    return (total.value, found) if supported.value else None
+
+
+def pass_build(coordinates: torch.Tensor, batch_dims: Optional[torch.Tensor], levels, maps, store: torch.Tensor):
+    """Second half of a pass build (mnt_pass_build): everything into ``store``."""
+    device = coordinates.device
+    with _on(device):
+        _check(load_library().mnt_pass_build(coordinates.data_ptr(), _ptr(batch_dims), ctypes.addressof(levels),
+                                             ctypes.addressof(maps), store.data_ptr(), _stream(device)))
 
 
 AHEAD_COORDS, AHEAD_DENSE, AHEAD_TABLES, AHEAD_INVERT = 0, 1, 2, 3

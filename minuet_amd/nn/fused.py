@@ -15,6 +15,7 @@ import torch
 from torch import nn
 
 from minuet_amd.nn import functional as F
+from minuet_amd.nn.functional import _C
 from minuet_amd.nn.activations import LeakyReLU, ReLU, ReLU6
 from minuet_amd.nn.convolutions import SparseConv
 from minuet_amd.nn.normalizations import BatchNorm
@@ -43,7 +44,10 @@ def batch_norm_affine(norm: torch.nn.BatchNorm1d):
         shift = -norm.running_mean.float() * scale
         if norm.bias is not None:
             shift = shift + norm.bias.float()
-    norm.__dict__["_minuet_affine"] = (key, scale, shift)
+    kept = (key, scale, shift)
+    if scale.is_cuda:
+        kept += (_C.load_host().Affine(norm, scale, shift),)
+    norm.__dict__["_minuet_affine"] = kept
     return scale, shift
 
 
@@ -67,6 +71,10 @@ def conv_norm_act(conv: SparseConv, norm: Optional[torch.nn.BatchNorm1d], act: O
     """``act(norm(conv(x)) + residual)``.  One pass when ``norm`` is in
     evaluation mode (or absent) and ``act`` is a ReLU / LeakyReLU / ReLU6 (or
     absent); otherwise the modules run one after another."""
+    if _C._host is not None:                    # nothing has changed since the last call: no Python in between
+        y = _C._host.conv_norm_act(conv, norm, act, x, residual)
+        if y is not None:
+            return y
     kind = _activation_of(act) if act is not None else ("none", 0.0)
     if (norm is None or _foldable(norm)) and kind is not None and x.F.is_cuda:
         scale, shift = batch_norm_affine(norm) if norm is not None else (None, None)

@@ -1,0 +1,104 @@
+"""The build of a whole pass (levels and maps at once) against the single calls."""
+import numpy as np
+import pytest
+import torch
+
+import minuet_amd as minuet
+from helpers import dev, random_cloud, sorted_unique
+from minuet_amd.nn.functional import _C
+from minuet_amd.nn.passplan import PassPlan
+from minuet_amd.unet import SparseUNet
+from minuet_amd.utils.helpers import generate_kernel_offsets
+
+pytestmark = pytest.mark.gpu
+
+
+def offsets_of(source_stride, kernel_size, dilation):
+    return np.ascontiguousarray(generate_kernel_offsets(3, kernel_size, source_stride, dilation), dtype=np.int64)
+
+
+@pytest.mark.parametrize("n,extent,stride,batches,ctype,itype", [
+    (1, 5, 2, 1, np.int32, None), (70, 9, 2, 1, np.int32, None), (5000, 40, 2, 3, np.int32, np.int32),
+    (5000, 40, 3, 2, np.int64, np.int64), (30000, 500, 2, 4, np.int32, np.int64), (200, 6, 4, 7, np.int32, np.int32)])
+def test_pass_build_equals_single_calls(n, extent, stride, batches, ctype, itype):
+    rng = np.random.default_rng(n)
+    bd = None
+    if batches > 1:
+        cuts = np.sort(rng.integers(0, n, size=batches - 1))
+        bd = np.concatenate([[0], cuts, [n]]).astype(itype)
+    c, bd = sorted_unique(random_cloud(n, extent, n, lo=-extent // 2, dtype=ctype), bd)
+    s1, s2, s4 = (1,) * 3, (stride,) * 3, (stride * stride,) * 3
+    one = (1, 1, 1)
+    sub = [(s, s, (3, 3, 3), one) for s in (s1, s2, s4)]
+    down = [(s1, s2, (2, 2, 2), one), (s2, s4, (2, 2, 2), one), (s2, s4, (3, 3, 3), one)]
+    requests = [("coords", s1, s2), ("coords", s2, s4)]
+    for key in sub:
+        requests += [("dense", key), ("groups", key), ("tables", key, True)]
+    for key in down:
+        requests += [("dense", key), ("invert", key), ("tables", key, False)]
+    index_dtype = torch.int32 if ctype == np.int32 else torch.int64
+    if itype is not None:
+        index_dtype = torch.int32 if itype == np.int32 else torch.int64
+    plan = PassPlan(requests, offsets_of, s1, index_dtype)
+    coords, dims = dev(c), dev(bd)
+    for _ in range(2):                                   # the second build finds the bitmaps the first has cleared
+        built = plan.build(coords, dims, None)
+    levels = {s1: (coords, dims)}
+    for source, target in ((s1, s2), (s2, s4)):
+        levels[target] = _C.target_coordinates(*levels[source], target)
+        got = built.coordinates[target]
+        assert torch.equal(got[0], levels[target][0]) and got[1] == target
+        assert (dims is None and got[2] is None) or torch.equal(got[2], levels[target][1])
+    for key in sub + down:
+        source, target, kernel, dilation = key
+        offsets = offsets_of(source, kernel, dilation)
+        dense, _ = _C.kernel_map_dense(levels[source][0], levels[target][0], offsets, levels[source][1],
+                                       levels[target][1])
+        assert torch.equal(built.dense(key, built.coordinates[source][0]), dense), key
+        assert built.dense(key, built.coordinates[source][0].clone()) is None       # another tensor: not served
+        num_sources = levels[source][0].shape[0]
+        if key in down:
+            assert torch.equal(built.inverse(key), _C.kernel_map_invert(dense, num_sources)), key
+        else:
+            ref = _C.kernel_map_offset_groups(dense, offsets)
+            got = built.groups(key, built.coordinates[source][0])
+            rows = ref.head[1:10].tolist()
+            assert torch.equal(got.head[:10], ref.head[:10]) and torch.equal(got.rank, ref.rank)
+            for j, count in enumerate(rows):
+                lo = j * dense.shape[1]
+                assert torch.equal(got.src[lo:lo + count, :3], ref.src[lo:lo + count, :3])
+        if index_dtype == torch.int32:
+            reorder = key in sub
+            ref = _C.kernel_map_tables(dense, num_sources, reorder)
+            got = built.tables(key, built.coordinates[source][0], reorder)
+            assert np.array_equal(got.sizes_host, ref["sizes_host"])
+            for name in ("source_masks", "target_masks", "in_idx", "out_idx"):
+                assert torch.equal(getattr(got, name), ref[name]), (key, name)
+            assert torch.equal(got.kernel_map_sizes, ref["sizes"])
+            if reorder:
+                assert np.array_equal(got.order_host, ref["order_host"])
+                assert torch.equal(got.kernel_map_order, ref["order"])
+
+
+@pytest.mark.parametrize("kind", ["fp16", "fp32"])
+def test_second_pass_of_a_network_equals_its_first(kind):
+    """The second pass after a reset builds everything at once; other clouds, the
+    same cloud again and a cache left alone give what a fresh cache gives."""
+    dtype = torch.float16 if kind == "fp16" else torch.float32
+    torch.manual_seed(0)
+    net = SparseUNet(4, 16, dtype=dtype, device="cuda").eval()
+    cache = minuet.nn.KernelMapCache(3, torch.int32, "cuda")
+    with torch.no_grad():
+        for seed, n in ((1, 3000), (2, 4100), (1, 3000), (3, 900)):
+            c, bd = sorted_unique(random_cloud(n, 30, seed, lo=-9), np.array([0, n // 3, n], dtype=np.int32))
+            x = minuet.SparseTensor(torch.randn(c.shape[0], 4, device="cuda").to(dtype), dev(c), batch_dims=dev(bd))
+            cache.reset()
+            minuet.set_kernel_map_cache(net, cache)
+            y = net(x)
+            assert (cache._built is not None) == (seed != 1 or cache._pass_plan is not None)
+            again = net(x)                                       # maps kept
+            minuet.set_kernel_map_cache(net, minuet.nn.KernelMapCache(3, torch.int32, "cuda"))
+            ref = net(x)
+            assert torch.equal(y.C, ref.C) and torch.equal(y.F, ref.F) and torch.equal(again.F, ref.F)
+            assert torch.equal(y.batch_dims, ref.batch_dims)
+    assert cache.num_coordinate_builds == 16 and cache.num_map_builds == 36
