@@ -587,6 +587,31 @@ int mnt_sparse_convolution_forward_implicit(const void *sources, const void *wei
 int mnt_kernel_map_invert(const int32_t *kernel_map, int64_t num_offsets, int64_t num_targets,
                           int64_t num_sources, int32_t *inverse_out, void *stream);
 
+/* ---- Before the first layer and after the last ---------------------------- */
+
+/* Voxels floor(p / voxel_size) of n points [n, ndim] (wide_points: double,
+ * else float; voxel_size[ndim], divided by in the points' precision), sorted and
+ * without duplicates: voxels_out has room for n rows of the coordinate type, the
+ * first *count_out are written.  reverse_out (nullable) [n] takes the row every
+ * point fell into.  What minuet/nn/functional/voxelize.py:11-35 sets out to do. */
+int mnt_voxelize(const void *points, int64_t n, int ndim, int wide_points, const double *voxel_size,
+                 int coord_dtype, void *voxels_out, int64_t *reverse_out, int64_t *count_out, void *stream);
+
+/* out[i] = row order[i] of the given tensors, whose rows of row_bytes bytes (a
+ * multiple of 2) are numbered one after the other; at most 64 tensors
+ * (host arrays of their device addresses and row counts). */
+int mnt_gather_rows(const void *const *sources, const int64_t *source_rows, int num_sources, int64_t row_bytes,
+                    const void *order, int index_dtype, int64_t n, void *out, void *stream);
+
+/* Host integers to device memory as kernel arguments: nothing is waited for. */
+int mnt_upload_ints(const int64_t *values, int64_t count, int index_dtype, void *out, void *stream);
+
+/* Sum (mean = 0) or mean of the feature rows of every cloud: out [num_batches,
+ * channels] of the feature type, added up in fp32; batch_dims null: one cloud of
+ * n rows (minuet/nn/functional/pooling.py). */
+int mnt_global_pool(const void *features, const void *batch_dims, int64_t n, int64_t num_batches, int64_t channels,
+                    int float_dtype, int index_dtype, int mean, void *out, void *stream);
+
 /* ---- Map: the coordinates and kernel maps of a whole pass in one build ------ */
 
 /* A network asks for the same coordinate levels and kernel maps for every

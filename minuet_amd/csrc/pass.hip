@@ -5,7 +5,7 @@
 // tables were 66 launches of 2 to 30 us with a wait on the host per level and
 // per table, each behind every layer enqueued before it.  Built together they
 // are about ten launches and one wait at the start of the pass (measured with
-// the layers that follow: 2.2 -> 1.5 ms for that network):
+// the layers that follow: 2.16 -> 1.69 ms for that network):
 //
 //   pass_mark_kernel     every source row sets its bit in the bitmap of every
 //                        level (a level's cell is floor(c / stride) of the

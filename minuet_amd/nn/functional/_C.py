@@ -46,6 +46,10 @@ SIGNATURES = {
     "mnt_stream_acquire": (_int, [_vp]),
     "mnt_stream_release": (_int, [_vp]),
     "mnt_host_wait_stats": (_int, [_pi64, _pi64, _int]),
+    "mnt_voxelize": (_int, [_vp, _i64, _int, _int, _vp, _int, _vp, _vp, _pi64, _vp]),
+    "mnt_gather_rows": (_int, [_vp, _vp, _int, _i64, _vp, _int, _i64, _vp, _vp]),
+    "mnt_upload_ints": (_int, [_vp, _i64, _int, _vp, _vp]),
+    "mnt_global_pool": (_int, [_vp, _vp, _i64, _i64, _i64, _int, _int, _int, _vp, _vp]),
     "mnt_pass_levels": (_int, [_vp, _i64, _int, _int, _vp, _i64, _int, _vp, _vp, _int, _vp, _int, _vp, _pi64,
                                _c.POINTER(_int), _vp]),
     "mnt_pass_build": (_int, [_vp, _vp, _vp, _vp, _vp, _vp]),
@@ -1510,6 +1514,69 @@ def cuda_time_gemm(allow_shortcut_matmul, parallel, threshold, weights, source_m
     """csrc/minuet/torch/cuda_sparse_convolution_forward.cu:7-48."""
     return _time_stage("mnt_time_gemm", (1 if allow_shortcut_matmul else 0, int(parallel)),
                        threshold, None, weights, source_masks, target_masks, kernel_map_sizes, True)
+
+
+# --------------------------------------------- before and after the layers ----
+
+MAX_GATHER_SOURCES = 64
+
+
+def voxelize(points: torch.Tensor, voxel_size: Sequence[float], dtype: torch.dtype, want_reverse: bool):
+    """Sorted distinct voxels of float32 / float64 points [N, D], N > 0, and (or
+    None) the int64 row every point fell into (mnt_voxelize)."""
+    device = _common_device([points])
+    n, ndim = points.shape
+    room = torch.empty((n, ndim), dtype=dtype, device=device)
+    reverse = torch.empty((n,), dtype=torch.int64, device=device) if want_reverse else None
+    sizes = (ctypes.c_double * ndim)(*voxel_size)
+    count = ctypes.c_int64(0)
+    with _on(device):
+        _check(load_library().mnt_voxelize(
+            points.data_ptr(), n, ndim, 1 if points.dtype == torch.float64 else 0, ctypes.addressof(sizes),
+            _INT[dtype], room.data_ptr(), _ptr(reverse), ctypes.byref(count), _stream(device)))
+    return room[:count.value], reverse
+
+
+def gather_rows(sources: Sequence[torch.Tensor], order: torch.Tensor) -> torch.Tensor:
+    """``torch.cat(sources)[order]`` for up to 64 contiguous [N_i, C] tensors of one
+    type, in one launch (mnt_gather_rows)."""
+    device = _common_device([*sources, order])
+    n, channels = order.shape[0], sources[0].shape[1]
+    out = torch.empty((n, channels), dtype=sources[0].dtype, device=device)
+    count = len(sources)
+    pointers = (ctypes.c_void_p * count)(*[t.data_ptr() for t in sources])
+    rows = (ctypes.c_int64 * count)(*[t.shape[0] for t in sources])
+    with _on(device):
+        _check(load_library().mnt_gather_rows(
+            ctypes.addressof(pointers), ctypes.addressof(rows), count, channels * out.element_size(),
+            order.data_ptr(), _INT[order.dtype], n, out.data_ptr(), _stream(device)))
+    return out
+
+
+def upload_ints(values: Sequence[int], dtype: torch.dtype, device: torch.device) -> torch.Tensor:
+    """A small 1-D int32 / int64 tensor from host integers, without the wait that a
+    copy from pageable memory brings (mnt_upload_ints)."""
+    out = torch.empty((len(values),), dtype=dtype, device=device)
+    array = (ctypes.c_int64 * max(1, len(values)))(*values)
+    with _on(device):
+        _check(load_library().mnt_upload_ints(ctypes.addressof(array), len(values), _INT[dtype], _ptr(out),
+                                              _stream(device)))
+    return out
+
+
+def global_pool(features: torch.Tensor, batch_dims: Optional[torch.Tensor], mean: bool) -> torch.Tensor:
+    """Sum or mean of the rows of every cloud (mnt_global_pool): [B, C], or [C]
+    without ``batch_dims``."""
+    device = _common_device([features] + ([batch_dims] if batch_dims is not None else []))
+    n, channels = features.shape
+    batches = batch_dims.numel() - 1 if batch_dims is not None else 1
+    out = torch.empty((channels,) if batch_dims is None else (batches, channels), dtype=features.dtype, device=device)
+    with _on(device):
+        _check(load_library().mnt_global_pool(
+            _ptr(features), _ptr(batch_dims), n, batches, channels, _FLOAT[features.dtype],
+            _INT[batch_dims.dtype] if batch_dims is not None else 0, 1 if mean else 0, out.data_ptr(),
+            _stream(device)))
+    return out
 
 
 # ------------------------------------------------------------------ memory ----

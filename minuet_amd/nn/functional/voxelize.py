@@ -25,6 +25,11 @@ def voxelize(coordinates: torch.Tensor, voxel_size=1, dtype: torch.dtype = torch
     if not coordinates.is_cuda:
         raise NotImplementedError
     ndim = coordinates.shape[1]
+    if (coordinates.dtype in (torch.float32, torch.float64) and dtype in (torch.int32, torch.int64)
+            and coordinates.shape[0] > 0 and 1 <= ndim <= 4):
+        unique, reverse = _C.voxelize(coordinates.contiguous(), as_tuple(voxel_size, size=ndim, name="voxel_size"),
+                                      dtype, return_reverse_indices)
+        return (unique, reverse) if return_reverse_indices else unique
     size = torch.tensor(as_tuple(voxel_size, size=ndim, name="voxel_size"), dtype=coordinates.dtype,
                         device=coordinates.device)
     voxels = torch.floor(coordinates / size).to(dtype).contiguous()
@@ -52,9 +57,18 @@ def collate(coordinates: Sequence[torch.Tensor], features: Optional[Sequence[tor
     stacked = torch.cat(list(coordinates), dim=0).contiguous()
     if not stacked.is_cuda:
         raise NotImplementedError
-    counts = torch.tensor([0] + [int(c.shape[0]) for c in coordinates], dtype=torch.int64)
-    batch_dims = torch.cumsum(counts, dim=0).to(dtype=stacked.dtype, device=stacked.device)
+    ends = [0]
+    for cloud in coordinates:
+        ends.append(ends[-1] + int(cloud.shape[0]))
+    batch_dims = _C.upload_ints(ends, stacked.dtype, stacked.device)
     order, ordered = _C.sort_coordinates(stacked, batch_dims)
     if features is None:
         return ordered, batch_dims
+    first = features[0]
+    if (len(features) <= _C.MAX_GATHER_SOURCES and first.element_size() in (2, 4, 8) and not (
+            torch.is_grad_enabled() and any(f.requires_grad for f in features))
+            and all(f.dim() == 2 and f.is_contiguous() and f.dtype == first.dtype and f.shape[1] == first.shape[1]
+                    and f.device == stacked.device and f.shape[0] == c.shape[0]
+                    for f, c in zip(features, coordinates)) and first.shape[1] > 0):
+        return ordered, batch_dims, _C.gather_rows(features, order)
     return ordered, batch_dims, torch.cat(list(features), dim=0)[order.long()]

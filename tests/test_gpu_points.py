@@ -1,0 +1,64 @@
+"""Voxelisation, collating and global pools at the edges of their tiles."""
+import numpy as np
+import pytest
+import torch
+
+import minuet_oracle as orc
+from helpers import dev, host, random_cloud, sorted_unique
+from minuet_amd.nn import functional as F
+from minuet_amd.tensors import SparseTensor
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,ndim,ftype,dtype", [(1, 3, np.float32, torch.int32), (2049, 3, np.float64, torch.int64),
+                                                (5000, 2, np.float32, torch.int32), (4096, 4, np.float32, torch.int64),
+                                                (1049089, 3, np.float32, torch.int32)])
+def test_voxelize_against_numpy(n, ndim, ftype, dtype):
+    points = np.random.default_rng(n).normal(size=(n, ndim)).astype(ftype)
+    size = tuple(0.11 + 0.07 * k for k in range(ndim))
+    voxels, reverse = F.voxelize(dev(points), voxel_size=size, dtype=dtype, return_reverse_indices=True)
+    expect, inverse = np.unique(np.floor(points / np.asarray(size, dtype=ftype)).astype(np.int64), axis=0,
+                                return_inverse=True)
+    assert voxels.dtype == dtype and reverse.dtype == torch.int64
+    np.testing.assert_array_equal(host(voxels), expect)
+    np.testing.assert_array_equal(host(reverse), inverse.reshape(-1))
+
+
+@pytest.mark.parametrize("rows,channels", [((7,), 1), ((0, 3, 900), 6), ((5000, 1, 20000), 64), ((300, 41), 257),
+                                           ((130,), 1100)])
+@pytest.mark.parametrize("kind", ["fp32", "fp16", "bf16"])
+def test_global_pools(rows, channels, kind):
+    dtype = {"fp32": torch.float32, "fp16": torch.float16, "bf16": torch.bfloat16}[kind]
+    bounds = np.concatenate([[0], np.cumsum(rows)])
+    n = int(bounds[-1])
+    f = torch.randn(n, channels, device="cuda").to(dtype)
+    c = dev(np.arange(3 * n, dtype=np.int32).reshape(n, 3))
+    for itype in (np.int32, np.int64):
+        x = SparseTensor(f, c, batch_dims=dev(bounds.astype(itype)))
+        exact = f.double().cpu().numpy()
+        for pool, fold in ((F.global_avg_pool, np.mean), (F.global_sum_pool, np.sum)):
+            got = pool(x).double().cpu().numpy().reshape(len(rows), channels)
+            for g, count in enumerate(rows):
+                if count == 0:
+                    assert np.isnan(got[g]).all() if fold is np.mean else (got[g] == 0).all()
+                    continue
+                part = exact[bounds[g]:bounds[g + 1]]
+                want = fold(part, axis=0)
+                eps = {"fp32": 1e-5, "fp16": 1e-3, "bf16": 8e-3}[kind]
+                scale = np.abs(part).sum(axis=0) / (count if fold is np.mean else 1)
+                assert (np.abs(got[g] - want) <= eps * np.abs(want) + 1e-6 * scale).all()
+
+
+@pytest.mark.parametrize("channels,dtype", [(1, torch.float16), (4, torch.float16), (3, torch.float32), (8, torch.float32)])
+@pytest.mark.parametrize("clouds", [1, 3, 70])
+def test_collate_carries_rows(channels, dtype, clouds):
+    coords = [sorted_unique(random_cloud(5 + 40 * (k % 3), 30, k))[0] for k in range(clouds)]
+    feats = [torch.randn(c.shape[0], channels, device="cuda").to(dtype) for c in coords]
+    ordered, dims, rows = F.collate([dev(c) for c in coords], feats)
+    plain, plain_dims = F.collate([dev(c) for c in coords])
+    bounds = np.concatenate([[0], np.cumsum([c.shape[0] for c in coords])])
+    order = orc.arg_sort_coordinates(np.concatenate(coords), bounds.astype(np.int32))
+    assert torch.equal(ordered, plain) and torch.equal(dims, plain_dims)
+    np.testing.assert_array_equal(host(dims), bounds)
+    assert torch.equal(rows, torch.cat(feats)[dev(order.astype(np.int64))])
