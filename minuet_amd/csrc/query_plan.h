@@ -6,6 +6,9 @@
 // this block instead; the query kernel reads it from device memory.
 #pragma once
 
+#include <algorithm>
+#include <cstring>
+
 #include "device_utils.h"
 
 namespace mnt {
@@ -14,55 +17,73 @@ constexpr int kPlanGroupSpan = 4;                // key span of one offset group
 constexpr int kPlanMaxOffsets = 64;              // one lane per offset
 constexpr int kPlanInts = 6 * kPlanMaxOffsets;   // 4 words per group + 2 per member
 
-// Kernel offsets as launch arguments (rows past the count are ignored), and
-// what the host worked out about them for a cloud that is mapped onto itself:
-// halves != 0 when the offsets come in pairs d / -d (no offset named twice, at
-// least one pair); kind[o] is then 0 for the offset of a pair that is looked
-// up (the one whose first non-zero coordinate is positive, i.e. whose key delta
-// is), 1 for its mirror image, 2 for the zero offset, and mirror[o] the index
-// of the offset's mirror image.
+// Kernel offsets as launch arguments, and what can be said about them before the
+// bounds of the cloud (which is mapped onto itself) are known.  halves != 0 when
+// the offsets come in pairs d / -d (no offset named twice, at least one pair);
+// kind[o] is then 0 for the offset of a pair that is looked up (the one whose
+// first non-zero coordinate is positive, i.e. whose key delta is), 1 for its
+// mirror image, 2 for the zero offset, and mirror[o] the index of the offset's
+// mirror image.  The offsets that are looked up (all of them without halves) are
+// listed in ascending order of their coordinates, equal ones by index.  That is
+// the order of their key deltas: a field of the key has room for the difference
+// of any two offsets, so the first coordinate that differs decides.
 struct OffsetTable {
-  int v[kPlanMaxOffsets][MNT_MAX_NDIM];
+  int v[kPlanMaxOffsets][MNT_MAX_NDIM];   // the looked-up offsets in that order
+  int reach_lo[MNT_MAX_NDIM];             // least and largest step along each axis, over all offsets
+  int reach_hi[MNT_MAX_NDIM];
+  int num_kept;                           // offsets that are looked up
   int halves;
+  signed char origin[kPlanMaxOffsets];    // which offset each looked-up one is
   signed char kind[kPlanMaxOffsets];
   signed char mirror[kPlanMaxOffsets];
 };
 
-// Fills halves / kind / mirror of `table` from its first num_offsets rows.
-inline void classify_offset_pairs(OffsetTable &table, int num_offsets, int ndim, bool allow) {
-  table.halves = 0;
-  for (int o = 0; o < kPlanMaxOffsets; ++o) {
-    table.kind[o] = 0;
-    table.mirror[o] = -1;
-  }
-  if (!allow || num_offsets > kPlanMaxOffsets) return;
-  bool paired = true, any_positive = false;
-  for (int o = 0; o < num_offsets && paired; ++o) {
-    int sign = 0;
-    for (int k = 0; k < ndim && sign == 0; ++k) sign = table.v[o][k] > 0 ? 1 : table.v[o][k] < 0 ? -1 : 0;
-    int mirror = -1;
-    for (int p = 0; p < num_offsets; ++p) {
-      bool negated = true, same = true;
-      for (int k = 0; k < ndim; ++k) {
-        negated = negated && table.v[p][k] == -table.v[o][k];
-        same = same && table.v[p][k] == table.v[o][k];
-      }
-      if (negated && mirror < 0) mirror = p;
-      if (same && p != o) paired = false;                     // an offset named twice
+// The table of num_offsets <= kPlanMaxOffsets offsets, rows of ndim coordinates.
+inline OffsetTable make_offset_table(const int64_t *offsets, int num_offsets, int ndim, bool allow_halves) {
+  OffsetTable table;
+  memset(&table, 0, sizeof(table));
+  memset(table.mirror, -1, sizeof(table.mirror));
+  int order[kPlanMaxOffsets];
+  for (int o = 0; o < num_offsets; ++o) {
+    for (int k = 0; k < ndim; ++k) {
+      const int step = static_cast<int>(offsets[o * ndim + k]);
+      table.reach_lo[k] = std::min(table.reach_lo[k], step);
+      table.reach_hi[k] = std::max(table.reach_hi[k], step);
     }
-    paired = paired && mirror >= 0;
-    table.kind[o] = static_cast<signed char>(sign > 0 ? 0 : sign == 0 ? 2 : 1);
-    table.mirror[o] = static_cast<signed char>(mirror);
-    any_positive = any_positive || sign > 0;
+    order[o] = o;
   }
-  if (paired && any_positive) {
-    table.halves = 1;
-    return;
+  const auto compare = [&](int a, int b) {
+    for (int k = 0; k < ndim; ++k) {
+      const int64_t u = offsets[a * ndim + k], v = offsets[b * ndim + k];
+      if (u != v) return u < v ? -1 : 1;
+    }
+    return 0;
+  };
+  std::sort(order, order + num_offsets, [&](int a, int b) {
+    const int c = compare(a, b);
+    return c != 0 ? c < 0 : a < b;
+  });
+  // ascending and without repeats, the mirror image of the i-th is the i-th from the end
+  bool paired = allow_halves && num_offsets > 1;
+  for (int i = 0; i < num_offsets && paired; ++i) {
+    const int64_t *d = offsets + static_cast<int64_t>(order[i]) * ndim;
+    const int64_t *m = offsets + static_cast<int64_t>(order[num_offsets - 1 - i]) * ndim;
+    for (int k = 0; k < ndim; ++k) paired = paired && d[k] == -m[k];
+    paired = paired && (i == 0 || compare(order[i - 1], order[i]) != 0);
   }
-  for (int o = 0; o < kPlanMaxOffsets; ++o) {
-    table.kind[o] = 0;
-    table.mirror[o] = -1;
+  table.halves = paired ? 1 : 0;
+  for (int i = 0; i < num_offsets; ++i) {
+    const int o = order[i];
+    if (paired) {
+      const int other = num_offsets - 1 - i;
+      table.kind[o] = static_cast<signed char>(i > other ? 0 : i == other ? 2 : 1);
+      table.mirror[o] = static_cast<signed char>(order[other]);
+      if (i <= other) continue;
+    }
+    for (int k = 0; k < ndim; ++k) table.v[table.num_kept][k] = static_cast<int>(offsets[o * ndim + k]);
+    table.origin[table.num_kept++] = static_cast<signed char>(o);
   }
+  return table;
 }
 
 struct DevicePlan {
@@ -98,47 +119,47 @@ struct DevicePlan {
   const unsigned *window_starts;  // [window_buckets + 1]
 };
 
-struct PlanScratch {        // LDS of the wavefront that builds the plan
-  int inverse[kPlanMaxOffsets];              // offset at each place of the ascending delta order
-};
-
 __device__ __forceinline__ int plan_bits(unsigned long long range) {
   return range == 0 ? 0 : 64 - __builtin_clzll(range);
+}
+
+// What lane l of the planning wavefront takes from the launch arguments: looked-up
+// offset l and what is said about offset l.  Read with the lane's index (a load
+// per lane; picking them out of scalar registers took some 400 instructions) and
+// before the bounds are there.
+struct PlanLane {
+  int d[MNT_MAX_NDIM];
+  int origin, kind, mirror;
+};
+
+__device__ __forceinline__ PlanLane load_plan_lane(const OffsetTable &offsets) {
+  const int lane = lane_id();
+  PlanLane in;
+#pragma unroll
+  for (int k = 0; k < MNT_MAX_NDIM; ++k) in.d[k] = offsets.v[lane][k];
+  in.origin = offsets.origin[lane];
+  in.kind = offsets.kind[lane];
+  in.mirror = offsets.mirror[lane];
+  return in;
 }
 
 // Run by ONE whole wavefront.  bounds = lo[4], hi[4] of the cloud (sources and
 // targets are the same rows); the frame leaves room for every offset on both
 // sides of every field, so key(q + offset) == key(q) + delta(offset).
 // `declined` is the verdict of the launches before (non-zero: stop).
-__device__ __forceinline__ void make_plan_on_device(const long long *__restrict__ bounds,
+// The launch that carries it waits for it, so everything that needs no bounds is
+// in `offsets` already and no step here is a loop over cross-lane reads (with
+// the ordering and the ranges worked out here it took 10 us, of 28 us for
+// sorting 2 000 rows).
+__device__ __forceinline__ void make_plan_on_device(const long long *__restrict__ bounds, const PlanLane &in,
                                                     const OffsetTable &offsets, int num_offsets,
-                                                    int ndim, unsigned declined, PlanScratch &lds,
-                                                    DevicePlan *__restrict__ out,
+                                                    int ndim, unsigned declined, DevicePlan *__restrict__ out,
                                                     const unsigned *__restrict__ bucket_starts = nullptr,
                                                     int msd_cap = 0) {
   const int lane = lane_id();
-  // lane o takes offset o: selects on scalar operands, no indexed access to the arguments
-  int d[MNT_MAX_NDIM] = {0, 0, 0, 0};
-#pragma unroll
-  for (int l = 0; l < kPlanMaxOffsets; ++l) {
-#pragma unroll
-    for (int k = 0; k < MNT_MAX_NDIM; ++k) d[k] = lane == l ? offsets.v[l][k] : d[k];
-  }
   const bool live = lane < num_offsets;
   Frame f;
   int bits = 0;
-  int reach_lo[MNT_MAX_NDIM], reach_hi[MNT_MAX_NDIM];
-#pragma unroll
-  for (int k = 0; k < MNT_MAX_NDIM; ++k) {
-    int lo = live && k < ndim ? d[k] : 0, hi = lo;
-    for (int off = 32; off > 0; off >>= 1) {
-      const int a = __shfl_xor(lo, off), b = __shfl_xor(hi, off);
-      lo = a < lo ? a : lo;
-      hi = b > hi ? b : hi;
-    }
-    reach_lo[k] = lo < 0 ? lo : 0;
-    reach_hi[k] = hi > 0 ? hi : 0;
-  }
   bool fits = true;
 #pragma unroll
   for (int k = MNT_MAX_NDIM - 1; k >= 0; --k) {
@@ -147,8 +168,8 @@ __device__ __forceinline__ void make_plan_on_device(const long long *__restrict_
     f.width[k] = 0;
     if (k < ndim) {
       // coordinates are at most 64-bit and the reach is small: a range that wraps is caught below
-      const long long lo = bounds[k] + reach_lo[k];
-      const long long hi = bounds[MNT_MAX_NDIM + k] + reach_hi[k];
+      const long long lo = bounds[k] + offsets.reach_lo[k];
+      const long long hi = bounds[MNT_MAX_NDIM + k] + offsets.reach_hi[k];
       const unsigned long long range = static_cast<unsigned long long>(hi) - static_cast<unsigned long long>(lo);
       fits = fits && hi >= lo && lo <= bounds[k] && hi >= bounds[MNT_MAX_NDIM + k] && range < (1ull << 63);
       f.lo[k] = lo;
@@ -163,54 +184,28 @@ __device__ __forceinline__ void make_plan_on_device(const long long *__restrict_
   f.total_bits = bits;
   fits = fits && bits <= 63;
 
-  long long delta = 0;
+  long long mine = 0;
 #pragma unroll
   for (int k = 0; k < MNT_MAX_NDIM; ++k) {
     if (k < ndim) {
-      delta += static_cast<long long>(static_cast<unsigned long long>(static_cast<long long>(d[k])) << f.shift[k]);
+      mine += static_cast<long long>(static_cast<unsigned long long>(static_cast<long long>(in.d[k])) << f.shift[k]);
     }
   }
-  // what the host found out about the offsets: lane o takes entry o
   const bool halves = offsets.halves != 0;
-  int kind = 0, mirror = -1;
-#pragma unroll
-  for (int l = 0; l < kPlanMaxOffsets; ++l) {
-    kind = lane == l ? offsets.kind[l] : kind;
-    mirror = lane == l ? offsets.mirror[l] : mirror;
-  }
-  // the offsets that are looked up: all of them, or those of positive key delta
-  const bool kept = live && (!halves || kind == 0);
-  const int num_kept = __popcll(__ballot(kept));
-  // place among the kept offsets in ascending delta order (ties keep offset order)
-  int place = 0;
-  for (int p = 0; p < num_offsets; ++p) {
-    const long long other = __shfl(delta, p);
-    const bool other_kept = __shfl(kept ? 1 : 0, p) != 0;
-    place += other_kept && (other < delta || (other == delta && p < lane)) ? 1 : 0;
-  }
-  // lane i takes over the offset of place i; from here on lanes are places
-  if (kept) lds.inverse[place] = lane;
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  const int num_kept = offsets.num_kept;
   const bool placed = lane < num_kept;
-  const int origin = placed ? lds.inverse[lane] : lane;
-  const long long mine = __shfl(delta, origin);
-  int lead[MNT_MAX_NDIM];
-#pragma unroll
-  for (int k = 0; k < MNT_MAX_NDIM; ++k) lead[k] = __shfl(d[k], origin);
   // first place whose delta lies beyond this one's group span (num_kept if
   // none), and never more than kPlanGroupSpan + 1 members (repeated offsets)
-  int next = num_kept;
-  for (int p = num_kept - 1; p >= 0; --p) {
-    const long long other = __shfl(mine, p);
-    next = p > lane && other - mine > kPlanGroupSpan ? p : next;
+  int next = lane + kPlanGroupSpan + 1 < num_kept ? lane + kPlanGroupSpan + 1 : num_kept;
+#pragma unroll
+  for (int j = kPlanGroupSpan; j >= 1; --j) {
+    const long long other = __shfl(mine, lane + j < kWave ? lane + j : kWave - 1);
+    next = lane + j < num_kept && other - mine > kPlanGroupSpan ? lane + j : next;
   }
-  next = next < lane + kPlanGroupSpan + 1 ? next : lane + kPlanGroupSpan + 1;
   // the greedy grouping follows those links from place 0
   unsigned long long starts = 0;
   int num_groups = 0;
-  for (int cur = 0; cur < num_kept; cur = __shfl(next, cur)) {
+  for (int cur = 0; cur < num_kept; cur = __builtin_amdgcn_readlane(next, cur)) {
     starts |= 1ull << cur;
     ++num_groups;
   }
@@ -221,13 +216,13 @@ __device__ __forceinline__ void make_plan_on_device(const long long *__restrict_
   bool same_row = true;
 #pragma unroll
   for (int k = 0; k < MNT_MAX_NDIM; ++k) {
-    const int other = __shfl(lead[k], first_place);
-    same_row = same_row && (k + 1 >= ndim || other == lead[k]);
+    const int other = __shfl(in.d[k], first_place);
+    same_row = same_row && (k + 1 >= ndim || other == in.d[k]);
   }
   const bool in_rows = __ballot(placed && !same_row) == 0ull;
   if (placed) {
     out->tables[4 * num_groups + 2 * lane + 0] = static_cast<int>(mine - first_delta);
-    out->tables[4 * num_groups + 2 * lane + 1] = origin;
+    out->tables[4 * num_groups + 2 * lane + 1] = in.origin;
     if ((starts >> lane) & 1ull) {
       const unsigned long long first = static_cast<unsigned long long>(mine);
       out->tables[4 * group + 0] = static_cast<int>(static_cast<unsigned>(first & 0xffffffffull));
@@ -237,18 +232,15 @@ __device__ __forceinline__ void make_plan_on_device(const long long *__restrict_
     }
   }
   if (live) {
-    out->kind[lane] = halves ? kind : 0;
-    out->mirror[lane] = halves ? mirror : -1;
-    const bool writes = !halves || kind != 1;
+    out->kind[lane] = in.kind;
+    out->mirror[lane] = in.mirror;
+    const bool writes = in.kind != 1;
     const unsigned long long writers = __ballot(writes);
     if (writes) {
       const int y = __popcll(writers & ((1ull << lane) - 1ull));
-      out->rows[y] = lane | ((halves ? kind : 0) << 8) | ((halves ? mirror + 1 : 0) << 16);
+      out->rows[y] = lane | (in.kind << 8) | ((in.mirror + 1) << 16);
     }
   }
-  // an offset that is looked up must have a positive key delta, which is what
-  // the host's reading of its coordinates says; anything else stops the chain
-  const bool consistent = !halves || __ballot(kept && delta <= 0) == 0ull;
   const long long delta_min = __shfl(mine, 0);
   const long long delta_max = __shfl(mine, num_kept > 0 ? num_kept - 1 : 0);
   if (lane == 0) {
@@ -258,7 +250,7 @@ __device__ __forceinline__ void make_plan_on_device(const long long *__restrict_
     out->halves = halves ? 1 : 0;
     out->num_groups = num_groups;
     out->groups_in_rows = in_rows ? 1 : 0;
-    out->verdict = declined != 0 ? static_cast<int>(declined) : (fits && consistent ? 0 : 2);
+    out->verdict = declined != 0 ? static_cast<int>(declined) : (fits ? 0 : 2);
     out->num_offsets = num_offsets;
     // the sort's key: fields of the cloud's own ranges, coordinate 0 on top
     int sort_bits = 0, below_top = 0;
@@ -276,7 +268,7 @@ __device__ __forceinline__ void make_plan_on_device(const long long *__restrict_
     out->window_buckets = usable ? 1 << msd_cap : 0;
     out->window_shift = below_top;
     out->window_bucket_shift = sort_bits - msd_bits;
-    out->window_reach = reach_hi[0];
+    out->window_reach = offsets.reach_hi[0];
     out->window_lo = bounds[0];
     out->window_hi = bounds[MNT_MAX_NDIM];
     out->window_starts = bucket_starts;

@@ -619,7 +619,6 @@ constexpr int kBucketMax = 1 << kBucketMaxBits;
 constexpr int kBucketCap = 7680;              // rows of the largest bucket: its words, their padding and
                                               // the ranking kernel's tables fit 64 KiB of LDS
 constexpr int kBucketRows = 128;              // rows per bucket aimed at
-constexpr int64_t kBucketMinN = 2048;
 constexpr size_t kBucketHostOffset = 384;     // pinned block: largest bucket
 
 // Key layout of a sort that takes one round: fields from least to most
@@ -1305,9 +1304,8 @@ __global__ __launch_bounds__(kSortBlock) void bucket_rank_chain_kernel(
   if (blockIdx.x == 0) {
     // runs whatever the sort's verdict: the plan carries the verdict of the whole chain
     if (plan_out != nullptr && threadIdx.x < kWave) {
-      PlanScratch &scratch = *reinterpret_cast<PlanScratch *>(s_words);
-      static_assert(sizeof(PlanScratch) <= sizeof(s_words), "plan scratch must fit the word staging area");
-      make_plan_on_device(folded, offsets, num_offsets, ndim, declined, scratch, plan_out, bucket_starts, msd_cap);
+      const PlanLane lane_in = load_plan_lane(offsets);
+      make_plan_on_device(folded, lane_in, offsets, num_offsets, ndim, declined, plan_out, bucket_starts, msd_cap);
     }
     return;
   }
@@ -1500,6 +1498,215 @@ __global__ __launch_bounds__(1024) void bucket_pairs_kernel(const unsigned *__re
   }
 }
 
+// A cloud of up to kSmallSortRows rows, start to finish in one workgroup: bounds,
+// key layout, a counting split of the words (key above row index) by their top
+// bits into LDS, then every row counts the words of its part that are below its
+// own.  What such a cloud waits for is launches: bounds, fold and two radix
+// passes were nine of them, 39 us of kernels and a wait at 2 000 rows; this is
+// 8.4 us.  In here the time goes to LDS round trips, hence bounds folded in ten shuffles instead of forty-eight (see
+// fold_extremes), 4 096 parts, and the chain's query plan made by one wavefront
+// while the others place rows.
+// The split fails where more than kSmallPartRows rows agree in the top bits, or
+// where a key does not leave room for the row index: then nothing is written and
+// the verdict (status[0], host) says so.
+// With offsets it also clears `clear` and writes the query plan of a chain.
+constexpr int kSmallSortBlock = 1024;
+constexpr int kSmallSortItems = 4;
+constexpr int kSmallSortRows = kSmallSortBlock * kSmallSortItems;
+constexpr int kSmallPartBits = 12;
+constexpr unsigned kSmallPartRows = 384;
+
+struct SmallSortTell {            // where the host finds bounds and verdict (flag null: nobody waits)
+  long long *bounds;
+  unsigned *verdict;
+  unsigned long long *flag;
+  unsigned long long sequence;
+};
+
+// Minimum over the wavefront of eight values per lane; lane l ends with the
+// minimum of value l & 7.  Halving exchanges: in step d a lane keeps the values
+// whose bit d is its own and sends the others away (4 + 2 + 1 shuffles), then
+// the eight lanes groups fold (3).
+template <typename CT>
+__device__ __forceinline__ CT fold_extremes(const CT (&v)[8]) {
+  const int lane = lane_id();
+  CT four[4], two[2];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {                       // bit 2
+    const CT mine = lane & 4 ? v[i + 4] : v[i];
+    const CT other = __shfl_xor(lane & 4 ? v[i] : v[i + 4], 4);
+    four[i] = other < mine ? other : mine;
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {                       // bit 1
+    const CT mine = lane & 2 ? four[i + 2] : four[i];
+    const CT other = __shfl_xor(lane & 2 ? four[i] : four[i + 2], 2);
+    two[i] = other < mine ? other : mine;
+  }
+  CT one = lane & 1 ? two[1] : two[0];
+  const CT from = __shfl_xor(lane & 1 ? two[0] : two[1], 1);
+  one = from < one ? from : one;
+#pragma unroll
+  for (int d = 8; d < kWave; d <<= 1) {
+    const CT other = __shfl_xor(one, d);
+    one = other < one ? other : one;
+  }
+  return one;
+}
+
+template <typename CT, typename IT, bool kChain>
+__global__ __launch_bounds__(kSmallSortBlock) void small_sort_kernel(
+    const CT *__restrict__ coords, const IT *__restrict__ batch_dims, int num_batches, int ndim, int n, int idx_bits,
+    IT *__restrict__ indices_out, CT *__restrict__ sorted_out, SmallSortTell tell, long long *__restrict__ folded,
+    unsigned *__restrict__ status, unsigned *__restrict__ clear, int clear_words, OffsetTable offsets, int num_offsets,
+    DevicePlan *__restrict__ plan_out) {
+  constexpr int kWaves = kSmallSortBlock / kWave;
+  constexpr int kParts = 1 << kSmallPartBits;
+  constexpr int kPerThread = kParts / kSmallSortBlock;
+  static_assert(kWaves == 16 && kPerThread == 4, "the folds over wavefronts and the scan of the parts");
+  static_assert(2 * MNT_MAX_NDIM == 8, "eight extremes");
+  __shared__ __align__(16) unsigned long long s_words[kSmallSortRows];
+  __shared__ __align__(16) unsigned s_part[kParts];   // rows of a part, then its first row, then the row after its last
+  __shared__ unsigned s_wave[kWaves], s_most[kWaves];
+  __shared__ CT s_bounds[kWaves][8];
+  const int tid = threadIdx.x, wave = tid / kWave, lane = lane_id();
+  CT c[kSmallSortItems][MNT_MAX_NDIM];
+#pragma unroll
+  for (int r = 0; r < kSmallSortItems; ++r) {
+    const int i = r * kSmallSortBlock + tid;
+    load_row_raw<CT>(coords + static_cast<long long>(i < n ? i : n - 1) * ndim, ndim, c[r]);
+  }
+  *reinterpret_cast<uint4 *>(s_part + 4 * tid) = make_uint4(0u, 0u, 0u, 0u);
+  PlanLane lane_in;
+  if (kChain) {
+    if (wave == kWaves - 1) lane_in = load_plan_lane(offsets);
+    for (int i = tid; i < clear_words; i += kSmallSortBlock) clear[i] = 0u;
+  }
+  // rows past the end repeat the last one: no extreme changes.  (~v turns the order round.)
+  CT extreme[8];
+#pragma unroll
+  for (int k = 0; k < MNT_MAX_NDIM; ++k) {
+    extreme[k] = c[0][k];
+    extreme[MNT_MAX_NDIM + k] = ~c[0][k];
+#pragma unroll
+    for (int r = 1; r < kSmallSortItems; ++r) {
+      extreme[k] = c[r][k] < extreme[k] ? c[r][k] : extreme[k];
+      extreme[MNT_MAX_NDIM + k] = static_cast<CT>(~c[r][k]) < extreme[MNT_MAX_NDIM + k]
+                                      ? static_cast<CT>(~c[r][k]) : extreme[MNT_MAX_NDIM + k];
+    }
+  }
+  const CT folded_wave = fold_extremes<CT>(extreme);
+  if (lane < 8) s_bounds[wave][lane] = folded_wave;
+  __syncthreads();
+  CT all = s_bounds[lane / 8][lane % 8];
+  {
+    const CT second = s_bounds[8 + lane / 8][lane % 8];
+    all = second < all ? second : all;
+#pragma unroll
+    for (int d = 8; d < kWave; d <<= 1) {
+      const CT other = __shfl_xor(all, d);
+      all = other < all ? other : all;
+    }
+  }
+  long long b[2 * MNT_MAX_NDIM];                      // (slots past ndim repeat coordinate 0)
+#pragma unroll
+  for (int slot = 0; slot < 8; ++slot) {
+    const CT v = __shfl(all, slot);
+    b[slot] = uniform64(static_cast<long long>(slot < MNT_MAX_NDIM ? v : static_cast<CT>(~v)));
+  }
+  CoordSource<CT, IT> src;
+  src.coords = coords;
+  src.batch_dims = batch_dims;
+  src.perm = nullptr;
+  const int key_bits = single_round_spec(b, ndim, num_batches, src.spec);
+  const int word_bits = key_bits + idx_bits;
+  bool go = word_bits <= 64;
+  unsigned long long word[kSmallSortItems];
+  const int part_shift = word_bits > kSmallPartBits ? word_bits - kSmallPartBits : 0;
+  if (go) {
+#pragma unroll
+    for (int r = 0; r < kSmallSortItems; ++r) {
+      const int i = r * kSmallSortBlock + tid;
+      if (i >= n) continue;
+      unsigned long long key;
+      unsigned row;
+      src.pack(i, c[r], key, row);
+      word[r] = (key << idx_bits) | static_cast<unsigned long long>(row);
+      atomicAdd(&s_part[static_cast<unsigned>(word[r] >> part_shift)], 1u);
+    }
+  }
+  __syncthreads();
+  {
+    const uint4 count = *reinterpret_cast<const uint4 *>(s_part + 4 * tid);
+    const unsigned mine = count.x + count.y + count.z + count.w;
+    unsigned inclusive = mine;
+    unsigned most = max(max(count.x, count.y), max(count.z, count.w));
+    for (int off = 1; off < kWave; off <<= 1) {
+      const unsigned u = __shfl_up(inclusive, off);
+      if (lane >= off) inclusive += u;
+    }
+    const bool crowded = __any(most > kSmallPartRows);
+    if (lane == kWave - 1) s_wave[wave] = inclusive;
+    if (lane == 0) s_most[wave] = crowded ? 1u : 0u;
+    __syncthreads();
+    const unsigned theirs = s_wave[lane % kWaves];
+    go = go && !__any(s_most[lane % kWaves] != 0);    // the same in every thread
+    unsigned before = lane < wave ? theirs : 0u;      // (wave < 16: lanes 0 .. wave - 1)
+#pragma unroll
+    for (int d = 8; d >= 1; d >>= 1) before += __shfl_xor(before, d);
+    before = __shfl(before, 0);
+    const unsigned at = before + inclusive - mine;
+    *reinterpret_cast<uint4 *>(s_part + 4 * tid) =
+        make_uint4(at, at + count.x, at + count.x + count.y, at + count.x + count.y + count.z);
+  }
+  __syncthreads();
+  if (tid == 0) {
+    if (kChain) {
+#pragma unroll
+      for (int slot = 0; slot < 2 * MNT_MAX_NDIM; ++slot) folded[slot] = b[slot];
+      status[0] = go ? 0u : 1u;                       // (among the words cleared above, before a barrier)
+    }
+    if (tell.flag != nullptr) {
+#pragma unroll
+      for (int slot = 0; slot < 2 * MNT_MAX_NDIM; ++slot) tell.bounds[slot] = b[slot];
+      tell.verdict[0] = go ? 0u : 1u;
+      __threadfence_system();
+      __hip_atomic_store(tell.flag, tell.sequence, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+  }
+  if (go) {
+#pragma unroll
+    for (int r = 0; r < kSmallSortItems; ++r) {
+      const int i = r * kSmallSortBlock + tid;
+      if (i < n) s_words[atomicAdd(&s_part[static_cast<unsigned>(word[r] >> part_shift)], 1u)] = word[r];
+    }
+  }
+  __syncthreads();
+  if (kChain) {
+    if (wave == kWaves - 1 && plan_out != nullptr) {
+      make_plan_on_device(b, lane_in, offsets, num_offsets, ndim, go ? 0u : 1u, plan_out);
+    }
+  }
+  if (!go) return;
+  const KeySink<CT, IT> sink{src.spec, indices_out, sorted_out};
+  const unsigned long long idx_mask = (1ull << idx_bits) - 1ull;
+#pragma unroll
+  for (int r = 0; r < kSmallSortItems; ++r) {
+    const int e = r * kSmallSortBlock + tid;
+    if (e >= n) continue;
+    const unsigned long long mine = s_words[e];
+    const unsigned part = static_cast<unsigned>(mine >> part_shift);
+    const unsigned from = part == 0 ? 0u : s_part[part - 1], to = s_part[part];
+    unsigned rank = from, j = from;
+    for (; j + 4 <= to; j += 4) {                     // four reads in flight
+      const unsigned long long x0 = s_words[j], x1 = s_words[j + 1], x2 = s_words[j + 2], x3 = s_words[j + 3];
+      rank += (x0 < mine ? 1u : 0u) + (x1 < mine ? 1u : 0u) + (x2 < mine ? 1u : 0u) + (x3 < mine ? 1u : 0u);
+    }
+    for (; j < to; ++j) rank += s_words[j] < mine ? 1u : 0u;
+    sink.store(rank, mine >> idx_bits, static_cast<unsigned>(mine & idx_mask));
+  }
+}
+
 static bool chain_slabs_enabled() {
   static const bool on = [] {
     const char *text = std::getenv("MINUET_CHAIN_SLABS");
@@ -1523,7 +1730,7 @@ size_t chain_sort_words(int64_t n) {
 }
 
 bool chain_sort_takes(int64_t n, int64_t num_batches, int num_offsets) {
-  return n >= kBucketMinN && n <= bucket_sort_max_rows() && n <= (int64_t(1) << 21) && num_batches <= 1 &&
+  return (n <= kSmallSortRows || n <= bucket_sort_max_rows()) && n <= (int64_t(1) << 21) && num_batches <= 1 &&
          num_offsets >= 1 && num_offsets <= kPlanMaxOffsets;
 }
 
@@ -1532,6 +1739,14 @@ static void enqueue_chain_sort_typed(const CT *coords, int64_t n, int ndim, int3
                                      CT *sorted_out, const ChainSortBuffers &buf,
                                      const OffsetTable &offsets, int num_offsets, hipStream_t stream) {
   const int idx_bits = bit_width(static_cast<unsigned long long>(n - 1));
+  if (n <= kSmallSortRows) {
+    small_sort_kernel<CT, int32_t, true><<<1, kSmallSortBlock, 0, stream>>>(
+        coords, nullptr, 1, ndim, static_cast<int>(n), idx_bits, indices_out, sorted_out, SmallSortTell{}, buf.folded,
+        buf.status, buf.counters, buf.counter_words, offsets, num_offsets, buf.plan);
+    check_launch("small_sort_kernel");
+    profile_mark("sort_small", stream);
+    return;
+  }
   const int msd_cap = chain_sort_msd_bits(n);
   const int buckets = 1 << msd_cap;
   const int num_partials = static_cast<int>(std::min<int64_t>(div_ceil(n, kBoundsBlock * 4), kBucketBoundsBlocks));
@@ -1637,7 +1852,30 @@ static void arg_sort_typed(const CT *coords, int64_t n, int ndim, const IT *batc
   // bucket sort, first half: bounds partials, bucket histogram, scan and the
   // dealing step in a row; the scan kernel hands the bounds to the host
   const int batches_in_key = batched ? static_cast<int>(num_batches) : 1;
-  const bool try_buckets = n >= kBucketMinN && n <= bucket_sort_max_rows();
+  if (n <= kSmallSortRows) {
+    Arena &arena = scope.arena();
+    const unsigned long long sequence = arena.next_sequence();
+    char *pinned = static_cast<char *>(arena.pinned_device());
+    const SmallSortTell tell{reinterpret_cast<long long *>(pinned),
+                             reinterpret_cast<unsigned *>(pinned + kBucketHostOffset), arena.flag_device(3), sequence};
+    OffsetTable none;
+    memset(&none, 0, sizeof(none));
+    small_sort_kernel<CT, IT, false><<<1, kSmallSortBlock, 0, stream>>>(
+        coords, batched ? batch_dims : nullptr, batches_in_key, ndim, static_cast<int>(n),
+        bit_width(static_cast<unsigned long long>(n - 1)), indices_out, sorted_out, tell, nullptr, nullptr, nullptr, 0,
+        none, 0, nullptr);
+    check_launch("small_sort_kernel");
+    arena.wait_flag(3, sequence);
+    memcpy(h_bounds, arena.pinned(), sizeof(long long) * 8);
+    const unsigned verdict =
+        *reinterpret_cast<volatile unsigned *>(static_cast<char *>(arena.pinned()) + kBucketHostOffset);
+    profile_mark("sort_small+sync", stream);
+    if (verdict == 0) {
+      if (bounds_host_out != nullptr) memcpy(bounds_host_out, h_bounds, sizeof(long long) * 8);
+      return;
+    }
+  }
+  const bool try_buckets = n > kSmallSortRows && n <= bucket_sort_max_rows();
   const int idx_bits = bit_width(static_cast<unsigned long long>(n - 1));
   const int msd_cap = std::max(1, std::min(kBucketMaxBits, bit_width(static_cast<unsigned long long>(n / kBucketRows))));
   unsigned *bucket_starts = nullptr;
@@ -1689,7 +1927,7 @@ static void arg_sort_typed(const CT *coords, int64_t n, int ndim, const IT *batc
     check_launch("bucket_deal_kernel");
     arena.wait_flag(3, sequence);
     memcpy(h_bounds, arena.pinned(), sizeof(long long) * 8);
-  } else {
+  } else if (n > kSmallSortRows) {
     read_bounds(coords, n, nullptr, 0, ndim, sizeof(CT) == 4 ? MNT_INT32 : MNT_INT64, h_bounds, scope, stream);
   }
   if (bounds_host_out != nullptr) memcpy(bounds_host_out, h_bounds, sizeof(long long) * 8);

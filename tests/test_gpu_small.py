@@ -1,0 +1,55 @@
+"""Clouds around one workgroup: the sort in one launch and the split look-up of the chain."""
+import numpy as np
+import pytest
+
+import c_oracle
+import minuet_oracle as orc
+from helpers import dev, host, random_cloud, sorted_unique
+from minuet_amd.nn.functional import _C
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 1023, 1025, 4095, 4096, 4097])
+@pytest.mark.parametrize("shape", ["spread", "equal rows", "one column", "wide", "batched"])
+def test_sort_around_one_workgroup(n, shape):
+    rng = np.random.default_rng(n)
+    bd = None
+    if shape == "spread":
+        c = random_cloud(n, 200, n, lo=-100)
+    elif shape == "equal rows":                     # far more equal keys than a part takes
+        c = np.repeat(random_cloud(2, 5, n), n, axis=0)[rng.permutation(2 * n)[:n]]
+    elif shape == "one column":                     # the top bits agree
+        c = random_cloud(n, 3, n)
+        c[:, 2] = rng.integers(-3000, 3000, size=n)
+        c[0] = (1 << 20, 0, 0)
+    elif shape == "wide":                           # no room for the row index beside the key
+        c = rng.integers(-2 ** 20, 2 ** 20, size=(n, 3)).astype(np.int64)
+    else:
+        c = random_cloud(n, 30, n)
+        bd = np.concatenate([[0], np.sort(rng.integers(0, n + 1, size=4)), [n]]).astype(np.int64)
+    index, rows, bounds = _C.sort_coordinates(dev(c), dev(bd), return_bounds=True)
+    order = orc.arg_sort_coordinates(c, bd)
+    np.testing.assert_array_equal(host(index).astype(np.int64), order)
+    np.testing.assert_array_equal(host(rows), c[order])
+    np.testing.assert_array_equal(bounds[:3], c.min(0))
+    np.testing.assert_array_equal(bounds[4:7], c.max(0))
+
+
+@pytest.mark.parametrize("n", [1, 5, 511, 513, 2039, 4096, 4500])
+@pytest.mark.parametrize("kernel,extent,halves", [(3, 16, True), (3, 400, True), (2, 16, False)])
+def test_map_lists_of_small_clouds(n, kernel, extent, halves):
+    c, _ = sorted_unique(random_cloud(n, extent, n + kernel, lo=-extent // 2))
+    c = c[np.random.default_rng(n).permutation(c.shape[0])]
+    off = orc.generate_kernel_offsets(3, kernel, 1, 1)
+    index, rows, built = _C.sorted_kernel_map_lists(dev(c), off.astype(np.int64))
+    order = orc.arg_sort_coordinates(c)
+    np.testing.assert_array_equal(host(index).astype(np.int64), order)
+    np.testing.assert_array_equal(host(rows), c[order])
+    ref = c_oracle.query(c[order], c[order], off.astype(np.int32))
+    sizes = orc.compute_kernel_map_sizes(ref)
+    by_size = orc.stable_size_order(sizes)
+    ein, eout, _ = orc.kernel_map_pair_lists(ref[by_size])
+    np.testing.assert_array_equal(built["sizes_host"], np.asarray(sizes)[by_size])
+    np.testing.assert_array_equal(host(built["in_idx"]), ein)
+    np.testing.assert_array_equal(host(built["out_idx"]), eout)
