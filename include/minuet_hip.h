@@ -579,6 +579,28 @@ int mnt_sparse_convolution_forward_implicit(const void *sources, const void *wei
                                             const void *packed_weights,
                                             void *out, void *stream);
 
+/* Tiles of a dense kernel map (at most 128 offsets): its targets put in the
+ * order of the sets of offsets they have a source under, in tiles of 128, with
+ * each tile's live offsets and their source rows.  tiles_out holds
+ * mnt_kernel_map_tiles_size int32 words, 16-byte aligned.  Waits for nothing.
+ * mnt_kernel_map_tiles_share: the part of that work's time that one forward of
+ * the given shape saves by them, 0 where they do not pay or are not taken.  The
+ * reference has no counterpart. */
+int mnt_kernel_map_tiles_size(int64_t num_targets, int64_t num_offsets, int64_t *ints_out);
+int mnt_kernel_map_tiles(const int32_t *kernel_map, int64_t num_targets, int64_t num_offsets,
+                         int32_t *tiles_out, void *stream);
+double mnt_kernel_map_tiles_share(int64_t num_targets, int64_t num_offsets, int64_t num_source_features,
+                                  int64_t num_target_features, int float_dtype);
+
+/* mnt_sparse_convolution_forward_implicit for 16-bit features from the tiles of
+ * the kernel map; the weights packed (mnt_pack_weights), no narrow rows. */
+int mnt_sparse_convolution_forward_tiled(const void *sources, const void *packed_weights, const int32_t *tiles,
+                                         int64_t num_sources, int64_t num_targets, int64_t num_offsets,
+                                         int64_t num_source_features, int64_t num_target_features,
+                                         int float_dtype, const float *channel_scale,
+                                         const float *channel_shift, const void *residual, int activation,
+                                         float negative_slope, void *out, void *stream);
+
 /* The dense kernel map of the transposed layer that shares a forward layer's
  * map (minuet/nn/convolutions.py:119-133 reuses the forward map with the rank
  * tables swapped): inverse_out[O, S] with inverse_out[o][m] = t wherever

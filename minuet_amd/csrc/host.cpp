@@ -18,6 +18,7 @@
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/core/GradMode.h>
 #include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 
 #include <cstdint>
@@ -35,11 +36,20 @@ using TablesFn = int (*)(int64_t, int64_t, int, int64_t, int, double, const void
                          const void *, const void *, const void *, const int64_t *, int64_t, int64_t, int64_t,
                          int64_t, int64_t, int, int, const int32_t *, const float *, const float *, const void *,
                          int, float, const void *, const int64_t *, void *, void *);
+using TiledFn = int (*)(const void *, const void *, const int32_t *, int64_t, int64_t, int64_t, int64_t, int64_t, int,
+                        const float *, const float *, const void *, int, float, void *, void *);
+using TilesFn = int (*)(const int32_t *, int64_t, int64_t, int32_t *, void *);
+using TilesSizeFn = int (*)(int64_t, int64_t, int64_t *);
+using TilesShareFn = double (*)(int64_t, int64_t, int64_t, int64_t, int);
 using ErrorFn = const char *(*)();
 
 ImplicitFn g_implicit = nullptr;
 GroupsFn g_groups = nullptr;
 TablesFn g_tables = nullptr;
+TiledFn g_tiled = nullptr;
+TilesFn g_tiles = nullptr;
+TilesSizeFn g_tiles_size = nullptr;
+TilesShareFn g_tiles_share = nullptr;
 ErrorFn g_error = nullptr;
 
 // ------------------------------------------------------------ Python objects ----
@@ -127,6 +137,10 @@ struct MapEntry {
   // any layer has used it.
   const void *built_from;
   char used;
+  // Tiles of the map (kind kImplicit; null until they are made) and what they
+  // would have saved so far, over what making them takes (below 0: never).
+  PyObject *tiles;
+  double tiles_credit;
 };
 
 void map_entry_dealloc(PyObject *self) {
@@ -135,6 +149,7 @@ void map_entry_dealloc(PyObject *self) {
   Py_XDECREF(e->stride);
   Py_XDECREF(e->batch_dims);
   Py_XDECREF(e->keep);
+  Py_XDECREF(e->tiles);
   Py_TYPE(self)->tp_free(self);
 }
 
@@ -164,6 +179,8 @@ PyObject *map_entry_new(PyTypeObject *type, PyObject *args, PyObject *) {
   e->num_targets = num_targets;
   e->built_from = reinterpret_cast<const void *>(static_cast<uintptr_t>(built_from));
   e->used = 0;
+  e->tiles = nullptr;
+  e->tiles_credit = 0.0;
   for (Py_ssize_t i = 0; i < 8; ++i) {
     e->at[i] = nullptr;
     if (i < PyTuple_GET_SIZE(pointers) && !is_none(PyTuple_GET_ITEM(pointers, i))) {
@@ -289,6 +306,43 @@ inline bool vector_fits(const at::Tensor *t, int64_t channels, int device) {
          t->is_cuda() && t->device().index() == device;
 }
 
+// The tiles of a layer's map, or null where the layer runs without.  Tiles cost
+// two or more forwards to make and are kept with the map, so they are made once
+// the forwards that have run over it would have saved twice their price: a map
+// that a network reads a few times and drops never pays for them, one that is
+// read on and on soon does.
+constexpr double kTilesCredit = 2.0;
+constexpr int64_t kTilesMostInts = int64_t{1} << 29;
+
+const at::Tensor *tiles_of(MapEntry *map, const Layer *l, int64_t T, const at::Device &device, void *stream) {
+  if (map->tiles != nullptr) return tensor_of(map->tiles);
+  if (map->tiles_credit < 0.0) return nullptr;
+  const double share = g_tiles_share(T, l->num_offsets, l->in_channels, l->out_channels, l->float_code);
+  if (share == 0.0) return nullptr;
+  map->tiles_credit += share;
+  if (map->tiles_credit < kTilesCredit) return nullptr;
+  if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return nullptr;
+  map->tiles_credit = -1.0;
+  int64_t ints = 0;
+  if (g_tiles_size(T, l->num_offsets, &ints) != 0 || ints > kTilesMostInts) return nullptr;
+  at::Tensor tiles;
+  try {
+    tiles = at::detail::empty_cuda({ints}, at::kInt, device, std::nullopt);
+  } catch (const std::exception &) {                     // no room: the layer runs without
+    return nullptr;
+  }
+  if (g_tiles(static_cast<const int32_t *>(map->at[0]), T, l->num_offsets,
+              static_cast<int32_t *>(tiles.mutable_data_ptr()), stream) != 0) {
+    return nullptr;
+  }
+  map->tiles = THPVariable_Wrap(std::move(tiles));
+  if (map->tiles == nullptr) {
+    PyErr_Clear();
+    return nullptr;
+  }
+  return tensor_of(map->tiles);
+}
+
 PyObject *none() { Py_RETURN_NONE; }
 
 // The layer on `inputs`; None when anything is not as the Layer describes it.
@@ -393,6 +447,12 @@ PyObject *run_layer(Layer *l, PyObject *module_dict, PyObject *inputs, const Epi
   int status = 0;
   switch (l->kind) {
     case kImplicit:
+      if (const at::Tensor *tiles = tiles_of(map, l, T, kernel.device(), stream)) {
+        status = g_tiled(source, packed_at, static_cast<const int32_t *>(tiles->const_data_ptr()), S, T,
+                         l->num_offsets, l->in_channels, l->out_channels, l->float_code, scale_at, shift_at,
+                         data(residual), ep.activation, ep.slope, out.mutable_data_ptr(), stream);
+        break;
+      }
       status = g_implicit(source, weights_at, static_cast<const int32_t *>(map->at[0]), S, T, l->num_offsets,
                           l->in_channels, l->out_channels, l->float_code, scale_at, shift_at, data(residual),
                           ep.activation, ep.slope, packed_at, out.mutable_data_ptr(), stream);
@@ -636,6 +696,10 @@ PyObject *py_bind(PyObject *, PyObject *args) {
   g_implicit = reinterpret_cast<ImplicitFn>(address("mnt_sparse_convolution_forward_implicit"));
   g_groups = reinterpret_cast<GroupsFn>(address("mnt_sparse_convolution_forward_groups"));
   g_tables = reinterpret_cast<TablesFn>(address("mnt_sparse_convolution_forward_fused"));
+  g_tiled = reinterpret_cast<TiledFn>(address("mnt_sparse_convolution_forward_tiled"));
+  g_tiles = reinterpret_cast<TilesFn>(address("mnt_kernel_map_tiles"));
+  g_tiles_size = reinterpret_cast<TilesSizeFn>(address("mnt_kernel_map_tiles_size"));
+  g_tiles_share = reinterpret_cast<TilesShareFn>(address("mnt_kernel_map_tiles_share"));
   g_error = reinterpret_cast<ErrorFn>(address("mnt_last_error"));
   if (PyErr_Occurred()) return nullptr;
   g_sparse_tensor = reinterpret_cast<PyTypeObject *>(sparse_tensor);

@@ -26,8 +26,14 @@
 
 #include "conv_device.h"
 #include "device_utils.h"
+#include "implicit.h"
+#include "tiles.h"
 
 namespace mnt {
+
+template <typename T>
+void tiled_forward(const T *sources, const T *packed, const int *kernel_map, const int *tiles, int64_t S, int64_t Tn,
+                   int64_t O, int64_t K, int64_t N, const Epilogue &ep, T *out, hipStream_t stream);
 
 constexpr int kImplicitBlock = 256;
 constexpr int kImplicitTargets = 128;     // per workgroup, 32 per wavefront
@@ -56,128 +62,6 @@ typedef unsigned uint4v __attribute__((ext_vector_type(4)));
 // Source tensors stay below this many bytes: rows are addressed through 32-bit
 // buffer offsets.
 constexpr unsigned kMaxSourceBytes = 0xFFFFF000u;
-
-// One output row's worth of epilogue and store: four consecutive channels of
-// target t held by this lane.
-template <typename T>
-__device__ __forceinline__ void finish_four(float (&v)[4], const Epilogue &ep, long long t, int ch, int N,
-                                            unsigned char *__restrict__ out) {
-  typedef typename VecOf<4 * sizeof(T)>::type V;
-  if (ep.scale != nullptr) {
-#pragma unroll
-    for (int x = 0; x < 4; ++x) v[x] *= ep.scale[ch + x];
-  }
-  if (ep.shift != nullptr) {
-#pragma unroll
-    for (int x = 0; x < 4; ++x) v[x] += ep.shift[ch + x];
-  }
-  if (ep.residual != nullptr) {
-    const V raw = *reinterpret_cast<const V *>(static_cast<const unsigned char *>(ep.residual) +
-                                               (t * N + ch) * static_cast<long long>(sizeof(T)));
-    const T *e = reinterpret_cast<const T *>(&raw);
-#pragma unroll
-    for (int x = 0; x < 4; ++x) v[x] += to_float(e[x]);
-  }
-  if (ep.activation == MNT_ACT_RELU) {
-#pragma unroll
-    for (int x = 0; x < 4; ++x) v[x] = fmaxf(v[x], 0.0f);
-  } else if (ep.activation == MNT_ACT_LEAKY_RELU) {
-#pragma unroll
-    for (int x = 0; x < 4; ++x) v[x] = v[x] > 0.0f ? v[x] : v[x] * ep.slope;
-  } else if (ep.activation == MNT_ACT_RELU6) {
-#pragma unroll
-    for (int x = 0; x < 4; ++x) v[x] = fminf(fmaxf(v[x], 0.0f), 6.0f);
-  }
-  V raw;
-  T *e = reinterpret_cast<T *>(&raw);
-#pragma unroll
-  for (int x = 0; x < 4; ++x) e[x] = static_cast<T>(v[x]);
-  *reinterpret_cast<V *>(out + (t * N + ch) * static_cast<long long>(sizeof(T))) = raw;
-}
-
-// The same for one 16-byte piece of an output row (E = 16 / sizeof(T)
-// consecutive channels from `ch` on), its sums given in fp32.
-template <typename T, int E>
-__device__ __forceinline__ void finish_piece(float (&v)[E], const Epilogue &ep, long long t, int ch, int N,
-                                             unsigned char *__restrict__ out) {
-  if (ep.scale != nullptr) {
-#pragma unroll
-    for (int x = 0; x < E; ++x) v[x] *= ep.scale[ch + x];
-  }
-  if (ep.shift != nullptr) {
-#pragma unroll
-    for (int x = 0; x < E; ++x) v[x] += ep.shift[ch + x];
-  }
-  if (ep.residual != nullptr) {
-    const uint4 raw = *reinterpret_cast<const uint4 *>(static_cast<const unsigned char *>(ep.residual) +
-                                                       (t * N + ch) * static_cast<long long>(sizeof(T)));
-    const T *e = reinterpret_cast<const T *>(&raw);
-#pragma unroll
-    for (int x = 0; x < E; ++x) v[x] += to_float(e[x]);
-  }
-  if (ep.activation == MNT_ACT_RELU) {
-#pragma unroll
-    for (int x = 0; x < E; ++x) v[x] = fmaxf(v[x], 0.0f);
-  } else if (ep.activation == MNT_ACT_LEAKY_RELU) {
-#pragma unroll
-    for (int x = 0; x < E; ++x) v[x] = v[x] > 0.0f ? v[x] : v[x] * ep.slope;
-  } else if (ep.activation == MNT_ACT_RELU6) {
-#pragma unroll
-    for (int x = 0; x < E; ++x) v[x] = fminf(fmaxf(v[x], 0.0f), 6.0f);
-  }
-  uint4 raw;
-  T *e = reinterpret_cast<T *>(&raw);
-#pragma unroll
-  for (int x = 0; x < E; ++x) e[x] = static_cast<T>(v[x]);
-  *reinterpret_cast<uint4 *>(out + (t * N + ch) * static_cast<long long>(sizeof(T))) = raw;
-}
-
-// Epilogue and store of one 32 x 32 block of fp32 sums as the matrix
-// instructions leave it (lane (r, h) holds channels q * 8 + h * 4 .. + 3 of
-// target block_t0 + r in acc[q * 4 .. + 3]), for output rows that are whole
-// 16-byte pieces: the wavefront turns the block around in its own `turn` area
-// of LDS (kTurnBytes), so that one store instruction covers rows in contiguous
-// pieces of 64 bytes (128 in fp32), and the residual is read the same way.
-constexpr int kTurnRow = 32 * 4 + 16;
-constexpr int kTurnBytes = 32 * kTurnRow;
-
-template <typename T>
-__device__ __forceinline__ void store_turned_block(const floatx16 &acc, unsigned char *turn, int lane, int r,
-                                                   int h, long long block_t0, long long num_targets, int ch0,
-                                                   int N, const Epilogue &ep, unsigned char *__restrict__ out) {
-  constexpr int EPV = 16 / static_cast<int>(sizeof(T));
-  constexpr int kOutPieces = 32 / EPV;                          // 16-byte pieces of a block's output row
-  constexpr int kPieces = 32 * kOutPieces / 64;                 // per lane
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    *reinterpret_cast<float4 *>(turn + r * kTurnRow + (q * 8 + h * 4) * 4) =
-        make_float4(acc[q * 4], acc[q * 4 + 1], acc[q * 4 + 2], acc[q * 4 + 3]);
-  }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-  for (int i = 0; i < kPieces; ++i) {
-    const int piece = lane + i * 64;
-    const int pr = piece / kOutPieces, part = piece % kOutPieces;
-    const int ch = ch0 + part * EPV;
-    float v[EPV];
-#pragma unroll
-    for (int x = 0; x < EPV; x += 4) {
-      const float4 f = *reinterpret_cast<const float4 *>(turn + pr * kTurnRow + (part * EPV + x) * 4);
-      v[x] = f.x;
-      v[x + 1] = f.y;
-      v[x + 2] = f.z;
-      v[x + 3] = f.w;
-    }
-    if (block_t0 + pr < num_targets && ch < N) {                // N % EPV == 0: a piece is all in or all out
-      finish_piece<T, EPV>(v, ep, block_t0 + pr, ch, N, out);
-    }
-  }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // KS: 32-byte steps of K per pipeline stage.  A source row takes `chunks`
 // stages of KS * 32 bytes (Kp * sizeof(T) must be a multiple of that when
@@ -661,6 +545,18 @@ static void implicit_typed(const T *sources, const T *weights, const T *packed, 
     check_launch("pack_weights_kernel");
     profile_mark("pack_weights", stream);
   }
+  if constexpr (sizeof(T) == 2) {
+    // Up to two workgroups per compute unit tiled_forward_kernel's shorter
+    // stages count, beyond that this kernel's wavefronts that skip offsets of
+    // their own (64 -> 64 channels: 16.3 against 17.7 us at 60 000 targets,
+    // 51.6 and 47.8 at 200 000).
+    if (O > 1 && Tn <= static_cast<int64_t>(2 * kTileTargets) * compute_units() &&
+        O * Np * Kp * static_cast<int64_t>(sizeof(T)) < static_cast<int64_t>(kMaxSourceBytes)) {
+      tiled_forward<T>(sources, wt, kernel_map, nullptr, S, Tn, O, K, N, ep, out, stream);
+      profile_mark("implicit", stream);
+      return;
+    }
+  }
   const unsigned source_bytes = static_cast<unsigned>(S * K * sizeof(T));
   // stage width: 64 bytes for rows up to that, else 128; wider rows go in
   // chunks of 128 bytes (stages of 256 measured two to three times slower:
@@ -787,5 +683,63 @@ extern "C" int mnt_kernel_map_invert(const int32_t *kernel_map, int64_t num_offs
                                                                          total, inverse_out);
       check_launch("invert_map_kernel");
     }
+  });
+}
+
+// What tiles (mnt_kernel_map_tiles) would save of one forward, over what making
+// them takes; 0 where they do not pay or cannot be used.  Fitted to layers of
+// 32 to 128 channels over 100 000 to a million targets: a forward gets faster by
+// 1.1 us per million (offset, target) pairs and unit of (channel blocks + 1) x
+// 128-byte pieces of a row, making tiles takes 28 us and 2.5 us per million pairs.
+extern "C" double mnt_kernel_map_tiles_share(int64_t T, int64_t O, int64_t K, int64_t N, int float_dtype) {
+  if (float_dtype == MNT_FLOAT32 || O <= 8 || O > kTileMaxOffsets || T < 1 || K < 1 || N < 1 ||
+      (K * 2) % 16 != 0 || K * 2 > kImplicitMaxRowBytes || N % 4 != 0 || N > 32 * kImplicitMaxBlocks * kImplicitMaxGroups ||
+      narrow_fits(O, K, N, 2, true)) {
+    return 0.0;
+  }
+  // Below, the kernel without tiles is about as fast, and it adds up in another
+  // order: a layer's results do not change from one call to the next.
+  if (T <= static_cast<int64_t>(2 * kTileTargets) * compute_units()) return 0.0;
+  const double pairs = 1e-6 * static_cast<double>(T) * static_cast<double>(O);
+  const double pieces = K * 2 <= 64 ? 0.5 : static_cast<double>(div_ceil(K * 2, 128));
+  return 1.1 * pairs * static_cast<double>(div_ceil(N, 32) + 1) * pieces / (28.0 + 2.5 * pairs);
+}
+
+extern "C" int mnt_sparse_convolution_forward_tiled(
+    const void *sources, const void *packed_weights, const int32_t *tiles, int64_t S, int64_t T, int64_t O,
+    int64_t K, int64_t N, int float_dtype, const float *channel_scale, const float *channel_shift,
+    const void *residual, int activation, float negative_slope, void *out, void *stream_) {
+  return guarded([&] {
+    hipStream_t stream = static_cast<hipStream_t>(stream_);
+    MNT_CHECK(S >= 0 && T >= 0 && O >= 1 && K >= 1 && N >= 1 && S <= INT32_MAX && T <= INT32_MAX && O <= kTileMaxOffsets,
+              "bad shape S=%lld T=%lld O=%lld Cin=%lld Cout=%lld", (long long)S, (long long)T,
+              (long long)O, (long long)K, (long long)N);
+    MNT_CHECK(float_dtype == MNT_FLOAT16 || float_dtype == MNT_BFLOAT16, "the tiled forward takes 16-bit features");
+    MNT_CHECK(S * K * 2 < static_cast<int64_t>(kMaxSourceBytes),
+              "source features of %lld bytes exceed the 4 GiB a buffer resource addresses", (long long)(S * K * 2));
+    MNT_CHECK(K % 8 == 0 && K * 2 <= kImplicitMaxRowBytes && N % 4 == 0 && N <= 32 * kImplicitMaxBlocks * kImplicitMaxGroups,
+              "Unsupported channel counts for the tiled forward: Cin = %lld (a multiple of 8, at most %d), "
+              "Cout = %lld (a multiple of 4, at most %d)", (long long)K, kImplicitMaxRowBytes / 2, (long long)N,
+              32 * kImplicitMaxBlocks * kImplicitMaxGroups);
+    MNT_CHECK(activation >= MNT_ACT_NONE && activation <= MNT_ACT_RELU6, "unknown activation code %d", activation);
+    MNT_CHECK(reinterpret_cast<uintptr_t>(sources) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0 &&
+                  reinterpret_cast<uintptr_t>(residual) % 16 == 0 &&
+                  reinterpret_cast<uintptr_t>(packed_weights) % 16 == 0 &&
+                  reinterpret_cast<uintptr_t>(tiles) % 16 == 0 &&
+                  reinterpret_cast<uintptr_t>(channel_scale) % 4 == 0 &&
+                  reinterpret_cast<uintptr_t>(channel_shift) % 4 == 0,
+              "operands are not aligned (features, out, residual, weights, tiles: 16 bytes, scale / shift: 4 bytes)");
+    if (T == 0) return;
+    MNT_CHECK(out != nullptr && tiles != nullptr && packed_weights != nullptr, "null operand");
+    profile_mark("enter:implicit", stream);
+    const Epilogue ep = {channel_scale, channel_shift, residual, activation, negative_slope, nullptr};
+    if (float_dtype == MNT_FLOAT16) {
+      tiled_forward<half_t>(static_cast<const half_t *>(sources), static_cast<const half_t *>(packed_weights), nullptr,
+                            tiles, S, T, O, K, N, ep, static_cast<half_t *>(out), stream);
+    } else {
+      tiled_forward<bf16_t>(static_cast<const bf16_t *>(sources), static_cast<const bf16_t *>(packed_weights), nullptr,
+                            tiles, S, T, O, K, N, ep, static_cast<bf16_t *>(out), stream);
+    }
+    profile_mark("implicit", stream);
   });
 }

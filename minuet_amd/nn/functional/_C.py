@@ -103,6 +103,11 @@ SIGNATURES = {
     "mnt_sparse_convolution_forward_groups": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int,
                                                      _vp, _vp, _vp, _int, _c.c_float, _vp, _vp]),
     "mnt_pack_weights": (_int, [_vp, _i64, _i64, _i64, _int, _vp, _vp]),
+    "mnt_kernel_map_tiles_size": (_int, [_i64, _i64, ctypes.POINTER(_i64)]),
+    "mnt_kernel_map_tiles": (_int, [_vp, _i64, _i64, _vp, _vp]),
+    "mnt_kernel_map_tiles_share": (ctypes.c_double, [_i64, _i64, _i64, _i64, _int]),
+    "mnt_sparse_convolution_forward_tiled": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _vp, _vp, _vp,
+                                                    _int, ctypes.c_float, _vp, _vp]),
     "mnt_sparse_convolution_forward_implicit": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64,
                                                        _int, _vp, _vp, _vp, _int, _c.c_float, _vp,
                                                        _vp, _vp]),
@@ -168,7 +173,8 @@ def load_host():
     module = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(module)
     names = ("mnt_sparse_convolution_forward_implicit", "mnt_sparse_convolution_forward_groups",
-             "mnt_sparse_convolution_forward_fused", "mnt_last_error")
+             "mnt_sparse_convolution_forward_fused", "mnt_sparse_convolution_forward_tiled", "mnt_kernel_map_tiles",
+             "mnt_kernel_map_tiles_size", "mnt_kernel_map_tiles_share", "mnt_last_error")
     hooks = tuple(getattr(torch_module, name) for name in (
         "_global_forward_hooks", "_global_forward_pre_hooks", "_global_backward_hooks",
         "_global_backward_pre_hooks"))
@@ -1473,6 +1479,56 @@ def sparse_convolution_forward_implicit(sources: torch.Tensor, weights: torch.Te
             _ptr(sources), _ptr(weights), _ptr(kernel_map), S, T, O, K, N, fcode, _ptr(ep.scale),
             _ptr(ep.shift), _ptr(ep.residual), ACTIVATION_CODES[ep.activation],
             float(ep.negative_slope), _ptr(packed_weights), _ptr(out), _stream(device)))
+    return out
+
+
+def kernel_map_tiles(kernel_map: torch.Tensor) -> torch.Tensor:
+    """The tiles of a dense kernel map ``[O, N_out]`` (int32, at most 128
+    offsets): its targets in the order of the sets of offsets they use, what
+    ``sparse_convolution_forward_tiled`` walks."""
+    _ensure_ndim("kernel_map", kernel_map, 2)
+    if kernel_map.dtype != torch.int32:
+        _fail("tiles are made of an int32 kernel map")
+    device = _common_device([kernel_map])
+    O, T = kernel_map.shape
+    size = ctypes.c_int64()
+    _check(load_library().mnt_kernel_map_tiles_size(T, O, ctypes.byref(size)))
+    tiles = torch.empty(size.value, dtype=torch.int32, device=device)
+    kernel_map = kernel_map.contiguous()
+    with _on(device):
+        _check(load_library().mnt_kernel_map_tiles(_ptr(kernel_map), T, O, _ptr(tiles), _stream(device)))
+    return tiles
+
+
+def sparse_convolution_forward_tiled(sources: torch.Tensor, weights: torch.Tensor, tiles: torch.Tensor,
+                                     num_targets: int, packed_weights: torch.Tensor,
+                                     epilogue: Optional[Epilogue] = None) -> torch.Tensor:
+    """``sparse_convolution_forward_implicit`` for 16-bit features from the tiles of
+    the kernel map (``kernel_map_tiles``): the same sums, without the matrix work
+    on offsets that none of a tile's targets has a source under."""
+    _ensure_ndim("sources", sources, 2)
+    _ensure_ndim("weights", weights, 3)
+    _ensure_dim("sources", sources, 1, weights.shape[1])
+    device = _common_device([sources, weights, tiles, packed_weights])
+    dtype = weights.dtype
+    if sources.dtype != dtype:
+        _fail(f"Found tensors with two different scalar types ({sources.dtype} != {dtype})")
+    O, K, N = weights.shape
+    size = ctypes.c_int64()
+    _check(load_library().mnt_kernel_map_tiles_size(num_targets, O, ctypes.byref(size)))
+    if tiles.dtype != torch.int32 or tiles.numel() != size.value or not tiles.is_contiguous():
+        _fail("the tiles are not those of a map of that many targets and offsets")
+    _check_packed(packed_weights, weights)
+    sources = sources.contiguous()
+    if sources.data_ptr() % 16:
+        sources = sources.clone()
+    out = torch.empty((num_targets, N), dtype=dtype, device=device)
+    ep = Epilogue() if epilogue is None else epilogue.checked(num_targets, N, dtype, device)
+    with _on(device):
+        _check(load_library().mnt_sparse_convolution_forward_tiled(
+            _ptr(sources), _ptr(packed_weights), _ptr(tiles), sources.shape[0], num_targets, O, K, N,
+            _float_code(dtype, "sparse_convolution_forward_tiled"), _ptr(ep.scale), _ptr(ep.shift), _ptr(ep.residual),
+            ACTIVATION_CODES[ep.activation], float(ep.negative_slope), _ptr(out), _stream(device)))
     return out
 
 

@@ -1,0 +1,112 @@
+"""The output-stationary forward with and without tiles of targets that share
+their live offsets, against a plain fp32 product per offset."""
+import pytest
+import torch
+
+import minuet_amd as minuet
+from minuet_amd.nn import functional as F
+from minuet_amd.nn.functional import _C
+
+pytestmark = pytest.mark.gpu
+DEVICE = "cuda:0"
+
+
+def random_map(targets, sources, offsets, density, seed):
+    """A map whose targets use few offsets each, some of them none at all."""
+    gen = torch.Generator(device=DEVICE).manual_seed(seed)
+    index = torch.randint(0, sources, (offsets, targets), generator=gen, device=DEVICE, dtype=torch.int32)
+    liking = torch.rand(offsets, 1, generator=gen, device=DEVICE) * 2 * density
+    hit = torch.rand(offsets, targets, generator=gen, device=DEVICE) < liking
+    hit &= torch.rand(targets, generator=gen, device=DEVICE) > 0.1
+    return torch.where(hit, index, torch.full_like(index, -1))
+
+
+def reference(x, w, dense):
+    out = torch.zeros(dense.shape[1], w.shape[2], device=x.device)
+    for o in range(dense.shape[0]):
+        rows = x.float()[dense[o].clamp(min=0).long()] * (dense[o] >= 0)[:, None]
+        out += rows @ w[o].float()
+    return out
+
+
+def operands(targets, sources, offsets, cin, cout, dtype, seed=0, density=0.3):
+    gen = torch.Generator(device=DEVICE).manual_seed(seed + 1)
+    dense = random_map(targets, sources, offsets, density, seed)
+    x = torch.randn(sources, cin, generator=gen, device=DEVICE).to(dtype)
+    w = (torch.randn(offsets, cin, cout, generator=gen, device=DEVICE) / (cin * offsets * density) ** 0.5).to(dtype)
+    return dense, x, w
+
+
+def close(got, wanted, dtype):
+    bound = 4e-3 if dtype == torch.float16 else 2e-2
+    assert float((got.float() - wanted).norm() / wanted.norm().clamp(min=1e-6)) < bound
+
+
+# one target, tiles of one short of, exactly and one more than 128, several windows of 4 096 per die
+@pytest.mark.parametrize("targets,offsets", [(1, 27), (127, 27), (128, 9), (1025, 27), (5000, 33), (33000, 27),
+                                             (33000, 125), (2000, 128), (2000, 49), (2000, 50)])
+def test_tiles_are_the_targets(targets, offsets):
+    dense = random_map(targets, targets, offsets, 0.2, 5)
+    tiles = _C.kernel_map_tiles(dense).cpu()
+    windows = 8 * max(1, -(-targets // (8 * 4096)))
+    per_window = -(--(-targets // windows) // 128)
+    count = windows * per_window
+    rows, counts = tiles[:count * 128].view(count, 128), tiles[count * 128:count * 129]
+    offsets_at = count * 128 + -(-count // 4) * 4
+    numbers = tiles[offsets_at:offsets_at + count * offsets].view(count, offsets)
+    sources = tiles[offsets_at + -(-(count * offsets) // 4) * 4:].view(count, offsets, 128)
+    assert torch.equal(torch.sort(rows[rows >= 0])[0], torch.arange(targets, dtype=torch.int32))
+    dense = dense.cpu()
+    for t in range(count):
+        live, mine = int(counts[t]), rows[t]
+        assert (live == 0) == bool((mine < 0).all())
+        if live == 0:
+            continue
+        there = mine >= 0
+        entries = torch.where(there, dense[:, mine.clamp(min=0).long()], torch.tensor(-1, dtype=torch.int32))
+        used = torch.nonzero((entries >= 0).any(1))[:, 0].int()
+        assert torch.equal(numbers[t, :live], used if used.numel() else torch.zeros(1, dtype=torch.int32))
+        assert torch.equal(sources[t, :live], entries[numbers[t, :live].long()])
+
+
+# rows of one, two and a ragged number of 16-byte pieces, of one stage and of several; channel
+# blocks one to four and two groups; outputs that are no whole pieces; each number of workgroups
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("targets,offsets,cin,cout", [
+    (1, 27, 64, 64), (129, 27, 64, 64), (5000, 27, 32, 32), (5000, 27, 24, 12), (5000, 8, 16, 96), (20000, 27, 48, 64),
+    (20000, 2, 72, 128), (3000, 27, 128, 160), (3000, 33, 200, 36), (40000, 27, 64, 96), (66000, 9, 64, 128),
+    (90000, 27, 32, 32), (90000, 27, 40, 64), (300000, 3, 64, 64), (2000, 125, 64, 32)])
+def test_forward_matches_products(targets, offsets, cin, cout, dtype):
+    dense, x, w = operands(targets, 3000, offsets, cin, cout, dtype)
+    packed = F.pack_weights(w)
+    wanted = reference(x, w, dense)
+    close(_C.sparse_convolution_forward_implicit(x, w, dense, packed_weights=packed), wanted, dtype)
+    tiles = _C.kernel_map_tiles(dense)
+    close(_C.sparse_convolution_forward_tiled(x, w, tiles, targets, packed), wanted, dtype)
+    gen = torch.Generator(device=DEVICE).manual_seed(9)
+    scale, shift = (torch.randn(cout, generator=gen, device=DEVICE) for _ in range(2))
+    residual = torch.randn(targets, cout, generator=gen, device=DEVICE).to(dtype)
+    epilogue = F.Epilogue(scale, shift, residual, "relu", 0.0)
+    wanted = torch.relu(wanted * scale + shift + residual.float())
+    close(_C.sparse_convolution_forward_implicit(x, w, dense, epilogue=epilogue, packed_weights=packed), wanted, dtype)
+    close(_C.sparse_convolution_forward_tiled(x, w, tiles, targets, packed, epilogue=epilogue), wanted, dtype)
+
+
+@pytest.mark.parametrize("cin,cout,dtype", [(64, 64, torch.float16), (32, 32, torch.bfloat16), (24, 96, torch.float16),
+                                            (128, 64, torch.float16)])
+def test_layer_comes_to_use_tiles(cin, cout, dtype):
+    """A map that is read on and on gets tiles; the layer's results stay bit for bit."""
+    gen = torch.Generator(device=DEVICE).manual_seed(3)
+    cells = torch.randperm(1 << 20, generator=gen, device=DEVICE)[:100000]
+    coordinates = torch.stack([cells >> 13, (cells >> 6) & 127, cells & 63], 1).int()
+    coordinates = coordinates[F.build_sorted_index(coordinates)]
+    conv = minuet.nn.SparseConv3d(cin, cout, 3, dtype=dtype, device=DEVICE)
+    minuet.set_kernel_map_cache(conv, minuet.nn.KernelMapCache(3, torch.int32, DEVICE))
+    x = minuet.SparseTensor(torch.randn(100000, cin, generator=gen, device=DEVICE).to(dtype), coordinates)
+    with torch.no_grad():
+        first = conv(x).F
+        held = torch.cuda.memory_allocated()
+        for _ in range(60):
+            last = conv(x).F
+        assert torch.cuda.memory_allocated() > held + 100000 * 27 * 4      # the tiles
+    assert torch.equal(last, first)
