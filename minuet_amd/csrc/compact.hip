@@ -1,0 +1,278 @@
+// Output-stationary forward of an fp32 sparse convolution that multiplies hits
+// only: Gather -> GEMM -> Scatter
+// (csrc/minuet/cuda/functions/sparse_convolution.cu:504-661) in one kernel from
+// the dense kernel map, without buffer rows and without rank tables.
+#include <algorithm>
+
+#include "conv_device.h"
+#include "device_utils.h"
+#include "implicit.h"
+
+namespace mnt {
+
+constexpr unsigned kCompactNowhere = 0xFFFFF000u;   // past the end of every buffer: reads zeros
+
+typedef unsigned uint4v __attribute__((ext_vector_type(4)));
+typedef unsigned uint2v __attribute__((ext_vector_type(2)));
+
+template <int C>
+struct Floats {
+  float v[C];
+} __attribute__((aligned(4 * C)));
+
+struct CompactShape {
+  long long num_targets;
+  int num_offsets, K, N;
+  int chunks;                  // units of KI * 16 input channels
+};
+
+// A workgroup takes 64 targets and 16 * C output channels; its SPLIT wavefronts
+// take every SPLIT-th offset each.  fp32 matrix instructions are 16 times dearer
+// than 16-bit ones, so nothing but hits is multiplied: a wavefront lists the
+// hits of its offsets, 16 rows of one offset at a time are multiplied by
+// 16 x 16 x 4 instructions (K in pieces of 16 channels, KI of them per unit),
+// and the sums of their targets, which stand in LDS, go in and come out as the
+// instruction's accumulators.  Every wavefront has sums of its own; they are
+// added up in the order of the wavefronts at the end, so that a result is the
+// same whenever it is computed.
+//
+// What bounds it: on small clouds one wavefront's chain of map entry, source
+// rows, products (the unit after is asked for before one is multiplied), hence
+// the split; beyond, the weights, which every 16 rows read again: where
+// targets x input x output channels pass 75 million the three-kernel form is
+// the faster one again (see prefers_implicit).  fp32, 3 x 3 x 3, us a layer in
+// three kernels and here: 32 -> 32 channels over 3 000 voxels 11.4 / 5.7,
+// 20 000 17.9 / 11.3, 200 000 76 / 52; 64 -> 64 over 3 000 12.1 / 8.4, 12 000
+// 18.8 / 14.9; 128 -> 128 over 800 19.5 / 12.8.  (128 targets per workgroup
+// fill the 16 rows better, but their sums leave fewer wavefronts to a compute
+// unit: 17 to 40 % slower.)
+template <int C, int KI, int SPLIT, bool WHOLE>
+__global__ __launch_bounds__(64 * SPLIT) void compact_forward_kernel(
+    const float *__restrict__ sources, unsigned source_bytes, const float *__restrict__ weights,
+    unsigned weight_bytes, const int *__restrict__ kernel_map, CompactShape s, unsigned char *__restrict__ out,
+    Epilogue ep) {
+  constexpr int kCompactBatch = 32 / SPLIT;                // offsets whose hits a wavefront lists together
+  constexpr int kTargets = 64;
+  constexpr int kMost = kCompactBatch * kTargets;          // list entries
+  constexpr int kAccRow = 16 * C + 4;
+  struct Lists {
+    int source[kMost];
+    int offset[kMost / 16];
+    unsigned char target[kMost];
+  };
+  __shared__ __align__(16) float s_acc[SPLIT][(kTargets + 1) * kAccRow];
+  __shared__ __align__(16) Lists s_lists[SPLIT];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15;
+  const int q = lane >> 4;
+  const long long first = static_cast<long long>(blockIdx.x) * kTargets;
+  const int channel = blockIdx.y * 16 * C;
+  const int chunks = s.chunks;
+  float *const acc = s_acc[wv];
+  Lists &lists = s_lists[wv];
+
+  const __amdgpu_buffer_rsrc_t source_buffer = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float *>(sources), 0, source_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t weight_buffer = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float *>(weights), 0, weight_bytes, 0x00020000);
+  const unsigned row_bytes = static_cast<unsigned>(s.K) * 4u;
+  const unsigned line_bytes = static_cast<unsigned>(s.N) * 4u;
+  // lane (r, q) multiplies the C channels r * C .. of the workgroup's 16 * C
+  const bool in_width = channel + r * C < s.N;
+  const unsigned w_at = in_width ? static_cast<unsigned>(q) * 4u * line_bytes + static_cast<unsigned>(channel + r * C) * 4u
+                                 : kCompactNowhere;
+  struct Unit {
+    uint4 a[KI];
+    float w[KI][4][C];
+    unsigned targets;
+  };
+  auto fetch = [&](int g, int c, Unit &u) {
+    const int source = lists.source[g * 16 + r];
+    const int o = __builtin_amdgcn_readfirstlane(lists.offset[g]);
+    u.targets = *reinterpret_cast<const unsigned *>(&lists.target[g * 16 + q * 4]);
+    const unsigned chunk_at = static_cast<unsigned>(c) * (KI * 64u);
+    const unsigned row_at = source >= 0 ? static_cast<unsigned>(source) * row_bytes + q * 16u : kCompactNowhere;
+    const unsigned w_base = static_cast<unsigned>(o) * row_bytes * static_cast<unsigned>(s.N) + chunk_at / 4u * line_bytes;
+#pragma unroll
+    for (int i = 0; i < KI; ++i) {
+      const bool inside = WHOLE || chunk_at + i * 64u + q * 16u < row_bytes;
+      const uint4v v = __builtin_amdgcn_raw_buffer_load_b128(source_buffer, inside ? row_at : kCompactNowhere,
+                                                             chunk_at + i * 64u, 0);
+      u.a[i] = make_uint4(v.x, v.y, v.z, v.w);
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const unsigned at = inside ? w_at : kCompactNowhere;
+        const unsigned from = w_base + (i * 16u + x) * line_bytes;
+        if constexpr (C == 1) {
+          u.w[i][x][0] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(weight_buffer, at, from, 0));
+        } else if constexpr (C == 2) {
+          const uint2v v = __builtin_amdgcn_raw_buffer_load_b64(weight_buffer, at, from, 0);
+          u.w[i][x][0] = __uint_as_float(v.x);
+          u.w[i][x][1] = __uint_as_float(v.y);
+        } else {
+          const uint4v v = __builtin_amdgcn_raw_buffer_load_b128(weight_buffer, at, from, 0);
+          u.w[i][x][0] = __uint_as_float(v.x);
+          u.w[i][x][1] = __uint_as_float(v.y);
+          u.w[i][x][2] = __uint_as_float(v.z);
+          u.w[i][x][3] = __uint_as_float(v.w);
+        }
+      }
+    }
+  };
+  auto multiply = [&](const Unit &u) {
+    float *row[4];
+    floatx4 sum[C];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      row[j] = acc + ((u.targets >> (8 * j)) & 255u) * kAccRow + r * C;
+      const Floats<C> before = *reinterpret_cast<const Floats<C> *>(row[j]);
+#pragma unroll
+      for (int b = 0; b < C; ++b) sum[b][j] = before.v[b];
+    }
+#pragma unroll
+    for (int i = 0; i < KI; ++i) {
+      const float *a = reinterpret_cast<const float *>(&u.a[i]);
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+#pragma unroll
+        for (int b = 0; b < C; ++b) sum[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[x], u.w[i][x][b], sum[b], 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      Floats<C> after;
+#pragma unroll
+      for (int b = 0; b < C; ++b) after.v[b] = sum[b][j];
+      *reinterpret_cast<Floats<C> *>(row[j]) = after;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+
+  for (int first_offset = wv; first_offset < s.num_offsets || first_offset == wv; first_offset += SPLIT * kCompactBatch) {
+    int index[kCompactBatch];
+#pragma unroll
+    for (int j = 0; j < kCompactBatch; ++j) {
+      const long long o = min(first_offset + j * SPLIT, s.num_offsets - 1);
+      index[j] = kernel_map[o * s.num_targets + min(first + lane, s.num_targets - 1)];
+    }
+    if (first_offset == wv) {
+      float4 *const clear = reinterpret_cast<float4 *>(acc);
+      for (int i = lane; i < (kTargets + 1) * kAccRow / 4; i += 64) clear[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
+    int count = 0;
+#pragma unroll
+    for (int j = 0; j < kCompactBatch; ++j) {
+      const int o = first_offset + j * SPLIT;
+      const int from = count;
+      const bool hit = index[j] >= 0 && first + lane < s.num_targets && o < s.num_offsets;
+      const unsigned long long votes = __ballot(hit);
+      if (hit) {
+        const int p = count + __popcll(votes & lanes_below());
+        lists.source[p] = index[j];
+        lists.target[p] = static_cast<unsigned char>(lane);
+      }
+      count += __popcll(votes);
+      const int end = (count + 15) & ~15;      // the rest of 16 rows: no source, a target nobody asks for
+      if (lane < end - count) {
+        lists.source[count + lane] = -1;
+        lists.target[count + lane] = static_cast<unsigned char>(kTargets);
+      }
+      if (lane < (end - from) / 16) lists.offset[from / 16 + lane] = o;
+      count = end;
+    }
+    count = __builtin_amdgcn_readfirstlane(count);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const int units = count / 16 * chunks;
+    if (units == 0) continue;
+    int g = 0, c = 0;
+    auto advance = [&]() {
+      if (++c == chunks) {
+        c = 0;
+        if (g + 1 < count / 16) ++g;
+      }
+    };
+    Unit u0, u1;
+    fetch(0, 0, u0);
+    for (int u = 0; u < units; u += 2) {
+      advance();
+      fetch(g, c, u1);
+      multiply(u0);
+      advance();
+      fetch(g, c, u0);
+      if (u + 1 < units) multiply(u1);
+    }
+  }
+
+  __syncthreads();
+  for (int p = tid; p < kTargets * 4 * C; p += 64 * SPLIT) {
+    const int t = p / (4 * C), part = p % (4 * C);
+    if (first + t >= s.num_targets || channel + part * 4 >= s.N) continue;     // N % 4 == 0
+    float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int w = 0; w < SPLIT; ++w) {
+      const float4 f = *reinterpret_cast<const float4 *>(&s_acc[w][t * kAccRow + part * 4]);
+      v[0] += f.x;
+      v[1] += f.y;
+      v[2] += f.z;
+      v[3] += f.w;
+    }
+    finish_piece<float, 4>(v, ep, first + t, channel + part * 4, s.N, out);
+  }
+}
+
+void compact_forward(const float *sources, const float *weights, const int *kernel_map, int64_t S, int64_t Tn,
+                     int64_t O, int64_t K, int64_t N, const Epilogue &ep, float *out, hipStream_t stream) {
+  CompactShape s;
+  s.num_targets = Tn;
+  s.num_offsets = static_cast<int>(O);
+  s.K = static_cast<int>(K);
+  s.N = static_cast<int>(N);
+  s.chunks = static_cast<int>(div_ceil(K, 64));
+  const int ki = static_cast<int>(div_ceil(K, 16 * s.chunks));
+  const bool whole = K == 16 * ki * s.chunks;
+  // Eight wavefronts per workgroup while all of them find room at once (four to
+  // a SIMD: 64 -> 64 over 3 000 targets 8.4 against 9.2 us, over 12 000 19.7 and
+  // 14.9); one block of channels until there are enough workgroups without
+  // (64 -> 64 over 12 000 targets 14.9, in four blocks 18.5; over 25 000 25.4
+  // and 20.6).
+  const int64_t tiles = div_ceil(Tn, int64_t{64}), cols = div_ceil(N, int64_t{16});
+  const int64_t waves = 4 * tiles * cols, room = 16 * static_cast<int64_t>(compute_units());
+  const int split = 2 * waves <= room ? 8 : 4;
+  const int c = 6 * waves < 7 * room ? 1 : N % 64 == 0 ? 4 : N % 32 == 0 ? 2 : 1;
+  const dim3 grid(static_cast<unsigned>(tiles), static_cast<unsigned>(div_ceil(N, int64_t{16} * c)));
+#define MNT_COMPACT(C, KI, SPLIT)                                                                              \
+  if (whole) {                                                                                                 \
+    compact_forward_kernel<C, KI, SPLIT, true><<<grid, 64 * SPLIT, 0, stream>>>(                               \
+        sources, static_cast<unsigned>(S * K * 4), weights, static_cast<unsigned>(O * K * N * 4), kernel_map, s, \
+        reinterpret_cast<unsigned char *>(out), ep);                                                           \
+  } else {                                                                                                     \
+    compact_forward_kernel<C, KI, SPLIT, false><<<grid, 64 * SPLIT, 0, stream>>>(                              \
+        sources, static_cast<unsigned>(S * K * 4), weights, static_cast<unsigned>(O * K * N * 4), kernel_map, s, \
+        reinterpret_cast<unsigned char *>(out), ep);                                                           \
+  }
+#define MNT_COMPACT_K(C, SPLIT)               \
+  switch (ki) {                               \
+    case 1: MNT_COMPACT(C, 1, SPLIT) break;   \
+    case 2: MNT_COMPACT(C, 2, SPLIT) break;   \
+    case 3: MNT_COMPACT(C, 3, SPLIT) break;   \
+    default: MNT_COMPACT(C, 4, SPLIT) break;  \
+  }
+  if (split == 8) {
+    MNT_COMPACT_K(1, 8)
+  } else if (c == 1) {
+    MNT_COMPACT_K(1, 4)
+  } else if (c == 2) {
+    MNT_COMPACT_K(2, 4)
+  } else {
+    MNT_COMPACT_K(4, 4)
+  }
+#undef MNT_COMPACT_K
+#undef MNT_COMPACT
+  check_launch("compact_forward_kernel");
+}
+
+}  // namespace mnt

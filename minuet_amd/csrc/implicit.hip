@@ -35,6 +35,9 @@ template <typename T>
 void tiled_forward(const T *sources, const T *packed, const int *kernel_map, const int *tiles, int64_t S, int64_t Tn,
                    int64_t O, int64_t K, int64_t N, const Epilogue &ep, T *out, hipStream_t stream);
 
+void compact_forward(const float *sources, const float *weights, const int *kernel_map, int64_t S, int64_t Tn,
+                     int64_t O, int64_t K, int64_t N, const Epilogue &ep, float *out, hipStream_t stream);
+
 constexpr int kImplicitBlock = 256;
 constexpr int kImplicitTargets = 128;     // per workgroup, 32 per wavefront
 constexpr int kImplicitMaxBlocks = 4;     // 32-channel output blocks per channel group (128 channels)
@@ -529,6 +532,15 @@ static void implicit_typed(const T *sources, const T *weights, const T *packed, 
         profile_mark("implicit", stream);
         return;
       }
+    }
+  }
+  if constexpr (sizeof(T) == 4) {
+    // fp32 products are dear: hits only, wherever the weights are given as they are
+    if (O > 1 && weights != nullptr && reinterpret_cast<uintptr_t>(weights) % 16 == 0 &&
+        O * K * N * 4 < static_cast<int64_t>(kMaxSourceBytes)) {
+      compact_forward(sources, weights, kernel_map, S, Tn, O, K, N, ep, out, stream);
+      profile_mark("implicit", stream);
+      return;
     }
   }
   const int kc = kChunkBytes / static_cast<int>(sizeof(T));

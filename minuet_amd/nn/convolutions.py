@@ -902,14 +902,19 @@ class SparseConv(Module):
                             target_batch_dims=batch_dims, kernel_size=self.kernel_size,
                             kernel_dilation=self.dilation)
             sources = inputs.F
-            # the route depends on the layer, the feature type and the tunable
-            # dataflow only: decided once, then looked up
-            route_key = (sources.dtype, sources.is_cuda, self._tunable_config.get("dataflow", "auto"))
+            # the route depends on the layer, the feature type, the tunable
+            # dataflow and, in fp32, the size: decided once, then looked up
+            dataflow = self._tunable_config.get("dataflow", "auto")
+            hits = (sources.dtype == torch.float32 and dataflow == "auto" and sources.is_cuda
+                    and self.kernel.dtype == torch.float32
+                    and F.prefers_hits(self.kernel.shape[0], self.in_channels, self.out_channels, sources.dtype,
+                                       sources.shape[0]))
+            route_key = (sources.dtype, sources.is_cuda, dataflow, hits)
             route = self._routes.get(route_key)
             if route is None:
                 grouped = self._takes_offset_groups(sources)
                 pad = 0 if grouped else self._row_padding(sources)
-                route = (pad, not grouped and self._takes_implicit(sources, pad), grouped)
+                route = (pad, not grouped and (hits or self._takes_implicit(sources, pad)), grouped)
                 self._routes[route_key] = route
             pad, implicit, grouped = route
             groups = cache.get_offset_groups(**map_args) if grouped and self._tuning_data is None else None

@@ -1,0 +1,58 @@
+"""The fp32 single-kernel forward, which multiplies hits only."""
+import pytest
+import torch
+
+import minuet_amd as minuet
+from minuet_amd.nn import functional as F
+from minuet_amd.nn.functional import _C
+
+from test_gpu_tiles import DEVICE, operands, reference
+
+pytestmark = pytest.mark.gpu
+
+
+# targets about a workgroup's 64; K of one to four pieces of 16, ragged, and more than one unit;
+# N in one, two and four blocks and less than one; offsets fewer and more than a wavefront lists at once
+@pytest.mark.parametrize("targets,offsets,cin,cout", [
+    (1, 27, 4, 4), (63, 2, 16, 16), (65, 27, 32, 32), (1000, 8, 20, 36), (1000, 27, 48, 64), (700, 125, 32, 20),
+    (3000, 27, 100, 64), (500, 33, 256, 128), (30000, 27, 64, 64), (30000, 9, 64, 96), (70000, 27, 12, 32)])
+def test_forward_matches_products(targets, offsets, cin, cout):
+    dense, x, w = operands(targets, 3000, offsets, cin, cout, torch.float32)
+    wanted = reference(x.double(), w.double(), dense)
+
+    def check(got, wanted):
+        assert float((got.double() - wanted).norm() / wanted.norm().clamp(min=1e-6)) < 1e-6
+
+    out = _C.sparse_convolution_forward_implicit(x, w, dense)
+    check(out, wanted)
+    assert torch.equal(out, _C.sparse_convolution_forward_implicit(x, w, dense))
+    gen = torch.Generator(device=DEVICE).manual_seed(9)
+    scale, shift = (torch.randn(cout, generator=gen, device=DEVICE) for _ in range(2))
+    residual = torch.randn(targets, cout, generator=gen, device=DEVICE)
+    epilogue = F.Epilogue(scale, shift, residual, "relu", 0.0)
+    check(_C.sparse_convolution_forward_implicit(x, w, dense, epilogue=epilogue),
+          torch.relu(wanted * scale + shift + residual))
+
+
+def test_layer_takes_it_by_size():
+    assert F.prefers_hits(27, 32, 32, torch.float32, 10 ** 6) and F.prefers_hits(27, 64, 64, torch.float32, 12000)
+    assert not F.prefers_hits(27, 64, 64, torch.float32, 30000)
+    assert not F.prefers_hits(27, 30, 32, torch.float32, 100) and not F.prefers_hits(1, 32, 32, torch.float32, 100)
+    gen = torch.Generator(device=DEVICE).manual_seed(3)
+    conv = minuet.nn.SparseConv3d(64, 64, 3, dtype=torch.float32, device=DEVICE)
+    results = []
+    for rows, tables in ((2000, 0), (40000, 1)):
+        cells = torch.randperm(1 << 16, generator=gen, device=DEVICE)[:rows]
+        coordinates = torch.stack([cells >> 10, (cells >> 5) & 31, cells & 31], 1).int()
+        coordinates = coordinates[F.build_sorted_index(coordinates)]
+        cache = minuet.nn.KernelMapCache(3, torch.int32, DEVICE)
+        minuet.set_kernel_map_cache(conv, cache)
+        x = minuet.SparseTensor(torch.randn(rows, 64, generator=gen, device=DEVICE), coordinates)
+        with torch.no_grad():
+            out = conv(x).F
+            assert torch.equal(conv(x).F, out)
+        assert len(cache._kernel_maps_cache) == tables
+        dense, _ = _C.kernel_map_dense(coordinates, coordinates, cache._kernel_offsets((1, 1, 1), (3, 3, 3), (1, 1, 1)), None, None)
+        wanted = reference(x.F.double(), conv.kernel.detach().double(), dense)
+        results.append(float((out.double() - wanted).norm() / wanted.norm()))
+    assert max(results) < 1e-6

@@ -22,10 +22,11 @@ def random_map(targets, sources, offsets, density, seed):
 
 
 def reference(x, w, dense):
-    out = torch.zeros(dense.shape[1], w.shape[2], device=x.device)
+    kind = torch.float64 if x.dtype == torch.float64 else torch.float32
+    out = torch.zeros(dense.shape[1], w.shape[2], device=x.device, dtype=kind)
     for o in range(dense.shape[0]):
-        rows = x.float()[dense[o].clamp(min=0).long()] * (dense[o] >= 0)[:, None]
-        out += rows @ w[o].float()
+        rows = x.to(kind)[dense[o].clamp(min=0).long()] * (dense[o] >= 0)[:, None]
+        out += rows @ w[o].to(kind)
     return out
 
 
