@@ -26,7 +26,7 @@ struct CompactShape {
   int chunks;                  // units of KI * 16 input channels
 };
 
-// A workgroup takes 64 targets and 16 * C output channels; its SPLIT wavefronts
+// A workgroup takes TARGETS targets and 16 * C output channels; its SPLIT wavefronts
 // take every SPLIT-th offset each.  fp32 matrix instructions are 16 times dearer
 // than 16-bit ones, so nothing but hits is multiplied: a wavefront lists the
 // hits of its offsets, 16 rows of one offset at a time are multiplied by
@@ -41,18 +41,19 @@ struct CompactShape {
 // the split; beyond, the weights, which every 16 rows read again: where
 // targets x input x output channels pass 75 million the three-kernel form is
 // the faster one again (see prefers_implicit).  fp32, 3 x 3 x 3, us a layer in
-// three kernels and here: 32 -> 32 channels over 3 000 voxels 11.4 / 5.7,
-// 20 000 17.9 / 11.3, 200 000 76 / 52; 64 -> 64 over 3 000 12.1 / 8.4, 12 000
-// 18.8 / 14.9; 128 -> 128 over 800 19.5 / 12.8.  (128 targets per workgroup
+// three kernels and here: 32 -> 32 channels over 3 000 voxels 11.4 / 4.9,
+// 20 000 17.9 / 11.2, 200 000 76 / 52; 64 -> 64 over 3 000 12.1 / 8.4, 12 000
+// 18.8 / 14.9; 256 -> 256 over 135 28 / 22.  (128 targets per workgroup
 // fill the 16 rows better, but their sums leave fewer wavefronts to a compute
 // unit: 17 to 40 % slower.)
-template <int C, int KI, int SPLIT, bool WHOLE>
+template <int C, int KI, int SPLIT, int TARGETS, bool WHOLE>
 __global__ __launch_bounds__(64 * SPLIT) void compact_forward_kernel(
     const float *__restrict__ sources, unsigned source_bytes, const float *__restrict__ weights,
     unsigned weight_bytes, const int *__restrict__ kernel_map, CompactShape s, unsigned char *__restrict__ out,
     Epilogue ep) {
   constexpr int kCompactBatch = 32 / SPLIT;                // offsets whose hits a wavefront lists together
-  constexpr int kTargets = 64;
+  constexpr int kTargets = TARGETS;
+  constexpr int kAtOnce = 64 / TARGETS;                    // offsets that a wavefront's lanes look at together
   constexpr int kMost = kCompactBatch * kTargets;          // list entries
   constexpr int kAccRow = 16 * C + 4;
   struct Lists {
@@ -152,11 +153,11 @@ __global__ __launch_bounds__(64 * SPLIT) void compact_forward_kernel(
   };
 
   for (int first_offset = wv; first_offset < s.num_offsets || first_offset == wv; first_offset += SPLIT * kCompactBatch) {
-    int index[kCompactBatch];
+    int index[kCompactBatch / kAtOnce];
 #pragma unroll
-    for (int j = 0; j < kCompactBatch; ++j) {
-      const long long o = min(first_offset + j * SPLIT, s.num_offsets - 1);
-      index[j] = kernel_map[o * s.num_targets + min(first + lane, s.num_targets - 1)];
+    for (int j = 0; j < kCompactBatch / kAtOnce; ++j) {
+      const long long o = min(first_offset + (j * kAtOnce + lane / kTargets) * SPLIT, s.num_offsets - 1);
+      index[j] = kernel_map[o * s.num_targets + min(first + lane % kTargets, s.num_targets - 1)];
     }
     if (first_offset == wv) {
       float4 *const clear = reinterpret_cast<float4 *>(acc);
@@ -164,24 +165,29 @@ __global__ __launch_bounds__(64 * SPLIT) void compact_forward_kernel(
     }
     int count = 0;
 #pragma unroll
-    for (int j = 0; j < kCompactBatch; ++j) {
-      const int o = first_offset + j * SPLIT;
-      const int from = count;
-      const bool hit = index[j] >= 0 && first + lane < s.num_targets && o < s.num_offsets;
+    for (int j = 0; j < kCompactBatch / kAtOnce; ++j) {
+      const bool hit = index[j] >= 0 && first + lane % kTargets < s.num_targets &&
+                       first_offset + (j * kAtOnce + lane / kTargets) * SPLIT < s.num_offsets;
       const unsigned long long votes = __ballot(hit);
-      if (hit) {
-        const int p = count + __popcll(votes & lanes_below());
-        lists.source[p] = index[j];
-        lists.target[p] = static_cast<unsigned char>(lane);
+#pragma unroll
+      for (int part = 0; part < kAtOnce; ++part) {
+        constexpr unsigned long long kOwn = kTargets == 64 ? ~0ull : (1ull << (kTargets & 63)) - 1ull;
+        const unsigned long long own = votes & (kOwn << (part * kTargets & 63));
+        const int from = count;
+        if (hit && lane / kTargets == part) {
+          const int p = count + __popcll(own & lanes_below());
+          lists.source[p] = index[j];
+          lists.target[p] = static_cast<unsigned char>(lane % kTargets);
+        }
+        count += __popcll(own);
+        const int end = (count + 15) & ~15;    // the rest of 16 rows: no source, a target nobody asks for
+        if (lane < end - count) {
+          lists.source[count + lane] = -1;
+          lists.target[count + lane] = static_cast<unsigned char>(kTargets);
+        }
+        if (lane < (end - from) / 16) lists.offset[from / 16 + lane] = first_offset + (j * kAtOnce + part) * SPLIT;
+        count = end;
       }
-      count += __popcll(votes);
-      const int end = (count + 15) & ~15;      // the rest of 16 rows: no source, a target nobody asks for
-      if (lane < end - count) {
-        lists.source[count + lane] = -1;
-        lists.target[count + lane] = static_cast<unsigned char>(kTargets);
-      }
-      if (lane < (end - from) / 16) lists.offset[from / 16 + lane] = o;
-      count = end;
     }
     count = __builtin_amdgcn_readfirstlane(count);
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -234,44 +240,65 @@ void compact_forward(const float *sources, const float *weights, const int *kern
   s.chunks = static_cast<int>(div_ceil(K, 64));
   const int ki = static_cast<int>(div_ceil(K, 16 * s.chunks));
   const bool whole = K == 16 * ki * s.chunks;
-  // Eight wavefronts per workgroup while all of them find room at once (four to
-  // a SIMD: 64 -> 64 over 3 000 targets 8.4 against 9.2 us, over 12 000 19.7 and
-  // 14.9); one block of channels until there are enough workgroups without
-  // (64 -> 64 over 12 000 targets 14.9, in four blocks 18.5; over 25 000 25.4
-  // and 20.6).
-  const int64_t tiles = div_ceil(Tn, int64_t{64}), cols = div_ceil(N, int64_t{16});
-  const int64_t waves = 4 * tiles * cols, room = 16 * static_cast<int64_t>(compute_units());
-  const int split = 2 * waves <= room ? 8 : 4;
-  const int c = 6 * waves < 7 * room ? 1 : N % 64 == 0 ? 4 : N % 32 == 0 ? 2 : 1;
-  const dim3 grid(static_cast<unsigned>(tiles), static_cast<unsigned>(div_ceil(N, int64_t{16} * c)));
-#define MNT_COMPACT(C, KI, SPLIT)                                                                              \
-  if (whole) {                                                                                                 \
-    compact_forward_kernel<C, KI, SPLIT, true><<<grid, 64 * SPLIT, 0, stream>>>(                               \
-        sources, static_cast<unsigned>(S * K * 4), weights, static_cast<unsigned>(O * K * N * 4), kernel_map, s, \
-        reinterpret_cast<unsigned char *>(out), ep);                                                           \
-  } else {                                                                                                     \
-    compact_forward_kernel<C, KI, SPLIT, false><<<grid, 64 * SPLIT, 0, stream>>>(                              \
-        sources, static_cast<unsigned>(S * K * 4), weights, static_cast<unsigned>(O * K * N * 4), kernel_map, s, \
-        reinterpret_cast<unsigned char *>(out), ep);                                                           \
-  }
-#define MNT_COMPACT_K(C, SPLIT)               \
-  switch (ki) {                               \
-    case 1: MNT_COMPACT(C, 1, SPLIT) break;   \
-    case 2: MNT_COMPACT(C, 2, SPLIT) break;   \
-    case 3: MNT_COMPACT(C, 3, SPLIT) break;   \
-    default: MNT_COMPACT(C, 4, SPLIT) break;  \
-  }
-  if (split == 8) {
-    MNT_COMPACT_K(1, 8)
-  } else if (c == 1) {
-    MNT_COMPACT_K(1, 4)
-  } else if (c == 2) {
-    MNT_COMPACT_K(2, 4)
+  // One block of channels per workgroup, and fewer targets the fewer workgroups
+  // that leaves, so that small clouds reach the whole chip (256 -> 256 channels
+  // over 135 targets: 45 us with 64 targets per workgroup, 22 with 16; 32 -> 32
+  // over 3 000 6.5 and, with 32, 4.9); all channels together only where there
+  // are workgroups without (64 -> 64 over 12 000 targets 14.8, in four blocks
+  // 18.6; over 25 000 24.9 and 20.7).  Eight wavefronts per workgroup while all
+  // of them find room at once.
+  const int64_t cus = compute_units(), cols = div_ceil(N, int64_t{16});
+  const int64_t full = div_ceil(Tn, int64_t{64}) * cols;         // workgroups of 64 targets and 16 channels
+  int c = 1, targets = 64, split = 4;
+  if (4 * full >= 19 * cus) {
+    c = N % 64 == 0 ? 4 : N % 32 == 0 ? 2 : 1;
+  } else if (16 * full >= 15 * cus) {
+    split = 4 * full <= 9 * cus ? 8 : 4;
+  } else if (20 * full >= 7 * cus) {
+    targets = 32;
+    split = 2 * full <= cus ? 8 : 4;
   } else {
-    MNT_COMPACT_K(4, 4)
+    targets = 16;
+    split = 8;
+  }
+  const dim3 grid(static_cast<unsigned>(div_ceil(Tn, int64_t{targets})), static_cast<unsigned>(div_ceil(cols, int64_t{c})));
+#define MNT_COMPACT_W(C, KI, SPLIT, TARGETS, WHOLE)                                                            \
+  compact_forward_kernel<C, KI, SPLIT, TARGETS, WHOLE><<<grid, 64 * SPLIT, 0, stream>>>(                       \
+      sources, static_cast<unsigned>(S * K * 4), weights, static_cast<unsigned>(O * K * N * 4), kernel_map, s, \
+      reinterpret_cast<unsigned char *>(out), ep)
+#define MNT_COMPACT(C, KI, SPLIT, TARGETS)             \
+  if (whole) {                                         \
+    MNT_COMPACT_W(C, KI, SPLIT, TARGETS, true);        \
+  } else {                                             \
+    MNT_COMPACT_W(C, KI, SPLIT, TARGETS, false);       \
+  }
+#define MNT_COMPACT_K(C, SPLIT, TARGETS)               \
+  switch (ki) {                                        \
+    case 1: MNT_COMPACT(C, 1, SPLIT, TARGETS) break;   \
+    case 2: MNT_COMPACT(C, 2, SPLIT, TARGETS) break;   \
+    case 3: MNT_COMPACT(C, 3, SPLIT, TARGETS) break;   \
+    default: MNT_COMPACT(C, 4, SPLIT, TARGETS) break;  \
+  }
+  if (c == 4) {
+    MNT_COMPACT_K(4, 4, 64)
+  } else if (c == 2) {
+    MNT_COMPACT_K(2, 4, 64)
+  } else if (targets == 16) {
+    MNT_COMPACT_K(1, 8, 16)
+  } else if (targets == 32) {
+    if (split == 8) {
+      MNT_COMPACT_K(1, 8, 32)
+    } else {
+      MNT_COMPACT_K(1, 4, 32)
+    }
+  } else if (split == 8) {
+    MNT_COMPACT_K(1, 8, 64)
+  } else {
+    MNT_COMPACT_K(1, 4, 64)
   }
 #undef MNT_COMPACT_K
 #undef MNT_COMPACT
+#undef MNT_COMPACT_W
   check_launch("compact_forward_kernel");
 }
 

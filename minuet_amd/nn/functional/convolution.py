@@ -53,7 +53,7 @@ def prefers_hits(num_offsets: int, num_source_features: int, num_target_features
     """Whether ``dataflow="auto"`` takes the single-kernel form for an fp32 layer
     over ``num_rows`` source rows.  That form multiplies hits only, 16 at a time,
     and reads the weights again for every 16: measured to be the faster one for
-    narrow layers of any size (32 -> 32 channels: 5.7 against 11.4 us over 3 000
+    narrow layers of any size (32 -> 32 channels: 4.9 against 11.4 us over 3 000
     voxels, 52 against 76 over 200 000) and for others up to 75 million rows x
     channels in x channels out (64 -> 64 over 12 000 voxels 14.9 against 18.8 us,
     over 20 000 27.9 and 24.6; 128 -> 128 over 3 000 19.1 and 21.4)."""

@@ -11,10 +11,11 @@ from test_gpu_tiles import DEVICE, operands, reference
 pytestmark = pytest.mark.gpu
 
 
-# targets about a workgroup's 64; K of one to four pieces of 16, ragged, and more than one unit;
+# targets about a workgroup's 16, 32 and 64; K of one to four pieces of 16, ragged, and more than one unit;
 # N in one, two and four blocks and less than one; offsets fewer and more than a wavefront lists at once
 @pytest.mark.parametrize("targets,offsets,cin,cout", [
     (1, 27, 4, 4), (63, 2, 16, 16), (65, 27, 32, 32), (1000, 8, 20, 36), (1000, 27, 48, 64), (700, 125, 32, 20),
+    (15, 27, 64, 16), (17, 27, 64, 64), (1500, 27, 64, 32), (3000, 27, 32, 64), (6000, 27, 64, 64),
     (3000, 27, 100, 64), (500, 33, 256, 128), (30000, 27, 64, 64), (30000, 9, 64, 96), (70000, 27, 12, 32)])
 def test_forward_matches_products(targets, offsets, cin, cout):
     dense, x, w = operands(targets, 3000, offsets, cin, cout, torch.float32)
