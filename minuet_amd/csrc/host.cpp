@@ -310,15 +310,16 @@ inline bool vector_fits(const at::Tensor *t, int64_t channels, int device) {
 // two or more forwards to make and are kept with the map, so they are made once
 // the forwards that have run over it would have saved twice their price: a map
 // that a network reads a few times and drops never pays for them, one that is
-// read on and on soon does.
+// read on and on soon does.  Layers of all widths and types share a map, so
+// whether this one can use tiles (a share of 0: it cannot) is asked first.
 constexpr double kTilesCredit = 2.0;
 constexpr int64_t kTilesMostInts = int64_t{1} << 29;
 
 const at::Tensor *tiles_of(MapEntry *map, const Layer *l, int64_t T, const at::Device &device, void *stream) {
-  if (map->tiles != nullptr) return tensor_of(map->tiles);
-  if (map->tiles_credit < 0.0) return nullptr;
   const double share = g_tiles_share(T, l->num_offsets, l->in_channels, l->out_channels, l->float_code);
   if (share == 0.0) return nullptr;
+  if (map->tiles != nullptr) return tensor_of(map->tiles);
+  if (map->tiles_credit < 0.0) return nullptr;
   map->tiles_credit += share;
   if (map->tiles_credit < kTilesCredit) return nullptr;
   if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return nullptr;

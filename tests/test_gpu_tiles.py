@@ -6,6 +6,7 @@ import torch
 import minuet_amd as minuet
 from minuet_amd.nn import functional as F
 from minuet_amd.nn.functional import _C
+from minuet_amd.unet import SparseUNet
 
 pytestmark = pytest.mark.gpu
 DEVICE = "cuda:0"
@@ -93,14 +94,18 @@ def test_forward_matches_products(targets, offsets, cin, cout, dtype):
     close(_C.sparse_convolution_forward_tiled(x, w, tiles, targets, packed, epilogue=epilogue), wanted, dtype)
 
 
+def scattered_cloud():
+    gen = torch.Generator(device=DEVICE).manual_seed(3)
+    cells = torch.randperm(1 << 20, generator=gen, device=DEVICE)[:100000]
+    coordinates = torch.stack([cells >> 13, (cells >> 6) & 127, cells & 63], 1).int()
+    return coordinates[F.build_sorted_index(coordinates)], gen
+
+
 @pytest.mark.parametrize("cin,cout,dtype", [(64, 64, torch.float16), (32, 32, torch.bfloat16), (24, 96, torch.float16),
                                             (128, 64, torch.float16)])
 def test_layer_comes_to_use_tiles(cin, cout, dtype):
     """A map that is read on and on gets tiles; the layer's results stay bit for bit."""
-    gen = torch.Generator(device=DEVICE).manual_seed(3)
-    cells = torch.randperm(1 << 20, generator=gen, device=DEVICE)[:100000]
-    coordinates = torch.stack([cells >> 13, (cells >> 6) & 127, cells & 63], 1).int()
-    coordinates = coordinates[F.build_sorted_index(coordinates)]
+    coordinates, gen = scattered_cloud()
     conv = minuet.nn.SparseConv3d(cin, cout, 3, dtype=dtype, device=DEVICE)
     minuet.set_kernel_map_cache(conv, minuet.nn.KernelMapCache(3, torch.int32, DEVICE))
     x = minuet.SparseTensor(torch.randn(100000, cin, generator=gen, device=DEVICE).to(dtype), coordinates)
@@ -111,3 +116,39 @@ def test_layer_comes_to_use_tiles(cin, cout, dtype):
             last = conv(x).F
         assert torch.cuda.memory_allocated() > held + 100000 * 27 * 4      # the tiles
     assert torch.equal(last, first)
+
+
+@pytest.mark.parametrize("cin,cout,dtype", [(4, 32, torch.float16), (8, 64, torch.bfloat16), (32, 32, torch.float32)])
+def test_layers_that_take_no_tiles_share_a_map_that_has_them(cin, cout, dtype):
+    """The map belongs to its kernel size and stride: once a wide layer has earned
+    it tiles, a stem or an fp32 layer over it runs as before."""
+    coordinates, gen = scattered_cloud()
+    wide = minuet.nn.SparseConv3d(64, 64, 3, dtype=torch.float16, device=DEVICE)
+    conv = minuet.nn.SparseConv3d(cin, cout, 3, dtype=dtype, device=DEVICE)
+    cache = minuet.nn.KernelMapCache(3, torch.int32, DEVICE)
+    for module in (wide, conv):
+        minuet.set_kernel_map_cache(module, cache)
+    x = minuet.SparseTensor(torch.randn(100000, cin, generator=gen, device=DEVICE).to(dtype), coordinates)
+    y = minuet.SparseTensor(torch.randn(100000, 64, generator=gen, device=DEVICE).half(), coordinates)
+    with torch.no_grad():
+        first = conv(x).F
+        for _ in range(20):
+            wide(y)
+            again = conv(x).F
+    assert torch.equal(again, first)
+
+
+def test_network_on_kept_maps():
+    """Ten passes over the same maps, and a captured one, equal the first."""
+    coordinates, gen = scattered_cloud()
+    torch.manual_seed(0)
+    net = SparseUNet(4, 32, dtype=torch.float16, device=DEVICE).eval()
+    minuet.set_kernel_map_cache(net, minuet.nn.KernelMapCache(3, torch.int32, DEVICE))
+    x = minuet.SparseTensor(torch.randn(100000, 4, generator=gen, device=DEVICE).half(), coordinates)
+    with torch.no_grad():
+        first = net(x).F
+        for _ in range(9):
+            assert torch.equal(net(x).F, first)
+    graphed = minuet.capture_forward(lambda: net(x))
+    for _ in range(3):
+        assert torch.equal(graphed.replay().F, first)
