@@ -16,12 +16,14 @@
 
 #include <ATen/ATen.h>
 #include <ATen/hip/EmptyTensor.h>
+#include <ATen/hip/HIPEvent.h>
 #include <c10/core/GradMode.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 
 #include <cstdint>
+#include <memory>
 
 namespace {
 
@@ -141,6 +143,11 @@ struct MapEntry {
   // would have saved so far, over what making them takes (below 0: never).
   PyObject *tiles;
   double tiles_credit;
+  // The stream that makes the tiles, the end of that work, and whether the host
+  // has seen it ended.
+  void *tiles_stream;
+  at::cuda::CUDAEvent *tiles_made;
+  char tiles_ready;
 };
 
 void map_entry_dealloc(PyObject *self) {
@@ -150,6 +157,7 @@ void map_entry_dealloc(PyObject *self) {
   Py_XDECREF(e->batch_dims);
   Py_XDECREF(e->keep);
   Py_XDECREF(e->tiles);
+  delete e->tiles_made;
   Py_TYPE(self)->tp_free(self);
 }
 
@@ -181,6 +189,9 @@ PyObject *map_entry_new(PyTypeObject *type, PyObject *args, PyObject *) {
   e->used = 0;
   e->tiles = nullptr;
   e->tiles_credit = 0.0;
+  e->tiles_stream = nullptr;
+  e->tiles_made = nullptr;
+  e->tiles_ready = 0;
   for (Py_ssize_t i = 0; i < 8; ++i) {
     e->at[i] = nullptr;
     if (i < PyTuple_GET_SIZE(pointers) && !is_none(PyTuple_GET_ITEM(pointers, i))) {
@@ -315,33 +326,59 @@ inline bool vector_fits(const at::Tensor *t, int64_t channels, int device) {
 constexpr double kTilesCredit = 2.0;
 constexpr int64_t kTilesMostInts = int64_t{1} << 29;
 
-const at::Tensor *tiles_of(MapEntry *map, const Layer *l, int64_t T, const at::Device &device, void *stream) {
-  const double share = g_tiles_share(T, l->num_offsets, l->in_channels, l->out_channels, l->float_code);
-  if (share == 0.0) return nullptr;
-  if (map->tiles != nullptr) return tensor_of(map->tiles);
-  if (map->tiles_credit < 0.0) return nullptr;
-  map->tiles_credit += share;
-  if (map->tiles_credit < kTilesCredit) return nullptr;
-  if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return nullptr;
-  map->tiles_credit = -1.0;
+bool make_tiles(MapEntry *map, const Layer *l, int64_t T, const at::Device &device, const c10::hip::HIPStream &stream) {
   int64_t ints = 0;
-  if (g_tiles_size(T, l->num_offsets, &ints) != 0 || ints > kTilesMostInts) return nullptr;
+  if (g_tiles_size(T, l->num_offsets, &ints) != 0 || ints > kTilesMostInts) return false;
   at::Tensor tiles;
   try {
     tiles = at::detail::empty_cuda({ints}, at::kInt, device, std::nullopt);
   } catch (const std::exception &) {                     // no room: the layer runs without
-    return nullptr;
+    return false;
   }
   if (g_tiles(static_cast<const int32_t *>(map->at[0]), T, l->num_offsets,
-              static_cast<int32_t *>(tiles.mutable_data_ptr()), stream) != 0) {
-    return nullptr;
+              static_cast<int32_t *>(tiles.mutable_data_ptr()), stream.stream()) != 0) {
+    return false;
   }
+  std::unique_ptr<at::cuda::CUDAEvent> made(new at::cuda::CUDAEvent());
+  made->record(c10::hip::HIPStreamMasqueradingAsCUDA(stream));
   map->tiles = THPVariable_Wrap(std::move(tiles));
   if (map->tiles == nullptr) {
     PyErr_Clear();
-    return nullptr;
+    return false;
   }
-  return tensor_of(map->tiles);
+  map->tiles_stream = stream.stream();
+  map->tiles_made = made.release();
+  return true;
+}
+
+// A call on the stream that makes the tiles comes after that work by itself.
+// One on another stream takes them once the host has seen the work ended: the
+// two streams owe each other nothing because of tiles, which no caller asked
+// for and none can wait for, and until then the layer without them gives the
+// same rows.  (The event is not asked during a capture, which forbids it.)  The
+// allocator is told of the other stream, which may still read the tiles when
+// the cache has dropped them.
+const at::Tensor *tiles_of(MapEntry *map, const Layer *l, int64_t T, const at::Device &device,
+                           const c10::hip::HIPStream &stream) {
+  const double share = g_tiles_share(T, l->num_offsets, l->in_channels, l->out_channels, l->float_code);
+  if (share == 0.0) return nullptr;
+  if (map->tiles == nullptr) {
+    if (map->tiles_credit < 0.0) return nullptr;
+    map->tiles_credit += share;
+    if (map->tiles_credit < kTilesCredit) return nullptr;
+    if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return nullptr;
+    map->tiles_credit = -1.0;
+    if (!make_tiles(map, l, T, device, stream)) return nullptr;
+  }
+  const at::Tensor *tiles = tensor_of(map->tiles);
+  if (map->tiles_stream == stream.stream()) return tiles;
+  if (map->tiles_ready == 0) {
+    if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return nullptr;
+    if (!map->tiles_made->query()) return nullptr;
+    map->tiles_ready = 1;
+  }
+  tiles->record_stream(c10::hip::HIPStreamMasqueradingAsCUDA(stream));
+  return tiles;
 }
 
 PyObject *none() { Py_RETURN_NONE; }
@@ -439,7 +476,8 @@ PyObject *run_layer(Layer *l, PyObject *module_dict, PyObject *inputs, const Epi
     }
   }
   at::Tensor out = at::detail::empty_cuda({T, l->out_channels}, kernel.scalar_type(), kernel.device(), std::nullopt);
-  void *stream = c10::hip::getCurrentHIPStream(l->device).stream();
+  const c10::hip::HIPStream current = c10::hip::getCurrentHIPStream(l->device);
+  void *stream = current.stream();
   auto data = [](const at::Tensor *t) -> const void * { return t == nullptr ? nullptr : t->const_data_ptr(); };
   const float *scale_at = static_cast<const float *>(data(scale));
   const float *shift_at = static_cast<const float *>(data(shift));
@@ -448,7 +486,7 @@ PyObject *run_layer(Layer *l, PyObject *module_dict, PyObject *inputs, const Epi
   int status = 0;
   switch (l->kind) {
     case kImplicit:
-      if (const at::Tensor *tiles = tiles_of(map, l, T, kernel.device(), stream)) {
+      if (const at::Tensor *tiles = tiles_of(map, l, T, kernel.device(), current)) {
         status = g_tiled(source, packed_at, static_cast<const int32_t *>(tiles->const_data_ptr()), S, T,
                          l->num_offsets, l->in_channels, l->out_channels, l->float_code, scale_at, shift_at,
                          data(residual), ep.activation, ep.slope, out.mutable_data_ptr(), stream);

@@ -1,5 +1,7 @@
 """The output-stationary forward with and without tiles of targets that share
 their live offsets, against a plain fp32 product per offset."""
+import ctypes
+
 import pytest
 import torch
 
@@ -152,3 +154,39 @@ def test_network_on_kept_maps():
     graphed = minuet.capture_forward(lambda: net(x))
     for _ in range(3):
         assert torch.equal(graphed.replay().F, first)
+
+
+def test_tiles_made_on_one_stream_and_read_on_another():
+    """The tiles' store addresses are read by other streams only when they are
+    written, and stay theirs until their last reader is done."""
+    coordinates, gen = scattered_cloud()
+    conv = minuet.nn.SparseConv3d(64, 64, 3, dtype=torch.float16, device=DEVICE)
+    cache = minuet.nn.KernelMapCache(3, torch.int32, DEVICE)
+    minuet.set_kernel_map_cache(conv, cache)
+    x = minuet.SparseTensor(torch.randn(100000, 64, generator=gen, device=DEVICE).half(), coordinates)
+    lib = _C.load_library()
+    size = ctypes.c_int64()
+    assert lib.mnt_kernel_map_tiles_size(100000, 27, ctypes.byref(size)) == 0
+    maker, reader = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.no_grad():
+        first = conv(x).F
+        held = torch.cuda.memory_allocated()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(maker):
+            torch.cuda._sleep(2_000_000)                 # the tiles are far from written when the other stream calls
+            for _ in range(60):
+                conv(x)
+                if torch.cuda.memory_allocated() >= held + 4 * size.value:
+                    break
+        assert torch.cuda.memory_allocated() >= held + 4 * size.value
+        with torch.cuda.stream(reader):
+            assert torch.equal(conv(x).F, first)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(reader):                  # with tiles now, read late, after the cache has let go of them
+            torch.cuda._sleep(2_000_000)
+            last = conv(x).F
+        cache.reset()
+        with torch.cuda.stream(maker):
+            taken = [torch.zeros(size.value, dtype=torch.int32, device=DEVICE) for _ in range(3)]
+        torch.cuda.synchronize()
+    assert torch.equal(last, first) and len(taken) == 3
