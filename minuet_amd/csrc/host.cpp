@@ -10,8 +10,14 @@
 // Layer.run checks that both still describe the call at hand.  Whatever is
 // not exactly as it was when the two were made sends the caller (None is
 // returned) through the Python code that makes them.
+//
+// Every entry point that touches a tensor stands between HANDLE_TH_ERRORS and
+// END_HANDLE_TH_ERRORS: what torch throws (no memory left, a tensor without
+// storage) reaches the caller as the Python exception it is, and no further.
+// What such a function owns meanwhile it holds in a Ref.
 #include <Python.h>
 
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <ATen/ATen.h>
@@ -86,6 +92,20 @@ inline PyObject *dict_of(PyObject *object) {
 // Borrowed lookup; null when the key is missing (no exception set).
 inline PyObject *look(PyObject *dict, PyObject *key) { return PyDict_GetItem(dict, key); }
 
+// An owned reference.
+struct Ref {
+  PyObject *object;
+  explicit Ref(PyObject *o = nullptr) : object(o) {}
+  Ref(const Ref &) = delete;
+  Ref &operator=(const Ref &) = delete;
+  ~Ref() { Py_XDECREF(object); }
+  PyObject *release() {
+    PyObject *o = object;
+    object = nullptr;
+    return o;
+  }
+};
+
 inline bool is_none(PyObject *o) { return o == nullptr || o == Py_None; }
 
 inline const at::Tensor *tensor_of(PyObject *o) {
@@ -104,13 +124,13 @@ struct Watched {
   int64_t version = 0;
 
   void set(PyObject *o) {
-    Py_XINCREF(o);
-    Py_XDECREF(object);
-    object = o;
     if (const at::Tensor *t = tensor_of(o)) {
       data = t->const_data_ptr();
       version = version_of(*t);
     }
+    Py_XINCREF(o);
+    Py_XDECREF(object);
+    object = o;
   }
   bool same(PyObject *o) const {
     if (o != object) return false;
@@ -246,6 +266,7 @@ void layer_dealloc(PyObject *self) {
 
 // Layer(module, kind, weights, packed, shape_id, shortcut, bias_shift)
 PyObject *layer_new(PyTypeObject *type, PyObject *args, PyObject *) {
+  HANDLE_TH_ERRORS
   PyObject *module, *weights, *packed, *shape_id, *bias_shift;
   int kind, shortcut;
   if (!PyArg_ParseTuple(args, "OiOOOiO", &module, &kind, &weights, &packed, &shape_id, &shortcut, &bias_shift)) {
@@ -260,8 +281,9 @@ PyObject *layer_new(PyTypeObject *type, PyObject *args, PyObject *) {
     PyErr_SetString(PyExc_ValueError, "Layer needs a convolution module, its weights and their packed copy");
     return nullptr;
   }
-  Layer *l = reinterpret_cast<Layer *>(type->tp_alloc(type, 0));
-  if (l == nullptr) return nullptr;
+  Ref made(type->tp_alloc(type, 0));
+  if (made.object == nullptr) return nullptr;
+  Layer *l = reinterpret_cast<Layer *>(made.object);
   new (&l->kernel) Watched();
   new (&l->bias) Watched();
   l->kernel.set(look(parameters, s_kernel));
@@ -294,11 +316,8 @@ PyObject *layer_new(PyTypeObject *type, PyObject *args, PyObject *) {
   l->threshold_value = l->has_threshold ? PyFloat_AsDouble(l->threshold) : 0.0;
   l->gather_tile_value = l->gather_tile == Py_None ? 0 : PyLong_AsLongLong(l->gather_tile);
   l->scatter_tile_value = l->scatter_tile == Py_None ? 0 : PyLong_AsLongLong(l->scatter_tile);
-  if (PyErr_Occurred()) {
-    Py_DECREF(l);
-    return nullptr;
-  }
-  return reinterpret_cast<PyObject *>(l);
+  return PyErr_Occurred() ? nullptr : made.release();
+  END_HANDLE_TH_ERRORS
 }
 
 PyTypeObject LayerType = {PyVarObject_HEAD_INIT(nullptr, 0)};
@@ -523,19 +542,14 @@ PyObject *run_layer(Layer *l, PyObject *module_dict, PyObject *inputs, const Epi
     return nullptr;
   }
   // the result: a SparseTensor like the ones SparseTensor.like makes
-  PyObject *result = g_sparse_tensor->tp_new(g_sparse_tensor, g_no_arguments, nullptr);
-  if (result == nullptr) return nullptr;
-  PyObject *features = THPVariable_Wrap(std::move(out));
-  const bool ok = features != nullptr && PyObject_SetAttr(result, s__features, features) == 0 &&
-                  PyObject_SetAttr(result, s__coordinates, out_coordinates) == 0 &&
-                  PyObject_SetAttr(result, s__stride, out_stride) == 0 &&
-                  PyObject_SetAttr(result, s__batch_dims, out_batch_dims) == 0;
-  Py_XDECREF(features);
-  if (!ok) {
-    Py_DECREF(result);
-    return nullptr;
-  }
-  return result;
+  Ref result(g_sparse_tensor->tp_new(g_sparse_tensor, g_no_arguments, nullptr));
+  if (result.object == nullptr) return nullptr;
+  const Ref features(THPVariable_Wrap(std::move(out)));
+  const bool ok = features.object != nullptr && PyObject_SetAttr(result.object, s__features, features.object) == 0 &&
+                  PyObject_SetAttr(result.object, s__coordinates, out_coordinates) == 0 &&
+                  PyObject_SetAttr(result.object, s__stride, out_stride) == 0 &&
+                  PyObject_SetAttr(result.object, s__batch_dims, out_batch_dims) == 0;
+  return ok ? result.release() : nullptr;
 }
 
 // The Layer a module keeps, or null.
@@ -558,6 +572,7 @@ int activation_code(PyObject *name) {
 
 // run(module, inputs, epilogue): the module's forward, or None.
 PyObject *py_run(PyObject *, PyObject *const *args, Py_ssize_t count) {
+  HANDLE_TH_ERRORS
   if (count != 3) {
     PyErr_SetString(PyExc_TypeError, "run(module, inputs, epilogue)");
     return nullptr;
@@ -566,30 +581,25 @@ PyObject *py_run(PyObject *, PyObject *const *args, Py_ssize_t count) {
   Layer *l = d == nullptr ? nullptr : layer_of(d);
   if (l == nullptr) return none();
   EpilogueArgs ep;
-  PyObject *held[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
+  Ref held[5];
   if (args[2] != Py_None) {
     PyObject *names[5] = {s_scale, s_shift, s_residual, s_activation, s_negative_slope};
     for (int i = 0; i < 5; ++i) {
-      held[i] = PyObject_GetAttr(args[2], names[i]);
-      if (held[i] == nullptr) {
-        for (PyObject *h : held) Py_XDECREF(h);
-        return nullptr;
-      }
+      held[i].object = PyObject_GetAttr(args[2], names[i]);
+      if (held[i].object == nullptr) return nullptr;
     }
-    ep.scale = held[0];
-    ep.shift = held[1];
-    ep.residual = held[2];
-    ep.activation = activation_code(held[3]);
-    ep.slope = static_cast<float>(PyFloat_AsDouble(held[4]));
+    ep.scale = held[0].object;
+    ep.shift = held[1].object;
+    ep.residual = held[2].object;
+    ep.activation = activation_code(held[3].object);
+    ep.slope = static_cast<float>(PyFloat_AsDouble(held[4].object));
+    if (PyErr_Occurred()) return nullptr;
   }
-  PyObject *result = nullptr;
-  if (!PyErr_Occurred()) {
-    Py_INCREF(l);
-    result = ep.activation < 0 ? none() : run_layer(l, d, args[1], ep);
-    Py_DECREF(l);
-  }
-  for (PyObject *h : held) Py_XDECREF(h);
-  return result;
+  if (ep.activation < 0) return none();
+  Py_INCREF(l);
+  const Ref keep(reinterpret_cast<PyObject *>(l));
+  return run_layer(l, d, args[1], ep);
+  END_HANDLE_TH_ERRORS
 }
 
 // ----------------------------------------------------------------- Affine ----
@@ -613,6 +623,7 @@ void affine_dealloc(PyObject *self) {
 
 // Affine(norm, scale, shift)
 PyObject *affine_new(PyTypeObject *type, PyObject *args, PyObject *) {
+  HANDLE_TH_ERRORS
   PyObject *norm, *scale, *shift;
   if (!PyArg_ParseTuple(args, "OOO", &norm, &scale, &shift)) return nullptr;
   PyObject *d = dict_of(norm);
@@ -622,8 +633,9 @@ PyObject *affine_new(PyTypeObject *type, PyObject *args, PyObject *) {
     PyErr_SetString(PyExc_ValueError, "Affine needs a module with buffers and parameters");
     return nullptr;
   }
-  Affine *a = reinterpret_cast<Affine *>(type->tp_alloc(type, 0));
-  if (a == nullptr) return nullptr;
+  Ref made(type->tp_alloc(type, 0));
+  if (made.object == nullptr) return nullptr;
+  Affine *a = reinterpret_cast<Affine *>(made.object);
   for (Watched *w : {&a->mean, &a->var, &a->weight, &a->bias}) new (w) Watched();
   a->mean.set(look(buffers, s_running_mean));
   a->var.set(look(buffers, s_running_var));
@@ -636,7 +648,8 @@ PyObject *affine_new(PyTypeObject *type, PyObject *args, PyObject *) {
   Py_INCREF(a->eps);
   Py_INCREF(scale);
   Py_INCREF(shift);
-  return reinterpret_cast<PyObject *>(a);
+  return made.release();
+  END_HANDLE_TH_ERRORS
 }
 
 PyTypeObject AffineType = {PyVarObject_HEAD_INIT(nullptr, 0)};
@@ -673,6 +686,7 @@ inline bool empty_dict(PyObject *d) { return d == nullptr || (PyDict_Check(d) &&
 // torch's Module.__call__, so it must be one whose call is its forward alone:
 // no hooks on it, none global, nothing overridden.
 PyObject *py_conv_norm_act(PyObject *, PyObject *const *args, Py_ssize_t count) {
+  HANDLE_TH_ERRORS
   if (count != 5) {
     PyErr_SetString(PyExc_TypeError, "conv_norm_act(conv, norm, act, x, residual)");
     return nullptr;
@@ -712,9 +726,9 @@ PyObject *py_conv_norm_act(PyObject *, PyObject *const *args, Py_ssize_t count) 
   }
   ep.residual = args[4];
   Py_INCREF(l);
-  PyObject *result = run_layer(l, d, args[3], ep);
-  Py_DECREF(l);
-  return result;
+  const Ref keep(reinterpret_cast<PyObject *>(l));
+  return run_layer(l, d, args[3], ep);
+  END_HANDLE_TH_ERRORS
 }
 
 // bind(addresses: dict name -> int, sparse_tensor, conv_types, norm_types, activations, global_hooks)

@@ -1,0 +1,22 @@
+"""The extension module with the host side of layer calls, as far as it needs no GPU."""
+import pytest
+import torch
+
+import minuet_amd as minuet
+from minuet_amd.nn.functional import _C
+
+
+def test_what_torch_throws_reaches_the_caller():
+    """A tensor without storage (here a sparse one) makes const_data_ptr throw
+    inside the module: a Python exception, not the end of the process."""
+    host = _C.load_host()
+    norm = minuet.nn.BatchNorm(4).eval()
+    norm._buffers["running_mean"] = torch.zeros(4).to_sparse()
+    with pytest.raises(RuntimeError):
+        host.Affine(norm, torch.ones(4), torch.zeros(4))
+    conv = minuet.nn.SparseConv3d(4, 4, 3)
+    weights, conv._parameters["kernel"] = conv.kernel.detach(), conv.kernel.detach().to_sparse()
+    with pytest.raises(RuntimeError):
+        host.Layer(conv, host.IMPLICIT, weights, weights, None, 0, None)
+    conv._parameters["kernel"] = weights                 # and the module is as usable as before
+    assert type(host.Layer(conv, host.IMPLICIT, weights, weights, None, 0, None)) is host.Layer
