@@ -276,9 +276,12 @@ PyObject *layer_new(PyTypeObject *type, PyObject *args, PyObject *) {
   const at::Tensor *w = tensor_of(weights);
   PyObject *parameters = d == nullptr ? nullptr : look(d, s__parameters);
   PyObject *config = d == nullptr ? nullptr : look(d, s__tunable_config);
+  // (a pruned, normalised or parametrised kernel or bias is no parameter of the
+  // module but made anew from others: nothing here would see it change)
   if (parameters == nullptr || config == nullptr || w == nullptr || w->dim() != 3 || tensor_of(packed) == nullptr ||
-      !w->is_contiguous()) {
-    PyErr_SetString(PyExc_ValueError, "Layer needs a convolution module, its weights and their packed copy");
+      !w->is_contiguous() || tensor_of(look(parameters, s_kernel)) == nullptr || look(parameters, s_bias) == nullptr) {
+    PyErr_SetString(PyExc_ValueError, "Layer needs a convolution module whose kernel and bias are its own parameters, "
+                                      "its weights and their packed copy");
     return nullptr;
   }
   Ref made(type->tp_alloc(type, 0));

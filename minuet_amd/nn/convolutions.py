@@ -960,8 +960,9 @@ class SparseConv(Module):
             cache._fast_maps.setdefault(shape_id, {})[inputs.stride] = entry
             key = cache._map_key(self.ndim, inputs.stride, stride, self.kernel_size, self.dilation, self.transposed)[0]
             cache._note_fast(("fast", shape_id, inputs.stride, name, key, self.transposed))
-        if not weights.is_contiguous():
-            return
+        parameters = self._parameters
+        if not weights.is_contiguous() or parameters.get("kernel") is None or "bias" not in parameters:
+            return                                  # (a pruned or parametrised kernel is made anew from others)
         self._fast = host.Layer(self, kind, weights, packed, shape_id, 1 if name == "TABLES" and
                                 self._allow_shortcut_matmul else 0,
                                 None if self.bias is None else self.bias.detach().float())

@@ -1,6 +1,8 @@
 """Layer calls from the second on, which take the extension module's way."""
 import pytest
 import torch
+import torch.nn.utils.parametrize
+import torch.nn.utils.prune as prune
 
 import minuet_amd as minuet
 from minuet_amd.nn import functional as F
@@ -37,3 +39,35 @@ def test_no_memory_left_is_an_exception():
         finally:
             torch.cuda.set_per_process_memory_fraction(1.0)
         assert torch.equal(conv(x).F, first)
+
+
+class Twice(torch.nn.Module):
+    def forward(self, kernel):
+        return 2 * kernel
+
+
+@pytest.mark.parametrize("made_by", ["prune kernel", "prune bias", "weight_norm", "parametrization"])
+def test_parameters_made_from_others(made_by):
+    """Call after call, and after what they are made from has changed."""
+    conv, x = layer_and_input(3000, 32, 32, torch.float16, bias=True)
+    plain, _ = layer_and_input(3000, 32, 32, torch.float16, bias=True)
+    conv(x)
+    conv(x)                                              # (a Layer is there when the parameter goes)
+    if made_by == "weight_norm":
+        torch.nn.utils.weight_norm(conv, "kernel")
+    elif made_by == "parametrization":
+        torch.nn.utils.parametrize.register_parametrization(conv, "kernel", Twice())
+    else:
+        prune.identity(conv, made_by.split()[1])
+    with torch.no_grad():
+        for step in range(3):
+            if step == 1:
+                source = {"prune kernel": "kernel_orig", "prune bias": "bias_orig", "weight_norm": "kernel_g"}.get(made_by)
+                part = conv.parametrizations.kernel.original if source is None else getattr(conv, source)
+                part.mul_(3.0)
+            results = [conv(x).F for _ in range(3)]
+            plain.kernel.copy_(conv.kernel)
+            plain.bias.copy_(conv.bias)
+            plain._kernel_map_cache.reset()
+            for y in results:
+                assert torch.equal(y, plain(x).F)

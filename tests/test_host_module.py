@@ -1,6 +1,7 @@
 """The extension module with the host side of layer calls, as far as it needs no GPU."""
 import pytest
 import torch
+import torch.nn.utils.prune
 
 import minuet_amd as minuet
 from minuet_amd.nn.functional import _C
@@ -20,3 +21,13 @@ def test_what_torch_throws_reaches_the_caller():
         host.Layer(conv, host.IMPLICIT, weights, weights, None, 0, None)
     conv._parameters["kernel"] = weights                 # and the module is as usable as before
     assert type(host.Layer(conv, host.IMPLICIT, weights, weights, None, 0, None)) is host.Layer
+
+
+@pytest.mark.parametrize("name", ["kernel", "bias"])
+def test_no_layer_for_parameters_made_from_others(name):
+    host = _C.load_host()
+    conv = minuet.nn.SparseConv3d(4, 4, 3, bias=True)
+    torch.nn.utils.prune.identity(conv, name)
+    weights = conv.kernel.detach()
+    with pytest.raises(ValueError, match="its own parameters"):
+        host.Layer(conv, host.IMPLICIT, weights, weights, None, 0, None)
