@@ -775,10 +775,11 @@ class SparseConv(Module):
         key = (kernel.data_ptr(), kernel._version, kernel.dtype, kernel.device, pad)
         if self._packed is None or self._packed[0] != key:
             with torch.no_grad():
-                weights = kernel.detach()
+                # (kept too: its storage cannot become another kernel's while the key names its address)
+                weights = held = kernel.detach()
                 if pad:
                     weights = torch.nn.functional.pad(weights, (0, 0, 0, pad))
-                self._packed = (key, weights, F.pack_weights(weights))
+                self._packed = (key, weights, F.pack_weights(weights), held)
         return self._packed[1], self._packed[2]
 
     def _row_padding(self, features: torch.Tensor) -> int:

@@ -202,3 +202,16 @@ def test_lookahead_layout_places_every_output():
     for bad in ((("tables", sub, True),), (("coords", two, (4, 4, 4)),), (("dense", down),), ()):
         with pytest.raises(ValueError):
             AheadLayout(bad, cache._kernel_offsets, one, 1 << 14, 3, torch.int32, None, 1)
+
+
+def test_padded_weights_are_those_of_the_present_kernel(monkeypatch):
+    """A kernel put in another's place is packed anew, also where the allocator
+    hands it the same memory."""
+    monkeypatch.setattr(minuet.nn.functional, "pack_weights", lambda weights: weights.clone())
+    conv = minuet.nn.SparseConv3d(3, 8, 3)
+    with torch.no_grad():
+        for value in range(1, 40):
+            del conv.kernel
+            conv.kernel = torch.nn.Parameter(torch.full((27, 3, 8), float(value)))
+            weights, packed = conv._packed_kernel(1)
+            assert bool((weights[:, :3] == value).all()) and bool((packed[:, :3] == value).all())
