@@ -906,16 +906,18 @@ class SparseConv(Module):
             # the route depends on the layer, the feature type, the tunable
             # dataflow and, in fp32, the size: decided once, then looked up
             dataflow = self._tunable_config.get("dataflow", "auto")
-            hits = (sources.dtype == torch.float32 and dataflow == "auto" and sources.is_cuda
-                    and self.kernel.dtype == torch.float32
-                    and F.prefers_hits(self.kernel.shape[0], self.in_channels, self.out_channels, sources.dtype,
-                                       sources.shape[0]))
+            volume = self.kernel.shape[0]
+            hits = None                             # (None: the rows do not matter)
+            if (sources.dtype == torch.float32 and dataflow == "auto" and volume > 1 and sources.is_cuda
+                    and self.kernel.dtype == torch.float32):
+                hits = F.prefers_hits(volume, self.in_channels, self.out_channels, sources.dtype, sources.shape[0])
             route_key = (sources.dtype, sources.is_cuda, dataflow, hits)
             route = self._routes.get(route_key)
             if route is None:
                 grouped = self._takes_offset_groups(sources)
                 pad = 0 if grouped else self._row_padding(sources)
-                route = (pad, not grouped and (hits or self._takes_implicit(sources, pad)), grouped)
+                implicit = self._takes_implicit(sources, pad) if hits is None else hits
+                route = (pad, not grouped and implicit, grouped)
                 self._routes[route_key] = route
             pad, implicit, grouped = route
             groups = cache.get_offset_groups(**map_args) if grouped and self._tuning_data is None else None

@@ -1410,6 +1410,7 @@ def kernel_map_invert(kernel_map: torch.Tensor, num_sources: int) -> torch.Tenso
 
 IMPLICIT_MAX_TARGET_FEATURES = 512
 IMPLICIT_MAX_SOURCE_ROW_BYTES = 2048
+IMPLICIT_MAX_SOURCE_BYTES = 0xFFFFF000           # source rows are addressed through 32-bit buffer offsets
 
 
 IMPLICIT_NARROW_LDS_BYTES = 64 * 1024

@@ -9,7 +9,7 @@ from ..kernel_map import KernelMap
 
 __all__ = ["cuda_time_gather", "cuda_time_scatter", "sparse_convolution_forward",
            "cuda_time_gemm", "set_gemm_parallel_level", "Epilogue", "pack_weights",
-           "prefers_implicit", "prefers_hits"]
+           "prefers_implicit", "prefers_hits", "hits_rows_limit"]
 
 pack_weights = _C.pack_weights
 
@@ -35,9 +35,9 @@ def prefers_implicit(num_offsets: int, num_source_features: int, num_target_feat
     bytes and up to 128 output channels, and for rows of up to 256 bytes with up
     to 64 output channels under kernels of more than 8 offsets (beyond that its
     matrix work on empty (offset, target) pairs outweighs the buffer traffic it
-    saves).  fp32 matrix work is 16x dearer, so there it only pays where most
-    (offset, target) pairs are hits, i.e. for small layers with strided 2^D
-    kernels."""
+    saves).  An fp32 layer of more than one offset goes by its rows instead
+    (``hits_rows_limit``); without rows to go by, this says yes to the narrow
+    ones with strided 2^D kernels, whose (offset, target) pairs are mostly hits."""
     if not _C.implicit_forward_supported(num_source_features, num_target_features, dtype, num_offsets):
         return False
     if dtype != torch.float32:
@@ -48,18 +48,31 @@ def prefers_implicit(num_offsets: int, num_source_features: int, num_target_feat
     return num_offsets <= 8 and num_source_features * num_target_features <= 1024
 
 
+def hits_rows_limit(num_offsets: int, num_source_features: int, num_target_features: int,
+                    dtype: torch.dtype) -> int:
+    """The most source rows over which ``dataflow="auto"`` takes the single-kernel
+    form for an fp32 layer of more than one offset (-1: over none).  That form
+    multiplies hits only, 16 at a time, and reads the weights again for every
+    16: measured to be the faster one for narrow layers of any size (32 -> 32
+    channels: 4.9 against 11.4 us over 3 000 voxels, 52 against 76 over 200 000)
+    and for others up to 75 million rows x channels in x channels out (64 -> 64
+    over 12 000 voxels 14.9 against 18.8 us, over 20 000 27.9 and 24.6; 128 ->
+    128 over 3 000 19.1 and 21.4).  It addresses source rows through 32-bit
+    buffer offsets, so features of 4 GiB and more go to the three kernels
+    whatever the width."""
+    if (dtype != torch.float32 or num_offsets <= 1
+            or not _C.implicit_forward_supported(num_source_features, num_target_features, dtype)):
+        return -1
+    most = (_C.IMPLICIT_MAX_SOURCE_BYTES - 1) // (num_source_features * dtype.itemsize)
+    work = num_source_features * num_target_features
+    return most if work <= 1024 else min(most, 75_000_000 // work)
+
+
 def prefers_hits(num_offsets: int, num_source_features: int, num_target_features: int, dtype: torch.dtype,
                  num_rows: int) -> bool:
     """Whether ``dataflow="auto"`` takes the single-kernel form for an fp32 layer
-    over ``num_rows`` source rows.  That form multiplies hits only, 16 at a time,
-    and reads the weights again for every 16: measured to be the faster one for
-    narrow layers of any size (32 -> 32 channels: 4.9 against 11.4 us over 3 000
-    voxels, 52 against 76 over 200 000) and for others up to 75 million rows x
-    channels in x channels out (64 -> 64 over 12 000 voxels 14.9 against 18.8 us,
-    over 20 000 27.9 and 24.6; 128 -> 128 over 3 000 19.1 and 21.4)."""
-    work = num_source_features * num_target_features
-    return (dtype == torch.float32 and num_offsets > 1 and (work <= 1024 or num_rows * work <= 75_000_000)
-            and _C.implicit_forward_supported(num_source_features, num_target_features, dtype))
+    over ``num_rows`` source rows (``hits_rows_limit``)."""
+    return num_rows <= hits_rows_limit(num_offsets, num_source_features, num_target_features, dtype)
 
 
 def cuda_time_gather(weights: torch.Tensor, source_masks: torch.Tensor,
@@ -153,10 +166,10 @@ def sparse_convolution_forward(sources: torch.Tensor, weights: torch.Tensor,
     if dataflow == "implicit" and dense is None:
         raise ValueError("the implicit dataflow needs a KernelMap with its dense map")
     if dense is not None and dataflow in ("auto", "implicit"):
-        if (dataflow == "implicit" or prefers_implicit(weights.shape[0], weights.shape[1],
-                                                       weights.shape[2], weights.dtype)
-                or prefers_hits(weights.shape[0], weights.shape[1], weights.shape[2], weights.dtype,
-                                sources.shape[0])):
+        shape = (weights.shape[0], weights.shape[1], weights.shape[2], weights.dtype)
+        if dataflow == "implicit" or (prefers_hits(*shape, sources.shape[0])
+                                      if weights.dtype == torch.float32 and weights.shape[0] > 1
+                                      else prefers_implicit(*shape)):
             return _C.sparse_convolution_forward_implicit(sources, weights, dense, epilogue=epilogue,
                                                           packed_weights=packed_weights)
     if dataflow == "list_driven":

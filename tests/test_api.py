@@ -170,6 +170,16 @@ def test_auto_dataflow_rule():
     assert prefers(8, 32, 32, single) and not prefers(27, 32, 32, single) and not prefers(8, 64, 64, single)
 
 
+def test_fp32_rule_stops_at_the_rows_that_can_be_addressed():
+    """Narrow layers go to the single-kernel form at any size but one: features
+    of 4 GiB, which that form cannot address, stay with the three kernels."""
+    prefers, single = minuet.nn.functional.prefers_hits, torch.float32
+    most = (0xFFFFF000 - 1) // (32 * 4)
+    for offsets in (8, 27):
+        assert prefers(offsets, 32, 32, single, most) and not prefers(offsets, 32, 32, single, most + 1)
+    assert not prefers(27, 4, 4, single, 2 ** 28) and prefers(27, 4, 4, single, 2 ** 27)
+
+
 def test_lookahead_layout_places_every_output():
     """The plan of a look-ahead session (no GPU needed): every output of every
     recipe entry gets a 256-byte aligned place of its own inside one allocation,
