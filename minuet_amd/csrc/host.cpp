@@ -251,6 +251,11 @@ struct Layer {
   int64_t gather_tile_value, scatter_tile_value;
   int64_t num_offsets, in_channels, out_channels;
   int64_t item_size;
+  // The source rows for which this kind is the one to take, and the module's
+  // Layer for the others, if it has run on such a cloud (both null and 0 to
+  // the most there are where the choice does not depend on rows).
+  int64_t rows_from, rows_to;
+  PyObject *other;
 };
 
 void layer_dealloc(PyObject *self) {
@@ -258,18 +263,23 @@ void layer_dealloc(PyObject *self) {
   l->kernel.clear();
   l->bias.clear();
   for (PyObject **o : {&l->weights, &l->packed, &l->stride, &l->dilation, &l->kernel_size, &l->shape_id,
-                       &l->dataflow, &l->threshold, &l->gather_tile, &l->scatter_tile, &l->bias_shift}) {
+                       &l->dataflow, &l->threshold, &l->gather_tile, &l->scatter_tile, &l->bias_shift, &l->other}) {
     Py_CLEAR(*o);
   }
   Py_TYPE(self)->tp_free(self);
 }
 
-// Layer(module, kind, weights, packed, shape_id, shortcut, bias_shift)
+PyTypeObject LayerType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+// Layer(module, kind, weights, packed, shape_id, shortcut, bias_shift, rows_from, rows_to, other)
 PyObject *layer_new(PyTypeObject *type, PyObject *args, PyObject *) {
   HANDLE_TH_ERRORS
   PyObject *module, *weights, *packed, *shape_id, *bias_shift;
+  PyObject *other = Py_None;
   int kind, shortcut;
-  if (!PyArg_ParseTuple(args, "OiOOOiO", &module, &kind, &weights, &packed, &shape_id, &shortcut, &bias_shift)) {
+  long long rows_from = 0, rows_to = INT64_MAX;
+  if (!PyArg_ParseTuple(args, "OiOOOiO|LLO", &module, &kind, &weights, &packed, &shape_id, &shortcut, &bias_shift,
+                        &rows_from, &rows_to, &other)) {
     return nullptr;
   }
   PyObject *d = dict_of(module);
@@ -307,6 +317,17 @@ PyObject *layer_new(PyTypeObject *type, PyObject *args, PyObject *) {
   l->gather_tile = hold(look(config, s_gather_tile_size));
   l->scatter_tile = hold(look(config, s_scatter_tile_size));
   l->bias_shift = hold(bias_shift);
+  l->rows_from = rows_from;
+  l->rows_to = rows_to;
+  if (Py_TYPE(other) == &LayerType) {                    // the module's Layer so far
+    Layer *last = reinterpret_cast<Layer *>(other);
+    if (last->kind != kind) {
+      Py_CLEAR(last->other);                             // two at most, and no circle
+      l->other = hold(other);
+    } else if (last->other != nullptr) {
+      l->other = hold(last->other);
+    }
+  }
   l->kind = kind;
   l->shortcut = shortcut;
   l->device = w->device().index();
@@ -322,8 +343,6 @@ PyObject *layer_new(PyTypeObject *type, PyObject *args, PyObject *) {
   return PyErr_Occurred() ? nullptr : made.release();
   END_HANDLE_TH_ERRORS
 }
-
-PyTypeObject LayerType = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
 // ------------------------------------------------------------------- runs ----
 
@@ -407,6 +426,17 @@ PyObject *none() { Py_RETURN_NONE; }
 
 // The layer on `inputs`; None when anything is not as the Layer describes it.
 PyObject *run_layer(Layer *l, PyObject *module_dict, PyObject *inputs, const EpilogueArgs &ep) {
+  // the one of the module's Layers that is for so many rows
+  if (Py_TYPE(inputs) != g_sparse_tensor) return none();
+  PyObject *in = dict_of(inputs);
+  const at::Tensor *x = in == nullptr ? nullptr : tensor_of(look(in, s__features));
+  if (x == nullptr || x->dim() != 2) return none();
+  const int64_t S = x->size(0);
+  if (S < l->rows_from || S > l->rows_to) {
+    if (l->other == nullptr) return none();
+    l = reinterpret_cast<Layer *>(l->other);
+    if (S < l->rows_from || S > l->rows_to) return none();
+  }
   // the module: same parameters, same settings, not being tuned
   PyObject *parameters = look(module_dict, s__parameters);
   PyObject *config = look(module_dict, s__tunable_config);
@@ -424,14 +454,10 @@ PyObject *run_layer(Layer *l, PyObject *module_dict, PyObject *inputs, const Epi
     if (kernel.requires_grad() || (b != nullptr && b->requires_grad())) return none();
   }
   // the input
-  if (Py_TYPE(inputs) != g_sparse_tensor) return none();
-  PyObject *in = dict_of(inputs);
-  if (in == nullptr) return none();
-  const at::Tensor *x = tensor_of(look(in, s__features));
   PyObject *coordinates = look(in, s__coordinates), *stride = look(in, s__stride);
   PyObject *batch_dims = look(in, s__batch_dims);
-  if (x == nullptr || coordinates == nullptr || stride == nullptr || batch_dims == nullptr) return none();
-  if (x->dim() != 2 || x->size(1) != l->in_channels || x->scalar_type() != kernel.scalar_type() || !x->is_cuda() ||
+  if (coordinates == nullptr || stride == nullptr || batch_dims == nullptr) return none();
+  if (x->size(1) != l->in_channels || x->scalar_type() != kernel.scalar_type() || !x->is_cuda() ||
       x->device().index() != l->device || !x->is_contiguous() || (c10::GradMode::is_enabled() && x->requires_grad())) {
     return none();
   }
@@ -439,7 +465,6 @@ PyObject *run_layer(Layer *l, PyObject *module_dict, PyObject *inputs, const Epi
   if (reinterpret_cast<uintptr_t>(source) % 16 != 0 || c10::hip::current_device() != l->device) return none();
   // its kernel map
   PyObject *out_coordinates = coordinates, *out_stride = stride, *out_batch_dims = batch_dims;
-  const int64_t S = x->size(0);
   int64_t T = S;
   MapEntry *map = nullptr;
   const at::Tensor *identity = nullptr;

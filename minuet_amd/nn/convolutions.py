@@ -26,6 +26,7 @@ from minuet_amd.utils.helpers import as_tuple, generate_kernel_offsets
 
 __all__ = ["SparseConv", "SparseConv3d", "KernelMapCache"]
 
+_MOST_ROWS = (1 << 63) - 1
 _TRANSPOSED_FIRST = ("Layer must transpose=True must have its corresponding non-transposed layer "
                      "before its execution")
 
@@ -878,6 +879,7 @@ class SparseConv(Module):
                                       epilogue.negative_slope)
             bias = None
         made = None                                 # (kind, weights, packed, map pointers, owners, index code)
+        rows = ()                                   # from how many to how many rows that kind is the one to take
         if self.is_trivial:
             features, made = self._pointwise(inputs.F, epilogue)
             coordinates, stride, batch_dims = inputs.C, inputs.stride, inputs.batch_dims
@@ -910,7 +912,9 @@ class SparseConv(Module):
             hits = None                             # (None: the rows do not matter)
             if (sources.dtype == torch.float32 and dataflow == "auto" and volume > 1 and sources.is_cuda
                     and self.kernel.dtype == torch.float32):
-                hits = F.prefers_hits(volume, self.in_channels, self.out_channels, sources.dtype, sources.shape[0])
+                most = F.hits_rows_limit(volume, self.in_channels, self.out_channels, sources.dtype)
+                hits = sources.shape[0] <= most
+                rows = (0, most) if hits else (most + 1, _MOST_ROWS)
             route_key = (sources.dtype, sources.is_cuda, dataflow, hits)
             route = self._routes.get(route_key)
             if route is None:
@@ -945,12 +949,15 @@ class SparseConv(Module):
         if batch_dims is not None and len(batch_dims) <= 2:
             batch_dims = None
         if made is not None and made[2] is not None and self._tuning_data is None:
-            self._keep_fast(made, inputs, features, coordinates, stride, batch_dims)
+            self._keep_fast(made, rows, inputs, features, coordinates, stride, batch_dims)
         return SparseTensor.like(inputs, features, coordinates, stride, batch_dims)
 
-    def _keep_fast(self, made, inputs, features, coordinates, stride, batch_dims):
+    def _keep_fast(self, made, rows, inputs, features, coordinates, stride, batch_dims):
         """Leaves what this call worked out for the extension module: the module's
-        side of it in ``_fast``, the map's side in the cache's ``_fast_maps``."""
+        side of it in ``_fast``, the map's side in the cache's ``_fast_maps``.
+        Where the kind depends on the size (``rows``), the Layer of the other kind
+        stays with the new one: each cloud gets the kernel that a fresh cache
+        would give it, whatever came before."""
         name, weights, packed, pointers, owners, index_code = made
         host = _C.load_host()
         kind = getattr(host, name)
@@ -968,7 +975,8 @@ class SparseConv(Module):
             return                                  # (a pruned or parametrised kernel is made anew from others)
         self._fast = host.Layer(self, kind, weights, packed, shape_id, 1 if name == "TABLES" and
                                 self._allow_shortcut_matmul else 0,
-                                None if self.bias is None else self.bias.detach().float())
+                                None if self.bias is None else self.bias.detach().float(),
+                                *(rows and (*rows, self._fast)))
 
     def _forward_tables(self, cache, map_args, sources, epilogue):
         """Gather -> GEMM -> Scatter through the rank tables (the reference's

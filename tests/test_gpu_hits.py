@@ -57,3 +57,31 @@ def test_layer_takes_it_by_size():
         wanted = reference(x.F.double(), conv.kernel.detach().double(), dense)
         results.append(float((out.double() - wanted).norm() / wanted.norm()))
     assert max(results) < 1e-6
+
+
+def test_kernel_follows_the_size_of_each_cloud():
+    """One layer and one cache over small, large and small clouds again: every one
+    runs the kernel that a fresh cache gives it, its second pass too, in each
+    order and from a plan that the cloud before has left."""
+    gen = torch.Generator(device=DEVICE).manual_seed(4)
+    torch.manual_seed(0)
+    conv = minuet.nn.SparseConv3d(64, 64, 3, dtype=torch.float32, device=DEVICE)
+    inputs = []
+    for rows in (2000, 40000):
+        cells = torch.randperm(1 << 16, generator=gen, device=DEVICE)[:rows]
+        coordinates = torch.stack([cells >> 10, (cells >> 5) & 31, cells & 31], 1).int()
+        coordinates = coordinates[F.build_sorted_index(coordinates)]
+        x = minuet.SparseTensor(torch.randn(rows, 64, generator=gen, device=DEVICE), coordinates)
+        minuet.set_kernel_map_cache(conv, minuet.nn.KernelMapCache(3, torch.int32, DEVICE))
+        conv.invalidate_cached_weights()
+        with torch.no_grad():
+            inputs.append((x, conv(x).F))
+    cache = minuet.nn.KernelMapCache(3, torch.int32, DEVICE)
+    minuet.set_kernel_map_cache(conv, cache)
+    conv.invalidate_cached_weights()
+    with torch.no_grad():
+        for large in (0, 0, 1, 1, 0, 1, 0, 0):
+            x, expected = inputs[large]
+            cache.reset()
+            assert torch.equal(conv(x).F, expected)      # bit for bit: the two kernels add up in different orders
+            assert torch.equal(conv(x).F, expected)
