@@ -244,7 +244,6 @@ struct Layer {
   PyObject *stride, *dilation, *kernel_size;  // the module's settings, by identity
   PyObject *shape_id;                         // key of this layer's map inside the cache's _fast_maps
   PyObject *dataflow, *threshold, *gather_tile, *scatter_tile;
-  PyObject *bias_shift;                       // fp32 copy of the bias, or None
   int kind, float_code, device;
   int shortcut, has_threshold;
   double threshold_value;
@@ -263,7 +262,7 @@ void layer_dealloc(PyObject *self) {
   l->kernel.clear();
   l->bias.clear();
   for (PyObject **o : {&l->weights, &l->packed, &l->stride, &l->dilation, &l->kernel_size, &l->shape_id,
-                       &l->dataflow, &l->threshold, &l->gather_tile, &l->scatter_tile, &l->bias_shift, &l->other}) {
+                       &l->dataflow, &l->threshold, &l->gather_tile, &l->scatter_tile, &l->other}) {
     Py_CLEAR(*o);
   }
   Py_TYPE(self)->tp_free(self);
@@ -271,15 +270,15 @@ void layer_dealloc(PyObject *self) {
 
 PyTypeObject LayerType = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
-// Layer(module, kind, weights, packed, shape_id, shortcut, bias_shift, rows_from, rows_to, other)
+// Layer(module, kind, weights, packed, shape_id, shortcut, rows_from, rows_to, other)
 PyObject *layer_new(PyTypeObject *type, PyObject *args, PyObject *) {
   HANDLE_TH_ERRORS
-  PyObject *module, *weights, *packed, *shape_id, *bias_shift;
+  PyObject *module, *weights, *packed, *shape_id;
   PyObject *other = Py_None;
   int kind, shortcut;
   long long rows_from = 0, rows_to = INT64_MAX;
-  if (!PyArg_ParseTuple(args, "OiOOOiO|LLO", &module, &kind, &weights, &packed, &shape_id, &shortcut, &bias_shift,
-                        &rows_from, &rows_to, &other)) {
+  if (!PyArg_ParseTuple(args, "OiOOOi|LLO", &module, &kind, &weights, &packed, &shape_id, &shortcut, &rows_from,
+                        &rows_to, &other)) {
     return nullptr;
   }
   PyObject *d = dict_of(module);
@@ -316,7 +315,6 @@ PyObject *layer_new(PyTypeObject *type, PyObject *args, PyObject *) {
   l->threshold = hold(look(config, s_threshold));
   l->gather_tile = hold(look(config, s_gather_tile_size));
   l->scatter_tile = hold(look(config, s_scatter_tile_size));
-  l->bias_shift = hold(bias_shift);
   l->rows_from = rows_from;
   l->rows_to = rows_to;
   if (Py_TYPE(other) == &LayerType) {                    // the module's Layer so far
@@ -503,14 +501,17 @@ PyObject *run_layer(Layer *l, PyObject *module_dict, PyObject *inputs, const Epi
     scale = tensor_of(ep.scale);
     if (scale == nullptr || !vector_fits(scale, l->out_channels, l->device)) return none();
   }
-  PyObject *shift_object = ep.shift;
+  at::Tensor bias;
   if (!is_none(l->bias.object)) {
     if (!is_none(ep.scale) || !is_none(ep.shift)) return none();
-    shift_object = l->bias_shift;
-    if (is_none(shift_object)) return none();
+    // (read at every call: a write through .data leaves no mark on the parameter)
+    bias = THPVariable_Unpack(l->bias.object);
+    if (bias.scalar_type() != at::kFloat) bias = bias.to(at::kFloat);
+    shift = &bias;
+  } else if (!is_none(ep.shift)) {
+    shift = tensor_of(ep.shift);
   }
-  if (!is_none(shift_object)) {
-    shift = tensor_of(shift_object);
+  if (shift != nullptr || !is_none(ep.shift)) {
     if (shift == nullptr || !vector_fits(shift, l->out_channels, l->device)) return none();
   }
   if (!is_none(ep.residual)) {

@@ -71,3 +71,17 @@ def test_parameters_made_from_others(made_by):
             plain._kernel_map_cache.reset()
             for y in results:
                 assert torch.equal(y, plain(x).F)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_bias_is_read_at_every_call(dtype):
+    """Also one written through ``.data``, which marks nothing."""
+    conv, x = layer_and_input(3000, 32, 32, dtype, bias=True)
+    with torch.no_grad():
+        conv(x)
+        assert conv._fast is not None
+        for step in range(3):
+            conv.bias.data.copy_(torch.randn(32, device=DEVICE))
+            again = conv(x).F
+            conv.invalidate_cached_weights()
+            assert torch.equal(again, conv(x).F)

@@ -18,9 +18,9 @@ def test_what_torch_throws_reaches_the_caller():
     conv = minuet.nn.SparseConv3d(4, 4, 3)
     weights, conv._parameters["kernel"] = conv.kernel.detach(), conv.kernel.detach().to_sparse()
     with pytest.raises(RuntimeError):
-        host.Layer(conv, host.IMPLICIT, weights, weights, None, 0, None)
+        host.Layer(conv, host.IMPLICIT, weights, weights, None, 0)
     conv._parameters["kernel"] = weights                 # and the module is as usable as before
-    assert type(host.Layer(conv, host.IMPLICIT, weights, weights, None, 0, None)) is host.Layer
+    assert type(host.Layer(conv, host.IMPLICIT, weights, weights, None, 0)) is host.Layer
 
 
 @pytest.mark.parametrize("name", ["kernel", "bias"])
@@ -30,4 +30,4 @@ def test_no_layer_for_parameters_made_from_others(name):
     torch.nn.utils.prune.identity(conv, name)
     weights = conv.kernel.detach()
     with pytest.raises(ValueError, match="its own parameters"):
-        host.Layer(conv, host.IMPLICIT, weights, weights, None, 0, None)
+        host.Layer(conv, host.IMPLICIT, weights, weights, None, 0)
