@@ -16,6 +16,7 @@ from typing import Optional, Sequence, Tuple
 
 import numpy as np
 import torch
+from torch.autograd import forward_ad
 
 _LIB_PATH = os.environ.get("MINUET_AMD_LIBRARY") or os.path.join(
     os.path.dirname(os.path.dirname(os.path.dirname(os.path.abspath(__file__)))), "lib",
@@ -1576,6 +1577,25 @@ def cuda_time_gemm(allow_shortcut_matmul, parallel, threshold, weights, source_m
 # --------------------------------------------- before and after the layers ----
 
 MAX_GATHER_SOURCES = 64
+MAX_GATHER_BYTES = 1 << 32                       # of rows that one launch of mnt_gather_rows moves, in pieces of two bytes or more
+MAX_POOL_CLOUDS, MAX_POOL_CHANNELS = 65535, 65536
+
+
+def plain(tensors: Sequence[torch.Tensor]) -> bool:
+    """Whether nothing but the values of these tensors counts, so that a library
+    call may stand in for tensor expressions on them: no gradient is recorded, no
+    tangent carried, nothing batched, traced or seen by a dispatch mode, and none
+    is of a class of its own."""
+    if (torch._C._get_tracing_state() is not None or torch._C._len_torch_dispatch_stack() > 0
+            or torch.compiler.is_compiling()):
+        return False
+    recorded, dual = torch.is_grad_enabled(), forward_ad._current_level >= 0
+    for t in tensors:
+        if (type(t) not in (torch.Tensor, torch.nn.Parameter) or (recorded and t.requires_grad)
+                or torch._C._functorch.is_functorch_wrapped_tensor(t)
+                or (dual and forward_ad.unpack_dual(t).tangent is not None)):
+            return False
+    return True
 
 
 def voxelize(points: torch.Tensor, voxel_size: Sequence[float], dtype: torch.dtype, want_reverse: bool):

@@ -1,7 +1,7 @@
 """Global pooling over each point cloud of a SparseTensor (mirrors
 minuet/nn/functional/pooling.py).  Sums and means of all clouds are one library
-call that reads the batch boundaries on the device; where gradients are
-recorded, and for maxima, they are plain tensor reductions."""
+call that reads the batch boundaries on the device; where gradients or tangents
+are recorded, and for maxima, they are plain tensor reductions."""
 import torch
 
 from . import _C
@@ -17,12 +17,12 @@ def _per_cloud(x, reduce):
 
 
 def _native(x) -> bool:
-    f = x.F
-    return (f.is_cuda and f.dim() == 2 and f.shape[1] > 0 and f.is_contiguous()
-            and f.dtype in (torch.float32, torch.float16, torch.bfloat16)
-            and not (f.requires_grad and torch.is_grad_enabled())
-            and (x.batch_dims is None or (x.batch_dims.is_contiguous()
-                                          and x.batch_dims.dtype in (torch.int32, torch.int64))))
+    f, dims = x.F, x.batch_dims
+    return (f.is_cuda and f.dim() == 2 and 0 < f.shape[1] <= _C.MAX_POOL_CHANNELS and f.shape[0] < 1 << 31
+            and f.dtype in (torch.float32, torch.float16, torch.bfloat16) and f.is_contiguous()
+            and (dims is None or (dims.device == f.device and dims.dtype in (torch.int32, torch.int64)
+                                  and dims.is_contiguous() and dims.shape[0] - 1 <= _C.MAX_POOL_CLOUDS))
+            and _C.plain((f,) if dims is None else (f, dims)))
 
 
 def global_avg_pool(x):

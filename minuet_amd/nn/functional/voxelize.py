@@ -65,10 +65,10 @@ def collate(coordinates: Sequence[torch.Tensor], features: Optional[Sequence[tor
     if features is None:
         return ordered, batch_dims
     first = features[0]
-    if (len(features) <= _C.MAX_GATHER_SOURCES and first.element_size() in (2, 4, 8) and not (
-            torch.is_grad_enabled() and any(f.requires_grad for f in features))
+    if (len(features) <= _C.MAX_GATHER_SOURCES and first.element_size() in (2, 4, 8) and _C.plain(features)
             and all(f.dim() == 2 and f.is_contiguous() and f.dtype == first.dtype and f.shape[1] == first.shape[1]
                     and f.device == stacked.device and f.shape[0] == c.shape[0]
-                    for f, c in zip(features, coordinates)) and first.shape[1] > 0):
+                    for f, c in zip(features, coordinates)) and first.shape[1] > 0
+            and ends[-1] * first.shape[1] * first.element_size() <= _C.MAX_GATHER_BYTES):
         return ordered, batch_dims, _C.gather_rows(features, order)
     return ordered, batch_dims, torch.cat(list(features), dim=0)[order.long()]

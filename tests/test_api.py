@@ -225,3 +225,24 @@ def test_padded_weights_are_those_of_the_present_kernel(monkeypatch):
             conv.kernel = torch.nn.Parameter(torch.full((27, 3, 8), float(value)))
             weights, packed = conv._packed_kernel(1)
             assert bool((weights[:, :3] == value).all()) and bool((packed[:, :3] == value).all())
+
+
+def test_what_a_library_call_may_stand_in_for():
+    """Pools and collating are one library call only where nothing but values counts."""
+    from torch.autograd import forward_ad
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from minuet_amd.nn.functional import _C
+    x, seen = torch.ones(4, 3), []
+    assert _C.plain([x, x]) and not _C.plain([x, torch.ones(2, requires_grad=True)])
+    with torch.no_grad():
+        assert _C.plain([torch.ones(2, requires_grad=True)])
+    with forward_ad.dual_level():
+        assert not _C.plain([x, forward_ad.make_dual(x, x)]) and _C.plain([x])
+    torch.vmap(lambda t: seen.append(_C.plain([t])) or t)(x)
+    torch.func.jvp(lambda t: seen.append(_C.plain([t])) or t, (x,), (x,))
+    torch.func.grad(lambda t: seen.append(_C.plain([t])) or t.sum())(x)
+    torch.jit.trace(lambda t: seen.append(_C.plain([t])) or t + 1, x, check_trace=False)
+    with TorchDispatchMode():
+        seen.append(_C.plain([x]))
+    assert seen and not any(seen)
+    assert not _C.plain([x.as_subclass(type("Own", (torch.Tensor,), {}))])

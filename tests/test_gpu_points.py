@@ -62,3 +62,39 @@ def test_collate_carries_rows(channels, dtype, clouds):
     assert torch.equal(ordered, plain) and torch.equal(dims, plain_dims)
     np.testing.assert_array_equal(host(dims), bounds)
     assert torch.equal(rows, torch.cat(feats)[dev(order.astype(np.int64))])
+
+
+def test_pools_beyond_values():
+    """Tangents, batched features and shapes outside the library call's give what
+    the tensor expressions give."""
+    from torch.autograd import forward_ad
+    c = torch.zeros(900, 3, dtype=torch.int32, device="cuda")
+    dims = torch.tensor([0, 400, 900], dtype=torch.int32, device="cuda")
+    f = torch.randn(900, 8, device="cuda")
+
+    def mean(features, d=dims):
+        return F.global_avg_pool(SparseTensor(features, c, batch_dims=d))
+
+    with forward_ad.dual_level():
+        tangent = forward_ad.unpack_dual(mean(forward_ad.make_dual(f, 2 * f))).tangent
+    torch.testing.assert_close(tangent, 2 * mean(f))
+    one = lambda features: mean(features, None)
+    torch.testing.assert_close(torch.func.jvp(one, (f,), (3 * f,))[1], 3 * one(f))
+    torch.testing.assert_close(torch.vmap(one)(torch.stack([f, -f])), torch.stack([one(f), -one(f)]))
+    torch.testing.assert_close(mean(f, dims.cpu()), mean(f))
+    with torch.no_grad():
+        many = torch.arange(70002, device="cuda").clamp(max=900)            # 70 001 clouds, most of them empty
+        total = F.global_sum_pool(SparseTensor(f, c, batch_dims=many))
+        assert torch.equal(total[:900], f) and not total[900:].any()
+        wide = torch.randn(3, 70000, device="cuda")
+        torch.testing.assert_close(F.global_sum_pool(SparseTensor(wide, c[:3])), wide.sum(0))
+
+
+def test_collate_carries_tangents():
+    from torch.autograd import forward_ad
+    coords = [dev(sorted_unique(random_cloud(50, 30, k))[0]) for k in range(2)]
+    feats = [torch.randn(c.shape[0], 4, device="cuda") for c in coords]
+    plain = F.collate(coords, feats)[2]
+    with forward_ad.dual_level():
+        rows = F.collate(coords, [forward_ad.make_dual(f, 2 * f) for f in feats])[2]
+        assert torch.equal(forward_ad.unpack_dual(rows).tangent, 2 * plain)
