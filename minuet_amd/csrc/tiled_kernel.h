@@ -18,6 +18,13 @@ struct RowSet {
   uint4 v[N];
 };
 
+// A lane's share of the source rows of a stage, and the lanes that have one.
+template <int N>
+struct Rows {
+  uint4 v[N];
+  unsigned long long takers;
+};
+
 typedef unsigned uint4v __attribute__((ext_vector_type(4)));
 
 constexpr unsigned kNowhere = 0xFFFFF000u;     // past the end of every source buffer: reads zeros
@@ -98,8 +105,10 @@ struct TiledShape {
 // channels, and walks the live offsets, 32 * KS bytes of a source row per stage.
 // TILED: the tiles of tiles.hip; otherwise 128 consecutive targets under every
 // offset of the dense map.  Tiled sums are those of implicit_forward_kernel bit
-// for bit (ascending offsets, the same 16 products per matrix instruction), so
-// that a layer may change from one to the other between two calls.
+// for bit (ascending offsets, the same 16 products per matrix instruction) while
+// weights are finite, so that a layer may change from one to the other between
+// two calls.  A weight that is not reaches the targets that share a wavefront
+// with one that uses its offset, in either kernel; which those are differs.
 // PAIRED (rows of up to 64 bytes): a stage is two offsets, one per half of the
 // wavefront's lanes, which halves what a stage costs besides its products.
 // WHOLE: a source row is exactly one stage (or half of one, PAIRED).
@@ -132,7 +141,9 @@ __global__ __launch_bounds__(256 * GROUPS) void tiled_forward_kernel(
   constexpr int kWRows = 256 / kRowPieces;               // weight rows the workgroup loads at a time
   constexpr int kWPieces = (Np + kWRows - 1) / kWRows;   // pieces per thread and stage
   constexpr int kLdsRow = kStageBytes + 16;
-  constexpr int kBufferBytes = Np * kLdsRow;
+  constexpr int kZeros = KS * 32;                        // after the rows of a block of 32 channels
+  constexpr int kBlockStride = 32 * kLdsRow + kZeros;
+  constexpr int kBufferBytes = NB * kBlockStride;
   constexpr int kSlotsPerStage = PAIRED ? 2 : 1;
   constexpr int kMeetBytes = NB * (GROUPS - 1) * 16384;
   constexpr int kLdsBytes = std::max({2 * GROUPS * kBufferBytes, 4 * std::min(NB, GROUPS) * kTurnBytes, kMeetBytes});
@@ -210,7 +221,8 @@ __global__ __launch_bounds__(256 * GROUPS) void tiled_forward_kernel(
     const int row = min(tid / kRowPieces + kWRows * i, Np - 1);
     w_at[i] = static_cast<unsigned>(min(first_channel + row, s.packed_rows - 1) * s.packed_row * ES +
                                     (PAIRED ? w_piece & 3 : w_piece) * 16);
-    w_put[i] = static_cast<unsigned>(row * kLdsRow + w_piece * 16) + group * 2 * kBufferBytes;
+    w_put[i] = static_cast<unsigned>(row / 32 * kBlockStride + row % 32 * kLdsRow + w_piece * 16) +
+               group * 2 * kBufferBytes;
   }
   auto load_w = [&](const Cursor &c) -> RowSet<kWPieces> {
     RowSet<kWPieces> set;
@@ -242,11 +254,12 @@ __global__ __launch_bounds__(256 * GROUPS) void tiled_forward_kernel(
   // them for each of the KS rows.
   constexpr unsigned kPieceStep = PAIRED ? 16u : 32u;
   const unsigned lane_at = (PAIRED ? 0u : h * 16u) + (QUADS ? (lane & (KS - 1)) * kPieceStep : 0u);
-  auto load_rows = [&](int index, const Cursor &c) -> RowSet<KS> {
-    RowSet<KS> set;
+  auto load_rows = [&](int index, const Cursor &c) -> Rows<KS> {
+    Rows<KS> set;
     const unsigned chunk_at = WHOLE || PAIRED ? 0u : static_cast<unsigned>(c.chunk) * kStageBytes;
     const bool take = index >= 0 && (PAIRED ? c.slot + h : c.slot) < live;
     const unsigned row_at = take ? static_cast<unsigned>(index) * row_bytes : kNowhere;
+    set.takers = __ballot(take);
 #pragma unroll
     for (int i = 0; i < KS; ++i) {
       unsigned at = (QUADS ? row_of_lane<KS>(row_at, i) : row_at + i * kPieceStep) + lane_at;
@@ -269,31 +282,46 @@ __global__ __launch_bounds__(256 * GROUPS) void tiled_forward_kernel(
   const Cursor c1 = next(c0), c2 = next(c1), c3 = next(c2);
   int m0 = load_index(c0.slot), m1 = load_index(c1.slot);
   RowSet<kWPieces> w1 = load_w(c0), w0;
-  RowSet<KS> a0 = load_rows(m0, c0), a1;
+  Rows<KS> a0 = load_rows(m0, c0), a1;
   w0 = load_w(c1);
   m0 = load_index(c2.slot);
   a1 = load_rows(m1, c1);
   store_w(0, w1);
+  for (int i = threadIdx.x; i < 2 * GROUPS * NB * kZeros / 16; i += 256 * GROUPS) {
+    *reinterpret_cast<uint4 *>(lds + i / (kZeros / 16) * kBlockStride + 32 * kLdsRow + i % (kZeros / 16) * 16) =
+        make_uint4(0u, 0u, 0u, 0u);
+  }
   w1 = load_w(c2);
   m1 = load_index(c3.slot);
   __syncthreads();
   Cursor at_a = c2, at_w = c3, at_m = next(c3);
-  const unsigned w_get = static_cast<unsigned>(r * kLdsRow + (PAIRED ? h * 64 : h * 16)) + group * 2 * kBufferBytes;
+  // An offset that none of a wavefront's 32 targets has a source under is
+  // multiplied like the others, but by zeros: one infinite or undefined weight
+  // there would make all of their sums undefined.  (Leaving the products out
+  // needs a branch around them: 36 % slower where QUADS turns rows between them.)
+  const unsigned w_here = static_cast<unsigned>(r * kLdsRow + (PAIRED ? h * 64 : h * 16)) + group * 2 * kBufferBytes;
+  const unsigned w_none = 32 * kLdsRow + group * 2 * kBufferBytes;
+  auto weights_for = [&](unsigned long long takers) -> unsigned {
+    const bool any = PAIRED ? (h == 0 ? static_cast<unsigned>(takers) : static_cast<unsigned>(takers >> 32)) != 0u
+                            : takers != 0ull;
+    return any ? w_here : w_none;
+  };
   int left = ((live + kSlotsPerStage * GROUPS - 1) / (kSlotsPerStage * GROUPS) * chunks + 1) >> 1;
-  RowSet<KS> rows;
+  Rows<KS> rows;
 #define MNT_STAGE(A, W, M, BUF)                                                                    \
   {                                                                                                \
     store_w(1 - (BUF), W);                                                                         \
+    const unsigned w_get = weights_for(QUADS ? rows.takers : A.takers);                            \
     uint4 f[KS][NB];                                                                               \
     _Pragma("unroll") for (int kk = 0; kk < KS; ++kk) {                                            \
       _Pragma("unroll") for (int b = 0; b < NB; ++b) {                                             \
         f[kk][b] = *reinterpret_cast<const uint4 *>(lds + (BUF) * kBufferBytes + w_get +           \
-                                                    b * 32 * kLdsRow + kk * kPieceStep);           \
+                                                    b * kBlockStride + kk * kPieceStep);           \
       }                                                                                            \
     }                                                                                              \
     __builtin_amdgcn_sched_barrier(0);                                                             \
     W = load_w(at_w);                                                                              \
-    RowSet<KS> coming = A;                                                                         \
+    Rows<KS> coming = A;                                                                           \
     if (!QUADS) rows = A;                                                                          \
     _Pragma("unroll") for (int kk = 0; kk < KS; ++kk) {                                            \
       _Pragma("unroll") for (int b = 0; b < NB; ++b) acc[b] = Mfma<T>::run(f[kk][b], rows.v[kk], acc[b]); \

@@ -96,6 +96,48 @@ def test_forward_matches_products(targets, offsets, cin, cout, dtype):
     close(_C.sparse_convolution_forward_tiled(x, w, tiles, targets, packed, epilogue=epilogue), wanted, dtype)
 
 
+def tile_rows(tiles, targets):
+    """The targets of every tile's places (-1: none), as test_tiles_are_the_targets reads them."""
+    windows = 8 * max(1, -(-targets // (8 * 4096)))
+    return tiles[:windows * -(--(-targets // windows) // 128) * 128]
+
+
+# both stage forms (two offsets of rows of 64 bytes, one of wider ones), one and two sets of wavefronts,
+# the kernel for large maps, and tiles whose lanes load alone and together
+@pytest.mark.parametrize("cin", [32, 64])
+@pytest.mark.parametrize("targets", [1, 3000, 60000, 70000, 90000])
+def test_undefined_weights_stay_with_their_offsets(targets, cin):
+    """A weight that is not finite reaches the 32 targets of a wavefront that uses
+    its offset, and no others: with it at offsets that nobody uses (the first,
+    the last, one between) every row is what it is without, and with it where one
+    target uses it the rows outside that target's wavefront are."""
+    dense, x, w = operands(targets, 3000, 27, cin, 64, torch.float16)
+    dense[[0, 5, 26]] = -1
+    dense[9] = -1
+    dense[9, targets // 2] = 7
+    spoilt = w.clone()
+    spoilt[[0, 5, 26], 0, 3] = torch.tensor([float("inf"), float("nan"), float("-inf")], device=DEVICE).half()
+    wild = spoilt.clone()
+    wild[9, 1, 2] = float("inf")
+    tiles = _C.kernel_map_tiles(dense)
+    place = tile_rows(tiles, targets).long()
+    plain = torch.arange(-(-targets // 32) * 32, device=DEVICE)
+
+    def rows_without(places):
+        groups = places.view(-1, 32)
+        return groups[~(groups == targets // 2).any(1)].flatten()
+
+    for forward, places in (
+            (lambda weights: _C.sparse_convolution_forward_implicit(x, weights, dense), plain),
+            (lambda weights: _C.sparse_convolution_forward_tiled(x, weights, tiles, targets, F.pack_weights(weights)), place)):
+        wanted = forward(w)
+        assert bool(wanted.isfinite().all())
+        assert torch.equal(forward(spoilt), wanted)
+        others = rows_without(places)
+        others = others[(others >= 0) & (others < targets)]
+        assert torch.equal(forward(wild)[others], wanted[others])
+
+
 def scattered_cloud():
     gen = torch.Generator(device=DEVICE).manual_seed(3)
     cells = torch.randperm(1 << 20, generator=gen, device=DEVICE)[:100000]
