@@ -38,9 +38,10 @@ struct CompactShape {
 //
 // What bounds it: on small clouds one wavefront's chain of map entry, source
 // rows, products (the unit after is asked for before one is multiplied), hence
-// the split; beyond, the weights, which every 16 rows read again: where
-// targets x input x output channels pass 75 million the three-kernel form is
-// the faster one again (see prefers_implicit).  fp32, 3 x 3 x 3, us a layer in
+// the split; beyond, the weights, which every 16 rows read again: from some
+// targets x input x output channels on (78 million for 3 x 3 x 3) the
+// three-kernel form is the faster one again (hits_rows_limit in
+// nn/functional/convolution.py has the line and both sides of it).  fp32, 3 x 3 x 3, us a layer in
 // three kernels and here: 32 -> 32 channels over 3 000 voxels 11.4 / 4.9,
 // 20 000 17.9 / 11.2, 200 000 76 / 52; 64 -> 64 over 3 000 12.1 / 8.4, 12 000
 // 18.8 / 14.9; 256 -> 256 over 135 28 / 22.  (128 targets per workgroup

@@ -51,21 +51,35 @@ def prefers_implicit(num_offsets: int, num_source_features: int, num_target_feat
 def hits_rows_limit(num_offsets: int, num_source_features: int, num_target_features: int,
                     dtype: torch.dtype) -> int:
     """The most source rows over which ``dataflow="auto"`` takes the single-kernel
-    form for an fp32 layer of more than one offset (-1: over none).  That form
-    multiplies hits only, 16 at a time, and reads the weights again for every
-    16: measured to be the faster one for narrow layers of any size (32 -> 32
-    channels: 4.9 against 11.4 us over 3 000 voxels, 52 against 76 over 200 000)
-    and for others up to 75 million rows x channels in x channels out (64 -> 64
-    over 12 000 voxels 14.9 against 18.8 us, over 20 000 27.9 and 24.6; 128 ->
-    128 over 3 000 19.1 and 21.4).  It addresses source rows through 32-bit
-    buffer offsets, so features of 4 GiB and more go to the three kernels
-    whatever the width."""
+    form for an fp32 layer of more than one offset (-1: over none).
+
+    That form multiplies hits only, 16 of one offset at a time, and reads the
+    weights again for every 16; the three kernels read them once per 128 rows
+    of their lists but write and read product rows.  So the line goes by rows x
+    channels in x channels out.  It lies at 2.1 thousand million of them over
+    the number of offsets, because rows have more hits the more offsets there
+    are, and at 110 million at most: over 160 to 190 layers each of 2x2x2
+    strided, 3x3x3 and 5x5x5 (three kinds of scene, 500 to 300 000 voxels, 24 to
+    256 channels) the layers chosen by it take 0.7, 0.7 and 1.7 % longer than by
+    the better choice for each.  Hits only against three kernels, us: 2x2x2 64 ->
+    128 over 10 000 voxels 10.9 / 14.5, 64 -> 64 over 30 000 15.8 / 14.7; 3x3x3 64
+    -> 64 over 10 000 12.3 to 21.0 / 13.0 to 20.6, over 20 000 26.4 / 21.7, 128 ->
+    128 over 3 000 19.0 / 21.3, over 10 000 40.8 / 25.2; 5x5x5 64 -> 64 over 1 000
+    17.7 / 19.4, over 10 000 32.6 to 67 / 25.3 to 40.6.  Up to 32 x 32 channels it
+    is the faster one at any size (3x3x3 over 200 000 52 / 76, 5x5x5 over 100 000
+    63 / 76), or about even (2x2x2 over 300 000 31.5 / 31.7 and, transposed, 36.9
+    / 33.6).
+
+    Source rows are addressed through 32-bit buffer offsets, so features of 4 GiB
+    and more go to the three kernels whatever the width."""
     if (dtype != torch.float32 or num_offsets <= 1
             or not _C.implicit_forward_supported(num_source_features, num_target_features, dtype)):
         return -1
     most = (_C.IMPLICIT_MAX_SOURCE_BYTES - 1) // (num_source_features * dtype.itemsize)
     work = num_source_features * num_target_features
-    return most if work <= 1024 else min(most, 75_000_000 // work)
+    if work <= 1024:
+        return most
+    return min(most, min(110_000_000, 2_100_000_000 // num_offsets) // work)
 
 
 def prefers_hits(num_offsets: int, num_source_features: int, num_target_features: int, dtype: torch.dtype,

@@ -180,6 +180,15 @@ def test_fp32_rule_stops_at_the_rows_that_can_be_addressed():
     assert not prefers(27, 4, 4, single, 2 ** 28) and prefers(27, 4, 4, single, 2 ** 27)
 
 
+def test_fp32_rule_follows_the_kernel_size():
+    """Wider layers change over at fewer rows the more offsets they have."""
+    prefers, single = minuet.nn.functional.prefers_hits, torch.float32
+    assert prefers(8, 64, 128, single, 13000) and not prefers(8, 64, 128, single, 14000)
+    assert prefers(27, 64, 64, single, 18900) and not prefers(27, 64, 64, single, 19100)
+    assert prefers(125, 64, 64, single, 4000) and not prefers(125, 64, 64, single, 4200)
+    assert prefers(125, 32, 32, single, 100000)
+
+
 def test_lookahead_layout_places_every_output():
     """The plan of a look-ahead session (no GPU needed): every output of every
     recipe entry gets a 256-byte aligned place of its own inside one allocation,
