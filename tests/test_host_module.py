@@ -31,3 +31,19 @@ def test_no_layer_for_parameters_made_from_others(name):
     weights = conv.kernel.detach()
     with pytest.raises(ValueError, match="its own parameters"):
         host.Layer(conv, host.IMPLICIT, weights, weights, None, 0)
+
+
+def test_no_thread_local_data_in_the_module():
+    """Thread-local data that nothing reads, in a module loaded late, makes glibc
+    before 2.39 take the slow way to that of every library: 20 % on the host side
+    of each torch operation (ELF program headers of type 7 say that there is some)."""
+    import struct
+    from minuet_amd.build import HOST_PATH
+    _C.load_host()
+    with open(HOST_PATH, "rb") as f:
+        header = f.read(64)
+        assert header[:6] == b"\x7fELF\x02\x01"
+        at, (size, count) = struct.unpack_from("<Q", header, 32)[0], struct.unpack_from("<HH", header, 54)
+        f.seek(at)
+        kinds = [struct.unpack_from("<I", f.read(size))[0] for _ in range(count)]
+    assert 7 not in kinds
