@@ -973,8 +973,9 @@ class SparseConv(Module):
         parameters = self._parameters
         if not weights.is_contiguous() or parameters.get("kernel") is None or "bias" not in parameters:
             return                                  # (a pruned or parametrised kernel is made anew from others)
-        self._fast = host.Layer(self, kind, weights, packed, shape_id, 1 if name == "TABLES" and
-                                self._allow_shortcut_matmul else 0, *(rows and (*rows, self._fast)))
+        # (past Module.__setattr__, which takes longer than all of the rest)
+        self.__dict__["_fast"] = host.Layer(self, kind, weights, packed, shape_id, 1 if name == "TABLES" and
+                                            self._allow_shortcut_matmul else 0, *(rows and (*rows, self._fast)))
 
     def _forward_tables(self, cache, map_args, sources, epilogue):
         """Gather -> GEMM -> Scatter through the rank tables (the reference's

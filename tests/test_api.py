@@ -255,3 +255,23 @@ def test_what_a_library_call_may_stand_in_for():
         seen.append(_C.plain([x]))
     assert seen and not any(seen)
     assert not _C.plain([x.as_subclass(type("Own", (torch.Tensor,), {}))])
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("affine", [True, False])
+def test_batch_norm_affine_is_the_fp32_expression(dtype, affine):
+    """Bit for bit, whatever the type of the module's tensors, which stay as they are."""
+    torch.manual_seed(0)
+    norm = minuet.nn.BatchNorm(37, affine=affine).to(dtype).eval()
+    with torch.no_grad():
+        for t in (*norm.parameters(), norm.running_mean):
+            t.normal_()
+        norm.running_var.uniform_(0.1, 2.0)
+        before = [t.clone() for t in norm.state_dict().values()]
+        scale = torch.rsqrt(norm.running_var.float() + norm.eps)
+        scale = scale * norm.weight.float() if affine else scale
+        shift = -norm.running_mean.float() * scale
+        shift = shift + norm.bias.float() if affine else shift
+        for got, wanted in zip(minuet.nn.fused.batch_norm_affine(norm), (scale, shift)):
+            assert got.dtype == torch.float32 and torch.equal(got, wanted)
+    assert all(torch.equal(a, b) for a, b in zip(before, norm.state_dict().values()))
