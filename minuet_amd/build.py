@@ -62,20 +62,22 @@ def build_host() -> str:
     return HOST_PATH
 
 
-def build_library(verbose: bool = True) -> str:
+def build_library(verbose: bool = True, host: bool = True) -> str:
     """Compile every HIP source, link the shared library and build the host
-    extension.  Always rebuilds."""
+    extension (``host``).  Always rebuilds; the library is there also where the
+    extension cannot be built, which is reported last."""
     os.makedirs(LIB_DIR, exist_ok=True)
     with ThreadPoolExecutor(max_workers=min(8, len(SOURCES) + 1)) as pool:
-        host = pool.submit(build_host)
+        extension = pool.submit(build_host) if host else None
         objects = list(pool.map(_compile, SOURCES))
-        host.result()
     cmd = [_hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *objects, "-o", LIB_PATH]
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"link failed:\n{proc.stdout}\n{proc.stderr}")
     if verbose:
         print(f"built {LIB_PATH}", file=sys.stderr)
+    if extension is not None:
+        extension.result()
     return LIB_PATH
 
 

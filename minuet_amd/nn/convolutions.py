@@ -960,6 +960,8 @@ class SparseConv(Module):
         would give it, whatever came before."""
         name, weights, packed, pointers, owners, index_code = made
         host = _C.load_host()
+        if host is None:
+            return
         kind = getattr(host, name)
         shape_id = None
         if pointers is not None:

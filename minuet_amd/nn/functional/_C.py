@@ -138,7 +138,7 @@ def load_library():
         return _lib
     if not os.path.exists(_LIB_PATH):
         from minuet_amd.build import build_library
-        build_library(verbose=False)
+        build_library(verbose=False, host=False)
     lib = ctypes.CDLL(_LIB_PATH)
     for name, (restype, argtypes) in SIGNATURES.items():
         fn = getattr(lib, name)
@@ -153,15 +153,29 @@ def load_library():
 
 
 _host = None
+_host_failed = False
 
 
 def load_host():
     """The extension module with the host side of layer calls (csrc/host.cpp),
     bound to the library's entry points; loaded once, built first only when no
-    build exists."""
-    global _host
-    if _host is not None:
+    build exists.  None, and one warning, where it can be neither: it is a short
+    cut past Python code that does the same, so layers run without it, each call
+    some 20 us slower on the host."""
+    global _host, _host_failed
+    if _host is not None or _host_failed:
         return _host
+    try:
+        _host = _bound_host()
+    except (RuntimeError, OSError, ImportError) as error:
+        _host_failed = True
+        import warnings
+        warnings.warn(f"[Minuet] no extension module for layer calls, which take the slower way: {error}",
+                      RuntimeWarning, stacklevel=2)
+    return _host
+
+
+def _bound_host():
     import importlib.util
     import torch.nn.modules.module as torch_module
     from minuet_amd.build import HOST_PATH, build_host
@@ -185,7 +199,6 @@ def load_host():
                 (convolutions.SparseConv, convolutions.SparseConv3d),
                 (normalizations.BatchNorm, torch.nn.BatchNorm1d),
                 {cls: ACTIVATION_CODES[name] for cls, name in codes.items()}, hooks)
-    _host = module
     return module
 
 

@@ -46,9 +46,11 @@ def batch_norm_affine(norm: torch.nn.BatchNorm1d):
         shift = (mean.float() * scale).neg_()
         if bias is not None:
             shift += bias.float()
-    kept = (key, scale, shift)
-    if scale.is_cuda:
-        kept += (_C.load_host().Affine(norm, scale, shift),)
+    # (the tensors stay with what was made of them: the key's addresses remain theirs)
+    kept = (key, scale, shift, (mean, var, weight, bias))
+    host = _C.load_host() if scale.is_cuda else None
+    if host is not None:
+        kept += (host.Affine(norm, scale, shift),)
     norm.__dict__["_minuet_affine"] = kept
     return scale, shift
 

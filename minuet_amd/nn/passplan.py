@@ -209,6 +209,8 @@ class BuiltPass:
         """Entries for the extension module: the layers that ran through it in
         the last pass find their maps without a detour through Python."""
         host = _C.load_host()
+        if host is None:
+            return
         index = self.device.index
         for request in self.plan.fast:
             _, shape_id, in_stride, kind, key, transposed = request

@@ -1,11 +1,15 @@
 """Layer calls from the second on, which take the extension module's way."""
+import numpy as np
 import pytest
 import torch
 import torch.nn.utils.parametrize
 import torch.nn.utils.prune as prune
 
 import minuet_amd as minuet
+from helpers import dev, random_cloud, sorted_unique
 from minuet_amd.nn import functional as F
+from minuet_amd.nn.functional import _C
+from minuet_amd.unet import SparseUNet
 
 pytestmark = pytest.mark.gpu
 DEVICE = torch.device("cuda:0")
@@ -85,3 +89,31 @@ def test_bias_is_read_at_every_call(dtype):
             again = conv(x).F
             conv.invalidate_cached_weights()
             assert torch.equal(again, conv(x).F)
+
+
+def test_network_without_the_extension_module(monkeypatch):
+    """The Python code alone: first pass, a pass from a plan, kept maps."""
+    torch.manual_seed(0)
+    net = SparseUNet(4, 16, dtype=torch.float16, device=DEVICE).eval()
+    c, bd = sorted_unique(random_cloud(3000, 30, 1, lo=-9), np.array([0, 1000, 3000], dtype=np.int32))
+    x = minuet.SparseTensor(torch.randn(c.shape[0], 4, device=DEVICE).half(), dev(c), batch_dims=dev(bd))
+
+    def passes():
+        cache = minuet.nn.KernelMapCache(3, torch.int32, DEVICE)
+        minuet.set_kernel_map_cache(net, cache)
+        with torch.no_grad():
+            results = []
+            for _ in range(2):
+                cache.reset()
+                results += [net(x).F, net(x).F]
+        return results
+
+    with_it = passes()
+    assert _C._host is not None
+    monkeypatch.setattr(_C, "_host", None)
+    monkeypatch.setattr(_C, "_host_failed", True)
+    for module in net.modules():
+        if hasattr(module, "invalidate_cached_weights"):
+            module.invalidate_cached_weights()
+    for a, b in zip(with_it, passes()):
+        assert torch.equal(a, b)

@@ -1,4 +1,6 @@
 """The extension module with the host side of layer calls, as far as it needs no GPU."""
+import warnings
+
 import pytest
 import torch
 import torch.nn.utils.prune
@@ -31,6 +33,23 @@ def test_no_layer_for_parameters_made_from_others(name):
     weights = conv.kernel.detach()
     with pytest.raises(ValueError, match="its own parameters"):
         host.Layer(conv, host.IMPLICIT, weights, weights, None, 0)
+
+
+def test_library_does_without_the_module(monkeypatch, tmp_path):
+    """Where it can be neither loaded nor built, one warning and None."""
+    from minuet_amd import build
+
+    def no_compiler():
+        raise RuntimeError("no compiler here")
+    monkeypatch.setattr(_C, "_host", None)
+    monkeypatch.setattr(_C, "_host_failed", False)
+    monkeypatch.setattr(build, "HOST_PATH", str(tmp_path / "minuet_host.so"))
+    monkeypatch.setattr(build, "build_host", no_compiler)
+    with pytest.warns(RuntimeWarning, match="no compiler here"):
+        assert _C.load_host() is None
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert _C.load_host() is None
 
 
 def test_no_thread_local_data_in_the_module():
