@@ -242,6 +242,7 @@ __global__ __launch_bounds__(256) void pass_invert_kernel(InvertJobs jobs) {
 // What mnt_pass_levels leaves for mnt_pass_build (kept in the arena's map
 // state: any other map build in between forgets it).
 struct PassState {
+  const void *coords, *levels, *maps;              // whose state this is
   PassSpecs specs;
   int64_t n, num_batches;
   int ndim, coord_dtype, index_dtype, num_levels, num_maps;
@@ -609,6 +610,9 @@ extern "C" int mnt_pass_levels(const void *coords, int64_t n, int ndim, int coor
     if (bounds_host_out != nullptr) {
       for (int i = 0; i < 8; ++i) bounds_host_out[i] = bounds[i];
     }
+    state.coords = coords;
+    state.levels = levels;
+    state.maps = maps;
     state.n = n;
     state.ndim = ndim;
     state.coord_dtype = coord_dtype;
@@ -629,10 +633,13 @@ extern "C" int mnt_pass_build(const void *coords, const void *batch_dims, mnt_pa
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     Arena &arena = Arena::of(stream);
     MNT_CHECK(arena.pass_pending, "mnt_pass_build called without a preceding mnt_pass_levels");
+    PassState &state = pass_state(arena);
+    // (two threads that take turns on one stream: the first to come back finds the other's state)
+    MNT_CHECK(state.coords == coords && state.levels == levels && state.maps == maps,
+              "mnt_pass_build called for another cloud or other lists than the mnt_pass_levels before it on this stream");
     arena.pass_pending = false;
     MNT_CHECK(coords != nullptr && base != nullptr && reinterpret_cast<uintptr_t>(base) % 256 == 0,
               "the block of a pass must be 256-byte aligned");
-    PassState &state = pass_state(arena);
     for (int i = 0; i < state.num_maps; ++i) {
       MNT_CHECK(!(maps[i].want & MNT_PASS_TABLES) || (maps[i].sizes_host != nullptr && maps[i].order_host != nullptr),
                 "map %d of the pass has nowhere to put its sizes", i);

@@ -102,3 +102,21 @@ def test_second_pass_of_a_network_equals_its_first(kind):
             assert torch.equal(y.C, ref.C) and torch.equal(y.F, ref.F) and torch.equal(again.F, ref.F)
             assert torch.equal(y.batch_dims, ref.batch_dims)
     assert cache.num_coordinate_builds == 16 and cache.num_map_builds == 36
+
+
+def test_build_belongs_to_the_levels_before_it():
+    """Threads that take turns on one stream: what another pass has left there in
+    between is not built into this one's block, and the other goes on."""
+    one, two = (1, 1, 1), (2, 2, 2)
+    requests = [("coords", one, two), ("dense", (one, one, (3, 3, 3), one)), ("dense", (one, two, (2, 2, 2), one))]
+    clouds = [dev(sorted_unique(random_cloud(n, 40, n))[0]) for n in (300, 5000)]
+    plans = [PassPlan(requests, offsets_of, one, torch.int32) for _ in clouds]
+    sizes = [_C.pass_levels(c, None, None, p.levels, p.num_levels, p.maps)[0] for c, p in zip(clouds, plans)]
+    stores = [torch.empty(size, dtype=torch.uint8, device="cuda") for size in sizes]
+    with pytest.raises(RuntimeError, match="another cloud or other lists"):
+        _C.pass_build(clouds[0], None, plans[0].levels, plans[0].maps, stores[0])
+    _C.pass_build(clouds[1], None, plans[1].levels, plans[1].maps, stores[1])
+    dense, _ = _C.kernel_map_dense(clouds[1], clouds[1], offsets_of(one, (3, 3, 3), one), None, None)
+    at = plans[1].maps[plans[1].map_of[requests[1][1]]].at[0]
+    assert torch.equal(stores[1].view(torch.int32)[at // 4:at // 4 + dense.numel()].view_as(dense), dense)
+    assert plans[0].build(clouds[0], None, None) is not None
