@@ -1838,6 +1838,10 @@ void enqueue_tables(std::vector<TableWork> &work, Scope &scope, unsigned long lo
       const size_t bytes = 8 + sizeof(unsigned) * 3 * static_cast<size_t>(w.num_offsets);
       MNT_CHECK(host_at + bytes <= Arena::kPinnedBytes, "too many kernel offsets for one batch of tables");
       w.host_at = static_cast<int>(host_at);
+      // The word may hold what another batch or a single build has left there, by
+      // chance the very number that is waited for.  (Nothing still writes here:
+      // every build waits for its own flag, which comes after its results.)
+      *reinterpret_cast<volatile unsigned long long *>(static_cast<char *>(arena.pinned()) + host_at) = 0;
       char *host = static_cast<char *>(arena.pinned_device()) + host_at;
       job.flag = reinterpret_cast<unsigned long long *>(host);
       job.plan_host = reinterpret_cast<unsigned *>(host + 8);

@@ -120,3 +120,30 @@ def test_build_belongs_to_the_levels_before_it():
     at = plans[1].maps[plans[1].map_of[requests[1][1]]].at[0]
     assert torch.equal(stores[1].view(torch.int32)[at // 4:at // 4 + dense.numel()].view_as(dense), dense)
     assert plans[0].build(clouds[0], None, None) is not None
+
+
+def test_tables_wait_for_their_own_flag():
+    """The word in pinned memory that says a map's tables are complete may hold the
+    order of an earlier map there, whose first two entries then read as a number:
+    whichever number the pass waits for, it is not taken for the flag."""
+    one, key = (1, 1, 1), ((1, 1, 1), (1, 1, 1), (3, 3, 3), (1, 1, 1))
+    offsets = offsets_of(one, (3, 3, 3), one)
+    cloud = dev(sorted_unique(random_cloud(60000, 300, 5))[0])
+    dense, _ = _C.kernel_map_dense(cloud, cloud, offsets, None, None)
+    expected = _C.kernel_map_tables(dense, cloud.shape[0], True)
+    plan = PassPlan([("dense", key), ("tables", key, True)], offsets_of, one, torch.int32)
+    for number in range(1, 27):
+        # a map whose order starts (number, 0): fewest hits under that offset, then under the first
+        counts = np.full(27, 40)
+        counts[[0, number]] = 20, 10
+        earlier = torch.full((27, 64), -1, dtype=torch.int32)
+        for o, count in enumerate(counts):
+            earlier[o, :count] = torch.arange(count, dtype=torch.int32)
+        torch.cuda.synchronize()
+        _C.cuda_device_reset()                           # the numbers start again
+        order = _C.kernel_map_tables(earlier.cuda(), 64, True)["order_host"]
+        assert order[0] == number and order[1] == 0
+        built = plan.build(cloud, None, np.array([0, 0, 0, 0, 299, 299, 299, 0], dtype=np.int64))
+        got = built.tables(key, cloud, True)
+        assert np.array_equal(got.sizes_host, expected["sizes_host"])
+        assert np.array_equal(got.order_host, expected["order_host"])
