@@ -225,6 +225,18 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(GatherSources src, con
 constexpr int kPoolBlock = 256;
 constexpr int kPoolInFlight = 8;
 
+// The rows of a cloud, kept inside the features as a slice of them would be:
+// boundaries come from the caller and are not checked on the host.
+struct CloudRows {
+  long long lo, hi;
+};
+template <typename IT>
+__device__ __forceinline__ CloudRows cloud_rows(const IT *__restrict__ batch_dims, long long cloud, long long n) {
+  if (batch_dims == nullptr) return {0, n};
+  const long long lo = min(max(static_cast<long long>(batch_dims[cloud]), 0ll), n);
+  return {lo, min(max(static_cast<long long>(batch_dims[cloud + 1]), lo), n)};
+}
+
 template <typename T, int VB, typename IT>
 __global__ __launch_bounds__(kPoolBlock) void pool_kernel(const unsigned char *__restrict__ features,
                                                           const IT *__restrict__ batch_dims, long long n, int channels,
@@ -236,8 +248,8 @@ __global__ __launch_bounds__(kPoolBlock) void pool_kernel(const unsigned char *_
   const int groups = kPoolBlock / lanes;
   const int group = threadIdx.x / lanes, lane = threadIdx.x - group * lanes;
   const int piece = blockIdx.z * lanes + lane;
-  const long long lo = batch_dims == nullptr ? 0 : static_cast<long long>(batch_dims[blockIdx.y]);
-  const long long hi = batch_dims == nullptr ? n : static_cast<long long>(batch_dims[blockIdx.y + 1]);
+  const CloudRows cloud = cloud_rows<IT>(batch_dims, blockIdx.y, n);
+  const long long lo = cloud.lo, hi = cloud.hi;
   const long long share = (hi - lo + gridDim.x - 1) / gridDim.x;
   const long long from = lo + blockIdx.x * share;
   const long long to = from + share < hi ? from + share : hi;
@@ -290,8 +302,8 @@ __global__ __launch_bounds__(256) void pool_fold_kernel(const float *__restrict_
   const float *at = partial + cloud * parts * channels + (i - cloud * channels);
   float sum = 0.0f;
   for (int p = 0; p < parts; ++p) sum += at[static_cast<long long>(p) * channels];
-  const long long rows = batch_dims == nullptr ? n : static_cast<long long>(batch_dims[cloud + 1]) -
-                                                         static_cast<long long>(batch_dims[cloud]);
+  const CloudRows of = cloud_rows<IT>(batch_dims, cloud, n);
+  const long long rows = of.hi - of.lo;
   out[i] = static_cast<T>(mean ? sum / static_cast<float>(rows) : sum);
 }
 

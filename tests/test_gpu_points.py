@@ -98,3 +98,17 @@ def test_collate_carries_tangents():
     with forward_ad.dual_level():
         rows = F.collate(coords, [forward_ad.make_dual(f, 2 * f) for f in feats])[2]
         assert torch.equal(forward_ad.unpack_dual(rows).tangent, 2 * plain)
+
+
+@pytest.mark.parametrize("bounds", [[0, 400, 5000], [0, 900, 900], [700, 200, 900], [0, 2000, 3000]])
+@pytest.mark.parametrize("rows", [900, 90000])
+def test_pools_stay_inside_the_features(bounds, rows):
+    """Boundaries past the last row or the wrong way round: what slices give."""
+    bounds = [b * rows // 900 for b in bounds]
+    f = torch.randn(rows, 64, device="cuda")
+    c = torch.zeros(rows, 3, dtype=torch.int32, device="cuda")
+    x = SparseTensor(f, c, batch_dims=torch.tensor(bounds, dtype=torch.int32, device="cuda"))
+    parts = [f[a:b].double() for a, b in zip(bounds, bounds[1:])]
+    torch.testing.assert_close(F.global_sum_pool(x).double(), torch.stack([p.sum(0) for p in parts]), rtol=1e-5, atol=1e-3)
+    torch.testing.assert_close(F.global_avg_pool(x).double(), torch.stack([p.mean(0) for p in parts]), rtol=1e-5, atol=1e-5,
+                               equal_nan=True)
