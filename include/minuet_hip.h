@@ -645,7 +645,10 @@ int mnt_global_pool(const void *features, const void *batch_dims, int64_t n, int
  * mnt_kernel_map_build called one after another.  The reference builds each of
  * them at the first layer that asks (minuet/nn/convolutions.py:58-173).
  *
- * Two calls, with no other library call on that stream in between:
+ * Two calls, with no other library call on that stream in between (a build for
+ * another cloud or other lists than the levels before it is refused, as is one
+ * after mnt_target_coordinates*; mnt_pass_levels in turn ends a pending
+ * mnt_target_coordinates_count):
  *   mnt_pass_levels  marks the levels (level l + 1 = levels[l], its stride a
  *                    multiple of the cloud's; level 0 is the cloud itself),
  *                    waits for their row counts and works out where in one

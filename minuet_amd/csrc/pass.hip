@@ -579,6 +579,7 @@ extern "C" int mnt_pass_levels(const void *coords, int64_t n, int ndim, int coor
     Arena &arena = Arena::of(stream);
     PassState &state = pass_state(arena);
     arena.pass_pending = false;
+    arena.pending.valid = false;             // (the levels' bitmaps lie where a count's result does)
     int inverses = 0, tables = 0;
     for (int i = 0; i < num_maps; ++i) {
       const mnt_pass_map &m = maps[i];

@@ -1,4 +1,6 @@
 """The build of a whole pass (levels and maps at once) against the single calls."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -120,6 +122,16 @@ def test_build_belongs_to_the_levels_before_it():
     at = plans[1].maps[plans[1].map_of[requests[1][1]]].at[0]
     assert torch.equal(stores[1].view(torch.int32)[at // 4:at // 4 + dense.numel()].view_as(dense), dense)
     assert plans[0].build(clouds[0], None, None) is not None
+
+    # a count of target coordinates and the levels of a pass share their block
+    lib, stride, count = _C.load_library(), (ctypes.c_int64 * 3)(2, 2, 2), ctypes.c_int64(0)
+    stream = _C._stream(clouds[0].device)
+    _C._check(lib.mnt_target_coordinates_count(clouds[0].data_ptr(), clouds[0].shape[0], 3, 0, stride, None, 1, 0, None,
+                                               ctypes.byref(count), stream))
+    assert _C.pass_levels(clouds[1], None, None, plans[1].levels, plans[1].num_levels, plans[1].maps)
+    out = torch.empty(count.value, 3, dtype=torch.int32, device="cuda")
+    assert lib.mnt_target_coordinates_fill(out.data_ptr(), None, stream) != 0
+    _C.pass_build(clouds[1], None, plans[1].levels, plans[1].maps, stores[1])
 
 
 def test_tables_wait_for_their_own_flag():
