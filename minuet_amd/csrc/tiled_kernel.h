@@ -123,12 +123,14 @@ struct TiledShape {
 // less, which wait for a tile's longest chain of stages.
 //
 // What bounds it: on small clouds that chain (0.3 us a stage), on large ones
-// the address units and the path from the second-level cache (94 % busy at a
-// million targets under 125 offsets: 26 M source rows of 128 bytes in 416 us,
-// half of them from beyond the L2).  64 -> 64 channels, 16-bit, us a layer
-// before (implicit_forward_kernel) and now: 3 000 targets 14.5 / 8.1, 25 000
-// 14.8 / 10.4, 60 000 17.7 / 16.3; in tiles 120 000 31.4 / 19.8, 200 000
-// 47.8 / 30.3, a million under 5 x 5 x 5 855 / 416.
+// the address units and the path from the second-level cache.  At a million
+// targets under 125 offsets, 25 M source rows of 128 bytes in 0.42 ms, the
+// address units are busy 81 % of the time and the matrix pipes 35 %; of 46 M
+// reads of the second-level cache nine in ten are hits there.  64 -> 64
+// channels, 16-bit, us a layer in implicit_forward_kernel and here: 3 000
+// targets of an object 14.9 / 8.8, 25 000 of a LiDAR scan 14.9 / 10.3, 60 000
+// of a room 18.2 / 17.4; in tiles, LiDAR, 120 000 32.3 / 20.0, 200 000 48.6 /
+// 32.7, a million under 5 x 5 x 5 836 / 424.
 template <typename T, int NB, int KS, bool TILED, bool PAIRED, bool WHOLE, bool QUADS, int GROUPS>
 __global__ __launch_bounds__(256 * GROUPS) void tiled_forward_kernel(
     const T *__restrict__ sources, unsigned source_bytes, const T *__restrict__ wt,

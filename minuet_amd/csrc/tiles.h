@@ -1,6 +1,6 @@
 // Tiles of targets that share their live offsets: what tile_sort_kernel and
 // tile_emit_kernel (tiles.hip) leave of a dense kernel map and
-// tiled_forward_kernel (tiled.hip) walks.
+// tiled_forward_kernel (tiled_kernel.h) walks.
 #pragma once
 
 #include <algorithm>

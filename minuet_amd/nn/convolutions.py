@@ -57,7 +57,16 @@ class KernelMapCache(object):
 
     Without it the cache keeps the list of what the last pass asked for and
     builds all of it at once at the first request after a ``reset()``
-    (:mod:`minuet_amd.nn.passplan`)."""
+    (:mod:`minuet_amd.nn.passplan`).
+
+    The dense map of more than 65 536 targets that 16-bit layers read again and
+    again gets tiles (csrc/tiles.hip), once the forwards over it would have
+    saved twice what making them takes: the second of a 64 -> 64 layer over a
+    million voxels under 5x5x5, the fifth over 200 000 under 3x3x3.  That call
+    takes 40 to 340 us longer on the device, the later ones about half the time
+    of the first; results are the same bit for bit.  Tiles take about as much
+    device memory as the dense map (at most 2 GiB a map; none where that much is
+    not to be had) and go with it at ``reset()``."""
 
     def __init__(self, ndim: int, dtype: torch.dtype, device: Union[str, torch.device],
                  layout: str = "minuet", disable_reordering: bool = False, lookahead: bool = False):
