@@ -584,13 +584,19 @@ int mnt_sparse_convolution_forward_implicit(const void *sources, const void *wei
  * each tile's live offsets and their source rows.  tiles_out holds
  * mnt_kernel_map_tiles_size int32 words, 16-byte aligned.  Waits for nothing.
  * mnt_kernel_map_tiles_share: the part of that work's time that one forward of
- * the given shape saves by them, 0 where they do not pay or are not taken.  The
- * reference has no counterpart. */
+ * the given shape saves by them, 0 where they do not pay or are not taken, 2
+ * where they are worth making for the first.  The reference has no counterpart. */
 int mnt_kernel_map_tiles_size(int64_t num_targets, int64_t num_offsets, int64_t *ints_out);
 int mnt_kernel_map_tiles(const int32_t *kernel_map, int64_t num_targets, int64_t num_offsets,
                          int32_t *tiles_out, void *stream);
 double mnt_kernel_map_tiles_share(int64_t num_targets, int64_t num_offsets, int64_t num_source_features,
                                   int64_t num_target_features, int float_dtype);
+
+/* 1 where mnt_sparse_convolution_forward_implicit (and _tiled) streams rows and
+ * weights of a layer of the given shape through LDS, which makes it the faster
+ * one for 16-bit layers too wide for the others. */
+int mnt_sparse_convolution_streamed(int64_t num_targets, int64_t num_offsets, int64_t num_source_features,
+                                    int64_t num_target_features, int float_dtype);
 
 /* mnt_sparse_convolution_forward_implicit for 16-bit features from the tiles of
  * the kernel map; the weights packed (mnt_pack_weights), no narrow rows. */

@@ -186,9 +186,27 @@ PyObject *map_entry_new(PyTypeObject *type, PyObject *args, PyObject *) {
   int kind, device, index_code;
   long long num_sources, num_targets;
   unsigned long long built_from = 0;
-  if (!PyArg_ParseTuple(args, "iOOOOiiLLO!|K", &kind, &coordinates, &stride, &batch_dims, &keep, &device, &index_code,
-                        &num_sources, &num_targets, &PyTuple_Type, &pointers, &built_from)) {
+  PyObject *tiles = Py_None;                  // those the current stream of `device` has made already
+  if (!PyArg_ParseTuple(args, "iOOOOiiLLO!|KO", &kind, &coordinates, &stride, &batch_dims, &keep, &device, &index_code,
+                        &num_sources, &num_targets, &PyTuple_Type, &pointers, &built_from, &tiles)) {
     return nullptr;
+  }
+  std::unique_ptr<at::cuda::CUDAEvent> made;
+  void *made_on = nullptr;
+  if (tiles != Py_None) {
+    if (tensor_of(tiles) == nullptr) {
+      PyErr_SetString(PyExc_TypeError, "tiles are a tensor");
+      return nullptr;
+    }
+    try {
+      const c10::hip::HIPStream stream = c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(device));
+      made_on = stream.stream();
+      made.reset(new at::cuda::CUDAEvent());
+      made->record(c10::hip::HIPStreamMasqueradingAsCUDA(stream));
+    } catch (const std::exception &error) {
+      PyErr_SetString(PyExc_RuntimeError, error.what());
+      return nullptr;
+    }
   }
   MapEntry *e = reinterpret_cast<MapEntry *>(type->tp_alloc(type, 0));
   if (e == nullptr) return nullptr;
@@ -207,10 +225,10 @@ PyObject *map_entry_new(PyTypeObject *type, PyObject *args, PyObject *) {
   e->num_targets = num_targets;
   e->built_from = reinterpret_cast<const void *>(static_cast<uintptr_t>(built_from));
   e->used = 0;
-  e->tiles = nullptr;
+  e->tiles = tiles == Py_None ? nullptr : hold(tiles);
   e->tiles_credit = 0.0;
-  e->tiles_stream = nullptr;
-  e->tiles_made = nullptr;
+  e->tiles_stream = made_on;
+  e->tiles_made = made.release();
   e->tiles_ready = 0;
   for (Py_ssize_t i = 0; i < 8; ++i) {
     e->at[i] = nullptr;
@@ -357,7 +375,9 @@ inline bool vector_fits(const at::Tensor *t, int64_t channels, int device) {
 }
 
 // The tiles of a layer's map, or null where the layer runs without.  Tiles cost
-// two or more forwards to make and are kept with the map, so they are made once
+// one or more forwards to make and are kept with the map.  A wide layer, which
+// loses half its time without, makes them at once (a share of kTilesCredit); the
+// others' are made once
 // the forwards that have run over it would have saved twice their price: a map
 // that a network reads a few times and drops never pays for them, one that is
 // read on and on soon does.  Layers of all widths and types share a map, so

@@ -35,6 +35,10 @@ template <typename T>
 void tiled_forward(const T *sources, const T *packed, const int *kernel_map, const int *tiles, int64_t S, int64_t Tn,
                    int64_t O, int64_t K, int64_t N, const Epilogue &ep, T *out, hipStream_t stream);
 
+template <typename T>
+void streamed_forward(const T *sources, const T *packed, const int *kernel_map, const int *tiles, int64_t S, int64_t Tn,
+                      int64_t O, int64_t K, int64_t N, const Epilogue &ep, T *out, hipStream_t stream);
+
 void compact_forward(const float *sources, const float *weights, const int *kernel_map, int64_t S, int64_t Tn,
                      int64_t O, int64_t K, int64_t N, const Epilogue &ep, float *out, hipStream_t stream);
 
@@ -65,6 +69,20 @@ typedef unsigned uint4v __attribute__((ext_vector_type(4)));
 // Source tensors stay below this many bytes: rows are addressed through 32-bit
 // buffer offsets.
 constexpr unsigned kMaxSourceBytes = 0xFFFFF000u;
+
+// The 16-bit layers that streamed_forward_kernel runs, with tiles and without:
+// rows of more than one and up to four 128-byte stages, and rows of one stage
+// under more output channels than tiled_forward_kernel holds at a time.  Shorter
+// rows cost the other kernels no more time (64 -> 64 channels over 16 000
+// targets 9.6 us against 10.3), a kernel of more than kTileMaxOffsets offsets
+// has no tiles and hits too few to be walked offset by offset.
+static bool streamed_takes(int64_t Tn, int64_t O, int64_t K, int64_t N) {
+  const int64_t row_bytes = 2 * K;
+  const int64_t weight_bytes = O * div_ceil(N, 32) * 32 * div_ceil(row_bytes, 128) * 128;
+  return O > 1 && O <= kTileMaxOffsets && (row_bytes > 128 || (row_bytes > 64 && N > 128)) && row_bytes <= 512 &&
+         row_bytes % 16 == 0 && N % 4 == 0 && N <= 32 * kImplicitMaxBlocks * kImplicitMaxGroups &&
+         weight_bytes < static_cast<int64_t>(kMaxSourceBytes) && Tn < (int64_t{1} << 30);
+}
 
 // KS: 32-byte steps of K per pipeline stage.  A source row takes `chunks`
 // stages of KS * 32 bytes (Kp * sizeof(T) must be a multiple of that when
@@ -558,6 +576,11 @@ static void implicit_typed(const T *sources, const T *weights, const T *packed, 
     profile_mark("pack_weights", stream);
   }
   if constexpr (sizeof(T) == 2) {
+    if (streamed_takes(Tn, O, K, N)) {
+      streamed_forward<T>(sources, wt, kernel_map, nullptr, S, Tn, O, K, N, ep, out, stream);
+      profile_mark("implicit", stream);
+      return;
+    }
     // Up to two workgroups per compute unit tiled_forward_kernel's shorter
     // stages count, beyond that this kernel's wavefronts that skip offsets of
     // their own (64 -> 64 channels: 16.3 against 17.7 us at 60 000 targets,
@@ -698,8 +721,18 @@ extern "C" int mnt_kernel_map_invert(const int32_t *kernel_map, int64_t num_offs
   });
 }
 
+extern "C" int mnt_sparse_convolution_streamed(int64_t T, int64_t O, int64_t K, int64_t N, int float_dtype) {
+  return float_dtype != MNT_FLOAT32 && T >= 0 && O >= 1 && K >= 1 && N >= 1 && streamed_takes(T, O, K, N) ? 1 : 0;
+}
+
 // What tiles (mnt_kernel_map_tiles) would save of one forward, over what making
-// them takes; 0 where they do not pay or cannot be used.  Fitted to layers of
+// them takes; 0 where they do not pay or cannot be used.
+// Layers of streamed_forward_kernel take 28 us for them at once where its
+// workgroups are more than twice the compute units: a map of a network is read
+// four to eight times (us without and with, 128 -> 128 channels over 18 600
+// targets of a LiDAR level 29.8 and 17.3, 256 -> 256 over 8 700 37 and 27, over
+// 25 600 of a scan 77 and 37; over 9 000, 128 -> 128: 15.2 and 13.4).
+// Others: fitted to layers of
 // 32 to 128 channels over 100 000 to a million targets: a forward gets faster by
 // 1.1 us per million (offset, target) pairs and unit of (channel blocks + 1) x
 // 128-byte pieces of a row, making tiles takes 28 us and 2.5 us per million pairs.
@@ -708,6 +741,9 @@ extern "C" double mnt_kernel_map_tiles_share(int64_t T, int64_t O, int64_t K, in
       (K * 2) % 16 != 0 || K * 2 > kImplicitMaxRowBytes || N % 4 != 0 || N > 32 * kImplicitMaxBlocks * kImplicitMaxGroups ||
       narrow_fits(O, K, N, 2, true)) {
     return 0.0;
+  }
+  if (streamed_takes(T, O, K, N)) {
+    return div_ceil(T, 64) * div_ceil(N, 64) > 2 * static_cast<int64_t>(compute_units()) ? 2.0 : 0.0;
   }
   // Below, the kernel without tiles is about as fast, and it adds up in another
   // order: a layer's results do not change from one call to the next.
@@ -745,7 +781,15 @@ extern "C" int mnt_sparse_convolution_forward_tiled(
     MNT_CHECK(out != nullptr && tiles != nullptr && packed_weights != nullptr, "null operand");
     profile_mark("enter:implicit", stream);
     const Epilogue ep = {channel_scale, channel_shift, residual, activation, negative_slope, nullptr};
-    if (float_dtype == MNT_FLOAT16) {
+    if (streamed_takes(T, O, K, N)) {
+      if (float_dtype == MNT_FLOAT16) {
+        streamed_forward<half_t>(static_cast<const half_t *>(sources), static_cast<const half_t *>(packed_weights),
+                                 nullptr, tiles, S, T, O, K, N, ep, static_cast<half_t *>(out), stream);
+      } else {
+        streamed_forward<bf16_t>(static_cast<const bf16_t *>(sources), static_cast<const bf16_t *>(packed_weights),
+                                 nullptr, tiles, S, T, O, K, N, ep, static_cast<bf16_t *>(out), stream);
+      }
+    } else if (float_dtype == MNT_FLOAT16) {
       tiled_forward<half_t>(static_cast<const half_t *>(sources), static_cast<const half_t *>(packed_weights), nullptr,
                             tiles, S, T, O, K, N, ep, static_cast<half_t *>(out), stream);
     } else {

@@ -27,6 +27,7 @@ from minuet_amd.utils.helpers import as_tuple, generate_kernel_offsets
 __all__ = ["SparseConv", "SparseConv3d", "KernelMapCache"]
 
 _MOST_ROWS = (1 << 63) - 1
+_MOST_TILE_ENTRIES = 1 << 29            # (tiles of 2 GiB)
 _TRANSPOSED_FIRST = ("Layer must transpose=True must have its corresponding non-transposed layer "
                      "before its execution")
 
@@ -61,7 +62,9 @@ class KernelMapCache(object):
 
     The dense map of more than 65 536 targets that 16-bit layers read again and
     again gets tiles (csrc/tiles.hip), once the forwards over it would have
-    saved twice what making them takes: the second of a 64 -> 64 layer over a
+    saved twice what making them takes; the first wide layer (rows of more than
+    128 bytes) over some thousand targets makes them at once.  Otherwise
+    that is the second of a 64 -> 64 layer over a
     million voxels under 5x5x5, the fifth over 200 000 under 3x3x3.  That call
     takes 40 to 340 us longer on the device, the later ones about half the time
     of the first; results are the same bit for bit.  Tiles take about as much
@@ -80,7 +83,8 @@ class KernelMapCache(object):
         self._key_memo = dict()
         self._dense_maps_cache = dict()         # key -> (dense kernel map [O, T], number of sources)
         self._inverse_maps_cache = dict()       # key -> its inverse [O, S] (transposed layers)
-        self._offset_groups_cache = dict()      # key -> offset-group tables of the dense map (False: none)
+        self._offset_groups_cache = dict()      # what wide layers read beside the dense map (False: nothing):
+                                                # key -> offset-group tables, (key, "tiles") -> tiles
         self._coordinates_cache = dict()
         self._bounds_cache = dict()
         self._requests = dict()                 # what this pass has asked for, in order (values unused)
@@ -411,6 +415,31 @@ class KernelMapCache(object):
                     self._requests.setdefault(("groups", key))
             self._offset_groups_cache[key] = entry
         return entry or None
+
+    def get_tiles(self, dense: torch.Tensor, in_channels: int, out_channels: int, dtype: torch.dtype,
+                  source_coordinates: torch.Tensor, source_stride, target_stride, kernel_size, kernel_dilation,
+                  transposed: bool = False) -> Optional[torch.Tensor]:
+        """The tiles of the dense kernel map ``dense``, for a wide layer of these
+        channels that makes them at its first call (None where it runs without).
+        Not in the reference, whose map has one order of targets."""
+        if torch.cuda.is_current_stream_capturing():
+            return None
+        key = (self._map_key(source_coordinates.shape[1], source_stride, target_stride, kernel_size, kernel_dilation,
+                             transposed)[0], "tiles", transposed)
+        stream = torch.cuda.current_stream(dense.device).cuda_stream
+        entry = self._offset_groups_cache.get(key)
+        if not entry:                        # (a wider layer of the same map may want them)
+            entry = False
+            offsets, targets = dense.shape
+            if (dense.is_contiguous() and offsets * targets <= _MOST_TILE_ENTRIES
+                    and _C.kernel_map_tiles_worth_making(targets, offsets, in_channels, out_channels, dtype)):
+                try:
+                    entry = (_C.kernel_map_tiles(dense), stream)
+                except torch.OutOfMemoryError:
+                    pass
+            self._offset_groups_cache[key] = entry
+        # (another stream owes nothing to the one that made them: the same rows without)
+        return entry[0] if entry and entry[1] == stream else None
 
     def _inverse_of(self, key) -> torch.Tensor:
         """Dense map of the transposed layer of ``key`` ([O, S]), made on first use."""
@@ -819,21 +848,23 @@ class SparseConv(Module):
             return False
         if dataflow == "implicit":
             return True
-        return F.prefers_implicit(self.kernel.shape[0], self.in_channels + pad, self.out_channels,
-                                  features.dtype)
+        shape = (self.kernel.shape[0], self.in_channels + pad, self.out_channels, features.dtype)
+        return F.prefers_implicit(*shape) or F.prefers_streamed(*shape)
 
     def _takes_offset_groups(self, features: torch.Tensor) -> bool:
         """Whether this call multiplies its offsets three at a time (the
         ``offset_groups`` dataflow): forced by the tunable ``dataflow``, or, under
-        ``auto``, for the wide 16-bit 3 x 3 x 3 layers that the single-kernel form
-        does not take, whose product rows are what bounds them."""
+        ``auto``, for the 16-bit 3 x 3 x 3 layers that are too wide to be streamed
+        and whose product rows are what bounds them."""
         dataflow = self._tunable_config.get("dataflow", "auto")
         if dataflow not in ("auto", "offset_groups") or not features.is_cuda or self.transposed:
             return False
         if (features.dtype != self.kernel.dtype or self.ndim != 3 or self.kernel.shape[0] != 27
                 or not _C.offset_groups_forward_supported(self.in_channels, self.out_channels, features.dtype)):
             return False
-        return dataflow == "offset_groups" or self.in_channels * features.element_size() >= 256
+        return dataflow == "offset_groups" or (
+            self.in_channels * features.element_size() >= 256
+            and not F.prefers_streamed(27, self.in_channels, self.out_channels, features.dtype))
 
     def _pointwise(self, features: torch.Tensor, epilogue: Optional[F.Epilogue]):
         """1x1x1 kernel, stride 1: a plain ``features @ W`` (reference:
@@ -946,11 +977,19 @@ class SparseConv(Module):
                 if pad:
                     sources = torch.nn.functional.pad(sources, (0, pad))
                 weights, packed = self._packed_kernel(pad)
-                features = _C.sparse_convolution_forward_implicit(sources, weights, dense,
-                                                                  epilogue=epilogue,
-                                                                  packed_weights=packed)
+                tiles = None
+                if packed is not None and F.prefers_streamed(volume, sources.shape[1], self.out_channels, sources.dtype):
+                    tiles = cache.get_tiles(dense, sources.shape[1], self.out_channels, sources.dtype, inputs.C,
+                                            inputs.stride, stride, self.kernel_size, self.dilation, self.transposed)
+                if tiles is not None:
+                    features = _C.sparse_convolution_forward_tiled(sources, weights, tiles, dense.shape[1], packed,
+                                                                   epilogue=epilogue)
+                else:
+                    features = _C.sparse_convolution_forward_implicit(sources, weights, dense,
+                                                                      epilogue=epilogue,
+                                                                      packed_weights=packed)
                 if not pad and dense.is_contiguous():
-                    made = ("IMPLICIT", weights, packed, (dense.data_ptr(),), dense, 0)
+                    made = ("IMPLICIT", weights, packed, (dense.data_ptr(),), dense, 0, tiles)
             else:
                 features, made = self._forward_tables(cache, map_args, sources, epilogue)
         if bias is not None:
@@ -967,7 +1006,8 @@ class SparseConv(Module):
         Where the kind depends on the size (``rows``), the Layer of the other kind
         stays with the new one: each cloud gets the kernel that a fresh cache
         would give it, whatever came before."""
-        name, weights, packed, pointers, owners, index_code = made
+        name, weights, packed, pointers, owners, index_code = made[:6]
+        tiles = made[6] if len(made) > 6 else None
         host = _C.load_host()
         if host is None:
             return
@@ -976,7 +1016,7 @@ class SparseConv(Module):
         if pointers is not None:
             shape_id = (kind, self.kernel_size, self.stride, self.dilation, self.transposed)
             entry = host.MapEntry(kind, coordinates, stride, batch_dims, owners, features.device.index, index_code,
-                                  inputs.F.shape[0], features.shape[0], pointers)
+                                  inputs.F.shape[0], features.shape[0], pointers, 0, tiles)
             cache = self._kernel_map_cache
             cache._fast_maps.setdefault(shape_id, {})[inputs.stride] = entry
             key = cache._map_key(self.ndim, inputs.stride, stride, self.kernel_size, self.dilation, self.transposed)[0]

@@ -107,6 +107,7 @@ SIGNATURES = {
     "mnt_kernel_map_tiles_size": (_int, [_i64, _i64, ctypes.POINTER(_i64)]),
     "mnt_kernel_map_tiles": (_int, [_vp, _i64, _i64, _vp, _vp]),
     "mnt_kernel_map_tiles_share": (ctypes.c_double, [_i64, _i64, _i64, _i64, _int]),
+    "mnt_sparse_convolution_streamed": (_int, [_i64, _i64, _i64, _i64, _int]),
     "mnt_sparse_convolution_forward_tiled": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _vp, _vp, _vp,
                                                     _int, ctypes.c_float, _vp, _vp]),
     "mnt_sparse_convolution_forward_implicit": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64,
@@ -1495,6 +1496,22 @@ def sparse_convolution_forward_implicit(sources: torch.Tensor, weights: torch.Te
             _ptr(ep.shift), _ptr(ep.residual), ACTIVATION_CODES[ep.activation],
             float(ep.negative_slope), _ptr(packed_weights), _ptr(out), _stream(device)))
     return out
+
+
+def streamed_forward_supported(num_offsets: int, num_source_features: int, num_target_features: int,
+                               dtype: torch.dtype) -> bool:
+    """Shapes that ``sparse_convolution_forward_implicit`` streams through LDS."""
+    if dtype not in (torch.float16, torch.bfloat16):
+        return False
+    return bool(load_library().mnt_sparse_convolution_streamed(
+        0, num_offsets, num_source_features, num_target_features, _float_code(dtype, "streamed_forward_supported")))
+
+
+def kernel_map_tiles_worth_making(num_targets: int, num_offsets: int, num_source_features: int,
+                                  num_target_features: int, dtype: torch.dtype) -> bool:
+    """Whether a layer of this shape makes the tiles of its map at its first call."""
+    return load_library().mnt_kernel_map_tiles_share(num_targets, num_offsets, num_source_features, num_target_features,
+                                                     _float_code(dtype, "kernel_map_tiles_worth_making")) >= 2.0
 
 
 def kernel_map_tiles(kernel_map: torch.Tensor) -> torch.Tensor:

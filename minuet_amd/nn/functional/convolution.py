@@ -9,7 +9,7 @@ from ..kernel_map import KernelMap
 
 __all__ = ["cuda_time_gather", "cuda_time_scatter", "sparse_convolution_forward",
            "cuda_time_gemm", "set_gemm_parallel_level", "Epilogue", "pack_weights",
-           "prefers_implicit", "prefers_hits", "hits_rows_limit"]
+           "prefers_implicit", "prefers_streamed", "prefers_hits", "hits_rows_limit"]
 
 pack_weights = _C.pack_weights
 
@@ -46,6 +46,17 @@ def prefers_implicit(num_offsets: int, num_source_features: int, num_target_feat
             return num_target_features <= 128
         return row_bytes <= 256 and num_target_features <= 64 and num_offsets > 8
     return num_offsets <= 8 and num_source_features * num_target_features <= 1024
+
+
+def prefers_streamed(num_offsets: int, num_source_features: int, num_target_features: int,
+                     dtype: torch.dtype) -> bool:
+    """Whether ``dataflow="auto"`` takes the single-kernel form for a layer too wide
+    for ``prefers_implicit``: 16-bit rows of 136 to 512 bytes (or of 72 and more
+    under more than 128 output channels), whose rows and weights stream through
+    LDS.  Against three kernels or offset groups, us a layer: 128 -> 128 channels
+    over 6 850 voxels 23.0 and 11.8, over 18 600 of a LiDAR level 27.7 and 17.3,
+    256 -> 256 over 2 000 27.1 and 16.8, over 25 600 of a scan 39.5 and 37.1."""
+    return _C.streamed_forward_supported(num_offsets, num_source_features, num_target_features, dtype)
 
 
 def hits_rows_limit(num_offsets: int, num_source_features: int, num_target_features: int,

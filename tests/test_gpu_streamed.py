@@ -1,0 +1,104 @@
+"""The forward of wide 16-bit layers whose rows and weights stream through LDS,
+with and without tiles, against a plain fp32 product per offset."""
+import pytest
+import torch
+
+import minuet_amd as minuet
+from minuet_amd.nn import functional as F
+from minuet_amd.nn.functional import _C
+from test_gpu_tiles import DEVICE, close, operands, reference, tile_rows
+
+pytestmark = pytest.mark.gpu
+
+# one target, one more and one fewer than a workgroup's; every shape of a workgroup (32 x 64, 64 x 64,
+# 128 x 64, 64 x 128, 128 x 128); rows of one to four stages, whole and ragged; outputs that are no whole
+# pieces and several column blocks; fewer offsets than the ring holds, and more than a wavefront has lanes
+SHAPES = [
+    (1, 27, 128, 128), (33, 3, 72, 4), (500, 2, 256, 512), (1000, 125, 136, 64), (1025, 27, 64, 160),
+    (2000, 27, 200, 36), (5000, 27, 128, 128), (4097, 9, 192, 100), (16500, 27, 128, 64), (20000, 8, 256, 32),
+    (9000, 27, 128, 128), (8300, 33, 144, 256), (50000, 27, 128, 128), (26000, 3, 192, 160), (25700, 128, 72, 256)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("targets,offsets,cin,cout", SHAPES)
+def test_forward_matches_products(targets, offsets, cin, cout, dtype):
+    assert _C.streamed_forward_supported(offsets, cin, cout, dtype)
+    dense, x, w = operands(targets, 3000, offsets, cin, cout, dtype)
+    packed = F.pack_weights(w)
+    tiles = _C.kernel_map_tiles(dense)
+    wanted = reference(x, w, dense)
+    plain = _C.sparse_convolution_forward_implicit(x, w, dense, packed_weights=packed)
+    close(plain, wanted, dtype)
+    assert torch.equal(_C.sparse_convolution_forward_tiled(x, w, tiles, targets, packed), plain)
+    gen = torch.Generator(device=DEVICE).manual_seed(9)
+    scale, shift = (torch.randn(cout, generator=gen, device=DEVICE) for _ in range(2))
+    residual = torch.randn(targets, cout, generator=gen, device=DEVICE).to(dtype)
+    epilogue = F.Epilogue(scale, shift, residual, "relu", 0.0)
+    wanted = torch.relu(wanted * scale + shift + residual.float())
+    plain = _C.sparse_convolution_forward_implicit(x, w, dense, epilogue=epilogue, packed_weights=packed)
+    close(plain, wanted, dtype)
+    assert torch.equal(_C.sparse_convolution_forward_tiled(x, w, tiles, targets, packed, epilogue=epilogue), plain)
+
+
+@pytest.mark.parametrize("targets,cin,cout", [(1, 128, 64), (1000, 256, 64), (5000, 128, 128), (17000, 192, 64),
+                                              (9000, 128, 128), (50000, 128, 128)])
+def test_undefined_numbers_stay_where_they_belong(targets, cin, cout):
+    """A weight that is not finite reaches the 32 targets that stand with one that
+    uses its offset, a feature that is not finite the targets that use its row,
+    and every other row is what it is without."""
+    dense, x, w = operands(targets, 3000, 27, cin, cout, torch.float16)
+    dense[[0, 5, 26]] = -1
+    dense[9] = -1
+    dense[9, targets // 2] = 7
+    packed = F.pack_weights(w)
+    tiles = _C.kernel_map_tiles(dense)
+    spoilt = w.clone()
+    spoilt[[0, 5, 26], 0, 3] = torch.tensor([float("inf"), float("nan"), float("-inf")], device=DEVICE).half()
+    wild = spoilt.clone()
+    wild[9, 1, 2] = float("inf")
+    bad = x.clone()
+    bad[7, 3], bad[11, cin - 1] = float("inf"), float("nan")
+    touched = ((dense == 7) | (dense == 11)).any(0)
+    wanted = _C.sparse_convolution_forward_implicit(x, w, dense, packed_weights=packed)
+    assert bool(wanted.isfinite().all())
+    places = torch.arange(-(-targets // 32) * 32, device=DEVICE)
+    for at, forward in (
+            (places, lambda f, weights: _C.sparse_convolution_forward_implicit(f, weights, dense)),
+            (tile_rows(tiles, targets).long(),
+             lambda f, weights: _C.sparse_convolution_forward_tiled(f, weights, tiles, targets, F.pack_weights(weights)))):
+        assert torch.equal(forward(x, spoilt), wanted)
+        groups = at.view(-1, 32)
+        others = groups[~(groups == targets // 2).any(1)].flatten()
+        others = others[(others >= 0) & (others < targets)]
+        assert torch.equal(forward(x, wild)[others], wanted[others])
+        got = forward(bad, w)
+        assert torch.equal(got[~touched], wanted[~touched]) and not bool(got[touched].isfinite().all(1).any())
+
+
+def test_a_layer_gives_the_same_rows_from_call_to_call():
+    """The first call, later ones through the extension module, one on another
+    stream, which has no tiles, and the replays of a captured one."""
+    from helpers import random_cloud, sorted_unique, dev
+    c, _ = sorted_unique(random_cloud(9000, 40, 3, lo=-9), None)
+    conv = minuet.nn.SparseConv3d(256, 256, 3, dtype=torch.float16, device=DEVICE)
+    cache = minuet.nn.KernelMapCache(3, torch.int32, DEVICE)
+    minuet.set_kernel_map_cache(conv, cache)
+    x = minuet.SparseTensor(torch.randn(c.shape[0], 256, device=DEVICE).half(), dev(c))
+    with torch.no_grad():
+        first = conv(x).F
+        assert [bool(entry) for entry in cache._offset_groups_cache.values()] == [True]     # tiles, kept with the map
+        assert torch.equal(conv(x).F, first)
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            other = conv(x).F
+        side.synchronize()
+        assert torch.equal(other, first)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = conv(x).F
+        for _ in range(3):
+            out.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, first)
