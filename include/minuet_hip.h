@@ -592,6 +592,23 @@ int mnt_kernel_map_tiles(const int32_t *kernel_map, int64_t num_targets, int64_t
 double mnt_kernel_map_tiles_share(int64_t num_targets, int64_t num_offsets, int64_t num_source_features,
                                   int64_t num_target_features, int float_dtype);
 
+/* The fp32 mnt_sparse_convolution_forward_implicit of a layer of more than one
+ * offset (Cin and Cout multiples of 4), the same bit for bit, from weights in the
+ * order in which its matrix instructions take them:
+ * packed[O][ceil(Cout / 16)][ceil(Cin / 16)][64][4], element (lane, x) of a block
+ * the weight of input channel 4 * (lane / 16) + x and output channel lane % 16
+ * of the block, zeros past the end.  mnt_pack_weights_in_lanes makes them of
+ * [O, Cin, Cout]; the caller keeps them for as long as the weights do not change.
+ * Same reference code as mnt_sparse_convolution_forward and mnt_pack_weights. */
+int mnt_pack_weights_in_lanes(const float *weights, int64_t num_offsets, int64_t num_source_features,
+                              int64_t num_target_features, float *packed_out, void *stream);
+int mnt_sparse_convolution_forward_in_lanes(const float *sources, const float *packed_weights,
+                                            const int32_t *kernel_map, int64_t num_sources, int64_t num_targets,
+                                            int64_t num_offsets, int64_t num_source_features,
+                                            int64_t num_target_features, const float *channel_scale,
+                                            const float *channel_shift, const void *residual, int activation,
+                                            float negative_slope, float *out, void *stream);
+
 /* 1 where mnt_sparse_convolution_forward_implicit (and _tiled) streams rows and
  * weights of a layer of the given shape through LDS, which makes it the faster
  * one for 16-bit layers too wide for the others. */

@@ -24,6 +24,8 @@ struct CompactShape {
   long long num_targets;
   int num_offsets, K, N;
   int chunks;                  // units of KI * 16 input channels
+  int columns;                 // workgroups side by side over the output channels
+  int steps;                   // of 16 input channels, in weights given in lane order
 };
 
 // A workgroup takes TARGETS targets and 16 * C output channels; its SPLIT wavefronts
@@ -36,18 +38,22 @@ struct CompactShape {
 // added up in the order of the wavefronts at the end, so that a result is the
 // same whenever it is computed.
 //
+// LANES: the weights come in the order of the instruction's lanes (pack_lanes),
+// one load of 1 KB where [O][K][N] takes four of 256 or 512 bytes.
+//
 // What bounds it: on small clouds one wavefront's chain of map entry, source
 // rows, products (the unit after is asked for before one is multiplied), hence
-// the split; beyond, the weights, which every 16 rows read again: from some
+// the split; beyond, fp32 products of 16 rows that are about half hits, and the
+// weights, which every 16 rows read again: from some
 // targets x input x output channels on (78 million for 3 x 3 x 3) the
 // three-kernel form is the faster one again (hits_rows_limit in
 // nn/functional/convolution.py has the line and both sides of it).  fp32, 3 x 3 x 3, us a layer in
 // three kernels and here: 32 -> 32 channels over 3 000 voxels 11.4 / 4.9,
-// 20 000 17.9 / 11.2, 200 000 76 / 52; 64 -> 64 over 3 000 12.1 / 8.4, 12 000
-// 18.8 / 14.9; 256 -> 256 over 135 28 / 22.  (128 targets per workgroup
+// 20 000 17.9 / 11.2, 200 000 76 / 51; 64 -> 64 over 3 000 12.1 / 8.4, 12 000
+// 18.8 / 14.9; 256 -> 256 over 135 28 / 16.  (128 targets per workgroup
 // fill the 16 rows better, but their sums leave fewer wavefronts to a compute
 // unit: 17 to 40 % slower.)
-template <int C, int KI, int SPLIT, int TARGETS, bool WHOLE>
+template <int C, int KI, int SPLIT, int TARGETS, bool WHOLE, bool LANES>
 __global__ __launch_bounds__(64 * SPLIT) void compact_forward_kernel(
     const float *__restrict__ sources, unsigned source_bytes, const float *__restrict__ weights,
     unsigned weight_bytes, const int *__restrict__ kernel_map, CompactShape s, unsigned char *__restrict__ out,
@@ -69,8 +75,8 @@ __global__ __launch_bounds__(64 * SPLIT) void compact_forward_kernel(
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15;
   const int q = lane >> 4;
-  const long long first = static_cast<long long>(blockIdx.x) * kTargets;
-  const int channel = blockIdx.y * 16 * C;
+  const long long first = static_cast<long long>(blockIdx.x / s.columns) * kTargets;
+  const int channel = static_cast<int>(blockIdx.x % s.columns + blockIdx.y) * 16 * C;
   const int chunks = s.chunks;
   float *const acc = s_acc[wv];
   Lists &lists = s_lists[wv];
@@ -81,10 +87,13 @@ __global__ __launch_bounds__(64 * SPLIT) void compact_forward_kernel(
       const_cast<float *>(weights), 0, weight_bytes, 0x00020000);
   const unsigned row_bytes = static_cast<unsigned>(s.K) * 4u;
   const unsigned line_bytes = static_cast<unsigned>(s.N) * 4u;
-  // lane (r, q) multiplies the C channels r * C .. of the workgroup's 16 * C
-  const bool in_width = channel + r * C < s.N;
-  const unsigned w_at = in_width ? static_cast<unsigned>(q) * 4u * line_bytes + static_cast<unsigned>(channel + r * C) * 4u
-                                 : kCompactNowhere;
+  // lane (r, q) multiplies the C channels r * C .. of the workgroup's 16 * C;
+  // with weights in lane order r, 16 + r, ..
+  const bool in_width = LANES || channel + r * C < s.N;
+  const unsigned w_at = LANES ? lane * 16u
+                        : in_width ? static_cast<unsigned>(q) * 4u * line_bytes + static_cast<unsigned>(channel + r * C) * 4u
+                                   : kCompactNowhere;
+  const unsigned blocks = (static_cast<unsigned>(s.N) + 15u) / 16u;
   struct Unit {
     uint4 a[KI];
     float w[KI][4][C];
@@ -103,6 +112,20 @@ __global__ __launch_bounds__(64 * SPLIT) void compact_forward_kernel(
       const uint4v v = __builtin_amdgcn_raw_buffer_load_b128(source_buffer, inside ? row_at : kCompactNowhere,
                                                              chunk_at + i * 64u, 0);
       u.a[i] = make_uint4(v.x, v.y, v.z, v.w);
+      if constexpr (LANES) {
+        const int step = c * KI + i;
+#pragma unroll
+        for (int b = 0; b < C; ++b) {
+          const unsigned at = WHOLE || step < s.steps ? w_at : kCompactNowhere;
+          const unsigned from = ((static_cast<unsigned>(o) * blocks + channel / 16 + b) * s.steps + step) * 1024u;
+          const uint4v w = __builtin_amdgcn_raw_buffer_load_b128(weight_buffer, at, from, 0);
+          u.w[i][0][b] = __uint_as_float(w.x);
+          u.w[i][1][b] = __uint_as_float(w.y);
+          u.w[i][2][b] = __uint_as_float(w.z);
+          u.w[i][3][b] = __uint_as_float(w.w);
+        }
+        continue;
+      }
 #pragma unroll
       for (int x = 0; x < 4; ++x) {
         const unsigned at = inside ? w_at : kCompactNowhere;
@@ -221,18 +244,55 @@ __global__ __launch_bounds__(64 * SPLIT) void compact_forward_kernel(
     float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int w = 0; w < SPLIT; ++w) {
-      const float4 f = *reinterpret_cast<const float4 *>(&s_acc[w][t * kAccRow + part * 4]);
-      v[0] += f.x;
-      v[1] += f.y;
-      v[2] += f.z;
-      v[3] += f.w;
+      if constexpr (LANES && C > 1) {
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+          const int ch = part * 4 + x;
+          v[x] += s_acc[w][t * kAccRow + ch % 16 * C + ch / 16];
+        }
+      } else {
+        const float4 f = *reinterpret_cast<const float4 *>(&s_acc[w][t * kAccRow + part * 4]);
+        v[0] += f.x;
+        v[1] += f.y;
+        v[2] += f.z;
+        v[3] += f.w;
+      }
     }
     finish_piece<float, 4>(v, ep, first + t, channel + part * 4, s.N, out);
   }
 }
 
-void compact_forward(const float *sources, const float *weights, const int *kernel_map, int64_t S, int64_t Tn,
-                     int64_t O, int64_t K, int64_t N, const Epilogue &ep, float *out, hipStream_t stream) {
+// lanes[o][block][step][lane][x] = w[o][16 step + 4 (lane / 16) + x][16 block + lane % 16]
+__global__ __launch_bounds__(256) void pack_lanes_kernel(const float *__restrict__ w, int K, int N, int blocks,
+                                                         int steps, long long pieces, uint4 *__restrict__ lanes) {
+  const long long stride = static_cast<long long>(gridDim.x) * 256;
+  for (long long i = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x; i < pieces; i += stride) {
+    const int lane = static_cast<int>(i & 63);
+    const long long group = i >> 6;
+    const int step = static_cast<int>(group % steps), block = static_cast<int>(group / steps % blocks);
+    const long long o = group / steps / blocks;
+    const int k0 = 16 * step + 4 * (lane >> 4), n = 16 * block + (lane & 15);
+    unsigned v[4];
+#pragma unroll
+    for (int x = 0; x < 4; ++x) v[x] = k0 + x < K && n < N ? __float_as_uint(w[(o * K + k0 + x) * N + n]) : 0u;
+    lanes[i] = make_uint4(v[0], v[1], v[2], v[3]);
+  }
+}
+
+int64_t lane_weight_floats(int64_t O, int64_t K, int64_t N) { return O * div_ceil(N, int64_t{16}) * div_ceil(K, int64_t{16}) * 256; }
+
+void pack_lanes(const float *weights, int64_t O, int64_t K, int64_t N, float *lanes, hipStream_t stream) {
+  const long long pieces = lane_weight_floats(O, K, N) / 4;
+  if (pieces == 0) return;
+  pack_lanes_kernel<<<grid_for(pieces, 256, 4096), 256, 0, stream>>>(
+      weights, static_cast<int>(K), static_cast<int>(N), static_cast<int>(div_ceil(N, int64_t{16})),
+      static_cast<int>(div_ceil(K, int64_t{16})), pieces, reinterpret_cast<uint4 *>(lanes));
+  check_launch("pack_lanes_kernel");
+}
+
+// `weights`: [O][K][N] or, with `lanes`, as pack_lanes leaves them.
+void compact_forward(const float *sources, const float *weights, bool lanes, const int *kernel_map, int64_t S,
+                     int64_t Tn, int64_t O, int64_t K, int64_t N, const Epilogue &ep, float *out, hipStream_t stream) {
   CompactShape s;
   s.num_targets = Tn;
   s.num_offsets = static_cast<int>(O);
@@ -241,37 +301,53 @@ void compact_forward(const float *sources, const float *weights, const int *kern
   s.chunks = static_cast<int>(div_ceil(K, 64));
   const int ki = static_cast<int>(div_ceil(K, 16 * s.chunks));
   const bool whole = K == 16 * ki * s.chunks;
-  // One block of channels per workgroup, and fewer targets the fewer workgroups
-  // that leaves, so that small clouds reach the whole chip (256 -> 256 channels
-  // over 135 targets: 45 us with 64 targets per workgroup, 22 with 16; 32 -> 32
-  // over 3 000 6.5 and, with 32, 4.9); all channels together only where there
-  // are workgroups without (64 -> 64 over 12 000 targets 14.8, in four blocks
-  // 18.6; over 25 000 24.9 and 20.7).  Eight wavefronts per workgroup while all
-  // of them find room at once.
+  // Targets, channel blocks and wavefronts of a workgroup by how many workgroups
+  // of 64 targets and 16 channels there are to a compute unit: small clouds need
+  // small workgroups to reach the whole chip, beyond that two blocks share the
+  // source rows.  Over 360 layers (three kinds of scene, 3x3x3 and strided
+  // 2x2x2, 48 to 40 000 targets, 16 to 256 channels) these lines cost 3.6 % on
+  // average over the best of 15 shapes for each (us: 256 -> 256 channels over 135
+  // targets 16 targets x 16 channels 15.9, 32 x 32 32; 128 -> 128 over 658 16 x 32
+  // 13.1, 16 x 16 16.5, 32 x 32 19.5; 64 -> 64 over 2 900 32 x 32 13.0, 64 x 16
+  // 14; 128 -> 128 over 3 600 64 x 32 22, 64 x 16 25.9).  Four blocks are worth it for
+  // weights as [O][K][N] only (8 -> 128 over 160 000 135 against 148).
   const int64_t cus = compute_units(), cols = div_ceil(N, int64_t{16});
-  const int64_t full = div_ceil(Tn, int64_t{64}) * cols;         // workgroups of 64 targets and 16 channels
-  int c = 1, targets = 64, split = 4;
-  if (4 * full >= 19 * cus) {
-    c = N % 64 == 0 ? 4 : N % 32 == 0 ? 2 : 1;
-  } else if (16 * full >= 15 * cus) {
-    split = 4 * full <= 9 * cus ? 8 : 4;
-  } else if (20 * full >= 7 * cus) {
-    targets = 32;
-    split = 2 * full <= cus ? 8 : 4;
+  const double full = static_cast<double>(div_ceil(Tn, int64_t{64}) * cols) / static_cast<double>(cus);
+  int c = 1, targets = 64, split = full < 2.25 ? 8 : 4;
+  if (N % 32 != 0) {
+    targets = full < 0.3 ? 16 : full < 0.9 ? 32 : 64;
+  } else if (full < 0.6) {
+    c = full >= 0.26 && full < 0.42 ? 2 : 1;
+    targets = full < 0.42 ? 16 : 32;
+  } else if (full < 1.37) {
+    c = full < 0.93 ? 2 : 1;
+    targets = full < 0.93 ? 32 : 64;
   } else {
-    targets = 16;
-    split = 8;
+    c = full >= 4.75 && N % 64 == 0 ? 4 : 2;
+    targets = full >= 1.95 && full < 3.0 ? 32 : 64;
+    split = full < 1.95 ? 8 : 4;
   }
-  const dim3 grid(static_cast<unsigned>(div_ceil(Tn, int64_t{targets})), static_cast<unsigned>(div_ceil(cols, int64_t{c})));
-#define MNT_COMPACT_W(C, KI, SPLIT, TARGETS, WHOLE)                                                            \
-  compact_forward_kernel<C, KI, SPLIT, TARGETS, WHOLE><<<grid, 64 * SPLIT, 0, stream>>>(                       \
-      sources, static_cast<unsigned>(S * K * 4), weights, static_cast<unsigned>(O * K * N * 4), kernel_map, s, \
+  s.steps = static_cast<int>(div_ceil(K, int64_t{16}));
+  // Columns side by side, so that the workgroups of a die share few of them and
+  // its L2 holds their weights, up to the threads a grid may have along x.
+  const int64_t rows = div_ceil(Tn, int64_t{targets}), columns = div_ceil(cols, int64_t{c});
+  const bool beside = rows * columns * 64 * split < (int64_t{1} << 32);
+  s.columns = beside ? static_cast<int>(columns) : 1;
+  const dim3 grid(static_cast<unsigned>(beside ? rows * columns : rows), static_cast<unsigned>(beside ? 1 : columns));
+  const unsigned weight_bytes = static_cast<unsigned>((lanes ? lane_weight_floats(O, K, N) : O * K * N) * 4);
+#define MNT_COMPACT_W(C, KI, SPLIT, TARGETS, WHOLE, LANES)                                                     \
+  compact_forward_kernel<C, KI, SPLIT, TARGETS, WHOLE, LANES><<<grid, 64 * SPLIT, 0, stream>>>(                \
+      sources, static_cast<unsigned>(S * K * 4), weights, weight_bytes, kernel_map, s,                         \
       reinterpret_cast<unsigned char *>(out), ep)
-#define MNT_COMPACT(C, KI, SPLIT, TARGETS)             \
-  if (whole) {                                         \
-    MNT_COMPACT_W(C, KI, SPLIT, TARGETS, true);        \
-  } else {                                             \
-    MNT_COMPACT_W(C, KI, SPLIT, TARGETS, false);       \
+#define MNT_COMPACT(C, KI, SPLIT, TARGETS)               \
+  if (lanes && whole) {                                  \
+    MNT_COMPACT_W(C, KI, SPLIT, TARGETS, true, true);    \
+  } else if (lanes) {                                    \
+    MNT_COMPACT_W(C, KI, SPLIT, TARGETS, false, true);   \
+  } else if (whole) {                                    \
+    MNT_COMPACT_W(C, KI, SPLIT, TARGETS, true, false);   \
+  } else {                                               \
+    MNT_COMPACT_W(C, KI, SPLIT, TARGETS, false, false);  \
   }
 #define MNT_COMPACT_K(C, SPLIT, TARGETS)               \
   switch (ki) {                                        \
@@ -283,7 +359,19 @@ void compact_forward(const float *sources, const float *weights, const int *kern
   if (c == 4) {
     MNT_COMPACT_K(4, 4, 64)
   } else if (c == 2) {
-    MNT_COMPACT_K(2, 4, 64)
+    if (targets == 16) {
+      MNT_COMPACT_K(2, 8, 16)
+    } else if (targets == 32) {
+      if (split == 8) {
+        MNT_COMPACT_K(2, 8, 32)
+      } else {
+        MNT_COMPACT_K(2, 4, 32)
+      }
+    } else if (split == 8) {
+      MNT_COMPACT_K(2, 8, 64)
+    } else {
+      MNT_COMPACT_K(2, 4, 64)
+    }
   } else if (targets == 16) {
     MNT_COMPACT_K(1, 8, 16)
   } else if (targets == 32) {
@@ -304,3 +392,17 @@ void compact_forward(const float *sources, const float *weights, const int *kern
 }
 
 }  // namespace mnt
+
+using namespace mnt;
+
+extern "C" int mnt_pack_weights_in_lanes(const float *weights, int64_t O, int64_t K, int64_t N, float *packed_out,
+                                         void *stream_) {
+  return guarded([&] {
+    MNT_CHECK(O >= 0 && O <= 65535 && K >= 1 && N >= 1 && K <= 65536 && N <= 65536,
+              "bad shape O=%lld Cin=%lld Cout=%lld", (long long)O, (long long)K, (long long)N);
+    if (O == 0) return;
+    MNT_CHECK(weights != nullptr && packed_out != nullptr, "null operand");
+    MNT_CHECK(reinterpret_cast<uintptr_t>(packed_out) % 16 == 0, "packed weights are not 16-byte aligned");
+    pack_lanes(weights, O, K, N, packed_out, static_cast<hipStream_t>(stream_));
+  });
+}

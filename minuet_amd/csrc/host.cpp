@@ -46,6 +46,8 @@ using TablesFn = int (*)(int64_t, int64_t, int, int64_t, int, double, const void
                          int, float, const void *, const int64_t *, void *, void *);
 using TiledFn = int (*)(const void *, const void *, const int32_t *, int64_t, int64_t, int64_t, int64_t, int64_t, int,
                         const float *, const float *, const void *, int, float, void *, void *);
+using LanesFn = int (*)(const void *, const void *, const int32_t *, int64_t, int64_t, int64_t, int64_t, int64_t,
+                        const float *, const float *, const void *, int, float, void *, void *);
 using TilesFn = int (*)(const int32_t *, int64_t, int64_t, int32_t *, void *);
 using TilesSizeFn = int (*)(int64_t, int64_t, int64_t *);
 using TilesShareFn = double (*)(int64_t, int64_t, int64_t, int64_t, int);
@@ -55,6 +57,7 @@ ImplicitFn g_implicit = nullptr;
 GroupsFn g_groups = nullptr;
 TablesFn g_tables = nullptr;
 TiledFn g_tiled = nullptr;
+LanesFn g_lanes = nullptr;
 TilesFn g_tiles = nullptr;
 TilesSizeFn g_tiles_size = nullptr;
 TilesShareFn g_tiles_share = nullptr;
@@ -263,6 +266,7 @@ struct Layer {
   PyObject *shape_id;                         // key of this layer's map inside the cache's _fast_maps
   PyObject *dataflow, *threshold, *gather_tile, *scatter_tile;
   int kind, float_code, device;
+  int in_lanes;                               // packed is in lane order (fp32)
   int shortcut, has_threshold;
   double threshold_value;
   int64_t gather_tile_value, scatter_tile_value;
@@ -352,6 +356,7 @@ PyObject *layer_new(PyTypeObject *type, PyObject *args, PyObject *) {
   l->num_offsets = w->size(0);
   l->in_channels = w->size(1);
   l->out_channels = w->size(2);
+  l->in_lanes = tensor_of(packed)->dim() == 5 ? 1 : 0;
   l->has_threshold = l->threshold == Py_None ? 0 : 1;
   l->threshold_value = l->has_threshold ? PyFloat_AsDouble(l->threshold) : 0.0;
   l->gather_tile_value = l->gather_tile == Py_None ? 0 : PyLong_AsLongLong(l->gather_tile);
@@ -554,6 +559,12 @@ PyObject *run_layer(Layer *l, PyObject *module_dict, PyObject *inputs, const Epi
   int status = 0;
   switch (l->kind) {
     case kImplicit:
+      if (l->in_lanes) {
+        status = g_lanes(source, packed_at, static_cast<const int32_t *>(map->at[0]), S, T, l->num_offsets,
+                         l->in_channels, l->out_channels, scale_at, shift_at, data(residual), ep.activation, ep.slope,
+                         out.mutable_data_ptr(), stream);
+        break;
+      }
       if (const at::Tensor *tiles = tiles_of(map, l, T, kernel.device(), current)) {
         status = g_tiled(source, packed_at, static_cast<const int32_t *>(tiles->const_data_ptr()), S, T,
                          l->num_offsets, l->in_channels, l->out_channels, l->float_code, scale_at, shift_at,
@@ -799,6 +810,7 @@ PyObject *py_bind(PyObject *, PyObject *args) {
   g_groups = reinterpret_cast<GroupsFn>(address("mnt_sparse_convolution_forward_groups"));
   g_tables = reinterpret_cast<TablesFn>(address("mnt_sparse_convolution_forward_fused"));
   g_tiled = reinterpret_cast<TiledFn>(address("mnt_sparse_convolution_forward_tiled"));
+  g_lanes = reinterpret_cast<LanesFn>(address("mnt_sparse_convolution_forward_in_lanes"));
   g_tiles = reinterpret_cast<TilesFn>(address("mnt_kernel_map_tiles"));
   g_tiles_size = reinterpret_cast<TilesSizeFn>(address("mnt_kernel_map_tiles_size"));
   g_tiles_share = reinterpret_cast<TilesShareFn>(address("mnt_kernel_map_tiles_share"));

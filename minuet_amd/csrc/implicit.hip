@@ -39,8 +39,9 @@ template <typename T>
 void streamed_forward(const T *sources, const T *packed, const int *kernel_map, const int *tiles, int64_t S, int64_t Tn,
                       int64_t O, int64_t K, int64_t N, const Epilogue &ep, T *out, hipStream_t stream);
 
-void compact_forward(const float *sources, const float *weights, const int *kernel_map, int64_t S, int64_t Tn,
-                     int64_t O, int64_t K, int64_t N, const Epilogue &ep, float *out, hipStream_t stream);
+void compact_forward(const float *sources, const float *weights, bool lanes, const int *kernel_map, int64_t S,
+                     int64_t Tn, int64_t O, int64_t K, int64_t N, const Epilogue &ep, float *out, hipStream_t stream);
+int64_t lane_weight_floats(int64_t O, int64_t K, int64_t N);
 
 constexpr int kImplicitBlock = 256;
 constexpr int kImplicitTargets = 128;     // per workgroup, 32 per wavefront
@@ -556,7 +557,7 @@ static void implicit_typed(const T *sources, const T *weights, const T *packed, 
     // fp32 products are dear: hits only, wherever the weights are given as they are
     if (O > 1 && weights != nullptr && reinterpret_cast<uintptr_t>(weights) % 16 == 0 &&
         O * K * N * 4 < static_cast<int64_t>(kMaxSourceBytes)) {
-      compact_forward(sources, weights, kernel_map, S, Tn, O, K, N, ep, out, stream);
+      compact_forward(sources, weights, false, kernel_map, S, Tn, O, K, N, ep, out, stream);
       profile_mark("implicit", stream);
       return;
     }
@@ -693,6 +694,39 @@ extern "C" int mnt_sparse_convolution_forward_implicit(
       implicit_typed<bf16_t>(static_cast<const bf16_t *>(sources), static_cast<const bf16_t *>(weights),
                              static_cast<const bf16_t *>(packed_weights), kernel_map, S, T, O, K, N, ep, static_cast<bf16_t *>(out), stream);
     }
+  });
+}
+
+extern "C" int mnt_sparse_convolution_forward_in_lanes(
+    const float *sources, const float *packed_weights, const int32_t *kernel_map, int64_t S, int64_t T, int64_t O,
+    int64_t K, int64_t N, const float *channel_scale, const float *channel_shift, const void *residual, int activation,
+    float negative_slope, float *out, void *stream_) {
+  return guarded([&] {
+    hipStream_t stream = static_cast<hipStream_t>(stream_);
+    MNT_CHECK(S >= 0 && T >= 0 && O > 1 && K >= 1 && N >= 1 && S <= INT32_MAX && T <= INT32_MAX && O <= 65535,
+              "bad shape S=%lld T=%lld O=%lld Cin=%lld Cout=%lld", (long long)S, (long long)T, (long long)O,
+              (long long)K, (long long)N);
+    MNT_CHECK(S * K * 4 < static_cast<int64_t>(kMaxSourceBytes) &&
+                  lane_weight_floats(O, K, N) * 4 < static_cast<int64_t>(kMaxSourceBytes),
+              "source features or weights exceed the 4 GiB a buffer resource addresses");
+    MNT_CHECK(K % 4 == 0 && K * 4 <= kImplicitMaxRowBytes && N % 4 == 0 &&
+                  N <= 32 * kImplicitMaxBlocks * kImplicitMaxGroups,
+              "Unsupported channel counts for weights in lane order: Cin = %lld (a multiple of 4, at most %d), "
+              "Cout = %lld (a multiple of 4, at most %d)",
+              (long long)K, kImplicitMaxRowBytes / 4, (long long)N, 32 * kImplicitMaxBlocks * kImplicitMaxGroups);
+    MNT_CHECK(activation >= MNT_ACT_NONE && activation <= MNT_ACT_RELU6, "unknown activation code %d", activation);
+    MNT_CHECK(reinterpret_cast<uintptr_t>(sources) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0 &&
+                  reinterpret_cast<uintptr_t>(residual) % 16 == 0 &&
+                  reinterpret_cast<uintptr_t>(packed_weights) % 16 == 0 &&
+                  reinterpret_cast<uintptr_t>(channel_scale) % 4 == 0 &&
+                  reinterpret_cast<uintptr_t>(channel_shift) % 4 == 0,
+              "operands are not aligned (features, out, residual, weights: 16 bytes, scale / shift: 4 bytes)");
+    if (T == 0) return;
+    MNT_CHECK(out != nullptr && kernel_map != nullptr && packed_weights != nullptr, "null operand");
+    const Epilogue ep = {channel_scale, channel_shift, residual, activation, negative_slope, nullptr};
+    profile_mark("enter:implicit", stream);
+    compact_forward(sources, packed_weights, true, kernel_map, S, T, O, K, N, ep, out, stream);
+    profile_mark("implicit", stream);
   });
 }
 

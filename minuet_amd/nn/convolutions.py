@@ -593,6 +593,7 @@ class SparseConv(Module):
         factory = {"device": device, "dtype": dtype}
         volume = int(np.prod(self.kernel_size))
         self._packed = None
+        self._lanes = None
         self._fast = None
         self.kernel = torch.nn.Parameter(torch.empty(volume, in_channels, out_channels, **factory))
         if bias:
@@ -669,6 +670,7 @@ class SparseConv(Module):
         nothing, so call this after them (``reset_parameters``, ``load_state_dict``
         and ``.to()`` / ``.half()`` / ``.cuda()`` do it themselves)."""
         self._packed = None
+        self._lanes = None
         self._fast = None
 
     def _load_from_state_dict(self, *args, **kwargs):
@@ -820,6 +822,22 @@ class SparseConv(Module):
                     weights = torch.nn.functional.pad(weights, (0, 0, 0, pad))
                 self._packed = (key, weights, F.pack_weights(weights), held)
         return self._packed[1], self._packed[2]
+
+    def _lane_kernel(self):
+        """``_packed_kernel`` of an fp32 layer that multiplies hits only, whose
+        kernel reads the weights in the order of its lanes (16 x 16 x 4 instructions
+        take them 1 KB at a load: 32 -> 32 channels over 200 000 voxels 55 and 50
+        us, 128 -> 64 over 2 900 27 and 21)."""
+        kernel = self.kernel
+        if (torch.is_grad_enabled() and kernel.requires_grad) or not _C.lane_weights_supported(kernel):
+            return self._packed_kernel()
+        key = (kernel.data_ptr(), kernel._version, kernel.dtype, kernel.device)
+        kept = self.__dict__.get("_lanes")          # (none in a module pickled before there were any)
+        if kept is None or kept[0] != key:
+            with torch.no_grad():
+                weights = kernel.detach()
+                kept = self._lanes = (key, weights, _C.pack_weights_in_lanes(weights))
+        return kept[1], kept[2]
 
     def _row_padding(self, features: torch.Tensor) -> int:
         """Zero input channels to append so that the feature rows of a 16-bit
@@ -976,9 +994,9 @@ class SparseConv(Module):
                 dense = cache.get_dense_kernel_map(**map_args)
                 if pad:
                     sources = torch.nn.functional.pad(sources, (0, pad))
-                weights, packed = self._packed_kernel(pad)
+                weights, packed = self._packed_kernel(pad) if not hits else self._lane_kernel()
                 tiles = None
-                if packed is not None and F.prefers_streamed(volume, sources.shape[1], self.out_channels, sources.dtype):
+                if packed is not None and not hits and F.prefers_streamed(volume, sources.shape[1], self.out_channels, sources.dtype):
                     tiles = cache.get_tiles(dense, sources.shape[1], self.out_channels, sources.dtype, inputs.C,
                                             inputs.stride, stride, self.kernel_size, self.dilation, self.transposed)
                 if tiles is not None:

@@ -107,6 +107,9 @@ SIGNATURES = {
     "mnt_kernel_map_tiles_size": (_int, [_i64, _i64, ctypes.POINTER(_i64)]),
     "mnt_kernel_map_tiles": (_int, [_vp, _i64, _i64, _vp, _vp]),
     "mnt_kernel_map_tiles_share": (ctypes.c_double, [_i64, _i64, _i64, _i64, _int]),
+    "mnt_pack_weights_in_lanes": (_int, [_vp, _i64, _i64, _i64, _vp, _vp]),
+    "mnt_sparse_convolution_forward_in_lanes": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _vp, _vp, _vp,
+                                                       _int, ctypes.c_float, _vp, _vp]),
     "mnt_sparse_convolution_streamed": (_int, [_i64, _i64, _i64, _i64, _int]),
     "mnt_sparse_convolution_forward_tiled": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _vp, _vp, _vp,
                                                     _int, ctypes.c_float, _vp, _vp]),
@@ -190,7 +193,8 @@ def _bound_host():
     spec.loader.exec_module(module)
     names = ("mnt_sparse_convolution_forward_implicit", "mnt_sparse_convolution_forward_groups",
              "mnt_sparse_convolution_forward_fused", "mnt_sparse_convolution_forward_tiled", "mnt_kernel_map_tiles",
-             "mnt_kernel_map_tiles_size", "mnt_kernel_map_tiles_share", "mnt_last_error")
+             "mnt_sparse_convolution_forward_in_lanes", "mnt_kernel_map_tiles_size", "mnt_kernel_map_tiles_share",
+             "mnt_last_error")
     hooks = tuple(getattr(torch_module, name) for name in (
         "_global_forward_hooks", "_global_forward_pre_hooks", "_global_backward_hooks",
         "_global_backward_pre_hooks"))
@@ -1400,6 +1404,36 @@ def pack_weights(weights: torch.Tensor) -> torch.Tensor:
     return packed
 
 
+def lane_weights_shape(weights: torch.Tensor):
+    """Shape of :func:`pack_weights_in_lanes`'s result for ``weights [O, C_in, C_out]``."""
+    O, K, N = weights.shape
+    return O, -(-N // 16), -(-K // 16), 64, 4
+
+
+def pack_weights_in_lanes(weights: torch.Tensor) -> torch.Tensor:
+    """fp32 ``weights [O, C_in, C_out]`` in the order in which
+    :func:`sparse_convolution_forward_implicit` multiplies them, 16 x 16 of one
+    offset after the other.  Kept by a layer like :func:`pack_weights`'s result."""
+    _ensure_ndim("weights", weights, 3)
+    device = _common_device([weights])
+    if weights.dtype != torch.float32:
+        _fail("pack_weights_in_lanes expects fp32 weights")
+    weights = weights.contiguous()
+    packed = torch.empty(lane_weights_shape(weights), dtype=weights.dtype, device=device)
+    O, K, N = weights.shape
+    with _on(device):
+        _check(load_library().mnt_pack_weights_in_lanes(_ptr(weights), O, K, N, _ptr(packed), _stream(device)))
+    return packed
+
+
+def lane_weights_supported(weights: torch.Tensor) -> bool:
+    """Whether the fp32 single-kernel forward takes these weights in lane order."""
+    O, K, N = weights.shape
+    blocks, steps = lane_weights_shape(weights)[1:3]
+    return (weights.dtype == torch.float32 and O > 1 and implicit_forward_supported(K, N, weights.dtype)
+            and O * blocks * steps * 1024 < IMPLICIT_MAX_SOURCE_BYTES)
+
+
 def _check_packed(packed: torch.Tensor, weights: torch.Tensor):
     if (tuple(packed.shape) != packed_weights_shape(weights) or packed.dtype != weights.dtype
             or packed.device != weights.device or not packed.is_contiguous()):
@@ -1456,7 +1490,9 @@ def sparse_convolution_forward_implicit(sources: torch.Tensor, weights: torch.Te
                                         epilogue: Optional[Epilogue] = None,
                                         packed_weights: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Output-stationary forward from the dense kernel map ``[O, N_out]`` (int32,
-    original offset order): one kernel, no gather / GEMM-output buffers."""
+    original offset order): one kernel, no gather / GEMM-output buffers.
+    ``packed_weights``: :func:`pack_weights` or, in fp32, :func:`pack_weights_in_lanes`
+    of ``weights``."""
     fn = "sparse_convolution_forward_implicit"
     device = sources.device
     dtype = weights.dtype
@@ -1488,6 +1524,17 @@ def sparse_convolution_forward_implicit(sources: torch.Tensor, weights: torch.Te
         sources = sources.clone()
     out = torch.empty((T, N), dtype=weights.dtype, device=device)
     ep = Epilogue() if epilogue is None else epilogue.checked(T, N, weights.dtype, device)
+    if packed_weights is not None and packed_weights.dim() == 5:
+        if (tuple(packed_weights.shape) != lane_weights_shape(weights) or not lane_weights_supported(weights)
+                or packed_weights.dtype != dtype or packed_weights.device != device
+                or not packed_weights.is_contiguous()):
+            _fail("packed_weights does not belong to these weights (shape, dtype, device or layout)")
+        with _on(device):
+            _check(load_library().mnt_sparse_convolution_forward_in_lanes(
+                _ptr(sources), _ptr(packed_weights), _ptr(kernel_map), S, T, O, K, N, _ptr(ep.scale), _ptr(ep.shift),
+                _ptr(ep.residual), ACTIVATION_CODES[ep.activation], float(ep.negative_slope), _ptr(out),
+                _stream(device)))
+        return out
     if packed_weights is not None:
         _check_packed(packed_weights, weights)
     with _on(device):

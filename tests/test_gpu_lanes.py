@@ -1,0 +1,80 @@
+"""fp32 layers that multiply hits only, with weights as given and in lane order:
+every workgroup shape, channel counts that fill no block, targets that fill no
+workgroup."""
+import pytest
+import torch
+
+import minuet_amd as minuet
+from minuet_amd.nn import functional as F
+from minuet_amd.nn.functional import _C
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(targets, offsets, K, N, density, seed):
+    gen = torch.Generator().manual_seed(seed)
+    sources = targets + 3
+    dense = torch.randint(0, sources, (offsets, targets), generator=gen, dtype=torch.int32)
+    dense[torch.rand(offsets, targets, generator=gen) >= density] = -1
+    x = torch.randn(sources, K, generator=gen)
+    w = torch.randn(offsets, K, N, generator=gen) / (K * offsets * density) ** 0.5
+    return dense, x, w
+
+
+def _oracle(dense, x, w):
+    out = torch.zeros(dense.shape[1], w.shape[2], dtype=torch.float64)
+    for o in range(dense.shape[0]):
+        t = torch.nonzero(dense[o] >= 0)[:, 0]
+        out[t] += x[dense[o][t].long()].double() @ w[o].double()
+    return out
+
+
+# workgroups of 64 targets and 16 channels to a compute unit pick the shape: from a handful to several
+@pytest.mark.parametrize("targets", [1, 15, 17, 130, 700, 2100, 5003, 9001, 20011])
+@pytest.mark.parametrize("offsets, K, N", [(27, 32, 32), (8, 64, 128), (27, 20, 36), (2, 4, 4), (27, 80, 64)])
+def test_lane_order_is_the_same_product(targets, offsets, K, N):
+    dense, x, w = _case(targets, offsets, K, N, 0.3, targets + K)
+    expected = _oracle(dense, x, w)
+    dense, x, w = dense.cuda(), x.cuda(), w.cuda()
+    plain = _C.sparse_convolution_forward_implicit(x, w, dense)
+    lanes = _C.sparse_convolution_forward_implicit(x, w, dense, packed_weights=_C.pack_weights_in_lanes(w))
+    # fp32 sums of up to offsets * K products of two unit normals over sqrt(their number)
+    bound = 8 * 2.0 ** -24 * (offsets * K) ** 0.5
+    assert (plain.cpu().double() - expected).abs().max() < bound
+    assert lanes.equal(plain)
+
+
+@pytest.mark.parametrize("activation", [None, "relu"])
+def test_lane_order_epilogue(activation):
+    dense, x, w = (t.cuda() for t in _case(333, 27, 48, 72, 0.4, 5))
+    epilogue = _C.Epilogue(torch.rand(72).cuda(), torch.randn(72).cuda(), torch.randn(333, 72).cuda(), activation)
+    plain = _C.sparse_convolution_forward_implicit(x, w, dense, epilogue=epilogue)
+    lanes = _C.sparse_convolution_forward_implicit(x, w, dense, epilogue=epilogue,
+                                                   packed_weights=_C.pack_weights_in_lanes(w))
+    assert lanes.equal(plain)
+
+
+def test_lane_weights_follow_the_parameter():
+    coordinates = torch.unique(torch.randint(0, 12, (900, 3), generator=torch.Generator().manual_seed(1),
+                                             dtype=torch.int32), dim=0).cuda()
+    coordinates = coordinates[F.build_sorted_index(coordinates)]
+    conv = minuet.nn.SparseConv3d(32, 32, 3, device="cuda")
+    conv.set_kernel_map_cache(minuet.nn.KernelMapCache(ndim=3, dtype=torch.int32, device="cuda"))
+    x = minuet.SparseTensor(torch.randn(len(coordinates), 32, device="cuda"), coordinates)
+    with torch.no_grad():
+        first = conv(x).F.clone()
+        lanes = conv._lanes[2]
+        assert conv(x).F.equal(first) and conv._lanes[2] is lanes      # (and past Python)
+        conv.kernel.mul_(2.0)                                          # in place: same storage, new version
+        assert conv(x).F.equal(2 * first) and conv._lanes[2] is not lanes
+        assert conv(x).F.equal(2 * first)
+    assert conv(x).F.detach().equal(2 * first)                         # gradients are recorded: as they are
+
+
+def test_refuses_another_layer_s_weights():
+    dense, x, w = (t.cuda() for t in _case(50, 27, 32, 32, 0.3, 2))
+    with pytest.raises((RuntimeError, ValueError)):
+        _C.sparse_convolution_forward_implicit(x, w, dense, packed_weights=_C.pack_weights_in_lanes(w[:8]))
+    with pytest.raises((RuntimeError, ValueError)):
+        _C.sparse_convolution_forward_implicit(x[:, :32].half(), w.half(), dense,
+                                               packed_weights=_C.pack_weights_in_lanes(w))
