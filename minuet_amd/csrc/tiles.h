@@ -16,10 +16,9 @@ constexpr int kTileMaxOffsets = 128;
 constexpr int kTileXcds = 8;                  // windows are dealt to the compute dies in turn
 
 // Targets are sorted within windows of consecutive ones.  The windows' number
-// is a multiple of the compute dies', and tile p belongs to window
-// (p / 8 / tiles_per_window) * 8 + p % 8: workgroups go to the dies in turn, so
-// that the tiles of a window stay on one die and find each other's source rows
-// in its L2.
+// is a multiple of the compute dies' and workgroups go to the dies in turn, so
+// window w's tiles, all at numbers of w % 8 modulo 8, stay on one die and find
+// each other's source rows in its L2.
 struct TileLayout {
   int windows, window, per_window;            // window: targets of one (a multiple of kTileTargets)
   int64_t tiles;                              // windows * per_window
@@ -38,6 +37,28 @@ struct TileLayout {
     ints = sources_at + tiles * slots * kTileTargets;
   }
 };
+
+// The number of the `place`-th longest tile of a window, which is when it runs.
+// The longest tiles of all windows go first: one of a map's rare tiles of 27
+// live offsets takes three times the average, and the chip waited for those of
+// the last windows.  Then the next longest of a band of windows at a time, as
+// many as leave their rows in a die's L2 (seven of 4096 128-byte rows), and not
+// window after window, whose long tiles leave gaps.  us a layer with 8 windows
+// after the other, all windows at a time, and so: 64 -> 64 channels of 16 bits
+// over 200 000 LiDAR voxels 33.9, 27.5, 26.7, over a room of 150 000 27.7, 22.0, 20.1;
+// 5x5x5 over a million 430, 423, 407; 32 -> 32 over a million 83.8, 83.8, 77.1.
+constexpr int kTileFirst = 2, kTileBand = 7;
+__device__ __forceinline__ int tile_number(int windows, int per_window, int window, int place) {
+  const int rows = windows / kTileXcds, row = window / kTileXcds;      // windows of a die
+  const int first = per_window < kTileFirst ? per_window : kTileFirst;
+  int at = place * rows + row;                                         // among the die's tiles
+  if (place >= first) {
+    const int band = row / kTileBand * kTileBand;
+    const int in_band = rows - band < kTileBand ? rows - band : kTileBand;
+    at = first * rows + band * (per_window - first) + (place - first) * in_band + row - band;
+  }
+  return at * kTileXcds + window % kTileXcds;
+}
 
 struct TileView {
   const int *rows;      // [tiles][128] target of a tile's place, -1 for none

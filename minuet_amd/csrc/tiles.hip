@@ -246,7 +246,7 @@ __global__ __launch_bounds__(kTileSortBlock) void tile_sort_kernel(
     const unsigned long long votes = __ballot(in && (theirs > mine || (theirs == mine && p < j)));
     if (p == 0 && j < per_window) {
       const int longer = __popc(static_cast<unsigned>(lane < 32 ? votes : votes >> 32));
-      const int tile = (blockIdx.x / kTileXcds * per_window + longer) * kTileXcds + blockIdx.x % kTileXcds;
+      const int tile = tile_number(gridDim.x, per_window, blockIdx.x, longer);
       counts[tile] = mine;
 #pragma unroll
       for (int w = 0; w < WORDS; ++w) masks[tile * WORDS + w] = s_tile[j][w];

@@ -232,3 +232,27 @@ def test_tiles_made_on_one_stream_and_read_on_another():
             taken = [torch.zeros(size.value, dtype=torch.int32, device=DEVICE) for _ in range(3)]
         torch.cuda.synchronize()
     assert torch.equal(last, first) and len(taken) == 3
+
+
+@pytest.mark.parametrize("targets", [1, 129, 32769, 7 * 32768 + 1, 16 * 32768 + 77])
+def test_every_target_has_one_place(targets):
+    """One window of tiles per die, several, more than a band of them and two
+    bands with a remainder: every target stands in one tile, and the tiles of
+    the smallest numbers are a window's longest."""
+    gen = torch.Generator(device="cuda").manual_seed(targets)
+    dense = torch.randint(0, targets, (9, targets), generator=gen, device="cuda", dtype=torch.int32)
+    dense[torch.rand(9, targets, generator=gen, device="cuda") < 0.8] = -1
+    windows = 8 * max(1, -(-targets // 32768))
+    window = -(-max(1, -(-targets // windows)) // 128) * 128
+    tiles = windows * window // 128
+    packed = _C.kernel_map_tiles(dense)
+    rows = packed[:tiles * 128].view(tiles, 128)
+    counts = packed[tiles * 128:tiles * 128 + tiles]
+    assert rows[rows >= 0].sort().values.equal(torch.arange(targets, device="cuda", dtype=torch.int32))
+    used = rows.amax(1) >= 0
+    assert (counts > 0).equal(used)
+    owner = torch.where(used, rows.amax(1) // window, -1)
+    assert (owner[used] % 8).equal(torch.arange(tiles, device="cuda", dtype=torch.int32)[used] % 8)
+    for w in range(0, windows, max(1, windows // 5)):
+        mine = counts[owner == w]
+        assert mine.equal(mine.sort(descending=True).values)
