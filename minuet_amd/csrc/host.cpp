@@ -166,6 +166,7 @@ struct MapEntry {
   // would have saved so far, over what making them takes (below 0: never).
   PyObject *tiles;
   double tiles_credit;
+  double tiles_saved;      // what they saved or would have saved all the layers that have run
   // The stream that makes the tiles, the end of that work, and whether the host
   // has seen it ended.
   void *tiles_stream;
@@ -230,6 +231,7 @@ PyObject *map_entry_new(PyTypeObject *type, PyObject *args, PyObject *) {
   e->used = 0;
   e->tiles = tiles == Py_None ? nullptr : hold(tiles);
   e->tiles_credit = 0.0;
+  e->tiles_saved = 0.0;
   e->tiles_stream = made_on;
   e->tiles_made = made.release();
   e->tiles_ready = 0;
@@ -250,7 +252,14 @@ PyObject *map_entry_used(PyObject *self, void *) {
   return PyBool_FromLong(reinterpret_cast<MapEntry *>(self)->used);
 }
 
+PyObject *map_entry_tiles_saved(PyObject *self, void *) {
+  return PyFloat_FromDouble(reinterpret_cast<MapEntry *>(self)->tiles_saved);
+}
+
 PyGetSetDef map_entry_getset[] = {{"used", map_entry_used, nullptr, "Whether a layer has run with this map.", nullptr},
+                                  {"tiles_saved", map_entry_tiles_saved, nullptr,
+                                   "What tiles saved, or would have saved, the layers that ran with this map, over "
+                                   "what making them takes.", nullptr},
                                   {nullptr, nullptr, nullptr, nullptr, nullptr}};
 
 PyTypeObject MapEntryType = {PyVarObject_HEAD_INIT(nullptr, 0)};
@@ -384,8 +393,9 @@ inline bool vector_fits(const at::Tensor *t, int64_t channels, int device) {
 // loses half its time without, makes them at once (a share of kTilesCredit); the
 // others' are made once
 // the forwards that have run over it would have saved twice their price: a map
-// that a network reads a few times and drops never pays for them, one that is
-// read on and on soon does.  Layers of all widths and types share a map, so
+// that a network reads a few times and drops does not pay for them there (a
+// pass that is built ahead makes them for less, from what the pass before it
+// would have saved), one that is read on and on soon does.  Layers of all widths and types share a map, so
 // whether this one can use tiles (a share of 0: it cannot) is asked first.
 constexpr double kTilesCredit = 2.0;
 constexpr int64_t kTilesMostInts = int64_t{1} << 29;
@@ -426,6 +436,7 @@ const at::Tensor *tiles_of(MapEntry *map, const Layer *l, int64_t T, const at::D
                            const c10::hip::HIPStream &stream) {
   const double share = g_tiles_share(T, l->num_offsets, l->in_channels, l->out_channels, l->float_code);
   if (share == 0.0) return nullptr;
+  map->tiles_saved += share;
   if (map->tiles == nullptr) {
     if (map->tiles_credit < 0.0) return nullptr;
     map->tiles_credit += share;

@@ -768,7 +768,7 @@ extern "C" int mnt_sparse_convolution_streamed(int64_t T, int64_t O, int64_t K, 
 // 25 600 of a scan 77 and 37; over 9 000, 128 -> 128: 15.2 and 13.4).
 // Others: fitted to layers of
 // 32 to 128 channels over 100 000 to a million targets: a forward gets faster by
-// 1.1 us per million (offset, target) pairs and unit of (channel blocks + 1) x
+// 1.3 us per million (offset, target) pairs and unit of (channel blocks + 1) x
 // 128-byte pieces of a row, making tiles takes 28 us and 2.5 us per million pairs.
 extern "C" double mnt_kernel_map_tiles_share(int64_t T, int64_t O, int64_t K, int64_t N, int float_dtype) {
   if (float_dtype == MNT_FLOAT32 || O <= 8 || O > kTileMaxOffsets || T < 1 || K < 1 || N < 1 ||
@@ -784,7 +784,7 @@ extern "C" double mnt_kernel_map_tiles_share(int64_t T, int64_t O, int64_t K, in
   if (T <= static_cast<int64_t>(2 * kTileTargets) * compute_units()) return 0.0;
   const double pairs = 1e-6 * static_cast<double>(T) * static_cast<double>(O);
   const double pieces = K * 2 <= 64 ? 0.5 : static_cast<double>(div_ceil(K * 2, 128));
-  return 1.1 * pairs * static_cast<double>(div_ceil(N, 32) + 1) * pieces / (28.0 + 2.5 * pairs);
+  return 1.3 * pairs * static_cast<double>(div_ceil(N, 32) + 1) * pieces / (28.0 + 2.5 * pairs);
 }
 
 extern "C" int mnt_sparse_convolution_forward_tiled(

@@ -10,6 +10,7 @@
 // buffer rows for every hit).
 #include <algorithm>
 #include <type_traits>
+#include <vector>
 
 #include "device_utils.h"
 #include "tiles.h"
@@ -18,21 +19,49 @@ namespace mnt {
 
 constexpr int kTileSortBlock = 1024;
 constexpr int kTileSortWaves = kTileSortBlock / kWave;
-constexpr int kTileSortItems = kTileWindow / kTileSortBlock;
 constexpr int kTileDigitBits = 7;
 constexpr int kTileDigits = 1 << kTileDigitBits;
 constexpr int kTileKeyBits = 49;              // of the offsets' bits, under the 12 bits of a place in the window
 constexpr int kTilePlaceBits = 12;
 static_assert(kTileWindow == 1 << kTilePlaceBits && kTileKeyBits % kTileDigitBits == 0, "a key and a place in one word");
 
+// The maps one set of launches takes: a network's pass makes the tiles of all its
+// maps at once, because the sort of one keeps 8 to 40 of 256 compute units busy
+// (the five maps of a network over 200 000 voxels: 160 us one after the other,
+// 37 together).
+constexpr int kTileJobs = 8;
+struct TileJob {
+  const int *dense;
+  long long num_targets;
+  int num_offsets, slots;
+  int windows, window, per_window;
+  int first_set, first_window, first_tile;     // workgroups of the jobs before
+  int *rows, *counts, *offsets, *sources;
+  unsigned *sets, *masks;
+};
+struct TileJobs {
+  TileJob job[kTileJobs];
+  int count;
+};
+
+__device__ __forceinline__ const TileJob &job_of(const TileJobs &jobs, int TileJob::*first) {
+  int j = 0;
+  while (j + 1 < jobs.count && static_cast<int>(blockIdx.x) >= jobs.job[j + 1].*first) ++j;
+  return jobs.job[j];
+}
+
 // The set of offsets of every target, WORDS words of 32 each ([WORDS][T]).  In a
 // launch of its own because it reads the whole dense map: the few workgroups
 // that sort would take 10 us for it, bound by what one compute unit can load.
 template <int WORDS>
-__global__ __launch_bounds__(256) void tile_sets_kernel(const int *__restrict__ dense, long long num_targets,
-                                                        int num_offsets, unsigned *__restrict__ sets) {
+__global__ __launch_bounds__(256) void tile_sets_kernel(const TileJobs jobs) {
   constexpr int kFlight = WORDS == 1 ? 27 : 16;
-  const long long t = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
+  const TileJob &job = job_of(jobs, &TileJob::first_set);
+  const int *__restrict__ dense = job.dense;
+  unsigned *__restrict__ sets = job.sets;
+  const long long num_targets = job.num_targets;
+  const int num_offsets = job.num_offsets;
+  const long long t = static_cast<long long>(blockIdx.x - job.first_set) * 256 + threadIdx.x;
   const int *column = dense + min(t, num_targets - 1);
 #pragma unroll
   for (int w = 0; w < WORDS; ++w) {
@@ -59,25 +88,42 @@ __global__ __launch_bounds__(256) void tile_sets_kernel(const int *__restrict__ 
 // digit bit.  Each tile's number of live offsets then ranks the tiles, longest
 // first, so that what runs last is short.
 template <int WORDS>
-__global__ __launch_bounds__(kTileSortBlock) void tile_sort_kernel(
-    const unsigned *__restrict__ sets, long long num_targets, int num_offsets, int window, int per_window,
-    int *__restrict__ rows, int *__restrict__ counts, unsigned *__restrict__ masks) {
-  __shared__ unsigned long long s_word[kTileWindow];
-  __shared__ unsigned s_mask[WORDS][kTileWindow];
-  __shared__ unsigned s_hist[kTileSortWaves][kTileDigits + 1];    // (+ 1: read down the wavefronts without conflicts)
-  __shared__ unsigned s_wave[kTileSortWaves];
-  __shared__ int s_count[kTileMaxOffsets];
-  __shared__ int s_chosen[kTileMaxOffsets];                      // offset of key bit k, from the top
-  __shared__ unsigned s_tile[kTileWindow / kTileTargets][WORDS];
-  __shared__ int s_live[kTileWindow / kTileTargets];
+struct TileSortLds {
+  unsigned long long word[kTileWindow];
+  unsigned mask[WORDS][kTileWindow];
+  unsigned hist[kTileSortWaves][kTileDigits + 1];    // (+ 1: read down the wavefronts without conflicts)
+  unsigned wave[kTileSortWaves];
+  int count[kTileMaxOffsets];
+  int chosen[kTileMaxOffsets];                       // offset of key bit k, from the top
+  unsigned tile[kTileWindow / kTileTargets][WORDS];
+  int live[kTileWindow / kTileTargets];
+};
+
+// ITEMS: the window's places in units of the block's threads.
+template <int WORDS, int ITEMS>
+__device__ __forceinline__ void tile_sort_body(const TileJob &job, TileSortLds<WORDS> &lds) {
+  constexpr int kTileSortItems = ITEMS;
+  const unsigned *__restrict__ sets = job.sets;
+  const long long num_targets = job.num_targets;
+  const int num_offsets = job.num_offsets, window = job.window, per_window = job.per_window;
+  const int this_window = blockIdx.x - job.first_window;
+  int *__restrict__ rows = job.rows;
+  int *__restrict__ counts = job.counts;
+  unsigned *__restrict__ masks = job.masks;
+  unsigned long long *const s_word = lds.word;
+  unsigned (*const s_mask)[kTileWindow] = lds.mask;
+  unsigned (*const s_hist)[kTileDigits + 1] = lds.hist;
+  unsigned *const s_wave = lds.wave;
+  int *const s_count = lds.count, *const s_chosen = lds.chosen, *const s_live = lds.live;
+  unsigned (*const s_tile)[WORDS] = lds.tile;
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
-  const long long first = static_cast<long long>(blockIdx.x) * window;
+  const long long first = static_cast<long long>(this_window) * window;
   const int here = static_cast<int>(min(static_cast<long long>(window), max(0ll, num_targets - first)));
   for (int i = tid; i < kTileMaxOffsets; i += kTileSortBlock) s_count[i] = 0;
   for (int i = tid; i < kTileWindow / kTileTargets * WORDS; i += kTileSortBlock) (&s_tile[0][0])[i] = 0u;
   __syncthreads();
 
-  // place wave * 256 + i * 64 + lane of the window
+  // place (wave * ITEMS + i) * 64 + lane of the window
   unsigned mask[kTileSortItems][WORDS];
   int place[kTileSortItems];
 #pragma unroll
@@ -246,7 +292,7 @@ __global__ __launch_bounds__(kTileSortBlock) void tile_sort_kernel(
     const unsigned long long votes = __ballot(in && (theirs > mine || (theirs == mine && p < j)));
     if (p == 0 && j < per_window) {
       const int longer = __popc(static_cast<unsigned>(lane < 32 ? votes : votes >> 32));
-      const int tile = tile_number(gridDim.x, per_window, blockIdx.x, longer);
+      const int tile = tile_number(job.windows, per_window, this_window, longer);
       counts[tile] = mine;
 #pragma unroll
       for (int w = 0; w < WORDS; ++w) masks[tile * WORDS + w] = s_tile[j][w];
@@ -263,16 +309,34 @@ __global__ __launch_bounds__(kTileSortBlock) void tile_sort_kernel(
   }
 }
 
+template <int WORDS>
+__global__ __launch_bounds__(kTileSortBlock) void tile_sort_kernel(const TileJobs jobs) {
+  __shared__ TileSortLds<WORDS> lds;
+  const TileJob &job = job_of(jobs, &TileJob::first_window);
+  if (job.window <= kTileSortBlock) {
+    tile_sort_body<WORDS, 1>(job, lds);
+  } else if (job.window <= 2 * kTileSortBlock) {
+    tile_sort_body<WORDS, 2>(job, lds);
+  } else {
+    tile_sort_body<WORDS, kTileWindow / kTileSortBlock>(job, lds);
+  }
+}
+
 // The source rows of a tile's live offsets, one row of 128 entries after the
 // other: a workgroup per tile, a thread per (target, every second live offset).
 template <int WORDS>
-__global__ __launch_bounds__(256) void tile_emit_kernel(const int *__restrict__ dense, long long num_targets,
-                                                        int num_offsets, int slots, const int *__restrict__ rows,
-                                                        const int *__restrict__ counts,
-                                                        const unsigned *__restrict__ masks, int *__restrict__ offsets,
-                                                        int *__restrict__ sources) {
+__global__ __launch_bounds__(256) void tile_emit_kernel(const TileJobs jobs) {
   __shared__ int s_offset[kTileMaxOffsets];
-  const long long tile = blockIdx.x;
+  const TileJob &job = job_of(jobs, &TileJob::first_tile);
+  const int *__restrict__ dense = job.dense;
+  const long long num_targets = job.num_targets;
+  const int num_offsets = job.num_offsets, slots = job.slots;
+  const int *__restrict__ rows = job.rows;
+  const int *__restrict__ counts = job.counts;
+  const unsigned *__restrict__ masks = job.masks;
+  int *__restrict__ offsets = job.offsets;
+  int *__restrict__ sources = job.sources;
+  const long long tile = blockIdx.x - job.first_tile;
   const int tid = threadIdx.x;
   const int live = counts[tile];
   const int row = rows[tile * kTileTargets + tid % kTileTargets];
@@ -322,30 +386,60 @@ __global__ __launch_bounds__(256) void tile_emit_kernel(const int *__restrict__ 
   }
 }
 
-void build_tiles(const int *dense, int64_t num_targets, int64_t num_offsets, int *tiles_out, hipStream_t stream) {
-  const TileLayout l(num_targets, num_offsets);
+struct TileRequest {
+  const int *dense;
+  int64_t num_targets, num_offsets;
+  int *out;
+};
+
+// The requests' maps have all up to 32 offsets, or all more.
+template <int WORDS>
+static void build_tiles(const TileRequest *requests, int count, hipStream_t stream) {
   Scope scope(stream);
-  const int words = num_offsets <= 32 ? 1 : 4;
-  unsigned *masks = scope.alloc<unsigned>(static_cast<size_t>(l.tiles) * words);
-  int *counts = tiles_out + l.counts_at;
-  unsigned *sets = scope.alloc<unsigned>(static_cast<size_t>(num_targets) * words);
-#define MNT_TILES(WORDS)                                                                                      \
-  tile_sets_kernel<WORDS><<<static_cast<unsigned>(div_ceil(num_targets, int64_t{256})), 256, 0, stream>>>(    \
-      dense, num_targets, static_cast<int>(num_offsets), sets);                                               \
-  check_launch("tile_sets_kernel");                                                                           \
-  tile_sort_kernel<WORDS><<<l.windows, kTileSortBlock, 0, stream>>>(                                          \
-      sets, num_targets, static_cast<int>(num_offsets), l.window, l.per_window, tiles_out, counts, masks);    \
-  check_launch("tile_sort_kernel");                                                                           \
-  tile_emit_kernel<WORDS><<<static_cast<unsigned>(l.tiles), 256, 0, stream>>>(                                \
-      dense, num_targets, static_cast<int>(num_offsets), l.slots, tiles_out, counts, masks,                   \
-      tiles_out + l.offsets_at, tiles_out + l.sources_at);                                                    \
-  check_launch("tile_emit_kernel")
-  if (words == 1) {
-    MNT_TILES(1);
-  } else {
-    MNT_TILES(4);
+  for (int from = 0; from < count; from += kTileJobs) {
+    TileJobs jobs = {};
+    jobs.count = std::min(kTileJobs, count - from);
+    int64_t set_blocks = 0, windows = 0, tiles = 0;
+    for (int j = 0; j < jobs.count; ++j) {
+      const TileRequest &r = requests[from + j];
+      const TileLayout l(r.num_targets, r.num_offsets);
+      TileJob &job = jobs.job[j];
+      job.dense = r.dense;
+      job.num_targets = r.num_targets;
+      job.num_offsets = static_cast<int>(r.num_offsets);
+      job.slots = l.slots;
+      job.windows = l.windows;
+      job.window = l.window;
+      job.per_window = l.per_window;
+      job.first_set = static_cast<int>(set_blocks);
+      job.first_window = static_cast<int>(windows);
+      job.first_tile = static_cast<int>(tiles);
+      job.rows = r.out;
+      job.counts = r.out + l.counts_at;
+      job.offsets = r.out + l.offsets_at;
+      job.sources = r.out + l.sources_at;
+      job.sets = scope.alloc<unsigned>(static_cast<size_t>(r.num_targets) * WORDS);
+      job.masks = scope.alloc<unsigned>(static_cast<size_t>(l.tiles) * WORDS);
+      set_blocks += div_ceil(r.num_targets, int64_t{256});
+      windows += l.windows;
+      tiles += l.tiles;
+    }
+    MNT_CHECK(set_blocks <= INT32_MAX, "tiles of %lld targets at once", (long long)(set_blocks * 256));
+    tile_sets_kernel<WORDS><<<static_cast<unsigned>(set_blocks), 256, 0, stream>>>(jobs);
+    check_launch("tile_sets_kernel");
+    tile_sort_kernel<WORDS><<<static_cast<unsigned>(windows), kTileSortBlock, 0, stream>>>(jobs);
+    check_launch("tile_sort_kernel");
+    tile_emit_kernel<WORDS><<<static_cast<unsigned>(tiles), 256, 0, stream>>>(jobs);
+    check_launch("tile_emit_kernel");
   }
-#undef MNT_TILES
+}
+
+static void check_tiles(const TileRequest &r) {
+  MNT_CHECK(r.num_targets >= 1 && r.num_targets <= INT32_MAX && r.num_offsets >= 1 && r.num_offsets <= kTileMaxOffsets,
+            "no tiles for %lld targets under %lld offsets (at most %d)", (long long)r.num_targets,
+            (long long)r.num_offsets, kTileMaxOffsets);
+  MNT_CHECK(r.dense != nullptr && r.out != nullptr, "null operand");
+  MNT_CHECK(reinterpret_cast<uintptr_t>(r.out) % 16 == 0, "tiles are not 16-byte aligned");
 }
 
 }  // namespace mnt
@@ -361,14 +455,23 @@ extern "C" int mnt_kernel_map_tiles_size(int64_t num_targets, int64_t num_offset
   });
 }
 
+extern "C" int mnt_kernel_map_tiles_batch(int64_t num_maps, const int32_t *const *kernel_maps,
+                                          const int64_t *num_targets, const int64_t *num_offsets,
+                                          int32_t *const *tiles_out, void *stream_) {
+  return guarded([&] {
+    MNT_CHECK(num_maps >= 0 && num_maps <= 65536, "tiles of %lld maps", (long long)num_maps);
+    std::vector<TileRequest> few, many;
+    for (int64_t i = 0; i < num_maps; ++i) {
+      const TileRequest r = {kernel_maps[i], num_targets[i], num_offsets[i], tiles_out[i]};
+      check_tiles(r);
+      (r.num_offsets <= 32 ? few : many).push_back(r);
+    }
+    build_tiles<1>(few.data(), static_cast<int>(few.size()), static_cast<hipStream_t>(stream_));
+    build_tiles<4>(many.data(), static_cast<int>(many.size()), static_cast<hipStream_t>(stream_));
+  });
+}
+
 extern "C" int mnt_kernel_map_tiles(const int32_t *kernel_map, int64_t num_targets, int64_t num_offsets,
                                     int32_t *tiles_out, void *stream_) {
-  return guarded([&] {
-    MNT_CHECK(num_targets >= 1 && num_targets <= INT32_MAX && num_offsets >= 1 && num_offsets <= kTileMaxOffsets,
-              "no tiles for %lld targets under %lld offsets (at most %d)", (long long)num_targets,
-              (long long)num_offsets, kTileMaxOffsets);
-    MNT_CHECK(kernel_map != nullptr && tiles_out != nullptr, "null operand");
-    MNT_CHECK(reinterpret_cast<uintptr_t>(tiles_out) % 16 == 0, "tiles are not 16-byte aligned");
-    build_tiles(kernel_map, num_targets, num_offsets, tiles_out, static_cast<hipStream_t>(stream_));
-  });
+  return mnt_kernel_map_tiles_batch(1, &kernel_map, &num_targets, &num_offsets, &tiles_out, stream_);
 }

@@ -27,7 +27,11 @@ from minuet_amd.utils.helpers import as_tuple, generate_kernel_offsets
 __all__ = ["SparseConv", "SparseConv3d", "KernelMapCache"]
 
 _MOST_ROWS = (1 << 63) - 1
-_MOST_TILE_ENTRIES = 1 << 29            # (tiles of 2 GiB)
+# What the tiles of a map have to save a pass, over what making them alone takes,
+# for the next pass to make them with all others: for a map that had none, and
+# to go on (so that a size that wavers does not change the plan every time).
+# Five maps take 49 us together and 137 one by one.
+_TILES_PAY, _TILES_STAY = 0.75, 0.5
 _TRANSPOSED_FIRST = ("Layer must transpose=True must have its corresponding non-transposed layer "
                      "before its execution")
 
@@ -65,7 +69,9 @@ class KernelMapCache(object):
     saved twice what making them takes; the first wide layer (rows of more than
     128 bytes) over some thousand targets makes them at once.  Otherwise
     that is the second of a 64 -> 64 layer over a
-    million voxels under 5x5x5, the fifth over 200 000 under 3x3x3.  That call
+    million voxels under 5x5x5, the fourth over 200 000 under 3x3x3, and a pass
+    that is planned makes those of all maps together where the pass before it
+    would have saved most of what they take.  That call
     takes 40 to 340 us longer on the device, the later ones about half the time
     of the first; results are the same bit for bit.  Tiles take about as much
     device memory as the dense map (at most 2 GiB a map; none where that much is
@@ -145,6 +151,7 @@ class KernelMapCache(object):
             for entry, request in self._built.entries:
                 if entry.used:                   # a layer that never came through Python
                     self._note_fast(request)
+            self._note_tiles(self._built)
             self._built = None
         requests, self._requests = self._requests, dict()
         if self._lookahead or not requests or not self._coordinates_cache:
@@ -153,7 +160,7 @@ class KernelMapCache(object):
         stride, (coordinates, _, batch_dims) = next(iter(self._coordinates_cache.items()))
         index_dtype = coordinates.dtype if batch_dims is None else batch_dims.dtype
         if (plan is not None and plan.stride == stride and plan.index_dtype == index_dtype
-                and len(plan.requests) == len(requests) and all(entry in requests for entry in plan.requests)):
+                and plan.is_for(requests)):
             return
         from minuet_amd.nn.passplan import PassPlan
         try:
@@ -178,6 +185,15 @@ class KernelMapCache(object):
             self._requests.setdefault(("dense", key))
             self._requests.setdefault(("tables", key, not self._disable_reordering))
         self._requests.setdefault(request)
+
+    def _note_tiles(self, built):
+        """Asks for the tiles of the maps whose layers would have saved enough by them."""
+        saved = {}
+        for entry, (_, _, _, _, key, transposed) in built.entries:
+            saved[key, transposed] = saved.get((key, transposed), 0.0) + entry.tiles_saved
+        for at, share in saved.items():
+            if share >= (_TILES_STAY if at in built.plan.tiles else _TILES_PAY):
+                self._requests.setdefault(("tiles", *at))
 
     def _open_pass(self, coordinates, stride, batch_dims):
         """First request of a pass: with a plan of the last one, builds everything on it."""
@@ -428,10 +444,14 @@ class KernelMapCache(object):
                              transposed)[0], "tiles", transposed)
         stream = torch.cuda.current_stream(dense.device).cuda_stream
         entry = self._offset_groups_cache.get(key)
+        if not entry and self._built is not None:
+            tiles = self._built.tiles_of(key[0], transposed, dense)
+            if tiles is not None:
+                entry = self._offset_groups_cache[key] = (tiles, self._built.stream)
         if not entry:                        # (a wider layer of the same map may want them)
             entry = False
             offsets, targets = dense.shape
-            if (dense.is_contiguous() and offsets * targets <= _MOST_TILE_ENTRIES
+            if (dense.is_contiguous() and offsets * targets <= _C.MOST_TILE_ENTRIES
                     and _C.kernel_map_tiles_worth_making(targets, offsets, in_channels, out_channels, dtype)):
                 try:
                     entry = (_C.kernel_map_tiles(dense), stream)

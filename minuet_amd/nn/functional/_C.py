@@ -106,6 +106,7 @@ SIGNATURES = {
     "mnt_pack_weights": (_int, [_vp, _i64, _i64, _i64, _int, _vp, _vp]),
     "mnt_kernel_map_tiles_size": (_int, [_i64, _i64, ctypes.POINTER(_i64)]),
     "mnt_kernel_map_tiles": (_int, [_vp, _i64, _i64, _vp, _vp]),
+    "mnt_kernel_map_tiles_batch": (_int, [_i64, _vp, _vp, _vp, _vp, _vp]),
     "mnt_kernel_map_tiles_share": (ctypes.c_double, [_i64, _i64, _i64, _i64, _int]),
     "mnt_pack_weights_in_lanes": (_int, [_vp, _i64, _i64, _i64, _vp, _vp]),
     "mnt_sparse_convolution_forward_in_lanes": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _vp, _vp, _vp,
@@ -1545,6 +1546,9 @@ def sparse_convolution_forward_implicit(sources: torch.Tensor, weights: torch.Te
     return out
 
 
+MOST_TILE_ENTRIES = 1 << 29                      # (offset, target) pairs of a map with tiles: 2 GiB of them
+
+
 def streamed_forward_supported(num_offsets: int, num_source_features: int, num_target_features: int,
                                dtype: torch.dtype) -> bool:
     """Shapes that ``sparse_convolution_forward_implicit`` streams through LDS."""
@@ -1559,6 +1563,24 @@ def kernel_map_tiles_worth_making(num_targets: int, num_offsets: int, num_source
     """Whether a layer of this shape makes the tiles of its map at its first call."""
     return load_library().mnt_kernel_map_tiles_share(num_targets, num_offsets, num_source_features, num_target_features,
                                                      _float_code(dtype, "kernel_map_tiles_worth_making")) >= 2.0
+
+
+def kernel_maps_tiles(kernel_maps, device: torch.device) -> list:
+    """:func:`kernel_map_tiles` of several dense maps, given as ``(address,
+    num_targets, num_offsets)`` each, in one set of launches."""
+    library = load_library()
+    count = len(kernel_maps)
+    size = _i64()
+    out = []
+    for _, targets, offsets in kernel_maps:
+        _check(library.mnt_kernel_map_tiles_size(targets, offsets, ctypes.byref(size)))
+        out.append(torch.empty(size.value, dtype=torch.int32, device=device))
+    columns = list(zip(*kernel_maps)) or [(), (), ()]
+    with _on(device):
+        _check(library.mnt_kernel_map_tiles_batch(
+            count, (_vp * count)(*columns[0]), (_i64 * count)(*columns[1]), (_i64 * count)(*columns[2]),
+            (_vp * count)(*(t.data_ptr() for t in out)), _stream(device)))
+    return out
 
 
 def kernel_map_tiles(kernel_map: torch.Tensor) -> torch.Tensor:

@@ -29,7 +29,9 @@ class PassPlan:
     ``requests``: ``("coords", source_stride, target_stride)``, ``("dense", key)``,
     ``("invert", key)``, ``("groups", key)``, ``("tables", key, reorder)`` with
     ``key`` the cache's ``(source_stride, target_stride, kernel_size, dilation)``,
-    and ``("fast", shape_id, in_stride, kind, key, transposed)`` for the layers
+    ``("tiles", key, transposed)`` where the layers would have saved more by the
+    tiles of the map (or its inverse) than making them takes, and
+    ``("fast", shape_id, in_stride, kind, key, transposed)`` for the layers
     that ran through the extension module.  Raises ``ValueError`` when they
     cannot be built from a cloud of stride ``stride``."""
 
@@ -91,6 +93,9 @@ class PassPlan:
             if item.want & _TABLES:
                 self.host_at[key] = self.host_words
                 self.host_words += 2 * offsets.shape[0]
+        # (the maps' tiles follow them in launches of their own, one set for all)
+        self.tiles = [(entry[1], entry[2]) for entry in self.requests if entry[0] == "tiles" and entry[1] in self.map_of
+                      and (not entry[2] or wants.get(entry[1], 0) & _INVERSE)]
         self.fast = [entry for entry in self.requests if entry[0] == "fast" and self._serves(entry)]
 
     def _serves(self, entry) -> bool:
@@ -119,6 +124,10 @@ class PassPlan:
         store = torch.empty(max(size, 256), dtype=torch.uint8, device=coordinates.device)
         _C.pass_build(coordinates, batch_dims, self.levels, self.maps, store)
         return BuiltPass(self, coordinates, batch_dims, bounds, store, hosts)
+
+    def is_for(self, requests) -> bool:
+        """Whether this is the plan of just these requests."""
+        return len(self.requests) == len(requests) and all(entry in requests for entry in self.requests)
 
     # pair lists get room for their worst case (every (offset, target) pair a hit)
     def _check_memory(self, rows: int) -> bool:
@@ -156,6 +165,27 @@ class BuiltPass:
         self.shape = {key: (plan.maps[i].num_offsets, plan.maps[i].num_sources, plan.maps[i].num_targets)
                       for key, i in plan.map_of.items()}
         self.entries = []                # (extension's entry, the request it stands for)
+        self.tiles = self._make_tiles()  # (key, transposed) -> tiles, made by the stream current now
+        self.stream = torch.cuda.current_stream(device).cuda_stream
+
+    def _make_tiles(self) -> dict:
+        maps = {}
+        for key, transposed in self.plan.tiles:
+            offsets, sources, targets = self.shape[key]
+            at, rows = self.at[key][1 if transposed else 0], sources if transposed else targets
+            if at >= 0 and 0 < rows and offsets * rows <= _C.MOST_TILE_ENTRIES:
+                maps[key, transposed] = (self.base + at, rows, offsets)
+        try:
+            return dict(zip(maps, _C.kernel_maps_tiles(list(maps.values()), self.device))) if maps else {}
+        except torch.OutOfMemoryError:   # the layers run without
+            return {}
+
+    def tiles_of(self, key, transposed: bool, dense: torch.Tensor) -> Optional[torch.Tensor]:
+        """The tiles made of the map ``dense``, if it is this pass's."""
+        tiles = self.tiles.get((key, transposed))
+        if tiles is None or dense.data_ptr() != self.base + self.at[key][1 if transposed else 0]:
+            return None
+        return tiles
 
     def _from(self, key, coordinates) -> bool:
         """Whether the map ``key`` was built from this very tensor of source coordinates."""
@@ -236,6 +266,7 @@ class BuiltPass:
                 batch_dims = None
             entry = host.MapEntry(getattr(host, kind), coordinates, stride, batch_dims, owners, index, 0,
                                   targets if transposed else sources, sources if transposed else targets, pointers,
-                                  self.coordinates[source][0].data_ptr())
+                                  self.coordinates[source][0].data_ptr(),
+                                  self.tiles.get((key, transposed)) if kind == "IMPLICIT" else None)
             fast_maps.setdefault(shape_id, {})[in_stride] = entry
             self.entries.append((entry, request))

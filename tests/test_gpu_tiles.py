@@ -256,3 +256,55 @@ def test_every_target_has_one_place(targets):
     for w in range(0, windows, max(1, windows // 5)):
         mine = counts[owner == w]
         assert mine.equal(mine.sort(descending=True).values)
+
+
+def test_planned_passes_make_the_tiles_of_all_maps_together():
+    """From the pass after the first planned one on: the same rows, from tiles that
+    are there before the first layer; a pass over a cloud too small for them has none."""
+    coordinates, gen = scattered_cloud()
+    torch.manual_seed(0)
+    layers = [minuet.nn.SparseConv3d(64, 64, 3, dtype=torch.float16, device=DEVICE) for _ in range(5)]
+    layers += [minuet.nn.SparseConv3d(64, 64, 2, stride=2, dtype=torch.float16, device=DEVICE)]
+    net = torch.nn.Sequential(*layers)
+    cache = minuet.nn.KernelMapCache(3, torch.int32, DEVICE)
+    minuet.set_kernel_map_cache(net, cache)
+    features = torch.randn(100000, 64, generator=gen, device=DEVICE).half()
+
+    def run(rows):
+        cache.reset()
+        out = net(minuet.SparseTensor(features[:rows], coordinates[:rows].contiguous())).F
+        return out, len(cache._built.tiles) if cache._built is not None else -1
+
+    with torch.no_grad():
+        first, _ = run(100000)
+        made = []
+        for _ in range(4):
+            again, tiles = run(100000)
+            made.append(tiles)
+            assert torch.equal(again, first)
+        assert made[0] <= 0 < made[-1]
+        small = [run(500)[0] for _ in range(4)]
+        assert cache._built.tiles == {} and all(torch.equal(s, small[0]) for s in small)
+        again, _ = run(100000)
+        assert torch.equal(again, first)
+
+
+@pytest.mark.parametrize("count", [1, 8, 9])
+def test_tiles_of_several_maps_at_once(count):
+    """One set of launches, and two; maps of up to 32 offsets and of more; windows
+    of one, two and four rounds of a workgroup."""
+    maps = [random_map(targets, 700, offsets, 0.3, targets + offsets).cuda()
+            for targets, offsets in ((9000, 27), (300, 27), (4100, 8), (130, 40), (40000, 27), (70, 125), (1, 2),
+                                     (20000, 27), (1000, 33))[:count]]
+    together = _C.kernel_maps_tiles([(m.data_ptr(), m.shape[1], m.shape[0]) for m in maps], torch.device(DEVICE))
+    for dense, tiles in zip(maps, together):
+        alone = _C.kernel_map_tiles(dense)
+        x, w = operands_of(dense)
+        assert _C.sparse_convolution_forward_tiled(x, w, tiles, dense.shape[1], F.pack_weights(w)).equal(
+            _C.sparse_convolution_forward_tiled(x, w, alone, dense.shape[1], F.pack_weights(w)))
+
+
+def operands_of(dense):
+    gen = torch.Generator(device=DEVICE).manual_seed(1)
+    return (torch.randn(700, 32, generator=gen, device=DEVICE).half(),
+            torch.randn(dense.shape[0], 32, 32, generator=gen, device=DEVICE).half())
