@@ -451,10 +451,11 @@ void tiled_forward(const T *sources, const T *packed, const int *kernel_map, con
   const int y = static_cast<int>(div_ceil(cols, nb));
   // Two sets of wavefronts up to a workgroup per compute unit.
   const bool two = !tiled && filled * y <= cus && O * s.chunks > 2;
-  // From 82 000 targets on lanes load together (100 000: 21.8 against 25.0 us,
-  // 70 000: even); tiles of large kernels have more stages to hide the latency
-  // behind and gain from a quarter of a million targets on only.
-  const bool quads = nb <= 2 && 2 * filled >= (O <= 32 ? 5 : 16) * cus;
+  // Lanes load together (64 -> 64 channels, 100 000 targets 18.4 against 19.3 us,
+  // 59 000 of a LiDAR level 17.7 and 22.5, though 70 000 of a room 17.9 and 16.8);
+  // tiles of large kernels have more stages to hide the latency behind and gain
+  // from a quarter of a million targets on only.
+  const bool quads = nb <= 2 && (O <= 32 || 2 * filled >= 16 * cus);
   const dim3 grid(static_cast<unsigned>(tiled ? l.tiles : filled), static_cast<unsigned>(y));
 #define MNT_TILED(NB, KS, TILED, PAIRED, WHOLE, QUADS, GROUPS)                                              \
   tiled_forward_kernel<T, NB, KS, TILED, PAIRED, WHOLE, QUADS, GROUPS><<<grid, 256 * GROUPS, 0, stream>>>(  \
