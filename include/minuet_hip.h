@@ -619,6 +619,20 @@ int mnt_sparse_convolution_forward_in_lanes(const float *sources, const float *p
 int mnt_sparse_convolution_streamed(int64_t num_targets, int64_t num_offsets, int64_t num_source_features,
                                     int64_t num_target_features, int float_dtype);
 
+/* mnt_sparse_convolution_forward_implicit for 16-bit features and kernel maps
+ * in which a target has one source at most, those of transposed layers whose
+ * kernel is their stride (others give the same results, slowly); the weights
+ * packed (mnt_pack_weights).  mnt_sparse_convolution_single: 1 for the shapes it
+ * takes, kernels of 8 offsets and rows of 144 to 512 bytes. */
+int mnt_sparse_convolution_single(int64_t num_offsets, int64_t num_source_features, int64_t num_target_features,
+                                  int float_dtype);
+int mnt_sparse_convolution_forward_single(const void *sources, const void *packed_weights, const int32_t *kernel_map,
+                                          int64_t num_sources, int64_t num_targets, int64_t num_offsets,
+                                          int64_t num_source_features, int64_t num_target_features, int float_dtype,
+                                          const float *channel_scale, const float *channel_shift,
+                                          const void *residual, int activation, float negative_slope, void *out,
+                                          void *stream);
+
 /* mnt_sparse_convolution_forward_implicit for 16-bit features from the tiles of
  * the kernel map; the weights packed (mnt_pack_weights), no narrow rows. */
 int mnt_sparse_convolution_forward_tiled(const void *sources, const void *packed_weights, const int32_t *tiles,

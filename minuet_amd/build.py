@@ -12,7 +12,7 @@ CSRC = os.path.join(_HERE, "csrc")
 LIB_DIR = os.path.join(_HERE, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libminuet_hip.so")
 HOST_PATH = os.path.join(LIB_DIR, "minuet_host.so")
-SOURCES = ["runtime.hip", "sort.hip", "unique.hip", "points.hip", "query.hip", "pass.hip", "conv.hip", "implicit.hip", "compact.hip", "tiles.hip", "tiled_half.hip", "tiled_bf16.hip", "streamed_half.hip", "streamed_bf16.hip", "lookahead.hip"]
+SOURCES = ["runtime.hip", "sort.hip", "unique.hip", "points.hip", "query.hip", "pass.hip", "conv.hip", "implicit.hip", "compact.hip", "tiles.hip", "tiled_half.hip", "tiled_bf16.hip", "streamed_half.hip", "streamed_bf16.hip", "single.hip", "lookahead.hip"]
 ARCH = "gfx950"
 FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC",

@@ -58,6 +58,7 @@ GroupsFn g_groups = nullptr;
 TablesFn g_tables = nullptr;
 TiledFn g_tiled = nullptr;
 LanesFn g_lanes = nullptr;
+TiledFn g_single = nullptr;
 TilesFn g_tiles = nullptr;
 TilesSizeFn g_tiles_size = nullptr;
 TilesShareFn g_tiles_share = nullptr;
@@ -301,7 +302,9 @@ void layer_dealloc(PyObject *self) {
 
 PyTypeObject LayerType = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
-// Layer(module, kind, weights, packed, shape_id, shortcut, rows_from, rows_to, other)
+// Layer(module, kind, weights, packed, shape_id, shortcut, rows_from, rows_to, other);
+// shortcut: of kind TABLES whether the centre offset may take one, of kind
+// IMPLICIT whether a target of the map has one source
 PyObject *layer_new(PyTypeObject *type, PyObject *args, PyObject *) {
   HANDLE_TH_ERRORS
   PyObject *module, *weights, *packed, *shape_id;
@@ -576,6 +579,12 @@ PyObject *run_layer(Layer *l, PyObject *module_dict, PyObject *inputs, const Epi
                          out.mutable_data_ptr(), stream);
         break;
       }
+      if (l->shortcut != 0) {                              // a target has one source
+        status = g_single(source, packed_at, static_cast<const int32_t *>(map->at[0]), S, T, l->num_offsets,
+                          l->in_channels, l->out_channels, l->float_code, scale_at, shift_at, data(residual),
+                          ep.activation, ep.slope, out.mutable_data_ptr(), stream);
+        break;
+      }
       if (const at::Tensor *tiles = tiles_of(map, l, T, kernel.device(), current)) {
         status = g_tiled(source, packed_at, static_cast<const int32_t *>(tiles->const_data_ptr()), S, T,
                          l->num_offsets, l->in_channels, l->out_channels, l->float_code, scale_at, shift_at,
@@ -822,6 +831,7 @@ PyObject *py_bind(PyObject *, PyObject *args) {
   g_tables = reinterpret_cast<TablesFn>(address("mnt_sparse_convolution_forward_fused"));
   g_tiled = reinterpret_cast<TiledFn>(address("mnt_sparse_convolution_forward_tiled"));
   g_lanes = reinterpret_cast<LanesFn>(address("mnt_sparse_convolution_forward_in_lanes"));
+  g_single = reinterpret_cast<TiledFn>(address("mnt_sparse_convolution_forward_single"));
   g_tiles = reinterpret_cast<TilesFn>(address("mnt_kernel_map_tiles"));
   g_tiles_size = reinterpret_cast<TilesSizeFn>(address("mnt_kernel_map_tiles_size"));
   g_tiles_share = reinterpret_cast<TilesShareFn>(address("mnt_kernel_map_tiles_share"));

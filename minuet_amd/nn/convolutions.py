@@ -889,6 +889,13 @@ class SparseConv(Module):
         shape = (self.kernel.shape[0], self.in_channels + pad, self.out_channels, features.dtype)
         return F.prefers_implicit(*shape) or F.prefers_streamed(*shape)
 
+    def _has_single_sources(self, features: torch.Tensor) -> bool:
+        """Whether a target of this layer has one source, and the kernel for that
+        takes the layer: the transposed layers whose kernel is their stride."""
+        return (self.transposed and self.kernel_size == self.stride and all(d == 1 for d in self.dilation)
+                and _C.single_forward_supported(self.kernel.shape[0], features.shape[1], self.out_channels,
+                                                features.dtype))
+
     def _takes_offset_groups(self, features: torch.Tensor) -> bool:
         """Whether this call multiplies its offsets three at a time (the
         ``offset_groups`` dataflow): forced by the tunable ``dataflow``, or, under
@@ -1016,10 +1023,13 @@ class SparseConv(Module):
                     sources = torch.nn.functional.pad(sources, (0, pad))
                 weights, packed = self._packed_kernel(pad) if not hits else self._lane_kernel()
                 tiles = None
-                if packed is not None and not hits and F.prefers_streamed(volume, sources.shape[1], self.out_channels, sources.dtype):
+                single = packed is not None and self._has_single_sources(sources)
+                if packed is not None and not hits and not single and F.prefers_streamed(volume, sources.shape[1], self.out_channels, sources.dtype):
                     tiles = cache.get_tiles(dense, sources.shape[1], self.out_channels, sources.dtype, inputs.C,
                                             inputs.stride, stride, self.kernel_size, self.dilation, self.transposed)
-                if tiles is not None:
+                if single:
+                    features = _C.sparse_convolution_forward_single(sources, weights, dense, packed, epilogue=epilogue)
+                elif tiles is not None:
                     features = _C.sparse_convolution_forward_tiled(sources, weights, tiles, dense.shape[1], packed,
                                                                    epilogue=epilogue)
                 else:
@@ -1027,7 +1037,7 @@ class SparseConv(Module):
                                                                       epilogue=epilogue,
                                                                       packed_weights=packed)
                 if not pad and dense.is_contiguous():
-                    made = ("IMPLICIT", weights, packed, (dense.data_ptr(),), dense, 0, tiles)
+                    made = ("IMPLICIT", weights, packed, (dense.data_ptr(),), dense, 0, tiles, single)
             else:
                 features, made = self._forward_tables(cache, map_args, sources, epilogue)
         if bias is not None:
@@ -1045,7 +1055,7 @@ class SparseConv(Module):
         stays with the new one: each cloud gets the kernel that a fresh cache
         would give it, whatever came before."""
         name, weights, packed, pointers, owners, index_code = made[:6]
-        tiles = made[6] if len(made) > 6 else None
+        tiles, single = made[6:] if len(made) > 6 else (None, False)
         host = _C.load_host()
         if host is None:
             return
@@ -1063,8 +1073,9 @@ class SparseConv(Module):
         if not weights.is_contiguous() or parameters.get("kernel") is None or "bias" not in parameters:
             return                                  # (a pruned or parametrised kernel is made anew from others)
         # (past Module.__setattr__, which takes longer than all of the rest)
-        self.__dict__["_fast"] = host.Layer(self, kind, weights, packed, shape_id, 1 if name == "TABLES" and
-                                            self._allow_shortcut_matmul else 0, *(rows and (*rows, self._fast)))
+        shortcut = single or (name == "TABLES" and self._allow_shortcut_matmul)
+        self.__dict__["_fast"] = host.Layer(self, kind, weights, packed, shape_id, 1 if shortcut else 0,
+                                            *(rows and (*rows, self._fast)))
 
     def _forward_tables(self, cache, map_args, sources, epilogue):
         """Gather -> GEMM -> Scatter through the rank tables (the reference's

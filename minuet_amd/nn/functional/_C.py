@@ -108,6 +108,9 @@ SIGNATURES = {
     "mnt_kernel_map_tiles": (_int, [_vp, _i64, _i64, _vp, _vp]),
     "mnt_kernel_map_tiles_batch": (_int, [_i64, _vp, _vp, _vp, _vp, _vp]),
     "mnt_kernel_map_tiles_share": (ctypes.c_double, [_i64, _i64, _i64, _i64, _int]),
+    "mnt_sparse_convolution_single": (_int, [_i64, _i64, _i64, _int]),
+    "mnt_sparse_convolution_forward_single": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _vp, _vp, _vp,
+                                                     _int, ctypes.c_float, _vp, _vp]),
     "mnt_pack_weights_in_lanes": (_int, [_vp, _i64, _i64, _i64, _vp, _vp]),
     "mnt_sparse_convolution_forward_in_lanes": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _vp, _vp, _vp,
                                                        _int, ctypes.c_float, _vp, _vp]),
@@ -194,8 +197,8 @@ def _bound_host():
     spec.loader.exec_module(module)
     names = ("mnt_sparse_convolution_forward_implicit", "mnt_sparse_convolution_forward_groups",
              "mnt_sparse_convolution_forward_fused", "mnt_sparse_convolution_forward_tiled", "mnt_kernel_map_tiles",
-             "mnt_sparse_convolution_forward_in_lanes", "mnt_kernel_map_tiles_size", "mnt_kernel_map_tiles_share",
-             "mnt_last_error")
+             "mnt_sparse_convolution_forward_in_lanes", "mnt_sparse_convolution_forward_single",
+             "mnt_kernel_map_tiles_size", "mnt_kernel_map_tiles_share", "mnt_last_error")
     hooks = tuple(getattr(torch_module, name) for name in (
         "_global_forward_hooks", "_global_forward_pre_hooks", "_global_backward_hooks",
         "_global_backward_pre_hooks"))
@@ -1556,6 +1559,45 @@ def streamed_forward_supported(num_offsets: int, num_source_features: int, num_t
         return False
     return bool(load_library().mnt_sparse_convolution_streamed(
         0, num_offsets, num_source_features, num_target_features, _float_code(dtype, "streamed_forward_supported")))
+
+
+def single_forward_supported(num_offsets: int, num_source_features: int, num_target_features: int,
+                             dtype: torch.dtype) -> bool:
+    """Shapes that ``sparse_convolution_forward_single`` takes."""
+    if dtype not in (torch.float16, torch.bfloat16):
+        return False
+    return bool(load_library().mnt_sparse_convolution_single(
+        num_offsets, num_source_features, num_target_features, _float_code(dtype, "single_forward_supported")))
+
+
+def sparse_convolution_forward_single(sources: torch.Tensor, weights: torch.Tensor, kernel_map: torch.Tensor,
+                                      packed_weights: torch.Tensor, epilogue: Optional[Epilogue] = None) -> torch.Tensor:
+    """``sparse_convolution_forward_implicit`` for a dense map whose targets have
+    one source at most (a transposed layer whose kernel is its stride)."""
+    _ensure_ndim("sources", sources, 2)
+    _ensure_ndim("weights", weights, 3)
+    _ensure_ndim("kernel_map", kernel_map, 2)
+    _ensure_dim("kernel_map", kernel_map, 0, weights.shape[0])
+    _ensure_dim("sources", sources, 1, weights.shape[1])
+    device = _common_device([sources, weights, kernel_map])
+    if kernel_map.dtype != torch.int32 or sources.dtype != weights.dtype:
+        _fail("the single-source forward expects an int32 kernel map and one feature type")
+    O, K, N = weights.shape
+    if not single_forward_supported(O, K, N, weights.dtype):
+        _fail("Unsupported shape for the single-source forward")
+    _check_packed(packed_weights, weights)
+    sources, kernel_map = sources.contiguous(), kernel_map.contiguous()
+    if sources.data_ptr() % 16:
+        sources = sources.clone()
+    S, T = sources.shape[0], kernel_map.shape[1]
+    out = torch.empty((T, N), dtype=weights.dtype, device=device)
+    ep = Epilogue() if epilogue is None else epilogue.checked(T, N, weights.dtype, device)
+    with _on(device):
+        _check(load_library().mnt_sparse_convolution_forward_single(
+            _ptr(sources), _ptr(packed_weights), _ptr(kernel_map), S, T, O, K, N,
+            _float_code(weights.dtype, "sparse_convolution_forward_single"), _ptr(ep.scale), _ptr(ep.shift),
+            _ptr(ep.residual), ACTIVATION_CODES[ep.activation], float(ep.negative_slope), _ptr(out), _stream(device)))
+    return out
 
 
 def kernel_map_tiles_worth_making(num_targets: int, num_offsets: int, num_source_features: int,
