@@ -525,6 +525,8 @@ class KernelMapCache(object):
                 self._dense_maps_cache[key] = (kernel_map.dense, kernel_map.num_sources)
                 self._kernel_maps_cache[key] = kernel_map
                 return kernel_map
+            if key not in self._dense_maps_cache:    # (no layer has asked Python for it in this pass)
+                self._take_dense(key, source_coordinates if not transposed else self._built.coordinates[key[0]][0])
         entry = self._dense_maps_cache.get(key)
         if entry is None and self._lookahead:
             # the worker builds the two halves as two items: take the dense map first

@@ -159,3 +159,24 @@ def test_tables_wait_for_their_own_flag():
         got = built.tables(key, cloud, True)
         assert np.array_equal(got.sizes_host, expected["sizes_host"])
         assert np.array_equal(got.order_host, expected["order_host"])
+
+
+def test_transposed_layer_changes_its_dataflow_in_a_planned_pass():
+    """Its tables are not on the pass's list, and the layer before it, which shares
+    the map, ran past Python: they come from the map that was built."""
+    gen = torch.Generator().manual_seed(1)
+    coordinates = torch.unique(torch.randint(0, 24, (5000, 3), generator=gen, dtype=torch.int32), dim=0).cuda()
+    coordinates = coordinates[minuet.nn.functional.build_sorted_index(coordinates)]
+    down = minuet.nn.SparseConv3d(32, 64, 2, stride=2, dtype=torch.float16, device="cuda")
+    up = minuet.nn.SparseConv(3, 64, 32, 2, stride=2, transposed=True, dtype=torch.float16, device="cuda")
+    net = torch.nn.Sequential(down, up)
+    cache = minuet.nn.KernelMapCache(ndim=3, dtype=torch.int32, device="cuda")
+    minuet.set_kernel_map_cache(net, cache)
+    x = minuet.SparseTensor(torch.randn(len(coordinates), 32, generator=gen).half().cuda(), coordinates)
+    with torch.no_grad():
+        for _ in range(3):
+            first = net(x).F
+            cache.reset()
+        up.tunable_config["dataflow"] = "gather_gemm_scatter"
+        other = net(x).F
+    assert torch.allclose(first, other, rtol=4e-3, atol=4e-3)
