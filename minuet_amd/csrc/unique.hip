@@ -242,7 +242,7 @@ __global__ __launch_bounds__(1024) void bitmap_scan_kernel(unsigned *__restrict_
 }
 
 template <typename CT, typename IT>
-__global__ __launch_bounds__(kScanBlock) void bitmap_emit_kernel(
+__global__ __launch_bounds__(kEmitBlock) void bitmap_emit_kernel(
     unsigned *__restrict__ bitmap, long long words, const unsigned *__restrict__ tile_bases,
     int tiles, TargetSpec spec, CT *__restrict__ out, IT *__restrict__ batch_dims_out) {
   emit_bitmap_tile<CT, IT>(bitmap, words, static_cast<int>(blockIdx.x), tile_bases[blockIdx.x],
@@ -309,7 +309,7 @@ static void target_count_typed(const CT *coords, int64_t n, int ndim, const int6
       bitmap_scan_kernel<<<1, 1024, 0, stream>>>(tile_bases, tiles, d, arena.flag_device(2), sequence);
       check_launch("bitmap_scan_kernel");
       if (early_out != nullptr) {
-        bitmap_emit_kernel<CT, IT><<<tiles, kScanBlock, 0, stream>>>(
+        bitmap_emit_kernel<CT, IT><<<tiles, kEmitBlock, 0, stream>>>(
             bitmap, words, tile_bases, tiles, spec, early_out, batched ? early_dims_out : nullptr);
         check_launch("bitmap_emit_kernel");
         arena.zero_bitmap_words = arena.zero_bitmap_words_after;
@@ -404,7 +404,7 @@ static void target_fill_typed(CT *out, IT *batch_dims_out, hipStream_t stream) {
     char *keep = static_cast<char *>(arena.persistent(0, 0));
     const unsigned *tile_bases = reinterpret_cast<const unsigned *>(keep);
     unsigned *bitmap = reinterpret_cast<unsigned *>(keep + kBitmapBasesBytes);
-    bitmap_emit_kernel<CT, IT><<<state.tiles, kScanBlock, 0, stream>>>(
+    bitmap_emit_kernel<CT, IT><<<state.tiles, kEmitBlock, 0, stream>>>(
         bitmap, state.words, tile_bases, state.tiles, spec, out,
         p.num_batches > 0 ? batch_dims_out : nullptr);
     check_launch("bitmap_emit_kernel");

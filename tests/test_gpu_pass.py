@@ -180,3 +180,25 @@ def test_transposed_layer_changes_its_dataflow_in_a_planned_pass():
         up.tunable_config["dataflow"] = "gather_gemm_scatter"
         other = net(x).F
     assert torch.allclose(first, other, rtol=4e-3, atol=4e-3)
+
+
+@pytest.mark.parametrize("size", [(96, 64, 64), (7, 130, 66)])
+def test_levels_of_a_full_block(size):
+    """Tiles of the levels' bitmaps with more rows than their keys fit in LDS
+    together, and words of which some rows do: asked for one by one, then planned."""
+    grids = torch.meshgrid(*(torch.arange(n, dtype=torch.int32) for n in size), indexing="ij")
+    coordinates = torch.stack([g.flatten() for g in grids], 1).cuda()
+    keep = torch.rand(len(coordinates), generator=torch.Generator().manual_seed(1)) > 0.02
+    coordinates = coordinates[keep.cuda()].contiguous()
+    net = torch.nn.Sequential(minuet.nn.SparseConv3d(8, 8, 2, stride=2, dtype=torch.float16, device="cuda"),
+                              minuet.nn.SparseConv3d(8, 8, 2, stride=2, dtype=torch.float16, device="cuda"))
+    cache = minuet.nn.KernelMapCache(ndim=3, dtype=torch.int32, device="cuda")
+    minuet.set_kernel_map_cache(net, cache)
+    x = minuet.SparseTensor(torch.ones(len(coordinates), 8, device="cuda").half(), coordinates)
+    expected = torch.unique(torch.div(coordinates, 4, rounding_mode="floor") * 4, dim=0)
+    with torch.no_grad():
+        for _ in range(3):
+            out = net(x)
+            assert out.C.equal(expected)
+            assert net[0](x).C.equal(torch.unique(torch.div(coordinates, 2, rounding_mode="floor") * 2, dim=0))
+            cache.reset()
