@@ -464,7 +464,10 @@ void streamed_forward(const T *sources, const T *packed, const int *kernel_map, 
   // longest of them, so the smallest shape that fits the chip in one go, then
   // the larger ones (us, 128 -> 128 channels, 2 000 targets: 32 x 64 10.0, 64 x
   // 64 10.4; 6 850: 64 x 64 11.8, 64 x 128 14.6; 18 600 in tiles: 64 x 128 17.3,
-  // 128 x 128 22.8; 60 000 in tiles: 33.0, 25.6).
+  // 128 x 128 22.8; 60 000 in tiles: 33.0, 25.6).  The line to the largest lies
+  // higher for rows of more than two stages, whose chains are longer (128 -> 256
+  // over 18 600 in tiles 33.2, 27.0; 256 -> 256 over 20 000 of a room 40.3, 42.4,
+  // over 25 600 of a LiDAR scan even, over 30 000 54.4, 45.0).
   auto workgroups = [&](int64_t tm, int64_t tn) { return div_ceil(Tn, tm) * div_ceil(N, tn); };
 #define MNT_STREAMED(MW, NW, KW, WM, WN, CH, RING)                                                                \
   {                                                                                                               \
@@ -492,7 +495,7 @@ void streamed_forward(const T *sources, const T *packed, const int *kernel_map, 
     MNT_STREAMED_K(1, 2, 2, 2, 1, 4)
   } else if (N <= 64) {
     MNT_STREAMED_K(2, 1, 2, 2, 2, 3)
-  } else if (2 * workgroups(128, 128) < 3 * cus) {
+  } else if (20 * workgroups(128, 128) < (s.row_bytes > 256 ? 30 : 21) * cus) {
     MNT_STREAMED_K(1, 2, 2, 2, 2, 3)
   } else {
     MNT_STREAMED_K(2, 2, 1, 2, 2, 3)
