@@ -603,6 +603,8 @@ double mnt_kernel_map_tiles_share(int64_t num_targets, int64_t num_offsets, int6
  * the weight of input channel 4 * (lane / 16) + x and output channel lane % 16
  * of the block, zeros past the end.  mnt_pack_weights_in_lanes makes them of
  * [O, Cin, Cout]; the caller keeps them for as long as the weights do not change.
+ * Without a kernel map target t's source under offset o is row t * O + o: a
+ * product of rows with their O * Cin channels cut into O pieces.
  * Same reference code as mnt_sparse_convolution_forward and mnt_pack_weights. */
 int mnt_pack_weights_in_lanes(const float *weights, int64_t num_offsets, int64_t num_source_features,
                               int64_t num_target_features, float *packed_out, void *stream);

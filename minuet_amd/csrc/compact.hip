@@ -181,7 +181,9 @@ __global__ __launch_bounds__(64 * SPLIT) void compact_forward_kernel(
 #pragma unroll
     for (int j = 0; j < kCompactBatch / kAtOnce; ++j) {
       const long long o = min(first_offset + (j * kAtOnce + lane / kTargets) * SPLIT, s.num_offsets - 1);
-      index[j] = kernel_map[o * s.num_targets + min(first + lane % kTargets, s.num_targets - 1)];
+      const long long t = min(first + lane % kTargets, s.num_targets - 1);
+      // (no map: the offsets are pieces of the target's own row)
+      index[j] = kernel_map != nullptr ? kernel_map[o * s.num_targets + t] : static_cast<int>(t * s.num_offsets + o);
     }
     if (first_offset == wv) {
       float4 *const clear = reinterpret_cast<float4 *>(acc);

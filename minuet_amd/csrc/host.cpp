@@ -146,7 +146,7 @@ struct Watched {
 
 // --------------------------------------------------------------- MapEntry ----
 
-enum Kind { kImplicit = 0, kGroups = 1, kTables = 2, kPointwise = 3 };
+enum Kind { kImplicit = 0, kGroups = 1, kTables = 2, kPointwise = 3, kPieces = 4 };
 
 // One kernel map as one kind of layer reads it: the coordinates its output
 // carries and the device addresses of its tables (`keep` holds their owners).
@@ -505,11 +505,13 @@ PyObject *run_layer(Layer *l, PyObject *module_dict, PyObject *inputs, const Epi
   int64_t T = S;
   MapEntry *map = nullptr;
   const at::Tensor *identity = nullptr;
-  if (l->kind == kPointwise) {
+  if (l->kind == kPointwise || l->kind == kPieces) {
     // 1 x 1 x 1: every row is its own source
-    identity = tensor_of(look(module_dict, s__identity_map));
-    if (identity == nullptr || identity->dim() != 2 || identity->size(1) < S || identity->device() != x->device()) {
-      return none();
+    if (l->kind == kPointwise) {
+      identity = tensor_of(look(module_dict, s__identity_map));
+      if (identity == nullptr || identity->dim() != 2 || identity->size(1) < S || identity->device() != x->device()) {
+        return none();
+      }
     }
     if (batch_dims != Py_None) {
       const at::Tensor *dims = tensor_of(batch_dims);
@@ -611,6 +613,13 @@ PyObject *run_layer(Layer *l, PyObject *module_dict, PyObject *inputs, const Epi
                         scale_at, shift_at, data(residual), ep.activation, ep.slope, packed_at,
                         static_cast<const int64_t *>(map->at[5]), out.mutable_data_ptr(), stream);
       break;
+    case kPieces: {
+      // the input channels in pieces, which the wavefronts of a workgroup share
+      const int64_t pieces = THPVariable_Unpack(l->packed).size(0);
+      status = g_lanes(source, packed_at, nullptr, S * pieces, S, pieces, l->in_channels / pieces, l->out_channels,
+                       scale_at, shift_at, data(residual), ep.activation, ep.slope, out.mutable_data_ptr(), stream);
+      break;
+    }
     default:
       status = g_implicit(source, weights_at, static_cast<const int32_t *>(identity->const_data_ptr()), S, T, 1,
                           l->in_channels, l->out_channels, l->float_code, scale_at, shift_at, data(residual),
@@ -904,5 +913,6 @@ PyMODINIT_FUNC PyInit_minuet_host() {
   PyModule_AddIntConstant(module, "GROUPS", kGroups);
   PyModule_AddIntConstant(module, "TABLES", kTables);
   PyModule_AddIntConstant(module, "POINTWISE", kPointwise);
+  PyModule_AddIntConstant(module, "PIECES", kPieces);
   return module;
 }

@@ -722,7 +722,8 @@ extern "C" int mnt_sparse_convolution_forward_in_lanes(
                   reinterpret_cast<uintptr_t>(channel_shift) % 4 == 0,
               "operands are not aligned (features, out, residual, weights: 16 bytes, scale / shift: 4 bytes)");
     if (T == 0) return;
-    MNT_CHECK(out != nullptr && kernel_map != nullptr && packed_weights != nullptr, "null operand");
+    MNT_CHECK(out != nullptr && packed_weights != nullptr, "null operand");
+    MNT_CHECK(kernel_map != nullptr || S == T * O, "without a kernel map a target has a source under every offset");
     const Epilogue ep = {channel_scale, channel_shift, residual, activation, negative_slope, nullptr};
     profile_mark("enter:implicit", stream);
     compact_forward(sources, packed_weights, true, kernel_map, S, T, O, K, N, ep, out, stream);

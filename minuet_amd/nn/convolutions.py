@@ -845,12 +845,15 @@ class SparseConv(Module):
                 self._packed = (key, weights, F.pack_weights(weights), held)
         return self._packed[1], self._packed[2]
 
-    def _lane_kernel(self):
+    def _lane_kernel(self, pieces: int = 1):
         """``_packed_kernel`` of an fp32 layer that multiplies hits only, whose
         kernel reads the weights in the order of its lanes (16 x 16 x 4 instructions
         take them 1 KB at a load: 32 -> 32 channels over 200 000 voxels 55 and 50
-        us, 128 -> 64 over 2 900 27 and 21)."""
+        us, 128 -> 64 over 2 900 27 and 21).  ``pieces``: a pointwise layer's,
+        its input channels cut into that many "offsets"."""
         kernel = self.kernel
+        if pieces > 1:
+            kernel = kernel.view(pieces, self.in_channels // pieces, self.out_channels)
         if (torch.is_grad_enabled() and kernel.requires_grad) or not _C.lane_weights_supported(kernel):
             return self._packed_kernel()
         key = (kernel.data_ptr(), kernel._version, kernel.dtype, kernel.device)
@@ -917,9 +920,21 @@ class SparseConv(Module):
         """1x1x1 kernel, stride 1: a plain ``features @ W`` (reference:
         convolutions.py:452-455).  Where the single-kernel forward takes the
         shape it runs there, as one offset whose kernel map is the identity,
-        so that an epilogue costs no extra pass; otherwise ``torch.mm``."""
+        so that an epilogue costs no extra pass, or, an fp32 layer over few rows,
+        as several offsets, the pieces of its input channels, which the
+        wavefronts of a workgroup share; otherwise ``torch.mm``.  Returns the
+        features, what ``_keep_fast`` takes and its rows."""
         weights = self.kernel.view(1, self.in_channels, self.out_channels)
         needs_grad = torch.is_grad_enabled() and (features.requires_grad or weights.requires_grad)
+        rows = ()
+        if (features.is_cuda and not needs_grad
+                and self._tunable_config.get("dataflow", "auto") == "auto" and features.dtype == weights.dtype):
+            most = F.pieces_rows_limit(self.in_channels, self.out_channels, weights.dtype)
+            rows = (most + 1, _MOST_ROWS) if most >= 0 else ()
+            if 0 < features.shape[0] <= most and features.is_contiguous():
+                whole, packed = self._lane_kernel(F.channel_pieces(self.in_channels))
+                out = _C.sparse_convolution_forward_pieces(features, packed, self.out_channels, epilogue=epilogue)
+                return out, ("PIECES", whole.view(weights.shape), packed, None, None, 0), (0, most)
         if (features.is_cuda and not needs_grad
                 and self._tunable_config.get("dataflow", "auto") not in ("gather_gemm_scatter", "list_driven")
                 and features.dtype == weights.dtype
@@ -927,17 +942,17 @@ class SparseConv(Module):
                 # measured against torch.mm plus a separate epilogue pass up to these widths;
                 # wider layers are plain library GEMM territory
                 and self.in_channels * weights.dtype.itemsize <= 512 and self.out_channels <= 128):
-            rows = features.shape[0]
+            count = features.shape[0]
             identity = self._identity_map
-            if identity is None or identity.shape[1] < rows or identity.device != features.device:
-                identity = torch.arange(rows, dtype=torch.int32, device=features.device).view(1, rows)
+            if identity is None or identity.shape[1] < count or identity.device != features.device:
+                identity = torch.arange(count, dtype=torch.int32, device=features.device).view(1, count)
                 self._identity_map = identity
             packed = self._packed_kernel()[1]
-            out = _C.sparse_convolution_forward_implicit(features, weights, identity[:, :rows],
+            out = _C.sparse_convolution_forward_implicit(features, weights, identity[:, :count],
                                                          epilogue=epilogue, packed_weights=packed)
-            return out, ("POINTWISE", weights.detach(), packed, None, None, 0)
+            return out, ("POINTWISE", weights.detach(), packed, None, None, 0), rows
         out = torch.mm(features, weights[0])
-        return out if epilogue is None else epilogue.apply(out), None
+        return out if epilogue is None else epilogue.apply(out), None, ()
 
     def forward(self, inputs: SparseTensor,
                 epilogue: Optional[F.Epilogue] = None) -> SparseTensor:
@@ -968,7 +983,7 @@ class SparseConv(Module):
         made = None                                 # (kind, weights, packed, map pointers, owners, index code)
         rows = ()                                   # from how many to how many rows that kind is the one to take
         if self.is_trivial:
-            features, made = self._pointwise(inputs.F, epilogue)
+            features, made, rows = self._pointwise(inputs.F, epilogue)
             coordinates, stride, batch_dims = inputs.C, inputs.stride, inputs.batch_dims
         else:
             cache = self._kernel_map_cache

@@ -1552,6 +1552,33 @@ def sparse_convolution_forward_implicit(sources: torch.Tensor, weights: torch.Te
 MOST_TILE_ENTRIES = 1 << 29                      # (offset, target) pairs of a map with tiles: 2 GiB of them
 
 
+def sparse_convolution_forward_pieces(sources: torch.Tensor, packed_weights: torch.Tensor, num_target_features: int,
+                                      epilogue: Optional[Epilogue] = None) -> torch.Tensor:
+    """fp32 ``sources [N, C_in] @ weights [C_in, C_out]`` for few rows, the weights as
+    :func:`pack_weights_in_lanes` of ``weights.view(pieces, C_in / pieces, C_out)``."""
+    _ensure_ndim("sources", sources, 2)
+    _ensure_ndim("packed_weights", packed_weights, 5)
+    device = _common_device([sources, packed_weights])
+    if sources.dtype != torch.float32 or packed_weights.dtype != torch.float32 or not packed_weights.is_contiguous():
+        _fail("the forward in pieces expects contiguous fp32 tensors")
+    rows, channels = sources.shape
+    pieces, blocks, steps = packed_weights.shape[:3]
+    N = num_target_features
+    if (channels % pieces or -(-(channels // pieces) // 16) != steps or tuple(packed_weights.shape[3:]) != (64, 4)
+            or -(-N // 16) != blocks):
+        _fail("packed_weights does not belong to these sources")
+    if not sources.is_contiguous() or sources.data_ptr() % 16:
+        sources = sources.contiguous().clone()
+    out = torch.empty((rows, N), dtype=sources.dtype, device=device)
+    ep = Epilogue() if epilogue is None else epilogue.checked(rows, N, sources.dtype, device)
+    with _on(device):
+        _check(load_library().mnt_sparse_convolution_forward_in_lanes(
+            _ptr(sources), _ptr(packed_weights), None, rows * pieces, rows, pieces, channels // pieces, N,
+            _ptr(ep.scale), _ptr(ep.shift), _ptr(ep.residual), ACTIVATION_CODES[ep.activation],
+            float(ep.negative_slope), _ptr(out), _stream(device)))
+    return out
+
+
 def streamed_forward_supported(num_offsets: int, num_source_features: int, num_target_features: int,
                                dtype: torch.dtype) -> bool:
     """Shapes that ``sparse_convolution_forward_implicit`` streams through LDS."""

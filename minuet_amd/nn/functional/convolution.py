@@ -9,7 +9,8 @@ from ..kernel_map import KernelMap
 
 __all__ = ["cuda_time_gather", "cuda_time_scatter", "sparse_convolution_forward",
            "cuda_time_gemm", "set_gemm_parallel_level", "Epilogue", "pack_weights",
-           "prefers_implicit", "prefers_streamed", "prefers_hits", "hits_rows_limit"]
+           "prefers_implicit", "prefers_streamed", "prefers_hits", "hits_rows_limit",
+           "pieces_rows_limit", "channel_pieces"]
 
 pack_weights = _C.pack_weights
 
@@ -91,6 +92,27 @@ def hits_rows_limit(num_offsets: int, num_source_features: int, num_target_featu
     if work <= 1024:
         return most
     return min(most, min(110_000_000, 2_100_000_000 // num_offsets) // work)
+
+
+def channel_pieces(num_source_features: int) -> int:
+    """Into how many pieces an fp32 pointwise layer over few rows cuts its input
+    channels: of 32, or of 16 where there are fewer than four of 32."""
+    return num_source_features // (32 if num_source_features % 32 == 0 and num_source_features >= 128 else 16)
+
+
+def pieces_rows_limit(num_source_features: int, num_target_features: int, dtype: torch.dtype) -> int:
+    """The most rows over which ``dataflow="auto"`` cuts an fp32 pointwise layer into
+    pieces (-1: over none).  They let a workgroup's wavefronts share a row, and
+    every 16 rows read the weights again, so that the line lies at 200 million
+    rows x input x output channels: us against the kernel for one offset 128 -> 64
+    over 2 900 rows 4.7 / 13.0, over 12 000 7.4 / 13.2, over 30 000 12.8 / 12.5,
+    64 -> 32 over 60 000 11.9 / 12.4, 128 -> 128 over 12 000 12.4 / 18.5, over
+    30 000 22.7 / 20.3; against the library and an output pass of its own 256 ->
+    128 over 660 4.9 / 38, over 8 200 13.4 / 36."""
+    if (dtype != torch.float32 or num_source_features % 16 != 0 or num_source_features < 48
+            or not _C.implicit_forward_supported(num_source_features, num_target_features, dtype)):
+        return -1
+    return 200_000_000 // (num_source_features * num_target_features)
 
 
 def prefers_hits(num_offsets: int, num_source_features: int, num_target_features: int, dtype: torch.dtype,

@@ -78,3 +78,35 @@ def test_refuses_another_layer_s_weights():
     with pytest.raises((RuntimeError, ValueError)):
         _C.sparse_convolution_forward_implicit(x[:, :32].half(), w.half(), dense,
                                                packed_weights=_C.pack_weights_in_lanes(w))
+
+
+# one workgroup and several, rows that fill none, pieces of 16 and of 32 channels, channels that fill no block
+@pytest.mark.parametrize("rows", [1, 33, 700, 5003])
+@pytest.mark.parametrize("K, N", [(48, 32), (64, 64), (128, 20), (256, 128), (512, 36)])
+def test_pointwise_layer_in_pieces(rows, K, N):
+    gen = torch.Generator().manual_seed(rows + K)
+    x, w = torch.randn(rows, K, generator=gen), torch.randn(K, N, generator=gen) / K ** 0.5
+    residual = torch.randn(rows, N, generator=gen)
+    pieces = F.channel_pieces(K)
+    packed = _C.pack_weights_in_lanes(w.view(pieces, K // pieces, N).cuda())
+    got = _C.sparse_convolution_forward_pieces(x.cuda(), packed, N, _C.Epilogue(residual=residual.cuda())).cpu()
+    expected = x.double() @ w.double() + residual.double()
+    assert (got.double() - expected).abs().max() < 8 * 2.0 ** -24 * K ** 0.5
+    with pytest.raises((RuntimeError, ValueError)):
+        _C.sparse_convolution_forward_pieces(x.cuda(), packed, N + 16)
+
+
+def test_pointwise_layer_takes_pieces_by_its_rows():
+    conv = minuet.nn.SparseConv3d(128, 64, 1, bias=True, device="cuda")
+    most = F.pieces_rows_limit(128, 64, torch.float32)
+    x = torch.randn(most + 5, 128, device="cuda")
+    coordinates = torch.zeros(most + 5, 3, dtype=torch.int32, device="cuda")
+    coordinates[:, 2] = torch.arange(most + 5)
+    with torch.no_grad():
+        expected = (x.double() @ conv.kernel[0].double() + conv.bias.double()).float()
+        for rows in (900, 900, most, most + 1, most + 5, 37, most + 1):
+            out = conv(minuet.SparseTensor(x[:rows], coordinates[:rows]))
+            assert torch.allclose(out.F, expected[:rows], rtol=0, atol=2e-5)
+        conv.kernel.mul_(2.0)
+        out = conv(minuet.SparseTensor(x[:900], coordinates[:900]))
+        assert torch.allclose(out.F, 2 * expected[:900] - conv.bias, rtol=0, atol=4e-5)
