@@ -677,6 +677,12 @@ int mnt_upload_ints(const int64_t *values, int64_t count, int index_dtype, void 
 int mnt_global_pool(const void *features, const void *batch_dims, int64_t n, int64_t num_batches, int64_t channels,
                     int float_dtype, int index_dtype, int mean, void *out, void *stream);
 
+/* out[b, n] = rows[b] . weights[n] + bias[n] (bias nullable), a classifier's head
+ * over pooled rows: a wavefront per output, sums in fp32.  The reference leaves
+ * it to torch.nn.Linear. */
+int mnt_linear(const void *rows, const void *weights, const void *bias, int64_t num_rows, int64_t channels,
+               int64_t classes, int float_dtype, void *out, void *stream);
+
 /* ---- Map: the coordinates and kernel maps of a whole pass in one build ------ */
 
 /* A network asks for the same coordinate levels and kernel maps for every
