@@ -102,4 +102,35 @@ __device__ __forceinline__ unsigned long long pack_row(const CT *__restrict__ ro
   return key;
 }
 
+// Minimum over the wavefront of eight values per lane; lane l ends with the
+// minimum of value l & 7.  Halving exchanges: in step d a lane keeps the values
+// whose bit d is its own and sends the others away (4 + 2 + 1 shuffles), then
+// the eight lanes groups fold (3).
+template <typename CT>
+__device__ __forceinline__ CT fold_extremes(const CT (&v)[8]) {
+  const int lane = lane_id();
+  CT four[4], two[2];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {                       // bit 2
+    const CT mine = lane & 4 ? v[i + 4] : v[i];
+    const CT other = __shfl_xor(lane & 4 ? v[i] : v[i + 4], 4);
+    four[i] = other < mine ? other : mine;
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {                       // bit 1
+    const CT mine = lane & 2 ? four[i + 2] : four[i];
+    const CT other = __shfl_xor(lane & 2 ? four[i] : four[i + 2], 2);
+    two[i] = other < mine ? other : mine;
+  }
+  CT one = lane & 1 ? two[1] : two[0];
+  const CT from = __shfl_xor(lane & 1 ? two[0] : two[1], 1);
+  one = from < one ? from : one;
+#pragma unroll
+  for (int d = 8; d < kWave; d <<= 1) {
+    const CT other = __shfl_xor(one, d);
+    one = other < one ? other : one;
+  }
+  return one;
+}
+
 }  // namespace mnt

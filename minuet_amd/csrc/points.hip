@@ -2,9 +2,10 @@
 // the feature rows of a collated batch, and the global pools.  Each took five
 // to eight tensor expressions with a read-back among them; here each is one
 // library call (minuet/nn/functional/voxelize.py:11-35, pooling.py).  Measured:
-// 100 000 points to voxels 148 -> 58 us; mean pools of 8 clouds of 3 000 voxels
+// 100 000 points to voxels 148 -> 56 us; mean pools of 8 clouds of 3 000 voxels
 // 91 us of kernels and a read-back -> 8 us.
 #include <algorithm>
+#include <limits>
 
 #include "conv_device.h"
 #include "device_utils.h"
@@ -31,6 +32,64 @@ __global__ __launch_bounds__(256) void voxel_kernel(const FT *__restrict__ point
   for (int d = 1; d < MNT_MAX_NDIM; ++d) size = k == d ? static_cast<FT>(sizes.v[d]) : size;
   const FT q = points[i] / size;
   out[i] = static_cast<CT>(sizeof(FT) == 4 ? floorf(static_cast<float>(q)) : floor(static_cast<double>(q)));
+}
+
+// The same for clouds that the bucket sort takes: the launch that has the rows in
+// registers leaves their extremes too, one part a workgroup, and clears the
+// sort's counters.  Bound by latency: 4.5 us at 100 003 points, where the two
+// launches are 3.2 and 4.6 and the gap between them; the whole call is 55.8
+// against 59.7 (5 000: 49 against 53; a million, where 128 workgroups are few
+// for the points: 163 both ways).  The chain of sorting launches that waits for
+// the host only once is 49 at 100 003 points, but clouds of walls, which crowd
+// more than 4 096 rows into one of its buckets from 65 000 points on, pay for
+// it and then for this sort: 75 against 55.
+constexpr int kVoxelRows = 4;
+template <typename FT, typename CT>
+__global__ __launch_bounds__(256) void voxel_bounds_kernel(const FT *__restrict__ points, long long n, int ndim,
+                                                           VoxelSizes sizes, CT *__restrict__ out,
+                                                           long long *__restrict__ partial,
+                                                           unsigned *__restrict__ zero, int zero_count) {
+  __shared__ CT s_extreme[256 / kWave][2 * MNT_MAX_NDIM];
+  const int tid = threadIdx.x;
+  for (int i = blockIdx.x * 256 + tid; i < zero_count; i += gridDim.x * 256) zero[i] = 0u;
+  FT size[MNT_MAX_NDIM];
+#pragma unroll
+  for (int k = 0; k < MNT_MAX_NDIM; ++k) size[k] = static_cast<FT>(sizes.v[k < ndim ? k : 0]);
+  CT extreme[2 * MNT_MAX_NDIM];                  // ~v turns the order round
+#pragma unroll
+  for (int k = 0; k < 2 * MNT_MAX_NDIM; ++k) extreme[k] = std::numeric_limits<CT>::max();
+  const long long stride = static_cast<long long>(gridDim.x) * 256;
+  for (long long i0 = static_cast<long long>(blockIdx.x) * 256 + tid; i0 < n; i0 += kVoxelRows * stride) {
+    FT p[kVoxelRows][MNT_MAX_NDIM];
+#pragma unroll
+    for (int r = 0; r < kVoxelRows; ++r) {
+      const long long i = i0 + r * stride;
+#pragma unroll
+      for (int k = 0; k < MNT_MAX_NDIM; ++k) p[r][k] = points[(i < n ? i : n - 1) * ndim + (k < ndim ? k : 0)];
+    }
+#pragma unroll
+    for (int r = 0; r < kVoxelRows; ++r) {
+      const long long i = i0 + r * stride;
+#pragma unroll
+      for (int k = 0; k < MNT_MAX_NDIM; ++k) {
+        const FT q = p[r][k] / size[k];
+        const CT v = static_cast<CT>(sizeof(FT) == 4 ? floorf(static_cast<float>(q)) : floor(static_cast<double>(q)));
+        if (i < n && k < ndim) out[i * ndim + k] = v;
+        extreme[k] = v < extreme[k] ? v : extreme[k];
+        const CT turned = static_cast<CT>(~v);
+        extreme[MNT_MAX_NDIM + k] = turned < extreme[MNT_MAX_NDIM + k] ? turned : extreme[MNT_MAX_NDIM + k];
+      }
+    }
+  }
+  const CT folded = fold_extremes<CT>(extreme);
+  if (lane_id() < 2 * MNT_MAX_NDIM) s_extreme[tid / kWave][lane_id()] = folded;
+  __syncthreads();
+  if (tid < 2 * MNT_MAX_NDIM) {
+    CT v = s_extreme[0][tid];
+#pragma unroll
+    for (int w = 1; w < 256 / kWave; ++w) v = s_extreme[w][tid] < v ? s_extreme[w][tid] : v;
+    partial[static_cast<long long>(blockIdx.x) * 8 + tid] = static_cast<long long>(tid < MNT_MAX_NDIM ? v : static_cast<CT>(~v));
+  }
 }
 
 // Distinct rows of sorted rows.  Each tile counts the rows that start a run; the
@@ -149,9 +208,9 @@ __global__ __launch_bounds__(kScanBlock) void run_emit_kernel(const CT *__restri
   if (!scanned && blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) host.tell(run);
 }
 
-template <typename CT>
-static void voxelize_typed(const void *points, int64_t n, int ndim, bool wide, const VoxelSizes &sizes,
-                           CT *voxels_out, long long *reverse_out, int64_t *count_out, hipStream_t stream) {
+template <typename FT, typename CT>
+static void voxelize_typed(const FT *points, int64_t n, int ndim, const VoxelSizes &sizes, CT *voxels_out,
+                           long long *reverse_out, int64_t *count_out, hipStream_t stream) {
   Scope scope(stream);
   Arena &arena = scope.arena();
   CT *voxels = scope.alloc<CT>(static_cast<size_t>(n) * ndim);
@@ -159,17 +218,17 @@ static void voxelize_typed(const void *points, int64_t n, int ndim, bool wide, c
   int *order = scope.alloc<int>(n);
   const int tiles = static_cast<int>(div_ceil(n, kRunTile));
   unsigned *tile_sums = scope.alloc<unsigned>(static_cast<size_t>(tiles) + 1);
-  const unsigned blocks = static_cast<unsigned>(div_ceil(n * ndim, 256));
-  if (wide) {
-    voxel_kernel<double, CT><<<blocks, 256, 0, stream>>>(static_cast<const double *>(points), n * ndim, ndim, sizes, voxels);
+  const SortStart start = sort_start(n, scope);
+  if (start.parts > 0) {
+    voxel_bounds_kernel<FT, CT><<<start.parts, 256, 0, stream>>>(points, n, ndim, sizes, voxels, start.partial,
+                                                                 start.clear, start.clear_words);
+    check_launch("voxel_bounds_kernel");
   } else {
-    voxel_kernel<float, CT><<<blocks, 256, 0, stream>>>(static_cast<const float *>(points), n * ndim, ndim, sizes, voxels);
+    voxel_kernel<FT, CT><<<static_cast<unsigned>(div_ceil(n * ndim, 256)), 256, 0, stream>>>(points, n * ndim, ndim,
+                                                                                            sizes, voxels);
+    check_launch("voxel_kernel");
   }
-  check_launch("voxel_kernel");
-  if (mnt_arg_sort_coordinates(voxels, n, ndim, sizeof(CT) == 4 ? MNT_INT32 : MNT_INT64, nullptr, 1, MNT_INT32, order,
-                               sorted, nullptr, stream) != 0) {
-    throw Error{mnt_last_error()};
-  }
+  sort_started_rows(voxels, n, ndim, sizeof(CT) == 4 ? MNT_INT32 : MNT_INT64, order, sorted, start, stream);
   volatile unsigned *h = reinterpret_cast<volatile unsigned *>(static_cast<char *>(arena.pinned()) + 256);
   unsigned *d = reinterpret_cast<unsigned *>(static_cast<char *>(arena.pinned_device()) + 256);
   const unsigned long long sequence = arena.next_sequence();
@@ -407,13 +466,17 @@ extern "C" int mnt_voxelize(const void *points, int64_t n, int ndim, int wide_po
     VoxelSizes sizes;
     for (int k = 0; k < MNT_MAX_NDIM; ++k) sizes.v[k] = voxel_size[k < ndim ? k : 0];
     long long *reverse = reinterpret_cast<long long *>(reverse_out);
+#define MNT_CALL(FT, CT)                                                                                    \
+  voxelize_typed<FT, CT>(static_cast<const FT *>(points), n, ndim, sizes, static_cast<CT *>(voxels_out), reverse, \
+                         count_out, stream)
     if (coord_dtype == MNT_INT32) {
-      voxelize_typed<int32_t>(points, n, ndim, wide_points != 0, sizes, static_cast<int32_t *>(voxels_out), reverse,
-                              count_out, stream);
+      if (wide_points != 0) MNT_CALL(double, int32_t);
+      else MNT_CALL(float, int32_t);
     } else {
-      voxelize_typed<int64_t>(points, n, ndim, wide_points != 0, sizes, static_cast<int64_t *>(voxels_out), reverse,
-                              count_out, stream);
+      if (wide_points != 0) MNT_CALL(double, int64_t);
+      else MNT_CALL(float, int64_t);
     }
+#undef MNT_CALL
   });
 }
 

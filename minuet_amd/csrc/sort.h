@@ -34,6 +34,23 @@ void radix_sort_pairs(unsigned long long *&keys, unsigned *&vals, unsigned long 
                       unsigned *&vals_alt, int64_t n, int bits, unsigned *counts,
                       hipStream_t stream);
 
+// ---- the sort of rows whose own launch folds their bounds ----
+
+// What the launch that makes the rows leaves for their sort: the extremes of
+// every workgroup (`parts` of them, [parts * 8] as bounds_kernel has them) and
+// `clear_words` cleared counters.  parts == 0: the sort has no use for them.
+struct SortStart {
+  long long *partial;
+  int parts;
+  unsigned *clear;
+  int clear_words;
+};
+SortStart sort_start(int64_t n, Scope &scope);
+// The int32 permutation and the sorted rows of one batch; launches as
+// mnt_arg_sort_coordinates does, without the pass over the rows for their bounds.
+void sort_started_rows(const void *rows, int64_t n, int ndim, int coord_dtype, int32_t *indices_out, void *sorted_out,
+                       const SortStart &start, hipStream_t stream);
+
 // ---- the bucket sort as a chain of launches that never waits for the host ----
 
 struct OffsetTable;

@@ -1523,37 +1523,6 @@ struct SmallSortTell {            // where the host finds bounds and verdict (fl
   unsigned long long sequence;
 };
 
-// Minimum over the wavefront of eight values per lane; lane l ends with the
-// minimum of value l & 7.  Halving exchanges: in step d a lane keeps the values
-// whose bit d is its own and sends the others away (4 + 2 + 1 shuffles), then
-// the eight lanes groups fold (3).
-template <typename CT>
-__device__ __forceinline__ CT fold_extremes(const CT (&v)[8]) {
-  const int lane = lane_id();
-  CT four[4], two[2];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {                       // bit 2
-    const CT mine = lane & 4 ? v[i + 4] : v[i];
-    const CT other = __shfl_xor(lane & 4 ? v[i] : v[i + 4], 4);
-    four[i] = other < mine ? other : mine;
-  }
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {                       // bit 1
-    const CT mine = lane & 2 ? four[i + 2] : four[i];
-    const CT other = __shfl_xor(lane & 2 ? four[i] : four[i + 2], 2);
-    two[i] = other < mine ? other : mine;
-  }
-  CT one = lane & 1 ? two[1] : two[0];
-  const CT from = __shfl_xor(lane & 1 ? two[0] : two[1], 1);
-  one = from < one ? from : one;
-#pragma unroll
-  for (int d = 8; d < kWave; d <<= 1) {
-    const CT other = __shfl_xor(one, d);
-    one = other < one ? other : one;
-  }
-  return one;
-}
-
 template <typename CT, typename IT, bool kChain>
 __global__ __launch_bounds__(kSmallSortBlock) void small_sort_kernel(
     const CT *__restrict__ coords, const IT *__restrict__ batch_dims, int num_batches, int ndim, int n, int idx_bits,
@@ -1840,10 +1809,20 @@ void enqueue_chain_sort(const void *coords, int64_t n, int ndim, int coord_dtype
   }
 }
 
+SortStart sort_start(int64_t n, Scope &scope) {
+  SortStart start = {};
+  if (n <= kSmallSortRows || n > bucket_sort_max_rows()) return start;
+  start.parts = static_cast<int>(std::min<int64_t>(div_ceil(n, kBoundsBlock * 4), kBucketBoundsBlocks));
+  start.partial = scope.alloc<long long>(static_cast<size_t>(start.parts) * 8);
+  start.clear_words = kBucketMax + 4;
+  start.clear = scope.alloc<unsigned>(start.clear_words);
+  return start;
+}
+
 template <typename CT, typename IT>
 static void arg_sort_typed(const CT *coords, int64_t n, int ndim, const IT *batch_dims,
                            int64_t num_batches, IT *indices_out, CT *sorted_out,
-                           int64_t *bounds_host_out, hipStream_t stream) {
+                           int64_t *bounds_host_out, hipStream_t stream, const SortStart *made = nullptr) {
   Scope scope(stream);
   const bool batched = batch_dims != nullptr && num_batches > 1;
 
@@ -1883,23 +1862,26 @@ static void arg_sort_typed(const CT *coords, int64_t n, int ndim, const IT *batc
   unsigned long long *bucket_words = nullptr;
   if (try_buckets) {
     Arena &arena = scope.arena();
-    unsigned *totals = scope.alloc<unsigned>(kBucketMax + 4);
+    const SortStart start = made != nullptr ? *made : sort_start(n, scope);
+    unsigned *totals = start.clear;
     unsigned *info = totals + kBucketMax;
     bucket_starts = scope.alloc<unsigned>(kBucketMax + 1);
     unsigned *cursors = scope.alloc<unsigned>(kBucketMax);
     // a bucket of m rows makes at most m / 256 + 1 pairs
     bucket_chunks = scope.alloc<uint4>(kBucketMax + static_cast<size_t>(n / kSortBlock) + 1);
     bucket_words = scope.alloc<unsigned long long>(n);
-    const int num_partials = static_cast<int>(std::min<int64_t>(div_ceil(n, kBoundsBlock * 4), kBucketBoundsBlocks));
-    long long *partial = scope.alloc<long long>(static_cast<size_t>(num_partials) * 8);
+    const int num_partials = start.parts;
+    long long *partial = start.partial;
     long long *folded = scope.alloc<long long>(2 * MNT_MAX_NDIM);
     const unsigned long long sequence = arena.next_sequence();
     long long *host_bounds = static_cast<long long *>(arena.pinned_device());
     unsigned *host_out = reinterpret_cast<unsigned *>(static_cast<char *>(arena.pinned_device()) + kBucketHostOffset);
     const IT *dims = batched ? batch_dims : nullptr;
-    bounds_kernel<CT><<<num_partials, kBoundsBlock, 0, stream>>>(coords, n, num_partials, nullptr, 0, ndim,
-                                                                 partial, totals, kBucketMax + 4);
-    check_launch("bounds_kernel");
+    if (made == nullptr) {
+      bounds_kernel<CT><<<num_partials, kBoundsBlock, 0, stream>>>(coords, n, num_partials, nullptr, 0, ndim,
+                                                                   partial, totals, start.clear_words);
+      check_launch("bounds_kernel");
+    }
     // rows per thread of the histogram and dealing kernels: 4, or 16 for a large cloud
     const bool large = n > (int64_t(1) << 18);
     const unsigned tiles = static_cast<unsigned>(div_ceil(n, kSortBlock * (large ? 16 : 4)));
@@ -2061,6 +2043,18 @@ static void arg_sort_typed(const CT *coords, int64_t n, int ndim, const IT *batc
     perm = vals;
   }
   profile_mark("sort_radix", stream);
+}
+
+void sort_started_rows(const void *rows, int64_t n, int ndim, int coord_dtype, int32_t *indices_out, void *sorted_out,
+                       const SortStart &start, hipStream_t stream) {
+  const SortStart *made = start.parts > 0 ? &start : nullptr;
+  if (coord_dtype == MNT_INT32) {
+    arg_sort_typed<int32_t, int32_t>(static_cast<const int32_t *>(rows), n, ndim, nullptr, 1, indices_out,
+                                     static_cast<int32_t *>(sorted_out), nullptr, stream, made);
+  } else {
+    arg_sort_typed<int64_t, int32_t>(static_cast<const int64_t *>(rows), n, ndim, nullptr, 1, indices_out,
+                                     static_cast<int64_t *>(sorted_out), nullptr, stream, made);
+  }
 }
 
 }  // namespace mnt

@@ -25,6 +25,20 @@ def test_voxelize_against_numpy(n, ndim, ftype, dtype):
     np.testing.assert_array_equal(host(reverse), inverse.reshape(-1))
 
 
+@pytest.mark.parametrize("n,ndim,ftype,dtype", [(4097, 4, np.float64, torch.int64), (5121, 1, np.float32, torch.int32),
+                                                (131073, 3, np.float64, torch.int32), (140001, 2, np.float32, torch.int64)])
+def test_voxels_leave_their_bounds(n, ndim, ftype, dtype):
+    """Clouds whose voxels and bounds come of one launch: one far corner in the last
+    row, one in the first, coordinates of both signs, runs of equal points."""
+    rng = np.random.default_rng(n)
+    points = rng.integers(-40, 40, size=(n, ndim)).astype(ftype) + ftype(0.5)
+    points[-1], points[0] = 3000.5, -2999.5
+    voxels, reverse = F.voxelize(dev(points), voxel_size=1.0, dtype=dtype, return_reverse_indices=True)
+    expect, inverse = np.unique(np.floor(points).astype(np.int64), axis=0, return_inverse=True)
+    np.testing.assert_array_equal(host(voxels), expect)
+    np.testing.assert_array_equal(host(reverse), inverse.reshape(-1))
+
+
 @pytest.mark.parametrize("rows,channels", [((7,), 1), ((0, 3, 900), 6), ((5000, 1, 20000), 64), ((300, 41), 257),
                                            ((130,), 1100)])
 @pytest.mark.parametrize("kind", ["fp32", "fp16", "bf16"])
