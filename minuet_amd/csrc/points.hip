@@ -576,7 +576,7 @@ extern "C" int mnt_linear(const void *rows, const void *weights, const void *bia
   return guarded([&] {
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     MNT_CHECK(num_rows >= 0 && classes >= 1 && channels >= 1 && channels <= INT32_MAX && num_rows <= INT32_MAX &&
-                  classes <= INT32_MAX && num_rows * classes <= INT32_MAX,
+                  classes <= INT32_MAX && num_rows * classes <= INT32_MAX - 4,
               "bad shape N=%lld Cin=%lld Cout=%lld", (long long)num_rows, (long long)channels, (long long)classes);
     if (num_rows == 0) return;
     MNT_CHECK(rows != nullptr && weights != nullptr && out != nullptr, "null argument");

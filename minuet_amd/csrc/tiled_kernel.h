@@ -115,9 +115,9 @@ struct TiledShape {
 // QUADS: KS lanes read neighbouring pieces of one row and turn them round among
 // themselves.  The first-level cache looks up one line per clock: 64 lanes on
 // 64 lines take 64 clocks per load instruction, in fours 16 (measured: 254 and
-// 131 clocks per 32 rows of 128 bytes, indices included).  The lane
-// permutations make a lone wavefront slower (13.4 against 11.2 us at 25 000
-// targets), so it is for launches that fill the chip.
+// 131 clocks per 32 rows of 128 bytes, indices included).  Without tiles the
+// lane permutations make a lone wavefront slower (13.4 against 11.2 us at 25 000
+// targets); where they pay with tiles is told at the launch.
 // GROUPS = 2: two sets of four wavefronts take every second stage each and
 // their sums meet in LDS, for launches of one workgroup per compute unit or
 // less, which wait for a tile's longest chain of stages.
@@ -125,12 +125,12 @@ struct TiledShape {
 // What bounds it: on small clouds that chain (0.3 us a stage), on large ones
 // the address units and the path from the second-level cache.  At a million
 // targets under 125 offsets, 25 M source rows of 128 bytes in 0.42 ms, the
-// address units are busy 81 % of the time and the matrix pipes 35 %; of 46 M
-// reads of the second-level cache nine in ten are hits there.  64 -> 64
+// address units are busy 89 % of the time and the matrix pipes 38 %; of 46 M
+// reads of the second-level cache four in five are hits there.  64 -> 64
 // channels, 16-bit, us a layer in implicit_forward_kernel and here: 3 000
 // targets of an object 14.9 / 8.8, 25 000 of a LiDAR scan 14.9 / 10.3, 60 000
-// of a room 18.2 / 17.4; in tiles, LiDAR, 120 000 32.3 / 20.0, 200 000 48.6 /
-// 32.7, a million under 5 x 5 x 5 836 / 424.
+// of a room 18.2 / 17.4; in tiles, LiDAR, 200 000 48.6 / 27, a
+// million under 5 x 5 x 5 836 / 407.
 template <typename T, int NB, int KS, bool TILED, bool PAIRED, bool WHOLE, bool QUADS, int GROUPS>
 __global__ __launch_bounds__(256 * GROUPS) void tiled_forward_kernel(
     const T *__restrict__ sources, unsigned source_bytes, const T *__restrict__ wt,
