@@ -114,8 +114,11 @@ class Arena {
   void set_growth(float g) { growth_ = g; }
   void set_page_size(size_t b) { page_size_ = b ? b : page_size_; }
 
-  // Pinned host staging block (64 KiB) for small read-backs and uploads.
+  // Pinned host staging block (64 KiB) for small read-backs and uploads; behind it
+  // kPinnedWords words that only kernels write which leave a number with each
+  // (wait_words).
   static constexpr size_t kPinnedBytes = 64 * 1024;
+  static constexpr int kPinnedWords = 4096;
   void *pinned();
   // Device-side address of the same block (kernels may write results there).
   void *pinned_device();
@@ -132,6 +135,13 @@ class Arena {
   void wait_flag(int slot, unsigned long long sequence);
   // The same for any word of the pinned block.
   void wait_word(volatile unsigned long long *word, unsigned long long sequence);
+  // `count` words behind the pinned block whose upper half is the sequence number's
+  // lower half (not zero) once a kernel has stored them: a word is its own flag, so
+  // many workgroups answer with neither a meeting nor a fence.  The lower halves.
+  unsigned long long *words_device() {
+    return reinterpret_cast<unsigned long long *>(static_cast<char *>(pinned_device()) + kPinnedBytes);
+  }
+  const volatile unsigned long long *wait_words(int count, unsigned long long sequence);
   // Long-lived device blocks that survive scopes (state of the two-phase entry
   // points; slot 0: target coordinates, slot 1: kernel-map build, slot 2: pass
   // builder).  Grows to at least `bytes`; 0 returns the current block.
@@ -176,6 +186,9 @@ class Arena {
   size_t cursor_ = 0;
   size_t page_size_ = size_t(8) << 20;
   float growth_ = 1.0f;
+  template <typename Done>
+  void spin(Done done);
+
   void *pinned_ = nullptr;
   void *pinned_device_ = nullptr;
   unsigned long long sequence_ = 0;

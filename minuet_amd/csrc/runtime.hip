@@ -192,8 +192,9 @@ size_t Arena::used() const {
 
 void *Arena::pinned() {
   if (!pinned_) {
-    MNT_HIP(hipHostMalloc(&pinned_, kPinnedBytes, hipHostMallocMapped | hipHostMallocCoherent));
-    memset(pinned_, 0, kPinnedBytes);
+    constexpr size_t bytes = kPinnedBytes + sizeof(unsigned long long) * kPinnedWords;
+    MNT_HIP(hipHostMalloc(&pinned_, bytes, hipHostMallocMapped | hipHostMallocCoherent));
+    memset(pinned_, 0, bytes);
     MNT_HIP(hipHostGetDevicePointer(&pinned_device_, pinned_, 0));
   }
   return pinned_;
@@ -217,7 +218,8 @@ void Arena::wait_flag(int slot, unsigned long long sequence) {
             sequence);
 }
 
-void Arena::wait_word(volatile unsigned long long *flag, unsigned long long sequence) {
+template <typename Done>
+void Arena::spin(Done done) {
   const auto start = std::chrono::steady_clock::now();
   struct Tally {
     std::chrono::steady_clock::time_point since;
@@ -229,18 +231,33 @@ void Arena::wait_word(volatile unsigned long long *flag, unsigned long long sequ
     }
   } tally{start};
   unsigned spins = 0;
-  while (*flag != sequence) {
+  while (!done()) {
     if ((++spins & 0x3FFFu) == 0) {
       const auto waited = std::chrono::steady_clock::now() - start;
       if (waited > std::chrono::seconds(2)) {
         MNT_HIP(hipStreamSynchronize(stream_));
-        MNT_CHECK(*flag == sequence, "a kernel finished without signalling its completion flag");
+        MNT_CHECK(done(), "a kernel finished without signalling its completion flag");
         break;
       }
     }
     __builtin_ia32_pause();
   }
   std::atomic_thread_fence(std::memory_order_acquire);
+}
+
+const volatile unsigned long long *Arena::wait_words(int count, unsigned long long sequence) {
+  const volatile unsigned long long *words =
+      reinterpret_cast<const volatile unsigned long long *>(static_cast<char *>(pinned()) + kPinnedBytes);
+  int at = 0;
+  spin([&] {
+    while (at < count && static_cast<unsigned>(words[at] >> 32) == static_cast<unsigned>(sequence)) ++at;
+    return at == count;
+  });
+  return words;
+}
+
+void Arena::wait_word(volatile unsigned long long *flag, unsigned long long sequence) {
+  spin([&] { return *flag == sequence; });
 }
 
 void *Arena::persistent(int slot, size_t bytes) {

@@ -374,6 +374,23 @@ def test_kernel_map_build(reorder, kernel, stride, batched):
     np.testing.assert_array_equal(host(out2), e2out)
 
 
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
+@pytest.mark.parametrize("sources,targets", [(1, 1), (1023, 1025), (3000, 1), (2, 70001)])
+def test_bounds_of_both_clouds_meet_on_the_host(dtype, sources, targets):
+    """Maps between clouds whose bounds are not known: extremes of either sign in the
+    first and last rows, one workgroup's rows and one more, several calls in a row."""
+    rng = np.random.default_rng(sources)
+    off = np.array([[0, 0, 0], [1, -1, 0], [-2, 0, 3]], dtype=dtype)
+    for far in (5, 1000, 7):
+        clouds = []
+        for n in (sources, targets):
+            rows = rng.integers(-far, far, size=(n, 3))
+            rows[0], rows[-1] = -far - n % 7, far + n % 5
+            clouds.append(np.unique(rows, axis=0).astype(dtype))
+        got = F.query_sorted_index_with_offsets(dev(clouds[0]), dev(clouds[1]), dev(off))
+        np.testing.assert_array_equal(host(got), orc.query_sorted_index_with_offsets(clouds[0], clouds[1], off))
+
+
 def test_voxelize_matches_numpy_unique():
     """floor(p / voxel) -> distinct voxels in lexicographic order, and the
     reverse map sends every point to its voxel (checked with np.unique)."""
