@@ -56,7 +56,14 @@ def prefers_streamed(num_offsets: int, num_source_features: int, num_target_feat
     under more than 128 output channels), whose rows and weights stream through
     LDS.  Against three kernels or offset groups, us a layer: 128 -> 128 channels
     over 6 850 voxels 23.0 and 11.8, over 18 600 of a LiDAR level 27.7 and 17.3,
-    256 -> 256 over 2 000 27.1 and 16.8, over 25 600 of a scan 39.5 and 37.1."""
+    256 -> 256 over 2 000 27.1 and 16.8, over 25 600 of a scan 39.5 and 37.1.  Not
+    rows of more than 384 bytes under up to 96 output channels and more than 8
+    offsets, which have four stages an offset and few product bytes to save: 256 ->
+    64 over 23 100 24.2 and 30.7, 256 -> 96 over 10 400 21.6 and 26.2, 256 -> 32 over
+    18 800 19.5 and 27.7 (the other way round over few voxels, 256 -> 32 over 2 300
+    22.6 and 16.9; 192 -> 64 over 22 000 24.0 and 24.0, over 13 800 19.7 and 15.9)."""
+    if num_offsets > 8 and num_source_features > 192 and num_target_features <= 96:
+        return False
     return _C.streamed_forward_supported(num_offsets, num_source_features, num_target_features, dtype)
 
 

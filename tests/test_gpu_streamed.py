@@ -102,3 +102,10 @@ def test_a_layer_gives_the_same_rows_from_call_to_call():
             graph.replay()
             torch.cuda.synchronize()
             assert torch.equal(out, first)
+
+
+@pytest.mark.parametrize("cin,cout,offsets,streams", [(256, 96, 27, False), (256, 104, 27, True), (200, 96, 9, False),
+                                                      (192, 96, 27, True), (256, 32, 8, True)])
+def test_which_wide_layers_are_streamed(cin, cout, offsets, streams):
+    """Both sides of the line between streaming and grouped products."""
+    assert F.prefers_streamed(offsets, cin, cout, torch.float16) == streams
