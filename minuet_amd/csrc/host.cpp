@@ -21,9 +21,12 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <ATen/ATen.h>
+#include <ATen/TracerMode.h>
+#include <ATen/autocast_mode.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/HIPEvent.h>
 #include <c10/core/GradMode.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
@@ -304,7 +307,8 @@ PyTypeObject LayerType = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
 // Layer(module, kind, weights, packed, shape_id, shortcut, rows_from, rows_to, other);
 // shortcut: of kind TABLES whether the centre offset may take one, of kind
-// IMPLICIT whether a target of the map has one source
+// IMPLICIT whether a target of the map has one source, of kind PIECES whether
+// autocast has a say (the layer would be torch.mm otherwise)
 PyObject *layer_new(PyTypeObject *type, PyObject *args, PyObject *) {
   HANDLE_TH_ERRORS
   PyObject *module, *weights, *packed, *shape_id;
@@ -461,6 +465,31 @@ const at::Tensor *tiles_of(MapEntry *map, const Layer *l, int64_t T, const at::D
 
 PyObject *none() { Py_RETURN_NONE; }
 
+// Whether nothing but the operand's value counts (plain in _C.py): it is of no
+// class of its own, records no gradient, carries no tangent and wraps nothing.
+bool plain(PyObject *o) {
+  if (is_none(o)) return true;
+  if (!THPVariable_CheckExact(o)) return false;
+  const at::Tensor &t = THPVariable_Unpack(o);
+  constexpr c10::DispatchKeySet kWrapped{c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
+                                         c10::DispatchKey::Functionalize, c10::DispatchKey::Python};
+  return !t.key_set().has_any(kWrapped) && !(c10::GradMode::is_enabled() && t.requires_grad()) &&
+         !t._fw_grad(/*level=*/0).defined();
+}
+
+// A 1 x 1 x 1 layer has derivatives, batching rules and a trace through
+// torch.mm: whether it may go past that, for these operands and here.
+bool stands_in(const Layer *l, PyObject *features, const EpilogueArgs &ep) {
+  if (c10::impl::TorchDispatchModeTLS::any_modes_set() || at::tracer::impl::is_dispatch_enabled() ||
+      (l->kind == kPieces && l->shortcut != 0 && at::autocast::is_autocast_enabled(at::kCUDA))) {
+    return false;
+  }
+  for (PyObject *o : {features, l->kernel.object, l->bias.object, ep.scale, ep.shift, ep.residual}) {
+    if (!plain(o)) return false;
+  }
+  return true;
+}
+
 // The layer on `inputs`; None when anything is not as the Layer describes it.
 PyObject *run_layer(Layer *l, PyObject *module_dict, PyObject *inputs, const EpilogueArgs &ep) {
   // the one of the module's Layers that is for so many rows
@@ -474,6 +503,7 @@ PyObject *run_layer(Layer *l, PyObject *module_dict, PyObject *inputs, const Epi
     l = reinterpret_cast<Layer *>(l->other);
     if (S < l->rows_from || S > l->rows_to) return none();
   }
+  if ((l->kind == kPointwise || l->kind == kPieces) && !stands_in(l, look(in, s__features), ep)) return none();
   // the module: same parameters, same settings, not being tuned
   PyObject *parameters = look(module_dict, s__parameters);
   PyObject *config = look(module_dict, s__tunable_config);

@@ -922,35 +922,41 @@ class SparseConv(Module):
         shape it runs there, as one offset whose kernel map is the identity,
         so that an epilogue costs no extra pass, or, an fp32 layer over few rows,
         as several offsets, the pieces of its input channels, which the
-        wavefronts of a workgroup share; otherwise ``torch.mm``.  Returns the
-        features, what ``_keep_fast`` takes and its rows."""
-        weights = self.kernel.view(1, self.in_channels, self.out_channels)
-        needs_grad = torch.is_grad_enabled() and (features.requires_grad or weights.requires_grad)
+        wavefronts of a workgroup share; otherwise ``torch.mm``, also where more
+        than the operands' values counts (``_C.plain``): derivatives in either
+        mode, vmap, tracing, dispatch modes.  Returns the features, what
+        ``_keep_fast`` takes and its rows."""
+        kernel = self.kernel
+        weights = kernel.view(1, self.in_channels, self.out_channels)
+        dataflow = self._tunable_config.get("dataflow", "auto")
+        operands = [features, kernel]
+        if epilogue is not None:
+            operands += [t for t in (epilogue.scale, epilogue.shift, epilogue.residual) if t is not None]
         rows = ()
-        if (features.is_cuda and not needs_grad
-                and self._tunable_config.get("dataflow", "auto") == "auto" and features.dtype == weights.dtype):
-            most = F.pieces_rows_limit(self.in_channels, self.out_channels, weights.dtype)
+        if (features.is_cuda and features.dtype == weights.dtype
+                and dataflow not in ("gather_gemm_scatter", "list_driven") and _C.plain(operands)):
+            # measured against torch.mm plus a separate epilogue pass up to these widths;
+            # wider layers of many rows are plain library GEMM territory
+            narrow = (_C.implicit_forward_supported(self.in_channels, self.out_channels, weights.dtype)
+                      and self.in_channels * weights.dtype.itemsize <= 512 and self.out_channels <= 128)
+            # (what torch.mm would otherwise make follows autocast)
+            most = (F.pieces_rows_limit(self.in_channels, self.out_channels, weights.dtype)
+                    if dataflow == "auto" and (narrow or not torch.is_autocast_enabled()) else -1)
             rows = (most + 1, _MOST_ROWS) if most >= 0 else ()
             if 0 < features.shape[0] <= most and features.is_contiguous():
                 whole, packed = self._lane_kernel(F.channel_pieces(self.in_channels))
                 out = _C.sparse_convolution_forward_pieces(features, packed, self.out_channels, epilogue=epilogue)
-                return out, ("PIECES", whole.view(weights.shape), packed, None, None, 0), (0, most)
-        if (features.is_cuda and not needs_grad
-                and self._tunable_config.get("dataflow", "auto") not in ("gather_gemm_scatter", "list_driven")
-                and features.dtype == weights.dtype
-                and _C.implicit_forward_supported(self.in_channels, self.out_channels, weights.dtype)
-                # measured against torch.mm plus a separate epilogue pass up to these widths;
-                # wider layers are plain library GEMM territory
-                and self.in_channels * weights.dtype.itemsize <= 512 and self.out_channels <= 128):
-            count = features.shape[0]
-            identity = self._identity_map
-            if identity is None or identity.shape[1] < count or identity.device != features.device:
-                identity = torch.arange(count, dtype=torch.int32, device=features.device).view(1, count)
-                self._identity_map = identity
-            packed = self._packed_kernel()[1]
-            out = _C.sparse_convolution_forward_implicit(features, weights, identity[:, :count],
-                                                         epilogue=epilogue, packed_weights=packed)
-            return out, ("POINTWISE", weights.detach(), packed, None, None, 0), rows
+                return out, ("PIECES", whole.view(weights.shape), packed, None, None, 0, None, not narrow), (0, most)
+            if narrow:
+                count = features.shape[0]
+                identity = self._identity_map
+                if identity is None or identity.shape[1] < count or identity.device != features.device:
+                    identity = torch.arange(count, dtype=torch.int32, device=features.device).view(1, count)
+                    self._identity_map = identity
+                packed = self._packed_kernel()[1]
+                out = _C.sparse_convolution_forward_implicit(features, weights, identity[:, :count],
+                                                             epilogue=epilogue, packed_weights=packed)
+                return out, ("POINTWISE", weights.detach(), packed, None, None, 0), rows
         out = torch.mm(features, weights[0])
         return out if epilogue is None else epilogue.apply(out), None, ()
 
@@ -980,7 +986,7 @@ class SparseConv(Module):
                 epilogue = F.Epilogue(epilogue.scale, shift, epilogue.residual, epilogue.activation,
                                       epilogue.negative_slope)
             bias = None
-        made = None                                 # (kind, weights, packed, map pointers, owners, index code)
+        made = None                                 # (kind, weights, packed, map pointers, owners, index code[, tiles, flag])
         rows = ()                                   # from how many to how many rows that kind is the one to take
         if self.is_trivial:
             features, made, rows = self._pointwise(inputs.F, epilogue)
@@ -1072,7 +1078,7 @@ class SparseConv(Module):
         stays with the new one: each cloud gets the kernel that a fresh cache
         would give it, whatever came before."""
         name, weights, packed, pointers, owners, index_code = made[:6]
-        tiles, single = made[6:] if len(made) > 6 else (None, False)
+        tiles, flag = made[6:] if len(made) > 6 else (None, False)
         host = _C.load_host()
         if host is None:
             return
@@ -1090,7 +1096,7 @@ class SparseConv(Module):
         if not weights.is_contiguous() or parameters.get("kernel") is None or "bias" not in parameters:
             return                                  # (a pruned or parametrised kernel is made anew from others)
         # (past Module.__setattr__, which takes longer than all of the rest)
-        shortcut = single or (name == "TABLES" and self._allow_shortcut_matmul)
+        shortcut = flag or (name == "TABLES" and self._allow_shortcut_matmul)
         self.__dict__["_fast"] = host.Layer(self, kind, weights, packed, shape_id, 1 if shortcut else 0,
                                             *(rows and (*rows, self._fast)))
 
