@@ -830,9 +830,10 @@ class SparseConv(Module):
         """``(weights, packed)``: the layer's weights (with ``pad`` zero input
         channels appended) and the same in the layout the matrix kernels stage,
         remade only when the parameter has changed (in-place updates bump its
-        version counter).  ``packed`` is None while gradients are recorded."""
+        version counter).  ``packed`` is None while gradients are recorded, and
+        for a kernel made in inference mode, which counts no versions."""
         kernel = self.kernel
-        if torch.is_grad_enabled() and kernel.requires_grad:
+        if (torch.is_grad_enabled() and kernel.requires_grad) or kernel.is_inference():
             padded = kernel if pad == 0 else torch.nn.functional.pad(kernel, (0, 0, 0, pad))
             return padded, None
         key = (kernel.data_ptr(), kernel._version, kernel.dtype, kernel.device, pad)
@@ -854,7 +855,8 @@ class SparseConv(Module):
         kernel = self.kernel
         if pieces > 1:
             kernel = kernel.view(pieces, self.in_channels // pieces, self.out_channels)
-        if (torch.is_grad_enabled() and kernel.requires_grad) or not _C.lane_weights_supported(kernel):
+        if ((torch.is_grad_enabled() and kernel.requires_grad) or kernel.is_inference()
+                or not _C.lane_weights_supported(kernel)):
             return self._packed_kernel()
         key = (kernel.data_ptr(), kernel._version, kernel.dtype, kernel.device)
         kept = self.__dict__.get("_lanes")          # (none in a module pickled before there were any)
@@ -939,9 +941,11 @@ class SparseConv(Module):
             # wider layers of many rows are plain library GEMM territory
             narrow = (_C.implicit_forward_supported(self.in_channels, self.out_channels, weights.dtype)
                       and self.in_channels * weights.dtype.itemsize <= 512 and self.out_channels <= 128)
-            # (what torch.mm would otherwise make follows autocast)
+            # (what torch.mm would otherwise make follows autocast, and a kernel made in
+            # inference mode says nothing of writes to it: no packed copy can be kept)
             most = (F.pieces_rows_limit(self.in_channels, self.out_channels, weights.dtype)
-                    if dataflow == "auto" and (narrow or not torch.is_autocast_enabled()) else -1)
+                    if dataflow == "auto" and not kernel.is_inference()
+                    and (narrow or not torch.is_autocast_enabled()) else -1)
             rows = (most + 1, _MOST_ROWS) if most >= 0 else ()
             if 0 < features.shape[0] <= most and features.is_contiguous():
                 whole, packed = self._lane_kernel(F.channel_pieces(self.in_channels))

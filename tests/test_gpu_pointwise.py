@@ -94,3 +94,23 @@ def test_dispatch_modes_and_autocast(cin, cout, dtype, kept):
         with torch.autocast("cuda", dtype=torch.bfloat16):
             assert call(x).dtype == (torch.bfloat16 if wide else dtype)
         assert call(x).dtype == dtype
+
+
+@pytest.mark.parametrize("size", [1, 3])
+@pytest.mark.parametrize("cin, cout, dtype", SHAPES)
+def test_parameters_made_in_inference_mode(cin, cout, dtype, size):
+    """They count no versions, so that nothing derived from them can be kept."""
+    with torch.inference_mode():
+        conv = minuet.nn.SparseConv3d(cin, cout, size, dtype=dtype, device=DEVICE)
+        conv.set_kernel_map_cache(minuet.nn.KernelMapCache(3, torch.int32, DEVICE))
+        cells = torch.randperm(4096, device=DEVICE)[:ROWS]
+        coordinates = torch.stack([cells >> 8, (cells >> 4) & 15, cells & 15], 1).int()
+        coordinates = coordinates[F.build_sorted_index(coordinates)]
+        x = minuet.SparseTensor(torch.randn(ROWS, cin, device=DEVICE).to(dtype), coordinates)
+        first = conv(x).F.clone()
+        assert conv(x).F.equal(first)
+        conv.kernel.mul_(2.0)
+        # (twice the sums, rounded: a result below the normal numbers may be off by their spacing)
+        spacing = 2.0 ** -24 if dtype == torch.float16 else 0.0
+        for _ in range(2):
+            assert ((conv(x).F.double() - 2 * first.double()).abs() <= spacing).all()
