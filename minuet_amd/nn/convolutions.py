@@ -903,11 +903,12 @@ class SparseConv(Module):
                 and _C.single_forward_supported(self.kernel.shape[0], features.shape[1], self.out_channels,
                                                 features.dtype))
 
-    def _takes_offset_groups(self, features: torch.Tensor) -> bool:
+    def _takes_offset_groups(self, features: torch.Tensor, streamed: bool = True) -> bool:
         """Whether this call multiplies its offsets three at a time (the
         ``offset_groups`` dataflow): forced by the tunable ``dataflow``, or, under
         ``auto``, for the 16-bit 3 x 3 x 3 layers that are too wide to be streamed
-        and whose product rows are what bounds them."""
+        (all wide ones where there is no streaming: ``streamed``) and whose product
+        rows are what bounds them."""
         dataflow = self._tunable_config.get("dataflow", "auto")
         if dataflow not in ("auto", "offset_groups") or not features.is_cuda or self.transposed:
             return False
@@ -916,7 +917,7 @@ class SparseConv(Module):
             return False
         return dataflow == "offset_groups" or (
             self.in_channels * features.element_size() >= 256
-            and not F.prefers_streamed(27, self.in_channels, self.out_channels, features.dtype))
+            and not (streamed and F.prefers_streamed(27, self.in_channels, self.out_channels, features.dtype)))
 
     def _pointwise(self, features: torch.Tensor, epilogue: Optional[F.Epilogue]):
         """1x1x1 kernel, stride 1: a plain ``features @ W`` (reference:
@@ -951,8 +952,8 @@ class SparseConv(Module):
                 whole, packed = self._lane_kernel(F.channel_pieces(self.in_channels))
                 out = _C.sparse_convolution_forward_pieces(features, packed, self.out_channels, epilogue=epilogue)
                 return out, ("PIECES", whole.view(weights.shape), packed, None, None, 0, None, not narrow), (0, most)
-            if narrow:
-                count = features.shape[0]
+            count, far = features.shape[0], F.implicit_rows_limit(self.in_channels, weights.dtype)
+            if narrow and count <= far:
                 identity = self._identity_map
                 if identity is None or identity.shape[1] < count or identity.device != features.device:
                     identity = torch.arange(count, dtype=torch.int32, device=features.device).view(1, count)
@@ -960,7 +961,7 @@ class SparseConv(Module):
                 packed = self._packed_kernel()[1]
                 out = _C.sparse_convolution_forward_implicit(features, weights, identity[:, :count],
                                                              epilogue=epilogue, packed_weights=packed)
-                return out, ("POINTWISE", weights.detach(), packed, None, None, 0), rows
+                return out, ("POINTWISE", weights.detach(), packed, None, None, 0), (rows[0] if rows else 0, far)
         out = torch.mm(features, weights[0])
         return out if epilogue is None else epilogue.apply(out), None, ()
 
@@ -1033,9 +1034,17 @@ class SparseConv(Module):
                 grouped = self._takes_offset_groups(sources)
                 pad = 0 if grouped else self._row_padding(sources)
                 implicit = self._takes_implicit(sources, pad) if hits is None else hits
-                route = (pad, not grouped and implicit, grouped)
+                route = (pad, not grouped and implicit, grouped, None)
+                if hits is None and route[1] and dataflow == "auto":
+                    # (where its features are past what that form addresses: as if there were no such form)
+                    route = (*route[:3], F.implicit_rows_limit(self.in_channels + pad, sources.dtype))
                 self._routes[route_key] = route
-            pad, implicit, grouped = route
+            pad, implicit, grouped, most = route
+            if most is not None:
+                rows = (0, most)
+                if sources.shape[0] > most:
+                    pad, implicit, grouped = 0, False, self._takes_offset_groups(sources, streamed=False)
+                    rows = (most + 1, _MOST_ROWS)
             groups = cache.get_offset_groups(**map_args) if grouped and self._tuning_data is None else None
             if groups is not None:
                 # offsets multiplied three at a time: needs the dense map and its group tables only

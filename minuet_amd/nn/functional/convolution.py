@@ -9,7 +9,7 @@ from ..kernel_map import KernelMap
 
 __all__ = ["cuda_time_gather", "cuda_time_scatter", "sparse_convolution_forward",
            "cuda_time_gemm", "set_gemm_parallel_level", "Epilogue", "pack_weights",
-           "prefers_implicit", "prefers_streamed", "prefers_hits", "hits_rows_limit",
+           "prefers_implicit", "prefers_streamed", "prefers_hits", "implicit_rows_limit", "hits_rows_limit",
            "pieces_rows_limit", "channel_pieces"]
 
 pack_weights = _C.pack_weights
@@ -67,6 +67,13 @@ def prefers_streamed(num_offsets: int, num_source_features: int, num_target_feat
     return _C.streamed_forward_supported(num_offsets, num_source_features, num_target_features, dtype)
 
 
+def implicit_rows_limit(num_source_features: int, dtype: torch.dtype) -> int:
+    """The most source rows of which the single-kernel form takes any: it addresses
+    them through 32-bit buffer offsets, so features of 4 GiB and more go to the
+    three kernels or the offset groups, which do not."""
+    return (_C.IMPLICIT_MAX_SOURCE_BYTES - 1) // (num_source_features * dtype.itemsize)
+
+
 def hits_rows_limit(num_offsets: int, num_source_features: int, num_target_features: int,
                     dtype: torch.dtype) -> int:
     """The most source rows over which ``dataflow="auto"`` takes the single-kernel
@@ -89,12 +96,11 @@ def hits_rows_limit(num_offsets: int, num_source_features: int, num_target_featu
     63 / 76), or about even (2x2x2 over 300 000 31.5 / 31.7 and, transposed, 36.9
     / 33.6).
 
-    Source rows are addressed through 32-bit buffer offsets, so features of 4 GiB
-    and more go to the three kernels whatever the width."""
+    Never more than ``implicit_rows_limit``."""
     if (dtype != torch.float32 or num_offsets <= 1
             or not _C.implicit_forward_supported(num_source_features, num_target_features, dtype)):
         return -1
-    most = (_C.IMPLICIT_MAX_SOURCE_BYTES - 1) // (num_source_features * dtype.itemsize)
+    most = implicit_rows_limit(num_source_features, dtype)
     work = num_source_features * num_target_features
     if work <= 1024:
         return most
@@ -223,7 +229,8 @@ def sparse_convolution_forward(sources: torch.Tensor, weights: torch.Tensor,
         shape = (weights.shape[0], weights.shape[1], weights.shape[2], weights.dtype)
         if dataflow == "implicit" or (prefers_hits(*shape, sources.shape[0])
                                       if weights.dtype == torch.float32 and weights.shape[0] > 1
-                                      else prefers_implicit(*shape)):
+                                      else prefers_implicit(*shape)
+                                      and sources.shape[0] <= implicit_rows_limit(weights.shape[1], weights.dtype)):
             return _C.sparse_convolution_forward_implicit(sources, weights, dense, epilogue=epilogue,
                                                           packed_weights=packed_weights)
     if dataflow == "list_driven":

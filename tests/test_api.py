@@ -189,6 +189,15 @@ def test_fp32_rule_follows_the_kernel_size():
     assert prefers(125, 32, 32, single, 100000)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_rows_that_the_single_kernel_form_addresses(dtype):
+    limit = minuet.nn.functional.implicit_rows_limit
+    for channels in (4, 100, 128, 256):
+        most = limit(channels, dtype)
+        row = channels * dtype.itemsize
+        assert most * row < 0xFFFFF000 <= (most + 1) * row      # (what the library refuses)
+
+
 def test_lookahead_layout_places_every_output():
     """The plan of a look-ahead session (no GPU needed): every output of every
     recipe entry gets a 256-byte aligned place of its own inside one allocation,

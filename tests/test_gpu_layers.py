@@ -117,3 +117,54 @@ def test_network_without_the_extension_module(monkeypatch):
             module.invalidate_cached_weights()
     for a, b in zip(with_it, passes()):
         assert torch.equal(a, b)
+
+
+# (channels, channels, kernel size, stride, transposed, type): one per kernel that addresses rows by 32 bits
+@pytest.mark.parametrize("cin,cout,size,stride,transposed,dtype", [
+    (128, 128, 3, 1, False, torch.float16), (256, 128, 3, 1, False, torch.bfloat16),
+    (128, 256, 2, 2, False, torch.float16), (128, 64, 2, 2, True, torch.float16), (64, 64, 3, 1, False, torch.float16),
+    (100, 96, 5, 1, False, torch.float16), (30, 32, 3, 1, False, torch.float16), (64, 64, 1, 1, False, torch.float16),
+    (32, 64, 1, 1, False, torch.float32), (32, 32, 1, 2, False, torch.float32), (64, 32, 3, 1, False, torch.float32)])
+def test_features_past_the_single_kernel_form(cin, cout, size, stride, transposed, dtype, monkeypatch):
+    """Features of 4 GiB and more run as if there were no such form, before and
+    after small ones; here from some hundred kilobytes on."""
+    gen = torch.Generator(device=DEVICE).manual_seed(cin)
+    torch.manual_seed(cin)
+    down = minuet.nn.SparseConv3d(4, cin, size, stride=stride, dtype=dtype, device=DEVICE) if transposed else None
+    conv = minuet.nn.SparseConv(3, cin, cout, size, stride=stride, transposed=transposed, dtype=dtype, device=DEVICE)
+    inputs = []
+    for rows in (400, 6000):
+        cells = torch.randperm(1 << 15, generator=gen, device=DEVICE)[:rows]
+        coordinates = torch.stack([cells >> 10, (cells >> 5) & 31, cells & 31], 1).int()
+        coordinates = coordinates[F.build_sorted_index(coordinates)]
+        x = minuet.SparseTensor(torch.randn(rows, 4 if transposed else cin, generator=gen, device=DEVICE).to(dtype), coordinates)
+        inputs.append(x)
+
+    def results(order):
+        cache = minuet.nn.KernelMapCache(3, torch.int32, DEVICE)
+        for module in (conv, down) if transposed else (conv,):
+            module.set_kernel_map_cache(cache)
+            module.invalidate_cached_weights()
+            module._routes.clear()
+        out = []
+        with torch.no_grad():
+            for i in order:
+                cache.reset()
+                x = inputs[i] if down is None else down(inputs[i])
+                out.append(conv(x).F)
+                assert torch.equal(out[-1], conv(x).F)
+        return out
+
+    small, large = results((0, 1))
+    calls = []
+    for name in ("implicit", "single", "tiled", "pieces"):
+        whole = getattr(_C, f"sparse_convolution_forward_{name}")
+        monkeypatch.setattr(_C, f"sparse_convolution_forward_{name}",
+                            lambda sources, *args, _whole=whole, **kw: calls.append(sources) or _whole(sources, *args, **kw))
+    limit = 2000 * cin * dtype.itemsize
+    monkeypatch.setattr(_C, "IMPLICIT_MAX_SOURCE_BYTES", limit)
+    for got, wanted in zip(results((1, 0, 1, 0, 0, 1)), (large, small, large, small, small, large)):
+        # sums of unit normals times uniform weights in another order, rounded once or twice
+        tolerance = 1e-5 if dtype == torch.float32 else 4 * torch.finfo(dtype).eps
+        assert float((got.double() - wanted.double()).norm() / wanted.double().norm()) < tolerance
+    assert calls and all(s.numel() * s.element_size() < limit for s in calls)
