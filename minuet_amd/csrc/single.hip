@@ -24,9 +24,10 @@ struct SingleShape {
 // those that have their source under its offset, about an eighth, and multiplies
 // 64 of them at a time: rows and weights go straight to LDS, 128 bytes of each at
 // a time, and the products from there to the targets' rows.  Targets without a
-// source go with the first wavefront's.  Where a target has two sources (the
-// caller says there is none) the wavefronts take 32 targets each under all
-// offsets instead.
+// source are the first wavefront's, which multiplies nothing for them: zeros
+// times an infinite or undefined weight are no zeros.  Where a target has two
+// sources (the caller says there is none) the wavefronts take 32 targets each
+// under all offsets instead.
 //
 // What bounds it: one workgroup a compute unit, whose wavefronts wait for their
 // map, their first rows and every next 128 bytes of them; so as few rounds of
@@ -107,6 +108,7 @@ __global__ __launch_bounds__(64 * kSingleWaves) void single_forward_kernel(
     }
     count += __popcll(votes);
   }
+  const int hits = __builtin_amdgcn_readfirstlane(count);      // (behind them: targets without a source)
   __syncthreads();
   for (int t = tid; t < here; t += 64 * kSingleWaves) {
     if (s_hits[t] > 1) s_many = 1;
@@ -204,17 +206,21 @@ __global__ __launch_bounds__(64 * kSingleWaves) void single_forward_kernel(
     }
   };
   if (!many) {
-    for (int from = 0; from < count; from += 64) {
-      const int groups = count - from > 32 ? 2 : 1;
-      auto target = [&](int row) -> int { return from + row < count ? s_target[wv][from + row] : -1; };
+    for (int from = 0; from < hits; from += 64) {
+      const int groups = hits - from > 32 ? 2 : 1;
+      auto target = [&](int row) -> int { return from + row < hits ? s_target[wv][from + row] : -1; };
       clear();
-      multiply(wv, groups, from + 64 < count, [&](int row) {
+      multiply(wv, groups, from + 64 < hits, [&](int row) {
         const int t = target(row);
         return t < 0 ? -1 : s_source[t];
       });
       store(groups, target);
     }
-    if (count == 0) wait_loads<0>();           // (none may land after the workgroup has gone)
+    if (hits == 0) wait_loads<0>();            // (none may land after the workgroup has gone)
+    clear();
+    for (int from = hits; from < count; from += 64) {
+      store(count - from > 32 ? 2 : 1, [&](int row) -> int { return from + row < count ? s_target[wv][from + row] : -1; });
+    }
     return;
   }
   ready = false;
@@ -222,10 +228,18 @@ __global__ __launch_bounds__(64 * kSingleWaves) void single_forward_kernel(
     auto target = [&](int row) -> int { return from + row < here ? from + row : -1; };
     clear();
     for (int o = 0; o < s.offsets; ++o) {
-      multiply(o, 1, false, [&](int row) {
+      auto source = [&](int row) {
         const int t = target(row);
         return t < 0 ? -1 : kernel_map[o * s.num_targets + first + t];
-      });
+      };
+      floatx16 before[2] = {acc[0][0], acc[0][1]};
+      multiply(o, 1, false, source);
+      const bool used = source(r) >= 0;        // (a lane's sums are those of target r)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) acc[0][b][j] = used ? acc[0][b][j] : before[b][j];
+      }
     }
     store(1, target);
   }

@@ -61,6 +61,27 @@ def test_epilogue_and_weights_that_are_not_finite():
     assert bool(got[~hit].isfinite().all()) and torch.allclose(got[~hit], other[~hit], rtol=2e-3, atol=2e-3)
 
 
+# the last of many workgroups and the only one; each wavefront's offset, those that list targets without a
+# source among them; maps that keep the promise and one that does not
+@pytest.mark.parametrize("targets", [20, 700, 40000])
+@pytest.mark.parametrize("double", [0.0, 0.02])
+def test_weights_that_are_not_finite_reach_their_targets_only(targets, double):
+    gen = torch.Generator().manual_seed(targets)
+    dense = _map(targets, 300, gen, empty=0.3, double=double)
+    dense[:, targets // 2:targets // 2 + 8] = -1
+    x, w = torch.randn(300, 136, generator=gen).half().cuda(), (torch.randn(8, 136, 48, generator=gen) / 12).half().cuda()
+    dense = dense.cuda()
+    plain = _C.sparse_convolution_forward_single(x, w, dense, F.pack_weights(w))
+    assert bool(plain.isfinite().all()) and bool((plain[(dense < 0).all(0)] == 0).all())
+    for offset in range(8):
+        spoilt = w.clone()
+        spoilt[offset, 130, 7], spoilt[offset, 0, 40] = float("inf"), float("nan")
+        got = _C.sparse_convolution_forward_single(x, spoilt, dense, F.pack_weights(spoilt))
+        reached = torch.zeros(targets, 48, dtype=torch.bool, device="cuda")
+        reached[:, [7, 40]] = (dense[offset] >= 0)[:, None]
+        assert torch.equal(got[~reached], plain[~reached]) and not bool(got[reached].isfinite().any())
+
+
 def test_layer_takes_it():
     """Down and up again, through the first call, the second and a planned pass."""
     gen = torch.Generator().manual_seed(1)
