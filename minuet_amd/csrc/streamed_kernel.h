@@ -83,9 +83,9 @@ __device__ __forceinline__ void meet() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts
 //
 // A target without a source under an offset takes part with zeros, which one
 // infinite or undefined weight would turn into sums that are undefined.  So
-// where sums are not finite the workgroup starts again and leaves out what none
-// of 32 targets has a source under (the same sums wherever those are finite): a
-// test per stage instead cost 15 % of it.
+// where sums are not finite the workgroup starts again, and every target keeps
+// what it has under an offset that it has no source under (the same sums
+// wherever those are finite): a test per stage instead cost 15 % of it.
 template <typename T, int MW, int NW, int KW, int WM, int WN, int NL, int BK, int CH, int RING, bool TILED>
 __global__ __launch_bounds__(64 * (MW * NW * KW + NL))
 __attribute__((amdgpu_waves_per_eu((MW * NW * KW + NL + 3) / 4, 8))) void streamed_forward_kernel(
@@ -404,7 +404,11 @@ __attribute__((amdgpu_waves_per_eu((MW * NW * KW + NL + 3) / 4, 8))) void stream
 #pragma unroll
           for (int kk = 0; kk < KS; ++kk) {
 #pragma unroll
-            for (int b = 0; b < WN; ++b) acc[a][b] = Mfma<T>::run(p.w[kk][b], p.x[kk][a], acc[a][b]);
+            for (int b = 0; b < WN; ++b) {
+              const floatx16 sum = Mfma<T>::run(p.w[kk][b], p.x[kk][a], acc[a][b]);
+#pragma unroll
+              for (int j = 0; j < 16; ++j) acc[a][b][j] = entry[a] >= 0 ? sum[j] : acc[a][b][j];
+            }
           }
         }
       }

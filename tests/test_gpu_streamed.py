@@ -43,9 +43,9 @@ def test_forward_matches_products(targets, offsets, cin, cout, dtype):
 @pytest.mark.parametrize("targets,cin,cout", [(1, 128, 64), (1000, 256, 64), (5000, 128, 128), (17000, 192, 64),
                                               (9000, 128, 128), (50000, 128, 128)])
 def test_undefined_numbers_stay_where_they_belong(targets, cin, cout):
-    """A weight that is not finite reaches the 32 targets that stand with one that
-    uses its offset, a feature that is not finite the targets that use its row,
-    and every other row is what it is without."""
+    """A weight that is not finite reaches none of the 32 targets that stand
+    together where none uses its offset, a feature that is not finite the targets
+    that use its row, and every other row is what it is without."""
     dense, x, w = operands(targets, 3000, 27, cin, cout, torch.float16)
     dense[[0, 5, 26]] = -1
     dense[9] = -1
@@ -73,6 +73,27 @@ def test_undefined_numbers_stay_where_they_belong(targets, cin, cout):
         assert torch.equal(forward(x, wild)[others], wanted[others])
         got = forward(bad, w)
         assert torch.equal(got[~touched], wanted[~touched]) and not bool(got[touched].isfinite().all(1).any())
+
+
+# strided, 3x3x3 and 5x5x5; every workgroup shape and rows of one to four stages among them
+@pytest.mark.parametrize("targets,offsets,cin,cout", [
+    (700, 8, 128, 256), (3000, 27, 64, 160), (5000, 27, 256, 128), (6000, 125, 136, 64), (17000, 8, 192, 96),
+    (9000, 27, 128, 128), (26000, 27, 144, 128)])
+def test_weights_that_are_not_finite_reach_their_targets_only(targets, offsets, cin, cout):
+    """Those that have a source under the offset, one by one."""
+    dense, x, w = operands(targets, 3000, offsets, cin, cout, torch.float16)
+    tiles = _C.kernel_map_tiles(dense)
+    plain = _C.sparse_convolution_forward_implicit(x, w, dense, packed_weights=F.pack_weights(w))
+    assert bool(plain.isfinite().all())
+    for offset in (0, offsets // 2, offsets - 1):
+        spoilt = w.clone()
+        spoilt[offset, cin - 1, 3], spoilt[offset, 0, cout - 1] = float("-inf"), float("nan")
+        reached = torch.zeros(targets, cout, dtype=torch.bool, device=DEVICE)
+        reached[:, [3, cout - 1]] = (dense[offset] >= 0)[:, None]
+        packed = F.pack_weights(spoilt)
+        for got in (_C.sparse_convolution_forward_implicit(x, spoilt, dense, packed_weights=packed),
+                    _C.sparse_convolution_forward_tiled(x, spoilt, tiles, targets, packed)):
+            assert torch.equal(got[~reached], plain[~reached]) and not bool(got[reached].isfinite().any())
 
 
 def test_a_layer_gives_the_same_rows_from_call_to_call():
