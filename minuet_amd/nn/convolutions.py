@@ -148,10 +148,16 @@ class KernelMapCache(object):
     def _plan_next_pass(self):
         """Turns the requests of the pass that ends here into the plan of the next one."""
         if self._built is not None:
+            saved = None                         # (key, transposed) -> what tiles saved, or would have
             for entry, request in self._built.entries:
                 if entry.used:                   # a layer that never came through Python
                     self._note_fast(request)
-            self._note_tiles(self._built)
+                    share = entry.tiles_saved
+                    if share:
+                        saved = {} if saved is None else saved
+                        saved[request[4:]] = saved.get(request[4:], 0.0) + share
+            if saved is not None:
+                self._note_tiles(saved, self._built.plan.tiles)
             self._built = None
         requests, self._requests = self._requests, dict()
         if self._lookahead or not requests or not self._coordinates_cache:
@@ -186,13 +192,10 @@ class KernelMapCache(object):
             self._requests.setdefault(("tables", key, not self._disable_reordering))
         self._requests.setdefault(request)
 
-    def _note_tiles(self, built):
+    def _note_tiles(self, saved, made):
         """Asks for the tiles of the maps whose layers would have saved enough by them."""
-        saved = {}
-        for entry, (_, _, _, _, key, transposed) in built.entries:
-            saved[key, transposed] = saved.get((key, transposed), 0.0) + entry.tiles_saved
         for at, share in saved.items():
-            if share >= (_TILES_STAY if at in built.plan.tiles else _TILES_PAY):
+            if share >= (_TILES_STAY if at in made else _TILES_PAY):
                 self._requests.setdefault(("tiles", *at))
 
     def _open_pass(self, coordinates, stride, batch_dims):

@@ -165,8 +165,9 @@ class BuiltPass:
         self.shape = {key: (plan.maps[i].num_offsets, plan.maps[i].num_sources, plan.maps[i].num_targets)
                       for key, i in plan.map_of.items()}
         self.entries = []                # (extension's entry, the request it stands for)
-        self.tiles = self._make_tiles()  # (key, transposed) -> tiles, made by the stream current now
-        self.stream = torch.cuda.current_stream(device).cuda_stream
+        self.tiles, self.stream = {}, None
+        if plan.tiles:                   # (key, transposed) -> tiles, and the stream that makes them
+            self.tiles, self.stream = self._make_tiles(), torch.cuda.current_stream(device).cuda_stream
 
     def _make_tiles(self) -> dict:
         maps = {}

@@ -202,3 +202,26 @@ def test_levels_of_a_full_block(size):
             assert out.C.equal(expected)
             assert net[0](x).C.equal(torch.unique(torch.div(coordinates, 2, rounding_mode="floor") * 2, dim=0))
             cache.reset()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_a_planned_pass_without_tiles_asks_nothing_about_them(dtype, monkeypatch):
+    """Neither which stream is current nor what tiles would have saved: each is a
+    microsecond or more of a layer that takes thirty with its map."""
+    c, _ = sorted_unique(random_cloud(3000, 20, 5, lo=-9), None)
+    conv = minuet.nn.SparseConv3d(32, 32, 3, dtype=dtype, device="cuda")
+    cache = minuet.nn.KernelMapCache(3, torch.int32, "cuda")
+    conv.set_kernel_map_cache(cache)
+    x = minuet.SparseTensor(torch.randn(c.shape[0], 32, device="cuda").to(dtype), dev(c))
+    with torch.no_grad():
+        first = conv(x).F
+        for _ in range(2):
+            cache.reset()
+            assert torch.equal(conv(x).F, first)
+        calls = []
+        monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: calls.append("stream"))
+        monkeypatch.setattr(type(cache), "_note_tiles", lambda *a: calls.append("tiles"))
+        cache.reset()
+        assert torch.equal(conv(x).F, first) and cache._built is not None
+        cache.reset()
+        assert not calls
