@@ -304,20 +304,38 @@ void compact_forward(const float *sources, const float *weights, bool lanes, con
   const int ki = static_cast<int>(div_ceil(K, 16 * s.chunks));
   const bool whole = K == 16 * ki * s.chunks;
   // Targets, channel blocks and wavefronts of a workgroup by how many workgroups
-  // of 64 targets and 16 channels there are to a compute unit: small clouds need
-  // small workgroups to reach the whole chip, beyond that two blocks share the
-  // source rows.  Over 360 layers (three kinds of scene, 3x3x3 and strided
-  // 2x2x2, 48 to 40 000 targets, 16 to 256 channels) these lines cost 3.6 % on
-  // average over the best of 15 shapes for each (us: 256 -> 256 channels over 135
-  // targets 16 targets x 16 channels 15.9, 32 x 32 32; 128 -> 128 over 658 16 x 32
-  // 13.1, 16 x 16 16.5, 32 x 32 19.5; 64 -> 64 over 2 900 32 x 32 13.0, 64 x 16
-  // 14; 128 -> 128 over 3 600 64 x 32 22, 64 x 16 25.9).  Four blocks are worth it for
-  // weights as [O][K][N] only (8 -> 128 over 160 000 135 against 148).
+  // of 64 targets and 16 channels there are to a compute unit (`full`): small
+  // clouds need small workgroups to reach the whole chip, beyond that two blocks
+  // share the source rows.  With one step of 16 input channels a workgroup is its
+  // map and its sums, and 32 targets are enough at any size; not for many targets
+  // and weights as [O][K][N], of which four blocks read whole lines.  Those have
+  // one block up to three workgroups, since a second doubles the loads of their
+  // weights (in lanes it does not).  `split` is the same for both forms of the
+  // weights, whose sums are then the same bit for bit.
+  //
+  // Over 1 057 layers of three kinds of scene (3x3x3 and strided 2x2x2, 130 to
+  // 580 000 targets, 4 to 256 channels) the form before there were two, and its
+  // lines, took 1.14 times as long as weights in lanes do and 1.05 times as long
+  // as [O][K][N] (the best of 14 shapes for each layer: 0.96 and 0.95 of these
+  // lines).  us, that form and here, lanes: 256 -> 256 channels over 130 targets
+  // 19.7 / 12.8, 128 -> 128 over 2 980 46 / 33, 8 -> 128 over 40 000 27.6 / 26.5;
+  // [O][K][N]: 64 -> 64 over 3 000 10.4 / 8.7 (two blocks 10.9), 128 -> 128 over
+  // 3 000 20.2 / 19.4 (22.0).  What two blocks cost is layers with few hits, whose
+  // blocks of rows are nearly empty, which the host cannot know: 96 -> 256 over
+  // 2 000 of a LiDAR scan 13.7 / 16.5 and, with one block, 13.7; where a target
+  // has 13 hits 35 / 26 and 32.
   const int64_t cus = compute_units(), cols = div_ceil(N, int64_t{16});
   const double full = static_cast<double>(div_ceil(Tn, int64_t{64}) * cols) / static_cast<double>(cus);
-  int c = 1, targets = 64, split = full < 2.25 ? 8 : 4;
+  int c = 1, targets = 64, split = full < 1.95 ? 8 : 4;
   if (N % 32 != 0) {
     targets = full < 0.3 ? 16 : full < 0.9 ? 32 : 64;
+    split = full < 2.25 ? 8 : 4;
+  } else if (K <= 16 && full >= 0.93 && (lanes || full < 4.75)) {
+    c = 2;
+    targets = 32;
+    split = full < 3.0 ? 8 : 4;
+  } else if (!lanes && K >= 32 && full < 3.0) {
+    targets = full < 0.26 ? 16 : full < 0.6 ? 32 : 64;
   } else if (full < 0.6) {
     c = full >= 0.26 && full < 0.42 ? 2 : 1;
     targets = full < 0.42 ? 16 : 32;
@@ -327,7 +345,6 @@ void compact_forward(const float *sources, const float *weights, bool lanes, con
   } else {
     c = full >= 4.75 && N % 64 == 0 ? 4 : 2;
     targets = full >= 1.95 && full < 3.0 ? 32 : 64;
-    split = full < 1.95 ? 8 : 4;
   }
   s.steps = static_cast<int>(div_ceil(K, int64_t{16}));
   // Columns side by side, so that the workgroups of a die share few of them and
@@ -377,11 +394,7 @@ void compact_forward(const float *sources, const float *weights, bool lanes, con
   } else if (targets == 16) {
     MNT_COMPACT_K(1, 8, 16)
   } else if (targets == 32) {
-    if (split == 8) {
-      MNT_COMPACT_K(1, 8, 32)
-    } else {
-      MNT_COMPACT_K(1, 4, 32)
-    }
+    MNT_COMPACT_K(1, 8, 32)
   } else if (split == 8) {
     MNT_COMPACT_K(1, 8, 64)
   } else {

@@ -44,6 +44,21 @@ def test_lane_order_is_the_same_product(targets, offsets, K, N):
     assert lanes.equal(plain)
 
 
+# 0.9, 1, 1.9, 2, 2.9, 3, 4.7 and 4.8 workgroups of 64 targets and 16 channels to each of 256 compute units:
+# both sides of every line of the layers with one step of 16 channels, and of [O][K][N] ones
+@pytest.mark.parametrize("targets", [3790, 4100, 7800, 8200, 11900, 12300, 19300, 19700])
+@pytest.mark.parametrize("offsets, K, N", [(27, 8, 64), (8, 16, 64), (27, 32, 64), (2, 80, 64)])
+def test_lane_order_at_the_lines_between_shapes(targets, offsets, K, N):
+    dense, x, w = _case(targets, offsets, K, N, 0.2, targets + K)
+    expected = _oracle(dense, x, w)
+    dense, x, w = dense.cuda(), x.cuda(), w.cuda()
+    plain = _C.sparse_convolution_forward_implicit(x, w, dense)
+    lanes = _C.sparse_convolution_forward_implicit(x, w, dense, packed_weights=_C.pack_weights_in_lanes(w))
+    # as above; the density is of the whole map, single targets have up to all offsets
+    assert (plain.cpu().double() - expected).abs().max() < 8 * 2.0 ** -24 * (offsets * K / 0.2) ** 0.5
+    assert lanes.equal(plain)
+
+
 @pytest.mark.parametrize("activation", [None, "relu"])
 def test_lane_order_epilogue(activation):
     dense, x, w = (t.cuda() for t in _case(333, 27, 48, 72, 0.4, 5))
