@@ -615,6 +615,15 @@ int mnt_sparse_convolution_forward_in_lanes(const float *sources, const float *p
                                             const float *channel_shift, const void *residual, int activation,
                                             float negative_slope, float *out, void *stream);
 
+/* The latter without a kernel map on weights as they are, [pieces, Cin / pieces,
+ * Cout] and so [Cin, Cout]: fp32 rows [N, Cin] of few, for 1x1x1 layers; the same
+ * bit for bit.  num_source_features: of a piece. */
+int mnt_sparse_convolution_forward_pieces(const float *sources, const float *weights, int64_t num_rows,
+                                          int64_t num_pieces, int64_t num_source_features,
+                                          int64_t num_target_features, const float *channel_scale,
+                                          const float *channel_shift, const void *residual, int activation,
+                                          float negative_slope, float *out, void *stream);
+
 /* 1 where mnt_sparse_convolution_forward_implicit (and _tiled) streams rows and
  * weights of a layer of the given shape through LDS, which makes it the faster
  * one for 16-bit layers too wide for the others. */

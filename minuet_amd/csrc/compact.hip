@@ -39,7 +39,10 @@ struct CompactShape {
 // same whenever it is computed.
 //
 // LANES: the weights come in the order of the instruction's lanes (pack_lanes),
-// one load of 1 KB where [O][K][N] takes four of 256 or 512 bytes.
+// one load of 1 KB where [O][K][N] takes four of 256 or 512 bytes.  For callers
+// that keep such a copy: a layer's weights are read where they are, because a
+// copy would miss what is written through .data or before a graph's replay
+// (which costs 8 % on average over 226 layers).
 //
 // What bounds it: on small clouds one wavefront's chain of map entry, source
 // rows, products (the unit after is asked for before one is multiplied), hence

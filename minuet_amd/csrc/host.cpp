@@ -49,8 +49,8 @@ using TablesFn = int (*)(int64_t, int64_t, int, int64_t, int, double, const void
                          int, float, const void *, const int64_t *, void *, void *);
 using TiledFn = int (*)(const void *, const void *, const int32_t *, int64_t, int64_t, int64_t, int64_t, int64_t, int,
                         const float *, const float *, const void *, int, float, void *, void *);
-using LanesFn = int (*)(const void *, const void *, const int32_t *, int64_t, int64_t, int64_t, int64_t, int64_t,
-                        const float *, const float *, const void *, int, float, void *, void *);
+using PiecesFn = int (*)(const void *, const void *, int64_t, int64_t, int64_t, int64_t, const float *, const float *,
+                         const void *, int, float, void *, void *);
 using TilesFn = int (*)(const int32_t *, int64_t, int64_t, int32_t *, void *);
 using TilesSizeFn = int (*)(int64_t, int64_t, int64_t *);
 using TilesShareFn = double (*)(int64_t, int64_t, int64_t, int64_t, int);
@@ -60,7 +60,7 @@ ImplicitFn g_implicit = nullptr;
 GroupsFn g_groups = nullptr;
 TablesFn g_tables = nullptr;
 TiledFn g_tiled = nullptr;
-LanesFn g_lanes = nullptr;
+PiecesFn g_pieces = nullptr;
 TiledFn g_single = nullptr;
 TilesFn g_tiles = nullptr;
 TilesSizeFn g_tiles_size = nullptr;
@@ -279,7 +279,6 @@ struct Layer {
   PyObject *shape_id;                         // key of this layer's map inside the cache's _fast_maps
   PyObject *dataflow, *threshold, *gather_tile, *scatter_tile;
   int kind, float_code, device;
-  int in_lanes;                               // packed is in lane order (fp32)
   int shortcut, has_threshold;
   double threshold_value;
   int64_t gather_tile_value, scatter_tile_value;
@@ -372,7 +371,6 @@ PyObject *layer_new(PyTypeObject *type, PyObject *args, PyObject *) {
   l->num_offsets = w->size(0);
   l->in_channels = w->size(1);
   l->out_channels = w->size(2);
-  l->in_lanes = tensor_of(packed)->dim() == 5 ? 1 : 0;
   l->has_threshold = l->threshold == Py_None ? 0 : 1;
   l->threshold_value = l->has_threshold ? PyFloat_AsDouble(l->threshold) : 0.0;
   l->gather_tile_value = l->gather_tile == Py_None ? 0 : PyLong_AsLongLong(l->gather_tile);
@@ -605,12 +603,6 @@ PyObject *run_layer(Layer *l, PyObject *module_dict, PyObject *inputs, const Epi
   int status = 0;
   switch (l->kind) {
     case kImplicit:
-      if (l->in_lanes) {
-        status = g_lanes(source, packed_at, static_cast<const int32_t *>(map->at[0]), S, T, l->num_offsets,
-                         l->in_channels, l->out_channels, scale_at, shift_at, data(residual), ep.activation, ep.slope,
-                         out.mutable_data_ptr(), stream);
-        break;
-      }
       if (l->shortcut != 0) {                              // a target has one source
         status = g_single(source, packed_at, static_cast<const int32_t *>(map->at[0]), S, T, l->num_offsets,
                           l->in_channels, l->out_channels, l->float_code, scale_at, shift_at, data(residual),
@@ -646,8 +638,8 @@ PyObject *run_layer(Layer *l, PyObject *module_dict, PyObject *inputs, const Epi
     case kPieces: {
       // the input channels in pieces, which the wavefronts of a workgroup share
       const int64_t pieces = THPVariable_Unpack(l->packed).size(0);
-      status = g_lanes(source, packed_at, nullptr, S * pieces, S, pieces, l->in_channels / pieces, l->out_channels,
-                       scale_at, shift_at, data(residual), ep.activation, ep.slope, out.mutable_data_ptr(), stream);
+      status = g_pieces(source, weights_at, S, pieces, l->in_channels / pieces, l->out_channels, scale_at, shift_at,
+                        data(residual), ep.activation, ep.slope, out.mutable_data_ptr(), stream);
       break;
     }
     default:
@@ -869,7 +861,7 @@ PyObject *py_bind(PyObject *, PyObject *args) {
   g_groups = reinterpret_cast<GroupsFn>(address("mnt_sparse_convolution_forward_groups"));
   g_tables = reinterpret_cast<TablesFn>(address("mnt_sparse_convolution_forward_fused"));
   g_tiled = reinterpret_cast<TiledFn>(address("mnt_sparse_convolution_forward_tiled"));
-  g_lanes = reinterpret_cast<LanesFn>(address("mnt_sparse_convolution_forward_in_lanes"));
+  g_pieces = reinterpret_cast<PiecesFn>(address("mnt_sparse_convolution_forward_pieces"));
   g_single = reinterpret_cast<TiledFn>(address("mnt_sparse_convolution_forward_single"));
   g_tiles = reinterpret_cast<TilesFn>(address("mnt_kernel_map_tiles"));
   g_tiles_size = reinterpret_cast<TilesSizeFn>(address("mnt_kernel_map_tiles_size"));

@@ -697,37 +697,58 @@ extern "C" int mnt_sparse_convolution_forward_implicit(
   });
 }
 
+// The forward that multiplies hits only, on weights of `weight_floats` values in
+// lane order (`lanes`) or as [O, Cin, Cout].
+static void forward_hits(const float *sources, const float *weights, bool lanes, int64_t weight_floats,
+                         const int32_t *kernel_map, int64_t S, int64_t T, int64_t O, int64_t K, int64_t N,
+                         const Epilogue &ep, float *out, hipStream_t stream) {
+  MNT_CHECK(S * K * 4 < static_cast<int64_t>(kMaxSourceBytes) &&
+                weight_floats * 4 < static_cast<int64_t>(kMaxSourceBytes),
+            "source features or weights exceed the 4 GiB a buffer resource addresses");
+  MNT_CHECK(K % 4 == 0 && K * 4 <= kImplicitMaxRowBytes && N % 4 == 0 &&
+                N <= 32 * kImplicitMaxBlocks * kImplicitMaxGroups,
+            "Unsupported channel counts for a forward of hits: Cin = %lld (a multiple of 4, at most %d), "
+            "Cout = %lld (a multiple of 4, at most %d)",
+            (long long)K, kImplicitMaxRowBytes / 4, (long long)N, 32 * kImplicitMaxBlocks * kImplicitMaxGroups);
+  MNT_CHECK(ep.activation >= MNT_ACT_NONE && ep.activation <= MNT_ACT_RELU6, "unknown activation code %d",
+            ep.activation);
+  MNT_CHECK(reinterpret_cast<uintptr_t>(sources) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0 &&
+                reinterpret_cast<uintptr_t>(ep.residual) % 16 == 0 && reinterpret_cast<uintptr_t>(weights) % 16 == 0 &&
+                reinterpret_cast<uintptr_t>(ep.scale) % 4 == 0 && reinterpret_cast<uintptr_t>(ep.shift) % 4 == 0,
+            "operands are not aligned (features, out, residual, weights: 16 bytes, scale / shift: 4 bytes)");
+  if (T == 0) return;
+  MNT_CHECK(out != nullptr && weights != nullptr, "null operand");
+  MNT_CHECK(kernel_map != nullptr || S == T * O, "without a kernel map a target has a source under every offset");
+  profile_mark("enter:implicit", stream);
+  compact_forward(sources, weights, lanes, kernel_map, S, T, O, K, N, ep, out, stream);
+  profile_mark("implicit", stream);
+}
+
 extern "C" int mnt_sparse_convolution_forward_in_lanes(
     const float *sources, const float *packed_weights, const int32_t *kernel_map, int64_t S, int64_t T, int64_t O,
     int64_t K, int64_t N, const float *channel_scale, const float *channel_shift, const void *residual, int activation,
     float negative_slope, float *out, void *stream_) {
   return guarded([&] {
-    hipStream_t stream = static_cast<hipStream_t>(stream_);
     MNT_CHECK(S >= 0 && T >= 0 && O > 1 && K >= 1 && N >= 1 && S <= INT32_MAX && T <= INT32_MAX && O <= 65535,
               "bad shape S=%lld T=%lld O=%lld Cin=%lld Cout=%lld", (long long)S, (long long)T, (long long)O,
               (long long)K, (long long)N);
-    MNT_CHECK(S * K * 4 < static_cast<int64_t>(kMaxSourceBytes) &&
-                  lane_weight_floats(O, K, N) * 4 < static_cast<int64_t>(kMaxSourceBytes),
-              "source features or weights exceed the 4 GiB a buffer resource addresses");
-    MNT_CHECK(K % 4 == 0 && K * 4 <= kImplicitMaxRowBytes && N % 4 == 0 &&
-                  N <= 32 * kImplicitMaxBlocks * kImplicitMaxGroups,
-              "Unsupported channel counts for weights in lane order: Cin = %lld (a multiple of 4, at most %d), "
-              "Cout = %lld (a multiple of 4, at most %d)",
-              (long long)K, kImplicitMaxRowBytes / 4, (long long)N, 32 * kImplicitMaxBlocks * kImplicitMaxGroups);
-    MNT_CHECK(activation >= MNT_ACT_NONE && activation <= MNT_ACT_RELU6, "unknown activation code %d", activation);
-    MNT_CHECK(reinterpret_cast<uintptr_t>(sources) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0 &&
-                  reinterpret_cast<uintptr_t>(residual) % 16 == 0 &&
-                  reinterpret_cast<uintptr_t>(packed_weights) % 16 == 0 &&
-                  reinterpret_cast<uintptr_t>(channel_scale) % 4 == 0 &&
-                  reinterpret_cast<uintptr_t>(channel_shift) % 4 == 0,
-              "operands are not aligned (features, out, residual, weights: 16 bytes, scale / shift: 4 bytes)");
-    if (T == 0) return;
-    MNT_CHECK(out != nullptr && packed_weights != nullptr, "null operand");
-    MNT_CHECK(kernel_map != nullptr || S == T * O, "without a kernel map a target has a source under every offset");
     const Epilogue ep = {channel_scale, channel_shift, residual, activation, negative_slope, nullptr};
-    profile_mark("enter:implicit", stream);
-    compact_forward(sources, packed_weights, true, kernel_map, S, T, O, K, N, ep, out, stream);
-    profile_mark("implicit", stream);
+    forward_hits(sources, packed_weights, true, lane_weight_floats(O, K, N), kernel_map, S, T, O, K, N, ep, out,
+                 static_cast<hipStream_t>(stream_));
+  });
+}
+
+extern "C" int mnt_sparse_convolution_forward_pieces(
+    const float *sources, const float *weights, int64_t rows, int64_t pieces, int64_t K, int64_t N,
+    const float *channel_scale, const float *channel_shift, const void *residual, int activation,
+    float negative_slope, float *out, void *stream_) {
+  return guarded([&] {
+    MNT_CHECK(rows >= 0 && pieces > 1 && pieces <= 65535 && K >= 1 && N >= 1 && rows <= INT32_MAX / pieces,
+              "bad shape N=%lld pieces=%lld Cin=%lld Cout=%lld", (long long)rows, (long long)pieces,
+              (long long)(pieces * K), (long long)N);
+    const Epilogue ep = {channel_scale, channel_shift, residual, activation, negative_slope, nullptr};
+    forward_hits(sources, weights, false, pieces * K * N, nullptr, rows * pieces, rows, pieces, K, N, ep, out,
+                 static_cast<hipStream_t>(stream_));
   });
 }
 

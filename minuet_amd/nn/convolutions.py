@@ -618,7 +618,6 @@ class SparseConv(Module):
         factory = {"device": device, "dtype": dtype}
         volume = int(np.prod(self.kernel_size))
         self._packed = None
-        self._lanes = None
         self._fast = None
         self.kernel = torch.nn.Parameter(torch.empty(volume, in_channels, out_channels, **factory))
         if bias:
@@ -695,7 +694,6 @@ class SparseConv(Module):
         nothing, so call this after them (``reset_parameters``, ``load_state_dict``
         and ``.to()`` / ``.half()`` / ``.cuda()`` do it themselves)."""
         self._packed = None
-        self._lanes = None
         self._fast = None
 
     def _load_from_state_dict(self, *args, **kwargs):
@@ -849,26 +847,6 @@ class SparseConv(Module):
                 self._packed = (key, weights, F.pack_weights(weights), held)
         return self._packed[1], self._packed[2]
 
-    def _lane_kernel(self, pieces: int = 1):
-        """``_packed_kernel`` of an fp32 layer that multiplies hits only, whose
-        kernel reads the weights in the order of its lanes (16 x 16 x 4 instructions
-        take them 1 KB at a load: 32 -> 32 channels over 200 000 voxels 55 and 50
-        us, 128 -> 64 over 2 900 27 and 21).  ``pieces``: a pointwise layer's,
-        its input channels cut into that many "offsets"."""
-        kernel = self.kernel
-        if pieces > 1:
-            kernel = kernel.view(pieces, self.in_channels // pieces, self.out_channels)
-        if ((torch.is_grad_enabled() and kernel.requires_grad) or kernel.is_inference()
-                or not _C.lane_weights_supported(kernel)):
-            return self._packed_kernel()
-        key = (kernel.data_ptr(), kernel._version, kernel.dtype, kernel.device)
-        kept = self.__dict__.get("_lanes")          # (none in a module pickled before there were any)
-        if kept is None or kept[0] != key:
-            with torch.no_grad():
-                weights = kernel.detach()
-                kept = self._lanes = (key, weights, _C.pack_weights_in_lanes(weights))
-        return kept[1], kept[2]
-
     def _row_padding(self, features: torch.Tensor) -> int:
         """Zero input channels to append so that the feature rows of a 16-bit
         layer become ones the single-kernel dataflow takes (4 or 8 bytes under
@@ -945,16 +923,16 @@ class SparseConv(Module):
             # wider layers of many rows are plain library GEMM territory
             narrow = (_C.implicit_forward_supported(self.in_channels, self.out_channels, weights.dtype)
                       and self.in_channels * weights.dtype.itemsize <= 512 and self.out_channels <= 128)
-            # (what torch.mm would otherwise make follows autocast, and a kernel made in
-            # inference mode says nothing of writes to it: no packed copy can be kept)
+            # (what torch.mm would otherwise make follows autocast)
             most = (F.pieces_rows_limit(self.in_channels, self.out_channels, weights.dtype)
-                    if dataflow == "auto" and not kernel.is_inference()
-                    and (narrow or not torch.is_autocast_enabled()) else -1)
+                    if dataflow == "auto" and kernel.is_contiguous() and kernel.data_ptr() % 16 == 0
+                    and not kernel.is_inference() and (narrow or not torch.is_autocast_enabled()) else -1)
             rows = (most + 1, _MOST_ROWS) if most >= 0 else ()
             if 0 < features.shape[0] <= most and features.is_contiguous():
-                whole, packed = self._lane_kernel(F.channel_pieces(self.in_channels))
-                out = _C.sparse_convolution_forward_pieces(features, packed, self.out_channels, epilogue=epilogue)
-                return out, ("PIECES", whole.view(weights.shape), packed, None, None, 0, None, not narrow), (0, most)
+                whole = kernel.detach()
+                pieces = whole.view(F.channel_pieces(self.in_channels), -1, self.out_channels)
+                out = _C.sparse_convolution_forward_pieces(features, pieces, self.out_channels, epilogue=epilogue)
+                return out, ("PIECES", whole, pieces, None, None, 0, None, not narrow), (0, most)
             count, far = features.shape[0], F.implicit_rows_limit(self.in_channels, weights.dtype)
             if narrow and count <= far:
                 identity = self._identity_map
@@ -1060,7 +1038,7 @@ class SparseConv(Module):
                 dense = cache.get_dense_kernel_map(**map_args)
                 if pad:
                     sources = torch.nn.functional.pad(sources, (0, pad))
-                weights, packed = self._packed_kernel(pad) if not hits else self._lane_kernel()
+                weights, packed = self._packed_kernel(pad)
                 tiles = None
                 single = packed is not None and self._has_single_sources(sources)
                 if packed is not None and not hits and not single and F.prefers_streamed(volume, sources.shape[1], self.out_channels, sources.dtype):

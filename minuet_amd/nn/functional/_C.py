@@ -115,6 +115,8 @@ SIGNATURES = {
     "mnt_pack_weights_in_lanes": (_int, [_vp, _i64, _i64, _i64, _vp, _vp]),
     "mnt_sparse_convolution_forward_in_lanes": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _vp, _vp, _vp,
                                                        _int, ctypes.c_float, _vp, _vp]),
+    "mnt_sparse_convolution_forward_pieces": (_int, [_vp, _vp, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _int,
+                                                     ctypes.c_float, _vp, _vp]),
     "mnt_sparse_convolution_streamed": (_int, [_i64, _i64, _i64, _i64, _int]),
     "mnt_sparse_convolution_forward_tiled": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _vp, _vp, _vp,
                                                     _int, ctypes.c_float, _vp, _vp]),
@@ -198,7 +200,7 @@ def _bound_host():
     spec.loader.exec_module(module)
     names = ("mnt_sparse_convolution_forward_implicit", "mnt_sparse_convolution_forward_groups",
              "mnt_sparse_convolution_forward_fused", "mnt_sparse_convolution_forward_tiled", "mnt_kernel_map_tiles",
-             "mnt_sparse_convolution_forward_in_lanes", "mnt_sparse_convolution_forward_single",
+             "mnt_sparse_convolution_forward_pieces", "mnt_sparse_convolution_forward_single",
              "mnt_kernel_map_tiles_size", "mnt_kernel_map_tiles_share", "mnt_last_error")
     hooks = tuple(getattr(torch_module, name) for name in (
         "_global_forward_hooks", "_global_forward_pre_hooks", "_global_backward_hooks",
@@ -1555,28 +1557,36 @@ MOST_TILE_ENTRIES = 1 << 29                      # (offset, target) pairs of a m
 
 def sparse_convolution_forward_pieces(sources: torch.Tensor, packed_weights: torch.Tensor, num_target_features: int,
                                       epilogue: Optional[Epilogue] = None) -> torch.Tensor:
-    """fp32 ``sources [N, C_in] @ weights [C_in, C_out]`` for few rows, the weights as
-    :func:`pack_weights_in_lanes` of ``weights.view(pieces, C_in / pieces, C_out)``."""
+    """fp32 ``sources [N, C_in] @ weights [C_in, C_out]`` for few rows, from
+    ``weights.view(pieces, C_in / pieces, C_out)`` or its :func:`pack_weights_in_lanes`."""
     _ensure_ndim("sources", sources, 2)
-    _ensure_ndim("packed_weights", packed_weights, 5)
+    lanes = packed_weights.dim() == 5
+    if not lanes:
+        _ensure_ndim("packed_weights", packed_weights, 3)
     device = _common_device([sources, packed_weights])
-    if sources.dtype != torch.float32 or packed_weights.dtype != torch.float32 or not packed_weights.is_contiguous():
+    if (sources.dtype != torch.float32 or packed_weights.dtype != torch.float32 or not packed_weights.is_contiguous()
+            or packed_weights.data_ptr() % 16):
         _fail("the forward in pieces expects contiguous fp32 tensors")
     rows, channels = sources.shape
-    pieces, blocks, steps = packed_weights.shape[:3]
-    N = num_target_features
-    if (channels % pieces or -(-(channels // pieces) // 16) != steps or tuple(packed_weights.shape[3:]) != (64, 4)
-            or -(-N // 16) != blocks):
+    pieces, N = packed_weights.shape[0], num_target_features
+    if channels % pieces:
+        _fail("packed_weights does not belong to these sources")
+    of_piece = channels // pieces
+    if tuple(packed_weights.shape[1:]) != ((-(-N // 16), -(-of_piece // 16), 64, 4) if lanes else (of_piece, N)):
         _fail("packed_weights does not belong to these sources")
     if not sources.is_contiguous() or sources.data_ptr() % 16:
         sources = sources.contiguous().clone()
     out = torch.empty((rows, N), dtype=sources.dtype, device=device)
     ep = Epilogue() if epilogue is None else epilogue.checked(rows, N, sources.dtype, device)
+    finish = (_ptr(ep.scale), _ptr(ep.shift), _ptr(ep.residual), ACTIVATION_CODES[ep.activation],
+              float(ep.negative_slope), _ptr(out), _stream(device))
     with _on(device):
-        _check(load_library().mnt_sparse_convolution_forward_in_lanes(
-            _ptr(sources), _ptr(packed_weights), None, rows * pieces, rows, pieces, channels // pieces, N,
-            _ptr(ep.scale), _ptr(ep.shift), _ptr(ep.residual), ACTIVATION_CODES[ep.activation],
-            float(ep.negative_slope), _ptr(out), _stream(device)))
+        if lanes:
+            _check(load_library().mnt_sparse_convolution_forward_in_lanes(
+                _ptr(sources), _ptr(packed_weights), None, rows * pieces, rows, pieces, of_piece, N, *finish))
+        else:
+            _check(load_library().mnt_sparse_convolution_forward_pieces(
+                _ptr(sources), _ptr(packed_weights), rows, pieces, of_piece, N, *finish))
     return out
 
 

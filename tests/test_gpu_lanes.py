@@ -69,21 +69,45 @@ def test_lane_order_epilogue(activation):
     assert lanes.equal(plain)
 
 
-def test_lane_weights_follow_the_parameter():
+# hits only, of three kinds of map; the channels in pieces, wider than the library's product was left for either way
+@pytest.mark.parametrize("cin, cout, size, stride, transposed", [
+    (32, 32, 3, 1, False), (64, 128, 2, 2, False), (64, 32, 2, 2, True), (256, 128, 1, 1, False), (64, 256, 1, 1, False)])
+def test_layers_read_the_parameter_itself(cin, cout, size, stride, transposed):
+    """A write through ``.data`` leaves no mark on the parameter, one of the caller's
+    before a replay none that a captured pass could see."""
     coordinates = torch.unique(torch.randint(0, 12, (900, 3), generator=torch.Generator().manual_seed(1),
                                              dtype=torch.int32), dim=0).cuda()
     coordinates = coordinates[F.build_sorted_index(coordinates)]
-    conv = minuet.nn.SparseConv3d(32, 32, 3, device="cuda")
-    conv.set_kernel_map_cache(minuet.nn.KernelMapCache(ndim=3, dtype=torch.int32, device="cuda"))
-    x = minuet.SparseTensor(torch.randn(len(coordinates), 32, device="cuda"), coordinates)
+    cache = minuet.nn.KernelMapCache(ndim=3, dtype=torch.int32, device="cuda")
+    conv = minuet.nn.SparseConv(3, cin, cout, size, stride=stride, transposed=transposed, device="cuda")
+    conv.set_kernel_map_cache(cache)
+    x = minuet.SparseTensor(torch.randn(len(coordinates), cin, device="cuda"), coordinates)
     with torch.no_grad():
+        if transposed:
+            down = minuet.nn.SparseConv3d(cin, cin, size, stride=stride, device="cuda")
+            down.set_kernel_map_cache(cache)
+            x = down(x)
         first = conv(x).F.clone()
-        lanes = conv._lanes[2]
-        assert conv(x).F.equal(first) and conv._lanes[2] is lanes      # (and past Python)
+        assert conv(x).F.equal(first)                                  # (and past Python)
         conv.kernel.mul_(2.0)                                          # in place: same storage, new version
-        assert conv(x).F.equal(2 * first) and conv._lanes[2] is not lanes
         assert conv(x).F.equal(2 * first)
-    assert conv(x).F.detach().equal(2 * first)                         # gradients are recorded: as they are
+        assert conv(x).F.equal(2 * first)
+        conv.kernel.data.mul_(2.0)                                     # same storage, same version
+        assert conv(x).F.equal(4 * first)
+        conv._fast = None
+        conv.kernel.data.mul_(2.0)
+        assert conv(x).F.equal(8 * first)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = conv(x).F
+        for _ in range(3):
+            conv.kernel.mul_(0.5)
+            out.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert out.equal(conv(x).F)
+        assert out.equal(first)
+    assert conv(x).F.detach().allclose(first, rtol=0, atol=2e-5)       # gradients are recorded: as they are
 
 
 def test_refuses_another_layer_s_weights():
@@ -105,10 +129,14 @@ def test_pointwise_layer_in_pieces(rows, K, N):
     pieces = F.channel_pieces(K)
     packed = _C.pack_weights_in_lanes(w.view(pieces, K // pieces, N).cuda())
     got = _C.sparse_convolution_forward_pieces(x.cuda(), packed, N, _C.Epilogue(residual=residual.cuda())).cpu()
+    plain = w.view(pieces, K // pieces, N).cuda()
+    assert got.cuda().equal(_C.sparse_convolution_forward_pieces(x.cuda(), plain, N, _C.Epilogue(residual=residual.cuda())))
     expected = x.double() @ w.double() + residual.double()
     assert (got.double() - expected).abs().max() < 8 * 2.0 ** -24 * K ** 0.5
     with pytest.raises((RuntimeError, ValueError)):
         _C.sparse_convolution_forward_pieces(x.cuda(), packed, N + 16)
+    with pytest.raises((RuntimeError, ValueError)):
+        _C.sparse_convolution_forward_pieces(x.cuda(), plain, N + 4)
 
 
 def test_pointwise_layer_takes_pieces_by_its_rows():
