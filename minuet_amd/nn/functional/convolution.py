@@ -116,16 +116,22 @@ def channel_pieces(num_source_features: int) -> int:
 def pieces_rows_limit(num_source_features: int, num_target_features: int, dtype: torch.dtype) -> int:
     """The most rows over which ``dataflow="auto"`` cuts an fp32 pointwise layer into
     pieces (-1: over none).  They let a workgroup's wavefronts share a row, and
-    every 16 rows read the weights again, so that the line lies at 200 million
-    rows x input x output channels: us against the kernel for one offset 128 -> 64
-    over 2 900 rows 4.7 / 13.0, over 12 000 7.4 / 13.2, over 30 000 12.8 / 12.5,
-    64 -> 32 over 60 000 11.9 / 12.4, 128 -> 128 over 12 000 12.4 / 18.5, over
-    30 000 22.7 / 20.3; against the library and an output pass of its own 256 ->
-    128 over 660 4.9 / 38, over 8 200 13.4 / 36."""
+    every 16 rows read the weights again.  Where the kernel for one offset takes
+    the layer otherwise (up to 128 channels, in and out) the line lies at 1.2
+    million rows x output channels, which is when there are more workgroups than
+    the chip holds: us there and in pieces 128 -> 128 over 700 rows 14.3 / 4.5, 96
+    -> 128 over 9 000 12.6 / 8.6, 80 -> 48 over 20 000 8.1 / 7.8, over 26 000 8.3 /
+    9.1, 96 -> 64 over 30 000 8.9 / 11.9, 64 -> 32 over 60 000 7.7 / 11.1.  Against
+    the library and an output pass of its own it lies at 200 million rows x input
+    x output channels: 256 -> 32 over 700 22 / 4.8, 256 -> 128 over 4 500 21.5 / 12.7,
+    160 -> 128 over 9 000 22 / 13.3."""
     if (dtype != torch.float32 or num_source_features % 16 != 0 or num_source_features < 48
             or not _C.implicit_forward_supported(num_source_features, num_target_features, dtype)):
         return -1
-    return 200_000_000 // (num_source_features * num_target_features)
+    most = 200_000_000 // (num_source_features * num_target_features)
+    if num_source_features <= 128 and num_target_features <= 128:
+        most = min(most, 1_200_000 // num_target_features)
+    return most
 
 
 def prefers_hits(num_offsets: int, num_source_features: int, num_target_features: int, dtype: torch.dtype,

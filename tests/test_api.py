@@ -189,6 +189,15 @@ def test_fp32_rule_follows_the_kernel_size():
     assert prefers(125, 32, 32, single, 100000)
 
 
+# (channels, rows) where cutting the channels was measured slower than one offset, and where faster
+@pytest.mark.parametrize("cin, cout, slower, faster", [
+    (64, 32, 60000, 30000), (96, 64, 30000, 8000), (48, 128, 20000, 4500), (80, 48, 30000, 20000), (96, 128, 20000, 9000),
+    (256, 32, None, 9000), (160, 128, None, 9000), (48, 256, None, 9000)])
+def test_pointwise_layers_are_cut_where_that_is_faster(cin, cout, slower, faster):
+    most = minuet.nn.functional.pieces_rows_limit(cin, cout, torch.float32)
+    assert faster <= most and (slower is None or most < slower)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
 def test_rows_that_the_single_kernel_form_addresses(dtype):
     limit = minuet.nn.functional.implicit_rows_limit
