@@ -52,7 +52,7 @@ def prefers_implicit(num_offsets: int, num_source_features: int, num_target_feat
 def prefers_streamed(num_offsets: int, num_source_features: int, num_target_features: int,
                      dtype: torch.dtype) -> bool:
     """Whether ``dataflow="auto"`` takes the single-kernel form for a layer too wide
-    for ``prefers_implicit``: 16-bit rows of 136 to 512 bytes (or of 72 and more
+    for ``prefers_implicit``: 16-bit rows of 144 to 512 bytes (or of 80 and more
     under more than 128 output channels), whose rows and weights stream through
     LDS.  Against three kernels or offset groups, us a layer: 128 -> 128 channels
     over 6 850 voxels 23.0 and 11.8, over 18 600 of a LiDAR level 27.7 and 17.3,
@@ -61,8 +61,13 @@ def prefers_streamed(num_offsets: int, num_source_features: int, num_target_feat
     offsets, which have four stages an offset and few product bytes to save: 256 ->
     64 over 23 100 24.2 and 30.7, 256 -> 96 over 10 400 21.6 and 26.2, 256 -> 32 over
     18 800 19.5 and 27.7 (the other way round over few voxels, 256 -> 32 over 2 300
-    22.6 and 16.9; 192 -> 64 over 22 000 24.0 and 24.0, over 13 800 19.7 and 15.9)."""
-    if num_offsets > 8 and num_source_features > 192 and num_target_features <= 96:
+    22.6 and 16.9; 192 -> 64 over 22 000 24.0 and 24.0, over 13 800 19.7 and 15.9).
+    Nor more than 27 offsets, most of which a target has no source under and which
+    are walked all the same: 4x4x4 and 5x5x5, 256 -> 128 over 9 000 of a scan 29 and
+    94, 192 -> 224 over 20 000 of a room 73 and 203, 192 -> 64 over 26 000 23 and 49,
+    128 -> 128 over 40 000 66 and 99 (96 -> 128 over 4 000 28 and 19; over 79 layers,
+    with tiles and without, 1.2 times as long)."""
+    if num_offsets > 27 or (num_offsets > 8 and num_source_features > 192 and num_target_features <= 96):
         return False
     return _C.streamed_forward_supported(num_offsets, num_source_features, num_target_features, dtype)
 

@@ -123,7 +123,7 @@ def test_network_without_the_extension_module(monkeypatch):
 @pytest.mark.parametrize("cin,cout,size,stride,transposed,dtype", [
     (128, 128, 3, 1, False, torch.float16), (256, 128, 3, 1, False, torch.bfloat16),
     (128, 256, 2, 2, False, torch.float16), (128, 64, 2, 2, True, torch.float16), (64, 64, 3, 1, False, torch.float16),
-    (100, 96, 5, 1, False, torch.float16), (30, 32, 3, 1, False, torch.float16), (64, 64, 1, 1, False, torch.float16),
+    (96, 64, 5, 1, False, torch.float16), (30, 32, 3, 1, False, torch.float16), (64, 64, 1, 1, False, torch.float16),
     (32, 64, 1, 1, False, torch.float32), (32, 32, 1, 2, False, torch.float32), (64, 32, 3, 1, False, torch.float32)])
 def test_features_past_the_single_kernel_form(cin, cout, size, stride, transposed, dtype, monkeypatch):
     """Features of 4 GiB and more run as if there were no such form, before and
