@@ -875,7 +875,9 @@ class SparseConv(Module):
         if dataflow == "implicit":
             return True
         shape = (self.kernel.shape[0], self.in_channels + pad, self.out_channels, features.dtype)
-        return F.prefers_implicit(*shape) or F.prefers_streamed(*shape)
+        # (a copy of the rows, which every call makes, is more than streaming saves: 100 -> 64
+        # channels over 2 000 voxels 14.6 us in three kernels and 26.7, 150 -> 160 over 9 000 34.9 and 48.1)
+        return F.prefers_implicit(*shape) or (pad == 0 and F.prefers_streamed(*shape))
 
     def _has_single_sources(self, features: torch.Tensor) -> bool:
         """Whether a target of this layer has one source, and the kernel for that

@@ -132,3 +132,11 @@ def test_a_layer_gives_the_same_rows_from_call_to_call():
 def test_which_wide_layers_are_streamed(cin, cout, offsets, streams):
     """Both sides of the line between streaming and grouped products."""
     assert F.prefers_streamed(offsets, cin, cout, torch.float16) == streams
+
+
+@pytest.mark.parametrize("cin,streams", [(96, True), (100, False), (104, True), (150, False), (254, False), (256, True)])
+def test_rows_that_need_padding_are_not_streamed(cin, streams):
+    conv = minuet.nn.SparseConv3d(cin, 128, 3, dtype=torch.float16, device=DEVICE)
+    features = torch.empty(1, cin, dtype=torch.float16, device=DEVICE)
+    pad = conv._row_padding(features)
+    assert (pad == 0) == streams and conv._takes_implicit(features, pad) == streams
