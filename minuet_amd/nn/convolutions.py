@@ -1042,10 +1042,14 @@ class SparseConv(Module):
                     sources = torch.nn.functional.pad(sources, (0, pad))
                 weights, packed = self._packed_kernel(pad)
                 tiles = None
-                single = packed is not None and self._has_single_sources(sources)
-                if packed is not None and not hits and not single and F.prefers_streamed(volume, sources.shape[1], self.out_channels, sources.dtype):
+                single = not hits and self._has_single_sources(sources)
+                if (not hits and not single
+                        and F.prefers_streamed(volume, sources.shape[1], self.out_channels, sources.dtype)):
                     tiles = cache.get_tiles(dense, sources.shape[1], self.out_channels, sources.dtype, inputs.C,
                                             inputs.stride, stride, self.kernel_size, self.dilation, self.transposed)
+                kept = packed
+                if packed is None and (single or tiles is not None):
+                    packed = F.pack_weights(weights)            # (as the others do on their way)
                 if single:
                     features = _C.sparse_convolution_forward_single(sources, weights, dense, packed, epilogue=epilogue)
                 elif tiles is not None:
@@ -1056,7 +1060,7 @@ class SparseConv(Module):
                                                                       epilogue=epilogue,
                                                                       packed_weights=packed)
                 if not pad and dense.is_contiguous():
-                    made = ("IMPLICIT", weights, packed, (dense.data_ptr(),), dense, 0, tiles, single)
+                    made = ("IMPLICIT", weights, kept, (dense.data_ptr(),), dense, 0, tiles, single)
             else:
                 features, made = self._forward_tables(cache, map_args, sources, epilogue)
         if bias is not None:

@@ -140,3 +140,30 @@ def test_rows_that_need_padding_are_not_streamed(cin, streams):
     features = torch.empty(1, cin, dtype=torch.float16, device=DEVICE)
     pad = conv._row_padding(features)
     assert (pad == 0) == streams and conv._takes_implicit(features, pad) == streams
+
+
+# in tiles, and with one source a target
+@pytest.mark.parametrize("transposed", [False, True])
+def test_layers_that_record_gradients_run_the_same_kernels(transposed, monkeypatch):
+    from helpers import random_cloud, sorted_unique, dev
+    c, _ = sorted_unique(random_cloud(12000, 40, 3, lo=-9), None)
+    cache = minuet.nn.KernelMapCache(3, torch.int32, DEVICE)
+    conv = minuet.nn.SparseConv(3, 256, 192, 2 if transposed else 3, stride=2 if transposed else 1, transposed=transposed,
+                                dtype=torch.bfloat16, device=DEVICE)
+    conv.set_kernel_map_cache(cache)
+    x = minuet.SparseTensor(torch.randn(c.shape[0], 256, device=DEVICE).bfloat16(), dev(c))
+    with torch.no_grad():
+        if transposed:
+            down = minuet.nn.SparseConv3d(256, 256, 2, stride=2, dtype=torch.bfloat16, device=DEVICE)
+            down.set_kernel_map_cache(cache)
+            x = down(x)
+        wanted = conv(x).F
+    name = "sparse_convolution_forward_" + ("single" if transposed else "tiled")
+    whole, calls = getattr(_C, name), []
+    monkeypatch.setattr(_C, name, lambda *args, **options: calls.append(1) or whole(*args, **options))
+    for _ in range(2):
+        assert torch.equal(conv(x).F.detach(), wanted)
+    assert len(calls) == 2
+    with torch.no_grad():
+        conv.kernel.mul_(2.0)
+    assert torch.equal(conv(x).F.detach(), 2 * wanted)
