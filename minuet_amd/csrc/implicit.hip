@@ -784,10 +784,13 @@ extern "C" int mnt_sparse_convolution_streamed(int64_t T, int64_t O, int64_t K, 
 // What tiles (mnt_kernel_map_tiles) would save of one forward, over what making
 // them takes; 0 where they do not pay or cannot be used.
 // Layers of streamed_forward_kernel take 28 us for them at once where its
-// workgroups are more than twice the compute units: a map of a network is read
+// workgroups (of 128 targets and 64 channels, from 65 channels on of 64 and 128)
+// are more than the compute units and, without tiles, a second round of them
+// would walk every offset again: a map of a network is read
 // four to eight times (us without and with, 128 -> 128 channels over 18 600
 // targets of a LiDAR level 29.8 and 17.3, 256 -> 256 over 8 700 37 and 27, over
-// 25 600 of a scan 77 and 37; over 9 000, 128 -> 128: 15.2 and 13.4).
+// 25 600 of a scan 77 and 37; over 9 000, 160 -> 160 37 and 20, 256 -> 160 of an
+// object 48 and 28; 128 -> 128 over as many, one round, 15.2 and 13.4).
 // Others: fitted to layers of
 // 32 to 128 channels over 100 000 to a million targets: a forward gets faster by
 // 1.3 us per million (offset, target) pairs and unit of (channel blocks + 1) x
@@ -799,7 +802,8 @@ extern "C" double mnt_kernel_map_tiles_share(int64_t T, int64_t O, int64_t K, in
     return 0.0;
   }
   if (streamed_takes(T, O, K, N)) {
-    return div_ceil(T, 64) * div_ceil(N, 64) > 2 * static_cast<int64_t>(compute_units()) ? 2.0 : 0.0;
+    const int64_t columns = N <= 64 ? 1 : 2 * div_ceil(N, 128);
+    return div_ceil(T, 64) * columns > 2 * static_cast<int64_t>(compute_units()) ? 2.0 : 0.0;
   }
   // Below, the kernel without tiles is about as fast, and it adds up in another
   // order: a layer's results do not change from one call to the next.

@@ -167,3 +167,11 @@ def test_layers_that_record_gradients_run_the_same_kernels(transposed, monkeypat
     with torch.no_grad():
         conv.kernel.mul_(2.0)
     assert torch.equal(conv(x).F.detach(), 2 * wanted)
+
+
+# one round of workgroups on 256 compute units, and two
+@pytest.mark.parametrize("cout,most", [(32, 32768), (64, 32768), (96, 16384), (128, 16384), (160, 8192), (256, 8192),
+                                       (320, 5440)])
+def test_tiles_from_the_second_round_of_workgroups_on(cout, most):
+    worth = lambda targets: _C.kernel_map_tiles_worth_making(targets, 27, 192, cout, torch.float16)
+    assert not worth(most) and worth(most + 64)
