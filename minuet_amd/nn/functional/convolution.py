@@ -66,9 +66,26 @@ def prefers_streamed(num_offsets: int, num_source_features: int, num_target_feat
     are walked all the same: 4x4x4 and 5x5x5, 256 -> 128 over 9 000 of a scan 29 and
     94, 192 -> 224 over 20 000 of a room 73 and 203, 192 -> 64 over 26 000 23 and 49,
     128 -> 128 over 40 000 66 and 99 (96 -> 128 over 4 000 28 and 19; over 79 layers,
-    with tiles and without, 1.2 times as long)."""
-    if num_offsets > 27 or (num_offsets > 8 and num_source_features > 192 and num_target_features <= 96):
+    with tiles and without, 1.2 times as long).
+
+    Nor fp16 rows of more than 384 bytes under more than 128 channels of which the
+    workgroups' last 128 are half empty, or with a fourth stage that is half empty
+    itself (in bf16 the other forms take longer): 256 -> 160 over 26 000 with
+    dilation 2 31 and 39, 224 -> 144 over 60 000 62 and 102, 224
+    -> 192 over 20 000 31 and 39, 208 -> 160 of 12 000 21 and 25, 224 -> 256 of
+    8 000 23 and 28; over 30 such layers 1.1 times as long.
+
+    What stays slower: fp16 layers of few sources a target just before they get
+    tiles (160 -> 128 over 12 000 of a LiDAR scan 17.2 and 20.3), and strided layers
+    of many targets whose map is kept for many calls (256 -> 256 onto 35 000 30 and 50).
+    On new clouds, where the other forms have rank tables to build, those take 0.67
+    times as long (of 209 the slowest two 1.12, 256 -> 256 onto 35 000 103 and 92)."""
+    if num_offsets > 27:
         return False
+    if num_offsets > 8 and num_source_features > 192:
+        half_empty = num_source_features <= 224 or (num_target_features - 1) % 128 < 64
+        if num_target_features <= 96 or (dtype == torch.float16 and num_target_features > 128 and half_empty):
+            return False
     return _C.streamed_forward_supported(num_offsets, num_source_features, num_target_features, dtype)
 
 

@@ -125,10 +125,11 @@ def test_a_layer_gives_the_same_rows_from_call_to_call():
             assert torch.equal(out, first)
 
 
-@pytest.mark.parametrize("cin,cout,offsets,streams", [(256, 96, 27, False), (256, 104, 27, True), (200, 96, 9, False),
-                                                      (192, 96, 27, True), (256, 32, 8, True), (128, 128, 27, True),
-                                                      (128, 128, 36, False), (256, 128, 64, False),
-                                                      (192, 224, 125, False)])
+@pytest.mark.parametrize("cin,cout,offsets,streams", [
+    (256, 96, 27, False), (256, 104, 27, True), (200, 96, 9, False), (192, 96, 27, True), (256, 32, 8, True),
+    (128, 128, 27, True), (128, 128, 36, False), (256, 128, 64, False), (192, 224, 125, False),
+    (256, 192, 27, False), (256, 200, 27, True), (192, 160, 27, True), (224, 256, 27, False), (232, 256, 27, True),
+    (224, 128, 27, True), (256, 320, 27, False), (224, 256, 8, True)])
 def test_which_wide_layers_are_streamed(cin, cout, offsets, streams):
     """Both sides of the line between streaming and grouped products."""
     assert F.prefers_streamed(offsets, cin, cout, torch.float16) == streams
