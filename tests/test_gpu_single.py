@@ -28,10 +28,10 @@ def _oracle(dense, x, w):
     return out
 
 
-# workgroups of 128 targets, of one that is not full, of a share of the chip, of the most there are
-@pytest.mark.parametrize("targets", [1, 127, 129, 5000, 90001, 300007])
+# workgroups of 128 targets, of one that is not full, of a share of the chip in one round and in several
+@pytest.mark.parametrize("targets", [1, 127, 129, 5000, 60000, 90001, 300007])
 @pytest.mark.parametrize("K, N, dtype", [(72, 8, torch.float16), (128, 64, torch.float16), (136, 40, torch.bfloat16),
-                                         (256, 128, torch.bfloat16), (200, 72, torch.float16)])
+                                         (256, 128, torch.bfloat16), (200, 72, torch.float16), (160, 144, torch.float16)])
 @pytest.mark.parametrize("double", [0.0, 0.001])
 def test_one_source_a_target(targets, K, N, dtype, double):
     """(Targets with two sources are not what the kernel is for, and right all the same.)"""
