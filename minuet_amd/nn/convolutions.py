@@ -32,6 +32,11 @@ _MOST_ROWS = (1 << 63) - 1
 # to go on (so that a size that wavers does not change the plan every time).
 # Five maps take 49 us together and 137 one by one.
 _TILES_PAY, _TILES_STAY = 0.75, 0.5
+# Targets x output channels up to which a layer that records gradients, and so
+# packs its weights at every call, does without the kernel for one source a
+# target: packing is a call of its own there, 4 us of the 18 that the host takes
+# (96 -> 64 channels over 40 000 targets 18.3 and, with it, 22.4).
+_FEW_VALUES = 4_000_000
 _TRANSPOSED_FIRST = ("Layer must transpose=True must have its corresponding non-transposed layer "
                      "before its execution")
 
@@ -879,11 +884,11 @@ class SparseConv(Module):
         # channels over 2 000 voxels 14.6 us in three kernels and 26.7, 150 -> 160 over 9 000 34.9 and 48.1)
         return F.prefers_implicit(*shape) or (pad == 0 and F.prefers_streamed(*shape))
 
-    def _has_single_sources(self, features: torch.Tensor) -> bool:
+    def _has_single_sources(self, features: torch.Tensor, pad: int = 0) -> bool:
         """Whether a target of this layer has one source, and the kernel for that
         takes the layer: the transposed layers whose kernel is their stride."""
         return (self.transposed and self.kernel_size == self.stride and all(d == 1 for d in self.dilation)
-                and _C.single_forward_supported(self.kernel.shape[0], features.shape[1], self.out_channels,
+                and _C.single_forward_supported(self.kernel.shape[0], features.shape[1] + pad, self.out_channels,
                                                 features.dtype))
 
     def _takes_offset_groups(self, features: torch.Tensor, streamed: bool = True) -> bool:
@@ -915,12 +920,12 @@ class SparseConv(Module):
         kernel = self.kernel
         weights = kernel.view(1, self.in_channels, self.out_channels)
         dataflow = self._tunable_config.get("dataflow", "auto")
-        operands = [features, kernel]
-        if epilogue is not None:
-            operands += [t for t in (epilogue.scale, epilogue.shift, epilogue.residual) if t is not None]
         rows = ()
-        if (features.is_cuda and features.dtype == weights.dtype
-                and dataflow not in ("gather_gemm_scatter", "list_driven") and _C.plain(operands)):
+        if (features.is_cuda and not (torch.is_grad_enabled() and (kernel.requires_grad or features.requires_grad))
+                and features.dtype == weights.dtype and dataflow not in ("gather_gemm_scatter", "list_driven")
+                and _C.plain([features, kernel] if epilogue is None else
+                             [t for t in (features, kernel, epilogue.scale, epilogue.shift, epilogue.residual)
+                              if t is not None])):
             # measured against torch.mm plus a separate epilogue pass up to these widths;
             # wider layers of many rows are plain library GEMM territory
             narrow = (_C.implicit_forward_supported(self.in_channels, self.out_channels, weights.dtype)
@@ -1013,16 +1018,22 @@ class SparseConv(Module):
                 rows = (0, most) if hits else (most + 1, _MOST_ROWS)
             route_key = (sources.dtype, sources.is_cuda, dataflow, hits)
             route = self._routes.get(route_key)
-            if route is None:
+            if route is None or len(route) != 6:    # (fewer in a module that an older version has saved)
                 grouped = self._takes_offset_groups(sources)
                 pad = 0 if grouped else self._row_padding(sources)
                 implicit = self._takes_implicit(sources, pad) if hits is None else hits
-                route = (pad, not grouped and implicit, grouped, None)
-                if hits is None and route[1] and dataflow == "auto":
+                implicit = implicit and not grouped
+                single = tiled = False
+                most = None
+                if implicit and not hits:
+                    single = self._has_single_sources(sources, pad)
+                    tiled = not single and F.prefers_streamed(volume, self.in_channels + pad, self.out_channels,
+                                                              sources.dtype)
+                if hits is None and implicit and dataflow == "auto":
                     # (where its features are past what that form addresses: as if there were no such form)
-                    route = (*route[:3], F.implicit_rows_limit(self.in_channels + pad, sources.dtype))
-                self._routes[route_key] = route
-            pad, implicit, grouped, most = route
+                    most = F.implicit_rows_limit(self.in_channels + pad, sources.dtype)
+                route = self._routes[route_key] = (pad, implicit, grouped, most, single, tiled)
+            pad, implicit, grouped, most, single, tiled = route
             if most is not None:
                 rows = (0, most)
                 if sources.shape[0] > most:
@@ -1042,12 +1053,13 @@ class SparseConv(Module):
                     sources = torch.nn.functional.pad(sources, (0, pad))
                 weights, packed = self._packed_kernel(pad)
                 tiles = None
-                single = not hits and self._has_single_sources(sources)
-                if (not hits and not single
-                        and F.prefers_streamed(volume, sources.shape[1], self.out_channels, sources.dtype)):
+                kept = packed
+                if packed is None and single and dense.shape[1] * self.out_channels <= _FEW_VALUES:
+                    single = False
+                if tiled and (packed is not None or _C.kernel_map_tiles_worth_making(
+                        dense.shape[1], volume, sources.shape[1], self.out_channels, sources.dtype)):
                     tiles = cache.get_tiles(dense, sources.shape[1], self.out_channels, sources.dtype, inputs.C,
                                             inputs.stride, stride, self.kernel_size, self.dilation, self.transposed)
-                kept = packed
                 if packed is None and (single or tiles is not None):
                     packed = F.pack_weights(weights)            # (as the others do on their way)
                 if single:

@@ -11,6 +11,7 @@ There is no CPU or eager fallback: without the built library nothing works.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 from typing import Optional, Sequence, Tuple
 
@@ -1638,6 +1639,7 @@ def sparse_convolution_forward_single(sources: torch.Tensor, weights: torch.Tens
     return out
 
 
+@functools.lru_cache(maxsize=1024)
 def kernel_map_tiles_worth_making(num_targets: int, num_offsets: int, num_source_features: int,
                                   num_target_features: int, dtype: torch.dtype) -> bool:
     """Whether a layer of this shape makes the tiles of its map at its first call."""

@@ -147,7 +147,7 @@ def test_rows_that_need_padding_are_not_streamed(cin, streams):
 @pytest.mark.parametrize("transposed", [False, True])
 def test_layers_that_record_gradients_run_the_same_kernels(transposed, monkeypatch):
     from helpers import random_cloud, sorted_unique, dev
-    c, _ = sorted_unique(random_cloud(12000, 40, 3, lo=-9), None)
+    c, _ = sorted_unique(random_cloud(70000, 48, 3, lo=-9), None)
     cache = minuet.nn.KernelMapCache(3, torch.int32, DEVICE)
     conv = minuet.nn.SparseConv(3, 256, 192, 2 if transposed else 3, stride=2 if transposed else 1, transposed=transposed,
                                 dtype=torch.bfloat16, device=DEVICE)
