@@ -31,6 +31,7 @@
 #include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <memory>
 
@@ -189,68 +190,126 @@ void map_entry_dealloc(PyObject *self) {
   Py_TYPE(self)->tp_free(self);
 }
 
-PyObject *map_entry_new(PyTypeObject *type, PyObject *args, PyObject *) {
-  PyObject *coordinates, *stride, *batch_dims, *keep, *pointers;
+PyObject *hold(PyObject *o) {
+  Py_INCREF(o);
+  return o;
+}
+
+void swap_in(PyObject *&held, PyObject *o) {
+  PyObject *before = held;
+  held = hold(o);
+  Py_XDECREF(before);
+}
+
+// Tiles that the current stream of the map's device has made; false with a
+// Python error.
+bool take_tiles(MapEntry *e, PyObject *tiles) {
+  if (tensor_of(tiles) == nullptr) {
+    PyErr_SetString(PyExc_TypeError, "tiles are a tensor");
+    return false;
+  }
+  try {
+    const c10::hip::HIPStream stream = c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(e->device));
+    std::unique_ptr<at::cuda::CUDAEvent> made(new at::cuda::CUDAEvent());
+    made->record(c10::hip::HIPStreamMasqueradingAsCUDA(stream));
+    e->tiles_stream = stream.stream();
+    e->tiles_made = made.release();
+  } catch (const std::exception &error) {
+    PyErr_SetString(PyExc_RuntimeError, error.what());
+    return false;
+  }
+  e->tiles = hold(tiles);
+  return true;
+}
+
+struct MapArgs {
+  PyObject *coordinates, *stride, *batch_dims, *keep, *tiles;
   int kind, device, index_code;
   long long num_sources, num_targets;
-  unsigned long long built_from = 0;
-  PyObject *tiles = Py_None;                  // those the current stream of `device` has made already
-  if (!PyArg_ParseTuple(args, "iOOOOiiLLO!|KO", &kind, &coordinates, &stride, &batch_dims, &keep, &device, &index_code,
-                        &num_sources, &num_targets, &PyTuple_Type, &pointers, &built_from, &tiles)) {
-    return nullptr;
+  unsigned long long built_from;
+  const void *at[8];
+};
+
+bool parse_map(PyObject *args, MapArgs *a) {
+  PyObject *pointers;
+  a->built_from = 0;
+  a->tiles = Py_None;                         // those the current stream of `device` has made already
+  if (!PyArg_ParseTuple(args, "iOOOOiiLLO!|KO", &a->kind, &a->coordinates, &a->stride, &a->batch_dims, &a->keep,
+                        &a->device, &a->index_code, &a->num_sources, &a->num_targets, &PyTuple_Type, &pointers,
+                        &a->built_from, &a->tiles)) {
+    return false;
   }
-  std::unique_ptr<at::cuda::CUDAEvent> made;
-  void *made_on = nullptr;
-  if (tiles != Py_None) {
-    if (tensor_of(tiles) == nullptr) {
-      PyErr_SetString(PyExc_TypeError, "tiles are a tensor");
-      return nullptr;
-    }
-    try {
-      const c10::hip::HIPStream stream = c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(device));
-      made_on = stream.stream();
-      made.reset(new at::cuda::CUDAEvent());
-      made->record(c10::hip::HIPStreamMasqueradingAsCUDA(stream));
-    } catch (const std::exception &error) {
-      PyErr_SetString(PyExc_RuntimeError, error.what());
-      return nullptr;
-    }
-  }
-  MapEntry *e = reinterpret_cast<MapEntry *>(type->tp_alloc(type, 0));
-  if (e == nullptr) return nullptr;
-  auto hold = [](PyObject *o) {
-    Py_INCREF(o);
-    return o;
-  };
-  e->coordinates = hold(coordinates);
-  e->stride = hold(stride);
-  e->batch_dims = hold(batch_dims);
-  e->keep = hold(keep);
-  e->kind = kind;
-  e->device = device;
-  e->index_code = index_code;
-  e->num_sources = num_sources;
-  e->num_targets = num_targets;
-  e->built_from = reinterpret_cast<const void *>(static_cast<uintptr_t>(built_from));
-  e->used = 0;
-  e->tiles = tiles == Py_None ? nullptr : hold(tiles);
-  e->tiles_credit = 0.0;
-  e->tiles_saved = 0.0;
-  e->tiles_stream = made_on;
-  e->tiles_made = made.release();
-  e->tiles_ready = 0;
   for (Py_ssize_t i = 0; i < 8; ++i) {
-    e->at[i] = nullptr;
+    a->at[i] = nullptr;
     if (i < PyTuple_GET_SIZE(pointers) && !is_none(PyTuple_GET_ITEM(pointers, i))) {
-      e->at[i] = PyLong_AsVoidPtr(PyTuple_GET_ITEM(pointers, i));
+      a->at[i] = PyLong_AsVoidPtr(PyTuple_GET_ITEM(pointers, i));
     }
   }
-  if (PyErr_Occurred()) {
+  return PyErr_Occurred() == nullptr;
+}
+
+PyObject *map_entry_new(PyTypeObject *type, PyObject *args, PyObject *) {
+  MapArgs a;
+  if (!parse_map(args, &a)) return nullptr;
+  MapEntry *e = reinterpret_cast<MapEntry *>(type->tp_alloc(type, 0));       // (all zeros)
+  if (e == nullptr) return nullptr;
+  e->coordinates = hold(a.coordinates);
+  e->stride = hold(a.stride);
+  e->batch_dims = hold(a.batch_dims);
+  e->keep = hold(a.keep);
+  e->kind = a.kind;
+  e->device = a.device;
+  e->index_code = a.index_code;
+  e->num_sources = a.num_sources;
+  e->num_targets = a.num_targets;
+  e->built_from = reinterpret_cast<const void *>(static_cast<uintptr_t>(a.built_from));
+  std::copy(a.at, a.at + 8, e->at);
+  if (a.tiles != Py_None && !take_tiles(e, a.tiles)) {
     Py_DECREF(e);
     return nullptr;
   }
   return reinterpret_cast<PyObject *>(e);
 }
+
+// renew(the constructor's arguments): this entry as the constructor would make
+// it, but with its tiles and what is known about them; False, and nothing done,
+// where it is of another map.
+PyObject *map_entry_renew(PyObject *self, PyObject *args) {
+  MapEntry *e = reinterpret_cast<MapEntry *>(self);
+  MapArgs a;
+  if (!parse_map(args, &a)) return nullptr;
+  if (e->kind != a.kind || e->device != a.device || e->index_code != a.index_code ||
+      e->num_sources != a.num_sources || e->num_targets != a.num_targets || !std::equal(a.at, a.at + 8, e->at)) {
+    Py_RETURN_FALSE;
+  }
+  if (a.tiles != Py_None && e->tiles == nullptr && !take_tiles(e, a.tiles)) return nullptr;
+  swap_in(e->coordinates, a.coordinates);
+  swap_in(e->stride, a.stride);
+  swap_in(e->batch_dims, a.batch_dims);
+  swap_in(e->keep, a.keep);
+  e->built_from = reinterpret_cast<const void *>(static_cast<uintptr_t>(a.built_from));
+  Py_RETURN_TRUE;
+}
+
+// tiles_of(address, stream): the tiles of the map at that address, if this entry
+// has them and that stream made them.
+PyObject *map_entry_tiles_of(PyObject *self, PyObject *args) {
+  MapEntry *e = reinterpret_cast<MapEntry *>(self);
+  unsigned long long address, stream;
+  if (!PyArg_ParseTuple(args, "KK", &address, &stream)) return nullptr;
+  if (e->tiles == nullptr || reinterpret_cast<uintptr_t>(e->at[0]) != address ||
+      reinterpret_cast<uintptr_t>(e->tiles_stream) != stream) {
+    Py_RETURN_NONE;
+  }
+  return hold(e->tiles);
+}
+
+PyObject *py_reduce(PyObject *, PyObject *);
+
+PyMethodDef map_entry_methods[] = {{"__reduce__", py_reduce, METH_NOARGS, "Copies as None."},
+                                   {"renew", map_entry_renew, METH_VARARGS, "Describes the same map anew."},
+                                   {"tiles_of", map_entry_tiles_of, METH_VARARGS, "The tiles a stream has made."},
+                                   {nullptr, nullptr, 0, nullptr}};
 
 PyObject *map_entry_used(PyObject *self, void *) {
   return PyBool_FromLong(reinterpret_cast<MapEntry *>(self)->used);
@@ -906,7 +965,7 @@ bool ready(PyTypeObject &type, const char *name, size_t size, destructor dealloc
   type.tp_flags = Py_TPFLAGS_DEFAULT;
   type.tp_dealloc = dealloc;
   type.tp_new = make;
-  type.tp_methods = object_methods;
+  if (type.tp_methods == nullptr) type.tp_methods = object_methods;
   return PyType_Ready(&type) == 0;
 }
 
@@ -917,6 +976,7 @@ PyMODINIT_FUNC PyInit_minuet_host() {
   MNT_NAMES(MNT_INTERN)
 #undef MNT_INTERN
   MapEntryType.tp_getset = map_entry_getset;
+  MapEntryType.tp_methods = map_entry_methods;
   if (!ready(MapEntryType, "minuet_host.MapEntry", sizeof(MapEntry), map_entry_dealloc, map_entry_new) ||
       !ready(LayerType, "minuet_host.Layer", sizeof(Layer), layer_dealloc, layer_new) ||
       !ready(AffineType, "minuet_host.Affine", sizeof(Affine), affine_dealloc, affine_new)) {

@@ -442,32 +442,37 @@ class KernelMapCache(object):
 
     def get_tiles(self, dense: torch.Tensor, in_channels: int, out_channels: int, dtype: torch.dtype,
                   source_coordinates: torch.Tensor, source_stride, target_stride, kernel_size, kernel_dilation,
-                  transposed: bool = False) -> Optional[torch.Tensor]:
+                  transposed: bool = False, entry=None) -> Optional[torch.Tensor]:
         """The tiles of the dense kernel map ``dense``, for a wide layer of these
         channels that makes them at its first call (None where it runs without).
-        Not in the reference, whose map has one order of targets."""
+        ``entry``: what the extension module keeps of the map, which may have got
+        them from narrower layers.  Not in the reference, whose map has one order
+        of targets."""
         if torch.cuda.is_current_stream_capturing():
             return None
         key = (self._map_key(source_coordinates.shape[1], source_stride, target_stride, kernel_size, kernel_dilation,
                              transposed)[0], "tiles", transposed)
         stream = torch.cuda.current_stream(dense.device).cuda_stream
-        entry = self._offset_groups_cache.get(key)
-        if not entry and self._built is not None:
+        tiles = entry.tiles_of(dense.data_ptr(), stream) if entry is not None else None
+        if tiles is not None:
+            return tiles
+        kept = self._offset_groups_cache.get(key)
+        if not kept and self._built is not None:
             tiles = self._built.tiles_of(key[0], transposed, dense)
             if tiles is not None:
-                entry = self._offset_groups_cache[key] = (tiles, self._built.stream)
-        if not entry:                        # (a wider layer of the same map may want them)
-            entry = False
+                kept = self._offset_groups_cache[key] = (tiles, self._built.stream)
+        if not kept:                         # (a wider layer of the same map may want them)
+            kept = False
             offsets, targets = dense.shape
             if (dense.is_contiguous() and offsets * targets <= _C.MOST_TILE_ENTRIES
                     and _C.kernel_map_tiles_worth_making(targets, offsets, in_channels, out_channels, dtype)):
                 try:
-                    entry = (_C.kernel_map_tiles(dense), stream)
+                    kept = (_C.kernel_map_tiles(dense), stream)
                 except torch.OutOfMemoryError:
                     pass
-            self._offset_groups_cache[key] = entry
+            self._offset_groups_cache[key] = kept
         # (another stream owes nothing to the one that made them: the same rows without)
-        return entry[0] if entry and entry[1] == stream else None
+        return kept[0] if kept and kept[1] == stream else None
 
     def _inverse_of(self, key) -> torch.Tensor:
         """Dense map of the transposed layer of ``key`` ([O, S]), made on first use."""
@@ -1059,7 +1064,8 @@ class SparseConv(Module):
                 if tiled and (packed is not None or _C.kernel_map_tiles_worth_making(
                         dense.shape[1], volume, sources.shape[1], self.out_channels, sources.dtype)):
                     tiles = cache.get_tiles(dense, sources.shape[1], self.out_channels, sources.dtype, inputs.C,
-                                            inputs.stride, stride, self.kernel_size, self.dilation, self.transposed)
+                                            inputs.stride, stride, self.kernel_size, self.dilation, self.transposed,
+                                            self._map_entry("IMPLICIT", inputs.stride)[1])
                 if packed is None and (single or tiles is not None):
                     packed = F.pack_weights(weights)            # (as the others do on their way)
                 if single:
@@ -1083,6 +1089,15 @@ class SparseConv(Module):
             self._keep_fast(made, rows, inputs, features, coordinates, stride, batch_dims)
         return SparseTensor.like(inputs, features, coordinates, stride, batch_dims)
 
+    def _map_entry(self, name: str, stride):
+        """The shape under which the extension module finds this layer's map, and
+        what it keeps of the one for inputs of that stride (None: nothing)."""
+        host = _C.load_host()
+        if host is None:
+            return None, None
+        shape_id = (getattr(host, name), self.kernel_size, self.stride, self.dilation, self.transposed)
+        return shape_id, self._kernel_map_cache._fast_maps.get(shape_id, {}).get(stride)
+
     def _keep_fast(self, made, rows, inputs, features, coordinates, stride, batch_dims):
         """Leaves what this call worked out for the extension module: the module's
         side of it in ``_fast``, the map's side in the cache's ``_fast_maps``.
@@ -1097,11 +1112,13 @@ class SparseConv(Module):
         kind = getattr(host, name)
         shape_id = None
         if pointers is not None:
-            shape_id = (kind, self.kernel_size, self.stride, self.dilation, self.transposed)
-            entry = host.MapEntry(kind, coordinates, stride, batch_dims, owners, features.device.index, index_code,
-                                  inputs.F.shape[0], features.shape[0], pointers, 0, tiles)
             cache = self._kernel_map_cache
-            cache._fast_maps.setdefault(shape_id, {})[inputs.stride] = entry
+            shape_id, entry = self._map_entry(name, inputs.stride)
+            described = (kind, coordinates, stride, batch_dims, owners, features.device.index, index_code,
+                         inputs.F.shape[0], features.shape[0], pointers, 0, tiles)
+            # (layers of the same map, whatever their widths, share its tiles)
+            if entry is None or not entry.renew(*described):
+                cache._fast_maps.setdefault(shape_id, {})[inputs.stride] = host.MapEntry(*described)
             key = cache._map_key(self.ndim, inputs.stride, stride, self.kernel_size, self.dilation, self.transposed)[0]
             cache._note_fast(("fast", shape_id, inputs.stride, name, key, self.transposed))
         parameters = self._parameters

@@ -308,3 +308,42 @@ def operands_of(dense):
     gen = torch.Generator(device=DEVICE).manual_seed(1)
     return (torch.randn(700, 32, generator=gen, device=DEVICE).half(),
             torch.randn(dense.shape[0], 32, 32, generator=gen, device=DEVICE).half())
+
+
+@pytest.mark.parametrize("first", ["wide", "narrow"])
+def test_layers_of_one_map_make_its_tiles_once(first):
+    """Whichever asks for them, and whichever of the others describes the map to the
+    extension module after that."""
+    cells = torch.randperm(1 << 18, generator=torch.Generator().manual_seed(4))[:70000].cuda()
+    coordinates = torch.stack([cells >> 12, (cells >> 6) & 63, cells & 63], 1).int()
+    coordinates = coordinates[F.build_sorted_index(coordinates)]
+    cache = minuet.nn.KernelMapCache(3, torch.int32, "cuda")
+    layers = {width: minuet.nn.SparseConv3d(width, width, 3, dtype=torch.float16, device="cuda") for width in (128, 64, 32)}
+    inputs = {width: minuet.SparseTensor(torch.randn(len(coordinates), width, device="cuda").half(), coordinates)
+              for width in layers}
+    for layer in layers.values():
+        layer.set_kernel_map_cache(cache)
+    with torch.no_grad():
+        def run(width):
+            return layers[width](inputs[width]).F.double().sum().item()
+        wanted = {}
+        for width in (128, 64) if first == "wide" else (64, 128):
+            wanted[width] = run(width)
+            for _ in range(30):
+                run(width)
+        entry, = (entry for maps in cache._fast_maps.values() for entry in maps.values())
+        saved = entry.tiles_saved
+        assert saved > 0
+        torch.cuda.synchronize()
+        before = torch.cuda.memory_allocated()
+        for _ in range(3):
+            for width in (128, 64):
+                assert run(width) == wanted[width]
+        run(32)                                              # (describes the map once more)
+        weights = torch.cuda.memory_allocated() - before
+        for _ in range(30):
+            for width in (128, 64, 32):
+                run(width)
+        assert torch.cuda.memory_allocated() - before <= weights < 1 << 20       # (tiles take 8 MB)
+        kept, = (entry for maps in cache._fast_maps.values() for entry in maps.values())
+        assert kept is entry and kept.tiles_saved > saved
