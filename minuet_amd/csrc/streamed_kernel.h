@@ -15,6 +15,8 @@ namespace mnt {
 
 typedef int int4v __attribute__((ext_vector_type(4)));
 
+constexpr int kStreamedStage = 128;            // bytes of a row
+constexpr int kStreamedLoaders = 4;            // wavefronts of a workgroup that load
 constexpr unsigned kPastEnd = 0xFFFFF000u;     // past the end of every source buffer: reads zeros
 
 struct StreamedShape {
@@ -56,8 +58,8 @@ __device__ __forceinline__ void wait_loads() {
 }
 __device__ __forceinline__ void meet() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// A workgroup of MW x NW x KW wavefronts that multiply and NL that load takes TM
-// targets and TN output channels; a stage is BK bytes of the source rows and of
+// A workgroup of MW x NW x KW wavefronts that multiply and four that load takes TM
+// targets and TN output channels; a stage is 128 bytes of the source rows and of
 // the weights under one offset, CH stages an offset, RING of them in LDS.
 //
 // Those that load ask for stage L as soon as all have read stage L - RING, and
@@ -86,14 +88,14 @@ __device__ __forceinline__ void meet() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts
 // where sums are not finite the workgroup starts again, and every target keeps
 // what it has under an offset that it has no source under (the same sums
 // wherever those are finite): a test per stage instead cost 15 % of it.
-template <typename T, int MW, int NW, int KW, int WM, int WN, int NL, int BK, int CH, int RING, bool TILED>
-__global__ __launch_bounds__(64 * (MW * NW * KW + NL))
-__attribute__((amdgpu_waves_per_eu((MW * NW * KW + NL + 3) / 4, 8))) void streamed_forward_kernel(
+template <typename T, int MW, int NW, int KW, int WM, int WN, int CH, int RING, bool TILED>
+__global__ __launch_bounds__(64 * (MW * NW * KW + kStreamedLoaders))
+__attribute__((amdgpu_waves_per_eu((MW * NW * KW + kStreamedLoaders + 3) / 4, 8))) void streamed_forward_kernel(
     const T *__restrict__ sources, unsigned source_bytes, const T *__restrict__ wt,
     const int *__restrict__ kernel_map, TileView tiles, StreamedShape s, unsigned char *__restrict__ out,
     Epilogue ep) {
-  constexpr int TM = 32 * MW * WM, TN = 32 * NW * WN;
-  constexpr int NC = MW * NW * KW;                           // wavefronts that multiply
+  constexpr int TM = 32 * MW * WM, TN = 32 * NW * WN, BK = kStreamedStage;
+  constexpr int NC = MW * NW * KW, NL = kStreamedLoaders;    // wavefronts that multiply, and that load
   constexpr int kRowLanes = BK / 16;                         // lanes that load a row's stage
   constexpr int kLoadRows = 64 / kRowLanes;                  // rows of a load
   constexpr int kWaveRows = TM / NL;                         // of a wavefront that loads
@@ -102,7 +104,7 @@ __attribute__((amdgpu_waves_per_eu((MW * NW * KW + NL + 3) / 4, 8))) void stream
   static_assert(kRowLoads * NL * kLoadRows == TM && kWeightLoads * NL * kLoadRows == TN, "whole loads");
   static_assert(!TILED || kTileTargets % TM == 0, "whole parts of a tile");
   constexpr int KS = BK / 32 / KW;                           // products along K a wavefront makes of a stage
-  static_assert(KS >= 1 && KS * 32 * KW == BK && (BK == 64 || BK == 128), "stages are dealt out evenly");
+  static_assert(KS >= 1 && KS * 32 * KW == BK && BK == 128, "stages are dealt out evenly");
   static_assert(RING % CH == 0 && RING >= 2, "whole offsets in the ring");
   constexpr int kSlots = RING / CH;                          // offsets in the ring
   constexpr int kAhead = kSlots + 1;
@@ -136,7 +138,7 @@ __attribute__((amdgpu_waves_per_eu((MW * NW * KW + NL + 3) / 4, 8))) void stream
   const long long first_target = static_cast<long long>(blockIdx.x) * TM;
   // rows lie in LDS with their pieces exchanged so that eight rows' same piece
   // are in eight different places
-  auto place = [](int row, int piece) -> int { return BK == 128 ? piece ^ (row & 7) : piece ^ ((row >> 1) & 3); };
+  auto place = [](int row, int piece) -> int { return piece ^ (row & 7); };
   if (threadIdx.x == 0) *again = 0;
 
   // All meet when the first stage is there, once a stage, kEndMeets times at the
@@ -475,36 +477,42 @@ void streamed_forward(const T *sources, const T *packed, const int *kernel_map, 
   auto workgroups = [&](int64_t tm, int64_t tn) { return div_ceil(Tn, tm) * div_ceil(N, tn); };
 #define MNT_STREAMED(MW, NW, KW, WM, WN, CH, RING)                                                                \
   {                                                                                                               \
-    constexpr int TM = 32 * MW * WM, TN = 32 * NW * WN, threads = 64 * (4 + MW * NW * KW);                        \
+    constexpr int TM = 32 * MW * WM, TN = 32 * NW * WN, threads = 64 * (kStreamedLoaders + MW * NW * KW);         \
     const dim3 grid(static_cast<unsigned>(tiled ? l.tiles * (kTileTargets / TM) : div_ceil(Tn, int64_t{TM})),     \
                     static_cast<unsigned>(div_ceil(N, int64_t{TN})));                                             \
     if (tiled) {                                                                                                  \
-      streamed_forward_kernel<T, MW, NW, KW, WM, WN, 4, 128, CH, RING, true><<<grid, threads, 0, stream>>>(       \
+      streamed_forward_kernel<T, MW, NW, KW, WM, WN, CH, RING, true><<<grid, threads, 0, stream>>>(               \
           sources, source_bytes, packed, kernel_map, view, s, reinterpret_cast<unsigned char *>(out), ep);        \
     } else {                                                                                                      \
-      streamed_forward_kernel<T, MW, NW, KW, WM, WN, 4, 128, CH, RING, false><<<grid, threads, 0, stream>>>(      \
+      streamed_forward_kernel<T, MW, NW, KW, WM, WN, CH, RING, false><<<grid, threads, 0, stream>>>(              \
           sources, source_bytes, packed, kernel_map, view, s, reinterpret_cast<unsigned char *>(out), ep);        \
     }                                                                                                             \
   }
-#define MNT_STREAMED_K(MW, NW, KW, WM, WN, R1)                    \
-  switch (div_ceil(s.row_bytes, 128)) {                           \
-    case 1: MNT_STREAMED(MW, NW, KW, WM, WN, 1, R1) break;        \
+#define MNT_STREAMED_WIDE(MW, NW, KW, WM, WN)                     \
+  switch (div_ceil(s.row_bytes, kStreamedStage)) {                \
     case 2: MNT_STREAMED(MW, NW, KW, WM, WN, 2, 4) break;         \
     case 3: MNT_STREAMED(MW, NW, KW, WM, WN, 3, 3) break;         \
     default: MNT_STREAMED(MW, NW, KW, WM, WN, 4, 4) break;        \
+  }
+#define MNT_STREAMED_K(MW, NW, KW, WM, WN, R1)                    \
+  if (s.row_bytes <= kStreamedStage) {                            \
+    MNT_STREAMED(MW, NW, KW, WM, WN, 1, R1)                       \
+  } else {                                                        \
+    MNT_STREAMED_WIDE(MW, NW, KW, WM, WN)                         \
   }
   if (workgroups(32, 64) <= cus) {
     MNT_STREAMED_K(1, 1, 2, 1, 2, 4)
   } else if (workgroups(64, 64) <= cus) {
     MNT_STREAMED_K(1, 2, 2, 2, 1, 4)
-  } else if (N <= 64) {
-    MNT_STREAMED_K(2, 1, 2, 2, 2, 3)
+  } else if (N <= 64) {                        // (rows of one stage come with more than 128 channels)
+    MNT_STREAMED_WIDE(2, 1, 2, 2, 2)
   } else if (20 * workgroups(128, 128) < (s.row_bytes > 256 ? 30 : 21) * cus) {
     MNT_STREAMED_K(1, 2, 2, 2, 2, 3)
   } else {
     MNT_STREAMED_K(2, 2, 1, 2, 2, 3)
   }
 #undef MNT_STREAMED_K
+#undef MNT_STREAMED_WIDE
 #undef MNT_STREAMED
   check_launch("streamed_forward_kernel");
 }
