@@ -1035,8 +1035,12 @@ class SparseConv(Module):
                     tiled = not single and F.prefers_streamed(volume, self.in_channels + pad, self.out_channels,
                                                               sources.dtype)
                 if hits is None and implicit and dataflow == "auto":
-                    # (where its features are past what that form addresses: as if there were no such form)
+                    # (where its features are past what that form addresses, or what it is the
+                    # faster one for: as if there were no such form)
                     most = F.implicit_rows_limit(self.in_channels + pad, sources.dtype)
+                    if tiled:
+                        most = min(most, F.streamed_rows_limit(volume, self.in_channels, self.out_channels,
+                                                               sources.dtype))
                 route = self._routes[route_key] = (pad, implicit, grouped, most, single, tiled)
             pad, implicit, grouped, most, single, tiled = route
             if most is not None:

@@ -10,6 +10,7 @@ from ..kernel_map import KernelMap
 __all__ = ["cuda_time_gather", "cuda_time_scatter", "sparse_convolution_forward",
            "cuda_time_gemm", "set_gemm_parallel_level", "Epilogue", "pack_weights",
            "prefers_implicit", "prefers_streamed", "prefers_hits", "implicit_rows_limit", "hits_rows_limit",
+           "streamed_rows_limit",
            "pieces_rows_limit", "channel_pieces"]
 
 pack_weights = _C.pack_weights
@@ -62,31 +63,37 @@ def prefers_streamed(num_offsets: int, num_source_features: int, num_target_feat
     64 over 23 100 24.2 and 30.7, 256 -> 96 over 10 400 21.6 and 26.2, 256 -> 32 over
     18 800 19.5 and 27.7 (the other way round over few voxels, 256 -> 32 over 2 300
     22.6 and 16.9; 192 -> 64 over 22 000 24.0 and 24.0, over 13 800 19.7 and 15.9).
-    Nor more than 27 offsets, most of which a target has no source under and which
+    Nor more than 36 offsets, most of which a target has no source under and which
     are walked all the same: 4x4x4 and 5x5x5, 256 -> 128 over 9 000 of a scan 29 and
     94, 192 -> 224 over 20 000 of a room 73 and 203, 192 -> 64 over 26 000 23 and 49,
-    128 -> 128 over 40 000 66 and 99 (96 -> 128 over 4 000 28 and 19; over 79 layers,
-    with tiles and without, 1.2 times as long).
-
-    Nor fp16 rows of more than 384 bytes under more than 128 channels of which the
-    workgroups' last 128 are half empty, or with a fourth stage that is half empty
-    itself (in bf16 the other forms take longer): 256 -> 160 over 26 000 with
-    dilation 2 31 and 39, 224 -> 144 over 60 000 62 and 102, 224
-    -> 192 over 20 000 31 and 39, 208 -> 160 of 12 000 21 and 25, 224 -> 256 of
-    8 000 23 and 28; over 30 such layers 1.1 times as long.
+    128 -> 128 over 40 000 66 and 99 (96 -> 128 over 4 000 28 and 19; over 55 layers,
+    with tiles and without, 1.36 times as long; 3x3x4 over 33 layers 0.89).
 
     What stays slower: fp16 layers of few sources a target just before they get
     tiles (160 -> 128 over 12 000 of a LiDAR scan 17.2 and 20.3), and strided layers
-    of many targets whose map is kept for many calls (256 -> 256 onto 35 000 30 and 50).
-    On new clouds, where the other forms have rank tables to build, those take 0.67
-    times as long (of 209 the slowest two 1.12, 256 -> 256 onto 35 000 103 and 92)."""
-    if num_offsets > 27:
+    of many targets whose map is kept for many calls (256 -> 160 onto 20 000 19 and 30,
+    256 -> 256 onto 46 000 47 and 50).  On new clouds, where the other forms have rank
+    tables to build, those take 0.67 times as long (of 209 the slowest two 1.12)."""
+    if num_offsets > 36 or (num_offsets > 8 and num_source_features > 192 and num_target_features <= 96):
         return False
-    if num_offsets > 8 and num_source_features > 192:
-        half_empty = num_source_features <= 224 or (num_target_features - 1) % 128 < 64
-        if num_target_features <= 96 or (dtype == torch.float16 and num_target_features > 128 and half_empty):
-            return False
     return _C.streamed_forward_supported(num_offsets, num_source_features, num_target_features, dtype)
+
+
+def streamed_rows_limit(num_offsets: int, num_source_features: int, num_target_features: int,
+                        dtype: torch.dtype) -> int:
+    """The most source rows of which ``prefers_streamed`` holds.
+
+    Streamed workgroups take 128 output channels at a time, and fp16 3x3x3 layers of
+    more than 192 input channels whose last 128 are at least half empty do without
+    once workgroups of 64 x 64 no longer fit the chip in one go (offset groups and
+    streamed, us: 256 -> 160 over 26 000 with dilation 2 31 and 39, 224 -> 144 over
+    60 000 62 and 102, 224 -> 192 over 20 000 31 and 39, 208 -> 160 over 12 000 21 and
+    25; below, 256 -> 192 over 3 000 21 and 18, over 700 18 and 14).  In bf16 the
+    groups take longer: 256 -> 129 to 192 over 6 layers 0.85 times as long streamed."""
+    if (num_offsets == 27 and num_source_features > 192 and num_target_features > 128
+            and (num_target_features - 1) % 128 < 64 and dtype == torch.float16):
+        return 256 // -(-num_target_features // 64) * 64
+    return (1 << 63) - 1
 
 
 def implicit_rows_limit(num_source_features: int, dtype: torch.dtype) -> int:

@@ -127,12 +127,48 @@ def test_a_layer_gives_the_same_rows_from_call_to_call():
 
 @pytest.mark.parametrize("cin,cout,offsets,streams", [
     (256, 96, 27, False), (256, 104, 27, True), (200, 96, 9, False), (192, 96, 27, True), (256, 32, 8, True),
-    (128, 128, 27, True), (128, 128, 36, False), (256, 128, 64, False), (192, 224, 125, False),
-    (256, 192, 27, False), (256, 200, 27, True), (192, 160, 27, True), (224, 256, 27, False), (232, 256, 27, True),
-    (224, 128, 27, True), (256, 320, 27, False), (224, 256, 8, True)])
+    (128, 128, 27, True), (128, 128, 36, True), (128, 128, 45, False), (256, 128, 64, False), (192, 224, 125, False)])
 def test_which_wide_layers_are_streamed(cin, cout, offsets, streams):
     """Both sides of the line between streaming and grouped products."""
     assert F.prefers_streamed(offsets, cin, cout, torch.float16) == streams
+
+
+@pytest.mark.parametrize("rows,cout,dtype,streams", [(5000, 160, torch.float16, True), (5441, 160, torch.float16, False),
+                                                     (9000, 160, torch.bfloat16, True), (9000, 200, torch.float16, True),
+                                                     (9000, 128, torch.float16, True), (3300, 320, torch.float16, False)])
+def test_how_many_rows_are_streamed(rows, cout, dtype, streams, monkeypatch):
+    """Each cloud gets the kernel that a fresh cache would give it."""
+    generator = torch.Generator().manual_seed(rows)
+    conv = minuet.nn.SparseConv3d(256, cout, 3, dtype=dtype, device=DEVICE)
+    calls = []
+    for name in ("implicit", "tiled", "groups"):
+        whole = getattr(_C, f"sparse_convolution_forward_{name}")
+        monkeypatch.setattr(_C, f"sparse_convolution_forward_{name}",
+                            lambda *args, _whole=whole, _name=name, **kw: calls.append(_name) or _whole(*args, **kw))
+    wanted = {}
+    for count in (rows, 700, rows, 700):
+        cells = torch.randperm(1 << 15, generator=generator)[:count].sort()[0].to(DEVICE)
+        coordinates = torch.stack([cells >> 10, (cells >> 5) & 31, cells & 31], 1).int()
+        x = minuet.SparseTensor(torch.randn(count, 256, device=DEVICE).to(dtype), coordinates)
+        conv.set_kernel_map_cache(minuet.nn.KernelMapCache(3, torch.int32, DEVICE))
+        with torch.no_grad():
+            conv(x)
+            assert (calls[-1] == "groups") == (count == rows and not streams)
+            got = conv(x).F
+        wide = sum((x.F.double().new_zeros(count, cout).index_add_(0, t, x.F[s].double() @ conv.kernel[o].double())
+                    for o, s, t in _pairs(coordinates)))
+        # products of unit normals and uniform weights, rounded once or (grouped) twice
+        assert float((got.double() - wide).norm() / wide.norm()) < 4 * torch.finfo(dtype).eps
+
+
+def _pairs(coordinates):
+    key = lambda c: ((c[:, 0].long() + 1) * 64 + c[:, 1] + 1) * 64 + c[:, 2] + 1
+    keys = key(coordinates)
+    for o, offset in enumerate(minuet.utils.helpers.generate_kernel_offsets(3, 3, 1, 1)):
+        wanted = key(coordinates + torch.as_tensor(offset, device=coordinates.device, dtype=torch.int32))
+        at = torch.searchsorted(keys, wanted).clamp_(max=len(keys) - 1)
+        t = torch.nonzero(keys[at] == wanted)[:, 0]
+        yield o, at[t], t
 
 
 @pytest.mark.parametrize("cin,streams", [(96, True), (100, False), (104, True), (150, False), (254, False), (256, True)])
