@@ -53,7 +53,7 @@ struct CompactShape {
 // nn/functional/convolution.py has the line and both sides of it).  fp32, 3 x 3 x 3, us a layer in
 // three kernels and here: 32 -> 32 channels over 3 000 voxels 11.4 / 4.9,
 // 20 000 17.9 / 11.2, 200 000 76 / 51; 64 -> 64 over 3 000 12.1 / 8.4, 12 000
-// 18.8 / 14.9; 256 -> 256 over 135 28 / 16.  (128 targets per workgroup
+// 18.8 / 14.9; 256 -> 256 over 135 28 / 16 in lanes.  (128 targets per workgroup
 // fill the 16 rows better, but their sums leave fewer wavefronts to a compute
 // unit: 17 to 40 % slower.)
 template <int C, int KI, int SPLIT, int TARGETS, bool WHOLE, bool LANES>
@@ -309,27 +309,33 @@ void compact_forward(const float *sources, const float *weights, bool lanes, con
   // Targets, channel blocks and wavefronts of a workgroup by how many workgroups
   // of 64 targets and 16 channels there are to a compute unit (`full`): small
   // clouds need small workgroups to reach the whole chip, beyond that two blocks
-  // share the source rows.  With one step of 16 input channels a workgroup is its
+  // share the source rows (from 1.95 to 3 workgroups over 32 targets each: over 64
+  // those two blocks are one to one and a half workgroups a compute unit).  With
+  // one step of 16 input channels a workgroup is its
   // map and its sums, and 32 targets are enough at any size; not for many targets
   // and weights as [O][K][N], of which four blocks read whole lines.  Those have
-  // one block up to three workgroups, since a second doubles the loads of their
+  // one block up to 4.75 workgroups, since a second doubles the loads of their
   // weights (in lanes it does not).  `split` is the same for both forms of the
-  // weights, whose sums are then the same bit for bit.
+  // weights, whose sums are then the same bit for bit; a unit of less than two
+  // steps (K < 32) is short, and eight wavefronts pay a little longer.
   //
-  // Over 1 057 layers of three kinds of scene (3x3x3 and strided 2x2x2, 130 to
-  // 580 000 targets, 4 to 256 channels) the form before there were two, and its
-  // lines, took 1.14 times as long as weights in lanes do and 1.05 times as long
-  // as [O][K][N] (the best of 14 shapes for each layer: 0.96 and 0.95 of these
-  // lines).  us, that form and here, lanes: 256 -> 256 channels over 130 targets
+  // Weights in lanes, over 1 057 layers of three kinds of scene (3x3x3 and strided
+  // 2x2x2, 130 to 580 000 targets, 4 to 256 channels): the form before there were
+  // two, and its lines, took 1.14 times as long (the best of 14 shapes for each
+  // layer 0.96).  [O][K][N], which is what layers have, against that form: 1.00
+  // over 285 of them, 0.99 over 130 of 3 to 4.75 workgroups, 1.01 over 204 of 20 to
+  // 28 channels.  us, that form and here, lanes: 256 -> 256 channels over 130 targets
   // 19.7 / 12.8, 128 -> 128 over 2 980 46 / 33, 8 -> 128 over 40 000 27.6 / 26.5;
-  // [O][K][N]: 64 -> 64 over 3 000 10.4 / 8.7 (two blocks 10.9), 128 -> 128 over
-  // 3 000 20.2 / 19.4 (22.0).  What two blocks cost is layers with few hits, whose
-  // blocks of rows are nearly empty, which the host cannot know: 96 -> 256 over
-  // 2 000 of a LiDAR scan 13.7 / 16.5 and, with one block, 13.7; where a target
+  // [O][K][N]: 128 -> 128 over 700 14.5 / 10.7, 64 -> 64 over 3 000 10.4 / 8.7 (two
+  // blocks 10.9), 128 -> 128 over 3 000 20.2 / 19.4 (22.0), 48 -> 64 over 9 000 14.5 /
+  // 13.9; few hits and few offsets are slower: 80 -> 64 over 9 000 of 2x2x2 10.6 /
+  // 12.1, 64 -> 16 onto 13 700 5.8 / 6.7.  What two blocks cost is layers with few
+  // hits, whose blocks of rows are nearly empty, which the host cannot know: 96 -> 256
+  // over 2 000 of a LiDAR scan 13.7 / 16.5 and, with one block, 13.7; where a target
   // has 13 hits 35 / 26 and 32.
   const int64_t cus = compute_units(), cols = div_ceil(N, int64_t{16});
   const double full = static_cast<double>(div_ceil(Tn, int64_t{64}) * cols) / static_cast<double>(cus);
-  int c = 1, targets = 64, split = full < 1.95 ? 8 : 4;
+  int c = 1, targets = 64, split = full < (K < 32 ? 2.26 : 1.95) ? 8 : 4;
   if (N % 32 != 0) {
     targets = full < 0.3 ? 16 : full < 0.9 ? 32 : 64;
     split = full < 2.25 ? 8 : 4;
@@ -337,7 +343,7 @@ void compact_forward(const float *sources, const float *weights, bool lanes, con
     c = 2;
     targets = 32;
     split = full < 3.0 ? 8 : 4;
-  } else if (!lanes && K >= 32 && full < 3.0) {
+  } else if (!lanes && K > 16 && full < 4.75) {
     targets = full < 0.26 ? 16 : full < 0.6 ? 32 : 64;
   } else if (full < 0.6) {
     c = full >= 0.26 && full < 0.42 ? 2 : 1;

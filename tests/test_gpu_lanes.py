@@ -44,10 +44,10 @@ def test_lane_order_is_the_same_product(targets, offsets, K, N):
     assert lanes.equal(plain)
 
 
-# 0.9, 1, 1.9, 2, 2.9, 3, 4.7 and 4.8 workgroups of 64 targets and 16 channels to each of 256 compute units:
-# both sides of every line of the layers with one step of 16 channels, and of [O][K][N] ones
-@pytest.mark.parametrize("targets", [3790, 4100, 7800, 8200, 11900, 12300, 19300, 19700])
-@pytest.mark.parametrize("offsets, K, N", [(27, 8, 64), (8, 16, 64), (27, 32, 64), (2, 80, 64)])
+# 0.9, 1, 1.9, 2, 2.25, 2.3, 2.9, 3, 4.7 and 4.8 workgroups of 64 targets and 16 channels to each of 256 compute units:
+# both sides of every line of the layers with one step of 16 channels, with one and a half, and of [O][K][N] ones
+@pytest.mark.parametrize("targets", [3790, 4100, 7800, 8200, 9150, 9300, 11900, 12300, 19300, 19700])
+@pytest.mark.parametrize("offsets, K, N", [(27, 8, 64), (8, 16, 64), (27, 24, 64), (27, 32, 64), (2, 80, 64)])
 def test_lane_order_at_the_lines_between_shapes(targets, offsets, K, N):
     dense, x, w = _case(targets, offsets, K, N, 0.2, targets + K)
     expected = _oracle(dense, x, w)
