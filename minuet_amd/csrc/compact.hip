@@ -52,8 +52,8 @@ struct CompactShape {
 // three-kernel form is the faster one again (hits_rows_limit in
 // nn/functional/convolution.py has the line and both sides of it).  fp32, 3 x 3 x 3, us a layer in
 // three kernels and here: 32 -> 32 channels over 3 000 voxels 11.4 / 4.9,
-// 20 000 17.9 / 11.2, 200 000 76 / 51; 64 -> 64 over 3 000 12.1 / 8.4, 12 000
-// 18.8 / 14.9; 256 -> 256 over 135 28 / 16 in lanes.  (128 targets per workgroup
+// 20 000 17.9 / 11.2, 200 000 76 / 54; 64 -> 64 over 3 000 12.1 / 8.4, 12 000
+// 18.8 / 14.9; 256 -> 256 over 135 28 / 15.6 (in lanes 12.5).  (128 targets per workgroup
 // fill the 16 rows better, but their sums leave fewer wavefronts to a compute
 // unit: 17 to 40 % slower.)
 template <int C, int KI, int SPLIT, int TARGETS, bool WHOLE, bool LANES>
@@ -181,12 +181,18 @@ __global__ __launch_bounds__(64 * SPLIT) void compact_forward_kernel(
 
   for (int first_offset = wv; first_offset < s.num_offsets || first_offset == wv; first_offset += SPLIT * kCompactBatch) {
     int index[kCompactBatch / kAtOnce];
+    if (kernel_map != nullptr) {               // (outside the loop, which asks for all of them at once)
 #pragma unroll
-    for (int j = 0; j < kCompactBatch / kAtOnce; ++j) {
-      const long long o = min(first_offset + (j * kAtOnce + lane / kTargets) * SPLIT, s.num_offsets - 1);
-      const long long t = min(first + lane % kTargets, s.num_targets - 1);
-      // (no map: the offsets are pieces of the target's own row)
-      index[j] = kernel_map != nullptr ? kernel_map[o * s.num_targets + t] : static_cast<int>(t * s.num_offsets + o);
+      for (int j = 0; j < kCompactBatch / kAtOnce; ++j) {
+        const long long o = min(first_offset + (j * kAtOnce + lane / kTargets) * SPLIT, s.num_offsets - 1);
+        index[j] = kernel_map[o * s.num_targets + min(first + lane % kTargets, s.num_targets - 1)];
+      }
+    } else {                                   // the offsets are pieces of the target's own row
+#pragma unroll
+      for (int j = 0; j < kCompactBatch / kAtOnce; ++j) {
+        const int o = min(first_offset + (j * kAtOnce + lane / kTargets) * SPLIT, s.num_offsets - 1);
+        index[j] = static_cast<int>(min(first + lane % kTargets, s.num_targets - 1)) * s.num_offsets + o;
+      }
     }
     if (first_offset == wv) {
       float4 *const clear = reinterpret_cast<float4 *>(acc);
@@ -326,13 +332,13 @@ void compact_forward(const float *sources, const float *weights, bool lanes, con
   // over 285 of them, 0.99 over 130 of 3 to 4.75 workgroups, 1.01 over 204 of 20 to
   // 28 channels.  us, that form and here, lanes: 256 -> 256 channels over 130 targets
   // 19.7 / 12.8, 128 -> 128 over 2 980 46 / 33, 8 -> 128 over 40 000 27.6 / 26.5;
-  // [O][K][N]: 128 -> 128 over 700 14.5 / 10.7, 64 -> 64 over 3 000 10.4 / 8.7 (two
-  // blocks 10.9), 128 -> 128 over 3 000 20.2 / 19.4 (22.0), 48 -> 64 over 9 000 14.5 /
-  // 13.9; few hits and few offsets are slower: 80 -> 64 over 9 000 of 2x2x2 10.6 /
-  // 12.1, 64 -> 16 onto 13 700 5.8 / 6.7.  What two blocks cost is layers with few
-  // hits, whose blocks of rows are nearly empty, which the host cannot know: 96 -> 256
-  // over 2 000 of a LiDAR scan 13.7 / 16.5 and, with one block, 13.7; where a target
-  // has 13 hits 35 / 26 and 32.
+  // [O][K][N], objects: 128 -> 128 over 700 14.0 / 10.6, 32 -> 32 over 20 000 14.0 /
+  // 13.4, 64 -> 64 over 12 000 21.5 / 20.1, 28 -> 128 over 4 000 under 5x5x5 29.4 / 29.1;
+  // slower: 128 -> 128 over 3 000 25.8 / 27.7, 80 -> 64 over 9 000 of 2x2x2 10.6 / 12.1,
+  // 64 -> 16 onto 13 700 5.8 / 6.7.  What two blocks cost is layers with few hits,
+  // whose blocks of rows are nearly empty, which the host cannot know: in lanes 96 ->
+  // 256 over 2 000 of a LiDAR scan 13.7 / 16.5 and, with one block, 13.7; where a
+  // target has 13 hits 35 / 26 and 32.
   const int64_t cus = compute_units(), cols = div_ceil(N, int64_t{16});
   const double full = static_cast<double>(div_ceil(Tn, int64_t{64}) * cols) / static_cast<double>(cus);
   int c = 1, targets = 64, split = full < (K < 32 ? 2.26 : 1.95) ? 8 : 4;
