@@ -589,8 +589,9 @@ int mnt_sparse_convolution_forward_implicit(const void *sources, const void *wei
 int mnt_kernel_map_tiles_size(int64_t num_targets, int64_t num_offsets, int64_t *ints_out);
 int mnt_kernel_map_tiles(const int32_t *kernel_map, int64_t num_targets, int64_t num_offsets,
                          int32_t *tiles_out, void *stream);
-/* The tiles of several maps, one after the other in the arrays, in as many
- * launches as one map's take. */
+/* The tiles of several maps, one after the other in the arrays: three launches,
+ * which is what one map's take, for up to eight maps of up to 32 offsets and for
+ * up to eight of more. */
 int mnt_kernel_map_tiles_batch(int64_t num_maps, const int32_t *const *kernel_maps, const int64_t *num_targets,
                                const int64_t *num_offsets, int32_t *const *tiles_out, void *stream);
 double mnt_kernel_map_tiles_share(int64_t num_targets, int64_t num_offsets, int64_t num_source_features,

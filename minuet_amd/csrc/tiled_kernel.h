@@ -130,7 +130,7 @@ struct TiledShape {
 // channels, 16-bit, us a layer in implicit_forward_kernel and here: 3 000
 // targets of an object 14.9 / 8.8, 25 000 of a LiDAR scan 14.9 / 10.3, 60 000
 // of a room 18.2 / 17.4; in tiles, LiDAR, 200 000 48.6 / 27, a
-// million under 5 x 5 x 5 836 / 407.
+// million under 5 x 5 x 5 836 / 403.
 template <typename T, int NB, int KS, bool TILED, bool PAIRED, bool WHOLE, bool QUADS, int GROUPS>
 __global__ __launch_bounds__(256 * GROUPS) void tiled_forward_kernel(
     const T *__restrict__ sources, unsigned source_bytes, const T *__restrict__ wt,

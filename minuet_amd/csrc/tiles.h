@@ -44,9 +44,10 @@ struct TileLayout {
 // the last windows.  Then the next longest of a band of windows at a time, as
 // many as leave their rows in a die's L2 (seven of 4096 128-byte rows), and not
 // window after window, whose long tiles leave gaps.  us a layer with 8 windows
-// after the other, all windows at a time, and so: 64 -> 64 channels of 16 bits
-// over 200 000 LiDAR voxels 33.9, 27.5, 26.7, over a room of 150 000 27.7, 22.0, 20.1;
-// 5x5x5 over a million 430, 423, 407; 32 -> 32 over a million 83.8, 83.8, 77.1.
+// after the other and so: 64 -> 64 channels of 16 bits over 200 000 LiDAR voxels
+// 34.4 and 28.6, over a room of 150 000 26.3 and 20.4; over a million, where the last
+// windows are a small part, under 5x5x5 415 to 422 and 401 to 411, 32 -> 32 under 3x3x3
+// 85.7 and 84.2.
 constexpr int kTileFirst = 2, kTileBand = 7;
 __device__ __forceinline__ int tile_number(int windows, int per_window, int window, int place) {
   const int rows = windows / kTileXcds, row = window / kTileXcds;      // windows of a die

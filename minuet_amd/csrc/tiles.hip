@@ -27,8 +27,8 @@ static_assert(kTileWindow == 1 << kTilePlaceBits && kTileKeyBits % kTileDigitBit
 
 // The maps one set of launches takes: a network's pass makes the tiles of all its
 // maps at once, because the sort of one keeps 8 to 40 of 256 compute units busy
-// (the five maps of a network over 200 000 voxels: 160 us one after the other,
-// 37 together).
+// (the five maps of a network over 200 000 voxels: 156 us one after the other,
+// 51 together).
 constexpr int kTileJobs = 8;
 struct TileJob {
   const int *dense;

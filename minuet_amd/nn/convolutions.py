@@ -30,7 +30,7 @@ _MOST_ROWS = (1 << 63) - 1
 # What the tiles of a map have to save a pass, over what making them alone takes,
 # for the next pass to make them with all others: for a map that had none, and
 # to go on (so that a size that wavers does not change the plan every time).
-# Five maps take 49 us together and 137 one by one.
+# Five maps take 51 us together and 156 one by one.
 _TILES_PAY, _TILES_STAY = 0.75, 0.5
 # Targets x output channels up to which a layer that records gradients, and so
 # packs its weights at every call, does without the kernel for one source a
