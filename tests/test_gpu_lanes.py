@@ -69,6 +69,22 @@ def test_lane_order_epilogue(activation):
     assert lanes.equal(plain)
 
 
+def test_lane_weights_follow_the_parameter():
+    coordinates = torch.unique(torch.randint(0, 12, (900, 3), generator=torch.Generator().manual_seed(1),
+                                             dtype=torch.int32), dim=0).cuda()
+    coordinates = coordinates[F.build_sorted_index(coordinates)]
+    conv = minuet.nn.SparseConv3d(32, 32, 3, device="cuda")
+    conv.set_kernel_map_cache(minuet.nn.KernelMapCache(ndim=3, dtype=torch.int32, device="cuda"))
+    x = minuet.SparseTensor(torch.randn(len(coordinates), 32, device="cuda"), coordinates)
+    with torch.no_grad():
+        first = conv(x).F.clone()
+        assert conv(x).F.equal(first)                                  # (and past Python)
+        conv.kernel.mul_(2.0)                                          # in place: same storage, new version
+        assert conv(x).F.equal(2 * first)
+        assert conv(x).F.equal(2 * first)
+    assert conv(x).F.detach().equal(2 * first)                         # gradients are recorded: as they are
+
+
 # hits only, of three kinds of map; the channels in pieces, wider than the library's product was left for either way
 @pytest.mark.parametrize("cin, cout, size, stride, transposed", [
     (32, 32, 3, 1, False), (64, 128, 2, 2, False), (64, 32, 2, 2, True), (256, 128, 1, 1, False), (64, 256, 1, 1, False)])
