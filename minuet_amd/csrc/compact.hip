@@ -55,7 +55,10 @@ struct CompactShape {
 // 20 000 17.9 / 11.2, 200 000 76 / 54; 64 -> 64 over 3 000 12.1 / 8.4, 12 000
 // 18.8 / 14.9; 256 -> 256 over 135 28 / 15.6 (in lanes 12.5).  (128 targets per workgroup
 // fill the 16 rows better, but their sums leave fewer wavefronts to a compute
-// unit: 17 to 40 % slower.)
+// unit: 17 to 40 % slower.  Rows that four lanes load together and turn round:
+// 20 000 targets 13.0 -> 14.4; the hits of all wavefronts dealt out evenly: 12.1, but
+// 256 -> 256 over 130 targets 13.6 -> 14.9, and sums that go by the targets of a
+// workgroup.)
 template <int C, int KI, int SPLIT, int TARGETS, bool WHOLE, bool LANES>
 __global__ __launch_bounds__(64 * SPLIT) void compact_forward_kernel(
     const float *__restrict__ sources, unsigned source_bytes, const float *__restrict__ weights,
@@ -179,25 +182,21 @@ __global__ __launch_bounds__(64 * SPLIT) void compact_forward_kernel(
     __builtin_amdgcn_wave_barrier();
   };
 
-  for (int first_offset = wv; first_offset < s.num_offsets || first_offset == wv; first_offset += SPLIT * kCompactBatch) {
-    int index[kCompactBatch / kAtOnce];
-    if (kernel_map != nullptr) {               // (outside the loop, which asks for all of them at once)
+  int index[kCompactBatch / kAtOnce];          // (outside the loop over them, which asks for all of them at once)
+  auto load_map = [&](int first_offset) {
 #pragma unroll
-      for (int j = 0; j < kCompactBatch / kAtOnce; ++j) {
-        const long long o = min(first_offset + (j * kAtOnce + lane / kTargets) * SPLIT, s.num_offsets - 1);
-        index[j] = kernel_map[o * s.num_targets + min(first + lane % kTargets, s.num_targets - 1)];
-      }
-    } else {                                   // the offsets are pieces of the target's own row
-#pragma unroll
-      for (int j = 0; j < kCompactBatch / kAtOnce; ++j) {
-        const int o = min(first_offset + (j * kAtOnce + lane / kTargets) * SPLIT, s.num_offsets - 1);
-        index[j] = static_cast<int>(min(first + lane % kTargets, s.num_targets - 1)) * s.num_offsets + o;
-      }
+    for (int j = 0; j < kCompactBatch / kAtOnce; ++j) {
+      const int o = min(first_offset + (j * kAtOnce + lane / kTargets) * SPLIT, s.num_offsets - 1);
+      const long long target = min(first + lane % kTargets, s.num_targets - 1);
+      // without a map the offsets are pieces of the target's own row
+      index[j] = kernel_map != nullptr ? kernel_map[o * s.num_targets + target] : static_cast<int>(target) * s.num_offsets + o;
     }
-    if (first_offset == wv) {
-      float4 *const clear = reinterpret_cast<float4 *>(acc);
-      for (int i = lane; i < (kTargets + 1) * kAccRow / 4; i += 64) clear[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    }
+  };
+  load_map(wv);
+  for (int i = lane; i < (kTargets + 1) * kAccRow / 4; i += 64) {
+    reinterpret_cast<float4 *>(acc)[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  }
+  for (int first_offset = wv; first_offset < s.num_offsets; first_offset += SPLIT * kCompactBatch) {
     int count = 0;
 #pragma unroll
     for (int j = 0; j < kCompactBatch / kAtOnce; ++j) {
@@ -227,24 +226,38 @@ __global__ __launch_bounds__(64 * SPLIT) void compact_forward_kernel(
     count = __builtin_amdgcn_readfirstlane(count);
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
-    const int units = count / 16 * chunks;
-    if (units == 0) continue;
+    if (first_offset + SPLIT * kCompactBatch < s.num_offsets) load_map(first_offset + SPLIT * kCompactBatch);
+    int left = count / 16 * chunks;
+    if (left == 0) continue;
     int g = 0, c = 0;
     auto advance = [&]() {
       if (++c == chunks) {
         c = 0;
-        if (g + 1 < count / 16) ++g;
+        ++g;
       }
     };
+    // One unit ahead and none past the last: the loads of one that is not
+    // multiplied keep the address unit as long as another's (two of the nine a
+    // wavefront has over 20 000 targets; 256 -> 256 channels over 130 targets
+    // 15.4 -> 13.4 us without them, 128 -> 128 over 3 000 20.8 -> 19.8).  Three
+    // units in flight are no faster (14.6, 24.3).
     Unit u0, u1;
     fetch(0, 0, u0);
-    for (int u = 0; u < units; u += 2) {
+    for (; left > 2; left -= 2) {
       advance();
       fetch(g, c, u1);
       multiply(u0);
       advance();
       fetch(g, c, u0);
-      if (u + 1 < units) multiply(u1);
+      multiply(u1);
+    }
+    if (left == 2) {
+      advance();
+      fetch(g, c, u1);
+      multiply(u0);
+      multiply(u1);
+    } else {
+      multiply(u0);
     }
   }
 
