@@ -678,6 +678,16 @@ int mnt_voxelize(const void *points, int64_t n, int ndim, int wide_points, const
 int mnt_gather_rows(const void *const *sources, const int64_t *source_rows, int num_sources, int64_t row_bytes,
                     const void *order, int index_dtype, int64_t n, void *out, void *stream);
 
+/* One batch from up to 64 clouds (host arrays of the device addresses and row
+ * counts of [N_g, ndim] coordinates; at least one row in all): every cloud's rows
+ * sorted inside its range of sorted_out, the ranges' boundaries in batch_dims_out
+ * [num_clouds + 1] (of the coordinate type) and, features_out not null, the rows of
+ * `features` (row_bytes each, a multiple of 2) in the same order.
+ * bounds_host_out (nullable): minima [0..3], then maxima [4..7] of the coordinates. */
+int mnt_collate(const void *const *clouds, const void *const *features, const int64_t *cloud_rows, int num_clouds,
+                int ndim, int coord_dtype, int64_t row_bytes, void *sorted_out, void *batch_dims_out,
+                void *features_out, int64_t *bounds_host_out, void *stream);
+
 /* Host integers to device memory as kernel arguments: nothing is waited for. */
 int mnt_upload_ints(const int64_t *values, int64_t count, int index_dtype, void *out, void *stream);
 

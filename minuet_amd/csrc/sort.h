@@ -50,6 +50,11 @@ SortStart sort_start(int64_t n, Scope &scope);
 // mnt_arg_sort_coordinates does, without the pass over the rows for their bounds.
 void sort_started_rows(const void *rows, int64_t n, int ndim, int coord_dtype, int32_t *indices_out, void *sorted_out,
                        const SortStart &start, hipStream_t stream);
+// The same for rows of several batches, the permutation in the coordinates' type
+// and the extremes for the host (what mnt_arg_sort_coordinates gives).
+void sort_started_batches(const void *rows, int64_t n, int ndim, int coord_dtype, const void *batch_dims,
+                          int64_t num_batches, void *indices_out, void *sorted_out, int64_t *bounds_host_out,
+                          const SortStart &start, hipStream_t stream);
 
 // ---- the bucket sort as a chain of launches that never waits for the host ----
 

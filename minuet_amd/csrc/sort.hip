@@ -2077,6 +2077,23 @@ void sort_started_rows(const void *rows, int64_t n, int ndim, int coord_dtype, i
   }
 }
 
+void sort_started_batches(const void *rows, int64_t n, int ndim, int coord_dtype, const void *batch_dims,
+                          int64_t num_batches, void *indices_out, void *sorted_out, int64_t *bounds_host_out,
+                          const SortStart &start, hipStream_t stream) {
+  const SortStart *made = start.parts > 0 ? &start : nullptr;
+  if (coord_dtype == MNT_INT32) {
+    arg_sort_typed<int32_t, int32_t>(static_cast<const int32_t *>(rows), n, ndim,
+                                     static_cast<const int32_t *>(batch_dims), num_batches,
+                                     static_cast<int32_t *>(indices_out), static_cast<int32_t *>(sorted_out),
+                                     bounds_host_out, stream, made);
+  } else {
+    arg_sort_typed<int64_t, int64_t>(static_cast<const int64_t *>(rows), n, ndim,
+                                     static_cast<const int64_t *>(batch_dims), num_batches,
+                                     static_cast<int64_t *>(indices_out), static_cast<int64_t *>(sorted_out),
+                                     bounds_host_out, stream, made);
+  }
+}
+
 }  // namespace mnt
 
 using namespace mnt;

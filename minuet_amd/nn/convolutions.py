@@ -152,18 +152,22 @@ class KernelMapCache(object):
 
     def _plan_next_pass(self):
         """Turns the requests of the pass that ends here into the plan of the next one."""
-        if self._built is not None:
-            saved = None                         # (key, transposed) -> what tiles saved, or would have
-            for entry, request in self._built.entries:
+        built, self._built = self._built, None
+        if built is not None:
+            saved = {}                           # (key, transposed) -> what tiles saved, or would have
+            for entry, request in built.entries:
+                share = entry.tiles_saved
+                if share and entry.used:
+                    saved[request[4:]] = saved.get(request[4:], 0.0) + share
+            tiles = self._note_tiles(saved, built.plan.tiles) if saved else set()
+            if built.plan is self._pass_plan and built.plan.is_repeated(built, self._requests, tiles):
+                self._requests = dict()          # the plan stays
+                return
+            for entry, request in built.entries:
                 if entry.used:                   # a layer that never came through Python
                     self._note_fast(request)
-                    share = entry.tiles_saved
-                    if share:
-                        saved = {} if saved is None else saved
-                        saved[request[4:]] = saved.get(request[4:], 0.0) + share
-            if saved is not None:
-                self._note_tiles(saved, self._built.plan.tiles)
-            self._built = None
+            for request in tiles:
+                self._requests.setdefault(request)
         requests, self._requests = self._requests, dict()
         if self._lookahead or not requests or not self._coordinates_cache:
             return
@@ -182,26 +186,14 @@ class KernelMapCache(object):
     def _note_fast(self, request):
         """A layer ran with the map of ``request`` (see ``PassPlan``): so it has
         asked for that map, and for the level it leads to."""
-        _, _, _, kind, key, transposed = request
-        if key[0] != key[1]:
-            self._requests.setdefault(("coords", key[0], key[1]))
-        if kind == "IMPLICIT":
-            self._requests.setdefault(("dense", key))
-            if transposed:
-                self._requests.setdefault(("invert", key))
-        elif kind == "GROUPS":
-            self._requests.setdefault(("dense", key))
-            self._requests.setdefault(("groups", key))
-        else:
-            self._requests.setdefault(("dense", key))
-            self._requests.setdefault(("tables", key, not self._disable_reordering))
-        self._requests.setdefault(request)
+        from minuet_amd.nn.passplan import requests_of
+        for asked in requests_of(request, not self._disable_reordering):
+            self._requests.setdefault(asked)
 
-    def _note_tiles(self, saved, made):
-        """Asks for the tiles of the maps whose layers would have saved enough by them."""
-        for at, share in saved.items():
-            if share >= (_TILES_STAY if at in made else _TILES_PAY):
-                self._requests.setdefault(("tiles", *at))
+    @staticmethod
+    def _note_tiles(saved, made):
+        """The requests for the tiles of the maps whose layers would have saved enough by them."""
+        return {("tiles", *at) for at, share in saved.items() if share >= (_TILES_STAY if at in made else _TILES_PAY)}
 
     def _open_pass(self, coordinates, stride, batch_dims):
         """First request of a pass: with a plan of the last one, builds everything on it."""

@@ -50,6 +50,7 @@ SIGNATURES = {
     "mnt_host_wait_stats": (_int, [_pi64, _pi64, _int]),
     "mnt_voxelize": (_int, [_vp, _i64, _int, _int, _vp, _int, _vp, _vp, _pi64, _vp]),
     "mnt_gather_rows": (_int, [_vp, _vp, _int, _i64, _vp, _int, _i64, _vp, _vp]),
+    "mnt_collate": (_int, [_vp, _vp, _vp, _int, _int, _int, _i64, _vp, _vp, _vp, _vp, _vp]),
     "mnt_upload_ints": (_int, [_vp, _i64, _int, _vp, _vp]),
     "mnt_global_pool": (_int, [_vp, _vp, _i64, _i64, _i64, _int, _int, _int, _vp, _vp]),
     "mnt_pass_levels": (_int, [_vp, _i64, _int, _int, _vp, _i64, _int, _vp, _vp, _int, _vp, _int, _vp, _pi64,
@@ -1809,6 +1810,33 @@ def gather_rows(sources: Sequence[torch.Tensor], order: torch.Tensor) -> torch.T
             ctypes.addressof(pointers), ctypes.addressof(rows), count, channels * out.element_size(),
             order.data_ptr(), _INT[order.dtype], n, out.data_ptr(), _stream(device)))
     return out
+
+
+def collate(clouds: Sequence[torch.Tensor], features: Optional[Sequence[torch.Tensor]]):
+    """``(sorted coordinates, batch_dims, feature rows or None)`` of a batch in one
+    library call (mnt_collate): up to 64 clouds, contiguous [N_g, D] of one integer
+    type, with at least one row between them, and contiguous features [N_g, C] of one type."""
+    first = clouds[0]
+    device, dtype, ndim, count = first.device, first.dtype, first.shape[1], len(clouds)
+    sizes = [c.shape[0] for c in clouds]
+    n = sum(sizes)
+    ordered = torch.empty((n, ndim), dtype=dtype, device=device)
+    batch_dims = torch.empty((count + 1,), dtype=dtype, device=device)
+    rows, row_bytes, data = None, 0, None
+    addresses = ctypes.c_void_p * count
+    if features is not None:
+        channels = features[0].shape[1]
+        rows = torch.empty((n, channels), dtype=features[0].dtype, device=device)
+        row_bytes = channels * rows.element_size()
+        data = addresses(*[f.data_ptr() for f in features])
+    bounds = np.empty(8, dtype=np.int64)
+    with _on(device):
+        _check(load_library().mnt_collate(
+            addresses(*[c.data_ptr() for c in clouds]), data, (ctypes.c_int64 * count)(*sizes), count, ndim,
+            _INT[dtype], row_bytes, ordered.data_ptr(), batch_dims.data_ptr(), _ptr(rows), bounds.ctypes.data,
+            _stream(device)))
+    remember_bounds(ordered, bounds)
+    return ordered, batch_dims, rows
 
 
 def upload_ints(values: Sequence[int], dtype: torch.dtype, device: torch.device) -> torch.Tensor:

@@ -44,6 +44,36 @@ def voxelize(coordinates: torch.Tensor, voxel_size=1, dtype: torch.dtype = torch
     return unique, reverse
 
 
+def _one_call(coordinates: Sequence[torch.Tensor], features: Optional[Sequence[torch.Tensor]]) -> bool:
+    """Whether ``_C.collate`` takes these clouds: what it leaves out beside the
+    general way's tensor expressions is nothing that anybody sees."""
+    first = coordinates[0]
+    if (len(coordinates) > _C.MAX_GATHER_SOURCES or not isinstance(first, torch.Tensor) or not first.is_cuda
+            or first.dtype not in (torch.int32, torch.int64) or first.dim() != 2 or not 1 <= first.shape[1] <= 4
+            or not _C.plain(coordinates)):
+        return False
+    device, dtype, ndim, total = first.device, first.dtype, first.shape[1], 0
+    for c in coordinates:
+        if (c.dtype != dtype or c.device != device or c.dim() != 2 or c.shape[1] != ndim or not c.is_contiguous()):
+            return False
+        total += c.shape[0]
+    if not 0 < total <= 0x7FFFFFFF:
+        return False
+    if features is None:
+        return True
+    first = features[0]
+    if (not isinstance(first, torch.Tensor) or first.dim() != 2 or first.shape[1] == 0
+            or first.element_size() not in (2, 4, 8) or not _C.plain(features)
+            or total * first.shape[1] * first.element_size() > _C.MAX_GATHER_BYTES):
+        return False
+    dtype, channels = first.dtype, first.shape[1]
+    for f, c in zip(features, coordinates):
+        if (f.dtype != dtype or f.device != device or f.dim() != 2 or f.shape[1] != channels
+                or f.shape[0] != c.shape[0] or not f.is_contiguous()):
+            return False
+    return True
+
+
 def collate(coordinates: Sequence[torch.Tensor], features: Optional[Sequence[torch.Tensor]] = None):
     """One batch from several clouds of voxel coordinates (each free of
     duplicates, in any order): ``(coordinates, batch_dims)`` with every cloud
@@ -54,6 +84,9 @@ def collate(coordinates: Sequence[torch.Tensor], features: Optional[Sequence[tor
         raise ValueError("collate needs at least one cloud")
     if features is not None and len(features) != len(coordinates):
         raise ValueError("features and coordinates must list the same clouds")
+    if _one_call(coordinates, features):
+        ordered, batch_dims, rows = _C.collate(coordinates, features)
+        return (ordered, batch_dims) if features is None else (ordered, batch_dims, rows)
     stacked = torch.cat(list(coordinates), dim=0).contiguous()
     if not stacked.is_cuda:
         raise NotImplementedError

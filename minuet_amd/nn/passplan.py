@@ -21,6 +21,25 @@ from minuet_amd.nn.kernel_map import KernelMap
 __all__ = ["PassPlan", "BuiltPass"]
 
 _INVERSE, _GROUPS, _TABLES = 1, 2, 4
+_MAP_SHAPE = (_C.PassMap.num_offsets.offset // 8, _C.PassMap.num_sources.offset // 8, _C.PassMap.num_targets.offset // 8)
+_MAP_AT = _C.PassMap.at.offset // 8
+
+
+def requests_of(fast, reorder: bool):
+    """What a layer that ran through the extension module with the map of the request
+    ``fast`` (see ``PassPlan``) has asked for: that map, and the level it leads to."""
+    _, _, _, kind, key, transposed = fast
+    if key[0] != key[1]:
+        yield "coords", key[0], key[1]
+    yield "dense", key
+    if kind == "IMPLICIT":
+        if transposed:
+            yield "invert", key
+    elif kind == "GROUPS":
+        yield "groups", key
+    else:
+        yield "tables", key, reorder
+    yield fast
 
 
 class PassPlan:
@@ -97,6 +116,21 @@ class PassPlan:
         self.tiles = [(entry[1], entry[2]) for entry in self.requests if entry[0] == "tiles" and entry[1] in self.map_of
                       and (not entry[2] or wants.get(entry[1], 0) & _INVERSE)]
         self.fast = [entry for entry in self.requests if entry[0] == "fast" and self._serves(entry)]
+        # the library's results, one row of int64 words a map (the struct has no gaps)
+        self._map_words = np.frombuffer(self.maps, dtype=np.int64).reshape(len(self.map_of), -1)
+
+        # what there is beside tiles, and whether the layers of the extension module ask for all of it
+        self._tiles_asked = {entry for entry in self.requests if entry[0] == "tiles"}
+        self._asked = set(self.requests) - self._tiles_asked
+        self._fast_alone = self._asked == {asked for entry in self.fast
+                                           for asked in requests_of(entry, reorders.get(entry[4], False))}
+
+    def is_repeated(self, built, requests, tiles) -> bool:
+        """Whether a pass that ran on ``built``, whose layers asked Python for no more
+        than ``requests`` and would ask for ``tiles``, asked for just this plan's list:
+        ``is_for``, without putting that list together."""
+        return (self._fast_alone and tiles == self._tiles_asked and len(built.entries) == len(self.fast)
+                and all(entry.used for entry, _ in built.entries) and self._asked.issuperset(requests))
 
     def _serves(self, entry) -> bool:
         _, _, _, kind, key, transposed = entry
@@ -147,23 +181,26 @@ class BuiltPass:
         device = coordinates.device
         ndim = coordinates.shape[1]
         self.device = device
-        typed = store.view(coordinates.dtype)
+        typed = self.ints if coordinates.dtype == torch.int32 else store.view(coordinates.dtype)
         size = coordinates.dtype.itemsize
         self.coordinates = {plan.stride: (coordinates, plan.stride, batch_dims)}
+        boundaries = batch_dims.shape[0] if batch_dims is not None else 0
+        typed_dims = None if batch_dims is None else typed if batch_dims.dtype == coordinates.dtype else store.view(batch_dims.dtype)
+        self.batched = boundaries > 2    # (what says that there is one cloud is dropped)
         for target, level in plan.level_of.items():
             if level:
                 item = plan.levels[level - 1]
                 rows = typed.as_strided((item.count, ndim), (ndim, 1), item.coords_at // size)
                 dims = batch_dims
                 if item.batch_dims_at >= 0:
-                    dims = store.view(batch_dims.dtype).as_strided((batch_dims.shape[0],), (1,),
-                                                                   item.batch_dims_at // batch_dims.dtype.itemsize)
+                    dims = typed_dims.as_strided((boundaries,), (1,), item.batch_dims_at // batch_dims.dtype.itemsize)
                 elif batch_dims is not None:             # one cloud carrying its boundaries
                     dims = torch.tensor([0, item.count][:batch_dims.numel()], dtype=batch_dims.dtype, device=device)
                 self.coordinates[target] = (rows, target, dims)
-        self.at = {key: tuple(plan.maps[i].at) for key, i in plan.map_of.items()}
-        self.shape = {key: (plan.maps[i].num_offsets, plan.maps[i].num_sources, plan.maps[i].num_targets)
-                      for key, i in plan.map_of.items()}
+        words = plan._map_words.tolist()
+        self.at = {key: words[i][_MAP_AT:] for key, i in plan.map_of.items()}
+        o, s, t = _MAP_SHAPE
+        self.shape = {key: (words[i][o], words[i][s], words[i][t]) for key, i in plan.map_of.items()}
         self.entries = []                # (extension's entry, the request it stands for)
         self.tiles, self.stream = {}, None
         if plan.tiles:                   # (key, transposed) -> tiles, and the stream that makes them
@@ -246,24 +283,26 @@ class BuiltPass:
         for request in self.plan.fast:
             _, shape_id, in_stride, kind, key, transposed = request
             offsets, sources, targets = self.shape[key]
-            at = [None if a < 0 else self.base + a for a in self.at[key]]
             if kind == "IMPLICIT":
-                pointers = (at[1] if transposed else at[0],)
+                a = self.at[key][1 if transposed else 0]
+                pointers = (None if a < 0 else self.base + a,)
                 owners = self.store
             elif kind == "GROUPS":
                 table, address = self.plan._group_tables[key]
+                at = [None if a < 0 else self.base + a for a in self.at[key]]
                 pointers = (at[2], at[3], at[4], address)
                 owners = (self.store, table)
             else:
                 if not self.plan.reorders[key]:
                     continue
                 sizes_host, order_host = self._host(key)
+                at = [None if a < 0 else self.base + a for a in self.at[key]]
                 smask, tmask, in_idx = (at[6], at[5], at[8]) if transposed else (at[5], at[6], at[7])
                 pointers = (smask, tmask, at[10], at[9], sizes_host.ctypes.data, order_host.ctypes.data, in_idx)
                 owners = (self.store, self.hosts)
             source, target = (key[1], key[0]) if transposed else (key[0], key[1])
             coordinates, stride, batch_dims = self.coordinates[target]
-            if batch_dims is not None and len(batch_dims) <= 2:
+            if not self.batched:
                 batch_dims = None
             entry = host.MapEntry(getattr(host, kind), coordinates, stride, batch_dims, owners, index, 0,
                                   targets if transposed else sources, sources if transposed else targets, pointers,

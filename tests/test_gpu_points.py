@@ -6,6 +6,7 @@ import torch
 import minuet_oracle as orc
 from helpers import dev, host, random_cloud, sorted_unique
 from minuet_amd.nn import functional as F
+from minuet_amd.nn.functional import _C
 from minuet_amd.tensors import SparseTensor
 
 pytestmark = pytest.mark.gpu
@@ -76,6 +77,39 @@ def test_collate_carries_rows(channels, dtype, clouds):
     assert torch.equal(ordered, plain) and torch.equal(dims, plain_dims)
     np.testing.assert_array_equal(host(dims), bounds)
     assert torch.equal(rows, torch.cat(feats)[dev(order.astype(np.int64))])
+
+
+# rows in all: one, the small sort's 4 096 and one more, a bucket sort's, and more than it takes; clouds
+# without a row in front, between and behind; as many clouds as one call takes, and one more
+@pytest.mark.parametrize("sizes,ndim,dtype", [
+    ([1], 3, np.int32), ([0, 4091, 0, 5, 0], 3, np.int32), ([0, 4092, 5, 0], 4, np.int64), ([70] * 64, 2, np.int32),
+    ([70] * 65, 2, np.int64), ([40000, 1, 30001], 1, np.int64), ([131073, 2], 3, np.int32), ([2100001], 3, np.int32)])
+def test_collate_in_one_call(sizes, ndim, dtype):
+    coords = [random_cloud(n, 1 << 20, k, ndim=ndim, lo=-(1 << 19), dtype=dtype) for k, n in enumerate(sizes)]
+    feats = [torch.arange(3 * n, device="cuda", dtype=torch.float32).view(n, 3) - 7 * k for k, n in enumerate(sizes)]
+    ordered, dims, rows = F.collate([dev(c) for c in coords], feats)
+    bounds = np.concatenate([[0], np.cumsum(sizes)])
+    order = orc.arg_sort_coordinates(np.concatenate(coords), bounds.astype(dtype) if len(sizes) > 1 else None)
+    assert ordered.dtype == dims.dtype == torch.from_numpy(coords[0]).dtype
+    np.testing.assert_array_equal(host(ordered), np.concatenate(coords)[order])
+    np.testing.assert_array_equal(host(dims), bounds)
+    assert torch.equal(rows, torch.cat(feats)[dev(order.astype(np.int64))])
+    kept = _C.remembered_bounds(ordered)
+    stacked = np.concatenate(coords)
+    assert kept is None or (np.array_equal(kept[:ndim], stacked.min(0)) and np.array_equal(kept[4:4 + ndim], stacked.max(0)))
+
+
+def test_collate_of_other_forms():
+    """Clouds that the one call does not take: strided rows, mixed types."""
+    c = [dev(random_cloud(600, 50, k)) for k in range(2)]
+    f = [torch.randn(600, 2, device="cuda") for _ in c]
+    want = F.collate(c, f)
+    wide = [torch.stack([x, x], 2)[:, :, 0] for x in c]
+    assert not wide[0].is_contiguous()
+    for clouds, rows in ((wide, f), (c, [torch.stack([x, x], 2)[:, :, 0] for x in f])):
+        assert all(torch.equal(a, b) for a, b in zip(F.collate(clouds, rows), want))
+    mixed = F.collate([c[0].long(), c[1]], f)
+    assert mixed[0].dtype == torch.int64 and torch.equal(mixed[0].int(), want[0]) and torch.equal(mixed[2], want[2])
 
 
 def test_pools_beyond_values():
