@@ -565,10 +565,6 @@ __global__ __launch_bounds__(kQueryThreads) void query_kernel(
   // plus the reach.  The window is then a little larger than the exact one;
   // should it take more than one chunk, the searches are done after all.
   const bool by_buckets = halves && device_plan->window_buckets > 0;
-  // A cloud that fits one window chunk is the window itself: two searches of
-  // several dependent trips to memory less, for at most eight more keys staged
-  // per thread (a chain's query of 2 000 voxels: 19 -> 11 us with the split).
-  const bool whole_cloud = halves && !by_buckets && num_sources <= kWindowChunk;
   auto search_end = [&](int which) {
     const unsigned long long edge =
         which == 0 ? tgt(t0, frame) + static_cast<unsigned long long>(delta_min)
@@ -577,9 +573,7 @@ __global__ __launch_bounds__(kQueryThreads) void query_kernel(
     if (lane_id() == 0) s_bounds[which] = pos;
   };
   if (w < 2) {
-    if (whole_cloud) {
-      if (lane_id() == 0) s_bounds[w] = w == 0 ? t0 : num_sources;
-    } else if (!by_buckets) {
+    if (!by_buckets) {
       search_end(w);
     } else if (w == 0) {
       if (lane_id() == 0) s_bounds[0] = t0;
@@ -2302,6 +2296,36 @@ extern "C" int mnt_sorted_kernel_map_lists(const void *coords, int64_t n, int nd
     for (int64_t i = 0; i < num_offsets * ndim; ++i) {
       small_offsets = small_offsets && offsets_host[i] >= INT32_MIN / 2 && offsets_host[i] <= INT32_MAX / 2;
     }
+    // what a chain of launches leaves for the host: true where it went through
+    auto heard = [&](Arena &arena, unsigned long long sequence) -> bool {
+      arena.wait_flag(1, sequence);
+      const char *pinned = static_cast<const char *>(arena.pinned());
+      const long long *h_chain = reinterpret_cast<const long long *>(pinned + kChainHostOffset);
+      profile_mark("map_place+sync", stream);
+      if (h_chain[2 * MNT_MAX_NDIM] != 0) return false;
+      const unsigned *h_plan = reinterpret_cast<const unsigned *>(pinned + Arena::kPlanOffset);
+      for (int64_t j = 0; j < num_offsets; ++j) {
+        order_host_out[j] = h_plan[j];
+        sizes_host_out[j] = h_plan[2 * num_offsets + j];
+      }
+      memcpy(bounds_host_out, h_chain, sizeof(long long) * 2 * MNT_MAX_NDIM);
+      return true;
+    };
+    if (small_offsets && small_map_takes(n, static_cast<int>(std::min<int64_t>(num_offsets, 65535)))) {
+      profile_mark("enter:map_small", stream);
+      Arena &arena = Arena::of(stream);
+      arena.map_state_valid = false;
+      Scope scope(stream);
+      char *pinned_device = static_cast<char *>(arena.pinned_device());
+      const unsigned long long sequence = arena.next_sequence();
+      enqueue_small_map(coords, n, ndim, coord_dtype, offsets_host, static_cast<int>(num_offsets), map_halves_enabled(),
+                        reorder, indices_out, sorted_coords_out, in_idx_out, out_idx_out, sizes_dev_out, order_dev_out,
+                        scope, reinterpret_cast<unsigned *>(pinned_device + Arena::kPlanOffset),
+                        reinterpret_cast<long long *>(pinned_device + kChainHostOffset), arena.flag_device(1), sequence,
+                        stream);
+      if (heard(arena, sequence)) return;
+      // (crowded, equal rows, keys too wide: the calls below start over)
+    }
     if (small_offsets && chain_sort_takes(n, 1, static_cast<int>(num_offsets))) {
       profile_mark("enter:map_chain", stream);
       Arena &arena = Arena::of(stream);
@@ -2331,7 +2355,7 @@ extern "C" int mnt_sorted_kernel_map_lists(const void *coords, int64_t n, int nd
       unsigned *tile_mode = scope.alloc<unsigned>(num_tiles);
       unsigned *plan = scope.alloc<unsigned>(4 * num_offsets + 1);
       // (the cloud is mapped onto itself: offsets that come in pairs d / -d need one look-up per pair)
-      const OffsetTable table = make_offset_table(offsets_host, no, ndim, map_halves_enabled());
+      const OffsetTable table = make_offset_table<OffsetTable>(offsets_host, no, ndim, map_halves_enabled());
       int num_rows = 0;                            // offsets with rows of their own to write (DevicePlan::rows)
       for (int o = 0; o < no; ++o) num_rows += table.kind[o] != 1 ? 1 : 0;
       enqueue_chain_sort(coords, n, ndim, coord_dtype, indices_out, sorted_coords_out, buf, table, no, stream);
@@ -2358,18 +2382,7 @@ extern "C" int mnt_sorted_kernel_map_lists(const void *coords, int64_t n, int nd
                                                      sequence, sizes_dev_out, order_dev_out, buf.plan,
                                                      buf.folded, d_chain_host, repeats, total_copies(), kPlanMaxOffsets);
       check_launch("place_kernel");
-      arena.wait_flag(1, sequence);
-      const long long *h_chain = reinterpret_cast<const long long *>(static_cast<char *>(arena.pinned()) + kChainHostOffset);
-      profile_mark("map_place+sync", stream);
-      if (h_chain[2 * MNT_MAX_NDIM] == 0) {
-        const unsigned *h_plan = reinterpret_cast<const unsigned *>(static_cast<char *>(arena.pinned()) + Arena::kPlanOffset);
-        for (int64_t j = 0; j < num_offsets; ++j) {
-          order_host_out[j] = h_plan[j];
-          sizes_host_out[j] = h_plan[2 * num_offsets + j];
-        }
-        memcpy(bounds_host_out, h_chain, sizeof(long long) * 2 * MNT_MAX_NDIM);
-        return;
-      }
+      if (heard(arena, sequence)) return;
       // the chain declined (strong clustering, keys too wide): the calls below start over
     }
     if (mnt_arg_sort_coordinates(coords, n, ndim, coord_dtype, nullptr, 1, MNT_INT32, indices_out,

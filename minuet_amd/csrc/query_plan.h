@@ -27,23 +27,26 @@ constexpr int kPlanInts = 6 * kPlanMaxOffsets;   // 4 words per group + 2 per me
 // listed in ascending order of their coordinates, equal ones by index.  That is
 // the order of their key deltas: a field of the key has room for the difference
 // of any two offsets, so the first coordinate that differs decides.
-struct OffsetTable {
-  int v[kPlanMaxOffsets][MNT_MAX_NDIM];   // the looked-up offsets in that order
+template <int MOST>
+struct OffsetTableOf {
+  int v[MOST][MNT_MAX_NDIM];              // the looked-up offsets in that order
   int reach_lo[MNT_MAX_NDIM];             // least and largest step along each axis, over all offsets
   int reach_hi[MNT_MAX_NDIM];
   int num_kept;                           // offsets that are looked up
   int halves;
-  signed char origin[kPlanMaxOffsets];    // which offset each looked-up one is
-  signed char kind[kPlanMaxOffsets];
-  signed char mirror[kPlanMaxOffsets];
+  signed char origin[MOST];               // which offset each looked-up one is
+  signed char kind[MOST];
+  signed char mirror[MOST];
 };
+struct OffsetTable : OffsetTableOf<kPlanMaxOffsets> {};      // what a chain's kernels take
 
-// The table of num_offsets <= kPlanMaxOffsets offsets, rows of ndim coordinates.
-inline OffsetTable make_offset_table(const int64_t *offsets, int num_offsets, int ndim, bool allow_halves) {
-  OffsetTable table;
+// The table of num_offsets <= MOST offsets, rows of ndim coordinates.
+template <typename Table>
+inline Table make_offset_table(const int64_t *offsets, int num_offsets, int ndim, bool allow_halves) {
+  Table table;
   memset(&table, 0, sizeof(table));
   memset(table.mirror, -1, sizeof(table.mirror));
-  int order[kPlanMaxOffsets];
+  int order[sizeof(table.kind)];
   for (int o = 0; o < num_offsets; ++o) {
     for (int k = 0; k < ndim; ++k) {
       const int step = static_cast<int>(offsets[o * ndim + k]);

@@ -1524,40 +1524,48 @@ __global__ __launch_bounds__(1024) void bucket_pairs_kernel(const unsigned *__re
 // own.  What such a cloud waits for is launches: bounds, fold and two radix
 // passes were nine of them, 39 us of kernels and a wait at 2 000 rows; this is
 // 8.4 us.  In here the time goes to LDS round trips, hence bounds folded in ten shuffles instead of forty-eight (see
-// fold_extremes), 4 096 parts, and the chain's query plan made by one wavefront
-// while the others place rows.
+// fold_extremes) and 4 096 parts.
 // The split fails where more than kSmallPartRows rows agree in the top bits, or
 // where a key does not leave room for the row index: then nothing is written and
-// the verdict (status[0], host) says so.
-// With offsets it also clears `clear` and writes the query plan of a chain.
+// the verdict says so.
 constexpr int kSmallSortBlock = 1024;
 constexpr int kSmallSortItems = 4;
 constexpr int kSmallSortRows = kSmallSortBlock * kSmallSortItems;
 constexpr int kSmallPartBits = 12;
 constexpr unsigned kSmallPartRows = 384;
 
-struct SmallSortTell {            // where the host finds bounds and verdict (flag null: nobody waits)
+struct SmallSortTell {            // where the host finds bounds and verdict
   long long *bounds;
   unsigned *verdict;
   unsigned long long *flag;
   unsigned long long sequence;
 };
 
-template <typename CT, typename IT, bool kChain>
-__global__ __launch_bounds__(kSmallSortBlock) void small_sort_kernel(
-    const CT *__restrict__ coords, const IT *__restrict__ batch_dims, int num_batches, int ndim, int n, int idx_bits,
-    IT *__restrict__ indices_out, CT *__restrict__ sorted_out, SmallSortTell tell, long long *__restrict__ folded,
-    unsigned *__restrict__ status, unsigned *__restrict__ clear, int clear_words, OffsetTable offsets, int num_offsets,
-    DevicePlan *__restrict__ plan_out) {
-  constexpr int kWaves = kSmallSortBlock / kWave;
+struct SmallSortLds {
+  static constexpr int kWaves = kSmallSortBlock / kWave;
+  unsigned long long words[kSmallSortRows];
+  unsigned part[1 << kSmallPartBits];         // rows of a part, then its first row, then the row after its last
+  unsigned wave[kWaves], most[kWaves];
+  long long bounds[kWaves][8];
+};
+
+// What a workgroup knows of its cloud once the words lie in LDS part by part.
+struct SmallSorted {
+  long long b[2 * MNT_MAX_NDIM];              // extremes (slots past ndim repeat coordinate 0)
+  SortSpec spec;
+  int part_shift;                             // word >> this = part
+  bool go;
+};
+
+// The first half: everything up to the words in their parts.  `out.go` is the same in every thread.
+template <typename CT, typename IT>
+__device__ __forceinline__ void small_sort_deal(const CT *__restrict__ coords, const IT *__restrict__ batch_dims,
+                                                int num_batches, int ndim, int n, int idx_bits, SmallSortLds &lds,
+                                                SmallSorted &out) {
+  constexpr int kWaves = SmallSortLds::kWaves;
   constexpr int kParts = 1 << kSmallPartBits;
-  constexpr int kPerThread = kParts / kSmallSortBlock;
-  static_assert(kWaves == 16 && kPerThread == 4, "the folds over wavefronts and the scan of the parts");
+  static_assert(kWaves == 16 && kParts == 4 * kSmallSortBlock, "the folds over wavefronts and the scan of the parts");
   static_assert(2 * MNT_MAX_NDIM == 8, "eight extremes");
-  __shared__ __align__(16) unsigned long long s_words[kSmallSortRows];
-  __shared__ __align__(16) unsigned s_part[kParts];   // rows of a part, then its first row, then the row after its last
-  __shared__ unsigned s_wave[kWaves], s_most[kWaves];
-  __shared__ CT s_bounds[kWaves][8];
   const int tid = threadIdx.x, wave = tid / kWave, lane = lane_id();
   CT c[kSmallSortItems][MNT_MAX_NDIM];
 #pragma unroll
@@ -1565,12 +1573,7 @@ __global__ __launch_bounds__(kSmallSortBlock) void small_sort_kernel(
     const int i = r * kSmallSortBlock + tid;
     load_row_raw<CT>(coords + static_cast<long long>(i < n ? i : n - 1) * ndim, ndim, c[r]);
   }
-  *reinterpret_cast<uint4 *>(s_part + 4 * tid) = make_uint4(0u, 0u, 0u, 0u);
-  PlanLane lane_in;
-  if (kChain) {
-    if (wave == kWaves - 1) lane_in = load_plan_lane(offsets);
-    for (int i = tid; i < clear_words; i += kSmallSortBlock) clear[i] = 0u;
-  }
+  *reinterpret_cast<uint4 *>(lds.part + 4 * tid) = make_uint4(0u, 0u, 0u, 0u);
   // rows past the end repeat the last one: no extreme changes.  (~v turns the order round.)
   CT extreme[8];
 #pragma unroll
@@ -1585,11 +1588,11 @@ __global__ __launch_bounds__(kSmallSortBlock) void small_sort_kernel(
     }
   }
   const CT folded_wave = fold_extremes<CT>(extreme);
-  if (lane < 8) s_bounds[wave][lane] = folded_wave;
+  if (lane < 8) lds.bounds[wave][lane] = folded_wave;
   __syncthreads();
-  CT all = s_bounds[lane / 8][lane % 8];
+  CT all = static_cast<CT>(lds.bounds[lane / 8][lane % 8]);
   {
-    const CT second = s_bounds[8 + lane / 8][lane % 8];
+    const CT second = static_cast<CT>(lds.bounds[8 + lane / 8][lane % 8]);
     all = second < all ? second : all;
 #pragma unroll
     for (int d = 8; d < kWave; d <<= 1) {
@@ -1597,17 +1600,16 @@ __global__ __launch_bounds__(kSmallSortBlock) void small_sort_kernel(
       all = other < all ? other : all;
     }
   }
-  long long b[2 * MNT_MAX_NDIM];                      // (slots past ndim repeat coordinate 0)
 #pragma unroll
   for (int slot = 0; slot < 8; ++slot) {
     const CT v = __shfl(all, slot);
-    b[slot] = uniform64(static_cast<long long>(slot < MNT_MAX_NDIM ? v : static_cast<CT>(~v)));
+    out.b[slot] = uniform64(static_cast<long long>(slot < MNT_MAX_NDIM ? v : static_cast<CT>(~v)));
   }
   CoordSource<CT, IT> src;
   src.coords = coords;
   src.batch_dims = batch_dims;
   src.perm = nullptr;
-  const int key_bits = single_round_spec(b, ndim, num_batches, src.spec);
+  const int key_bits = single_round_spec(out.b, ndim, num_batches, src.spec);
   const int word_bits = key_bits + idx_bits;
   bool go = word_bits <= 64;
   unsigned long long word[kSmallSortItems];
@@ -1621,12 +1623,12 @@ __global__ __launch_bounds__(kSmallSortBlock) void small_sort_kernel(
       unsigned row;
       src.pack(i, c[r], key, row);
       word[r] = (key << idx_bits) | static_cast<unsigned long long>(row);
-      atomicAdd(&s_part[static_cast<unsigned>(word[r] >> part_shift)], 1u);
+      atomicAdd(&lds.part[static_cast<unsigned>(word[r] >> part_shift)], 1u);
     }
   }
   __syncthreads();
   {
-    const uint4 count = *reinterpret_cast<const uint4 *>(s_part + 4 * tid);
+    const uint4 count = *reinterpret_cast<const uint4 *>(lds.part + 4 * tid);
     const unsigned mine = count.x + count.y + count.z + count.w;
     unsigned inclusive = mine;
     unsigned most = max(max(count.x, count.y), max(count.z, count.w));
@@ -1635,65 +1637,370 @@ __global__ __launch_bounds__(kSmallSortBlock) void small_sort_kernel(
       if (lane >= off) inclusive += u;
     }
     const bool crowded = __any(most > kSmallPartRows);
-    if (lane == kWave - 1) s_wave[wave] = inclusive;
-    if (lane == 0) s_most[wave] = crowded ? 1u : 0u;
+    if (lane == kWave - 1) lds.wave[wave] = inclusive;
+    if (lane == 0) lds.most[wave] = crowded ? 1u : 0u;
     __syncthreads();
-    const unsigned theirs = s_wave[lane % kWaves];
-    go = go && !__any(s_most[lane % kWaves] != 0);    // the same in every thread
+    const unsigned theirs = lds.wave[lane % kWaves];
+    go = go && !__any(lds.most[lane % kWaves] != 0);  // the same in every thread
     unsigned before = lane < wave ? theirs : 0u;      // (wave < 16: lanes 0 .. wave - 1)
 #pragma unroll
     for (int d = 8; d >= 1; d >>= 1) before += __shfl_xor(before, d);
     before = __shfl(before, 0);
     const unsigned at = before + inclusive - mine;
-    *reinterpret_cast<uint4 *>(s_part + 4 * tid) =
+    *reinterpret_cast<uint4 *>(lds.part + 4 * tid) =
         make_uint4(at, at + count.x, at + count.x + count.y, at + count.x + count.y + count.z);
   }
   __syncthreads();
-  if (tid == 0) {
-    if (kChain) {
-#pragma unroll
-      for (int slot = 0; slot < 2 * MNT_MAX_NDIM; ++slot) folded[slot] = b[slot];
-      status[0] = go ? 0u : 1u;                       // (among the words cleared above, before a barrier)
-    }
-    if (tell.flag != nullptr) {
-#pragma unroll
-      for (int slot = 0; slot < 2 * MNT_MAX_NDIM; ++slot) tell.bounds[slot] = b[slot];
-      tell.verdict[0] = go ? 0u : 1u;
-      __threadfence_system();
-      __hip_atomic_store(tell.flag, tell.sequence, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
-  }
   if (go) {
 #pragma unroll
     for (int r = 0; r < kSmallSortItems; ++r) {
       const int i = r * kSmallSortBlock + tid;
-      if (i < n) s_words[atomicAdd(&s_part[static_cast<unsigned>(word[r] >> part_shift)], 1u)] = word[r];
+      if (i < n) lds.words[atomicAdd(&lds.part[static_cast<unsigned>(word[r] >> part_shift)], 1u)] = word[r];
     }
   }
   __syncthreads();
-  if (kChain) {
-    if (wave == kWaves - 1 && plan_out != nullptr) {
-      make_plan_on_device(b, lane_in, offsets, num_offsets, ndim, go ? 0u : 1u, plan_out);
-    }
+  out.spec = src.spec;
+  out.part_shift = part_shift;
+  out.go = go;
+}
+
+// The second half: the place of word number e in the order of all.
+__device__ __forceinline__ unsigned small_sort_rank(const SmallSortLds &lds, unsigned long long mine, int part_shift) {
+  const unsigned part = static_cast<unsigned>(mine >> part_shift);
+  const unsigned from = part == 0 ? 0u : lds.part[part - 1], to = lds.part[part];
+  unsigned rank = from, j = from;
+  for (; j + 4 <= to; j += 4) {                       // four reads in flight
+    const unsigned long long x0 = lds.words[j], x1 = lds.words[j + 1], x2 = lds.words[j + 2], x3 = lds.words[j + 3];
+    rank += (x0 < mine ? 1u : 0u) + (x1 < mine ? 1u : 0u) + (x2 < mine ? 1u : 0u) + (x3 < mine ? 1u : 0u);
   }
-  if (!go) return;
-  const KeySink<CT, IT> sink{src.spec, indices_out, sorted_out};
+  for (; j < to; ++j) rank += lds.words[j] < mine ? 1u : 0u;
+  return rank;
+}
+
+template <typename CT, typename IT>
+__global__ __launch_bounds__(kSmallSortBlock) void small_sort_kernel(
+    const CT *__restrict__ coords, const IT *__restrict__ batch_dims, int num_batches, int ndim, int n, int idx_bits,
+    IT *__restrict__ indices_out, CT *__restrict__ sorted_out, SmallSortTell tell) {
+  __shared__ __align__(16) SmallSortLds lds;
+  SmallSorted s;
+  small_sort_deal<CT, IT>(coords, batch_dims, num_batches, ndim, n, idx_bits, lds, s);
+  const int tid = threadIdx.x;
+  if (tid == 0) {
+#pragma unroll
+    for (int slot = 0; slot < 2 * MNT_MAX_NDIM; ++slot) tell.bounds[slot] = s.b[slot];
+    tell.verdict[0] = s.go ? 0u : 1u;
+    __threadfence_system();
+    __hip_atomic_store(tell.flag, tell.sequence, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+  if (!s.go) return;
+  const KeySink<CT, IT> sink{s.spec, indices_out, sorted_out};
   const unsigned long long idx_mask = (1ull << idx_bits) - 1ull;
 #pragma unroll
   for (int r = 0; r < kSmallSortItems; ++r) {
     const int e = r * kSmallSortBlock + tid;
     if (e >= n) continue;
-    const unsigned long long mine = s_words[e];
-    const unsigned part = static_cast<unsigned>(mine >> part_shift);
-    const unsigned from = part == 0 ? 0u : s_part[part - 1], to = s_part[part];
-    unsigned rank = from, j = from;
-    for (; j + 4 <= to; j += 4) {                     // four reads in flight
-      const unsigned long long x0 = s_words[j], x1 = s_words[j + 1], x2 = s_words[j + 2], x3 = s_words[j + 3];
-      rank += (x0 < mine ? 1u : 0u) + (x1 < mine ? 1u : 0u) + (x2 < mine ? 1u : 0u) + (x3 < mine ? 1u : 0u);
-    }
-    for (; j < to; ++j) rank += s_words[j] < mine ? 1u : 0u;
-    sink.store(rank, mine >> idx_bits, static_cast<unsigned>(mine & idx_mask));
+    const unsigned long long mine = lds.words[e];
+    sink.store(small_sort_rank(lds, mine, s.part_shift), mine >> idx_bits, static_cast<unsigned>(mine & idx_mask));
   }
+}
+
+// The whole Map step of a cloud that one workgroup sorts (mapped onto itself): a
+// workgroup per offset that is looked up, and one for the zero offset where the
+// offsets come in pairs.  Each sorts the cloud for itself, finds its offset's
+// sources among the keys in LDS, tells the others how many hits there are, hears
+// of theirs and writes the pair lists of its offset and of the mirror image where
+// all of them say that these begin.
+//
+// What bounds it: latency, 8.4 us of it the sort.  As three launches (sort, query,
+// lists) the step was 26.5 us of kernels and the gaps between them: 45.5 us a
+// call at 2 039 voxels under 3x3x3, 16.4 and 35.8 here.  The numbers are the only thing
+// that passes between workgroups, each in one word with the call's number beside
+// it, so nothing is cleared and no fence is needed.  A workgroup that has waited
+// `patience` ticks (of 10 ns) counts the hits it has not heard of itself: it
+// depends on no other to come to its end.
+struct SmallMapOut {
+  int *in_idx, *out_idx, *sizes, *order;      // (the last two nullable)
+  unsigned long long *counts;                 // [num_offsets]
+  unsigned *plan_host;                        // order, ., sizes: num_offsets words each
+  long long *chain_host;                      // extremes, then the verdict
+  unsigned long long *flag;
+  unsigned long long sequence;
+  int reorder;
+  unsigned patience;
+};
+constexpr int kSmallMapOffsets = 128;
+constexpr int kSmallMapCountBits = 13;
+static_assert(kSmallSortRows < 1 << kSmallMapCountBits, "a count beside the call's number");
+struct SmallMapTable : OffsetTableOf<kSmallMapOffsets> {};
+
+template <typename CT>
+__global__ __launch_bounds__(kSmallSortBlock) void small_map_kernel(
+    const CT *__restrict__ coords, int ndim, int n, int idx_bits, int *__restrict__ indices_out,
+    CT *__restrict__ sorted_out, SmallMapTable offsets, int num_offsets, int zero_offset, SmallMapOut out) {
+  constexpr int kWaves = SmallSortLds::kWaves;
+  __shared__ __align__(16) SmallSortLds lds;
+  __shared__ unsigned long long s_key[kSmallSortRows];      // the keys in order
+  __shared__ unsigned s_count[kSmallSortItems * kWaves];
+  __shared__ unsigned s_base[2], s_missing[kSmallMapOffsets / 32], s_own[kSmallMapOffsets];
+  const int tid = threadIdx.x, lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  // what this workgroup looks up, read while the cloud is on its way
+  const int kept = blockIdx.x;
+  const bool identity = kept == offsets.num_kept;
+  const int own = identity ? zero_offset : offsets.origin[kept];
+  const int twin = !identity && offsets.halves != 0 ? offsets.mirror[own] : -1;
+  SmallSorted s;
+  small_sort_deal<CT, int>(coords, nullptr, 1, ndim, n, idx_bits, lds, s);
+  const unsigned long long idx_mask = (1ull << idx_bits) - 1ull;
+  bool repeated = false;
+  if (s.go) {
+    const KeySink<CT, int> sink{s.spec, indices_out, sorted_out};
+#pragma unroll
+    for (int r = 0; r < kSmallSortItems; ++r) {
+      const int e = r * kSmallSortBlock + tid;
+      if (e >= n) continue;
+      const unsigned long long mine = lds.words[e];
+      const unsigned rank = small_sort_rank(lds, mine, s.part_shift);
+      s_key[rank] = mine >> idx_bits;
+      // (the workgroups write the sorted cloud together, 64 places each in turn; the
+      // words of a part lie in another order in each)
+      if ((rank >> 6) % gridDim.x == blockIdx.x) {
+        sink.store(rank, mine >> idx_bits, static_cast<unsigned>(mine & idx_mask));
+      }
+    }
+  }
+  __syncthreads();
+  if (s.go) {
+#pragma unroll
+    for (int r = 0; r < kSmallSortItems; ++r) {
+      const int i = r * kSmallSortBlock + tid;
+      repeated = repeated || (i + 1 < n && s_key[i] == s_key[i + 1]);
+    }
+  }
+  // equal rows: the halves do not mirror each other, and more than one row is a hit
+  const int verdict = !s.go ? 1 : __syncthreads_or(repeated ? 1 : 0) != 0 ? 3 : 0;
+  if (verdict != 0) {
+    if (blockIdx.x == 0 && tid == 0) {
+      out.chain_host[2 * MNT_MAX_NDIM] = static_cast<long long>(verdict);
+      __threadfence_system();
+      __hip_atomic_store(out.flag, out.sequence, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    return;
+  }
+
+  // the source of target i under a looked-up offset, or -1
+  auto source_of = [&](int i, int o) -> int {
+    const unsigned long long key = s_key[i];
+    unsigned long long wanted = 0;
+    bool inside = true;
+#pragma unroll
+    for (int k = 0; k < MNT_MAX_NDIM; ++k) {
+      if (k < ndim) {
+        const unsigned long long range =
+            static_cast<unsigned long long>(s.b[MNT_MAX_NDIM + k]) - static_cast<unsigned long long>(s.b[k]);
+        const unsigned long long v = ((key >> s.spec.shift[k]) & s.spec.mask[k]) +
+                                     static_cast<unsigned long long>(static_cast<long long>(offsets.v[o][k]));
+        inside = inside && v <= range;         // (below 0 it wraps to a huge value)
+        wanted |= v << s.spec.shift[k];
+      }
+    }
+    if (!inside) return -1;
+    const unsigned first = static_cast<unsigned>((wanted << idx_bits) >> s.part_shift);
+    const unsigned last = static_cast<unsigned>(((wanted << idx_bits) | idx_mask) >> s.part_shift);
+    unsigned from = first == 0 ? 0u : lds.part[first - 1], to = lds.part[last];
+    while (to - from > 4) {
+      const unsigned mid = (from + to) >> 1;
+      if (s_key[mid] <= wanted) {
+        from = mid;
+      } else {
+        to = mid;
+      }
+    }
+    int found = -1;
+#pragma unroll
+    for (unsigned x = 0; x < 4; ++x) {
+      const unsigned at = from + x < to ? from + x : 0u;
+      found = from < to && s_key[at] == wanted ? static_cast<int>(at) : found;
+    }
+    return found;
+  };
+  int found[kSmallSortItems];
+  unsigned long long votes[kSmallSortItems];
+#pragma unroll
+  for (int r = 0; r < kSmallSortItems; ++r) {
+    const int i = r * kSmallSortBlock + tid;
+    found[r] = i < n ? (identity ? i : source_of(i, kept)) : -1;
+    votes[r] = __ballot(found[r] >= 0);
+    if (lane == 0) s_count[r * kWaves + wave] = __popcll(votes[r]);
+  }
+  __syncthreads();
+  static_assert(kSmallSortItems * kWaves == kWave, "a lane per wavefront and item");
+  const unsigned mine = s_count[lane];
+  unsigned inclusive = mine;
+#pragma unroll
+  for (int off = 1; off < kWave; off <<= 1) {
+    const unsigned u = __shfl_up(inclusive, off);
+    if (lane >= off) inclusive += u;
+  }
+  const unsigned own_hits = __builtin_amdgcn_readlane(inclusive, kWave - 1);
+  if (tid == 0) {
+    __hip_atomic_store(out.counts + own, out.sequence << kSmallMapCountBits | own_hits, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+  }
+
+  // the hits of every offset: two of them a lane, in the first wavefront
+  constexpr int kEach = kSmallMapOffsets / kWave;
+  unsigned size[kEach];
+  if (wave == 0) {
+    unsigned long long heard[kEach];
+    int from[kEach];
+#pragma unroll
+    for (int e = 0; e < kEach; ++e) {
+      const int o = e * kWave + lane;
+      from[e] = o < num_offsets ? (offsets.halves != 0 && offsets.kind[o] == 1 ? offsets.mirror[o] : o) : own;
+    }
+    const long long start = wall_clock64();
+    bool all = false;
+    do {
+      all = true;
+#pragma unroll
+      for (int e = 0; e < kEach; ++e) {
+        heard[e] = load_through(out.counts + from[e]);
+        all = all && (heard[e] >> kSmallMapCountBits) == (out.sequence & (~0ull >> kSmallMapCountBits));
+      }
+      all = __ballot(!all) == 0ull;
+    } while (!all && wall_clock64() - start < static_cast<long long>(out.patience));
+#pragma unroll
+    for (int e = 0; e < kEach; ++e) {
+      const bool there = (heard[e] >> kSmallMapCountBits) == (out.sequence & (~0ull >> kSmallMapCountBits));
+      size[e] = static_cast<unsigned>(heard[e]) & ((1u << kSmallMapCountBits) - 1u);
+      const unsigned long long silent = __ballot(!there);
+      if (lane < 2) s_missing[2 * e + lane] = static_cast<unsigned>(silent >> (32 * lane));
+    }
+  }
+  __syncthreads();
+  if ((s_missing[0] | s_missing[1] | s_missing[2] | s_missing[3]) != 0u) {
+    // not heard of in time: counted here (every looked-up offset, whoever was silent)
+    for (int i = tid; i < kSmallMapOffsets; i += kSmallSortBlock) s_own[i] = 0u;
+    __syncthreads();
+    for (int row = 0; row < offsets.num_kept; ++row) {
+      unsigned hits = 0;
+      for (int i = tid; i < n; i += kSmallSortBlock) hits += source_of(i, row) >= 0 ? 1u : 0u;
+      for (int off = 32; off > 0; off >>= 1) hits += __shfl_xor(hits, off);
+      if (lane == 0 && hits != 0) {
+        atomicAdd(&s_own[offsets.origin[row]], hits);
+        if (offsets.halves != 0) atomicAdd(&s_own[offsets.mirror[offsets.origin[row]]], hits);
+      }
+    }
+    if (tid == 0 && zero_offset >= 0) s_own[zero_offset] = static_cast<unsigned>(n);
+    __syncthreads();
+    if (wave == 0) {
+#pragma unroll
+      for (int e = 0; e < kEach; ++e) size[e] = s_own[e * kWave + lane];
+    }
+  }
+  if (wave == 0) {
+    // Where a row of the lists begins: behind those of fewer hits, or of as many and a lower number.
+    auto size_of = [&](int o) -> unsigned {
+      const unsigned low = __builtin_amdgcn_readlane(size[0], o & (kWave - 1));
+      const unsigned high = __builtin_amdgcn_readlane(size[1], o & (kWave - 1));
+      return o < kWave ? low : high;
+    };
+    static_assert(kEach == 2, "two offsets a lane");
+#pragma unroll
+    for (int which = 0; which < 2; ++which) {
+      const int row = which == 0 ? own : twin;
+      const unsigned hits = row >= 0 ? size_of(row) : 0u;
+      unsigned before = 0;
+#pragma unroll
+      for (int e = 0; e < kEach; ++e) {
+        const int o = e * kWave + lane;
+        const bool first = out.reorder != 0 ? size[e] < hits || (size[e] == hits && o < row) : o < row;
+        before += o < num_offsets && first ? size[e] : 0u;
+      }
+      for (int off = 32; off > 0; off >>= 1) before += __shfl_xor(before, off);
+      if (lane == 0) s_base[which] = before;
+    }
+    if (blockIdx.x == 0) {
+      // the first workgroup tells the host: sizes and order, extremes, verdict
+      int place[kEach];
+#pragma unroll
+      for (int e = 0; e < kEach; ++e) place[e] = out.reorder != 0 ? 0 : e * kWave + lane;
+      if (out.reorder != 0) {
+        for (int p = 0; p < num_offsets; ++p) {
+          const unsigned other = size_of(p);
+#pragma unroll
+          for (int e = 0; e < kEach; ++e) {
+            place[e] += other < size[e] || (other == size[e] && p < e * kWave + lane) ? 1 : 0;
+          }
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < kEach; ++e) {
+        const int o = e * kWave + lane;
+        if (o >= num_offsets) continue;
+        out.plan_host[place[e]] = static_cast<unsigned>(o);
+        out.plan_host[2 * num_offsets + place[e]] = size[e];
+        if (out.order != nullptr) out.order[place[e]] = o;
+        if (out.sizes != nullptr) out.sizes[place[e]] = static_cast<int>(size[e]);
+      }
+      if (lane == 0) {
+#pragma unroll
+        for (int slot = 0; slot < 2 * MNT_MAX_NDIM; ++slot) out.chain_host[slot] = s.b[slot];
+        out.chain_host[2 * MNT_MAX_NDIM] = 0;
+        __threadfence_system();
+        __hip_atomic_store(out.flag, out.sequence, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+      }
+    }
+  }
+  __syncthreads();
+  const unsigned base = s_base[0], base_twin = s_base[1];
+#pragma unroll
+  for (int r = 0; r < kSmallSortItems; ++r) {
+    const unsigned earlier = __builtin_amdgcn_readlane(inclusive - mine, r * kWaves + wave);
+    if (found[r] < 0) continue;
+    const unsigned at = earlier + __popcll(votes[r] & lanes_below());
+    const int i = r * kSmallSortBlock + tid;
+    out.in_idx[base + at] = found[r];
+    out.out_idx[base + at] = i;
+    if (twin >= 0) {
+      out.in_idx[base_twin + at] = i;
+      out.out_idx[base_twin + at] = found[r];
+    }
+  }
+}
+
+bool small_map_takes(int64_t n, int num_offsets) { return n <= kSmallSortRows && num_offsets <= kSmallMapOffsets; }
+
+// Ticks of 10 ns that a workgroup waits for another's count: a hundred times what
+// it takes.  (MINUET_MAP_PATIENCE, for tests: 0 lets every workgroup count for itself.)
+static unsigned map_patience() {
+  const char *text = std::getenv("MINUET_MAP_PATIENCE");
+  return text == nullptr || *text == 0 ? 20000u : static_cast<unsigned>(std::max(0, std::atoi(text)));
+}
+
+void enqueue_small_map(const void *coords, int64_t n, int ndim, int coord_dtype, const int64_t *offsets_host,
+                       int num_offsets, bool allow_halves, int reorder, int32_t *indices_out, void *sorted_out,
+                       int32_t *in_idx, int32_t *out_idx, int32_t *sizes, int32_t *order, Scope &scope,
+                       unsigned *plan_host, long long *chain_host, unsigned long long *flag,
+                       unsigned long long sequence, hipStream_t stream) {
+  const SmallMapTable table = make_offset_table<SmallMapTable>(offsets_host, num_offsets, ndim, allow_halves);
+  int zero = -1;
+  for (int o = 0; o < num_offsets; ++o) zero = table.kind[o] == 2 ? o : zero;
+  const SmallMapOut out{in_idx, out_idx, sizes, order, scope.alloc<unsigned long long>(num_offsets), plan_host,
+                        chain_host, flag, sequence, reorder, map_patience()};
+  const unsigned blocks = static_cast<unsigned>(table.num_kept + (zero >= 0 ? 1 : 0));
+  const int idx_bits = bit_width(static_cast<unsigned long long>(n - 1));
+  if (coord_dtype == MNT_INT32) {
+    small_map_kernel<int32_t><<<blocks, kSmallSortBlock, 0, stream>>>(
+        static_cast<const int32_t *>(coords), ndim, static_cast<int>(n), idx_bits, indices_out,
+        static_cast<int32_t *>(sorted_out), table, num_offsets, zero, out);
+  } else {
+    small_map_kernel<int64_t><<<blocks, kSmallSortBlock, 0, stream>>>(
+        static_cast<const int64_t *>(coords), ndim, static_cast<int>(n), idx_bits, indices_out,
+        static_cast<int64_t *>(sorted_out), table, num_offsets, zero, out);
+  }
+  check_launch("small_map_kernel");
 }
 
 static bool chain_slabs_enabled() {
@@ -1719,7 +2026,7 @@ size_t chain_sort_words(int64_t n) {
 }
 
 bool chain_sort_takes(int64_t n, int64_t num_batches, int num_offsets) {
-  return (n <= kSmallSortRows || n <= bucket_sort_max_rows()) && n <= (int64_t(1) << 21) && num_batches <= 1 &&
+  return n > kSmallSortRows && n <= bucket_sort_max_rows() && n <= (int64_t(1) << 21) && num_batches <= 1 &&
          num_offsets >= 1 && num_offsets <= kPlanMaxOffsets;
 }
 
@@ -1728,14 +2035,6 @@ static void enqueue_chain_sort_typed(const CT *coords, int64_t n, int ndim, int3
                                      CT *sorted_out, const ChainSortBuffers &buf,
                                      const OffsetTable &offsets, int num_offsets, hipStream_t stream) {
   const int idx_bits = bit_width(static_cast<unsigned long long>(n - 1));
-  if (n <= kSmallSortRows) {
-    small_sort_kernel<CT, int32_t, true><<<1, kSmallSortBlock, 0, stream>>>(
-        coords, nullptr, 1, ndim, static_cast<int>(n), idx_bits, indices_out, sorted_out, SmallSortTell{}, buf.folded,
-        buf.status, buf.counters, buf.counter_words, offsets, num_offsets, buf.plan);
-    check_launch("small_sort_kernel");
-    profile_mark("sort_small", stream);
-    return;
-  }
   const int msd_cap = chain_sort_msd_bits(n);
   const int buckets = 1 << msd_cap;
   const int num_partials = static_cast<int>(std::min<int64_t>(div_ceil(n, kBoundsBlock * 4), kBucketBoundsBlocks));
@@ -1857,12 +2156,9 @@ static void arg_sort_typed(const CT *coords, int64_t n, int ndim, const IT *batc
     char *pinned = static_cast<char *>(arena.pinned_device());
     const SmallSortTell tell{reinterpret_cast<long long *>(pinned),
                              reinterpret_cast<unsigned *>(pinned + kBucketHostOffset), arena.flag_device(3), sequence};
-    OffsetTable none;
-    memset(&none, 0, sizeof(none));
-    small_sort_kernel<CT, IT, false><<<1, kSmallSortBlock, 0, stream>>>(
+    small_sort_kernel<CT, IT><<<1, kSmallSortBlock, 0, stream>>>(
         coords, batched ? batch_dims : nullptr, batches_in_key, ndim, static_cast<int>(n),
-        bit_width(static_cast<unsigned long long>(n - 1)), indices_out, sorted_out, tell, nullptr, nullptr, nullptr, 0,
-        none, 0, nullptr);
+        bit_width(static_cast<unsigned long long>(n - 1)), indices_out, sorted_out, tell);
     check_launch("small_sort_kernel");
     arena.wait_flag(3, sequence);
     memcpy(h_bounds, arena.pinned(), sizeof(long long) * 8);

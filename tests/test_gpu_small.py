@@ -1,6 +1,7 @@
 """Clouds around one workgroup: the sort in one launch and the split look-up of the chain."""
 import numpy as np
 import pytest
+import torch
 
 import c_oracle
 import minuet_oracle as orc
@@ -41,7 +42,10 @@ def test_sort_around_one_workgroup(n, shape):
 def test_map_lists_of_small_clouds(n, kernel, extent, halves):
     c, _ = sorted_unique(random_cloud(n, extent, n + kernel, lo=-extent // 2))
     c = c[np.random.default_rng(n).permutation(c.shape[0])]
-    off = orc.generate_kernel_offsets(3, kernel, 1, 1)
+    check_map_lists(c, orc.generate_kernel_offsets(3, kernel, 1, 1))
+
+
+def check_map_lists(c, off):
     index, rows, built = _C.sorted_kernel_map_lists(dev(c), off.astype(np.int64))
     order = orc.arg_sort_coordinates(c)
     np.testing.assert_array_equal(host(index).astype(np.int64), order)
@@ -53,3 +57,33 @@ def test_map_lists_of_small_clouds(n, kernel, extent, halves):
     np.testing.assert_array_equal(built["sizes_host"], np.asarray(sizes)[by_size])
     np.testing.assert_array_equal(host(built["in_idx"]), ein)
     np.testing.assert_array_equal(host(built["out_idx"]), eout)
+
+
+# 125 and 49 offsets (two a lane), offsets past the cloud, coordinates of 64 bits far apart, one to four
+# dimensions; workgroups that hear of the others' counts, and such that count for themselves
+@pytest.mark.parametrize("patience", [None, "0"])
+@pytest.mark.parametrize("n,ndim,kernel,dilation,dtype", [
+    (4096, 3, 5, 1, np.int32), (2039, 3, 3, 2, np.int64), (700, 2, 7, 1, np.int32), (65, 4, 3, 1, np.int32),
+    (3000, 1, 3, 1, np.int64), (1500, 3, 5, 40, np.int32), (4096, 3, 4, 1, np.int32)])
+def test_map_lists_in_one_launch(n, ndim, kernel, dilation, dtype, patience, monkeypatch):
+    if patience is not None:
+        monkeypatch.setenv("MINUET_MAP_PATIENCE", patience)
+    extent = int(round((3 * n) ** (1 / ndim)))
+    c, _ = sorted_unique(random_cloud(n, extent, n + kernel, ndim=ndim, lo=-extent // 2, dtype=dtype))
+    if dtype == np.int64:
+        c[-1] += 1 << 40 // ndim
+    c = c[np.random.default_rng(n).permutation(c.shape[0])]
+    check_map_lists(c, orc.generate_kernel_offsets(ndim, kernel, 1, dilation))
+
+
+def test_map_lists_of_equal_rows():
+    """The one launch turns such a cloud down, whoever of the workgroups sees it."""
+    c = random_cloud(3000, 12, 8, duplicates=0.3)
+    order = orc.arg_sort_coordinates(c)
+    off = orc.generate_kernel_offsets(3, 3, 1, 1)
+    index, rows, built = _C.sorted_kernel_map_lists(dev(c), off.astype(np.int64))
+    np.testing.assert_array_equal(host(index).astype(np.int64), order)
+    whole = _C.kernel_map_build(rows, rows, off.astype(np.int64), None, None, reorder=True, want_masks=False, want_lists=True)
+    for name in ("in_idx", "out_idx"):
+        assert torch.equal(built[name], whole[name])
+    np.testing.assert_array_equal(built["sizes_host"], whole["sizes_host"])
