@@ -226,7 +226,7 @@ __device__ __forceinline__ void resolve_chunk(
 template <bool kCollect>
 __device__ __forceinline__ void settle_group_staged(
     const unsigned (&cand)[kGroupSpan + 1], int p, unsigned long long d0, const int2 (&member)[kGroupSpan + 1],
-    int members, long long c0, bool inside, unsigned *s_counts, long long num_targets,
+    int first_member, int members, long long c0, bool inside, unsigned *s_counts, long long num_targets,
     const HitSink &sink, long long wave_t0, unsigned &votes_lo, unsigned &votes_hi) {
   const unsigned q0_rel = static_cast<unsigned>(d0);
   // the largest step of a group is kGroupSpan: one test of the key range for all members
@@ -250,7 +250,7 @@ __device__ __forceinline__ void settle_group_staged(
     int *slots = sink.stage + (static_cast<long long>(o) * num_targets + wave_t0);
     if (hit) slots[rank] = found_base + at;
     if (kCollect) {
-      const bool keeper = static_cast<int>(lane_id()) == o;
+      const bool keeper = static_cast<int>(lane_id()) == first_member + m;
       votes_lo = keeper ? lo : votes_lo;
       votes_hi = keeper ? hi : votes_hi;
     } else if (lane_id() == 0 && wave_t0 < num_targets) {
@@ -265,16 +265,16 @@ __device__ __forceinline__ void resolve_chunk_rows(
     const unsigned *__restrict__ win, const unsigned short *__restrict__ dir, int len, int zbits,
     unsigned num_rows, unsigned long long base, long long c0, unsigned long long key, bool valid,
     unsigned long long first_key, unsigned long long next_first, const int4 *s_groups,
-    const int2 *s_members, int num_groups, unsigned *s_counts, bool count_hits, long long t,
+    const int2 *s_members, int num_groups, int num_members, unsigned *s_counts, bool count_hits, long long t,
     long long num_targets, OT *__restrict__ kernel_map, const HitSink &sink) {
   OT *column = kernel_map + t;
   constexpr bool kStaged = kWholeWindow && kLists;
-  // staged form: up to 64 offsets leave their ballots in the lanes of one
-  // register pair; they are stored once, after the last group
-  const bool collect = kStaged && sink.num_offsets <= kWave;
+  // staged form: up to 64 looked-up offsets leave their ballots in the lanes of
+  // one register pair; they are stored once, after the last group
+  const bool collect = kStaged && num_members <= kWave;
   const long long wave_t0 = uniform64(t - lane_id());
   unsigned votes_lo = 0, votes_hi = 0;
-  unsigned long long mine = 0;                  // the offsets this workgroup looks up (a split takes a share of them)
+  unsigned long long mine = 0;                  // the members this workgroup looks up (a split takes a share of them)
   // three groups in lockstep: their directory reads, then their candidate
   // reads, are in flight together
   for (int g0 = 0; g0 < num_groups; g0 += kGroupsInFlight) {
@@ -348,16 +348,14 @@ __device__ __forceinline__ void resolve_chunk_rows(
         for (int x = 0; x <= kGroupSpan; ++x) cand[j][x] = at[x];
       }
       if (kStaged) {
+        const int first_member = __builtin_amdgcn_readfirstlane(group[j].z);
         const int members = __builtin_amdgcn_readfirstlane(group[j].w);
-#pragma unroll
-        for (int m = 0; m <= kGroupSpan; ++m) {
-          if (m < members) mine |= 1ull << (__builtin_amdgcn_readfirstlane(member[j][m].y) & 63);
-        }
         if (collect) {
-          settle_group_staged<true>(cand[j], p[j], d0[j], member[j], members, c0, inside[j], s_counts,
+          mine |= ((1ull << members) - 1ull) << first_member;
+          settle_group_staged<true>(cand[j], p[j], d0[j], member[j], first_member, members, c0, inside[j], s_counts,
                                     num_targets, sink, wave_t0, votes_lo, votes_hi);
         } else {
-          settle_group_staged<false>(cand[j], p[j], d0[j], member[j], members, c0, inside[j], s_counts,
+          settle_group_staged<false>(cand[j], p[j], d0[j], member[j], first_member, members, c0, inside[j], s_counts,
                                      num_targets, sink, wave_t0, votes_lo, votes_hi);
         }
       } else {
@@ -368,9 +366,9 @@ __device__ __forceinline__ void resolve_chunk_rows(
     }
   }
   if (collect && wave_t0 < num_targets) {
-    // lane o holds the ballot of offset o
-    const int o = lane_id();
-    if (o < sink.num_offsets && ((mine >> o) & 1ull) != 0ull) {
+    // lane m holds the ballot of member m's offset
+    if (((mine >> lane_id()) & 1ull) != 0ull) {
+      const int o = s_members[lane_id()].y;
       const unsigned long long votes = (static_cast<unsigned long long>(votes_hi) << 32) | votes_lo;
       sink.masks[static_cast<long long>(o) * sink.num_wave_tiles + (wave_t0 >> 6)] = votes;
       atomicAdd(&s_counts[o], static_cast<unsigned>(__popcll(votes)));
@@ -545,12 +543,17 @@ __global__ __launch_bounds__(kQueryThreads) void query_kernel(
   // last lines of the kernel, which would otherwise wait for a trip to memory
   __shared__ short s_mirror[kPlanMaxOffsets];
   __shared__ int s_zero_offset;
-  if (halves && w == 2) {                      // one wavefront, a lane per offset (at most 64 of them in a chain)
-    const int o = lane_id();
-    const bool named = o < num_offsets && o < kPlanMaxOffsets;
-    if (named) s_mirror[o] = static_cast<short>(device_plan->mirror[o]);
-    const unsigned long long zero = __ballot(named && device_plan->kind[o] == 2);
-    if (o == 0) s_zero_offset = zero != 0ull ? __builtin_ctzll(zero) : -1;
+  if (halves && w == 2) {                      // one wavefront, kPlanEach offsets a lane
+    int zero_offset = -1;
+#pragma unroll
+    for (int e = 0; e < kPlanEach; ++e) {
+      const int o = e * kWave + lane_id();
+      const bool named = o < num_offsets;
+      if (named) s_mirror[o] = static_cast<short>(device_plan->mirror[o]);
+      const unsigned long long zero = __ballot(named && device_plan->kind[o] == 2);
+      if (zero != 0ull) zero_offset = e * kWave + __builtin_ctzll(zero);
+    }
+    if (lane_id() == 0) s_zero_offset = zero_offset;
   }
 
   // ---- window of sources that can match any (offset, target) pair of the tile:
@@ -658,13 +661,14 @@ __global__ __launch_bounds__(kQueryThreads) void query_kernel(
     const unsigned long long answers_from = c == 0 ? 0ull : first_key;
     const unsigned long long answers_to = c == num_chunks - 1 ? ~0ull : next_first;
     const bool counting = tile_counts != nullptr;
+    const int num_members = s_all_groups[num_groups - 1].z + s_all_groups[num_groups - 1].w;
 #define MNT_RESOLVE(WHOLE)                                                                         \
     if (by_rows) {                                                                                 \
       resolve_chunk_rows<OT, WHOLE, kLists>(reinterpret_cast<const unsigned *>(win), s_dir, len,   \
                                             zbits, static_cast<unsigned>(num_rows), base, c0, key, \
                                             valid, answers_from, answers_to, s_groups, s_members,  \
-                                            my_groups, s_counts, counting, t, num_targets,        \
-                                            kernel_map, sink);                                     \
+                                            my_groups, num_members, s_counts, counting, t,         \
+                                            num_targets, kernel_map, sink);                        \
     } else if (narrow) {                                                                           \
       resolve_chunk<unsigned, OT, WHOLE, kLists>(reinterpret_cast<const unsigned *>(win), top,     \
                                                  base, c0, key, valid, answers_from, answers_to,   \
@@ -1112,7 +1116,7 @@ __global__ __launch_bounds__(kPlaceBlock) void place_kernel(
     packed = chain_plan->rows[blockIdx.y - 1];                       // row 0 of the grid is the teller above
     repeated = repeats != nullptr ? repeats[0] : 0u;
   }
-  unsigned total_mine = 0;                       // hits of offset tid (tid < num_offsets <= 64 when there are copies)
+  unsigned total_mine = 0;                       // hits of offset tid (tid < num_offsets <= 128 when there are copies)
   if (total_copies > 1) {
     unsigned part[kMaxTotalCopies];
 #pragma unroll
@@ -2245,6 +2249,21 @@ static bool map_halves_enabled() {
 
 constexpr size_t kChainHostOffset = 128;      // pinned block: bounds (8 words), then the chain's verdict
 
+// The query plan of rows that another sort has left, from bounds that the host
+// knows, and cleared counters: what a chain's sort leaves its query.
+struct PlanBounds {
+  long long v[2 * MNT_MAX_NDIM];
+};
+__global__ __launch_bounds__(256) void chain_plan_kernel(PlanBounds bounds, OffsetTable offsets, int num_offsets,
+                                                         int ndim, DevicePlan *__restrict__ plan_out,
+                                                         long long *__restrict__ folded,
+                                                         unsigned *__restrict__ counters, int counter_words) {
+  const int tid = threadIdx.x;
+  for (int i = tid; i < counter_words; i += 256) counters[i] = 0u;
+  if (tid < 2 * MNT_MAX_NDIM) folded[tid] = bounds.v[tid];
+  if (tid < kWave) make_plan_on_device(bounds.v, load_plan_lane(offsets), offsets, num_offsets, ndim, 0u, plan_out);
+}
+
 template <typename CT>
 static void launch_query_chain(const CT *sorted, int64_t n, int ndim, int num_offsets,
                                unsigned *tile_counts, int num_tiles, const HitSink &sink,
@@ -2296,21 +2315,23 @@ extern "C" int mnt_sorted_kernel_map_lists(const void *coords, int64_t n, int nd
     for (int64_t i = 0; i < num_offsets * ndim; ++i) {
       small_offsets = small_offsets && offsets_host[i] >= INT32_MIN / 2 && offsets_host[i] <= INT32_MAX / 2;
     }
-    // what a chain of launches leaves for the host: true where it went through
-    auto heard = [&](Arena &arena, unsigned long long sequence) -> bool {
+    // the verdict of a chain of launches, and where that is 0 what it left for the host
+    auto hear = [&](Arena &arena, unsigned long long sequence) -> int {
       arena.wait_flag(1, sequence);
       const char *pinned = static_cast<const char *>(arena.pinned());
       const long long *h_chain = reinterpret_cast<const long long *>(pinned + kChainHostOffset);
       profile_mark("map_place+sync", stream);
-      if (h_chain[2 * MNT_MAX_NDIM] != 0) return false;
+      const int verdict = static_cast<int>(h_chain[2 * MNT_MAX_NDIM]);
+      if (verdict != 0) return verdict;
       const unsigned *h_plan = reinterpret_cast<const unsigned *>(pinned + Arena::kPlanOffset);
       for (int64_t j = 0; j < num_offsets; ++j) {
         order_host_out[j] = h_plan[j];
         sizes_host_out[j] = h_plan[2 * num_offsets + j];
       }
       memcpy(bounds_host_out, h_chain, sizeof(long long) * 2 * MNT_MAX_NDIM);
-      return true;
+      return 0;
     };
+    int verdict = 1;                                   // (1: not sorted, 2: keys too wide, 3: equal rows)
     if (small_offsets && small_map_takes(n, static_cast<int>(std::min<int64_t>(num_offsets, 65535)))) {
       profile_mark("enter:map_small", stream);
       Arena &arena = Arena::of(stream);
@@ -2323,10 +2344,21 @@ extern "C" int mnt_sorted_kernel_map_lists(const void *coords, int64_t n, int nd
                         scope, reinterpret_cast<unsigned *>(pinned_device + Arena::kPlanOffset),
                         reinterpret_cast<long long *>(pinned_device + kChainHostOffset), arena.flag_device(1), sequence,
                         stream);
-      if (heard(arena, sequence)) return;
+      verdict = hear(arena, sequence);
+      if (verdict == 0) return;
       // (crowded, equal rows, keys too wide: the calls below start over)
     }
-    if (small_offsets && chain_sort_takes(n, 1, static_cast<int>(num_offsets))) {
+    const bool few_offsets = small_offsets && num_offsets <= kPlanMaxOffsets && n <= (int64_t(1) << 21) && verdict == 1;
+    // (the cloud is mapped onto itself: offsets that come in pairs d / -d need one look-up
+    // per pair, so the 64 lanes of the planning wavefront take the 125 of 5x5x5.  By the
+    // separate calls and so, us: 10 000 voxels 137 and 75, 100 000 147 and 102, 300 000
+    // 223 and 145.)
+    const OffsetTable table = few_offsets ? make_offset_table<OffsetTable>(offsets_host, static_cast<int>(num_offsets),
+                                                                           ndim, map_halves_enabled())
+                                          : OffsetTable{};
+    const bool chained = few_offsets && table.num_kept <= kPlanMaxKept;
+    bool sorted = false;
+    if (chained) {
       profile_mark("enter:map_chain", stream);
       Arena &arena = Arena::of(stream);
       arena.map_state_valid = false;
@@ -2335,58 +2367,82 @@ extern "C" int mnt_sorted_kernel_map_lists(const void *coords, int64_t n, int nd
       const int buckets = 1 << chain_sort_msd_bits(n);
       const int num_tiles = static_cast<int>(div_ceil(n, kTargetsPerTile));
       const int64_t num_wave_tiles = div_ceil(n, kWave);
-      ChainSortBuffers buf;
-      buf.partial = scope.alloc<long long>(128 * 8);
-      buf.folded = scope.alloc<long long>(2 * MNT_MAX_NDIM);
       // bucket totals, cursors, the copies of the hits per offset, the equal-rows flag
       // (and the sort's status words, which must start at zero like the rest)
-      buf.counter_words = 2 * buckets + kMaxTotalCopies * kPlanMaxOffsets + 1 + 4;
-      buf.counters = scope.alloc<unsigned>(buf.counter_words);
-      buf.info = scope.alloc<unsigned>(4);
-      buf.status = buf.counters + (buf.counter_words - 4);
-      buf.chunks = scope.alloc<uint4>(chain_sort_max_pairs(n));
-      buf.words = scope.alloc<unsigned long long>(chain_sort_words(n));
-      buf.starts = scope.alloc<unsigned>(buckets + 1);
-      buf.plan = scope.alloc<DevicePlan>(1);
-      unsigned *row_totals = buf.counters + 2 * buckets;
+      const int counter_words = 2 * buckets + kMaxTotalCopies * kPlanMaxOffsets + 1 + 4;
+      unsigned *counters = scope.alloc<unsigned>(counter_words);
+      unsigned *row_totals = counters + 2 * buckets;
+      unsigned *repeats = row_totals + kMaxTotalCopies * kPlanMaxOffsets;
+      long long *folded = scope.alloc<long long>(2 * MNT_MAX_NDIM);
+      DevicePlan *device_plan = scope.alloc<DevicePlan>(1);
       int *stage = scope.alloc<int>(static_cast<size_t>(num_offsets) * n);
       unsigned long long *masks = scope.alloc<unsigned long long>(static_cast<size_t>(num_offsets) * num_wave_tiles);
       unsigned *tile_counts = scope.alloc<unsigned>(static_cast<size_t>(num_offsets) * num_tiles);
       unsigned *tile_mode = scope.alloc<unsigned>(num_tiles);
       unsigned *plan = scope.alloc<unsigned>(4 * num_offsets + 1);
-      // (the cloud is mapped onto itself: offsets that come in pairs d / -d need one look-up per pair)
-      const OffsetTable table = make_offset_table<OffsetTable>(offsets_host, no, ndim, map_halves_enabled());
       int num_rows = 0;                            // offsets with rows of their own to write (DevicePlan::rows)
       for (int o = 0; o < no; ++o) num_rows += table.kind[o] != 1 ? 1 : 0;
-      enqueue_chain_sort(coords, n, ndim, coord_dtype, indices_out, sorted_coords_out, buf, table, no, stream);
-      unsigned *repeats = row_totals + kMaxTotalCopies * kPlanMaxOffsets;
-      const HitSink sink{stage, masks, row_totals, tile_mode, num_wave_tiles, no, repeats, total_copies(),
-                         kPlanMaxOffsets};
-      char *pinned_device = static_cast<char *>(arena.pinned_device());
-      unsigned *d_plan_host = reinterpret_cast<unsigned *>(pinned_device + Arena::kPlanOffset);
-      long long *d_chain_host = reinterpret_cast<long long *>(pinned_device + kChainHostOffset);
-      const unsigned long long sequence = arena.next_sequence();
-      if (coord_dtype == MNT_INT32) {
-        launch_query_chain<int32_t>(static_cast<const int32_t *>(sorted_coords_out), n, ndim, no, tile_counts,
-                                    num_tiles, sink, buf.plan, stream);
-      } else {
-        launch_query_chain<int64_t>(static_cast<const int64_t *>(sorted_coords_out), n, ndim, no, tile_counts,
-                                    num_tiles, sink, buf.plan, stream);
+      // query and lists of the sorted rows; the verdict
+      auto lists = [&]() -> int {
+        const HitSink sink{stage, masks, row_totals, tile_mode, num_wave_tiles, no, repeats, total_copies(),
+                           kPlanMaxOffsets};
+        char *pinned_device = static_cast<char *>(arena.pinned_device());
+        unsigned *d_plan_host = reinterpret_cast<unsigned *>(pinned_device + Arena::kPlanOffset);
+        long long *d_chain_host = reinterpret_cast<long long *>(pinned_device + kChainHostOffset);
+        const unsigned long long sequence = arena.next_sequence();
+        if (coord_dtype == MNT_INT32) {
+          launch_query_chain<int32_t>(static_cast<const int32_t *>(sorted_coords_out), n, ndim, no, tile_counts,
+                                      num_tiles, sink, device_plan, stream);
+        } else {
+          launch_query_chain<int64_t>(static_cast<const int64_t *>(sorted_coords_out), n, ndim, no, tile_counts,
+                                      num_tiles, sink, device_plan, stream);
+        }
+        profile_mark("query", stream);
+        // a workgroup per four tiles and per offset that is looked up (or is the zero offset); row 0 tells the host
+        dim3 grid(static_cast<unsigned>(div_ceil(num_tiles, kPlaceTiles)), static_cast<unsigned>(num_rows + 1));
+        place_kernel<true><<<grid, kPlaceBlock, 0, stream>>>(
+            stage, masks, tile_counts, row_totals, tile_mode, n, no, num_tiles, num_wave_tiles, reorder, in_idx_out,
+            out_idx_out, plan, d_plan_host, arena.flag_device(1), sequence, sizes_dev_out, order_dev_out, device_plan,
+            folded, d_chain_host, repeats, total_copies(), kPlanMaxOffsets);
+        check_launch("place_kernel");
+        return hear(arena, sequence);
+      };
+      if (chain_sort_takes(n)) {
+        ChainSortBuffers buf;
+        buf.partial = scope.alloc<long long>(128 * 8);
+        buf.folded = folded;
+        buf.counters = counters;
+        buf.counter_words = counter_words;
+        buf.info = scope.alloc<unsigned>(4);
+        buf.status = counters + (counter_words - 4);
+        buf.chunks = scope.alloc<uint4>(chain_sort_max_pairs(n));
+        buf.words = scope.alloc<unsigned long long>(chain_sort_words(n));
+        buf.starts = scope.alloc<unsigned>(buckets + 1);
+        buf.plan = device_plan;
+        enqueue_chain_sort(coords, n, ndim, coord_dtype, indices_out, sorted_coords_out, buf, table, no, stream);
+        verdict = lists();
+        if (verdict == 0) return;
       }
-      profile_mark("query", stream);
-      // a workgroup per four tiles and per offset that is looked up (or is the zero offset); row 0 tells the host
-      dim3 grid(static_cast<unsigned>(div_ceil(num_tiles, kPlaceTiles)), static_cast<unsigned>(num_rows + 1));
-      place_kernel<true><<<grid, kPlaceBlock, 0, stream>>>(stage, masks, tile_counts, row_totals, tile_mode, n, no,
-                                                     num_tiles, num_wave_tiles, reorder, in_idx_out,
-                                                     out_idx_out, plan, d_plan_host, arena.flag_device(1),
-                                                     sequence, sizes_dev_out, order_dev_out, buf.plan,
-                                                     buf.folded, d_chain_host, repeats, total_copies(), kPlanMaxOffsets);
-      check_launch("place_kernel");
-      if (heard(arena, sequence)) return;
-      // the chain declined (strong clustering, keys too wide): the calls below start over
+      if (verdict == 1) {
+        // The chain's sort turned the cloud down (strong clustering): the other
+        // sort, which waits for the host, and then the same launches.  With the
+        // separate calls' query, of every offset, and so, us: a room of 150 000 voxels
+        // under 3x3x3 173 and 155, a million of a scan 302 and 271, under 5x5x5 722 and 479.
+        if (mnt_arg_sort_coordinates(coords, n, ndim, coord_dtype, nullptr, 1, MNT_INT32, indices_out,
+                                     sorted_coords_out, bounds_host_out, stream_) != 0) {
+          throw Error{mnt_last_error()};
+        }
+        sorted = true;
+        PlanBounds bounds;
+        for (int i = 0; i < 2 * MNT_MAX_NDIM; ++i) bounds.v[i] = bounds_host_out[i];
+        chain_plan_kernel<<<1, 256, 0, stream>>>(bounds, table, no, ndim, device_plan, folded, counters, counter_words);
+        check_launch("chain_plan_kernel");
+        verdict = lists();
+        if (verdict == 0) return;
+      }
     }
-    if (mnt_arg_sort_coordinates(coords, n, ndim, coord_dtype, nullptr, 1, MNT_INT32, indices_out,
-                                 sorted_coords_out, bounds_host_out, stream_) != 0) {
+    if (!sorted && mnt_arg_sort_coordinates(coords, n, ndim, coord_dtype, nullptr, 1, MNT_INT32, indices_out,
+                                            sorted_coords_out, bounds_host_out, stream_) != 0) {
       throw Error{mnt_last_error()};
     }
     if (mnt_kernel_map_lists(sorted_coords_out, n, sorted_coords_out, n, offsets_host, num_offsets, ndim,

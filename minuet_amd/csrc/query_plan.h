@@ -14,8 +14,10 @@
 namespace mnt {
 
 constexpr int kPlanGroupSpan = 4;                // key span of one offset group (kGroupSpan of the query)
-constexpr int kPlanMaxOffsets = 64;              // one lane per offset
-constexpr int kPlanInts = 6 * kPlanMaxOffsets;   // 4 words per group + 2 per member
+constexpr int kPlanMaxOffsets = 128;
+constexpr int kPlanMaxKept = 64;                 // offsets that are looked up: one lane each
+constexpr int kPlanInts = 6 * kPlanMaxKept;      // 4 words per group + 2 per member
+constexpr int kPlanEach = kPlanMaxOffsets / kWave;
 
 // Kernel offsets as launch arguments, and what can be said about them before the
 // bounds of the cloud (which is mapped onto itself) are known.  halves != 0 when
@@ -127,12 +129,12 @@ __device__ __forceinline__ int plan_bits(unsigned long long range) {
 }
 
 // What lane l of the planning wavefront takes from the launch arguments: looked-up
-// offset l and what is said about offset l.  Read with the lane's index (a load
+// offset l and what is said about offsets l and 64 + l.  Read with the lane's index (a load
 // per lane; picking them out of scalar registers took some 400 instructions) and
 // before the bounds are there.
 struct PlanLane {
   int d[MNT_MAX_NDIM];
-  int origin, kind, mirror;
+  int origin, kind[kPlanEach], mirror[kPlanEach];
 };
 
 __device__ __forceinline__ PlanLane load_plan_lane(const OffsetTable &offsets) {
@@ -141,8 +143,11 @@ __device__ __forceinline__ PlanLane load_plan_lane(const OffsetTable &offsets) {
 #pragma unroll
   for (int k = 0; k < MNT_MAX_NDIM; ++k) in.d[k] = offsets.v[lane][k];
   in.origin = offsets.origin[lane];
-  in.kind = offsets.kind[lane];
-  in.mirror = offsets.mirror[lane];
+#pragma unroll
+  for (int e = 0; e < kPlanEach; ++e) {
+    in.kind[e] = offsets.kind[e * kWave + lane];
+    in.mirror[e] = offsets.mirror[e * kWave + lane];
+  }
   return in;
 }
 
@@ -160,7 +165,6 @@ __device__ __forceinline__ void make_plan_on_device(const long long *__restrict_
                                                     const unsigned *__restrict__ bucket_starts = nullptr,
                                                     int msd_cap = 0) {
   const int lane = lane_id();
-  const bool live = lane < num_offsets;
   Frame f;
   int bits = 0;
   bool fits = true;
@@ -234,15 +238,19 @@ __device__ __forceinline__ void make_plan_on_device(const long long *__restrict_
       out->tables[4 * group + 3] = next - lane;
     }
   }
-  if (live) {
-    out->kind[lane] = in.kind;
-    out->mirror[lane] = in.mirror;
-    const bool writes = in.kind != 1;
+  int rows = 0;
+#pragma unroll
+  for (int e = 0; e < kPlanEach; ++e) {
+    const int o = e * kWave + lane;
+    const bool live = o < num_offsets;
+    const bool writes = live && in.kind[e] != 1;
     const unsigned long long writers = __ballot(writes);
-    if (writes) {
-      const int y = __popcll(writers & ((1ull << lane) - 1ull));
-      out->rows[y] = lane | (in.kind << 8) | ((in.mirror + 1) << 16);
+    if (live) {
+      out->kind[o] = in.kind[e];
+      out->mirror[o] = in.mirror[e];
     }
+    if (writes) out->rows[rows + __popcll(writers & lanes_below())] = o | (in.kind[e] << 8) | ((in.mirror[e] + 1) << 16);
+    rows += __popcll(writers);
   }
   const long long delta_min = __shfl(mine, 0);
   const long long delta_max = __shfl(mine, num_kept > 0 ? num_kept - 1 : 0);

@@ -92,9 +92,9 @@ struct ChainSortBuffers {
   DevicePlan *plan;              // query plan written by the ranking launch (nullable)
 };
 
-// Whether the chain takes a cloud of n rows (one batch) with this many offsets;
-// the final word is the chain's own (status[0]), known once it has run.
-bool chain_sort_takes(int64_t n, int64_t num_batches, int num_offsets);
+// Whether the chain takes a cloud of n rows (one batch); the final word is the
+// chain's own (status[0]), known once it has run.
+bool chain_sort_takes(int64_t n);
 // log2 of the number of buckets the chain uses for n rows, and the most
 // (bucket, chunk) pairs its ranking launch can have.
 int chain_sort_msd_bits(int64_t n);

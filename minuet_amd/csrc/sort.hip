@@ -2025,9 +2025,8 @@ size_t chain_sort_words(int64_t n) {
   return std::max(packed, (static_cast<size_t>(1) << chain_sort_msd_bits(n)) * kChainBucketCap);
 }
 
-bool chain_sort_takes(int64_t n, int64_t num_batches, int num_offsets) {
-  return n > kSmallSortRows && n <= bucket_sort_max_rows() && n <= (int64_t(1) << 21) && num_batches <= 1 &&
-         num_offsets >= 1 && num_offsets <= kPlanMaxOffsets;
+bool chain_sort_takes(int64_t n) {
+  return n > kSmallSortRows && n <= bucket_sort_max_rows() && n <= (int64_t(1) << 21);
 }
 
 template <typename CT>

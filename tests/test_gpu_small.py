@@ -76,6 +76,18 @@ def test_map_lists_in_one_launch(n, ndim, kernel, dilation, dtype, patience, mon
     check_map_lists(c, orc.generate_kernel_offsets(ndim, kernel, 1, dilation))
 
 
+# the chain of launches under 65 to 128 offsets that come in pairs (64 kept at most), with the largest that do
+# and one that does not take it; one tile more than one, several buckets, windows of more than one chunk
+@pytest.mark.parametrize("n,ndim,kernel,dilation,dtype", [
+    (4097, 3, 5, 1, np.int32), (70000, 3, 5, 1, np.int64), (20000, 2, 11, 1, np.int32), (9000, 1, 127, 1, np.int32),
+    (9000, 1, 129, 1, np.int32), (6000, 3, 5, 7, np.int32), (12000, 3, 4, 1, np.int32)])
+def test_map_lists_of_many_offsets(n, ndim, kernel, dilation, dtype):
+    extent = int(round((4 * n) ** (1 / ndim)))
+    c, _ = sorted_unique(random_cloud(2 * n, extent, n + kernel, ndim=ndim, lo=-extent // 2, dtype=dtype))
+    c = c[np.random.default_rng(n).permutation(c.shape[0])][:n]
+    check_map_lists(c, orc.generate_kernel_offsets(ndim, kernel, 1, dilation))
+
+
 def test_map_lists_of_equal_rows():
     """The one launch turns such a cloud down, whoever of the workgroups sees it."""
     c = random_cloud(3000, 12, 8, duplicates=0.3)
