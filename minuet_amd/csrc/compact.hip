@@ -34,9 +34,9 @@ struct CompactShape {
 // hits of its offsets, 16 rows of one offset at a time are multiplied by
 // 16 x 16 x 4 instructions (K in pieces of 16 channels, KI of them per unit),
 // and the sums of their targets, which stand in LDS, go in and come out as the
-// instruction's accumulators.  Every wavefront has sums of its own; they are
-// added up in the order of the wavefronts at the end, so that a result is the
-// same whenever it is computed.
+// instruction's accumulators (AFTER: the products are added to them).  Every
+// wavefront has sums of its own; they are added up in the order of the wavefronts
+// at the end, so that a result is the same whenever it is computed.
 //
 // LANES: the weights come in the order of the instruction's lanes (pack_lanes),
 // one load of 1 KB where [O][K][N] takes four of 256 or 512 bytes.  For callers
@@ -49,8 +49,9 @@ struct CompactShape {
 // the split; beyond, fp32 products of 16 rows that are about half hits, and the
 // weights, which every 16 rows read again: from some
 // targets x input x output channels on (78 million for 3 x 3 x 3) the
-// three-kernel form is the faster one again (hits_rows_limit in
-// nn/functional/convolution.py has the line and both sides of it).  fp32, 3 x 3 x 3, us a layer in
+// three-kernel form is the faster one again, unless there are few input channels
+// (hits_rows_limit and hits_rows_from in nn/functional/convolution.py have the
+// lines and both sides of them).  fp32, 3 x 3 x 3, us a layer in
 // three kernels and here: 32 -> 32 channels over 3 000 voxels 11.4 / 4.9,
 // 20 000 17.9 / 11.2, 200 000 76 / 54; 64 -> 64 over 3 000 12.1 / 8.4, 12 000
 // 18.8 / 14.9; 256 -> 256 over 135 28 / 15.6 (in lanes 12.5).  (128 targets per workgroup
@@ -59,7 +60,7 @@ struct CompactShape {
 // 20 000 targets 13.0 -> 14.4; the hits of all wavefronts dealt out evenly: 12.1, but
 // 256 -> 256 over 130 targets 13.6 -> 14.9, and sums that go by the targets of a
 // workgroup.)
-template <int C, int KI, int SPLIT, int TARGETS, bool WHOLE, bool LANES>
+template <int C, int KI, int SPLIT, int TARGETS, bool WHOLE, bool LANES, bool AFTER>
 __global__ __launch_bounds__(64 * SPLIT) void compact_forward_kernel(
     const float *__restrict__ sources, unsigned source_bytes, const float *__restrict__ weights,
     unsigned weight_bytes, const int *__restrict__ kernel_map, CompactShape s, unsigned char *__restrict__ out,
@@ -154,13 +155,14 @@ __global__ __launch_bounds__(64 * SPLIT) void compact_forward_kernel(
   };
   auto multiply = [&](const Unit &u) {
     float *row[4];
+    Floats<C> before[4];
     floatx4 sum[C];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       row[j] = acc + ((u.targets >> (8 * j)) & 255u) * kAccRow + r * C;
-      const Floats<C> before = *reinterpret_cast<const Floats<C> *>(row[j]);
+      before[j] = *reinterpret_cast<const Floats<C> *>(row[j]);
 #pragma unroll
-      for (int b = 0; b < C; ++b) sum[b][j] = before.v[b];
+      for (int b = 0; b < C; ++b) sum[b][j] = AFTER ? 0.0f : before[j].v[b];
     }
 #pragma unroll
     for (int i = 0; i < KI; ++i) {
@@ -175,7 +177,7 @@ __global__ __launch_bounds__(64 * SPLIT) void compact_forward_kernel(
     for (int j = 0; j < 4; ++j) {
       Floats<C> after;
 #pragma unroll
-      for (int b = 0; b < C; ++b) after.v[b] = sum[b][j];
+      for (int b = 0; b < C; ++b) after.v[b] = AFTER ? before[j].v[b] + sum[b][j] : sum[b][j];
       *reinterpret_cast<Floats<C> *>(row[j]) = after;
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -374,6 +376,17 @@ void compact_forward(const float *sources, const float *weights, bool lanes, con
     c = full >= 4.75 && N % 64 == 0 ? 4 : 2;
     targets = full >= 1.95 && full < 3.0 ? 32 : 64;
   }
+  // Layers that three kernels would take otherwise (hits_rows_limit has the lines):
+  // there a target's sum takes products that have been added up offset by offset,
+  // and so it does here.  Where sums go in as accumulators (64 to 128 channels by
+  // 3x3x3 over 100 000 voxels) they are off by 1.1 to 1.3 times as much, added
+  // afterwards as much as there; it takes 2 to 8 % longer.  (Added while the next
+  // 16 rows are multiplied: 232 registers instead of 160, 10 % longer.)
+  const bool after = !lanes && K <= 48 && K * N > 1024 && O >= 27 && S * K * N > 2100000000 / O;
+  if (after) {
+    targets = 64;
+    split = 4;
+  }
   s.steps = static_cast<int>(div_ceil(K, int64_t{16}));
   // Columns side by side, so that the workgroups of a die share few of them and
   // its L2 holds their weights, up to the threads a grid may have along x.
@@ -382,19 +395,19 @@ void compact_forward(const float *sources, const float *weights, bool lanes, con
   s.columns = beside ? static_cast<int>(columns) : 1;
   const dim3 grid(static_cast<unsigned>(beside ? rows * columns : rows), static_cast<unsigned>(beside ? 1 : columns));
   const unsigned weight_bytes = static_cast<unsigned>((lanes ? lane_weight_floats(O, K, N) : O * K * N) * 4);
-#define MNT_COMPACT_W(C, KI, SPLIT, TARGETS, WHOLE, LANES)                                                     \
-  compact_forward_kernel<C, KI, SPLIT, TARGETS, WHOLE, LANES><<<grid, 64 * SPLIT, 0, stream>>>(                \
+#define MNT_COMPACT_W(C, KI, SPLIT, TARGETS, WHOLE, LANES, AFTER)                                              \
+  compact_forward_kernel<C, KI, SPLIT, TARGETS, WHOLE, LANES, AFTER><<<grid, 64 * SPLIT, 0, stream>>>(                \
       sources, static_cast<unsigned>(S * K * 4), weights, weight_bytes, kernel_map, s,                         \
       reinterpret_cast<unsigned char *>(out), ep)
 #define MNT_COMPACT(C, KI, SPLIT, TARGETS)               \
   if (lanes && whole) {                                  \
-    MNT_COMPACT_W(C, KI, SPLIT, TARGETS, true, true);    \
+    MNT_COMPACT_W(C, KI, SPLIT, TARGETS, true, true, false);    \
   } else if (lanes) {                                    \
-    MNT_COMPACT_W(C, KI, SPLIT, TARGETS, false, true);   \
+    MNT_COMPACT_W(C, KI, SPLIT, TARGETS, false, true, false);   \
   } else if (whole) {                                    \
-    MNT_COMPACT_W(C, KI, SPLIT, TARGETS, true, false);   \
+    MNT_COMPACT_W(C, KI, SPLIT, TARGETS, true, false, false);   \
   } else {                                               \
-    MNT_COMPACT_W(C, KI, SPLIT, TARGETS, false, false);  \
+    MNT_COMPACT_W(C, KI, SPLIT, TARGETS, false, false, false);  \
   }
 #define MNT_COMPACT_K(C, SPLIT, TARGETS)               \
   switch (ki) {                                        \
@@ -403,7 +416,27 @@ void compact_forward(const float *sources, const float *weights, bool lanes, con
     case 3: MNT_COMPACT(C, 3, SPLIT, TARGETS) break;   \
     default: MNT_COMPACT(C, 4, SPLIT, TARGETS) break;  \
   }
-  if (c == 4) {
+#define MNT_COMPACT_AFTER(C, KI)                           \
+  if (whole) {                                             \
+    MNT_COMPACT_W(C, KI, 4, 64, true, false, true);        \
+  } else {                                                 \
+    MNT_COMPACT_W(C, KI, 4, 64, false, false, true);       \
+  }
+#define MNT_COMPACT_AFTER_K(C)                       \
+  switch (ki) {                                      \
+    case 1: MNT_COMPACT_AFTER(C, 1) break;           \
+    case 2: MNT_COMPACT_AFTER(C, 2) break;           \
+    default: MNT_COMPACT_AFTER(C, 3) break;          \
+  }
+  if (after) {
+    if (c == 4) {
+      MNT_COMPACT_AFTER_K(4)
+    } else if (c == 2) {
+      MNT_COMPACT_AFTER_K(2)
+    } else {
+      MNT_COMPACT_AFTER_K(1)
+    }
+  } else if (c == 4) {
     MNT_COMPACT_K(4, 4, 64)
   } else if (c == 2) {
     if (targets == 16) {
@@ -428,6 +461,8 @@ void compact_forward(const float *sources, const float *weights, bool lanes, con
   } else {
     MNT_COMPACT_K(1, 4, 64)
   }
+#undef MNT_COMPACT_AFTER_K
+#undef MNT_COMPACT_AFTER
 #undef MNT_COMPACT_K
 #undef MNT_COMPACT
 #undef MNT_COMPACT_W

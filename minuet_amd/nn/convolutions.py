@@ -1011,8 +1011,14 @@ class SparseConv(Module):
             if (sources.dtype == torch.float32 and dataflow == "auto" and volume > 1 and sources.is_cuda
                     and self.kernel.dtype == torch.float32):
                 most = F.hits_rows_limit(volume, self.in_channels, self.out_channels, sources.dtype)
-                hits = sources.shape[0] <= most
-                rows = (0, most) if hits else (most + 1, _MOST_ROWS)
+                again = F.hits_rows_from(volume, self.in_channels, self.out_channels, sources.dtype)
+                far = F.implicit_rows_limit(self.in_channels, sources.dtype)
+                count = sources.shape[0]
+                hits = count <= most or again <= count <= far
+                if hits:
+                    rows = (0, most) if count <= most else (again, far)
+                else:
+                    rows = (most + 1, again - 1) if count < again else (far + 1, _MOST_ROWS)
             route_key = (sources.dtype, sources.is_cuda, dataflow, hits)
             route = self._routes.get(route_key)
             if route is None or len(route) != 6:    # (fewer in a module that an older version has saved)

@@ -10,7 +10,7 @@ from ..kernel_map import KernelMap
 __all__ = ["cuda_time_gather", "cuda_time_scatter", "sparse_convolution_forward",
            "cuda_time_gemm", "set_gemm_parallel_level", "Epilogue", "pack_weights",
            "prefers_implicit", "prefers_streamed", "prefers_hits", "implicit_rows_limit", "hits_rows_limit",
-           "streamed_rows_limit",
+           "hits_rows_from", "streamed_rows_limit",
            "pieces_rows_limit", "channel_pieces"]
 
 pack_weights = _C.pack_weights
@@ -125,15 +125,45 @@ def hits_rows_limit(num_offsets: int, num_source_features: int, num_target_featu
     63 / 76), or about even (2x2x2 over 300 000 31.5 / 31.7 and, transposed, 36.9
     / 33.6).
 
+    So it is for at most 16 input channels under 3x3x3 to 5x5x5, where products
+    cost next to nothing and product rows as much as ever (0.4 to 0.96 times as
+    long over 120 layers of 64 to 512 output channels and 3 000 to 300 000 voxels;
+    one of 1.02): 3x3x3 16 -> 96 over 40 000 voxels of a room 26 / 35, over 200 000
+    of a LiDAR scan 113 / 236, 16 -> 256 over 100 000 of objects 148 / 311; 5x5x5 16 ->
+    256 over 20 000 83 / 92.
+
     Never more than ``implicit_rows_limit``."""
     if (dtype != torch.float32 or num_offsets <= 1
             or not _C.implicit_forward_supported(num_source_features, num_target_features, dtype)):
         return -1
     most = implicit_rows_limit(num_source_features, dtype)
     work = num_source_features * num_target_features
-    if work <= 1024:
+    if work <= 1024 or (num_source_features <= 16 and 27 <= num_offsets <= 125):
         return most
     return min(most, min(110_000_000, 2_100_000_000 // num_offsets) // work)
+
+
+def hits_rows_from(num_offsets: int, num_source_features: int, num_target_features: int,
+                   dtype: torch.dtype) -> int:
+    """The fewest source rows past ``hits_rows_limit`` over which ``dataflow="auto"``
+    takes the single-kernel form again (one more than ``implicit_rows_limit``:
+    over none).
+
+    From some 100 million products on, product rows outgrow the caches and the
+    three kernels slow down, the single-kernel form does not.  With up to 48 input
+    channels it is then the faster one for every kind of scene, LiDAR first and
+    rooms, whose voxels have the fewest neighbours, last; us here and in three
+    kernels, 3x3x3: 48 -> 64 over 250 000 voxels of a room 128 / 137, over 200 000
+    108 / 102, of objects 180 / 249; 32 -> 64 of a LiDAR scan 132 / 228; 5x5x5: 48 -> 64
+    over 150 000 of a room 207 / 242, over 100 000 153 / 147, 32 -> 64 of a LiDAR scan
+    177 / 297.  (64 input channels: over 300 000 of a LiDAR scan 259 / 386, of a room
+    171 / 181, but 64 -> 48 164 / 156, and with the sums that ``compact_forward``
+    keeps for these layers 8 % more.)"""
+    far = implicit_rows_limit(num_source_features, dtype) + 1
+    if (hits_rows_limit(num_offsets, num_source_features, num_target_features, dtype) < 0
+            or num_source_features > 48 or not 27 <= num_offsets <= 125):
+        return far
+    return min(far, 130_000 if num_offsets == 125 else 250_000)
 
 
 def channel_pieces(num_source_features: int) -> int:
@@ -166,8 +196,10 @@ def pieces_rows_limit(num_source_features: int, num_target_features: int, dtype:
 def prefers_hits(num_offsets: int, num_source_features: int, num_target_features: int, dtype: torch.dtype,
                  num_rows: int) -> bool:
     """Whether ``dataflow="auto"`` takes the single-kernel form for an fp32 layer
-    over ``num_rows`` source rows (``hits_rows_limit``)."""
-    return num_rows <= hits_rows_limit(num_offsets, num_source_features, num_target_features, dtype)
+    over ``num_rows`` source rows (``hits_rows_limit``, ``hits_rows_from``)."""
+    layer = (num_offsets, num_source_features, num_target_features, dtype)
+    return num_rows <= hits_rows_limit(*layer) or (
+        hits_rows_from(*layer) <= num_rows <= implicit_rows_limit(num_source_features, dtype))
 
 
 def cuda_time_gather(weights: torch.Tensor, source_masks: torch.Tensor,

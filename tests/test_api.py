@@ -189,6 +189,20 @@ def test_fp32_rule_follows_the_kernel_size():
     assert prefers(125, 32, 32, single, 100000)
 
 
+def test_fp32_rule_for_few_input_channels():
+    """Past the line product rows outgrow the caches: few input channels never leave the single-kernel form, a
+    few more come back to it."""
+    prefers, single = minuet.nn.functional.prefers_hits, torch.float32
+    assert all(prefers(27, 16, 256, single, rows) for rows in (1000, 50000, 10 ** 6))
+    for offsets, back in ((27, 250000), (125, 130000)):
+        assert prefers(offsets, 48, 64, single, 1000) and prefers(offsets, 48, 64, single, back)
+        assert not prefers(offsets, 48, 64, single, 30000) and not prefers(offsets, 48, 64, single, back - 1)
+        assert not prefers(offsets, 64, 64, single, 10 ** 6)
+    assert not prefers(8, 48, 64, single, 10 ** 6)
+    most = (0xFFFFF000 - 1) // (48 * 4)
+    assert prefers(27, 48, 64, single, most) and not prefers(27, 48, 64, single, most + 1)
+
+
 # (channels, rows) where cutting the channels was measured slower than one offset, and where faster
 @pytest.mark.parametrize("cin, cout, slower, faster", [
     (64, 32, 60000, 30000), (96, 64, 30000, 8000), (48, 128, 20000, 4500), (80, 48, 30000, 20000), (96, 128, 20000, 9000),

@@ -85,3 +85,29 @@ def test_kernel_follows_the_size_of_each_cloud():
             cache.reset()
             assert torch.equal(conv(x).F, expected)      # bit for bit: the two kernels add up in different orders
             assert torch.equal(conv(x).F, expected)
+
+
+@pytest.mark.parametrize("rows, targets, cin, cout", [
+    (60000, 1, 16, 96), (60000, 65, 20, 68), (45000, 333, 48, 64), (52000, 129, 48, 36), (30000, 5003, 16, 256),
+    (60000, 13001, 28, 96), (80000, 64, 4, 512)])
+def test_products_are_added_after_in_large_layers(rows, targets, cin, cout):
+    """Few input channels over so many rows that three kernels would take the layer otherwise."""
+    assert rows * cin * cout > 2_100_000_000 // 27
+    gen = torch.Generator(device=DEVICE).manual_seed(rows + cout)
+    x = torch.randn(rows, cin, generator=gen, device=DEVICE)
+    w = torch.randn(27, cin, cout, generator=gen, device=DEVICE)
+    dense = torch.randint(-rows, rows, (27, targets), generator=gen, device=DEVICE, dtype=torch.int32).clamp(min=-1)
+    x[int(dense[3].max())] = 0.0
+    wanted, size = (torch.zeros(targets, cout, dtype=torch.float64, device=DEVICE) for _ in range(2))
+    for offset in range(27):
+        hit = (dense[offset] >= 0).nonzero()[:, 0]
+        picked, weight = x[dense[offset, hit].long()].double(), w[offset].double()
+        wanted[hit] += picked @ weight
+        size[hit] += picked.abs() @ weight.abs()
+    out = _C.sparse_convolution_forward_implicit(x, w, dense)
+    # every value is rounded in at most cin additions of an offset and 27 + 4 of offsets and wavefronts
+    assert bool(((out.double() - wanted).abs() <= (cin + 31) * 2.0 ** -24 * size).all())
+    assert torch.equal(out, _C.sparse_convolution_forward_implicit(x, w, dense))
+    w[5, 0, 0] = float("inf")                            # what a target has no source for does not reach it
+    out = _C.sparse_convolution_forward_implicit(x, w, dense)
+    assert bool(out[dense[5] < 0].isfinite().all())
