@@ -37,7 +37,15 @@ def prefers_implicit(num_offsets: int, num_source_features: int, num_target_feat
     bytes and up to 128 output channels, and for rows of up to 256 bytes with up
     to 64 output channels under kernels of more than 8 offsets (beyond that its
     matrix work on empty (offset, target) pairs outweighs the buffer traffic it
-    saves).  An fp32 layer of more than one offset goes by its rows instead
+    saves).  With rows of up to 64 bytes there is so little of that work that up to
+    36 offsets, and 5x5x5, take any number of output channels: a second 128 of them
+    cost as much as the first, the three kernels' product rows more (us, three
+    kernels and here: 3x3x3 24 -> 256 over 200 000 voxels of a LiDAR scan 326 / 66, 32
+    -> 160 over 5 000 of a room 19 / 10, over 1 000 15 / 11; 2x2x2 16 -> 160 over 50 000
+    28 / 16; 5x5x5 32 -> 256 over 200 000 805 / 157, over 30 000 of a room 72 / 69, 32 ->
+    160 there 63 / 64).  Not kernels in between, where a target has a smaller share of
+    its offsets (4x4x4 32 -> 160 over 50 000 of a room 53 / 64), nor larger ones
+    (6x6x6 32 -> 256 over 50 000 155 / 200).  An fp32 layer of more than one offset goes by its rows instead
     (``hits_rows_limit``); without rows to go by, this says yes to the narrow
     ones with strided 2^D kernels, whose (offset, target) pairs are mostly hits."""
     if not _C.implicit_forward_supported(num_source_features, num_target_features, dtype, num_offsets):
@@ -45,7 +53,7 @@ def prefers_implicit(num_offsets: int, num_source_features: int, num_target_feat
     if dtype != torch.float32:
         row_bytes = num_source_features * dtype.itemsize
         if row_bytes <= 128:
-            return num_target_features <= 128
+            return num_target_features <= 128 or (row_bytes <= 64 and (num_offsets <= 36 or num_offsets == 125))
         return row_bytes <= 256 and num_target_features <= 64 and num_offsets > 8
     return num_offsets <= 8 and num_source_features * num_target_features <= 1024
 

@@ -163,6 +163,8 @@ def test_auto_dataflow_rule():
     half, single = torch.float16, torch.float32
     assert prefers(27, 32, 32, half) and prefers(27, 64, 128, half) and prefers(8, 64, 128, torch.bfloat16)
     assert not prefers(27, 64, 256, half)                 # too many output channels
+    assert prefers(27, 32, 256, half) and prefers(8, 8, 132, half) and prefers(125, 16, 512, half)      # short rows
+    assert not prefers(64, 32, 256, half) and not prefers(216, 32, 160, half) and not prefers(27, 40, 160, half)
     assert prefers(27, 128, 64, half) and not prefers(27, 128, 128, half)
     assert not prefers(8, 128, 64, half)                  # strided 2^3 kernel: one hit in eight
     assert not prefers(27, 256, 64, half)                 # 512-byte rows

@@ -168,3 +168,34 @@ def test_features_past_the_single_kernel_form(cin, cout, size, stride, transpose
         tolerance = 1e-5 if dtype == torch.float32 else 4 * torch.finfo(dtype).eps
         assert float((got.double() - wanted.double()).norm() / wanted.double().norm()) < tolerance
     assert calls and all(s.numel() * s.element_size() < limit for s in calls)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("kernel, cin, cout", [(3, 32, 132), (3, 8, 512), (2, 16, 160), (5, 24, 256), (3, 4, 160), (3, 20, 256)])
+def test_wide_layers_of_short_rows(kernel, cin, cout, dtype):
+    """Past 128 output channels: the single-kernel form, where rows are padded for it from 10 000 voxels on."""
+    gen = torch.Generator(device="cuda").manual_seed(cin + cout)
+    conv = minuet.nn.SparseConv3d(cin, cout, kernel, dtype=dtype, device="cuda")
+    for rows in (1, 700, 9999, 10000, 700):
+        cells = torch.randperm(1 << 16, generator=gen, device="cuda")[:rows]
+        coordinates = torch.stack([cells >> 10, (cells >> 5) & 31, cells & 31], 1).int()
+        coordinates = coordinates[minuet.nn.functional.build_sorted_index(coordinates)]
+        cache = minuet.nn.KernelMapCache(3, torch.int32, "cuda")
+        minuet.set_kernel_map_cache(conv, cache)
+        x = minuet.SparseTensor(torch.randn(rows, cin, generator=gen, device="cuda").to(dtype), coordinates)
+        with torch.no_grad():
+            out = conv(x).F
+            assert torch.equal(conv(x).F, out)
+        assert len(cache._kernel_maps_cache) == (cin % 8 != 0 and rows < 10000)
+        dense, _ = _C.kernel_map_dense(coordinates, coordinates,
+                                       cache._kernel_offsets((1, 1, 1), (kernel,) * 3, (1, 1, 1)), None, None)
+        weights = conv.kernel.detach().double()
+        wanted, size = (torch.zeros(rows, cout, dtype=torch.float64, device="cuda") for _ in range(2))
+        for offset in range(dense.shape[0]):
+            hit = (dense[offset] >= 0).nonzero()[:, 0]
+            picked = x.F[dense[offset, hit].long()].double()
+            wanted[hit] += picked @ weights[offset]
+            size[hit] += picked.abs() @ weights[offset].abs()
+        # one rounding of the result, and with product rows one of each; sums in 32 bits
+        bound = torch.finfo(dtype).eps * (wanted.abs() + (0 if len(cache._kernel_maps_cache) == 0 else 1) * size)
+        assert bool(((out.double() - wanted).abs() <= bound + 1e-5 * size + 1e-7).all())
