@@ -886,7 +886,17 @@ class SparseConv(Module):
         shape = (self.kernel.shape[0], self.in_channels + pad, self.out_channels, features.dtype)
         # (a copy of the rows, which every call makes, is more than streaming saves: 100 -> 64
         # channels over 2 000 voxels 14.6 us in three kernels and 26.7, 150 -> 160 over 9 000 34.9 and 48.1)
-        return F.prefers_implicit(*shape) or (pad == 0 and F.prefers_streamed(*shape))
+        return (F.prefers_implicit(*shape) or (pad == 0 and F.prefers_streamed(*shape))
+                or F.implicit_rows_from(*shape) <= features.shape[0])
+
+    def _single_kernel_from(self, dtype: torch.dtype) -> int:
+        """The fewest rows over which ``auto`` takes the single-kernel form for a
+        16-bit layer (0: the number of rows does not matter)."""
+        if self.out_channels > 128 and self.in_channels % 8 != 0 and self.in_channels <= 32:
+            return _PADDED_WIDE_ROWS
+        shape = (self.kernel.shape[0], -(-self.in_channels // 8) * 8, self.out_channels, dtype)
+        begin = F.implicit_rows_from(*shape)
+        return begin if begin <= F.implicit_rows_limit(shape[1], dtype) else 0
 
     def _has_single_sources(self, features: torch.Tensor, pad: int = 0) -> bool:
         """Whether a target of this layer has one source, and the kernel for that
@@ -1026,7 +1036,10 @@ class SparseConv(Module):
                     rows = (0, most) if count <= most else (again, far)
                 else:
                     rows = (most + 1, again - 1) if count < again else (far + 1, _MOST_ROWS)
-            small = hits is None and self.out_channels > 128 and sources.shape[0] < _PADDED_WIDE_ROWS
+            begin = 0                               # (rows from which the single-kernel form may be taken)
+            if hits is None and dataflow == "auto" and sources.dtype != torch.float32:
+                begin = self._single_kernel_from(sources.dtype)
+            small = sources.shape[0] < begin
             route_key = (sources.dtype, sources.is_cuda, dataflow, hits, small)
             route = self._routes.get(route_key)
             if route is None:
@@ -1036,8 +1049,8 @@ class SparseConv(Module):
                 implicit = implicit and not grouped
                 single = tiled = False
                 most, few = None, ()
-                if implicit and pad and small and dataflow == "auto":
-                    pad, implicit, few = 0, False, (0, _PADDED_WIDE_ROWS - 1)
+                if small:
+                    pad, implicit, few = 0, False, (0, begin - 1)
                 if implicit and not hits:
                     single = self._has_single_sources(sources, pad)
                     tiled = not single and F.prefers_streamed(volume, self.in_channels + pad, self.out_channels,
@@ -1053,7 +1066,7 @@ class SparseConv(Module):
             pad, implicit, grouped, most, single, tiled, few = route
             rows = few or rows
             if most is not None:
-                rows = (0, most)
+                rows = (begin, most)
                 if sources.shape[0] > most:
                     pad, implicit, grouped = 0, False, self._takes_offset_groups(sources, streamed=False)
                     rows = (most + 1, _MOST_ROWS)

@@ -10,7 +10,7 @@ from ..kernel_map import KernelMap
 __all__ = ["cuda_time_gather", "cuda_time_scatter", "sparse_convolution_forward",
            "cuda_time_gemm", "set_gemm_parallel_level", "Epilogue", "pack_weights",
            "prefers_implicit", "prefers_streamed", "prefers_hits", "implicit_rows_limit", "hits_rows_limit",
-           "hits_rows_from", "streamed_rows_limit",
+           "hits_rows_from", "streamed_rows_limit", "implicit_rows_from",
            "pieces_rows_limit", "channel_pieces"]
 
 pack_weights = _C.pack_weights
@@ -102,6 +102,34 @@ def streamed_rows_limit(num_offsets: int, num_source_features: int, num_target_f
             and (num_target_features - 1) % 128 < 64 and dtype == torch.float16):
         return 256 // -(-num_target_features // 64) * 64
     return (1 << 63) - 1
+
+
+def implicit_rows_from(num_offsets: int, num_source_features: int, num_target_features: int,
+                       dtype: torch.dtype) -> int:
+    """The fewest source rows over which ``dataflow="auto"`` takes the single-kernel
+    form for a 16-bit layer that is not in its shape the faster one there
+    (``prefers_implicit``, ``prefers_streamed``); one more than
+    ``implicit_rows_limit``: over none.
+
+    5x5x5 layers whose product rows outgrow the caches: rows of 80 to 128 bytes and
+    more than 128 output channels, of which the second 128 cost as much as the
+    first, so half of them more than a whole, and rows of up to 256 bytes and 97 to
+    128 output channels.  us, three kernels and here, the slowest and the fastest
+    kind of scene: 64 -> 256 over 100 000 voxels of a room 312 / 239, of a LiDAR scan 333
+    / 178 (over 30 000 of a room 72 / 84), 64 -> 160 over 150 000 333 / 278 and 447 / 205
+    (over 100 000 of a room 219 / 234), 128 -> 128 over 150 000 282 / 264 and 369 / 185
+    (over 100 000 of a room 172 / 215).  Not 128 -> 160 (250 000 of a room 570 / 666) nor
+    128 -> 256 (481 / 496 over 150 000)."""
+    far = implicit_rows_limit(num_source_features, dtype) + 1
+    if (dtype == torch.float32 or num_offsets != 125
+            or not _C.implicit_forward_supported(num_source_features, num_target_features, dtype, num_offsets)):
+        return far
+    row_bytes = num_source_features * dtype.itemsize
+    if 64 < row_bytes <= 128 and num_target_features > 128:
+        return min(far, 100_000 if (num_target_features - 1) % 128 >= 64 else 150_000)
+    if 128 < row_bytes <= 256 and 96 < num_target_features <= 128:
+        return min(far, 150_000)
+    return far
 
 
 def implicit_rows_limit(num_source_features: int, dtype: torch.dtype) -> int:

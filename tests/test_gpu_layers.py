@@ -199,3 +199,29 @@ def test_wide_layers_of_short_rows(kernel, cin, cout, dtype):
         # one rounding of the result, and with product rows one of each; sums in 32 bits
         bound = torch.finfo(dtype).eps * (wanted.abs() + (0 if len(cache._kernel_maps_cache) == 0 else 1) * size)
         assert bool(((out.double() - wanted).abs() <= bound + 1e-5 * size + 1e-7).all())
+
+
+@pytest.mark.parametrize("cin, cout, begin", [(64, 256, 100000), (44, 160, 150000), (128, 128, 150000)])
+def test_wide_layers_of_many_offsets(cin, cout, begin):
+    """5x5x5: the single-kernel form from so many rows on, whichever comes first."""
+    gen = torch.Generator(device="cuda").manual_seed(cin)
+    torch.manual_seed(cin)
+    conv = minuet.nn.SparseConv3d(cin, cout, 5, dtype=torch.float16, device="cuda")
+    for rows in (begin, begin - 1, 1000, begin):
+        cells = torch.randperm(1 << 21, generator=gen, device="cuda")[:rows]
+        coordinates = torch.stack([cells >> 14, (cells >> 7) & 127, cells & 127], 1).int()
+        coordinates = coordinates[F.build_sorted_index(coordinates)]
+        cache = minuet.nn.KernelMapCache(3, torch.int32, "cuda")
+        minuet.set_kernel_map_cache(conv, cache)
+        x = minuet.SparseTensor(torch.randn(rows, cin, generator=gen, device="cuda").half(), coordinates)
+        with torch.no_grad():
+            out = conv(x).F
+            dense, _ = _C.kernel_map_dense(coordinates, coordinates, cache._kernel_offsets((1, 1, 1), (5, 5, 5), (1, 1, 1)), None, None)
+            pad = -cin % 8
+            weights = torch.nn.functional.pad(conv.kernel, (0, 0, 0, pad)).contiguous()
+            wanted = _C.sparse_convolution_forward_implicit(torch.nn.functional.pad(x.F, (0, pad)), weights, dense)
+            again = conv(x).F
+        assert len(cache._kernel_maps_cache) == (rows < begin)
+        # (the three kernels round their product rows, of which there are at most 125)
+        bound = 125 * 2.0 ** -11 * float(wanted.float().abs().max()) if rows < begin else 0.0
+        assert float((out.float() - wanted.float()).abs().max()) <= bound and torch.equal(out, again)
