@@ -625,6 +625,12 @@ int mnt_sparse_convolution_forward_pieces(const float *sources, const float *wei
                                           const float *channel_shift, const void *residual, int activation,
                                           float negative_slope, float *out, void *stream);
 
+/* Rows of 16-bit values [N, C] with zeros after them, [N, padded C], for a layer
+ * whose rows are padded to ones that mnt_sparse_convolution_forward_implicit takes:
+ * of 4 or 8 bytes or a multiple of 16. */
+int mnt_pad_rows(const void *rows, int64_t num_rows, int64_t channels, int64_t padded_channels, int float_dtype,
+                 void *out, void *stream);
+
 /* 1 where mnt_sparse_convolution_forward_implicit (and _tiled) streams rows and
  * weights of a layer of the given shape through LDS, which makes it the faster
  * one for 16-bit layers too wide for the others. */

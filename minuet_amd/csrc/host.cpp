@@ -52,6 +52,7 @@ using TiledFn = int (*)(const void *, const void *, const int32_t *, int64_t, in
                         const float *, const float *, const void *, int, float, void *, void *);
 using PiecesFn = int (*)(const void *, const void *, int64_t, int64_t, int64_t, int64_t, const float *, const float *,
                          const void *, int, float, void *, void *);
+using PadFn = int (*)(const void *, int64_t, int64_t, int64_t, int, void *, void *);
 using TilesFn = int (*)(const int32_t *, int64_t, int64_t, int32_t *, void *);
 using TilesSizeFn = int (*)(int64_t, int64_t, int64_t *);
 using TilesShareFn = double (*)(int64_t, int64_t, int64_t, int64_t, int);
@@ -63,6 +64,7 @@ TablesFn g_tables = nullptr;
 TiledFn g_tiled = nullptr;
 PiecesFn g_pieces = nullptr;
 TiledFn g_single = nullptr;
+PadFn g_pad = nullptr;
 TilesFn g_tiles = nullptr;
 TilesSizeFn g_tiles_size = nullptr;
 TilesShareFn g_tiles_share = nullptr;
@@ -581,7 +583,9 @@ PyObject *run_layer(Layer *l, PyObject *module_dict, PyObject *inputs, const Epi
   PyObject *coordinates = look(in, s__coordinates), *stride = look(in, s__stride);
   PyObject *batch_dims = look(in, s__batch_dims);
   if (coordinates == nullptr || stride == nullptr || batch_dims == nullptr) return none();
-  if (x->size(1) != l->in_channels || x->scalar_type() != kernel.scalar_type() || !x->is_cuda() ||
+  // (rows that the layer pads have the kernel's channels, its weights the padded row's)
+  const int64_t channels = l->kind == kImplicit ? kernel.size(1) : l->in_channels;
+  if (x->size(1) != channels || x->scalar_type() != kernel.scalar_type() || !x->is_cuda() ||
       x->device().index() != l->device || !x->is_contiguous() || (c10::GradMode::is_enabled() && x->requires_grad())) {
     return none();
   }
@@ -660,6 +664,16 @@ PyObject *run_layer(Layer *l, PyObject *module_dict, PyObject *inputs, const Epi
   const void *weights_at = THPVariable_Unpack(l->weights).const_data_ptr();
   const void *packed_at = THPVariable_Unpack(l->packed).const_data_ptr();
   int status = 0;
+  at::Tensor padded;
+  if (channels != l->in_channels) {
+    padded = at::detail::empty_cuda({S, l->in_channels}, kernel.scalar_type(), kernel.device(), std::nullopt);
+    status = g_pad(source, S, channels, l->in_channels, l->float_code, padded.mutable_data_ptr(), stream);
+    if (status != 0) {
+      PyErr_SetString(PyExc_RuntimeError, g_error());
+      return nullptr;
+    }
+    source = padded.const_data_ptr();
+  }
   switch (l->kind) {
     case kImplicit:
       if (l->shortcut != 0) {                              // a target has one source
@@ -922,6 +936,7 @@ PyObject *py_bind(PyObject *, PyObject *args) {
   g_tiled = reinterpret_cast<TiledFn>(address("mnt_sparse_convolution_forward_tiled"));
   g_pieces = reinterpret_cast<PiecesFn>(address("mnt_sparse_convolution_forward_pieces"));
   g_single = reinterpret_cast<TiledFn>(address("mnt_sparse_convolution_forward_single"));
+  g_pad = reinterpret_cast<PadFn>(address("mnt_pad_rows"));
   g_tiles = reinterpret_cast<TilesFn>(address("mnt_kernel_map_tiles"));
   g_tiles_size = reinterpret_cast<TilesSizeFn>(address("mnt_kernel_map_tiles_size"));
   g_tiles_share = reinterpret_cast<TilesShareFn>(address("mnt_kernel_map_tiles_share"));

@@ -27,13 +27,6 @@ from minuet_amd.utils.helpers import as_tuple, generate_kernel_offsets
 __all__ = ["SparseConv", "SparseConv3d", "KernelMapCache"]
 
 _MOST_ROWS = (1 << 63) - 1
-
-# A wide layer (more than 128 output channels) whose rows have to be padded for the
-# single-kernel form pays for that at every call, about 30 us of the host's time, and
-# saves more over as many rows or more: 4 -> 160 channels over 10 000 voxels of a room
-# 31.6 us against 34.1 in three kernels, over 5 000 34.2 and 27.8 (20 -> 256 over
-# 200 000 of a LiDAR scan 125 and 782)
-_PADDED_WIDE_ROWS = 10_000
 # What the tiles of a map have to save a pass, over what making them alone takes,
 # for the next pass to make them with all others: for a map that had none, and
 # to go on (so that a size that wavers does not change the plan every time).
@@ -884,16 +877,14 @@ class SparseConv(Module):
         if dataflow == "implicit":
             return True
         shape = (self.kernel.shape[0], self.in_channels + pad, self.out_channels, features.dtype)
-        # (a copy of the rows, which every call makes, is more than streaming saves: 100 -> 64
-        # channels over 2 000 voxels 14.6 us in three kernels and 26.7, 150 -> 160 over 9 000 34.9 and 48.1)
+        # (a copy of the rows, which every call makes, is more than streaming saves where it is made by the
+        # library: 100 -> 64 channels over 2 000 voxels 14.6 us in three kernels and 26.7)
         return (F.prefers_implicit(*shape) or (pad == 0 and F.prefers_streamed(*shape))
                 or F.implicit_rows_from(*shape) <= features.shape[0])
 
     def _single_kernel_from(self, dtype: torch.dtype) -> int:
         """The fewest rows over which ``auto`` takes the single-kernel form for a
         16-bit layer (0: the number of rows does not matter)."""
-        if self.out_channels > 128 and self.in_channels % 8 != 0 and self.in_channels <= 32:
-            return _PADDED_WIDE_ROWS
         shape = (self.kernel.shape[0], -(-self.in_channels // 8) * 8, self.out_channels, dtype)
         begin = F.implicit_rows_from(*shape)
         return begin if begin <= F.implicit_rows_limit(shape[1], dtype) else 0
@@ -1103,7 +1094,7 @@ class SparseConv(Module):
                     features = _C.sparse_convolution_forward_implicit(sources, weights, dense,
                                                                       epilogue=epilogue,
                                                                       packed_weights=packed)
-                if not pad and dense.is_contiguous():
+                if dense.is_contiguous():
                     made = ("IMPLICIT", weights, kept, (dense.data_ptr(),), dense, 0, tiles, single)
             else:
                 features, made = self._forward_tables(cache, map_args, sources, epilogue)

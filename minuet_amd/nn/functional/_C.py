@@ -119,6 +119,7 @@ SIGNATURES = {
                                                        _int, ctypes.c_float, _vp, _vp]),
     "mnt_sparse_convolution_forward_pieces": (_int, [_vp, _vp, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _int,
                                                      ctypes.c_float, _vp, _vp]),
+    "mnt_pad_rows": (_int, [_vp, _i64, _i64, _i64, _int, _vp, _vp]),
     "mnt_sparse_convolution_streamed": (_int, [_i64, _i64, _i64, _i64, _int]),
     "mnt_sparse_convolution_forward_tiled": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _vp, _vp, _vp,
                                                     _int, ctypes.c_float, _vp, _vp]),
@@ -202,7 +203,7 @@ def _bound_host():
     spec.loader.exec_module(module)
     names = ("mnt_sparse_convolution_forward_implicit", "mnt_sparse_convolution_forward_groups",
              "mnt_sparse_convolution_forward_fused", "mnt_sparse_convolution_forward_tiled", "mnt_kernel_map_tiles",
-             "mnt_sparse_convolution_forward_pieces", "mnt_sparse_convolution_forward_single",
+             "mnt_sparse_convolution_forward_pieces", "mnt_sparse_convolution_forward_single", "mnt_pad_rows",
              "mnt_kernel_map_tiles_size", "mnt_kernel_map_tiles_share", "mnt_last_error")
     hooks = tuple(getattr(torch_module, name) for name in (
         "_global_forward_hooks", "_global_forward_pre_hooks", "_global_backward_hooks",
