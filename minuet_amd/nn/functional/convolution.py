@@ -299,7 +299,8 @@ def sparse_convolution_forward(sources: torch.Tensor, weights: torch.Tensor,
     single-kernel output-stationary form (needs ``kernel_map.dense`` and
     ``weights`` in their original offset order, as a layer holds them) and
     ``"auto"`` takes the implicit form where it is the faster one: 16-bit
-    features whose rows it can stage, and fp32 layers that are narrow or small.
+    features whose rows it can stage, and fp32 layers that are narrow, small or, with
+    few input channels, large.
 
     ``"list_driven"`` is Gather-GEMM-Scatter without the rank tables: the GEMM
     reads its rows through the pair list and writes its products in
