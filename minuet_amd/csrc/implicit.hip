@@ -368,11 +368,11 @@ __global__ __launch_bounds__(kImplicitBlock) void implicit_forward_kernel(
 // (step, channel block, lane) = 8 elements of K' for one output channel), and
 // each wavefront takes its blocks of 32 targets from there.  Nothing is
 // pipelined by hand: the kernel is short on registers, and the wavefronts a
-// SIMD holds cover each other's trips to memory.
+// SIMD holds cover each other's trips to memory, which bound it.  (So 64 channels
+// have four steps in flight: 110 to 118 registers instead of 168 to 203.)
 // Dynamic LDS: steps * NB KiB of weight pieces + 4 turn areas.
 constexpr int kNarrowBlock = 256;
-constexpr int kNarrowBlocksPerWave = 2;    // 32-target blocks a wavefront takes
-constexpr int kNarrowSteps = 8;            // steps of K' whose rows are in flight together
+constexpr int kNarrowMostBlocks = 8;       // 32-target blocks a wavefront takes at most
 constexpr int kNarrowMaxLds = 64 * 1024;
 
 // Whether narrow_forward_kernel takes the layer: 16-bit rows of 4, 8 or 16
@@ -389,10 +389,11 @@ static bool narrow_fits(int64_t O, int64_t K, int64_t N, int esize, bool has_wei
 }
 
 template <typename T, int NB, int RB>
-__global__ __launch_bounds__(kNarrowBlock, NB == 1 ? 4 : 2) void narrow_forward_kernel(
+__global__ __launch_bounds__(kNarrowBlock, NB <= 2 ? 4 : 2) void narrow_forward_kernel(
     const unsigned char *__restrict__ sources, const T *__restrict__ weights,
     const int *__restrict__ kernel_map, long long num_targets, int num_offsets, int N, int steps,
-    unsigned char *__restrict__ out, Epilogue ep) {
+    int blocks_per_wave, unsigned char *__restrict__ out, Epilogue ep) {
+  constexpr int kNarrowSteps = NB == 2 ? 4 : 8;                 // of K', whose rows are in flight together
   constexpr int SL = 16 / RB;                                   // source rows per operand piece
   constexpr int KR = RB / static_cast<int>(sizeof(T));          // input channels
   typedef typename VecOf<RB>::type RowVec;
@@ -423,9 +424,9 @@ __global__ __launch_bounds__(kNarrowBlock, NB == 1 ? 4 : 2) void narrow_forward_
   const uint4 *w_pieces = reinterpret_cast<const uint4 *>(narrow_lds) + lane;
   unsigned char *turn = narrow_lds + static_cast<size_t>(steps) * NB * 1024 + wv * kTurnBytes;
   const bool turned = (static_cast<long long>(N) * sizeof(T)) % 16 == 0;
-  for (int j = 0; j < kNarrowBlocksPerWave; ++j) {
+  for (int j = 0; j < blocks_per_wave; ++j) {
     const long long block_t0 =
-        ((static_cast<long long>(blockIdx.x) * kNarrowBlocksPerWave + j) * (kNarrowBlock / 64) + wv) * 32;
+        ((static_cast<long long>(blockIdx.x) * blocks_per_wave + j) * (kNarrowBlock / 64) + wv) * 32;
     if (block_t0 >= num_targets) break;
     const long long t = block_t0 + r;
     const bool t_ok = t < num_targets;
@@ -545,12 +546,36 @@ static void implicit_typed(const T *sources, const T *weights, const T *packed, 
         const int steps = static_cast<int>(div_ceil(O * K, 16));
         const int blocks = static_cast<int>(div_ceil(N, 32));
         const size_t lds = static_cast<size_t>(steps) * blocks * 1024 + (kNarrowBlock / 64) * kTurnBytes;
-        const unsigned grid = static_cast<unsigned>(
-            div_ceil(Tn, int64_t{32} * (kNarrowBlock / 64) * kNarrowBlocksPerWave));
+        // As many targets to a workgroup as make the fewest rounds of workgroups
+        // full ones, where to start one and to bring its weights takes about half as
+        // long as a block of a wavefront's.  `held`: what the chip holds at once, by
+        // registers (launch bounds) and LDS.  Two blocks a wavefront whatever the size
+        // were 782 workgroups over 200 000 targets, 14 of them for a second round; us,
+        // that (with eight steps in flight for 64 channels) and here: 4 -> 64 over 200 000
+        // 21.7 / 15.3, 600 000 50 / 31, 10 000 9.4 / 6.5; 4 -> 96 over 200 000 25.0 /
+        // 20.2, 4 -> 128 29.6 / 25.7, 8 -> 64 29.9 / 22.4.
+        const int64_t wavefronts = blocks == 1 && narrow_bytes == 8 ? 5
+                                   : blocks <= 2                    ? 4
+                                   : blocks == 3 && narrow_bytes == 8 ? 3
+                                                                      : 2;
+        const int64_t held =
+            compute_units() * std::min<int64_t>(wavefronts, 160 * 1024 / static_cast<int64_t>(lds));
+        int blocks_per_wave = 1;
+        double least = 0.0;
+        for (int b = 1; b <= kNarrowMostBlocks; ++b) {
+          const int64_t groups = div_ceil(Tn, int64_t{32} * (kNarrowBlock / 64) * b);
+          const double takes = static_cast<double>(div_ceil(groups, held)) * (b + 0.5);
+          if (b == 1 || takes < least) {
+            least = takes;
+            blocks_per_wave = b;
+          }
+        }
+        const unsigned grid =
+            static_cast<unsigned>(div_ceil(Tn, int64_t{32} * (kNarrowBlock / 64) * blocks_per_wave));
 #define MNT_NARROW(NB, RB)                                                                              \
   narrow_forward_kernel<T, NB, RB><<<grid, kNarrowBlock, lds, stream>>>(                                \
       reinterpret_cast<const unsigned char *>(sources), weights, kernel_map, Tn, static_cast<int>(O),   \
-      static_cast<int>(N), steps, reinterpret_cast<unsigned char *>(out), ep)
+      static_cast<int>(N), steps, blocks_per_wave, reinterpret_cast<unsigned char *>(out), ep)
 #define MNT_NARROW_RB(NB)            \
   if (narrow_bytes == 4) {           \
     MNT_NARROW(NB, 4);               \

@@ -1008,3 +1008,24 @@ def test_module_takes_offset_groups_for_wide_layers(kind, stride, n, extent):
     diff = (auto.float() - three.float()).abs().max().item()
     ulp = three.float().abs().max().item() * 2.0 ** (-7 if kind == "bf16" else -10)
     assert diff <= max(2e-2 * three.float().pow(2).mean().sqrt().item(), ulp), diff
+
+
+@pytest.mark.parametrize("kind", ["fp16", "bf16"])
+@pytest.mark.parametrize("targets, cin, cout", [
+    (140001, 4, 64), (300001, 4, 32), (262145, 2, 48), (70001, 4, 128), (100000, 4, 96), (99999, 8, 64), (65537, 8, 100),
+    (66000, 8, 20), (1050000, 2, 4)])
+def test_short_rows_over_many_targets(targets, cin, cout, kind):
+    """Several blocks of targets a wavefront, and a last workgroup that is not full."""
+    gen = torch.Generator(device="cuda").manual_seed(targets)
+    x = torch.randn(5000, cin, generator=gen, device="cuda").to(TORCH[kind])
+    w = torch.randn(27, cin, cout, generator=gen, device="cuda").to(TORCH[kind])
+    dense = torch.randint(-10000, 5000, (27, targets), generator=gen, device="cuda", dtype=torch.int32).clamp(min=-1)
+    wanted, size = (torch.zeros(targets, cout, device="cuda") for _ in range(2))
+    for offset in range(27):
+        hit = (dense[offset] >= 0).nonzero()[:, 0]
+        picked, weight = x[dense[offset, hit].long()].float(), w[offset].float()
+        wanted[hit] += picked @ weight
+        size[hit] += picked.abs() @ weight.abs()
+    out = _C.sparse_convolution_forward_implicit(x, w, dense)
+    # products are exact in 32 bits; both sums round at most 27 x 8 times, the result once
+    assert bool(((out.float() - wanted).abs() <= torch.finfo(TORCH[kind]).eps * wanted.abs() + 440 * 2.0 ** -24 * size).all())
