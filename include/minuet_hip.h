@@ -627,7 +627,7 @@ int mnt_sparse_convolution_forward_pieces(const float *sources, const float *wei
 
 /* Rows of 16-bit values [N, C] with zeros after them, [N, padded C], for a layer
  * whose rows are padded to ones that mnt_sparse_convolution_forward_implicit takes:
- * of 4 or 8 bytes or a multiple of 16. */
+ * of 4 or 8 bytes or a multiple of 16 (rows of 32-bit values as of twice as many). */
 int mnt_pad_rows(const void *rows, int64_t num_rows, int64_t channels, int64_t padded_channels, int float_dtype,
                  void *out, void *stream);
 

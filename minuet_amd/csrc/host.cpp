@@ -667,7 +667,10 @@ PyObject *run_layer(Layer *l, PyObject *module_dict, PyObject *inputs, const Epi
   at::Tensor padded;
   if (channels != l->in_channels) {
     padded = at::detail::empty_cuda({S, l->in_channels}, kernel.scalar_type(), kernel.device(), std::nullopt);
-    status = g_pad(source, S, channels, l->in_channels, l->float_code, padded.mutable_data_ptr(), stream);
+    // (of 32-bit values as of twice as many of 16 bits)
+    const int halves = l->item_size == 4 ? 2 : 1;
+    status = g_pad(source, S, halves * channels, halves * l->in_channels, halves == 2 ? 1 : l->float_code,
+                   padded.mutable_data_ptr(), stream);
     if (status != 0) {
       PyErr_SetString(PyExc_RuntimeError, g_error());
       return nullptr;

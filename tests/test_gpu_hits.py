@@ -111,3 +111,30 @@ def test_products_are_added_after_in_large_layers(rows, targets, cin, cout):
     w[5, 0, 0] = float("inf")                            # what a target has no source for does not reach it
     out = _C.sparse_convolution_forward_implicit(x, w, dense)
     assert bool(out[dense[5] < 0].isfinite().all())
+
+
+@pytest.mark.parametrize("kernel, cin, cout", [(3, 3, 32), (3, 1, 4), (2, 3, 64), (5, 2, 48)])
+def test_layers_of_less_than_four_channels(kernel, cin, cout):
+    """Rows of less than four values are padded to four, at the first call and from the second on."""
+    gen = torch.Generator(device=DEVICE).manual_seed(cin)
+    torch.manual_seed(cin)
+    conv = minuet.nn.SparseConv3d(cin, cout, kernel, dtype=torch.float32, device=DEVICE, bias=True)
+    for rows in (1, 700, 6000):
+        cells = torch.randperm(1 << 16, generator=gen, device=DEVICE)[:rows]
+        coordinates = torch.stack([cells >> 10, (cells >> 5) & 31, cells & 31], 1).int()
+        coordinates = coordinates[F.build_sorted_index(coordinates)]
+        cache = minuet.nn.KernelMapCache(3, torch.int32, DEVICE)
+        minuet.set_kernel_map_cache(conv, cache)
+        dense, _ = _C.kernel_map_dense(coordinates, coordinates,
+                                       cache._kernel_offsets((1, 1, 1), (kernel,) * 3, (1, 1, 1)), None, None)
+        with torch.no_grad():
+            for turn in range(3):
+                conv.kernel.mul_(-0.5)
+                x = minuet.SparseTensor(torch.randn(rows, cin, generator=gen, device=DEVICE), coordinates)
+                out = conv(x).F
+                wanted = reference(x.F.double(), conv.kernel.double(), dense)
+                size = reference(x.F.abs().double(), conv.kernel.abs().double(), dense) + conv.bias.abs()
+                # a value is rounded at most cin x offsets times in its sums and twice at the end
+                bound = (cin * kernel ** 3 + 16) * 2.0 ** -24 * size
+                assert bool(((out.double() - wanted - conv.bias.double()).abs() <= bound).all())
+        assert len(cache._kernel_maps_cache) == 0 and conv._fast is not None
