@@ -27,6 +27,14 @@ from minuet_amd.utils.helpers import as_tuple, generate_kernel_offsets
 __all__ = ["SparseConv", "SparseConv3d", "KernelMapCache"]
 
 _MOST_ROWS = (1 << 63) - 1
+
+# A layer that records gradients pads rows and weights at every call, some 16 us of the
+# host's time: fp32 layers of less than four input channels and 16-bit ones of more than
+# 128 output channels do so from this many output values (of source rows) on.  us in three
+# kernels and padded: fp32 3 -> 16 over 1 000 26 / 36, 3 -> 64 over 20 000 29 / 36, over 200 000
+# 131 / 74; fp16 20 -> 256 over 2 000 29 / 37, 4 -> 160 over 20 000 48 / 37.
+_PADDED_VALUES = 2_000_000
+
 # What the tiles of a map have to save a pass, over what making them alone takes,
 # for the next pass to make them with all others: for a map that had none, and
 # to go on (so that a size that wavers does not change the plan every time).
@@ -849,6 +857,9 @@ class SparseConv(Module):
                 self._packed = (key, weights, F.pack_weights(weights), held)
         return self._packed[1], self._packed[2]
 
+    def _records(self) -> bool:
+        return torch.is_grad_enabled() and self.kernel.requires_grad
+
     def _row_padding(self, features: torch.Tensor) -> int:
         """Zero input channels to append so that the feature rows of a 16-bit
         layer become ones the single-kernel dataflow takes (4 or 8 bytes under
@@ -882,12 +893,22 @@ class SparseConv(Module):
         return (F.prefers_implicit(*shape) or (pad == 0 and F.prefers_streamed(*shape))
                 or F.implicit_rows_from(*shape) <= features.shape[0])
 
-    def _single_kernel_from(self, dtype: torch.dtype) -> int:
-        """The fewest rows over which ``auto`` takes the single-kernel form for a
-        16-bit layer (0: the number of rows does not matter)."""
-        shape = (self.kernel.shape[0], -(-self.in_channels // 8) * 8, self.out_channels, dtype)
-        begin = F.implicit_rows_from(*shape)
-        return begin if begin <= F.implicit_rows_limit(shape[1], dtype) else 0
+    def _lines(self, dtype: torch.dtype, channels: int):
+        """Of a layer whose rows have so many channels, once they are padded: in
+        fp32 the rows up to which, from which on and up to which at all the
+        kernel of hits takes it, in 16 bits the fewest over which ``auto`` takes the
+        single-kernel form (0: their number does not matter).  Kept with the routes."""
+        lines = self._routes.get(("lines", dtype))
+        if lines is None:
+            layer = (self.kernel.shape[0], channels, self.out_channels, dtype)
+            far = F.implicit_rows_limit(channels, dtype)
+            if dtype == torch.float32:
+                lines = (F.hits_rows_limit(*layer), F.hits_rows_from(*layer), far)
+            else:
+                begin = F.implicit_rows_from(*layer)
+                lines = begin if begin <= far else 0
+            self._routes[("lines", dtype)] = lines
+        return lines
 
     def _has_single_sources(self, features: torch.Tensor, pad: int = 0) -> bool:
         """Whether a target of this layer has one source, and the kernel for that
@@ -1022,18 +1043,20 @@ class SparseConv(Module):
                 # the three kernels', us there and here 3 -> 64 over 20 000 26.1 / 15.2, over 200 000 134 / 69,
                 # 3 -> 16 over 1 000 18.5 / 15.0; of five to eight values the error is up to 1.26 times)
                 channels = max(self.in_channels, 4)
-                most = F.hits_rows_limit(volume, channels, self.out_channels, sources.dtype)
-                again = F.hits_rows_from(volume, channels, self.out_channels, sources.dtype)
-                far = F.implicit_rows_limit(channels, sources.dtype)
+                most, again, far = self._lines(sources.dtype, channels)
                 count = sources.shape[0]
                 hits = count <= most or again <= count <= far
+                if channels != self.in_channels and count * self.out_channels < _PADDED_VALUES and self._records():
+                    hits = False
                 if hits:
                     rows = (0, most) if count <= most else (again, far)
                 else:
                     rows = (most + 1, again - 1) if count < again else (far + 1, _MOST_ROWS)
             begin = 0                               # (rows from which the single-kernel form may be taken)
             if hits is None and dataflow == "auto" and sources.dtype != torch.float32:
-                begin = self._single_kernel_from(sources.dtype)
+                begin = self._lines(sources.dtype, -(-self.in_channels // 8) * 8)
+                if self.out_channels > 128 and self.in_channels % 8 and self.in_channels <= 32 and self._records():
+                    begin = -(-_PADDED_VALUES // self.out_channels)
             small = sources.shape[0] < begin
             route_key = (sources.dtype, sources.is_cuda, dataflow, hits, small)
             route = self._routes.get(route_key)

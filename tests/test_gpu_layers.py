@@ -275,3 +275,23 @@ def test_pad_rows_refuses_what_it_cannot_write():
                       (rows.data_ptr(), 4, 3, 8, 1, out.data_ptr() + 2), (None, 4, 3, 8, 1, out.data_ptr()),
                       (rows.data_ptr(), 1 << 40, 3, 8, 1, out.data_ptr())):
         assert call(*arguments, None) != 0
+
+
+@pytest.mark.parametrize("dtype, cin, cout, rows, tables", [
+    (torch.float32, 3, 64, 1000, 1), (torch.float32, 3, 64, 40000, 0), (torch.float16, 4, 160, 1000, 1),
+    (torch.float16, 20, 256, 9000, 0), (torch.float16, 16, 160, 1000, 0), (torch.float32, 4, 64, 1000, 0)])
+def test_layers_that_record_gradients_pad_where_it_pays(dtype, cin, cout, rows, tables):
+    """The same values with and without a record, whichever form each takes, in both orders."""
+    conv, x = layer_and_input(rows, cin, cout, dtype)
+    bound = 4 * torch.finfo(dtype).eps if dtype != torch.float32 else 1e-5
+    for order in ((True, False), (False, True)):
+        results = []
+        for recorded in order:
+            cache = minuet.nn.KernelMapCache(3, torch.int32, DEVICE)
+            minuet.set_kernel_map_cache(conv, cache)
+            with torch.set_grad_enabled(recorded):
+                for _ in range(2):
+                    results.append(conv(x).F.float())
+            assert len(cache._kernel_maps_cache) == (tables if recorded else 0)
+        for other in results[1:]:
+            assert float((other - results[0]).abs().max()) <= bound * 27 * float(results[0].abs().max())
