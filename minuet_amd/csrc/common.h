@@ -144,8 +144,15 @@ class Arena {
   const volatile unsigned long long *wait_words(int count, unsigned long long sequence);
   // Long-lived device blocks that survive scopes (state of the two-phase entry
   // points; slot 0: target coordinates, slot 1: kernel-map build, slot 2: pass
-  // builder).  Grows to at least `bytes`; 0 returns the current block.
+  // builder, slot 3: words()).  Grows to at least `bytes`; 0 returns the current block.
   void *persistent(int slot, size_t bytes);
+  // kWords words of device memory through which the workgroups of one launch tell each
+  // other numbers: zero when the block is made, and written by nothing but such
+  // launches, which leave the number of their call (next_sequence) with each.  No
+  // call of this arena ever has that number again, and a new arena makes a new
+  // block, so a word that has the call's number was written by that call.
+  static constexpr int kWords = 128;
+  unsigned long long *words();
 
   hipStream_t stream() const { return stream_; }
 
@@ -192,9 +199,10 @@ class Arena {
   void *pinned_ = nullptr;
   void *pinned_device_ = nullptr;
   unsigned long long sequence_ = 0;
-  static constexpr int kPersistentSlots = 3;
-  void *persistent_[kPersistentSlots] = {nullptr, nullptr, nullptr};
-  size_t persistent_size_[kPersistentSlots] = {0, 0, 0};
+  static constexpr int kPersistentSlots = 4;
+  void *persistent_[kPersistentSlots] = {nullptr, nullptr, nullptr, nullptr};
+  size_t persistent_size_[kPersistentSlots] = {0, 0, 0, 0};
+  bool words_cleared_ = false;
   // guarded by the registry's mutex
   bool held_ = false, pinned_by_thread_ = false;
   unsigned long long holder_ = 0;            // token of the thread inside a call / that pinned it

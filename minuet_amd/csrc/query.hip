@@ -2336,12 +2336,11 @@ extern "C" int mnt_sorted_kernel_map_lists(const void *coords, int64_t n, int nd
       profile_mark("enter:map_small", stream);
       Arena &arena = Arena::of(stream);
       arena.map_state_valid = false;
-      Scope scope(stream);
       char *pinned_device = static_cast<char *>(arena.pinned_device());
       const unsigned long long sequence = arena.next_sequence();
       enqueue_small_map(coords, n, ndim, coord_dtype, offsets_host, static_cast<int>(num_offsets), map_halves_enabled(),
                         reorder, indices_out, sorted_coords_out, in_idx_out, out_idx_out, sizes_dev_out, order_dev_out,
-                        scope, reinterpret_cast<unsigned *>(pinned_device + Arena::kPlanOffset),
+                        arena.words(), reinterpret_cast<unsigned *>(pinned_device + Arena::kPlanOffset),
                         reinterpret_cast<long long *>(pinned_device + kChainHostOffset), arena.flag_device(1), sequence,
                         stream);
       verdict = hear(arena, sequence);

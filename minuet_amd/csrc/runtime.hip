@@ -146,6 +146,7 @@ void Arena::free_all(bool synchronise) {
   map_state_valid = false;
   pass_pending = false;
   zero_bitmap_words = 0;
+  words_cleared_ = false;
 }
 
 void Arena::reset_device() {
@@ -271,6 +272,20 @@ void *Arena::persistent(int slot, size_t bytes) {
     if (slot == 0) zero_bitmap_words = 0;
   }
   return persistent_[slot];
+}
+
+__global__ __launch_bounds__(Arena::kWords) void clear_words_kernel(unsigned long long *__restrict__ words) {
+  words[threadIdx.x] = 0ull;
+}
+
+unsigned long long *Arena::words() {
+  auto *block = static_cast<unsigned long long *>(persistent(3, sizeof(unsigned long long) * kWords));
+  if (!words_cleared_) {
+    clear_words_kernel<<<1, kWords, 0, stream_>>>(block);
+    check_launch("clear_words_kernel");
+    words_cleared_ = true;
+  }
+  return block;
 }
 
 // ---- stage profiler -------------------------------------------------------

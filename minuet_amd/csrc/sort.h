@@ -60,13 +60,14 @@ void sort_started_batches(const void *rows, int64_t n, int ndim, int coord_dtype
 
 bool small_map_takes(int64_t n, int num_offsets);
 // The int32 permutation, the sorted rows and the pair lists of a cloud mapped onto
-// itself, in one launch.  For the host: order, nothing and sizes in plan_host
+// itself, in one launch; `words` and `sequence` are Arena::words() and a number of that
+// arena.  For the host: order, nothing and sizes in plan_host
 // (num_offsets words each), the extremes and the verdict (not 0: nothing was
 // written but it) in chain_host, then the flag.
 void enqueue_small_map(const void *coords, int64_t n, int ndim, int coord_dtype, const int64_t *offsets_host,
                        int num_offsets, bool allow_halves, int reorder, int32_t *indices_out, void *sorted_out,
-                       int32_t *in_idx, int32_t *out_idx, int32_t *sizes, int32_t *order, Scope &scope,
-                       unsigned *plan_host, long long *chain_host, unsigned long long *flag,
+                       int32_t *in_idx, int32_t *out_idx, int32_t *sizes, int32_t *order,
+                       unsigned long long *words, unsigned *plan_host, long long *chain_host, unsigned long long *flag,
                        unsigned long long sequence, hipStream_t stream);
 
 // ---- the bucket sort as a chain of launches that never waits for the host ----

@@ -1715,12 +1715,14 @@ __global__ __launch_bounds__(kSmallSortBlock) void small_sort_kernel(
 // lists) the step was 26.5 us of kernels and the gaps between them: 45.5 us a
 // call at 2 039 voxels under 3x3x3, 16.4 and 35.8 here.  The numbers are the only thing
 // that passes between workgroups, each in one word with the call's number beside
-// it, so nothing is cleared and no fence is needed.  A workgroup that has waited
+// it, so nothing is cleared from call to call and no fence is needed.  (The words
+// are Arena::words(): scratch would hold what other calls have left, and a
+// coordinate or a count of theirs may look like a number of this call.)  A workgroup that has waited
 // `patience` ticks (of 10 ns) counts the hits it has not heard of itself: it
 // depends on no other to come to its end.
 struct SmallMapOut {
   int *in_idx, *out_idx, *sizes, *order;      // (the last two nullable)
-  unsigned long long *counts;                 // [num_offsets]
+  unsigned long long *counts;                 // [num_offsets] of Arena::words()
   unsigned *plan_host;                        // order, ., sizes: num_offsets words each
   long long *chain_host;                      // extremes, then the verdict
   unsigned long long *flag;
@@ -1731,6 +1733,7 @@ struct SmallMapOut {
 constexpr int kSmallMapOffsets = 128;
 constexpr int kSmallMapCountBits = 13;
 static_assert(kSmallSortRows < 1 << kSmallMapCountBits, "a count beside the call's number");
+static_assert(kSmallMapOffsets <= Arena::kWords, "a word for every offset");
 struct SmallMapTable : OffsetTableOf<kSmallMapOffsets> {};
 
 template <typename CT>
@@ -1981,14 +1984,14 @@ static unsigned map_patience() {
 
 void enqueue_small_map(const void *coords, int64_t n, int ndim, int coord_dtype, const int64_t *offsets_host,
                        int num_offsets, bool allow_halves, int reorder, int32_t *indices_out, void *sorted_out,
-                       int32_t *in_idx, int32_t *out_idx, int32_t *sizes, int32_t *order, Scope &scope,
-                       unsigned *plan_host, long long *chain_host, unsigned long long *flag,
+                       int32_t *in_idx, int32_t *out_idx, int32_t *sizes, int32_t *order,
+                       unsigned long long *words, unsigned *plan_host, long long *chain_host, unsigned long long *flag,
                        unsigned long long sequence, hipStream_t stream) {
   const SmallMapTable table = make_offset_table<SmallMapTable>(offsets_host, num_offsets, ndim, allow_halves);
   int zero = -1;
   for (int o = 0; o < num_offsets; ++o) zero = table.kind[o] == 2 ? o : zero;
-  const SmallMapOut out{in_idx, out_idx, sizes, order, scope.alloc<unsigned long long>(num_offsets), plan_host,
-                        chain_host, flag, sequence, reorder, map_patience()};
+  const SmallMapOut out{in_idx, out_idx, sizes, order, words, plan_host, chain_host, flag, sequence, reorder,
+                        map_patience()};
   const unsigned blocks = static_cast<unsigned>(table.num_kept + (zero >= 0 ? 1 : 0));
   const int idx_bits = bit_width(static_cast<unsigned long long>(n - 1));
   if (coord_dtype == MNT_INT32) {

@@ -6,6 +6,7 @@ import torch
 import c_oracle
 import minuet_oracle as orc
 from helpers import dev, host, random_cloud, sorted_unique
+from minuet_amd.nn import functional as F
 from minuet_amd.nn.functional import _C
 
 pytestmark = pytest.mark.gpu
@@ -99,3 +100,25 @@ def test_map_lists_of_equal_rows():
     for name in ("in_idx", "out_idx"):
         assert torch.equal(built[name], whole[name])
     np.testing.assert_array_equal(built["sizes_host"], whole["sizes_host"])
+
+
+# The library's scratch memory begins with integers that look like the words the workgroups of the next call
+# answer each other with: the call's number (1, 2, ... after a reset) above 13 bits of a count.  A sort of more than
+# 4 096 rows leaves its extremes there, a batch that is collated its 64-bit coordinates.
+@pytest.mark.parametrize("patience", [None, "0"])
+@pytest.mark.parametrize("left_by", ["sort", "collate"])
+def test_map_lists_after_calls_that_leave_such_words(left_by, patience, monkeypatch):
+    if patience is not None:
+        monkeypatch.setenv("MINUET_MAP_PATIENCE", patience)
+    c, _ = sorted_unique(random_cloud(600, 14, 5, lo=-7))
+    off = orc.generate_kernel_offsets(3, 3, 1, 1)
+    for _ in range(2):
+        torch.cuda.synchronize()
+        _C.cuda_device_reset()
+        for number in range(2, 18, 2):           # (one number for the sort or the batch, one for the map)
+            rows = random_cloud(5000 if left_by == "sort" else 300, 1 << 13, number, lo=number << 13, dtype=np.int64)
+            if left_by == "sort":
+                _C.sort_coordinates(dev(rows), None)
+            else:
+                F.collate([dev(rows)])
+            check_map_lists(c, off)
