@@ -469,6 +469,7 @@ __global__ __launch_bounds__(kQueryThreads) void query_kernel(
   // half are kept here as well, and equal rows, which break the symmetry, are
   // reported.
   bool halves = false;
+  int num_members = num_offsets;
   if (device_plan != nullptr) {
     // a launch inside a chain that never went back to the host: the verdict of
     // the launches before it and the plan come from device memory.  The values
@@ -485,6 +486,7 @@ __global__ __launch_bounds__(kQueryThreads) void query_kernel(
     frame.total_bits = __builtin_amdgcn_readfirstlane(device_plan->frame.total_bits);
     tables = device_plan->tables;
     num_groups = __builtin_amdgcn_readfirstlane(device_plan->num_groups);
+    num_members = __builtin_amdgcn_readfirstlane(device_plan->num_members);
     delta_min = uniform64(device_plan->delta_min);
     delta_max = uniform64(device_plan->delta_max);
     const int in_rows = __builtin_amdgcn_readfirstlane(device_plan->groups_in_rows);
@@ -524,7 +526,7 @@ __global__ __launch_bounds__(kQueryThreads) void query_kernel(
   const long long t_end = t0 + kTargetsPerTile < num_targets ? t0 + kTargetsPerTile : num_targets;
 
   if (tables != nullptr) {
-    for (int i = tid; i < 4 * num_groups + 2 * num_offsets; i += kQueryThreads) s_dynamic[i] = tables[i];
+    for (int i = tid; i < 4 * num_groups + 2 * num_members; i += kQueryThreads) s_dynamic[i] = tables[i];
   } else if (w == kQueryThreads / kWave - 1) {
     const int count = 4 * num_groups + 2 * num_offsets;
 #pragma unroll
@@ -661,7 +663,6 @@ __global__ __launch_bounds__(kQueryThreads) void query_kernel(
     const unsigned long long answers_from = c == 0 ? 0ull : first_key;
     const unsigned long long answers_to = c == num_chunks - 1 ? ~0ull : next_first;
     const bool counting = tile_counts != nullptr;
-    const int num_members = s_all_groups[num_groups - 1].z + s_all_groups[num_groups - 1].w;
 #define MNT_RESOLVE(WHOLE)                                                                         \
     if (by_rows) {                                                                                 \
       resolve_chunk_rows<OT, WHOLE, kLists>(reinterpret_cast<const unsigned *>(win), s_dir, len,   \

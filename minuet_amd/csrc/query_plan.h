@@ -97,7 +97,7 @@ struct DevicePlan {
   int num_groups;
   int groups_in_rows;       // every group's offsets differ in the last coordinate only
   int verdict;              // 0: go; otherwise the chain stops (sort declined, or keys beyond 63 bits)
-  int num_offsets;
+  int num_members;          // offsets that are looked up
   int tables[kPlanInts];    // groups (first delta low / high, first member, members), then members (step, offset)
   // A cloud mapped onto itself under offsets that come in pairs d / -d: the
   // hits of -d are those of d with source and target exchanged, in the same
@@ -262,7 +262,7 @@ __device__ __forceinline__ void make_plan_on_device(const long long *__restrict_
     out->num_groups = num_groups;
     out->groups_in_rows = in_rows ? 1 : 0;
     out->verdict = declined != 0 ? static_cast<int>(declined) : (fits ? 0 : 2);
-    out->num_offsets = num_offsets;
+    out->num_members = num_kept;
     // the sort's key: fields of the cloud's own ranges, coordinate 0 on top
     int sort_bits = 0, below_top = 0;
 #pragma unroll
