@@ -345,12 +345,17 @@ struct Layer {
   int64_t gather_tile_value, scatter_tile_value;
   int64_t num_offsets, in_channels, out_channels;
   int64_t item_size;
-  // The source rows for which this kind is the one to take, and the module's
-  // Layer for the others, if it has run on such a cloud (both null and 0 to
-  // the most there are where the choice does not depend on rows).
+  // The source rows for which this kind is the one to take, and a Layer of the
+  // module for others, if it has run on such a cloud, which names the next (null,
+  // and 0 to the most there are, where the choice does not depend on rows).
   int64_t rows_from, rows_to;
   PyObject *other;
 };
+
+// Layers that a module keeps: a kind may be the one to take over several ranges
+// of rows (an fp32 layer multiplies hits, writes product rows, multiplies hits
+// again and, where features are past 32-bit offsets, writes product rows).
+constexpr int kMostLayers = 4;
 
 void layer_dealloc(PyObject *self) {
   Layer *l = reinterpret_cast<Layer *>(self);
@@ -415,15 +420,6 @@ PyObject *layer_new(PyTypeObject *type, PyObject *args, PyObject *) {
   l->scatter_tile = hold(look(config, s_scatter_tile_size));
   l->rows_from = rows_from;
   l->rows_to = rows_to;
-  if (Py_TYPE(other) == &LayerType) {                    // the module's Layer so far
-    Layer *last = reinterpret_cast<Layer *>(other);
-    if (last->kind != kind) {
-      Py_CLEAR(last->other);                             // two at most, and no circle
-      l->other = hold(other);
-    } else if (last->other != nullptr) {
-      l->other = hold(last->other);
-    }
-  }
   l->kind = kind;
   l->shortcut = shortcut;
   l->device = w->device().index();
@@ -436,7 +432,23 @@ PyObject *layer_new(PyTypeObject *type, PyObject *args, PyObject *) {
   l->threshold_value = l->has_threshold ? PyFloat_AsDouble(l->threshold) : 0.0;
   l->gather_tile_value = l->gather_tile == Py_None ? 0 : PyLong_AsLongLong(l->gather_tile);
   l->scatter_tile_value = l->scatter_tile == Py_None ? 0 : PyLong_AsLongLong(l->scatter_tile);
-  return PyErr_Occurred() ? nullptr : made.release();
+  if (PyErr_Occurred()) return nullptr;
+  // the module's Layers so far: those for other rows stay, the latest first
+  Layer *last = l;
+  PyObject *next = Py_TYPE(other) == &LayerType ? hold(other) : nullptr;
+  for (int count = 1; next != nullptr && count < kMostLayers;) {
+    const Ref before(next);
+    Layer *b = reinterpret_cast<Layer *>(next);
+    next = b->other;                                     // (taken from it)
+    b->other = nullptr;
+    if (b->rows_to < l->rows_from || b->rows_from > l->rows_to) {
+      last->other = hold(before.object);
+      last = b;
+      ++count;
+    }
+  }
+  Py_XDECREF(next);
+  return made.release();
   END_HANDLE_TH_ERRORS
 }
 
@@ -557,11 +569,12 @@ PyObject *run_layer(Layer *l, PyObject *module_dict, PyObject *inputs, const Epi
   const at::Tensor *x = in == nullptr ? nullptr : tensor_of(look(in, s__features));
   if (x == nullptr || x->dim() != 2) return none();
   const int64_t S = x->size(0);
-  if (S < l->rows_from || S > l->rows_to) {
+  while (S < l->rows_from || S > l->rows_to) {
     if (l->other == nullptr) return none();
     l = reinterpret_cast<Layer *>(l->other);
-    if (S < l->rows_from || S > l->rows_to) return none();
   }
+  Py_INCREF(l);
+  const Ref keep(reinterpret_cast<PyObject *>(l));
   if ((l->kind == kPointwise || l->kind == kPieces) && !stands_in(l, look(in, s__features), ep)) return none();
   // the module: same parameters, same settings, not being tuned
   PyObject *parameters = look(module_dict, s__parameters);
@@ -783,8 +796,6 @@ PyObject *py_run(PyObject *, PyObject *const *args, Py_ssize_t count) {
     if (PyErr_Occurred()) return nullptr;
   }
   if (ep.activation < 0) return none();
-  Py_INCREF(l);
-  const Ref keep(reinterpret_cast<PyObject *>(l));
   return run_layer(l, d, args[1], ep);
   END_HANDLE_TH_ERRORS
 }
@@ -912,8 +923,6 @@ PyObject *py_conv_norm_act(PyObject *, PyObject *const *args, Py_ssize_t count) 
     }
   }
   ep.residual = args[4];
-  Py_INCREF(l);
-  const Ref keep(reinterpret_cast<PyObject *>(l));
   return run_layer(l, d, args[3], ep);
   END_HANDLE_TH_ERRORS
 }

@@ -1147,8 +1147,8 @@ class SparseConv(Module):
     def _keep_fast(self, made, rows, inputs, features, coordinates, stride, batch_dims):
         """Leaves what this call worked out for the extension module: the module's
         side of it in ``_fast``, the map's side in the cache's ``_fast_maps``.
-        Where the kind depends on the size (``rows``), the Layer of the other kind
-        stays with the new one: each cloud gets the kernel that a fresh cache
+        Where the kind depends on the size (``rows``), the Layers for other sizes
+        stay with the new one: each cloud gets the kernel that a fresh cache
         would give it, whatever came before."""
         name, weights, packed, pointers, owners, index_code = made[:6]
         tiles, flag = made[6:] if len(made) > 6 else (None, False)

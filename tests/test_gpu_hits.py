@@ -138,3 +138,39 @@ def test_layers_of_less_than_four_channels(kernel, cin, cout):
                 bound = (cin * kernel ** 3 + 16) * 2.0 ** -24 * size
                 assert bool(((out.double() - wanted - conv.bias.double()).abs() <= bound).all())
         assert len(cache._kernel_maps_cache) == 0 and conv._fast is not None
+
+
+@pytest.mark.parametrize("dtype, kernel, cin, cout, sizes", [
+    (torch.float32, 3, 32, 64, (10000, 60000, 260000)),      # hits, product rows, hits again
+    (torch.float16, 5, 64, 256, (1000, 101000)),             # product rows, one kernel
+    (torch.float32, 3, 64, 64, (2000, 40000))])              # hits, product rows
+def test_layers_for_every_size_are_kept(dtype, kernel, cin, cout, sizes):
+    """A layer that has seen clouds of every range of rows goes through no Python code for any of them, in any
+    order, also after its weights have changed and been seen by all."""
+    gen = torch.Generator(device=DEVICE).manual_seed(11)
+    torch.manual_seed(1)
+    conv = minuet.nn.SparseConv3d(cin, cout, kernel, dtype=dtype, device=DEVICE)
+    inputs = []
+    for rows in sizes:
+        cells = torch.randperm(1 << 21, generator=gen, device=DEVICE)[:rows]
+        coordinates = torch.stack([cells >> 14, (cells >> 7) & 127, cells & 127], 1).int()
+        coordinates = coordinates[F.build_sorted_index(coordinates)]
+        x = minuet.SparseTensor(torch.randn(rows, cin, generator=gen, device=DEVICE).to(dtype), coordinates)
+        inputs.append((x, minuet.nn.KernelMapCache(3, torch.int32, DEVICE)))
+    came = []
+    keep = conv._keep_fast
+    conv._keep_fast = lambda *args: (came.append(args[0][0]), keep(*args))
+    with torch.no_grad():
+        for turn in range(2):
+            wanted = []
+            for x, cache in inputs:
+                minuet.set_kernel_map_cache(conv, cache)
+                wanted.append(conv(x).F)
+            assert len(came) == len(sizes)
+            for at in (*range(len(sizes)), *range(len(sizes) - 1, -1, -1), 0, len(sizes) - 1):
+                x, cache = inputs[at]
+                minuet.set_kernel_map_cache(conv, cache)
+                assert torch.equal(conv(x).F, wanted[at])
+            assert len(came) == len(sizes)
+            came.clear()
+            conv.kernel.mul_(-0.5)
