@@ -646,6 +646,10 @@ class SparseConv(Module):
         self._routes = dict()
         self._trivial = None
 
+    def __setstate__(self, state):
+        super().__setstate__(state)
+        self._routes = dict()                       # (those of another version may be of another form)
+
     @property
     def _allow_shortcut_matmul(self) -> bool:
         return (all(x == 1 for x in self.dilation) and all(x == 1 for x in self.stride)
@@ -888,25 +892,28 @@ class SparseConv(Module):
         if dataflow == "implicit":
             return True
         shape = (self.kernel.shape[0], self.in_channels + pad, self.out_channels, features.dtype)
+        form = F.layer_form(self.stride, self.dilation, self.transposed)
         # (a copy of the rows, which every call makes, is more than streaming saves where it is made by the
         # library: 100 -> 64 channels over 2 000 voxels 14.6 us in three kernels and 26.7)
-        return (F.prefers_implicit(*shape) or (pad == 0 and F.prefers_streamed(*shape))
-                or F.implicit_rows_from(*shape) <= features.shape[0])
+        return (F.prefers_implicit(*shape, form) or (pad == 0 and F.prefers_streamed(*shape))
+                or F.implicit_rows_from(*shape, form) <= features.shape[0])
 
     def _lines(self, dtype: torch.dtype, channels: int):
         """Of a layer whose rows have so many channels, once they are padded: in
         fp32 the rows up to which, from which on and up to which at all the
-        kernel of hits takes it, in 16 bits the fewest over which ``auto`` takes the
-        single-kernel form (0: their number does not matter).  Kept with the routes."""
+        kernel of hits takes it, in 16 bits those up to which and from which on ``auto``
+        takes the single-kernel form (-1 and 0: their number does not matter).  Kept with
+        the routes."""
         lines = self._routes.get(("lines", dtype))
         if lines is None:
-            layer = (self.kernel.shape[0], channels, self.out_channels, dtype)
+            layer = (self.kernel.shape[0], channels, self.out_channels, dtype,
+                     F.layer_form(self.stride, self.dilation, self.transposed))
             far = F.implicit_rows_limit(channels, dtype)
             if dtype == torch.float32:
                 lines = (F.hits_rows_limit(*layer), F.hits_rows_from(*layer), far)
             else:
                 begin = F.implicit_rows_from(*layer)
-                lines = begin if begin <= far else 0
+                lines = (F.implicit_rows_few(*layer), begin) if begin <= far else (-1, 0)
             self._routes[("lines", dtype)] = lines
         return lines
 
@@ -1052,12 +1059,12 @@ class SparseConv(Module):
                     rows = (0, most) if count <= most else (again, far)
                 else:
                     rows = (most + 1, again - 1) if count < again else (far + 1, _MOST_ROWS)
-            begin = 0                               # (rows from which the single-kernel form may be taken)
+            few, begin = -1, 0                      # (rows up to and from which the single-kernel form may be taken)
             if hits is None and dataflow == "auto" and sources.dtype != torch.float32:
-                begin = self._lines(sources.dtype, -(-self.in_channels // 8) * 8)
+                few, begin = self._lines(sources.dtype, -(-self.in_channels // 8) * 8)
                 if self.out_channels > 128 and self.in_channels % 8 and self.in_channels <= 32 and self._records():
-                    begin = -(-_PADDED_VALUES // self.out_channels)
-            small = sources.shape[0] < begin
+                    few, begin = -1, max(begin, -(-_PADDED_VALUES // self.out_channels))
+            small = few < sources.shape[0] < begin
             route_key = (sources.dtype, sources.is_cuda, dataflow, hits, small)
             route = self._routes.get(route_key)
             if route is None:
@@ -1068,9 +1075,9 @@ class SparseConv(Module):
                 implicit = self._takes_implicit(sources, pad) if hits is None else hits
                 implicit = implicit and not grouped
                 single = tiled = False
-                most, few = None, ()
+                most = None
                 if small:
-                    pad, implicit, few = 0, False, (0, begin - 1)
+                    pad, implicit = 0, False
                 if implicit and not hits:
                     single = self._has_single_sources(sources, pad)
                     tiled = not single and F.prefers_streamed(volume, self.in_channels + pad, self.out_channels,
@@ -1082,11 +1089,12 @@ class SparseConv(Module):
                     if tiled:
                         most = min(most, F.streamed_rows_limit(volume, self.in_channels, self.out_channels,
                                                                sources.dtype))
-                route = self._routes[route_key] = (pad, implicit, grouped, most, single, tiled, few)
-            pad, implicit, grouped, most, single, tiled, few = route
-            rows = few or rows
+                route = self._routes[route_key] = (pad, implicit, grouped, most, single, tiled)
+            pad, implicit, grouped, most, single, tiled = route
+            if small:
+                rows = (few + 1, begin - 1)
             if most is not None:
-                rows = (begin, most)
+                rows = (begin, most) if sources.shape[0] >= begin else (0, few)
                 if sources.shape[0] > most:
                     pad, implicit, grouped = 0, False, self._takes_offset_groups(sources, streamed=False)
                     rows = (most + 1, _MOST_ROWS)

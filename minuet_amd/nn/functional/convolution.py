@@ -10,7 +10,8 @@ from ..kernel_map import KernelMap
 __all__ = ["cuda_time_gather", "cuda_time_scatter", "sparse_convolution_forward",
            "cuda_time_gemm", "set_gemm_parallel_level", "Epilogue", "pack_weights",
            "prefers_implicit", "prefers_streamed", "prefers_hits", "implicit_rows_limit", "hits_rows_limit",
-           "hits_rows_from", "streamed_rows_limit", "implicit_rows_from",
+           "hits_rows_from", "streamed_rows_limit", "implicit_rows_from", "implicit_rows_few", "layer_form",
+           "prefers_implicit_over",
            "pieces_rows_limit", "channel_pieces"]
 
 pack_weights = _C.pack_weights
@@ -29,8 +30,19 @@ def set_gemm_parallel_level(level: int):
     GEMM_PARALLEL_LEVEL = level
 
 
+def layer_form(stride, dilation, transposed: bool) -> str:
+    """What the rules below ask of a layer beside its shape, because it decides how
+    many of its offsets have a source: ``"plain"`` (stride 1), ``"dilated"`` (stride 1),
+    ``"strided"`` and ``"transposed"`` (stride 2 at most, no dilation), or ``"other"``."""
+    if all(s == 1 for s in stride):
+        return "plain" if all(d == 1 for d in dilation) else "dilated"
+    if any(s > 2 for s in stride) or any(d != 1 for d in dilation):
+        return "other"
+    return "transposed" if transposed else "strided"
+
+
 def prefers_implicit(num_offsets: int, num_source_features: int, num_target_features: int,
-                     dtype: torch.dtype) -> bool:
+                     dtype: torch.dtype, form: str = "plain") -> bool:
     """Whether ``dataflow="auto"`` takes the single-kernel form for a layer of
     this shape: it must fit that kernel, and it must be the faster one, which
     measurements say it is for 16-bit features with source rows of up to 128
@@ -38,14 +50,17 @@ def prefers_implicit(num_offsets: int, num_source_features: int, num_target_feat
     to 64 output channels under kernels of more than 8 offsets (beyond that its
     matrix work on empty (offset, target) pairs outweighs the buffer traffic it
     saves).  With rows of up to 64 bytes there is so little of that work that up to
-    36 offsets, and 5x5x5, take any number of output channels: a second 128 of them
+    36 offsets take any number of output channels, and 5x5x5 over few rows and over
+    many (``implicit_rows_few``, ``implicit_rows_from``): a second 128 of them
     cost as much as the first, the three kernels' product rows more (us, three
     kernels and here: 3x3x3 24 -> 256 over 200 000 voxels of a LiDAR scan 326 / 66, 32
     -> 160 over 5 000 of a room 19 / 10, over 1 000 15 / 11; 2x2x2 16 -> 160 over 50 000
-    28 / 16; 5x5x5 32 -> 256 over 200 000 805 / 157, over 30 000 of a room 72 / 69, 32 ->
-    160 there 63 / 64).  Not kernels in between, where a target has a smaller share of
+    28 / 16; over 290 layers of 8 to 36 offsets, strided and transposed ones among them,
+    1 000 to 300 000 voxels of three kinds of scene, 0.76 times as long at most).  Not
+    kernels in between, where a target has a smaller share of
     its offsets (4x4x4 32 -> 160 over 50 000 of a room 53 / 64), nor larger ones
-    (6x6x6 32 -> 256 over 50 000 155 / 200).  An fp32 layer of more than one offset goes by its rows instead
+    (6x6x6 32 -> 256 over 50 000 155 / 200), nor strides of 3 and more (3x3x3 32 -> 512
+    transposed 1.2 to 1.3 times as long over 30 000).  An fp32 layer of more than one offset goes by its rows instead
     (``hits_rows_limit``); without rows to go by, this says yes to the narrow
     ones with strided 2^D kernels, whose (offset, target) pairs are mostly hits."""
     if not _C.implicit_forward_supported(num_source_features, num_target_features, dtype, num_offsets):
@@ -53,7 +68,8 @@ def prefers_implicit(num_offsets: int, num_source_features: int, num_target_feat
     if dtype != torch.float32:
         row_bytes = num_source_features * dtype.itemsize
         if row_bytes <= 128:
-            return num_target_features <= 128 or (row_bytes <= 64 and (num_offsets <= 36 or num_offsets == 125))
+            return num_target_features <= 128 or (row_bytes <= 64 and form != "other"
+                                                  and (num_offsets <= 36 or num_offsets == 125))
         return row_bytes <= 256 and num_target_features <= 64 and num_offsets > 8
     return num_offsets <= 8 and num_source_features * num_target_features <= 1024
 
@@ -105,31 +121,57 @@ def streamed_rows_limit(num_offsets: int, num_source_features: int, num_target_f
 
 
 def implicit_rows_from(num_offsets: int, num_source_features: int, num_target_features: int,
-                       dtype: torch.dtype) -> int:
-    """The fewest source rows over which ``dataflow="auto"`` takes the single-kernel
-    form for a 16-bit layer that is not in its shape the faster one there
-    (``prefers_implicit``, ``prefers_streamed``); one more than
-    ``implicit_rows_limit``: over none.
+                       dtype: torch.dtype, form: str = "plain") -> int:
+    """The fewest source rows past ``implicit_rows_few`` over which ``dataflow="auto"``
+    takes the single-kernel form for a 16-bit layer that is not in its shape the
+    faster one over any number of them (``prefers_implicit``, ``prefers_streamed``); one
+    more than ``implicit_rows_limit``: over none.
 
-    5x5x5 layers whose product rows outgrow the caches: rows of 80 to 128 bytes and
+    5x5x5 layers whose product rows outgrow the caches: rows of up to 64 bytes and
+    more than 128 output channels; rows of 80 to 128 bytes and
     more than 128 output channels, of which the second 128 cost as much as the
     first, so half of them more than a whole, and rows of up to 256 bytes and 97 to
     128 output channels.  us, three kernels and here, the slowest and the fastest
-    kind of scene: 64 -> 256 over 100 000 voxels of a room 312 / 239, of a LiDAR scan 333
+    kind of scene: 32 -> 256 over 100 000 voxels 0.3 times as long of a LiDAR scan and
+    0.4 of a room (over 50 000 1.5 and 1.2); 64 -> 256 over 100 000 of a room 312 / 239, of a LiDAR scan 333
     / 178 (over 30 000 of a room 72 / 84), 64 -> 160 over 150 000 333 / 278 and 447 / 205
     (over 100 000 of a room 219 / 234), 128 -> 128 over 150 000 282 / 264 and 369 / 185
     (over 100 000 of a room 172 / 215).  Not 128 -> 160 (250 000 of a room 570 / 666) nor
-    128 -> 256 (481 / 496 over 150 000)."""
+    128 -> 256 (481 / 496 over 150 000).  Strided layers have targets of fewer sources: 64 -> 160
+    over 150 000 takes 0.75 to 1.13 times as long as in three kernels, 128 -> 128 over 250 000
+    0.5 to 1.12, with a dilation of 2 0.4 to 1.06 and 0.4 to 1.15, so these two are for
+    plain and transposed layers (0.35 to 0.6); 64 -> 256 strided 0.6 to 0.84, dilated 0.5 to 0.92."""
     far = implicit_rows_limit(num_source_features, dtype) + 1
-    if (dtype == torch.float32 or num_offsets != 125
+    if (dtype == torch.float32 or num_offsets != 125 or form == "other"
             or not _C.implicit_forward_supported(num_source_features, num_target_features, dtype, num_offsets)):
         return far
     row_bytes = num_source_features * dtype.itemsize
-    if 64 < row_bytes <= 128 and num_target_features > 128:
-        return min(far, 100_000 if (num_target_features - 1) % 128 >= 64 else 150_000)
-    if 128 < row_bytes <= 256 and 96 < num_target_features <= 128:
+    dense = form in ("plain", "transposed")
+    if row_bytes <= 128 and num_target_features > 128 and (row_bytes <= 64 or (num_target_features - 1) % 128 >= 64):
+        return min(far, 100_000)
+    if dense and ((row_bytes <= 128 and num_target_features > 128)
+                  or (128 < row_bytes <= 256 and 96 < num_target_features <= 128)):
         return min(far, 150_000)
     return far
+
+
+def implicit_rows_few(num_offsets: int, num_source_features: int, num_target_features: int,
+                      dtype: torch.dtype, form: str = "plain") -> int:
+    """The most source rows short of ``implicit_rows_from`` over which ``auto`` takes
+    the single-kernel form for the layer spoken of there (-1: over none).
+
+    5x5x5, rows of up to 64 bytes, more than 128 output channels: a workgroup walks
+    all 125 offsets whatever the number of rows, which costs less than two more launches
+    while the chip is not full, and more from then on until product rows outgrow the
+    caches.  Times as long as in three kernels, LiDAR / room / object: 32 -> 256 over 3 000
+    0.86 / 0.51 / 0.46, 6 000 0.88 / 0.57 / 0.50, 12 000 1.07 / 0.83 / 0.71, 20 000 1.53 / 1.06 /
+    0.80, 50 000 1.54 / 1.21 / 0.51; 32 -> 512 over 6 000 1.09 / 0.74 / 0.61; 32 -> 256 with a
+    dilation of 2 over 12 000 1.12 / 0.92 / 0.94, transposed over 9 000 1.22 / 1.02 / 1.05,
+    strided over 12 000 0.93 / 0.70 / 0.52."""
+    if (num_offsets != 125 or dtype == torch.float32 or num_target_features <= 128
+            or not prefers_implicit(num_offsets, num_source_features, num_target_features, dtype, form)):
+        return -1
+    return (20_000 if form in ("plain", "strided") else 12_000) // -(-num_target_features // 128)
 
 
 def implicit_rows_limit(num_source_features: int, dtype: torch.dtype) -> int:
@@ -139,8 +181,17 @@ def implicit_rows_limit(num_source_features: int, dtype: torch.dtype) -> int:
     return (_C.IMPLICIT_MAX_SOURCE_BYTES - 1) // (num_source_features * dtype.itemsize)
 
 
+def prefers_implicit_over(num_offsets: int, num_source_features: int, num_target_features: int,
+                          dtype: torch.dtype, num_rows: int, form: str = "plain") -> bool:
+    """``prefers_implicit`` over ``num_rows`` source rows."""
+    layer = (num_offsets, num_source_features, num_target_features, dtype, form)
+    most, begin = implicit_rows_limit(num_source_features, dtype), implicit_rows_from(*layer)
+    return (prefers_implicit(*layer) and num_rows <= most
+            and not (begin <= most and implicit_rows_few(*layer) < num_rows < begin))
+
+
 def hits_rows_limit(num_offsets: int, num_source_features: int, num_target_features: int,
-                    dtype: torch.dtype) -> int:
+                    dtype: torch.dtype, form: str = "plain") -> int:
     """The most source rows over which ``dataflow="auto"`` takes the single-kernel
     form for an fp32 layer of more than one offset (-1: over none).
 
@@ -161,12 +212,17 @@ def hits_rows_limit(num_offsets: int, num_source_features: int, num_target_featu
     63 / 76), or about even (2x2x2 over 300 000 31.5 / 31.7 and, transposed, 36.9
     / 33.6).
 
-    So it is for at most 16 input channels under 3x3x3 to 5x5x5, where products
+    So it is for at most 16 input channels under 27 to 125 offsets, where products
     cost next to nothing and product rows as much as ever (0.4 to 0.96 times as
     long over 120 layers of 64 to 512 output channels and 3 000 to 300 000 voxels;
     one of 1.02): 3x3x3 16 -> 96 over 40 000 voxels of a room 26 / 35, over 200 000
     of a LiDAR scan 113 / 236, 16 -> 256 over 100 000 of objects 148 / 311; 5x5x5 16 ->
-    256 over 20 000 83 / 92.
+    256 over 20 000 83 / 92.  That holds for odd kernel sizes (3x3x5, 3x5x5, 7x7x1, 3x3x9
+    and 11x11x1 0.29 to 1.08 times as long, LiDAR scans of 30 000 to 60 000 voxels last), dilated
+    (0.4 to 1.03) and strided (0.4 to 1.05), and for transposed 3x3x3 layers (0.6 to 1.07;
+    5x5x5 0.57 to 1.13); not for even ones, where a LiDAR scan of 12 000 to 130 000 voxels takes
+    1.1 to 1.3 times as long (3x3x4, 4x4x4, 5x5x4), nor for strides of 3 and more (3x3x3
+    transposed 0.7 to 1.4).
 
     Never more than ``implicit_rows_limit``."""
     if (dtype != torch.float32 or num_offsets <= 1
@@ -174,13 +230,14 @@ def hits_rows_limit(num_offsets: int, num_source_features: int, num_target_featu
         return -1
     most = implicit_rows_limit(num_source_features, dtype)
     work = num_source_features * num_target_features
-    if work <= 1024 or (num_source_features <= 16 and 27 <= num_offsets <= 125):
+    if work <= 1024 or (num_source_features <= 16 and 27 <= num_offsets <= 125 and num_offsets % 2 == 1
+                        and (form in ("plain", "dilated", "strided") or (form == "transposed" and num_offsets == 27))):
         return most
     return min(most, min(110_000_000, 2_100_000_000 // num_offsets) // work)
 
 
 def hits_rows_from(num_offsets: int, num_source_features: int, num_target_features: int,
-                   dtype: torch.dtype) -> int:
+                   dtype: torch.dtype, form: str = "plain") -> int:
     """The fewest source rows past ``hits_rows_limit`` over which ``dataflow="auto"``
     takes the single-kernel form again (one more than ``implicit_rows_limit``:
     over none).
@@ -194,10 +251,17 @@ def hits_rows_from(num_offsets: int, num_source_features: int, num_target_featur
     over 150 000 of a room 207 / 242, over 100 000 153 / 147, 32 -> 64 of a LiDAR scan
     177 / 297.  (64 input channels: over 300 000 of a LiDAR scan 259 / 386, of a room
     171 / 181, but 64 -> 48 164 / 156, and with the sums that ``compact_forward``
-    keeps for these layers 8 % more.)"""
+    keeps for these layers 8 % more.)  Times as long, 32 and 48 -> 64 to 256 over 250 000
+    voxels: 3x3x5 0.66 to 0.95, 3x5x5 0.58 to 0.96, 7x7x1 0.48 to 0.92, 3x3x9 0.67 to 1.02; 5x5x5 over
+    130 000 0.67 to 0.98.  Kernels of even sizes are slower there (3x3x4, 4x4x4, 5x5x4 0.74 to 1.29
+    times) unless they have at most 16 input channels (0.55 to 0.91; over 130 000 up to 1.12).
+    Dilated, strided and transposed layers never come back to it: targets that have fewer sources
+    leave the 16 rows of a product emptier (3x3x3 with a dilation of 3 1.0 to 1.17 times as
+    long over 250 000 voxels of objects, strided 0.94 to 1.06, 5x5x5 48 -> 256 1.11)."""
     far = implicit_rows_limit(num_source_features, dtype) + 1
-    if (hits_rows_limit(num_offsets, num_source_features, num_target_features, dtype) < 0
-            or num_source_features > 48 or not 27 <= num_offsets <= 125):
+    if (hits_rows_limit(num_offsets, num_source_features, num_target_features, dtype, form) < 0
+            or form != "plain" or not 27 <= num_offsets <= 125
+            or num_source_features > (48 if num_offsets % 2 == 1 else 16)):
         return far
     return min(far, 130_000 if num_offsets == 125 else 250_000)
 
@@ -230,10 +294,10 @@ def pieces_rows_limit(num_source_features: int, num_target_features: int, dtype:
 
 
 def prefers_hits(num_offsets: int, num_source_features: int, num_target_features: int, dtype: torch.dtype,
-                 num_rows: int) -> bool:
+                 num_rows: int, form: str = "plain") -> bool:
     """Whether ``dataflow="auto"`` takes the single-kernel form for an fp32 layer
     over ``num_rows`` source rows (``hits_rows_limit``, ``hits_rows_from``)."""
-    layer = (num_offsets, num_source_features, num_target_features, dtype)
+    layer = (num_offsets, num_source_features, num_target_features, dtype, form)
     return num_rows <= hits_rows_limit(*layer) or (
         hits_rows_from(*layer) <= num_rows <= implicit_rows_limit(num_source_features, dtype))
 
@@ -330,11 +394,12 @@ def sparse_convolution_forward(sources: torch.Tensor, weights: torch.Tensor,
     if dataflow == "implicit" and dense is None:
         raise ValueError("the implicit dataflow needs a KernelMap with its dense map")
     if dense is not None and dataflow in ("auto", "implicit"):
-        shape = (weights.shape[0], weights.shape[1], weights.shape[2], weights.dtype)
-        if dataflow == "implicit" or (prefers_hits(*shape, sources.shape[0])
+        rows, shape = sources.shape[0], (weights.shape[0], weights.shape[1], weights.shape[2], weights.dtype)
+        # (what a map says of the layer's stride; a dilation it does not)
+        form = "plain" if rows == dense.shape[1] else "strided" if rows > dense.shape[1] else "transposed"
+        if dataflow == "implicit" or (prefers_hits(*shape, rows, form)
                                       if weights.dtype == torch.float32 and weights.shape[0] > 1
-                                      else prefers_implicit(*shape)
-                                      and sources.shape[0] <= implicit_rows_limit(weights.shape[1], weights.dtype)):
+                                      else prefers_implicit_over(*shape, rows, form)):
             return _C.sparse_convolution_forward_implicit(sources, weights, dense, epilogue=epilogue,
                                                           packed_weights=packed_weights)
     if dataflow == "list_driven":

@@ -309,3 +309,39 @@ def test_batch_norm_affine_is_the_fp32_expression(dtype, affine):
         for got, wanted in zip(minuet.nn.fused.batch_norm_affine(norm), (scale, shift)):
             assert got.dtype == torch.float32 and torch.equal(got, wanted)
     assert all(torch.equal(a, b) for a, b in zip(before, norm.state_dict().values()))
+
+
+def test_rules_follow_the_form_of_a_layer():
+    """Both sides of each line that a stride, a dilation or the kernel's sizes move."""
+    F, half, single = minuet.nn.functional, torch.float16, torch.float32
+    form = F.layer_form
+    assert form((1, 1), (1, 1), False) == form((1, 1), (1, 1), True) == "plain" and form((1,), (2,), False) == "dilated"
+    assert form((2, 1), (1, 1), False) == "strided" and form((2, 2), (1, 1), True) == "transposed"
+    assert form((3,), (1,), False) == form((2,), (2,), True) == "other"
+    # 16 bits, more than 128 output channels: up to 36 offsets over any rows, 5x5x5 over few and over many
+    assert all(F.prefers_implicit_over(27, 32, 256, half, rows) for rows in (100, 30000, 10 ** 6))
+    assert not F.prefers_implicit(27, 32, 256, half, "other") and F.prefers_implicit(27, 32, 128, half, "other")
+    assert not F.prefers_implicit(125, 32, 256, half, "other")
+    for cout, kind, few in ((256, "plain", 10000), (512, "plain", 5000), (160, "strided", 10000),
+                            (256, "dilated", 6000), (132, "transposed", 6000)):
+        assert F.implicit_rows_few(125, 32, cout, half, kind) == few
+        took = [rows for rows in (few, few + 1, 99999, 100000) if F.prefers_implicit_over(125, 32, cout, half, rows, kind)]
+        assert took == [few, 100000]
+    never = F.implicit_rows_limit(64, half) + 1
+    assert [F.implicit_rows_from(125, 64, 160, half, kind) for kind in ("plain", "strided", "dilated", "transposed")] == [
+        150000, never, never, 150000]
+    assert [F.implicit_rows_from(125, 64, 256, half, kind) for kind in ("strided", "dilated", "other")] == [100000, 100000, never]
+    # fp32: few input channels under odd kernels, and plain layers that come back
+    for offsets, kind, all_rows in ((27, "plain", True), (75, "dilated", True), (125, "strided", True), (27, "transposed", True),
+                                    (125, "transposed", False), (64, "plain", False), (27, "other", False)):
+        assert F.prefers_hits(offsets, 16, 256, single, 60000, kind) == all_rows
+    assert F.prefers_hits(64, 16, 256, single, 250000) and not F.prefers_hits(64, 16, 256, single, 249999)
+    assert not F.prefers_hits(64, 32, 256, single, 300000) and F.prefers_hits(75, 32, 256, single, 300000)
+    assert not any(F.prefers_hits(27, 32, 256, single, 10 ** 6, kind) for kind in ("dilated", "strided", "transposed", "other"))
+
+
+def test_saved_layers_work_out_their_routes_anew():
+    import pickle
+    conv = minuet.nn.SparseConv(3, 4, 8, 3)
+    conv._routes["lines", torch.float16] = 7          # as another version may have kept them
+    assert pickle.loads(pickle.dumps(conv))._routes == {} and conv._routes

@@ -295,3 +295,35 @@ def test_layers_that_record_gradients_pad_where_it_pays(dtype, cin, cout, rows, 
             assert len(cache._kernel_maps_cache) == (tables if recorded else 0)
         for other in results[1:]:
             assert float((other - results[0]).abs().max()) <= bound * 27 * float(results[0].abs().max())
+
+
+@pytest.mark.parametrize("kind, dtype, kernel, cin, cout, tables", [
+    ("plain", torch.float16, 5, 32, 160, {700: 0, 11000: 1, 100000: 0}), ("strided", torch.float16, 5, 64, 160, {150000: 1}),
+    ("strided", torch.float16, 5, 32, 160, {11000: 1, 100000: 0}), ("dilated", torch.float16, 5, 128, 128, {150000: 1}),
+    ("plain", torch.float32, 4, 16, 80, {700: 0, 50000: 1, 250000: 0}), ("strided", torch.float32, 3, 32, 64, {260000: 1}),
+    ("dilated", torch.float32, 3, 16, 96, {50000: 0})])
+def test_rules_follow_the_form_of_a_layer(kind, dtype, kernel, cin, cout, tables):
+    """What a layer runs on each side of the lines, and that it is the values of the forced three kernels."""
+    gen = torch.Generator(device=DEVICE).manual_seed(cin + kernel)
+    torch.manual_seed(2)
+    conv = minuet.nn.SparseConv3d(cin, cout, kernel, stride=2 if kind == "strided" else 1,
+                                  dilation=2 if kind == "dilated" else 1, dtype=dtype, device=DEVICE)
+    for turn in range(2):
+        for rows, built in tables.items():
+            cells = torch.randperm(1 << 21, generator=gen, device=DEVICE)[:rows]
+            coordinates = torch.stack([cells >> 14, (cells >> 7) & 127, cells & 127], 1).int()
+            coordinates = coordinates[F.build_sorted_index(coordinates)]
+            x = minuet.SparseTensor(torch.randn(rows, cin, generator=gen, device=DEVICE).to(dtype), coordinates)
+            results = []
+            for flow in ("auto", "gather_gemm_scatter"):
+                conv._tunable_config["dataflow"] = flow
+                cache = minuet.nn.KernelMapCache(3, torch.int32, DEVICE)
+                minuet.set_kernel_map_cache(conv, cache)
+                with torch.no_grad():
+                    results.append(conv(x).F.double())
+                    assert torch.equal(conv(x).F.double(), results[-1])
+                assert len(cache._kernel_maps_cache) == (built if flow == "auto" else 1)
+            # fp16: product rows and both results are rounded to nearest, in the 2-norm 3 x 2^-11 / sqrt(3) = 8.5e-4;
+            # fp32: two orders of 27 x 64 additions at most, each about sqrt(27 x 64) x 2^-24 / sqrt(3) = 1.4e-6
+            bound = {torch.float32: 3e-6, torch.float16: 1e-3}[dtype]
+            assert float((results[0] - results[1]).norm() / results[1].norm()) <= bound
