@@ -591,12 +591,14 @@ extern "C" int mnt_gather_rows(const void *const *sources, const int64_t *source
                                void *stream_) {
   return guarded([&] {
     hipStream_t stream = static_cast<hipStream_t>(stream_);
-    MNT_CHECK(row_bytes >= 1, "bad argument");
+    MNT_CHECK(sources != nullptr && source_rows != nullptr && row_bytes >= 1, "bad argument");
+    MNT_CHECK(num_sources >= 1 && num_sources <= kGatherSources, "between 1 and %d tensors but found %d",
+              kGatherSources, num_sources);
     int_size(index_dtype);
+    if (n == 0) return;                            // (of however many rows)
     int64_t rows = 0;
     uintptr_t align = 0;
     const GatherSources src = gather_sources(sources, source_rows, num_sources, rows, align);
-    if (n == 0) return;
     MNT_CHECK(n <= rows, "more rows asked for than there are");
     gather_rows(src, align, row_bytes, order, index_dtype, n, out, stream);
   });

@@ -128,3 +128,17 @@ def test_one_caller_thread_per_stream():
         assert done["status"] == 0
     finally:
         _C.stream_release(None)
+
+
+def test_no_rows_are_gathered_from_any_number():
+    """Nothing is asked of tensors of which no row is wanted, however many they have between them."""
+    lib = _C.load_library()
+    tensors, sizes = (ctypes.c_void_p * 2)(16, 16), (ctypes.c_int64 * 2)(2 ** 31, 5)
+
+    def gather(count, n, row_bytes=8):
+        return lib.mnt_gather_rows(ctypes.addressof(tensors), ctypes.addressof(sizes), count, row_bytes, None, 0, n,
+                                   None, None)
+
+    assert gather(2, 0) == 0
+    assert gather(0, 0) != 0 and gather(65, 0) != 0 and gather(2, 0, 0) != 0 and gather(2, 1) != 0
+    lib.mnt_reset_error()
