@@ -62,8 +62,9 @@ bool small_map_takes(int64_t n, int num_offsets);
 // The int32 permutation, the sorted rows and the pair lists of a cloud mapped onto
 // itself, in one launch; `words` and `sequence` are Arena::words() and a number of that
 // arena.  For the host: order, nothing and sizes in plan_host
-// (num_offsets words each), the extremes and the verdict (not 0: nothing was
-// written but it) in chain_host, then the flag.
+// (num_offsets words each), the extremes and the verdict in chain_host, then the
+// flag.  Verdict 1 (crowded, or key and row index do not fit 64 bits): nothing was
+// written but it; 3 (equal rows): it, permutation and sorted rows, no list.
 void enqueue_small_map(const void *coords, int64_t n, int ndim, int coord_dtype, const int64_t *offsets_host,
                        int num_offsets, bool allow_halves, int reorder, int32_t *indices_out, void *sorted_out,
                        int32_t *in_idx, int32_t *out_idx, int32_t *sizes, int32_t *order,

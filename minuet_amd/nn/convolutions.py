@@ -1046,8 +1046,9 @@ class SparseConv(Module):
             hits = None                             # (None: the rows do not matter)
             if (sources.dtype == torch.float32 and dataflow == "auto" and volume > 1 and sources.is_cuda
                     and self.kernel.dtype == torch.float32):
-                # (rows of one to three values are padded to four: error against 64 bits 1.00 to 1.04 times
-                # the three kernels', us there and here 3 -> 64 over 20 000 26.1 / 15.2, over 200 000 134 / 69,
+                # (rows of one to three values are padded to four: error against 64 bits 0.8 to 1.02 times
+                # the three kernels', least of one value and most of three; us there and here 3 -> 64 over
+                # 20 000 26.1 / 15.2, over 200 000 134 / 69,
                 # 3 -> 16 over 1 000 18.5 / 15.0; of five to eight values the error is up to 1.26 times)
                 channels = max(self.in_channels, 4)
                 most, again, far = self._lines(sources.dtype, channels)

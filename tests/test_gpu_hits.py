@@ -140,6 +140,55 @@ def test_layers_of_less_than_four_channels(kernel, cin, cout):
         assert len(cache._kernel_maps_cache) == 0 and conv._fast is not None
 
 
+@pytest.mark.parametrize("kernel, cin, cout, rows", [(3, 1, 32, 20000), (3, 2, 64, 20000), (3, 3, 64, 20000), (2, 3, 16, 20000),
+                                                     (5, 3, 32, 6000), (3, 3, 256, 50000)])
+def test_padded_layers_are_as_exact_as_three_kernels(kernel, cin, cout, rows):
+    """Against 64 bits.  Over 99 layers of three kinds of scene the errors are 0.81 to 1.02 times as large; of the
+    320 000 values and more that there are here the norm of the error scatters by 1 / sqrt(2 x 320 000) < 0.2 %."""
+    gen = torch.Generator(device=DEVICE).manual_seed(rows + cin)
+    torch.manual_seed(cout)
+    conv = minuet.nn.SparseConv3d(cin, cout, kernel, dtype=torch.float32, device=DEVICE)
+    cells = torch.randperm(1 << 18, generator=gen, device=DEVICE)[:rows]
+    coordinates = torch.stack([cells >> 12, (cells >> 6) & 63, cells & 63], 1).int()
+    coordinates = coordinates[F.build_sorted_index(coordinates)]
+    x = minuet.SparseTensor(torch.randn(rows, cin, generator=gen, device=DEVICE), coordinates)
+    errors = []
+    for flow in ("auto", "gather_gemm_scatter"):
+        conv._tunable_config["dataflow"] = flow
+        cache = minuet.nn.KernelMapCache(3, torch.int32, DEVICE)
+        minuet.set_kernel_map_cache(conv, cache)
+        with torch.no_grad():
+            out = conv(x).F
+        assert len(cache._kernel_maps_cache) == (flow != "auto")
+        dense, _ = _C.kernel_map_dense(coordinates, coordinates, cache._kernel_offsets((1, 1, 1), (kernel,) * 3, (1, 1, 1)),
+                                       None, None)
+        wanted = reference(x.F.double(), conv.kernel.detach().double(), dense)
+        errors.append(float((out.double() - wanted).norm() / wanted.norm()))
+    assert errors[0] <= 1.03 * errors[1]
+
+
+def test_padded_layers_keep_their_weights_until_told():
+    """Weights of less than four input channels are kept padded: they follow what leaves a mark on the parameter,
+    and a write through .data once the layer is told of it.  (Of four channels the parameter itself is read.)"""
+    for cin, sees in ((3, False), (4, True)):
+        gen = torch.Generator(device=DEVICE).manual_seed(cin)
+        conv = minuet.nn.SparseConv3d(cin, 32, 3, dtype=torch.float32, device=DEVICE)
+        minuet.set_kernel_map_cache(conv, minuet.nn.KernelMapCache(3, torch.int32, DEVICE))
+        cells = torch.randperm(1 << 15, generator=gen, device=DEVICE)[:3000]
+        coordinates = torch.stack([cells >> 10, (cells >> 5) & 31, cells & 31], 1).int()
+        coordinates = coordinates[F.build_sorted_index(coordinates)]
+        x = minuet.SparseTensor(torch.randn(3000, cin, generator=gen, device=DEVICE), coordinates)
+        with torch.no_grad():
+            before = [conv(x).F for _ in range(2)][1]
+            conv.kernel.mul_(2.0)
+            assert torch.equal(conv(x).F, 2.0 * before)
+            conv(x)
+            conv.kernel.data.mul_(2.0)
+            assert torch.equal(conv(x).F, (4.0 if sees else 2.0) * before)
+            conv.invalidate_cached_weights()
+            assert torch.equal(conv(x).F, 4.0 * before) and torch.equal(conv(x).F, 4.0 * before)
+
+
 @pytest.mark.parametrize("dtype, kernel, cin, cout, sizes", [
     (torch.float32, 3, 32, 64, (10000, 60000, 260000)),      # hits, product rows, hits again
     (torch.float16, 5, 64, 256, (1000, 101000)),             # product rows, one kernel

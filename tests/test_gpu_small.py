@@ -46,18 +46,42 @@ def test_map_lists_of_small_clouds(n, kernel, extent, halves):
     check_map_lists(c, orc.generate_kernel_offsets(3, kernel, 1, 1))
 
 
-def check_map_lists(c, off):
+def look_up(rows, off):
+    """The map by a table of the rows (the C oracle packs a row into one key)."""
+    at = {row: i for i, row in enumerate(map(tuple, rows.tolist()))}
+    return np.array([[at.get(row, -1) for row in map(tuple, (rows + step).tolist())] for step in off], dtype=np.int32)
+
+
+def check_map_lists(c, off, query=None):
     index, rows, built = _C.sorted_kernel_map_lists(dev(c), off.astype(np.int64))
     order = orc.arg_sort_coordinates(c)
     np.testing.assert_array_equal(host(index).astype(np.int64), order)
     np.testing.assert_array_equal(host(rows), c[order])
-    ref = c_oracle.query(c[order], c[order], off.astype(np.int32))
+    ref = query(c[order], off) if query else c_oracle.query(c[order], c[order], off.astype(np.int32))
     sizes = orc.compute_kernel_map_sizes(ref)
     by_size = orc.stable_size_order(sizes)
     ein, eout, _ = orc.kernel_map_pair_lists(ref[by_size])
     np.testing.assert_array_equal(built["sizes_host"], np.asarray(sizes)[by_size])
     np.testing.assert_array_equal(host(built["in_idx"]), ein)
     np.testing.assert_array_equal(host(built["out_idx"]), eout)
+
+
+# clouds that the one launch turns down: more rows than a part takes agree in the top bits of the key, and keys
+# that leave no room for the row index (59 bits, which the chain's query takes, and 66, which it does not)
+@pytest.mark.parametrize("n", [500, 4000])
+@pytest.mark.parametrize("shape", ["crowded", "wide", "too wide"])
+@pytest.mark.parametrize("kernel", [3, 4, 5])
+def test_map_lists_of_clouds_turned_down(n, shape, kernel):
+    if shape == "crowded":
+        c = random_cloud(3 * n, 3, n + kernel)
+        c[:, 2] = np.random.default_rng(n).integers(-3000, 3000, size=3 * n)
+        c[0] = (1 << 20, 0, 0)
+    else:
+        c = random_cloud(2 * n, 24, n, lo=-12, dtype=np.int64)
+        c[0] = (1 << 19, (1 << 18) + 3, (1 << 19) + 1) if shape == "wide" else (1 << 21, 1 << 21, 1 << 21)
+    c, _ = sorted_unique(c)
+    c = np.concatenate([c[:n // 2], c[-(n // 2):]])
+    check_map_lists(c[np.random.default_rng(n).permutation(c.shape[0])], orc.generate_kernel_offsets(3, kernel, 1, 1), look_up)
 
 
 # 125 and 49 offsets (two a lane), offsets past the cloud, coordinates of 64 bits far apart, one to four
