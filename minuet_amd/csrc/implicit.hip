@@ -94,7 +94,10 @@ static bool streamed_takes(int64_t Tn, int64_t O, int64_t K, int64_t N) {
 // price of twice the accumulators and source-row registers.
 // PLAIN: a source row is exactly one stage (no chunks, no ragged end), which
 // spares the hot loop the chunk bookkeeping and the end-of-row tests.
-template <typename T, int NB, int KS, int MW, bool PLAIN>
+// KEEP (MW = 1): a weight that is not finite reaches the targets that have a
+// source under its offset only (keep_to_sources), as in the three kernels; else
+// those that share a wavefront with one.
+template <typename T, int NB, int KS, int MW, bool PLAIN, bool KEEP>
 __device__ __forceinline__ void implicit_forward_body(
     const T *__restrict__ sources, unsigned source_bytes, const T *__restrict__ wt,
     const int *__restrict__ kernel_map, long long num_targets, int num_offsets, int K, int N,
@@ -310,6 +313,15 @@ __device__ __forceinline__ void implicit_forward_body(
   }
 #undef MNT_STAGE
 
+  float seen = 0.0f;                           // the largest of the sums that are stored
+  auto keep = [&]() {
+    if constexpr (KEEP) {
+      keep_to_sources<T, NB, 1>(
+          acc[0], seen, sources, K, wt, packed_row, packed_rows, first_channel, N, h, 0, num_offsets,
+          [&](int o) { return kernel_map[static_cast<long long>(o) * num_targets + t_safe[0]]; },
+          [](int o) { return o; }, [&]() { return t_ok[0] ? t[0] : -1ll; }, ep, out);
+    }
+  };
   // Output.  A lane holds 4 consecutive channels of one target per accumulator
   // group and neighbouring lanes hold different targets: written as they are,
   // every lane's few bytes are a request of their own.  Where output rows are
@@ -326,9 +338,11 @@ __device__ __forceinline__ void implicit_forward_body(
 #pragma unroll
       for (int b = 0; b < NB; ++b) {
         if (first_channel + b * 32 >= N) break;
+        if constexpr (KEEP) seen = largest_of<16>(acc[m][b], seen);
         store_turned_block<T>(acc[m][b], turn, lane, r, h, block_t0, num_targets, first_channel + b * 32, N, ep, out);
       }
     }
+    keep();
     return;
   }
 #pragma unroll
@@ -343,18 +357,20 @@ __device__ __forceinline__ void implicit_forward_body(
         float v[4];
 #pragma unroll
         for (int x = 0; x < 4; ++x) v[x] = acc[m][b][q * 4 + x];
+        if constexpr (KEEP) seen = largest_of<4>(v, seen);
         finish_four<T>(v, ep, t[m], ch, N, out);
       }
     }
   }
+  keep();
 }
 
-template <typename T, int NB, int KS, int MW, bool PLAIN>
-__global__ __launch_bounds__(kImplicitBlock) void implicit_forward_kernel(
+template <typename T, int NB, int KS, int MW, bool PLAIN, bool KEEP>
+__global__ __launch_bounds__(kImplicitBlock, KEEP ? 3 : 1) void implicit_forward_kernel(
     const T *__restrict__ sources, unsigned source_bytes, const T *__restrict__ wt,
     const int *__restrict__ kernel_map, long long num_targets, int num_offsets, int K, int N,
     int chunks, int packed_row, int packed_rows, unsigned char *__restrict__ out, Epilogue ep) {
-  implicit_forward_body<T, NB, KS, MW, PLAIN>(sources, source_bytes, wt, kernel_map, num_targets, num_offsets, K, N,
+  implicit_forward_body<T, NB, KS, MW, PLAIN, KEEP>(sources, source_bytes, wt, kernel_map, num_targets, num_offsets, K, N,
                                        chunks, packed_row, packed_rows, out, ep);
 }
 
@@ -657,21 +673,32 @@ static void implicit_typed(const T *sources, const T *weights, const T *packed, 
   const dim3 grid(static_cast<unsigned>(div_ceil(Tn, kImplicitTargets * (wide ? 2 : 1))),
                   static_cast<unsigned>(groups));
   const bool plain = chunks == 1 && K * static_cast<int64_t>(sizeof(T)) == stage_bytes;
-#define MNT_IMPLICIT(NB, KS, MW)                                                                   \
+#define MNT_IMPLICIT_K(NB, KS, MW, KEEP)                                                           \
   if (plain) {                                                                                     \
-    implicit_forward_kernel<T, NB, KS, MW, true><<<grid, kImplicitBlock, 0, stream>>>(             \
+    implicit_forward_kernel<T, NB, KS, MW, true, KEEP><<<grid, kImplicitBlock, 0, stream>>>(       \
         sources, source_bytes, wt, kernel_map, Tn, static_cast<int>(O), static_cast<int>(K),       \
         static_cast<int>(N), chunks, Kp, Np, reinterpret_cast<unsigned char *>(out), ep);          \
   } else {                                                                                         \
-    implicit_forward_kernel<T, NB, KS, MW, false><<<grid, kImplicitBlock, 0, stream>>>(            \
+    implicit_forward_kernel<T, NB, KS, MW, false, KEEP><<<grid, kImplicitBlock, 0, stream>>>(      \
         sources, source_bytes, wt, kernel_map, Tn, static_cast<int>(O), static_cast<int>(K),       \
         static_cast<int>(N), chunks, Kp, Np, reinterpret_cast<unsigned char *>(out), ep);          \
   }
+#define MNT_IMPLICIT(NB, KS, MW) MNT_IMPLICIT_K(NB, KS, MW, false)
 #define MNT_IMPLICIT_KS(NB, MW)           \
   if (stage_bytes == 64) {                \
     MNT_IMPLICIT(NB, 2, MW);              \
   } else {                                \
     MNT_IMPLICIT(NB, 4, MW);              \
+  }
+  if constexpr (sizeof(T) == 2) {
+    // 16-bit rows of up to 64 bytes under several groups of channels (`auto` takes these
+    // layers here where three kernels would write their product rows)
+    if (groups > 1 && stage_bytes == 64) {
+      MNT_IMPLICIT_K(kImplicitMaxBlocks, 2, 1, true)
+      check_launch("implicit_forward_kernel");
+      profile_mark("implicit", stream);
+      return;
+    }
   }
   switch (blocks) {
     case 1: MNT_IMPLICIT_KS(1, 1); break;
@@ -687,6 +714,7 @@ static void implicit_typed(const T *sources, const T *weights, const T *packed, 
   }
 #undef MNT_IMPLICIT_KS
 #undef MNT_IMPLICIT
+#undef MNT_IMPLICIT_K
   check_launch("implicit_forward_kernel");
   profile_mark("implicit", stream);
 }

@@ -109,6 +109,8 @@ struct TiledShape {
 // weights are finite, so that a layer may change from one to the other between
 // two calls.  A weight that is not reaches the targets that share a wavefront
 // with one that uses its offset, in either kernel; which those are differs.
+// KEEP (rows of up to 64 bytes under more than 128 channels): those that have a
+// source under its offset only (keep_to_sources), as in the three kernels.
 // PAIRED (rows of up to 64 bytes): a stage is two offsets, one per half of the
 // wavefront's lanes, which halves what a stage costs besides its products.
 // WHOLE: a source row is exactly one stage (or half of one, PAIRED).
@@ -131,7 +133,7 @@ struct TiledShape {
 // targets of an object 14.9 / 8.8, 25 000 of a LiDAR scan 14.9 / 10.3, 60 000
 // of a room 18.2 / 17.4; in tiles, LiDAR, 200 000 48.6 / 27, a
 // million under 5 x 5 x 5 836 / 403.
-template <typename T, int NB, int KS, bool TILED, bool PAIRED, bool WHOLE, bool QUADS, int GROUPS>
+template <typename T, int NB, int KS, bool TILED, bool PAIRED, bool WHOLE, bool QUADS, int GROUPS, bool KEEP>
 __global__ __launch_bounds__(256 * GROUPS) void tiled_forward_kernel(
     const T *__restrict__ sources, unsigned source_bytes, const T *__restrict__ wt,
     const int *__restrict__ kernel_map, TileView tiles, TiledShape s, unsigned char *__restrict__ out, Epilogue ep) {
@@ -221,8 +223,10 @@ __global__ __launch_bounds__(256 * GROUPS) void tiled_forward_kernel(
 #pragma unroll
   for (int i = 0; i < kWPieces; ++i) {
     const int row = min(tid / kRowPieces + kWRows * i, Np - 1);
-    w_at[i] = static_cast<unsigned>(min(first_channel + row, s.packed_rows - 1) * s.packed_row * ES +
-                                    (PAIRED ? w_piece & 3 : w_piece) * 16);
+    const int channel = min(first_channel + row, s.packed_rows - 1);
+    // (in 24 bits where the 64-bit product's register pair came to hold what is being loaded: 4 to 8 % of a layer)
+    const int channel_at = KEEP ? static_cast<int>(__umul24(channel, s.packed_row * ES)) : channel * s.packed_row * ES;
+    w_at[i] = static_cast<unsigned>(channel_at + (PAIRED ? w_piece & 3 : w_piece) * 16);
     w_put[i] = static_cast<unsigned>(row / 32 * kBlockStride + row % 32 * kLdsRow + w_piece * 16) +
                group * 2 * kBufferBytes;
   }
@@ -393,12 +397,25 @@ __global__ __launch_bounds__(256 * GROUPS) void tiled_forward_kernel(
     }
     __syncthreads();
   }
+  float seen = 0.0f;                           // the largest of the sums that are stored
+  auto keep = [&]() {
+    if constexpr (KEEP) {
+      keep_to_sources<T, NB, GROUPS>(
+          acc, seen, sources, s.K, wt, s.packed_row, s.packed_rows, first_channel, s.N, h, group, live,
+          [&](int slot) {
+            return TILED ? tiles.sources[(tile * s.slots + slot) * kTileTargets + wv * 32 + r]
+                         : kernel_map[slot * s.num_targets + target];
+          },
+          [&](int slot) { return TILED ? offsets_at[slot] : slot; },
+          [&]() { return static_cast<long long>(row_of(wv * 32 + r)); }, ep, out);
+    }
+  };
   if ((static_cast<long long>(s.N) * ES) % 16 != 0) {      // output rows are no whole 16-byte pieces
     const int row = row_of(wv * 32 + r);
-    if (row < 0) return;
+    if (!KEEP && row < 0) return;
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
-      if (b % GROUPS != group) continue;
+      if (b % GROUPS != group || (KEEP && row < 0)) continue;
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int ch = first_channel + b * 32 + q * 8 + h * 4;
@@ -406,9 +423,11 @@ __global__ __launch_bounds__(256 * GROUPS) void tiled_forward_kernel(
         float v[4];
 #pragma unroll
         for (int x = 0; x < 4; ++x) v[x] = acc[b][q * 4 + x];
+        if constexpr (KEEP) seen = largest_of<4>(v, seen);
         finish_four<T>(v, ep, row, ch, s.N, out);
       }
     }
+    keep();
     return;
   }
   unsigned char *turn = lds + (group * 4 + wv) * kTurnBytes;
@@ -416,8 +435,10 @@ __global__ __launch_bounds__(256 * GROUPS) void tiled_forward_kernel(
   for (int b = 0; b < NB; ++b) {
     if (first_channel + b * 32 >= s.N) break;
     if (b % GROUPS != group) continue;
+    if constexpr (KEEP) seen = largest_of<16>(acc[b], seen);
     store_turned_rows<T>(acc[b], turn, lane, r, h, out_row, first_channel + b * 32, s.N, ep, out);
   }
+  keep();
 }
 
 template <typename T>
@@ -456,21 +477,28 @@ void tiled_forward(const T *sources, const T *packed, const int *kernel_map, con
   // tiles of large kernels have more stages to hide the latency behind and gain
   // from a quarter of a million targets on only.
   const bool quads = nb <= 2 && (O <= 32 || 2 * filled >= 16 * cus);
+  const bool keep = row_bytes <= 64 && N > 128;
   const dim3 grid(static_cast<unsigned>(tiled ? l.tiles : filled), static_cast<unsigned>(y));
-#define MNT_TILED(NB, KS, TILED, PAIRED, WHOLE, QUADS, GROUPS)                                              \
-  tiled_forward_kernel<T, NB, KS, TILED, PAIRED, WHOLE, QUADS, GROUPS><<<grid, 256 * GROUPS, 0, stream>>>(  \
+#define MNT_TILED_K(NB, KS, TILED, PAIRED, WHOLE, QUADS, GROUPS, KEEP)                                            \
+  tiled_forward_kernel<T, NB, KS, TILED, PAIRED, WHOLE, QUADS, GROUPS, KEEP><<<grid, 256 * GROUPS, 0, stream>>>(  \
       sources, source_bytes, packed, kernel_map, view, s, reinterpret_cast<unsigned char *>(out), ep)
+#define MNT_TILED(NB, KS, TILED, PAIRED, WHOLE, QUADS, GROUPS)                 \
+  if ((PAIRED || KS == 2) && keep) {                                           \
+    MNT_TILED_K(NB, KS, TILED, PAIRED, WHOLE, QUADS, GROUPS, (PAIRED || KS == 2)); \
+  } else {                                                                     \
+    MNT_TILED_K(NB, KS, TILED, PAIRED, WHOLE, QUADS, GROUPS, false);           \
+  }
 #define MNT_TILED_Q(NB, KS, WHOLE)                               \
   if (NB <= 2 && quads) {                                        \
-    MNT_TILED(NB, KS, true, false, WHOLE, (NB <= 2), 1);         \
+    MNT_TILED(NB, KS, true, false, WHOLE, (NB <= 2), 1)          \
   } else {                                                       \
-    MNT_TILED(NB, KS, true, false, WHOLE, false, 1);             \
+    MNT_TILED(NB, KS, true, false, WHOLE, false, 1)              \
   }
 #define MNT_TILED_G(NB, PAIRED, WHOLE)                           \
   if (two) {                                                     \
-    MNT_TILED(NB, 4, false, PAIRED, WHOLE, false, 2);            \
+    MNT_TILED(NB, 4, false, PAIRED, WHOLE, false, 2)             \
   } else {                                                       \
-    MNT_TILED(NB, 4, false, PAIRED, WHOLE, false, 1);            \
+    MNT_TILED(NB, 4, false, PAIRED, WHOLE, false, 1)             \
   }
 #define MNT_TILED_N(NB)                                          \
   if (tiled && stage_bytes == 64) {                              \
@@ -506,6 +534,7 @@ void tiled_forward(const T *sources, const T *packed, const int *kernel_map, con
 #undef MNT_TILED_G
 #undef MNT_TILED_Q
 #undef MNT_TILED
+#undef MNT_TILED_K
   check_launch("tiled_forward_kernel");
 }
 

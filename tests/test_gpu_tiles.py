@@ -347,3 +347,48 @@ def test_layers_of_one_map_make_its_tiles_once(first):
         assert torch.cuda.memory_allocated() - before <= weights < 1 << 20       # (tiles take 8 MB)
         kept, = (entry for maps in cache._fast_maps.values() for entry in maps.values())
         assert kept is entry and kept.tiles_saved > saved
+
+
+# the kernel for few targets with one and two sets of wavefronts, the one for many, tiles of both; one to four
+# groups of channels, a last one of less than a block; rows of 16 to 64 bytes
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("targets,offsets,cin,cout", [
+    (1, 27, 32, 132), (3000, 27, 8, 512), (700, 8, 24, 160), (60000, 27, 16, 256), (70000, 27, 32, 132), (90000, 8, 24, 384),
+    (5000, 125, 32, 160), (66000, 125, 8, 136)])
+def test_weights_that_are_not_finite_under_many_channels(targets, offsets, cin, cout, dtype):
+    """Rows of up to 64 bytes and more than 128 output channels, which three kernels took before: a weight that is
+    not finite reaches the targets that have a source under its offset, one by one."""
+    dense, x, w = operands(targets, 3000, offsets, cin, cout, dtype)
+    tiles = _C.kernel_map_tiles(dense)
+    spoilt = w.clone()
+    reached = torch.zeros(targets, cout, dtype=torch.bool, device=DEVICE)
+    for offset, value in ((0, "inf"), (offsets // 2, "nan"), (offsets - 1, "-inf")):
+        spoilt[offset, cin - 1, 3], spoilt[offset, 0, cout - 1] = float(value), float(value)
+        reached[:, [3, cout - 1]] |= (dense[offset] >= 0)[:, None]
+    wanted = reference(x, w, dense)
+    size = reference(x.abs(), w.abs(), dense)
+    # sums of up to 125 x 32 products in 32 bits, in whichever order, and one rounding
+    bound = torch.finfo(dtype).eps * wanted.abs() + 2 * offsets * cin * 2.0 ** -24 * size + 1e-7
+    plain = [_C.sparse_convolution_forward_implicit(x, w, dense), _C.sparse_convolution_forward_tiled(
+        x, w, tiles, targets, F.pack_weights(w))]
+    got = [_C.sparse_convolution_forward_implicit(x, spoilt, dense), _C.sparse_convolution_forward_tiled(
+        x, spoilt, tiles, targets, F.pack_weights(spoilt))]
+    for before, after in zip(plain, got):
+        assert bool(((before.float() - wanted).abs() <= bound).all())
+        assert not bool(after[reached].isfinite().any())
+        assert bool(((after.float() - wanted).abs() <= bound)[~reached].all())
+        untouched = torch.ones(cout, dtype=torch.bool, device=DEVICE)
+        untouched[[3, cout - 1]] = False
+        assert torch.equal(after[:, untouched], before[:, untouched])
+    gen = torch.Generator(device=DEVICE).manual_seed(4)
+    scale, shift = (torch.randn(cout, generator=gen, device=DEVICE) for _ in range(2))
+    residual = torch.randn(targets, cout, generator=gen, device=DEVICE).to(dtype)
+    for act, slope in (("relu", 0.0), ("leaky_relu", 0.25), (None, 0.0)):
+        epilogue = F.Epilogue(scale, shift, residual, act, slope)
+        finished = wanted * scale + shift + residual
+        finished = torch.where(finished > 0, finished, finished * slope) if act else finished
+        limit = torch.finfo(dtype).eps * finished.abs() + scale.abs() * bound + 4 * 2.0 ** -24 * (
+            scale.abs() * wanted.abs() + shift.abs() + residual.abs()) + 1e-7
+        for after in (_C.sparse_convolution_forward_implicit(x, spoilt, dense, epilogue=epilogue),
+                      _C.sparse_convolution_forward_tiled(x, spoilt, tiles, targets, F.pack_weights(spoilt), epilogue=epilogue)):
+            assert bool(((after.float() - finished).abs() <= limit)[~reached].all())
